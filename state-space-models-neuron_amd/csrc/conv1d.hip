@@ -15,8 +15,10 @@
 // loses that contribution).  dw/db are reduced in fp32: registers -> LDS per block ->
 // per-block partials in the workspace -> one small second-stage kernel.  No float atomics.
 //
-// A generic path (any strides, k <= 8, any C) covers the channel-major (b, C, l) layout of
-// ConvNKI and unaligned shapes with one thread per output element.
+// The channel-major (b, C, l) layout of ConvNKI has its own kernels (conv_*_cm_kernel): a lane owns consecutive tokens
+// of one row, so the taps of an output come from the lane's own window and nothing is loaded per tap.
+//
+// A generic path (any strides, k <= 8) covers the rest with one thread per output element.
 #include "common.hpp"
 
 namespace m2 {
@@ -59,10 +61,12 @@ constexpr int kSEG = M2_CONV_SEG;    // token segments per block (y dimension)
 static_assert(kTLF % kUNR == 0 && kTLB % kUNR == 0 && kUNR >= 3, "segments are whole load groups; the dx lag fits one group");
 
 // streaming loads/stores of the activations (optionally non-temporal: nothing is re-read soon enough to be worth caching)
+// The vectors promise the alignment of an element only: gfx950 issues the same wide access either way, so rows that start
+// anywhere (an odd number of channels, of tokens, or of columns in front of a slice) take the vector kernels as well.
 template <int BYTES> struct StreamVec;
-template <> struct StreamVec<16> { typedef uint32_t type __attribute__((ext_vector_type(4))); };
-template <> struct StreamVec<8> { typedef uint32_t type __attribute__((ext_vector_type(2))); };
-template <> struct StreamVec<4> { typedef uint32_t type; };
+template <> struct StreamVec<16> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(2))); };
+template <> struct StreamVec<8> { typedef uint32_t type __attribute__((ext_vector_type(2), aligned(2))); };
+template <> struct StreamVec<4> { typedef uint32_t type __attribute__((aligned(2))); };
 template <typename T, int V>
 __device__ __forceinline__ RawVec<T, V> ld_stream(const T* __restrict__ p) {
     using S = typename StreamVec<V * (int)sizeof(T)>::type;
@@ -79,6 +83,15 @@ __device__ __forceinline__ void st_stream(T* __restrict__ p, const float (&in)[V
 #pragma unroll
     for (int i = 0; i < V; ++i) e[i] = from_f32<T>(in[i]);
     if (M2_CONV_NT) __builtin_nontemporal_store(raw, reinterpret_cast<S*>(p)); else *reinterpret_cast<S*>(p) = raw;
+}
+// cached load of V elements from anywhere (windows that neighbours read too)
+template <typename T, int V>
+__device__ __forceinline__ void ld_elems(const T* __restrict__ p, float (&out)[V]) {
+    using S = typename StreamVec<V * (int)sizeof(T)>::type;
+    const S v = *reinterpret_cast<const S*>(p);
+    const T* e = reinterpret_cast<const T*>(&v);
+#pragma unroll
+    for (int i = 0; i < V; ++i) out[i] = to_f32(e[i]);
 }
 
 __device__ __forceinline__ float ld_param(const void* p, int pd, int64_t i) {
@@ -101,7 +114,7 @@ __device__ __forceinline__ void load_taps(const void* __restrict__ w, const void
 #pragma unroll
     for (int i = 0; i < V * 4 / TV; ++i) {
         float tmp[TV];
-        loadv<WT, TV>(wp + i * TV, tmp);
+        ld_elems<WT, TV>(wp + i * TV, tmp);
 #pragma unroll
         for (int e = 0; e < TV; ++e) flat[i * TV + e] = tmp[e];
     }
@@ -116,7 +129,7 @@ __device__ __forceinline__ void load_taps(const void* __restrict__ w, const void
 #pragma unroll
         for (int i = 0; i < V / BV; ++i) {
             float tmp[BV];
-            loadv<WT, BV>(static_cast<const WT*>(bias) + c0 + i * BV, tmp);
+            ld_elems<WT, BV>(static_cast<const WT*>(bias) + c0 + i * BV, tmp);
 #pragma unroll
             for (int e = 0; e < BV; ++e) bv[i * BV + e] = tmp[e];
         }
@@ -133,9 +146,9 @@ conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     const int64_t cv = (int64_t)blockIdx.x * kCVT + threadIdx.x;
     const int64_t seg = (int64_t)blockIdx.y * kSEG + threadIdx.y;
     const int64_t b = blockIdx.z;
-    const int64_t c0 = cv * V;
     const int64_t t0 = seg * kTLF;
-    if (c0 >= C || t0 >= l) return;
+    if (cv * V >= C || t0 >= l) return;
+    const int64_t c0 = cv * V < C - V ? cv * V : C - V;     // the last vector ends with the row (it may repeat channels: same values)
 
     float wv[4][V], bv[V];
     load_taps<WT, V>(w, bias, c0, wv, bv);
@@ -144,9 +157,9 @@ conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     float h0[V], h1[V], h2[V];   // x[t-3], x[t-2], x[t-1]
 #pragma unroll
     for (int j = 0; j < V; ++j) h0[j] = h1[j] = h2[j] = 0.f;
-    if (t0 - 3 >= 0) loadv<T, V>(xp + (t0 - 3) * xsl, h0);
-    if (t0 - 2 >= 0) loadv<T, V>(xp + (t0 - 2) * xsl, h1);
-    if (t0 - 1 >= 0) loadv<T, V>(xp + (t0 - 1) * xsl, h2);
+    if (t0 - 3 >= 0) ld_elems<T, V>(xp + (t0 - 3) * xsl, h0);
+    if (t0 - 2 >= 0) ld_elems<T, V>(xp + (t0 - 2) * xsl, h1);
+    if (t0 - 1 >= 0) ld_elems<T, V>(xp + (t0 - 1) * xsl, h2);
     auto step = [&](const RawVec<T, V>& r, T* __restrict__ yq) {
         float out[V], cur[V];
         cvtv<T, V>(r, cur);
@@ -210,9 +223,9 @@ conv_bwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     const int64_t cv = (int64_t)blockIdx.x * kCVT + threadIdx.x;
     const int64_t seg = (int64_t)blockIdx.y * kSEG + threadIdx.y;
     const int64_t b = blockIdx.z;
-    const int64_t c0 = cv * V;
+    const int64_t c0 = cv * V < C - V ? cv * V : C - V;     // the last vector ends with the row (it may repeat channels: same values)
     const int64_t t0 = seg * kTLB;
-    const bool active = (c0 < C) && (t0 < l);
+    const bool active = (cv * V < C) && (t0 < l);
 
     float acc[5][V];
 #pragma unroll
@@ -230,9 +243,9 @@ conv_bwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
         float g0[V], g1[V], g2[V];   // g[t-3..t-1]
 #pragma unroll
         for (int j = 0; j < V; ++j) h0[j] = h1[j] = h2[j] = g0[j] = g1[j] = g2[j] = 0.f;
-        if (t0 - 3 >= 0) loadv<T, V>(xp + (t0 - 3) * xsl, h0);
-        if (t0 - 2 >= 0) loadv<T, V>(xp + (t0 - 2) * xsl, h1);
-        if (t0 - 1 >= 0) loadv<T, V>(xp + (t0 - 1) * xsl, h2);
+        if (t0 - 3 >= 0) ld_elems<T, V>(xp + (t0 - 3) * xsl, h0);
+        if (t0 - 2 >= 0) ld_elems<T, V>(xp + (t0 - 2) * xsl, h1);
+        if (t0 - 1 >= 0) ld_elems<T, V>(xp + (t0 - 1) * xsl, h2);
         // one token: g[t] from x[t-3..t] and dy[t]; the weight/bias sums if the token is this thread's own; dx[t-3] to dq if emit
         auto step = [&](const RawVec<T, V>& rx, const RawVec<T, V>& rg, bool own, bool emit, T* __restrict__ dq) {
             float g[V], cur[V], gy[V];
@@ -324,8 +337,9 @@ conv_bwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     const int64_t pslot = (int64_t)blockIdx.z * gridDim.y + blockIdx.y;
     for (int e = tid; e < 5 * kCVT * V; e += kCVT * kSEG) {
         const int i = e / (kCVT * V), cc = e % (kCVT * V);
-        const int64_t c = (int64_t)blockIdx.x * kCVT * V + cc;
-        if (c < C) {
+        const int64_t cb = (int64_t)blockIdx.x * kCVT * V + cc / V * V;      // first channel of the owning thread
+        const int64_t c = (cb < C - V ? cb : C - V) + cc % V;
+        if (cb < C) {
             float s = 0.f;
 #pragma unroll
             for (int r = 0; r < kSEG; ++r) s += red[r][i][cc];
@@ -362,6 +376,131 @@ conv_reduce_partials_kernel(const float* __restrict__ part, int64_t nslots, int6
     if (!live || q != 0) return;
     if (i < k) st_param(dw, pd, c * k + i, s);
     else if (db) st_param(db, pd, c, s);
+}
+
+// ------------------------------------------------------------------------------------------
+// Channel-major path, k == 4: tokens contiguous in x, y (and dx).
+//
+// N tokens [t, t + N) of a row of l as fp32: one vector access where they all exist, zeros outside the row.
+template <typename T, int N>
+__device__ __forceinline__ void ld_tokens(const T* __restrict__ row, int64_t t, int64_t l, float (&out)[N]) {
+    if (t >= 0 && t + N <= l) {
+        ld_elems<T, N>(row + t, out);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) out[i] = (t + i >= 0 && t + i < l) ? to_f32(row[t + i]) : 0.f;
+    }
+}
+template <typename T, int N>
+__device__ __forceinline__ void st_tokens(T* __restrict__ row, int64_t t, int64_t l, const float (&in)[N]) {
+    if (t + N <= l) {
+        st_stream<T, N>(row + t, in);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if (t + i < l) row[t + i] = from_f32<T>(in[i]);
+    }
+}
+template <typename WT>
+__device__ __forceinline__ void ld_row_taps(const void* __restrict__ w, const void* __restrict__ bias, int64_t c, float (&wv)[4], float& bv) {
+    ld_elems<WT, 4>(static_cast<const WT*>(w) + c * 4, wv);
+    bv = bias ? to_f32(static_cast<const WT*>(bias)[c]) : 0.f;
+}
+
+// One thread per 16-byte piece of a row: its own tokens and the 4 before them (an L1 hit: the neighbour's own), eight
+// waves' worth of pieces per SIMD in flight.  HBM bound.
+template <typename T, typename WT, int ACT>
+__global__ void __launch_bounds__(256)
+conv_fwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias, T* __restrict__ y,
+                   int64_t l, uint32_t C, uint32_t pieces, uint32_t total, int64_t xsb, int64_t xsc, int64_t ysb, int64_t ysc) {
+    constexpr int V = VecTraits<T>::kVec;
+    const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
+    if (idx >= total) return;
+    const uint32_t row = idx / pieces, b = row / C, c = row - b * C;
+    const int64_t t0 = (int64_t)(idx - row * pieces) * V;
+    const T* xr = x + b * xsb + c * xsc;
+    float h[4], cur[V], wv[4], bv, o[V];
+    ld_tokens<T, V>(xr, t0, l, cur);
+    ld_tokens<T, 4>(xr, t0 - 4, l, h);
+    ld_row_taps<WT>(w, bias, c, wv, bv);
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        float z = bv;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) z += wv[k] * (i + k < 3 ? h[1 + i + k] : cur[i + k - 3]);
+        o[i] = act_f<ACT>(z);
+    }
+    st_tokens<T, V>(y + b * ysb + c * ysc, t0, l, o);
+}
+
+// One wave per (channel, split): its lanes walk the channel's pieces of two vectors of tokens over all rows of the batch,
+// so the sums of dw and db stay in registers until the end and one wave's reduction finishes a channel (splits > 1: fp32
+// partials for conv_reduce_partials_kernel).  A lane recomputes the three tokens behind its own for the dx lag: 3 in 16
+// (bf16) more activations, against a cross-lane exchange that would break at every row end.
+template <typename T, typename WT, int ACT>
+__global__ void __launch_bounds__(256)
+conv_bwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias, const T* __restrict__ dy,
+                   T* __restrict__ dx, float* __restrict__ part, void* __restrict__ dw, void* __restrict__ db,
+                   int64_t l, uint32_t C, uint32_t splits, uint32_t pieces, uint32_t per_split, uint32_t total,
+                   int64_t xsb, int64_t xsc, int64_t gsb, int64_t gsc, int64_t dsb, int64_t dsc) {
+    constexpr int V = VecTraits<T>::kVec, N = 2 * V;
+    const uint32_t unit = blockIdx.x * 4u + (threadIdx.x >> 6);
+    if (unit >= C * splits) return;
+    const uint32_t split = unit / C, c = unit - split * C;
+    const uint32_t end = (split + 1) * per_split < total ? (split + 1) * per_split : total;
+    float wv[4], bv, acc[5];
+    ld_row_taps<WT>(w, bias, c, wv, bv);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) acc[k] = 0.f;
+    for (uint32_t p = split * per_split + (threadIdx.x & 63); p < end; p += 64) {
+        const uint32_t b = p / pieces;
+        const int64_t t0 = (int64_t)(p - b * pieces) * N;
+        const T* xr = x + b * xsb + c * xsc;
+        const T* gr = dy + b * gsb + c * gsc;
+        T* dr = dx + b * dsb + c * dsc;
+        float xa[4], xb[V], xc[V], xd[4], ga[V], gb[V], gc[4];
+        ld_tokens<T, V>(xr, t0, l, xb);
+        ld_tokens<T, V>(gr, t0, l, ga);
+        ld_tokens<T, V>(xr, t0 + V, l, xc);
+        ld_tokens<T, V>(gr, t0 + V, l, gb);
+        ld_tokens<T, 4>(xr, t0 - 4, l, xa);
+        ld_tokens<T, 4>(xr, t0 + N, l, xd);
+        ld_tokens<T, 4>(gr, t0 + N, l, gc);
+        float xw[N + 8], g[N + 4];                 // x[t0 - 4 ...], dy -> g = dy * act'(z) from t0 on
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { xw[i] = xa[i]; xw[4 + N + i] = xd[i]; g[N + i] = gc[i]; }
+#pragma unroll
+        for (int i = 0; i < V; ++i) { xw[4 + i] = xb[i]; xw[4 + V + i] = xc[i]; g[i] = ga[i]; g[V + i] = gb[i]; }
+#pragma unroll
+        for (int i = 0; i < N + 3; ++i) {
+            const float z = bv + wv[0] * xw[i + 1] + wv[1] * xw[i + 2] + wv[2] * xw[i + 3] + wv[3] * xw[i + 4];
+            g[i] *= act_grad_f<ACT>(z);            // dy is 0 behind the row's end
+            if (i < N) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) acc[k] += xw[i + 1 + k] * g[i];
+                acc[4] += g[i];
+            }
+        }
+        float oa[V], ob[V];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float o = wv[3] * g[i] + wv[2] * g[i + 1] + wv[1] * g[i + 2] + wv[0] * g[i + 3];
+            if (i < V) oa[i] = o; else ob[i - V] = o;
+        }
+        st_tokens<T, V>(dr, t0, l, oa);
+        if (t0 + V < l) st_tokens<T, V>(dr, t0 + V, l, ob);
+    }
+#pragma unroll
+    for (int k = 0; k < 5; ++k) acc[k] = warp_sum(acc[k]);
+    if ((threadIdx.x & 63) == 0) {
+        constexpr int pd = std::is_same<WT, float>::value ? M2_F32 : M2_BF16;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            if (splits > 1) part[((int64_t)split * C + c) * 5 + k] = acc[k];
+            else if (k < 4) st_param(dw, pd, (int64_t)c * 4 + k, acc[k]);
+            else if (db) st_param(db, pd, c, acc[k]);
+        }
+    }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -463,20 +602,27 @@ template <typename T> constexpr int conv_vec(bool bwd) {
     return v < 2 ? 2 : v;
 }
 
-template <typename T, int V>
-bool fast_path_ok(const m2_conv1d_params* p, bool bwd) {
-    if (p->k != 4 || p->x_stride_c != 1 || p->y_stride_c != 1) return false;
-    if (p->channels % V) return false;
-    if (p->x_stride_b % V || p->x_stride_l % V || p->y_stride_b % V || p->y_stride_l % V) return false;
-    auto al = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) % (V * sizeof(T))) == 0; };
-    if (!al(p->x)) return false;
-    if (reinterpret_cast<uintptr_t>(p->w) % 16 || reinterpret_cast<uintptr_t>(p->bias) % 16) return false;   // vector tap loads
-    if (!bwd && !al(p->y)) return false;
-    if (bwd) {
-        if (p->dx_stride_c != 1 || p->dx_stride_b % V || p->dx_stride_l % V) return false;
-        if (!al(p->dy) || !al(p->dx)) return false;
-    }
-    return true;
+// Channels-last kernels: unit channel strides; a row must hold one vector.
+template <int V>
+bool channels_last_ok(const m2_conv1d_params* p, bool bwd) {
+    return p->k == 4 && p->x_stride_c == 1 && p->y_stride_c == 1 && p->channels >= V && (!bwd || p->dx_stride_c == 1);
+}
+// Channel-major kernels: unit token strides; the flattened pieces are counted in 32 bits.
+bool channel_major_ok(const m2_conv1d_params* p, bool bwd) {
+    return p->k == 4 && p->x_stride_l == 1 && p->y_stride_l == 1 && (!bwd || p->dx_stride_l == 1) &&
+           p->channels < (int64_t(1) << 24) && p->batch * p->channels * ceil_div(p->seqlen, (int64_t)4) < (int64_t(1) << 31);
+}
+
+// calls f<parameter type, activation>
+template <typename F>
+void conv_dispatch(const m2_conv1d_params* p, F&& f) {
+    auto act = [&](auto wt) {
+        using WT = decltype(wt);
+        if (p->activation == M2_ACT_SILU) f(WT{}, std::integral_constant<int, M2_ACT_SILU>{});
+        else if (p->activation == M2_ACT_RELU) f(WT{}, std::integral_constant<int, M2_ACT_RELU>{});
+        else f(WT{}, std::integral_constant<int, M2_ACT_NONE>{});
+    };
+    if (p->param_dtype == M2_F32) act(float{}); else act(bf16_t{});
 }
 
 int check_common(const m2_conv1d_params* p) {
@@ -496,19 +642,20 @@ int launch_fwd(const m2_conv1d_params* p, hipStream_t st) {
     const T* x = static_cast<const T*>(p->x);
     T* y = static_cast<T*>(p->y);
     constexpr int V = conv_vec<T>(false);
-    if (fast_path_ok<T, V>(p, false) && p->activation != M2_ACT_RELU) {
-        const int64_t CV = C / V, nseg = ceil_div(l, kTLF);
+    if (channels_last_ok<V>(p, false)) {
+        const int64_t CV = ceil_div(C, (int64_t)V), nseg = ceil_div(l, kTLF);
         dim3 grid((unsigned)ceil_div(CV, kCVT), (unsigned)ceil_div(nseg, kSEG), (unsigned)nb), block(kCVT, kSEG);
         M2_REQUIRE(grid.y <= 65535, M2_ERR_SHAPE, "conv1d: sequence too long for the grid");
-        auto go = [&](auto kern) {
-            kern<<<grid, block, 0, st>>>(x, p->w, p->bias, y, l, C, p->x_stride_b, p->x_stride_l, p->y_stride_b, p->y_stride_l);
-        };
-        const bool silu = p->activation == M2_ACT_SILU;
-        if (p->param_dtype == M2_F32) {
-            if (silu) go(conv_fwd_cl_kernel<T, float, V, M2_ACT_SILU>); else go(conv_fwd_cl_kernel<T, float, V, M2_ACT_NONE>);
-        } else {
-            if (silu) go(conv_fwd_cl_kernel<T, bf16_t, V, M2_ACT_SILU>); else go(conv_fwd_cl_kernel<T, bf16_t, V, M2_ACT_NONE>);
-        }
+        conv_dispatch(p, [&](auto wt, auto act) {
+            conv_fwd_cl_kernel<T, decltype(wt), V, decltype(act)::value><<<grid, block, 0, st>>>(
+                x, p->w, p->bias, y, l, C, p->x_stride_b, p->x_stride_l, p->y_stride_b, p->y_stride_l);
+        });
+    } else if (channel_major_ok(p, false)) {
+        const int64_t pieces = ceil_div(l, (int64_t)VecTraits<T>::kVec), total = nb * C * pieces;
+        conv_dispatch(p, [&](auto wt, auto act) {
+            conv_fwd_cm_kernel<T, decltype(wt), decltype(act)::value><<<(unsigned)ceil_div(total, (int64_t)256), 256, 0, st>>>(
+                x, p->w, p->bias, y, l, (uint32_t)C, (uint32_t)pieces, (uint32_t)total, p->x_stride_b, p->x_stride_c, p->y_stride_b, p->y_stride_c);
+        });
     } else {
         const int64_t total = nb * l * C;
         const int tf = (p->x_stride_l == 1 && p->x_stride_c != 1) ? 1 : 0;
@@ -526,8 +673,8 @@ int launch_bwd(const m2_conv1d_params* p, hipStream_t st) {
     const T* dy = static_cast<const T*>(p->dy);
     T* dx = static_cast<T*>(p->dx);
     constexpr int V = conv_vec<T>(true);
-    if (fast_path_ok<T, V>(p, true) && p->activation != M2_ACT_RELU) {
-        const int64_t CV = C / V, nseg = ceil_div(l, kTLB);
+    if (channels_last_ok<V>(p, true)) {
+        const int64_t CV = ceil_div(C, (int64_t)V), nseg = ceil_div(l, kTLB);
         dim3 grid((unsigned)ceil_div(CV, kCVT), (unsigned)ceil_div(nseg, kSEG), (unsigned)nb), block(kCVT, kSEG);
         M2_REQUIRE(grid.y <= 65535, M2_ERR_SHAPE, "conv1d: sequence too long for the grid");
         const int64_t nslots = (int64_t)grid.y * grid.z;
@@ -535,19 +682,35 @@ int launch_bwd(const m2_conv1d_params* p, hipStream_t st) {
         M2_REQUIRE(p->workspace && p->workspace_bytes >= need, M2_ERR_WORKSPACE,
                    "conv1d_bwd: workspace %zu bytes < %zu needed", p->workspace_bytes, need);
         float* part = static_cast<float*>(p->workspace);
-        auto go = [&](auto kern) {
-            kern<<<grid, block, 0, st>>>(x, p->w, p->bias, dy, dx, part, l, C, p->x_stride_b, p->x_stride_l, p->y_stride_b, p->y_stride_l,
-                                         p->dx_stride_b, p->dx_stride_l);
-        };
-        const bool silu = p->activation == M2_ACT_SILU;
-        if (p->param_dtype == M2_F32) {
-            if (silu) go(conv_bwd_cl_kernel<T, float, V, M2_ACT_SILU>); else go(conv_bwd_cl_kernel<T, float, V, M2_ACT_NONE>);
-        } else {
-            if (silu) go(conv_bwd_cl_kernel<T, bf16_t, V, M2_ACT_SILU>); else go(conv_bwd_cl_kernel<T, bf16_t, V, M2_ACT_NONE>);
-        }
+        conv_dispatch(p, [&](auto wt, auto act) {
+            conv_bwd_cl_kernel<T, decltype(wt), V, decltype(act)::value><<<grid, block, 0, st>>>(
+                x, p->w, p->bias, dy, dx, part, l, C, p->x_stride_b, p->x_stride_l, p->y_stride_b, p->y_stride_l, p->dx_stride_b, p->dx_stride_l);
+        });
         int rc = check_launch("conv1d_bwd");
         if (rc) return rc;
         conv_reduce_partials_kernel<<<(unsigned)ceil_div(C * 5 * 4, (int64_t)256), 256, 0, st>>>(part, nslots, C, 4, p->dw, p->db, p->param_dtype);
+        return check_launch("conv1d_bwd_reduce");
+    }
+    if (channel_major_ok(p, true)) {
+        const int64_t pieces = ceil_div(l, (int64_t)(2 * VecTraits<T>::kVec)), total = nb * pieces;
+        // enough waves to fill the chip (about 24 per CU), each with at least one whole round of its lanes; never more
+        // splits than the partial rows that m2_conv1d_bwd_workspace_bytes sizes
+        int64_t splits = ceil_div((int64_t)24 * device_cus(), C);
+        if (splits > total / 64) splits = total / 64;
+        if (splits < 1) splits = 1;
+        const int64_t per_split = ceil_div(total, splits);
+        splits = ceil_div(total, per_split);
+        float* part = static_cast<float*>(p->workspace);
+        M2_REQUIRE(splits == 1 || (part && p->workspace_bytes >= (size_t)(splits * C * 5) * sizeof(float)), M2_ERR_WORKSPACE,
+                   "conv1d_bwd: workspace %zu bytes < %zu needed", p->workspace_bytes, (size_t)(splits * C * 5) * sizeof(float));
+        conv_dispatch(p, [&](auto wt, auto act) {
+            conv_bwd_cm_kernel<T, decltype(wt), decltype(act)::value><<<(unsigned)ceil_div(C * splits, (int64_t)4), 256, 0, st>>>(
+                x, p->w, p->bias, dy, dx, part, p->dw, p->db, l, (uint32_t)C, (uint32_t)splits, (uint32_t)pieces, (uint32_t)per_split,
+                (uint32_t)total, p->x_stride_b, p->x_stride_c, p->y_stride_b, p->y_stride_c, p->dx_stride_b, p->dx_stride_c);
+        });
+        int rc = check_launch("conv1d_bwd");
+        if (rc || splits == 1) return rc;
+        conv_reduce_partials_kernel<<<(unsigned)ceil_div(C * 5 * 4, (int64_t)256), 256, 0, st>>>(part, splits, C, 4, p->dw, p->db, p->param_dtype);
         return check_launch("conv1d_bwd_reduce");
     }
     const int64_t total = nb * l * C;
