@@ -1,4 +1,4 @@
-"""Build libmamba2_hip.so (gfx950) in-tree with hipcc.
+"""Build libmamba2_hip.so (gfx950) in-tree with hipcc, and the operators' host code (_native.so) with the C++ compiler.
 
     python state-space-models-neuron_amd/build.py [--force] [-j N]
 
@@ -9,12 +9,14 @@ import argparse
 import concurrent.futures as cf
 import os
 import subprocess
-import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "mamba2", "libmamba2_hip.so")
+NATIVE = os.path.join(HERE, "mamba2", "_native.so")
+NATIVE_SRC = os.path.join(CSRC, "binding.cpp")
 SOURCES = ["api.hip", "conv1d.hip", "decode.hip", "glue.hip", "ssd_fwd.hip", "ssd_bwd.hip"]
 FLAGS = ["-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
          "-Wno-unused-command-line-argument", "-Wno-inline-asm",
@@ -37,6 +39,15 @@ def _stale(target, deps):
     return any(os.path.getmtime(d) > t for d in deps)
 
 
+def _native_command():
+    """The C++ compiler's line for _native.so: host code only, against torch's headers and libraries."""
+    from torch.utils import cpp_extension
+    inc = [f"-I{d}" for d in cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]]]
+    libs = [f"-L{d}" for d in cpp_extension.library_paths("cuda")] + ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"]
+    return [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__",
+            "-DTORCH_EXTENSION_NAME=_native"] + inc + [NATIVE_SRC, "-o", NATIVE] + libs
+
+
 def build(force=False, jobs=None, verbose=True):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     os.makedirs(OBJ, exist_ok=True)
@@ -49,9 +60,12 @@ def build(force=False, jobs=None, verbose=True):
         obj = os.path.join(OBJ, s.replace(".hip", ".o"))
         if force or _stale(obj, [src] + headers):
             todo.append((src, obj))
-    jobs = jobs or min(8, max(1, len(todo)))
+    cmds = {src: [hipcc] + FLAGS + ["-c", src, "-o", obj] for src, obj in todo}
+    if force or _stale(NATIVE, [NATIVE_SRC, headers[-1]]):
+        cmds[NATIVE_SRC] = _native_command()
+    jobs = jobs or min(8, max(1, len(cmds)))
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
-        futs = {ex.submit(_run, [hipcc] + FLAGS + ["-c", src, "-o", obj]): src for src, obj in todo}
+        futs = {ex.submit(_run, cmd): src for src, cmd in cmds.items()}
         for f in cf.as_completed(futs):
             out = f.result()
             if verbose:

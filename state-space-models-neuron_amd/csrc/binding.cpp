@@ -1,0 +1,725 @@
+// The host path of the operators in C++: argument checks, output and scratch allocation, the parameter structs of the C ABI
+// and the autograd nodes.  Python only names the operators (mamba2/*.py).
+//
+// An eager call at the sizes of a short prompt or a decode step is bound by the host: the ctypes form of this code (attribute
+// access on ~40 struct fields, view and stream objects, one Python autograd node per operator) took 25-60 us per operator,
+// several times the kernels' own time.
+//
+// The library is not linked: its entry points come from the ctypes loader (bind()), so that both sides always use the
+// build that _lib.load() opened.  Scratch comes from the caching allocator per call: it is ordered by the stream it was
+// allocated on, so calls from several threads and streams never share it.
+#include <torch/extension.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/DeviceGuard.h>
+
+#include <initializer_list>
+#include <map>
+#include <string>
+
+#include "../../include/mamba2_hip.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// ----------------------------------------------------------------------------------------------- the library
+#define M2_BOUND(F) \
+    F(m2_last_error) F(m2_conv1d_fwd) F(m2_conv1d_bwd_workspace_bytes) F(m2_conv1d_bwd) F(m2_ssd_chunk_states_bytes) \
+    F(m2_ssd_fwd_workspace_bytes) F(m2_ssd_fwd) F(m2_ssd_bwd_workspace_bytes) F(m2_ssd_bwd) F(m2_decode_workspace_bytes) \
+    F(m2_decode_step) F(m2_decode_step_static) F(m2_rmsnorm_gated_fwd) F(m2_rmsnorm_gated_bwd_workspace_bytes) \
+    F(m2_rmsnorm_gated_bwd) F(m2_add_rmsnorm)
+struct Lib {
+#define M2_FIELD(name) decltype(&::name) name = nullptr;
+    M2_BOUND(M2_FIELD)
+#undef M2_FIELD
+} lib;
+
+std::vector<std::string> bound_names() {
+#define M2_NAME(name) #name,
+    return {M2_BOUND(M2_NAME)};
+#undef M2_NAME
+}
+
+void bind(const std::map<std::string, uintptr_t>& addresses) {
+#define M2_SET(name) lib.name = reinterpret_cast<decltype(lib.name)>(addresses.at(#name));
+    M2_BOUND(M2_SET)
+#undef M2_SET
+}
+
+void check(int rc, const char* what) {
+    if (rc == M2_OK) return;
+    const bool bad_argument = rc == M2_ERR_SHAPE || rc == M2_ERR_DTYPE || rc == M2_ERR_ALIGN || rc == M2_ERR_NULL;
+    TORCH_CHECK_VALUE(!bad_argument, what, ": ", lib.m2_last_error(), " (code ", rc, ")");
+    TORCH_CHECK(false, what, ": ", lib.m2_last_error(), " (code ", rc, ")");
+}
+
+// ----------------------------------------------------------------------------------------------- small helpers
+void require_gpu(std::initializer_list<const Tensor*> tensors) {
+    for (const Tensor* t : tensors)
+        TORCH_CHECK(!t || !t->defined() || t->is_cuda(), "mamba2 HIP kernels need tensors on a GPU device (got ",
+                    t ? t->device().str() : "", "); there is no CPU path");
+}
+
+int dtype_code(const Tensor& t) {
+    if (t.scalar_type() == at::kFloat) return M2_F32;
+    if (t.scalar_type() == at::kBFloat16) return M2_BF16;
+    TORCH_CHECK_VALUE(false, "unsupported dtype ", t.scalar_type(), ": the HIP kernels take float32 or bfloat16");
+}
+
+const Tensor& or_none(const OptTensor& t) {
+    static const Tensor none;
+    return t ? *t : none;
+}
+
+template <typename T = void> T* ptr(const Tensor& t) { return t.defined() ? static_cast<T*>(t.data_ptr()) : nullptr; }
+char* at_column(const Tensor& t, int64_t column) { return static_cast<char*>(t.data_ptr()) + column * t.element_size(); }
+
+// The body of an operator: autograd off, the tensors' device current, its stream at hand.
+struct Scope {
+    at::AutoDispatchBelowADInplaceOrView no_autograd;
+    c10::OptionalDeviceGuard guard;
+    void* stream;
+    explicit Scope(const Tensor& t) : guard(t.device()) {
+        stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
+    }
+};
+
+// fp32 contiguous values of a parameter-like tensor (the tensor itself when it already is)
+Tensor f32(const Tensor& t) { return t.defined() ? t.to(at::kFloat).contiguous() : t; }
+
+Tensor scratch(size_t bytes, const Tensor& like) {
+    return at::empty({static_cast<int64_t>(bytes)}, like.options().dtype(at::kByte));
+}
+Tensor empty_f32(at::IntArrayRef shape, const Tensor& like) { return at::empty(shape, like.options().dtype(at::kFloat)); }
+
+// ----------------------------------------------------------------------------------------------- conv1d
+struct Blc { int64_t b, l, c, sb, sl, sc; };
+Blc blc(const Tensor& t, bool channels_last) {
+    const int L = channels_last ? 1 : 2, C = channels_last ? 2 : 1;
+    return {t.size(0), t.size(L), t.size(C), t.stride(0), t.stride(L), t.stride(C)};
+}
+
+void check_conv(const Tensor& input, const Tensor& weight, const Tensor& bias, bool channels_last) {
+    TORCH_CHECK_VALUE(input.dim() == 3 && weight.dim() == 3 && weight.size(1) == 1, "expected input (B, C, L) or (B, L, C) and weight (C, 1, k)");
+    TORCH_CHECK_VALUE(!bias.defined() || (bias.dim() == 1 && bias.size(0) == weight.size(0) && bias.scalar_type() == weight.scalar_type()),
+                      "bias must have shape (C,) and the dtype of weight");
+    require_gpu({&input, &weight, &bias});
+    const int64_t channels = input.size(channels_last ? 2 : 1);
+    TORCH_CHECK_VALUE(weight.size(0) == channels, "weight has ", weight.size(0), " channels, input has ", channels);
+}
+
+// x, y / dy and dx are given as (pointer, strides): columns of packed buffers need no view objects
+struct Strided { void* p; int64_t sb, sl, sc; };
+m2_conv1d_params conv_params(const Strided& x, const Tensor& w, const Tensor& bias, const Strided& y, int64_t b, int64_t l, int64_t c,
+                             int dtype, int activation) {
+    m2_conv1d_params p{};
+    p.x = x.p; p.w = ptr(w); p.bias = ptr(bias);
+    p.batch = b; p.seqlen = l; p.channels = c; p.k = static_cast<int32_t>(w.size(-1));
+    p.x_stride_b = x.sb; p.x_stride_l = x.sl; p.x_stride_c = x.sc;
+    p.y_stride_b = y.sb; p.y_stride_l = y.sl; p.y_stride_c = y.sc;
+    p.dtype = dtype; p.param_dtype = dtype_code(w); p.activation = activation;
+    return p;
+}
+
+Tensor conv1d_forward(const Tensor& input, const Tensor& weight, const OptTensor& bias_, int64_t activation, bool channels_last, const OptTensor& out) {
+    const Tensor& bias = or_none(bias_);
+    check_conv(input, weight, bias, channels_last);
+    Scope scope(input);
+    const Tensor w = weight.contiguous(), bi = bias.defined() ? bias.contiguous() : bias;
+    Tensor y = out ? *out : at::empty(input.sizes(), input.options());
+    const Blc xi = blc(input, channels_last), yi = blc(y, channels_last);
+    m2_conv1d_params p = conv_params({ptr(input), xi.sb, xi.sl, xi.sc}, w, bi, {ptr(y), yi.sb, yi.sl, yi.sc}, xi.b, xi.l, xi.c,
+                                     dtype_code(input), static_cast<int>(activation));
+    p.y = ptr(y);
+    check(lib.m2_conv1d_fwd(&p, scope.stream), "m2_conv1d_fwd");
+    return y;
+}
+
+// the launch shared by the operator and the fused core; returns (dw, db)
+std::pair<Tensor, Tensor> launch_conv_bwd(const Strided& x, const Tensor& weight, const Tensor& bias, const Strided& dy, const Strided& dx,
+                                          int64_t b, int64_t l, int64_t c, const Tensor& like, int activation, void* stream) {
+    const Tensor w = weight.contiguous(), bi = bias.defined() ? bias.contiguous() : bias;
+    Tensor dw = at::empty(w.sizes(), w.options()), db = bi.defined() ? at::empty(bi.sizes(), bi.options()) : Tensor();
+    m2_conv1d_params p = conv_params(x, w, bi, dy, b, l, c, dtype_code(like), activation);
+    p.dy = dy.p; p.dx = dx.p; p.dw = ptr(dw); p.db = ptr(db);
+    p.dx_stride_b = dx.sb; p.dx_stride_l = dx.sl; p.dx_stride_c = dx.sc;
+    p.workspace_bytes = lib.m2_conv1d_bwd_workspace_bytes(b, l, c, p.k);
+    const Tensor ws = scratch(p.workspace_bytes, like);
+    p.workspace = ptr(ws);
+    check(lib.m2_conv1d_bwd(&p, stream), "m2_conv1d_bwd");
+    return {dw, db};
+}
+
+std::tuple<Tensor, Tensor, Tensor> conv1d_backward(const Tensor& input, const Tensor& weight, const OptTensor& bias_, const Tensor& d_output,
+                                                   int64_t activation, bool channels_last, const OptTensor& out_dx) {
+    const Tensor& bias = or_none(bias_);
+    check_conv(input, weight, bias, channels_last);
+    require_gpu({&d_output});
+    Scope scope(input);
+    const Tensor dy = d_output.to(input.scalar_type());
+    Tensor dx = out_dx ? *out_dx : at::empty(input.sizes(), input.options());
+    const Blc xi = blc(input, channels_last), gi = blc(dy, channels_last), di = blc(dx, channels_last);
+    auto [dw, db] = launch_conv_bwd({ptr(input), xi.sb, xi.sl, xi.sc}, weight, bias, {ptr(dy), gi.sb, gi.sl, gi.sc}, {ptr(dx), di.sb, di.sl, di.sc},
+                                    xi.b, xi.l, xi.c, input, static_cast<int>(activation), scope.stream);
+    return {dx, dw, db};
+}
+
+// conv1d_grouped.py:265-292: forward(input, weight, bias, activation), backward -> (dinput, dweight, dbias)
+struct ConvFn : torch::autograd::Function<ConvFn> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& input, const Tensor& weight, const OptTensor& bias, int64_t activation, bool channels_last) {
+        ctx->save_for_backward({input, weight, or_none(bias)});
+        ctx->saved_data["activation"] = activation;
+        ctx->saved_data["channels_last"] = channels_last;
+        return conv1d_forward(input, weight, bias, activation, channels_last, std::nullopt);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        auto [dx, dw, db] = conv1d_backward(s[0], s[1], s[2].defined() ? OptTensor(s[2]) : std::nullopt, grads[0],
+                                            ctx->saved_data["activation"].toInt(), ctx->saved_data["channels_last"].toBool(), std::nullopt);
+        return {dx, dw, db, Tensor(), Tensor()};
+    }
+};
+Tensor conv1d(const Tensor& input, const Tensor& weight, const OptTensor& bias, int64_t activation, bool channels_last) {
+    check_conv(input, weight, or_none(bias), channels_last);
+    return ConvFn::apply(input, weight, bias, activation, channels_last);
+}
+
+// ----------------------------------------------------------------------------------------------- SSD scan
+void check_inner(const char* name, const Tensor& t) {
+    TORCH_CHECK_VALUE(t.stride(-1) == 1 || t.size(-1) <= 1, name, ": innermost dimension must be contiguous (stride ", t.stride(-1), ")");
+}
+
+void check_ssd(const Tensor& dt, const Tensor& A, const Tensor& X, const Tensor& B, const Tensor& C, const Tensor& D, const Tensor& S0, const Tensor& dt_bias) {
+    TORCH_CHECK_VALUE(X.dim() == 4 && B.dim() == 4 && C.dim() == 4 && dt.dim() == 3, "expected dt (b,l,h), X (b,l,h,p), B/C (b,l,g,n)");
+    const int64_t b = X.size(0), l = X.size(1), h = X.size(2);
+    TORCH_CHECK_VALUE(dt.size(0) == b && dt.size(1) == l && dt.size(2) == h, "dt shape ", dt.sizes(), " != (", b, ", ", l, ", ", h, ")");
+    TORCH_CHECK_VALUE(B.sizes() == C.sizes() && B.size(0) == b && B.size(1) == l, "B ", B.sizes(), " / C ", C.sizes(), " do not match X ", X.sizes());
+    TORCH_CHECK_VALUE(h % B.size(2) == 0, "n_heads ", h, " not divisible by n_groups ", B.size(2));
+    TORCH_CHECK_VALUE(A.dim() == 1 && A.size(0) == h && (!D.defined() || (D.dim() == 1 && D.size(0) == h)), "A and D must have shape (n_heads,)");
+    TORCH_CHECK_VALUE(B.scalar_type() == X.scalar_type() && C.scalar_type() == X.scalar_type(), "X, B and C must share one dtype");
+    TORCH_CHECK_VALUE(dt.scalar_type() == X.scalar_type() || dt.scalar_type() == at::kFloat, "dt must be float32 or have the dtype of X");
+    check_inner("X", X); check_inner("B", B); check_inner("C", C); check_inner("dt", dt);
+    TORCH_CHECK_VALUE(!S0.defined() || (S0.dim() == 4 && S0.size(0) == b && S0.size(1) == h && S0.size(2) == X.size(3) && S0.size(3) == B.size(3)),
+                      "initial_state must have shape (b, h, p, n)");
+    TORCH_CHECK_VALUE(!dt_bias.defined() || (dt_bias.dim() == 1 && dt_bias.size(0) == h), "dt_bias must have shape (n_heads,)");
+    require_gpu({&dt, &A, &X, &B, &C, &D, &S0, &dt_bias});
+}
+
+// A, D, dt_bias: fp32 contiguous (or undefined)
+m2_ssd_params ssd_params(const Tensor& dt, const Tensor& A, const Tensor& X, const Tensor& B, const Tensor& C, const Tensor& D, const Tensor& dt_bias) {
+    m2_ssd_params p{};
+    p.x = ptr(X); p.dt = ptr(dt); p.A = ptr<float>(A); p.B = ptr(B); p.C = ptr(C); p.D = ptr<float>(D); p.dt_bias = ptr<float>(dt_bias);
+    p.batch = X.size(0); p.seqlen = X.size(1); p.nheads = X.size(2); p.headdim = X.size(3); p.dstate = B.size(3); p.ngroups = B.size(2);
+    p.x_stride_b = X.stride(0); p.x_stride_l = X.stride(1); p.x_stride_h = X.stride(2);
+    p.dt_stride_b = dt.stride(0); p.dt_stride_l = dt.stride(1);
+    p.B_stride_b = B.stride(0); p.B_stride_l = B.stride(1); p.B_stride_g = B.stride(2);
+    p.C_stride_b = C.stride(0); p.C_stride_l = C.stride(1); p.C_stride_g = C.stride(2);
+    p.dtype = dtype_code(X); p.dt_dtype = dtype_code(dt);
+    return p;
+}
+
+Tensor alloc_chunk_states(const Tensor& dt, const Tensor& A, const Tensor& X, const Tensor& B, const Tensor& C) {
+    const m2_ssd_params p = ssd_params(dt, A, X, B, C, Tensor(), Tensor());
+    return scratch(lib.m2_ssd_chunk_states_bytes(&p), X);
+}
+
+void* chunk_states_ptr(const m2_ssd_params& p, const Tensor& states) {
+    if (!states.defined()) return nullptr;
+    const size_t need = lib.m2_ssd_chunk_states_bytes(&p);
+    TORCH_CHECK_VALUE(states.is_contiguous() && static_cast<size_t>(states.numel() * states.element_size()) == need,
+                      "chunk_states must be a contiguous buffer of ", need, " bytes (see alloc_chunk_states)");
+    return ptr(states);
+}
+
+void launch_ssd_fwd(m2_ssd_params& p, const Tensor& like, void* stream) {
+    p.workspace_bytes = lib.m2_ssd_fwd_workspace_bytes(&p);
+    const Tensor ws = scratch(p.workspace_bytes, like);
+    p.workspace = ptr(ws);
+    check(lib.m2_ssd_fwd(&p, stream), "m2_ssd_fwd");
+}
+void launch_ssd_bwd(m2_ssd_params& p, const Tensor& like, void* stream) {
+    p.workspace_bytes = lib.m2_ssd_bwd_workspace_bytes(&p);
+    const Tensor ws = scratch(p.workspace_bytes, like);
+    p.workspace = ptr(ws);
+    check(lib.m2_ssd_bwd(&p, stream), "m2_ssd_bwd");
+}
+
+std::tuple<Tensor, Tensor> ssd_forward(const Tensor& dt, const Tensor& A, const Tensor& X, const Tensor& B, const Tensor& C, const OptTensor& D_,
+                                       const OptTensor& S0_, bool want_final_state, const OptTensor& states, const OptTensor& dt_bias_) {
+    check_ssd(dt, A, X, B, C, or_none(D_), or_none(S0_), or_none(dt_bias_));
+    Scope scope(X);
+    const Tensor A32 = f32(A), D32 = f32(or_none(D_)), S0 = f32(or_none(S0_)), bias = f32(or_none(dt_bias_));
+    Tensor Y = at::empty(X.sizes(), X.options());
+    Tensor S = want_final_state ? empty_f32({X.size(0), X.size(2), X.size(3), B.size(3)}, X) : Tensor();
+    m2_ssd_params p = ssd_params(dt, A32, X, B, C, D32, bias);
+    p.initial_state = ptr<float>(S0); p.final_state = ptr<float>(S); p.y = ptr(Y);
+    p.chunk_states = chunk_states_ptr(p, or_none(states));
+    p.y_stride_b = Y.stride(0); p.y_stride_l = Y.stride(1); p.y_stride_h = Y.stride(2);
+    launch_ssd_fwd(p, X, scope.stream);
+    return {Y, S};
+}
+
+struct SsdGrads { Tensor ddt, dA, dX, dB, dC, dD, dS0, d_bias; };
+SsdGrads ssd_backward_impl(const Tensor& dt, const Tensor& A, const Tensor& X, const Tensor& B, const Tensor& C, const Tensor& D, const Tensor& dY_,
+                           const Tensor& S0_, const Tensor& dSf_, bool want_dinitial, const Tensor& out_dX, const Tensor& out_dB,
+                           const Tensor& out_dC, const Tensor& states, const Tensor& dt_bias, const Tensor& out_ddt) {
+    check_ssd(dt, A, X, B, C, D, S0_, dt_bias);
+    require_gpu({&dY_, &dSf_});
+    Scope scope(X);
+    const int64_t b = X.size(0), l = X.size(1), h = X.size(2), hd = X.size(3), g = B.size(2), n = B.size(3);
+    const Tensor A32 = f32(A), D32 = f32(D), S0 = f32(S0_), dSf = f32(dSf_), bias = f32(dt_bias);
+    // rows of dy are read as 16-byte vectors where they lie
+    Tensor dY = dY_;
+    if (dY.scalar_type() != X.scalar_type()) dY = dY.to(X.scalar_type());
+    const int64_t es = dY.element_size();
+    if (dY.stride(-1) != 1 || (dY.stride(0) * es) % 16 || (dY.stride(1) * es) % 16 || (dY.stride(2) * es) % 16 ||
+        reinterpret_cast<uintptr_t>(dY.data_ptr()) % 16)
+        dY = dY.clone(at::MemoryFormat::Contiguous);
+    TORCH_CHECK_VALUE(!out_ddt.defined() || (out_ddt.sizes() == dt.sizes() && out_ddt.scalar_type() == dt.scalar_type() && out_ddt.stride(-1) == 1),
+                      "out_ddt must have the shape and dtype of dt, heads contiguous");
+    SsdGrads r;
+    r.ddt = out_ddt.defined() ? out_ddt : at::empty({b, l, h}, dt.options());
+    r.dX = out_dX.defined() ? out_dX : at::empty({b, l, h, hd}, X.options());
+    r.dB = out_dB.defined() ? out_dB : at::empty({b, l, g, n}, B.options());
+    r.dC = out_dC.defined() ? out_dC : at::empty({b, l, g, n}, C.options());
+    // the per-head gradients share one allocation
+    const Tensor heads = empty_f32({3, h}, X);
+    r.dA = heads.select(0, 0);
+    if (D.defined()) r.dD = heads.select(0, 1);
+    if (dt_bias.defined()) r.d_bias = heads.select(0, 2);
+    if (want_dinitial) r.dS0 = empty_f32({b, h, hd, n}, X);
+    m2_ssd_params p = ssd_params(dt, A32, X, B, C, D32, bias);
+    p.initial_state = ptr<float>(S0); p.dy = ptr(dY); p.d_final_state = ptr<float>(dSf);
+    p.chunk_states = chunk_states_ptr(p, states);
+    p.dx = ptr(r.dX); p.ddt = ptr(r.ddt); p.dA = ptr<float>(r.dA); p.dB = ptr(r.dB); p.dC = ptr(r.dC); p.dD = ptr<float>(r.dD);
+    p.d_initial_state = ptr<float>(r.dS0); p.d_dt_bias = ptr<float>(r.d_bias);
+    p.dy_stride_b = dY.stride(0); p.dy_stride_l = dY.stride(1); p.dy_stride_h = dY.stride(2);
+    p.dx_stride_b = r.dX.stride(0); p.dx_stride_l = r.dX.stride(1); p.dx_stride_h = r.dX.stride(2);
+    p.ddt_stride_b = r.ddt.stride(0); p.ddt_stride_l = r.ddt.stride(1);
+    p.dB_stride_b = r.dB.stride(0); p.dB_stride_l = r.dB.stride(1); p.dB_stride_g = r.dB.stride(2);
+    p.dC_stride_b = r.dC.stride(0); p.dC_stride_l = r.dC.stride(1); p.dC_stride_g = r.dC.stride(2);
+    launch_ssd_bwd(p, X, scope.stream);
+    return r;
+}
+
+py::object ssd_backward(const Tensor& dt, const Tensor& A, const Tensor& X, const Tensor& B, const Tensor& C, const OptTensor& D, const Tensor& dY,
+                        const OptTensor& S0, const OptTensor& dSf, bool want_dinitial, const OptTensor& out_dX, const OptTensor& out_dB,
+                        const OptTensor& out_dC, const OptTensor& states, const OptTensor& dt_bias, const OptTensor& out_ddt) {
+    const SsdGrads r = ssd_backward_impl(dt, A, X, B, C, or_none(D), dY, or_none(S0), or_none(dSf), want_dinitial, or_none(out_dX), or_none(out_dB),
+                                         or_none(out_dC), or_none(states), or_none(dt_bias), or_none(out_ddt));
+    if (dt_bias) return py::make_tuple(r.ddt, r.dA, r.dX, r.dB, r.dC, r.dD, r.dS0, r.d_bias);
+    return py::make_tuple(r.ddt, r.dA, r.dX, r.dB, r.dC, r.dD, r.dS0);
+}
+
+// mamba2_kernel.py:488-519: forward(dt, A, X, B, C, D) -> Y, backward -> (ddt, dA, dX, dB, dC, dD), with the initial and the
+// final state as extensions.  The chunk states are kept for the backward when one can follow.
+struct SsdFn : torch::autograd::Function<SsdFn> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& dt, const Tensor& A, const Tensor& X, const Tensor& B, const Tensor& C,
+                                 const OptTensor& D, const OptTensor& S0, bool return_final_state, bool keep_states) {
+        OptTensor states;
+        if (keep_states && X.numel() > 0) states = alloc_chunk_states(dt, A, X, B, C);
+        auto [Y, S] = ssd_forward(dt, A, X, B, C, D, S0, return_final_state, states, std::nullopt);
+        ctx->save_for_backward({dt, A, X, B, C, or_none(D), or_none(S0), or_none(states)});
+        ctx->set_materialize_grads(false);
+        if (return_final_state) return {Y, S};
+        return {Y};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const Tensor &dt = s[0], &A = s[1], &X = s[2], &D = s[5], &S0 = s[6];
+        const Tensor dSf = grads.size() > 1 ? grads[1] : Tensor();
+        variable_list out(9);
+        if (!grads[0].defined() && !dSf.defined()) return out;
+        const Tensor dY = grads[0].defined() ? grads[0] : at::zeros(X.sizes(), X.options());
+        const SsdGrads r = ssd_backward_impl(dt, A, X, s[3], s[4], D, dY, S0, dSf, S0.defined() && ctx->needs_input_grad(S0.defined() && D.defined() ? 6 : 5),
+                                             Tensor(), Tensor(), Tensor(), s[7], Tensor(), Tensor());
+        out[0] = r.ddt; out[1] = r.dA.to(A.scalar_type()); out[2] = r.dX; out[3] = r.dB; out[4] = r.dC;
+        if (D.defined()) out[5] = r.dD.to(D.scalar_type());
+        out[6] = r.dS0;
+        return out;
+    }
+};
+py::object mamba2_kernel(const Tensor& dt, const Tensor& A, const Tensor& X, const Tensor& B, const Tensor& C, const OptTensor& D, const OptTensor& S0,
+                         bool return_final_state, bool save_states) {
+    check_ssd(dt, A, X, B, C, or_none(D), or_none(S0), Tensor());
+    bool needs = false;
+    if (at::GradMode::is_enabled())
+        for (const Tensor* t : {&dt, &A, &X, &B, &C, &or_none(D), &or_none(S0)}) needs |= t->defined() && t->requires_grad();
+    const variable_list r = SsdFn::apply(dt, A, X, B, C, D, S0, return_final_state, save_states && needs);
+    if (return_final_state) return py::make_tuple(r[0], r[1]);
+    return py::cast(r[0]);
+}
+
+// ----------------------------------------------------------------------------------------------- gated RMSNorm
+// (rows, channels, row stride) of a (..., channels) tensor whose leading dimensions collapse to one stride
+struct Rows { int64_t rows, channels, stride; };
+Rows rows2d(const Tensor& t, const char* name) {
+    const int64_t ch = t.size(-1);
+    TORCH_CHECK_VALUE(t.stride(-1) == 1 || ch <= 1, name, ": innermost dimension must be contiguous");
+    if (t.dim() == 1) return {1, ch, ch};
+    const int64_t sr = t.stride(-2);
+    int64_t expect = sr;
+    for (int64_t k = t.dim() - 2; k >= 0; --k) {
+        TORCH_CHECK_VALUE(t.size(k) == 1 || t.stride(k) == expect, name, ": rows are not evenly strided (shape ", t.sizes(), ", strides ", t.strides(), ")");
+        expect *= t.size(k);
+    }
+    return {ch ? t.numel() / ch : 0, ch, sr};
+}
+// rows that can be read as 16-byte vectors where they lie; others are copied once
+bool vec_ok(const Tensor& t) {
+    const Rows r = rows2d(t, "tensor");
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && (r.stride * t.element_size()) % 16 == 0;
+}
+Tensor aligned(const Tensor& t) { return vec_ok(t) ? t : t.clone(at::MemoryFormat::Contiguous); }
+
+m2_rmsnorm_params norm_params(const Tensor& x, const Tensor& z, const Tensor& w32, int64_t n_groups, double eps) {
+    m2_rmsnorm_params p{};
+    const Rows xr = rows2d(x, "x");
+    p.x = ptr(x); p.x_stride_row = xr.stride;
+    if (z.defined()) { p.z = ptr(z); p.z_stride_row = rows2d(z, "z").stride; }
+    p.rows = xr.rows; p.channels = xr.channels; p.n_groups = static_cast<int32_t>(n_groups);
+    p.dtype = dtype_code(x); p.eps = static_cast<float>(eps); p.weight = ptr<float>(w32);
+    return p;
+}
+void check_norm(const Tensor& x, const Tensor& z) {
+    TORCH_CHECK_VALUE(!z.defined() || (z.sizes() == x.sizes() && z.scalar_type() == x.scalar_type()), "rmsnorm_gated: z must have the shape and dtype of x");
+}
+
+Tensor rmsnorm_forward(const Tensor& x_, const OptTensor& z_, const Tensor& weight, int64_t n_groups, double eps, at::ScalarType out_dtype) {
+    require_gpu({&x_, &or_none(z_), &weight});
+    check_norm(x_, or_none(z_));
+    TORCH_CHECK_VALUE(out_dtype == at::kFloat || out_dtype == x_.scalar_type(), "rmsnorm_gated: out_dtype must be float32 or the dtype of x");
+    Scope scope(x_);
+    const Tensor x = aligned(x_), z = z_ ? aligned(*z_) : Tensor(), w32 = f32(weight);
+    m2_rmsnorm_params p = norm_params(x, z, w32, n_groups, eps);
+    Tensor out = at::empty(x.sizes(), x.options().dtype(out_dtype));
+    p.out = ptr(out); p.out_stride_row = x.size(-1); p.out_f32 = out_dtype == at::kFloat;
+    check(lib.m2_rmsnorm_gated_fwd(&p, scope.stream), "m2_rmsnorm_gated_fwd");
+    return out;
+}
+
+std::tuple<Tensor, Tensor, Tensor> rmsnorm_backward(const Tensor& x_, const OptTensor& z_, const Tensor& weight, const Tensor& d_out, int64_t n_groups,
+                                                    double eps, const OptTensor& out_dz) {
+    require_gpu({&x_, &or_none(z_), &weight, &d_out});
+    check_norm(x_, or_none(z_));
+    Scope scope(x_);
+    Tensor g = d_out.to(x_.scalar_type());
+    if (g.stride(-1) != 1 || !vec_ok(g)) g = g.clone(at::MemoryFormat::Contiguous);
+    const Tensor x = aligned(x_), z = z_ ? aligned(*z_) : Tensor(), w32 = f32(weight);
+    m2_rmsnorm_params p = norm_params(x, z, w32, n_groups, eps);
+    p.d_out = ptr(g); p.d_out_stride_row = rows2d(g, "d_out").stride;
+    Tensor dx = at::empty(x.sizes(), x.options()), dz;
+    p.dx = ptr(dx); p.dx_stride_row = x.size(-1);
+    if (z.defined()) {
+        TORCH_CHECK_VALUE(!out_dz || (out_dz->scalar_type() == x.scalar_type() && out_dz->sizes() == x.sizes()),
+                          "rmsnorm_gated_bwd: out_dz must have the shape and dtype of x");
+        dz = out_dz && vec_ok(*out_dz) ? *out_dz : at::empty(x.sizes(), x.options());
+        p.dz = ptr(dz); p.dz_stride_row = rows2d(dz, "out_dz").stride;
+    }
+    Tensor dw = empty_f32({x.size(-1)}, x);
+    p.d_weight = ptr<float>(dw);
+    p.workspace_bytes = lib.m2_rmsnorm_gated_bwd_workspace_bytes(p.rows, p.channels, p.n_groups, p.dtype);
+    const Tensor ws = scratch(p.workspace_bytes, x);
+    p.workspace = ptr(ws);
+    check(lib.m2_rmsnorm_gated_bwd(&p, scope.stream), "m2_rmsnorm_gated_bwd");
+    if (z.defined() && out_dz && !dz.is_same(*out_dz)) {
+        out_dz->copy_(dz);
+        dz = *out_dz;
+    }
+    return {dx, dw, dz};
+}
+
+struct NormFn : torch::autograd::Function<NormFn> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const OptTensor& z, const Tensor& weight, int64_t n_groups, double eps, at::ScalarType out_dtype) {
+        ctx->save_for_backward({x, or_none(z), weight});
+        ctx->saved_data["n_groups"] = n_groups;
+        ctx->saved_data["eps"] = eps;
+        return rmsnorm_forward(x, z, weight, n_groups, eps, out_dtype);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        auto [dx, dw, dz] = rmsnorm_backward(s[0], s[1].defined() ? OptTensor(s[1]) : std::nullopt, s[2], grads[0], ctx->saved_data["n_groups"].toInt(),
+                                             ctx->saved_data["eps"].toDouble(), std::nullopt);
+        return {dx, dz, dw.to(s[2].scalar_type()), Tensor(), Tensor(), Tensor()};
+    }
+};
+Tensor rmsnorm(const Tensor& x, const OptTensor& z, const Tensor& weight, int64_t n_groups, double eps, at::ScalarType out_dtype) {
+    return NormFn::apply(x, z, weight, n_groups, eps, out_dtype);
+}
+
+Tensor add_rmsnorm(const Tensor& residual, const OptTensor& delta_, const Tensor& w32, double eps, at::ScalarType out_dtype) {
+    require_gpu({&residual, &or_none(delta_), &w32});
+    TORCH_CHECK_VALUE(residual.scalar_type() == at::kFloat && residual.is_contiguous(), "add_rmsnorm_: the residual stream must be contiguous float32");
+    Tensor delta = or_none(delta_);
+    TORCH_CHECK_VALUE(!delta.defined() || (delta.sizes() == residual.sizes() && delta.scalar_type() == out_dtype),
+                      "add_rmsnorm_: delta must have the residual's shape and the output dtype");
+    Scope scope(residual);
+    const Rows r = rows2d(residual, "residual");
+    if (delta.defined() && delta.stride(-1) != 1) delta = delta.contiguous();
+    Tensor out = at::empty(residual.sizes(), residual.options().dtype(out_dtype));
+    check(lib.m2_add_rmsnorm(ptr<float>(residual), r.stride, ptr(delta), delta.defined() ? rows2d(delta, "delta").stride : 0, ptr<float>(w32), ptr(out),
+                             r.channels, r.rows, r.channels, static_cast<float>(eps), dtype_code(out), scope.stream), "m2_add_rmsnorm");
+    return out;
+}
+
+// ----------------------------------------------------------------------------------------------- fused mixer core
+constexpr double kNormEps = 1e-5;      // fixed in the reference's fused kernel (fused_kernel.py:254)
+
+// [z | xBC | dt] columns of the packed projection output; the kernels read them where they lie
+struct Packed {
+    Tensor zx;
+    int64_t b, l, h, g, n, d, p, conv, sb, sl;
+    Packed(const Tensor& t, int64_t g_, int64_t n_, int64_t d_, int64_t p_) : g(g_), n(n_), d(d_), p(p_) {
+        TORCH_CHECK_VALUE(t.dim() == 3, "zxBCdt must be (b, l, width)");
+        h = d / p; conv = d + 2 * g * n;
+        TORCH_CHECK_VALUE(t.size(2) == d + conv + h, "zxBCdt width ", t.size(2), " != 2*d_inner + 2*g*n + h = ", d + conv + h);
+        const bool even = t.stride(2) == 1 && (t.size(0) <= 1 || t.stride(0) == t.size(1) * t.stride(1));
+        zx = even ? t : t.contiguous();
+        b = zx.size(0); l = zx.size(1); sb = zx.stride(0); sl = zx.stride(1);
+    }
+    Tensor z() const { return zx.narrow(2, 0, d); }
+    Tensor dt() const { return zx.narrow(2, d + conv, h); }
+    Strided xBC() const { return {at_column(zx, d), sb, sl, 1}; }
+};
+
+// the scan's parameters with x, B and C as columns of the packed conv output
+m2_ssd_params core_ssd_params(const Packed& k, const Tensor& conv_out, const Tensor& A, const Tensor& D, const Tensor& dt_bias) {
+    m2_ssd_params p{};
+    const int64_t sb = conv_out.stride(0), sl = conv_out.stride(1);
+    p.x = ptr(conv_out); p.B = at_column(conv_out, k.d); p.C = at_column(conv_out, k.d + k.g * k.n); p.dt = at_column(k.zx, k.d + k.conv);
+    p.A = ptr<float>(A); p.D = ptr<float>(D); p.dt_bias = ptr<float>(dt_bias);
+    p.batch = k.b; p.seqlen = k.l; p.nheads = k.h; p.headdim = k.p; p.dstate = k.n; p.ngroups = k.g;
+    p.x_stride_b = p.B_stride_b = p.C_stride_b = sb;
+    p.x_stride_l = p.B_stride_l = p.C_stride_l = sl;
+    p.x_stride_h = k.p; p.B_stride_g = p.C_stride_g = k.n;
+    p.dt_stride_b = k.sb; p.dt_stride_l = k.sl;
+    p.dtype = p.dt_dtype = dtype_code(conv_out);
+    return p;
+}
+
+void check_core(const Packed& k, const Tensor& A, const Tensor& D, const Tensor& conv_w, const Tensor& conv_b, const Tensor& dt_bias, const Tensor& norm_w) {
+    require_gpu({&k.zx, &A, &D, &conv_w, &conv_b, &dt_bias, &norm_w});
+    TORCH_CHECK_VALUE(k.g > 0 && k.h % k.g == 0, "n_heads ", k.h, " not divisible by n_groups ", k.g);
+    TORCH_CHECK_VALUE(A.dim() == 1 && A.size(0) == k.h && (!D.defined() || (D.dim() == 1 && D.size(0) == k.h)), "A and D must have shape (n_heads,)");
+    TORCH_CHECK_VALUE(dt_bias.dim() == 1 && dt_bias.size(0) == k.h, "dt_bias must have shape (n_heads,)");
+    TORCH_CHECK_VALUE(norm_w.dim() == 1 && norm_w.size(0) == k.d, "norm_weight must have shape (d_inner,)");
+    TORCH_CHECK_VALUE(conv_w.dim() == 3 && conv_w.size(0) == k.conv && conv_w.size(1) == 1, "conv1d_weight must be (", k.conv, ", 1, k)");
+    TORCH_CHECK_VALUE(!conv_b.defined() || (conv_b.dim() == 1 && conv_b.size(0) == k.conv && conv_b.scalar_type() == conv_w.scalar_type()),
+                      "bias must have shape (C,) and the dtype of weight");
+}
+
+struct CoreOut { Tensor norm_out, conv_out, scan_out, states; };
+// A, D, dt_bias fp32.  want_norm false: only what the backward needs (conv output, scan output, chunk states).
+CoreOut core_forward(const Packed& k, const Tensor& A, const Tensor& D, const Tensor& conv_w, const Tensor& conv_b, const Tensor& dt_bias,
+                     const Tensor& norm_w, bool keep_states, bool want_norm, void* stream) {
+    CoreOut r;
+    r.conv_out = at::empty({k.b, k.l, k.conv}, k.zx.options());
+    const Tensor w = conv_w.contiguous(), bi = conv_b.defined() ? conv_b.contiguous() : conv_b;
+    m2_conv1d_params c = conv_params(k.xBC(), w, bi, {ptr(r.conv_out), k.l * k.conv, k.conv, 1}, k.b, k.l, k.conv, dtype_code(k.zx), M2_ACT_SILU);
+    c.y = ptr(r.conv_out);
+    check(lib.m2_conv1d_fwd(&c, stream), "m2_conv1d_fwd");
+    m2_ssd_params p = core_ssd_params(k, r.conv_out, A, D, dt_bias);
+    if (keep_states && k.zx.numel() > 0) {
+        r.states = scratch(lib.m2_ssd_chunk_states_bytes(&p), k.zx);
+        p.chunk_states = ptr(r.states);
+    }
+    r.scan_out = at::empty({k.b, k.l, k.d}, k.zx.options());
+    p.y = ptr(r.scan_out); p.y_stride_b = k.l * k.d; p.y_stride_l = k.d; p.y_stride_h = k.p;
+    launch_ssd_fwd(p, k.zx, stream);
+    if (want_norm) r.norm_out = rmsnorm_forward(r.scan_out, k.z(), norm_w, k.g, kNormEps, k.zx.scalar_type());
+    return r;
+}
+
+struct CoreGrads { Tensor zx, A, D, conv_w, conv_b, dt_bias, norm_w; };
+// The packed gradient has rows of whole 128-byte cache lines (10576 columns of bf16 are 165.25 lines, and every wave-wide
+// access to a column slice of such a buffer straddles two lines in three rows out of four); its consumers take a leading
+// dimension.
+CoreGrads core_backward(const Packed& k, const Tensor& d_out, const Tensor& A, const Tensor& D, const Tensor& conv_w, const Tensor& conv_b,
+                        const Tensor& dt_bias, const Tensor& norm_w, const Tensor& conv_out, const Tensor& scan_out, const Tensor& states, void* stream) {
+    CoreGrads r;
+    const int64_t width = k.zx.size(2), per_line = 128 / k.zx.element_size(), pitch = (width + per_line - 1) / per_line * per_line;
+    r.zx = at::empty({k.b, k.l, pitch}, k.zx.options());
+    if (pitch != width) r.zx = r.zx.narrow(2, 0, width);
+    auto [d_scan, d_norm_w, dz] = rmsnorm_backward(scan_out, k.z(), norm_w, d_out, k.g, kNormEps, r.zx.narrow(2, 0, k.d));
+    r.norm_w = d_norm_w;
+    // the scan's gradients leave as one packed [dx | dB | dC] buffer, that of the raw dt in its columns of r.zx
+    const Tensor d_conv = at::empty({k.b, k.l, k.conv}, k.zx.options());
+    m2_ssd_params p = core_ssd_params(k, conv_out, A, D, dt_bias);
+    p.chunk_states = chunk_states_ptr(p, states);
+    p.dy = ptr(d_scan); p.dy_stride_b = k.l * k.d; p.dy_stride_l = k.d; p.dy_stride_h = k.p;
+    p.dx = ptr(d_conv); p.dB = at_column(d_conv, k.d); p.dC = at_column(d_conv, k.d + k.g * k.n);
+    p.dx_stride_b = p.dB_stride_b = p.dC_stride_b = k.l * k.conv;
+    p.dx_stride_l = p.dB_stride_l = p.dC_stride_l = k.conv;
+    p.dx_stride_h = k.p; p.dB_stride_g = p.dC_stride_g = k.n;
+    p.ddt = at_column(r.zx, k.d + k.conv); p.ddt_stride_b = r.zx.stride(0); p.ddt_stride_l = r.zx.stride(1);
+    const Tensor heads = empty_f32({3, k.h}, k.zx);
+    r.A = heads.select(0, 0); r.dt_bias = heads.select(0, 1);
+    if (D.defined()) r.D = heads.select(0, 2);
+    p.dA = ptr<float>(r.A); p.dD = ptr<float>(r.D); p.d_dt_bias = ptr<float>(r.dt_bias);
+    launch_ssd_bwd(p, k.zx, stream);
+    std::tie(r.conv_w, r.conv_b) = launch_conv_bwd(k.xBC(), conv_w, conv_b, {ptr(d_conv), k.l * k.conv, k.conv, 1},
+                                                   {at_column(r.zx, k.d), r.zx.stride(0), r.zx.stride(1), 1}, k.b, k.l, k.conv, k.zx, M2_ACT_SILU, stream);
+    return r;
+}
+
+py::tuple forward_parts(const Tensor& zx, const Tensor& A, const OptTensor& D, const Tensor& conv_w, const OptTensor& conv_b, const Tensor& dt_bias,
+                        const Tensor& norm_w, int64_t g, int64_t n, int64_t d, int64_t hd, bool keep_states) {
+    Scope scope(zx);
+    const Packed k(zx, g, n, d, hd);
+    check_core(k, A, or_none(D), conv_w, or_none(conv_b), dt_bias, norm_w);
+    const CoreOut r = core_forward(k, f32(A), f32(or_none(D)), conv_w, or_none(conv_b), f32(dt_bias), norm_w, keep_states, true, scope.stream);
+    return py::make_tuple(r.norm_out, r.conv_out, r.scan_out, r.states);
+}
+py::tuple backward_parts(const Tensor& d_out, const Tensor& zx, const Tensor& A, const OptTensor& D, const Tensor& conv_w, const OptTensor& conv_b,
+                         const Tensor& dt_bias, const Tensor& norm_w, const Tensor& conv_out, const Tensor& scan_out, const OptTensor& states,
+                         int64_t g, int64_t n, int64_t d, int64_t hd) {
+    Scope scope(zx);
+    const Packed k(zx, g, n, d, hd);
+    check_core(k, A, or_none(D), conv_w, or_none(conv_b), dt_bias, norm_w);
+    const CoreGrads r = core_backward(k, d_out, f32(A), f32(or_none(D)), conv_w, or_none(conv_b), f32(dt_bias), norm_w, conv_out, scan_out,
+                                      or_none(states), scope.stream);
+    return py::make_tuple(r.zx, r.A.to(A.scalar_type()), D ? r.D.to(D->scalar_type()) : Tensor(), r.conv_w, r.conv_b, r.dt_bias.to(dt_bias.scalar_type()),
+                          r.norm_w.to(norm_w.scalar_type()));
+}
+
+// fused_kernel.py:423-487.  caching: the conv output, scan output and chunk states are kept; otherwise only the inputs are,
+// and the backward recomputes those three (not the norm, which it does not need).
+struct CoreFn : torch::autograd::Function<CoreFn> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& zx, const Tensor& A, const OptTensor& D, const Tensor& conv_w, const OptTensor& conv_b,
+                          const Tensor& dt_bias, const Tensor& norm_w, int64_t g, int64_t n, int64_t d, int64_t hd, bool keep) {
+        Scope scope(zx);
+        const Packed k(zx, g, n, d, hd);
+        check_core(k, A, or_none(D), conv_w, or_none(conv_b), dt_bias, norm_w);
+        const CoreOut r = core_forward(k, f32(A), f32(or_none(D)), conv_w, or_none(conv_b), f32(dt_bias), norm_w, keep, true, scope.stream);
+        variable_list saved = {zx, A, or_none(D), conv_w, or_none(conv_b), dt_bias, norm_w};
+        if (keep) { saved.push_back(r.conv_out); saved.push_back(r.scan_out); saved.push_back(r.states); }
+        ctx->save_for_backward(std::move(saved));
+        ctx->saved_data["dims"] = std::vector<int64_t>{g, n, d, hd};
+        return r.norm_out;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const std::vector<int64_t> dims = ctx->saved_data["dims"].toIntVector();
+        Scope scope(s[0]);
+        const Packed k(s[0], dims[0], dims[1], dims[2], dims[3]);
+        const Tensor A = f32(s[1]), D = f32(s[2]), dt_bias = f32(s[5]), norm_w = f32(s[6]);
+        CoreOut f;
+        if (s.size() > 7) { f.conv_out = s[7]; f.scan_out = s[8]; f.states = s[9]; }
+        else f = core_forward(k, A, D, s[3], s[4], dt_bias, norm_w, true, false, scope.stream);
+        const CoreGrads r = core_backward(k, grads[0], A, D, s[3], s[4], dt_bias, norm_w, f.conv_out, f.scan_out, f.states, scope.stream);
+        variable_list out(12);
+        out[0] = r.zx; out[1] = r.A.to(s[1].scalar_type());
+        if (s[2].defined()) out[2] = r.D.to(s[2].scalar_type());
+        out[3] = r.conv_w; out[4] = r.conv_b; out[5] = r.dt_bias.to(s[5].scalar_type()); out[6] = r.norm_w.to(s[6].scalar_type());
+        return out;
+    }
+};
+Tensor fused_core(const Tensor& zx, const Tensor& A, const OptTensor& D, const Tensor& conv_w, const OptTensor& conv_b, const Tensor& dt_bias,
+                  const Tensor& norm_w, int64_t g, int64_t n, int64_t d, int64_t hd, bool caching) {
+    require_gpu({&zx});
+    bool keep = caching && at::GradMode::is_enabled();
+    return CoreFn::apply(zx, A, D, conv_w, conv_b, dt_bias, norm_w, g, n, d, hd, keep);
+}
+
+// Inference forward that hands the sequence over to the decode step: final SSM state and last W conv inputs into the cache.
+Tensor fused_prefill(const Tensor& zx, const Tensor& A, const OptTensor& D, const Tensor& conv_w, const OptTensor& conv_b_, const Tensor& dt_bias,
+                     const Tensor& norm_w, int64_t g, int64_t n, int64_t d, int64_t hd, const Tensor& conv_state, const Tensor& ssm_state, bool continuing) {
+    require_gpu({&zx, &conv_state, &ssm_state});
+    Scope scope(zx);
+    const Packed k(zx, g, n, d, hd);
+    const Tensor& conv_b = or_none(conv_b_);
+    check_core(k, A, or_none(D), conv_w, conv_b, dt_bias, norm_w);
+    const int64_t taps = conv_w.size(2);
+    TORCH_CHECK_VALUE(conv_state.dim() == 3 && conv_state.size(0) == k.b && conv_state.size(1) == k.conv && conv_state.size(2) >= taps - 1,
+                      "conv_state must be (b, conv_dim, W >= k-1), got ", conv_state.sizes());
+    TORCH_CHECK_VALUE(ssm_state.dim() == 4 && ssm_state.size(0) == k.b && ssm_state.size(1) == k.h && ssm_state.size(2) == hd && ssm_state.size(3) == n &&
+                          ssm_state.scalar_type() == at::kFloat, "ssm_state must be (b, h, p, n) float32");
+    if (k.l == 0) return at::empty({k.b, 0, d}, zx.options());
+    const int64_t W = conv_state.size(2);
+    const Tensor xBC = k.zx.narrow(2, d, k.conv);
+    Tensor conv_out, tail;
+    if (continuing) {
+        // the cached inputs go in front of the new ones; the outputs for them are dropped
+        const Tensor hist = at::cat({conv_state.transpose(1, 2).to(xBC.scalar_type()), xBC}, 1);
+        conv_out = conv1d_forward(hist, conv_w, conv_b_, M2_ACT_SILU, true, std::nullopt).narrow(1, W, k.l);
+        tail = hist.narrow(1, k.l, W);
+    } else {
+        conv_out = conv1d_forward(xBC, conv_w, conv_b_, M2_ACT_SILU, true, std::nullopt);
+        tail = k.l >= W ? xBC.narrow(1, k.l - W, W) : at::cat({at::zeros({k.b, W - k.l, k.conv}, xBC.options()), xBC}, 1);
+    }
+    const Tensor A32 = f32(A), D32 = f32(or_none(D)), bias = f32(dt_bias);
+    m2_ssd_params p = core_ssd_params(k, conv_out, A32, D32, bias);
+    const Tensor y = at::empty({k.b, k.l, d}, zx.options()), S = at::empty_like(ssm_state, at::MemoryFormat::Contiguous);
+    const Tensor S0 = continuing ? ssm_state.contiguous() : Tensor();
+    p.initial_state = ptr<float>(S0); p.final_state = ptr<float>(S);
+    p.y = ptr(y); p.y_stride_b = k.l * d; p.y_stride_l = d; p.y_stride_h = hd;
+    launch_ssd_fwd(p, zx, scope.stream);
+    ssm_state.copy_(S);
+    conv_state.copy_(tail.transpose(1, 2));
+    return rmsnorm_forward(y, k.z(), norm_w, g, kNormEps, zx.scalar_type());
+}
+
+// ----------------------------------------------------------------------------------------------- decode step
+std::tuple<Tensor, Tensor, Tensor> decode_step(const Tensor& xBC, const Tensor& conv_state, const Tensor& conv_w, const OptTensor& conv_b_, const Tensor& S,
+                                               const Tensor& dt, const Tensor& A_, const OptTensor& D_, int64_t g, int64_t activation,
+                                               const OptTensor& dt_bias_, const OptTensor& out, bool static_scratch) {
+    const Tensor &conv_b = or_none(conv_b_), &dt_bias = or_none(dt_bias_);
+    TORCH_CHECK_VALUE(S.dim() == 4 && xBC.dim() == 3 && conv_state.dim() == 3 && dt.dim() == 3, "expected xBC (b,1,Cx), conv_state (b,Cx,W), S (b,h,p,n), dt (b,1,h)");
+    const int64_t b = S.size(0), h = S.size(1), p_ = S.size(2), n = S.size(3), d = h * p_, cx = xBC.size(2);
+    TORCH_CHECK_VALUE(S.scalar_type() == at::kFloat, "the SSM state must be float32");
+    TORCH_CHECK_VALUE(conv_state.scalar_type() == xBC.scalar_type() && dt.scalar_type() == xBC.scalar_type(), "xBC, conv_state and dt must share one dtype");
+    TORCH_CHECK_VALUE(S.is_contiguous() && conv_state.is_contiguous(), "S and conv_state must be contiguous (they are updated in place)");
+    TORCH_CHECK_VALUE(xBC.stride(2) == 1 && dt.stride(2) == 1, "xBC and dt must be contiguous in their last dimension");
+    require_gpu({&xBC, &conv_state, &conv_w, &conv_b, &S, &dt, &A_, &or_none(D_), &dt_bias});
+    TORCH_CHECK_VALUE(!dt_bias.defined() || (dt_bias.dim() == 1 && dt_bias.size(0) == h), "dt_bias must have shape (n_heads,)");
+    TORCH_CHECK_VALUE(!out || (out->dim() == 3 && out->size(0) == b && out->size(1) == 1 && out->size(2) == d && out->scalar_type() == xBC.scalar_type() &&
+                               out->stride(2) == 1 && out->device() == xBC.device()),
+                      "out must be (batch, 1, n_heads * d_head) in the dtype of xBC, on its device");
+    Scope scope(xBC);
+    const Tensor w = conv_w.contiguous(), bi = conv_b.defined() ? conv_b.contiguous() : conv_b;
+    const Tensor A = f32(A_), D = f32(or_none(D_)), bias = f32(dt_bias);
+    Tensor Y = out ? *out : at::empty({b, 1, d}, xBC.options());
+    m2_decode_params p{};
+    p.xBC = ptr(xBC); p.conv_state = ptr(conv_state); p.conv_w = ptr(w); p.conv_b = ptr(bi);
+    p.S = ptr<float>(S); p.dt = ptr(dt); p.A = ptr<float>(A); p.D = ptr<float>(D); p.y = ptr(Y); p.dt_bias = ptr<float>(bias);
+    p.batch = b; p.nheads = h; p.headdim = p_; p.dstate = n; p.ngroups = g;
+    p.k = static_cast<int32_t>(w.size(-1)); p.W = static_cast<int32_t>(conv_state.size(2));
+    TORCH_CHECK_VALUE(w.numel() == cx * p.k && conv_state.size(0) == b && conv_state.size(1) == cx, "conv weight and state must have ", cx, " channels");
+    p.xBC_stride_b = xBC.stride(0); p.dt_stride_b = dt.stride(0); p.y_stride_b = Y.stride(0);
+    p.dtype = dtype_code(xBC); p.param_dtype = dtype_code(w); p.activation = static_cast<int32_t>(activation);
+    if (static_scratch) {
+        check(lib.m2_decode_step_static(&p, scope.stream), "m2_decode_step_static");
+    } else {
+        p.workspace_bytes = lib.m2_decode_workspace_bytes(b, h, p_, n, g);
+        const Tensor ws = scratch(p.workspace_bytes, xBC);
+        p.workspace = ptr(ws);
+        check(lib.m2_decode_step(&p, scope.stream), "m2_decode_step");
+    }
+    return {Y, conv_state, S};
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    m.def("bound_names", &bound_names);
+    m.def("bind", &bind);
+    m.def("conv1d_forward", &conv1d_forward);
+    m.def("conv1d_backward", &conv1d_backward);
+    m.def("conv1d", &conv1d);
+    m.def("alloc_chunk_states", &alloc_chunk_states);
+    m.def("ssd_forward", &ssd_forward);
+    m.def("ssd_backward", &ssd_backward);
+    m.def("mamba2_kernel", &mamba2_kernel);
+    m.def("rmsnorm_forward", &rmsnorm_forward);
+    m.def("rmsnorm_backward", &rmsnorm_backward);
+    m.def("rmsnorm", &rmsnorm);
+    m.def("add_rmsnorm", &add_rmsnorm);
+    m.def("forward_parts", &forward_parts);
+    m.def("backward_parts", &backward_parts);
+    m.def("fused_core", &fused_core);
+    m.def("fused_prefill", &fused_prefill);
+    m.def("decode_step", &decode_step);
+}

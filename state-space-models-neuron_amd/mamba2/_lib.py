@@ -1,7 +1,8 @@
-"""ctypes binding of libmamba2_hip.so (the C ABI declared in include/mamba2_hip.h).
+"""ctypes binding of libmamba2_hip.so (the C ABI declared in include/mamba2_hip.h) and the loader of the operators' host code.
 
 The structures below mirror the C structs field for field.  ``load()`` raises if
-the library is missing: there is no CPU or PyTorch fallback in this package.
+the library is missing: there is no CPU or PyTorch fallback in this package.  ``native()`` is the C++ module behind the
+operators (csrc/binding.cpp), bound to the library that ``load()`` opened.
 """
 import ctypes as C
 import weakref
@@ -98,6 +99,7 @@ SYMBOLS = {
 }
 
 _lib = None
+_native = None
 
 
 def load(path=None):
@@ -120,6 +122,21 @@ def load(path=None):
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+def native():
+    """The C++ host code of the operators (``mamba2/_native.so``), its entry points bound to the loaded library."""
+    global _native
+    if _native is None:
+        lib = load()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise RuntimeError("mamba2/_native.so is missing or does not load: build it with "
+                               f"`python state-space-models-neuron_amd/build.py` (there is no fallback path): {e}") from e
+        module.bind({name: C.cast(getattr(lib, name), C.c_void_p).value for name in module.bound_names()})
+        _native = module
+    return _native
 
 
 def check(rc, what):
