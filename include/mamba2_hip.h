@@ -239,6 +239,18 @@ int m2_add_rmsnorm(float* residual, int64_t residual_stride_row, const void* del
                    const float* weight, void* out, int64_t out_stride_row, int64_t rows, int64_t channels, float eps,
                    int32_t dtype, void* stream);
 
+/* The small parameters of a mixer layer as the kernels take them, and their gradients back, in one launch each
+ * (mamba2/mamba2_mixer.py:225-236: A = -exp(A_log.float()) and the casts around it).
+ * m2_mixer_params:       out (3 * nheads + channels) fp32 = [ -exp(A_log) | D | dt_bias | norm_weight ].
+ * m2_mixer_params_grads: dA, dD, d_dt_bias (nheads) and d_norm_weight (channels) fp32 into the parameters' own types;
+ *                        the gradient of A_log is dA * A with A the first nheads values of m2_mixer_params' out.
+ * D may be NULL (then so is its gradient, and out's second part is unset).  *_dtype: M2_F32 or M2_BF16. */
+int m2_mixer_params(const void* A_log, int32_t A_dtype, const void* D, int32_t D_dtype, const void* dt_bias, int32_t dt_bias_dtype,
+                    const void* norm_weight, int32_t norm_dtype, float* out, int64_t nheads, int64_t channels, void* stream);
+int m2_mixer_params_grads(const float* A, const float* dA, const float* dD, const float* d_dt_bias, const float* d_norm_weight,
+                          void* dA_log, int32_t A_dtype, void* dD_out, int32_t D_dtype, void* d_dt_bias_out, int32_t dt_bias_dtype,
+                          void* d_norm_out, int32_t norm_dtype, int64_t nheads, int64_t channels, void* stream);
+
 /* ------------------------------------------------------------------ self tests / probes
  * m2_mfma_selftest: C (M x N fp32, row-major) = A (M x K) * Bt (N x K)^T through the same
  * LDS-staged MFMA tile code the SSD kernels use.  M, N multiples of 128; K multiple of 32.

@@ -30,7 +30,7 @@ using torch::autograd::variable_list;
     F(m2_last_error) F(m2_conv1d_fwd) F(m2_conv1d_bwd_workspace_bytes) F(m2_conv1d_bwd) F(m2_ssd_chunk_states_bytes) \
     F(m2_ssd_fwd_workspace_bytes) F(m2_ssd_fwd) F(m2_ssd_bwd_workspace_bytes) F(m2_ssd_bwd) F(m2_decode_workspace_bytes) \
     F(m2_decode_step) F(m2_decode_step_static) F(m2_rmsnorm_gated_fwd) F(m2_rmsnorm_gated_bwd_workspace_bytes) \
-    F(m2_rmsnorm_gated_bwd) F(m2_add_rmsnorm)
+    F(m2_rmsnorm_gated_bwd) F(m2_add_rmsnorm) F(m2_mixer_params) F(m2_mixer_params_grads)
 struct Lib {
 #define M2_FIELD(name) decltype(&::name) name = nullptr;
     M2_BOUND(M2_FIELD)
@@ -624,6 +624,81 @@ Tensor fused_core(const Tensor& zx, const Tensor& A, const OptTensor& D, const T
     return CoreFn::apply(zx, A, D, conv_w, conv_b, dt_bias, norm_w, g, n, d, hd, keep);
 }
 
+// ----------------------------------------------------------------------------------------------- whole mixer layer
+// mamba2_mixer.py:213-240: in_proj -> core -> out_proj as one node, the plain products by the library that torch uses, the
+// small parameters cast (and A = -exp(A_log) formed) by one kernel and their gradients cast back by one.
+Tensor project(const Tensor& x, const Tensor& w, const Tensor& bias) {
+    return bias.defined() ? at::addmm(bias, x, w.t()) : at::mm(x, w.t());
+}
+
+struct MixerFn : torch::autograd::Function<MixerFn> {
+    enum { kHidden, kInW, kALog, kD, kDtBias, kConvW, kNormW, kOutW, kConvB, kInB, kOutB, kSmall, kZx, kNormOut, kConvOut, kScanOut, kStates };
+    static Tensor forward(AutogradContext* ctx, const Tensor& hidden, const Tensor& in_w, const Tensor& A_log, const Tensor& D, const Tensor& dt_bias,
+                          const Tensor& conv_w, const Tensor& norm_w, const Tensor& out_w, const OptTensor& conv_b, const OptTensor& in_b,
+                          const OptTensor& out_b, int64_t g, int64_t n, int64_t d, int64_t hd, bool differentiable, bool recompute) {
+        Scope scope(hidden);
+        const int64_t b = hidden.size(0), l = hidden.size(1), h = d / hd;
+        const Tensor x = hidden.reshape({b * l, hidden.size(2)});
+        const Tensor zx = project(x, in_w, or_none(in_b)).view({b, l, in_w.size(0)});
+        const Packed k(zx, g, n, d, hd);
+        check_core(k, A_log, D, conv_w, or_none(conv_b), dt_bias, norm_w);
+        const Tensor small = empty_f32({3 * h + d}, zx);
+        const Tensor a = A_log.contiguous(), dd = D.contiguous(), tb = dt_bias.contiguous(), nw = norm_w.contiguous();
+        check(lib.m2_mixer_params(ptr(a), dtype_code(a), ptr(dd), dtype_code(dd), ptr(tb), dtype_code(tb), ptr(nw), dtype_code(nw), ptr<float>(small),
+                                  h, d, scope.stream), "m2_mixer_params");
+        const CoreOut r = core_forward(k, small.narrow(0, 0, h), small.narrow(0, h, h), conv_w, or_none(conv_b), small.narrow(0, 2 * h, h),
+                                       small.narrow(0, 3 * h, d), differentiable && !recompute, true, scope.stream);
+        const Tensor y = r.norm_out.view({b * l, d});
+        if (differentiable) {
+            variable_list saved = {hidden, in_w, A_log, D, dt_bias, conv_w, norm_w, out_w, or_none(conv_b), or_none(in_b), or_none(out_b), small, zx, y};
+            if (!recompute) { saved.push_back(r.conv_out); saved.push_back(r.scan_out); saved.push_back(r.states); }
+            ctx->save_for_backward(std::move(saved));
+            ctx->saved_data["dims"] = std::vector<int64_t>{g, n, d, hd};
+        }
+        return project(y, out_w, or_none(out_b)).view({b, l, out_w.size(0)});
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const std::vector<int64_t> dims = ctx->saved_data["dims"].toIntVector();
+        const Tensor& zx = s[kZx];
+        Scope scope(zx);
+        const Packed k(zx, dims[0], dims[1], dims[2], dims[3]);
+        const int64_t rows = k.b * k.l;
+        const Tensor& small = s[kSmall];
+        const Tensor A = small.narrow(0, 0, k.h), D = small.narrow(0, k.h, k.h), dt_bias = small.narrow(0, 2 * k.h, k.h), norm_w = small.narrow(0, 3 * k.h, k.d);
+        variable_list out(17);
+        const Tensor dy = grads[0].reshape({rows, s[kOutW].size(0)});
+        if (ctx->needs_input_grad(kOutW)) out[kOutW] = at::mm(dy.t(), s[kNormOut]);
+        if (s[kOutB].defined()) out[kOutB] = dy.sum(0);
+        const Tensor d_core = at::mm(dy, s[kOutW]).view({k.b, k.l, k.d});
+        CoreOut f;
+        if (s.size() > kConvOut) { f.conv_out = s[kConvOut]; f.scan_out = s[kScanOut]; f.states = s[kStates]; }
+        else f = core_forward(k, A, D, s[kConvW], s[kConvB], dt_bias, norm_w, true, false, scope.stream);
+        const CoreGrads r = core_backward(k, d_core, A, D, s[kConvW], s[kConvB], dt_bias, norm_w, f.conv_out, f.scan_out, f.states, scope.stream);
+        for (const int i : {kALog, kD, kDtBias, kNormW}) out[i] = at::empty(s[i].sizes(), s[i].options());
+        check(lib.m2_mixer_params_grads(ptr<float>(A), ptr<float>(r.A), ptr<float>(r.D), ptr<float>(r.dt_bias), ptr<float>(r.norm_w), ptr(out[kALog]),
+                                        dtype_code(s[kALog]), ptr(out[kD]), dtype_code(s[kD]), ptr(out[kDtBias]), dtype_code(s[kDtBias]), ptr(out[kNormW]),
+                                        dtype_code(s[kNormW]), k.h, k.d, scope.stream), "m2_mixer_params_grads");
+        out[kConvW] = r.conv_w; out[kConvB] = r.conv_b;
+        const Tensor d_zx = r.zx.view({rows, zx.size(2)});
+        if (ctx->needs_input_grad(kHidden)) out[kHidden] = at::mm(d_zx, s[kInW]).view(s[kHidden].sizes());
+        if (ctx->needs_input_grad(kInW)) out[kInW] = at::mm(d_zx.t(), s[kHidden].reshape({rows, s[kHidden].size(2)}));
+        if (s[kInB].defined()) out[kInB] = d_zx.sum(0);
+        return out;
+    }
+};
+Tensor mixer(const Tensor& hidden, const Tensor& in_w, const Tensor& A_log, const Tensor& D, const Tensor& dt_bias, const Tensor& conv_w, const Tensor& norm_w,
+             const Tensor& out_w, const OptTensor& conv_b, const OptTensor& in_b, const OptTensor& out_b, int64_t g, int64_t n, int64_t d, int64_t hd,
+             bool recompute) {
+    require_gpu({&hidden, &in_w, &out_w});
+    TORCH_CHECK_VALUE(hidden.dim() == 3, "hidden_states must be (batch, seqlen, hidden_size)");
+    bool differentiable = false;
+    if (at::GradMode::is_enabled())
+        for (const Tensor* t : {&hidden, &in_w, &A_log, &D, &dt_bias, &conv_w, &norm_w, &out_w, &or_none(conv_b), &or_none(in_b), &or_none(out_b)})
+            differentiable |= t->defined() && t->requires_grad();
+    return MixerFn::apply(hidden, in_w, A_log, D, dt_bias, conv_w, norm_w, out_w, conv_b, in_b, out_b, g, n, d, hd, differentiable, recompute);
+}
+
 // Inference forward that hands the sequence over to the decode step: final SSM state and last W conv inputs into the cache.
 Tensor fused_prefill(const Tensor& zx, const Tensor& A, const OptTensor& D, const Tensor& conv_w, const OptTensor& conv_b_, const Tensor& dt_bias,
                      const Tensor& norm_w, int64_t g, int64_t n, int64_t d, int64_t hd, const Tensor& conv_state, const Tensor& ssm_state, bool continuing) {
@@ -720,6 +795,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("forward_parts", &forward_parts);
     m.def("backward_parts", &backward_parts);
     m.def("fused_core", &fused_core);
+    m.def("mixer", &mixer);
     m.def("fused_prefill", &fused_prefill);
     m.def("decode_step", &decode_step);
 }

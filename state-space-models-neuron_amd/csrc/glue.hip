@@ -12,6 +12,8 @@
 // 8192), its channels in registers as 16-byte vectors; a workgroup walks a block of rows, so the per-channel weight
 // and -- in the backward -- the dw accumulators stay in registers across rows.  dw and d_bias leave as per-block
 // partials in a caller-owned workspace and are summed in a fixed order by a second small kernel (no atomics).
+#include <initializer_list>
+
 #include "common.hpp"
 
 namespace m2 {
@@ -420,6 +422,38 @@ add_rmsnorm_kernel(float* __restrict__ res, int64_t res_sr, const T* __restrict_
     }
 }
 
+// Parameter casts of a mixer layer: a few thousand values, one launch instead of one per parameter and operation (each
+// such launch costs the host 4-5 us; the layer's step had seven in front of its kernels and eight behind them).
+__device__ __forceinline__ float ld_as_f32(const void* p, int dt, int64_t i) {
+    return dt == M2_F32 ? static_cast<const float*>(p)[i] : to_f32(static_cast<const bf16_t*>(p)[i]);
+}
+__device__ __forceinline__ void st_from_f32(void* p, int dt, int64_t i, float v) {
+    if (dt == M2_F32) static_cast<float*>(p)[i] = v;
+    else static_cast<bf16_t*>(p)[i] = from_f32<bf16_t>(v);
+}
+struct MixerParams { const void *A_log, *D, *dt_bias, *norm; int a, d, b, w; };
+__global__ void __launch_bounds__(256)
+mixer_params_kernel(const MixerParams p, float* __restrict__ out, int64_t nheads, int64_t channels) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < nheads) {
+        out[i] = -expf(ld_as_f32(p.A_log, p.a, i));
+        if (p.D) out[nheads + i] = ld_as_f32(p.D, p.d, i);
+        out[2 * nheads + i] = ld_as_f32(p.dt_bias, p.b, i);
+    }
+    if (i < channels) out[3 * nheads + i] = ld_as_f32(p.norm, p.w, i);
+}
+struct MixerGrads { const float *A, *dA, *dD, *db, *dw; void *A_log, *D, *dt_bias, *norm; int a, d, b, w; };
+__global__ void __launch_bounds__(256)
+mixer_params_grads_kernel(const MixerGrads p, int64_t nheads, int64_t channels) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < nheads) {
+        st_from_f32(p.A_log, p.a, i, p.dA[i] * p.A[i]);
+        if (p.D) st_from_f32(p.D, p.d, i, p.dD[i]);
+        st_from_f32(p.dt_bias, p.b, i, p.db[i]);
+    }
+    if (i < channels) st_from_f32(p.norm, p.w, i, p.dw[i]);
+}
+
 int check_norm_common(const m2_rmsnorm_params* p, const char* what) {
     M2_REQUIRE(p, M2_ERR_NULL, "%s: NULL params", what);
     M2_REQUIRE(p->rows >= 0 && p->channels > 0 && p->n_groups > 0 && p->channels % p->n_groups == 0, M2_ERR_SHAPE,
@@ -559,4 +593,33 @@ extern "C" int m2_add_rmsnorm(float* residual, int64_t residual_stride_row, cons
                                                                                      delta_stride_row, weight, static_cast<T*>(out),
                                                                                      out_stride_row, (int)channels, eps)));
     return check_launch("add_rmsnorm_kernel");
+}
+
+extern "C" int m2_mixer_params(const void* A_log, int32_t A_dtype, const void* D, int32_t D_dtype, const void* dt_bias, int32_t dt_bias_dtype,
+                               const void* norm_weight, int32_t norm_dtype, float* out, int64_t nheads, int64_t channels, void* stream) {
+    using namespace m2;
+    M2_REQUIRE(nheads > 0 && channels > 0, M2_ERR_SHAPE, "mixer_params: heads %lld, channels %lld", (long long)nheads, (long long)channels);
+    M2_REQUIRE(A_log && dt_bias && norm_weight && out, M2_ERR_NULL, "mixer_params: A_log, dt_bias, norm_weight and out are required");
+    for (const int32_t dt : {A_dtype, D_dtype, dt_bias_dtype, norm_dtype})
+        M2_REQUIRE(dt == M2_F32 || dt == M2_BF16, M2_ERR_DTYPE, "mixer_params: unsupported dtype %d", (int)dt);
+    const int64_t n = nheads > channels ? nheads : channels;
+    mixer_params_kernel<<<(unsigned)ceil_div(n, (int64_t)256), 256, 0, static_cast<hipStream_t>(stream)>>>(
+        MixerParams{A_log, D, dt_bias, norm_weight, A_dtype, D_dtype, dt_bias_dtype, norm_dtype}, out, nheads, channels);
+    return check_launch("mixer_params_kernel");
+}
+
+extern "C" int m2_mixer_params_grads(const float* A, const float* dA, const float* dD, const float* d_dt_bias, const float* d_norm_weight,
+                                     void* dA_log, int32_t A_dtype, void* dD_out, int32_t D_dtype, void* d_dt_bias_out, int32_t dt_bias_dtype,
+                                     void* d_norm_out, int32_t norm_dtype, int64_t nheads, int64_t channels, void* stream) {
+    using namespace m2;
+    M2_REQUIRE(nheads > 0 && channels > 0, M2_ERR_SHAPE, "mixer_params_grads: heads %lld, channels %lld", (long long)nheads, (long long)channels);
+    M2_REQUIRE(A && dA && d_dt_bias && d_norm_weight && dA_log && d_dt_bias_out && d_norm_out && (!dD_out || dD), M2_ERR_NULL,
+               "mixer_params_grads: a gradient or its destination is missing");
+    for (const int32_t dt : {A_dtype, D_dtype, dt_bias_dtype, norm_dtype})
+        M2_REQUIRE(dt == M2_F32 || dt == M2_BF16, M2_ERR_DTYPE, "mixer_params_grads: unsupported dtype %d", (int)dt);
+    const int64_t n = nheads > channels ? nheads : channels;
+    mixer_params_grads_kernel<<<(unsigned)ceil_div(n, (int64_t)256), 256, 0, static_cast<hipStream_t>(stream)>>>(
+        MixerGrads{A, dA, dD, d_dt_bias, d_norm_weight, dA_log, dD_out, d_dt_bias_out, d_norm_out, A_dtype, D_dtype, dt_bias_dtype, norm_dtype},
+        nheads, channels);
+    return check_launch("mixer_params_grads_kernel");
 }

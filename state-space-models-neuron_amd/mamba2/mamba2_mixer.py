@@ -20,11 +20,17 @@ from .configuration_mamba2 import Mamba2Config
 from .conv1d_grouped import ConvNKI
 from .fused_kernel import mamba2_fused_kernel, mamba2_fused_kernel_with_caching, mamba2_fused_prefill
 from .mamba2_kernel_inference import mamba2_kernel_inference
-from . import glue
+from . import _lib, glue
 
 
 def softplus(x, threshold=10):
     return torch.where(x < threshold, torch.log1p(torch.exp(torch.clamp(x, max=threshold))), x)
+
+
+def _plain_linear(m):
+    """True if calling ``m`` is nothing but its product: an ``nn.Linear`` itself, no subclass or wrapper, no hooks."""
+    return type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                                         or nn.modules.module._has_any_global_hook())
 
 
 class Mamba2Cache:
@@ -154,6 +160,11 @@ class Mamba2Mixer(nn.Module):
                                                cache_params.conv_states[self.layer_idx], cache_params.ssm_states[self.layer_idx],
                                                continuing=cache_params.seqlen_offset > 0)
             return self.out_proj(scan_output)
+        if _plain_linear(self.in_proj) and _plain_linear(self.out_proj) and not torch.is_autocast_enabled():
+            # one native node for the layer: the projections' products, the core, and the small parameters' casts
+            return _lib.native().mixer(hidden_states, self.in_proj.weight, self.A_log, self.D, self.dt_bias, self.conv1d.weight, self.norm.weight,
+                                       self.out_proj.weight, self.conv1d.bias, self.in_proj.bias, self.out_proj.bias, self.n_groups_tp,
+                                       self.ssm_state_size, self.intermediate_size_tp, self.head_dim, self.recompute_core)
         A = -torch.exp(self.A_log.float())
         zxBCdt = self.in_proj(hidden_states)
         core = mamba2_fused_kernel if self.recompute_core else mamba2_fused_kernel_with_caching
