@@ -176,10 +176,28 @@ class Mamba2Mixer(nn.Module):
                 cache_position: Optional[torch.LongTensor] = None, attention_mask: Optional[torch.Tensor] = None):
         return self.nki_kernels_forward(hidden_states, cache_params, cache_position, attention_mask)
 
+    def _native_step(self):
+        """True if the step is the native one: inference on plain projections and norm (no wrappers, hooks or autocast)."""
+        return (not torch.is_grad_enabled() and _plain_linear(self.in_proj) and _plain_linear(self.out_proj)
+                and type(self.norm) is MambaRMSNormGated and not torch.is_autocast_enabled())
+
+    def _step(self, cache_params, hidden=None, residual=None, delta=None, block_norm=None):
+        """One token through the layer: ``hidden`` (b, 1, D) -> the layer's output; or, with ``residual`` (fp32, in place), what is
+        still to be added to it and ``block_norm``, the whole block: residual += delta; mixer(norm(residual)) is added to the
+        residual as well (returns None) or comes back to be added."""
+        A, D, dt_bias = self._inference_params()
+        conv, norm, i = self.conv1d, self.norm, self.layer_idx
+        weight, eps = (None, 0.0) if block_norm is None else (_lib.f32_param(block_norm.weight), block_norm.variance_epsilon)
+        return _lib.native().mixer_step(hidden, residual, delta, weight, eps, self.in_proj.weight, self.in_proj.bias, conv.weight, conv.bias, A, D, dt_bias,
+                                        _lib.f32_param(norm.weight), norm.eps, norm.n_groups if norm.rmsnorm_within_groups else 1, self.out_proj.weight,
+                                        self.out_proj.bias, cache_params.conv_states[i], cache_params.ssm_states[i], self.n_groups_tp)
+
     def step(self, hidden_states, cache_params: Optional[Mamba2Cache] = None):
         """hidden_states: (B, 1, D) -> same shape; updates the layer's conv and SSM state."""
         batch, seqlen, dim = hidden_states.shape
         assert seqlen == 1
+        if self._native_step():
+            return self._step(cache_params, hidden=hidden_states)
         zxBCdt = self.in_proj(hidden_states)
         n_groups, d_state, d_inner, d_head = self.n_groups_tp, self.ssm_state_size, self.intermediate_size_tp, self.head_dim
         n_heads = d_inner // d_head

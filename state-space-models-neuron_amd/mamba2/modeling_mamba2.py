@@ -18,9 +18,9 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from . import glue
+from . import _lib, glue
 from .configuration_mamba2 import Mamba2Config
-from .mamba2_mixer import Mamba2Cache, Mamba2Mixer
+from .mamba2_mixer import Mamba2Cache, Mamba2Mixer, _plain_linear
 
 
 class Mamba2RMSNorm(nn.Module):
@@ -170,19 +170,28 @@ class Mamba2Model(Mamba2PreTrainedModel):
     def step(self, input_ids, cache_params: Optional[Mamba2Cache] = None):
         """input_ids: int64 (batch, 1), one token per sequence -> hidden states (batch, 1, hidden) after the final norm.
         The caller advances ``cache_params.seqlen_offset`` (a host integer, so that a captured step stays replayable)."""
+        residual, delta = self._step_residual(input_ids, cache_params)
+        if residual is not None:
+            return glue.add_rmsnorm_(residual, delta, self.norm_f.weight, self.norm_f.variance_epsilon, self.layers[0].mixer.in_proj.weight.dtype)
         x = self.embeddings(input_ids)
-        act = self.layers[0].mixer.in_proj.weight.dtype if len(self.layers) else x.dtype
-        if not (self.config.residual_in_fp32 and not torch.is_grad_enabled() and x.is_cuda and glue.add_rmsnorm_ok(x.shape[-1], act)):
-            for mixer_block in self.layers:
-                x = mixer_block.step(x, cache_params=cache_params)
-            return self.norm_f(x)
-        # fp32 residual stream: each block's residual add and the next norm are one kernel (the same arithmetic as
-        # Mamba2Block.step followed by Mamba2RMSNorm: fp32 sum, fp32 norm, one rounding to the activation dtype)
-        residual, delta = x.float().contiguous(), None
         for mixer_block in self.layers:
-            normed = glue.add_rmsnorm_(residual, delta, mixer_block.norm.weight, mixer_block.norm.variance_epsilon, act)
-            delta = mixer_block.mixer.step(normed, cache_params=cache_params)
-        return glue.add_rmsnorm_(residual, delta, self.norm_f.weight, self.norm_f.variance_epsilon, act)
+            x = mixer_block.step(x, cache_params=cache_params)
+        return self.norm_f(x)
+
+    def _step_residual(self, input_ids, cache_params):
+        """The fp32 residual stream (batch, 1, hidden) behind the last block and what is still to be added to it (or None), for
+        inference with ``residual_in_fp32``: each block's norm and residual add are part of its kernels or of one pass between
+        them (the same arithmetic as Mamba2Block.step, fp32 sums and norm).  (None, None) where the blocks have to be called one
+        by one."""
+        if not (self.config.residual_in_fp32 and len(self.layers) and all(blk.mixer._native_step() and type(blk.norm) is Mamba2RMSNorm for blk in self.layers)):
+            return None, None
+        x = self.embeddings(input_ids)
+        if not (x.is_cuda and glue.add_rmsnorm_ok(x.shape[-1], self.layers[0].mixer.in_proj.weight.dtype)):
+            return None, None
+        residual, delta = x.to(torch.float32, copy=True, memory_format=torch.contiguous_format), None
+        for mixer_block in self.layers:
+            delta = mixer_block.mixer._step(cache_params, residual=residual, delta=delta, block_norm=mixer_block.norm)
+        return residual, delta
 
 
 class Mamba2ForCausalLM(Mamba2PreTrainedModel):
@@ -232,6 +241,10 @@ class Mamba2ForCausalLM(Mamba2PreTrainedModel):
 
     def step(self, idx, cache_params: Optional[Mamba2Cache] = None):
         """idx: int64 (batch, 1) -> logits (batch, 1, vocab) fp32; the layers' states in ``cache_params`` advance by one token."""
+        residual, delta = self.backbone._step_residual(idx, cache_params) if _plain_linear(self.lm_head) else (None, None)
+        if residual is not None:
+            norm_f = self.backbone.norm_f
+            return _lib.native().norm_linear(residual, delta, _lib.f32_param(norm_f.weight), norm_f.variance_epsilon, self.lm_head.weight, self.lm_head.bias)
         hidden_states = self.backbone.step(idx, cache_params=cache_params)
         return self.lm_head(hidden_states.to(self.lm_head.weight.dtype)).float()
 

@@ -1,0 +1,84 @@
+"""GPU: the small products and the three-launch decode step of a layer, at the edges of their tiles (rows and outputs that are no
+multiple of 16, fewer k steps than waves, one and two column tiles, shapes that fall back), against fp64 on the CPU."""
+import pytest
+import torch
+
+from oracle.decode import decode_step_ref
+from oracle.mixer import rmsnorm_gated_ref, softplus_ref
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _rel(got, ref):
+    return ((got.double().cpu() - ref).norm() / ref.norm()).item()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 5, 32), (3, 16, 96), (16, 33, 1024), (17, 100, 2560), (32, 4384, 1024), (8, 20000, 256)])
+@pytest.mark.parametrize("x_kind,out_kind", [(0, 0), (1, 1), (0, 2)])
+def test_linear_small(M, N, K, x_kind, out_kind):
+    from mamba2 import _lib
+    lib = _lib.load()
+    if not lib.m2_linear_small_fits(M, N, K, x_kind, 1):
+        pytest.skip("normalised rows beyond the LDS limit take the separate norm")
+    gen = torch.Generator().manual_seed(M + N)
+    w = (torch.randn(N, K, generator=gen) / K ** 0.5).bfloat16().to(DEV)
+    bias = torch.randn(N, generator=gen).bfloat16().to(DEV)
+    nw = (1 + 0.1 * torch.randn(K, generator=gen)).to(DEV)
+    x = torch.randn(M, K, generator=gen).to(DEV)
+    x = x if x_kind == 1 else x.bfloat16()
+    base = torch.randn(M, N, generator=gen)
+    out = base.bfloat16().to(DEV) if out_kind == 0 else base.to(DEV)
+    p = _lib.LinearParams()
+    p.x, p.w, p.bias, p.norm_weight, p.out = (_lib.ptr(t) for t in (x, w, bias, nw, out))
+    p.M, p.N, p.K, p.x_stride_row, p.out_stride_row, p.nheads, p.norm_groups = M, N, K, K, N, 1, 1
+    p.x_kind, p.out_kind, p.eps = x_kind, out_kind, 1e-5
+    _lib.check(lib.m2_linear_small(p, _lib.stream_ptr()), "m2_linear_small")
+    xd = x.double().cpu()
+    if x_kind == 1:
+        xd = nw.double().cpu() * xd * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + 1e-5)
+    ref = xd @ w.double().cpu().T + bias.double().cpu() + (base.double() if out_kind == 2 else 0)
+    assert _rel(out, ref) < 5e-3
+
+
+@pytest.mark.parametrize("b,h,p,n,g,W,groups_norm", [(1, 8, 64, 128, 1, 4, True), (3, 6, 64, 64, 2, 3, True), (16, 4, 128, 64, 1, 4, False),
+                                                     (17, 8, 128, 128, 8, 4, True), (5, 24, 64, 128, 8, 4, False), (33, 8, 64, 128, 1, 3, True)])
+@pytest.mark.parametrize("block", [False, True])
+def test_layer_step_against_oracle(b, h, p, n, g, W, groups_norm, block):
+    from mamba2.configuration_mamba2 import Mamba2Config
+    from mamba2.mamba2_mixer import Mamba2Cache
+    from mamba2.modeling_mamba2 import Mamba2Block
+    d, hidden = h * p, h * p // 2
+    cfg = Mamba2Config(num_heads=h, head_dim=p, hidden_size=hidden, state_size=n, n_groups=g, num_hidden_layers=1, rmsnorm_within_groups=groups_norm)
+    torch.manual_seed(b + h)
+    blk = Mamba2Block(cfg, 0).bfloat16().to(DEV)
+    cache = Mamba2Cache(cfg, b, dtype=torch.bfloat16, device=DEV, conv_width=W)
+    for t in (cache.conv_states[0], cache.ssm_states[0]):
+        t.normal_(0, 0.5)
+    x = torch.randn(b, 1, hidden, device=DEV)
+    m = blk.mixer
+    f = lambda t: t.detach().double().cpu()
+    xin = f(x) if block else f(x.bfloat16())
+    u = f(blk.norm.weight) * xin * torch.rsqrt(xin.pow(2).mean(-1, keepdim=True) + blk.norm.variance_epsilon) if block else xin
+    zx = u @ f(m.in_proj.weight).T
+    cx = d + 2 * g * n
+    y, cs, S = decode_step_ref(zx[..., d:d + cx], f(cache.conv_states[0]), f(m.conv1d.weight).squeeze(1), f(m.conv1d.bias), f(cache.ssm_states[0]),
+                               softplus_ref(zx[..., d + cx:] + f(m.dt_bias)), -torch.exp(f(m.A_log)), f(m.D), n_groups=g)
+    ref = rmsnorm_gated_ref(y, zx[..., :d], f(m.norm.weight), g if groups_norm else 1, m.norm.eps) @ f(m.out_proj.weight).T
+    with torch.no_grad():
+        got = blk.step(x, cache_params=cache) if block else m.step(x.bfloat16(), cache_params=cache)
+    assert _rel(got, ref + xin if block else ref) < 2e-2
+    assert _rel(cache.conv_states[0], cs) < 5e-3 and _rel(cache.ssm_states[0], S) < 1e-2
+    # the residual form: the block inside Mamba2Model.step
+    if block:
+        for t, r in ((cache.conv_states[0], cs), (cache.ssm_states[0], S)):
+            assert torch.isfinite(t).all()
+        c2 = Mamba2Cache(cfg, b, dtype=torch.bfloat16, device=DEV, conv_width=W)
+        c3 = Mamba2Cache(cfg, b, dtype=torch.bfloat16, device=DEV, conv_width=W)
+        with torch.no_grad():
+            res = x.clone()
+            delta = m._step(c2, residual=res, block_norm=blk.norm)
+            want = blk.step(x, cache_params=c3)
+        res = res if delta is None else res + delta
+        assert _rel(res, want.double().cpu()) < 5e-3
+        assert _rel(c2.ssm_states[0], c3.ssm_states[0].double().cpu()) < 1e-2
