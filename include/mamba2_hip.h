@@ -240,29 +240,34 @@ int m2_add_rmsnorm(float* residual, int64_t residual_stride_row, const void* del
                    int32_t dtype, void* stream);
 
 /* Small products of the token-by-token loop (the projections and the LM head for up to 32 sequences), bf16 operands, fp32
- * accumulation:  out[m][n] = bias[n] + sum_k X[m][k] * w[n][k],  w (N, K) contiguous.
- *   x_kind 0: X = x, bf16 rows.
- *   x_kind 1: x fp32 rows;  X = norm_weight * x * rsqrt(mean(x^2) + eps)  (Mamba2RMSNorm in front of in_proj or of the head).
- *   x_kind 2: x bf16 rows h = y * silu(z), head_sq (M, nheads) fp32 sums of h^2 per head;
- *             X = norm_weight * h * rsqrt(group mean of h^2 + eps)        (the gated norm in front of out_proj).
- *   out_kind 0: bf16;  1: fp32;  2: fp32, added to what is there (the residual stream).
- * M <= 32, K a multiple of 32; x_kind 1, 2: M * (K + 8) * 2 bytes within 40 KB, at most 8 norm groups: m2_linear_small_fits()
- * says whether a shape is taken.
+ * accumulation:  out[m][n] = bias[n] + scale[m] * sum_k x[m][k] * w[n][k],  w (N, K) contiguous, x bf16 rows.
+ *   sq NULL: scale = 1.  Otherwise x is a row times a norm weight, sq (M, nsq) the sums of squares of the row without it, and
+ *   scale = rsqrt(sum(sq[m]) / K + eps): the RMS norm (Mamba2RMSNorm) in front of the product, finished behind it.  groups > 1:
+ *   the row is groups equal parts, each with nsq / groups sums and a scale of its own (the gated norm).
+ *   out_kind 0: bf16;  1: fp32;  2: fp32, added to what is there (the residual stream); with next_weight (N) also the new rows
+ *   times it, next_x (M, N) bf16, and their sums of squares, next_sq (M, ceil(N / 16)): x, sq and nsq of the next product.
+ * M <= 32, K a multiple of 64; groups: 1, or such that K splits into equal shares of waves inside each:
+ * m2_linear_small_fits() says whether a shape is taken.
+ * m2_decode_rows: the head of such a chain: residual (rows, channels) fp32 += delta (set != 0: = delta; delta may be NULL
+ * otherwise), x = bf16(residual * weight), sq (rows, 1).
  * m2_decode_layer: one decode step of a whole mixer layer in three launches (mamba2/mamba2_mixer.py:243-282): `in` writes
  * zxBCdt (bf16 rows, in->out), the scan reads it and the states of `dec` (updated in place; dec's xBC, dt, y and workspace
- * are not used), leaves h (batch, nheads * headdim) bf16 and head_sq (batch, nheads) fp32 in the caller's scratch, and
- * `out` (x = h, x_kind 2) writes the result.  headdim and dstate 64 or 128, conv width 4, bf16. */
+ * are not used) and writes the gated rows times norm_weight to out->x (batch, nheads * headdim) bf16 and their sums to
+ * out->sq (batch, nheads) fp32 -- the caller's scratch -- and `out` writes the result.  headdim and dstate 64 or 128, conv
+ * width 4, bf16. */
 typedef struct m2_linear_params {
-    const void* x; const void* w; const void* bias; const float* norm_weight; const float* head_sq;
-    void* out;
-    int64_t M, N, K, nheads, x_stride_row, out_stride_row;
-    int32_t x_kind, out_kind, norm_groups;
+    const void* x; const void* w; const void* bias; const float* sq;
+    void* out; const float* next_weight; void* next_x; float* next_sq;
+    int64_t M, N, K, nsq, x_stride_row, out_stride_row;
+    int32_t out_kind, groups;
     float eps;
 } m2_linear_params;
 
-int m2_linear_small_fits(int64_t M, int64_t N, int64_t K, int32_t x_kind, int32_t norm_groups);
+int m2_linear_small_fits(int64_t M, int64_t N, int64_t K, int32_t groups);
 int m2_linear_small(const m2_linear_params* p, void* stream);
-int m2_decode_layer(const m2_linear_params* in, const m2_decode_params* dec, const m2_linear_params* out, void* h, float* head_sq, void* stream);
+int m2_decode_rows(float* residual, const void* delta, int32_t delta_dtype, int32_t set, const float* weight, void* x, float* sq, int64_t rows,
+                   int64_t channels, void* stream);
+int m2_decode_layer(const m2_linear_params* in, const m2_decode_params* dec, const float* norm_weight, const m2_linear_params* out, void* stream);
 
 /* The small parameters of a mixer layer as the kernels take them, and their gradients back, in one launch each
  * (mamba2/mamba2_mixer.py:225-236: A = -exp(A_log.float()) and the casts around it).

@@ -30,7 +30,7 @@ using torch::autograd::variable_list;
     F(m2_last_error) F(m2_conv1d_fwd) F(m2_conv1d_bwd_workspace_bytes) F(m2_conv1d_bwd) F(m2_ssd_chunk_states_bytes) \
     F(m2_ssd_fwd_workspace_bytes) F(m2_ssd_fwd) F(m2_ssd_bwd_workspace_bytes) F(m2_ssd_bwd) F(m2_decode_workspace_bytes) \
     F(m2_decode_step) F(m2_decode_step_static) F(m2_rmsnorm_gated_fwd) F(m2_rmsnorm_gated_bwd_workspace_bytes) \
-    F(m2_rmsnorm_gated_bwd) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_layer) F(m2_mixer_params) F(m2_mixer_params_grads)
+    F(m2_rmsnorm_gated_bwd) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_rows) F(m2_decode_layer) F(m2_mixer_params) F(m2_mixer_params_grads)
 struct Lib {
 #define M2_FIELD(name) decltype(&::name) name = nullptr;
     M2_BOUND(M2_FIELD)
@@ -777,28 +777,35 @@ std::tuple<Tensor, Tensor, Tensor> decode_step(const Tensor& xBC, const Tensor& 
 }
 
 // ----------------------------------------------------------------------------------------------- decode step of a layer
-// mamba2_mixer.py:243-282, and with `residual` the block around it (modeling_mamba2.py:133-140): in place on the layer's
-// states and on the residual stream.
+// mamba2_mixer.py:243-282, and with a residual stream the block around it (modeling_mamba2.py:133-140): in place on the layer's
+// states and on the stream.
 struct StepArgs {
     const Tensor &in_w, &in_b, &conv_w, &conv_b, &A, &D, &dt_bias, &norm_w, &out_w, &out_b, &conv_state, &ssm_state;
     int64_t g, norm_groups;
     double eps;
 };
 
-bool linear_takes(const Tensor& x, const Tensor& w, const Tensor& bias) {
-    return x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && w.is_contiguous() && (!bias.defined() || bias.is_contiguous());
+// The fp32 residual rows of a model's step between two of its layers: either `delta` is still to be added (separate kernels),
+// or `x` holds the rows times the next norm's weight and `sq` their sums of squares (chained kernels), or neither.
+struct ResidualStream {
+    Tensor rows, delta, x, sq;
+    Tensor first;                  // embedding rows that `rows` is yet to be set to
+};
+
+bool linear_takes(const Tensor& w, const Tensor& bias) {
+    return w.scalar_type() == at::kBFloat16 && w.is_contiguous() && (!bias.defined() || (bias.is_contiguous() && bias.scalar_type() == at::kBFloat16));
 }
 
 m2_linear_params linear_params(const Tensor& w, const Tensor& bias, int64_t rows) {
     m2_linear_params p{};
-    p.w = ptr(w); p.bias = ptr(bias); p.M = rows; p.N = w.size(0); p.K = w.size(1); p.norm_groups = 1; p.nheads = 1;
+    p.w = ptr(w); p.bias = ptr(bias); p.M = rows; p.N = w.size(0); p.K = w.size(1); p.groups = 1;
     return p;
 }
 
 // out = x w^T + bias for a few bf16 rows; the library's product where the kernel does not take the shape
 Tensor linear_rows(const Tensor& x, const Tensor& w, const Tensor& bias, void* stream) {
     m2_linear_params p = linear_params(w, bias, x.size(0));
-    if (!linear_takes(x, w, bias) || !lib.m2_linear_small_fits(p.M, p.N, p.K, 0, 1)) return project(x, w, bias);
+    if (x.scalar_type() != at::kBFloat16 || !linear_takes(w, bias) || !lib.m2_linear_small_fits(p.M, p.N, p.K, 1)) return project(x, w, bias);
     const Tensor xr = aligned(x);
     Tensor out = at::empty({p.M, p.N}, x.options());
     p.x = ptr(xr); p.x_stride_row = xr.stride(0); p.out = ptr(out); p.out_stride_row = p.N;
@@ -806,56 +813,102 @@ Tensor linear_rows(const Tensor& x, const Tensor& w, const Tensor& bias, void* s
     return out;
 }
 
-// hidden: (b, hidden) rows, or undefined with residual (b, hidden) fp32, what is still to be added to it, and its norm.
-// Returns the layer's output rows; nothing where they were added to the residual.
-Tensor step_rows(const Tensor& hidden, const Tensor& residual, const Tensor& delta, const Tensor& block_norm, double block_eps, const StepArgs& a, void* stream) {
+// the stream's rows, set from the embedding if they are not yet
+const Tensor& stream_rows(ResidualStream& r) {
+    if (r.first.defined()) {
+        r.rows = r.first.to(at::kFloat, /*non_blocking=*/false, /*copy=*/true, at::MemoryFormat::Contiguous);
+        r.first = Tensor();
+    }
+    return r.rows;
+}
+
+// x and sq of the stream for a norm weight
+void stream_heads(ResidualStream& r, const Tensor& norm_w, void* stream) {
+    if (r.x.defined()) return;
+    const bool set = r.first.defined();
+    const Tensor src = set ? r.first.contiguous() : (r.delta.defined() ? r.delta.contiguous() : Tensor());
+    if (set) r.rows = at::empty(src.sizes(), src.options().dtype(at::kFloat));
+    r.x = at::empty(r.rows.sizes(), r.rows.options().dtype(at::kBFloat16));
+    r.sq = at::empty({r.rows.size(0), 1}, r.rows.options());
+    check(lib.m2_decode_rows(ptr<float>(r.rows), ptr(src), src.defined() ? dtype_code(src) : M2_F32, set, ptr<float>(norm_w), ptr(r.x), ptr<float>(r.sq), r.rows.size(0),
+                             r.rows.size(1), stream), "m2_decode_rows");
+    r.first = r.delta = Tensor();
+}
+
+void set_rows(m2_linear_params& p, const Tensor& x, const Tensor& sq, double eps) {
+    p.x = ptr(x); p.x_stride_row = x.stride(0); p.sq = ptr<float>(sq); p.nsq = sq.defined() ? sq.size(1) : 0; p.eps = static_cast<float>(eps);
+}
+
+// hidden: (b, hidden) rows -> the layer's output rows.  With a stream instead, the block: its norm, the layer, and the sum in the
+// stream; next_norm: the weight of the norm that will read it, if that is known.
+Tensor step_rows(const Tensor& hidden, ResidualStream* r, const Tensor& block_norm, double block_eps, const Tensor& next_norm, const StepArgs& a, void* stream) {
     const int64_t b = a.ssm_state.size(0), h = a.ssm_state.size(1), hd = a.ssm_state.size(2), n = a.ssm_state.size(3), d = h * hd;
     const at::TensorOptions act = a.in_w.options();
-    const Tensor zx = at::empty({b, a.in_w.size(0)}, act);
+    const at::ScalarType act_type = a.in_w.scalar_type();
     m2_linear_params in = linear_params(a.in_w, a.in_b, b), out = linear_params(a.out_w, a.out_b, b);
-    out.norm_groups = static_cast<int32_t>(a.norm_groups); out.nheads = h; out.eps = static_cast<float>(a.eps); out.norm_weight = ptr<float>(a.norm_w);
-    out.x_kind = 2;
-    const Tensor first = residual.defined() ? residual : aligned(hidden);
-    in.x_kind = residual.defined() && lib.m2_linear_small_fits(in.M, in.N, in.K, 1, 1) ? 1 : 0;
-    const bool fused = linear_takes(zx, a.in_w, a.in_b) && linear_takes(zx, a.out_w, a.out_b) && (residual.defined() || hidden.scalar_type() == at::kBFloat16) &&
-                       lib.m2_linear_small_fits(in.M, in.N, in.K, in.x_kind, 1) && lib.m2_linear_small_fits(out.M, out.N, out.K, 2, out.norm_groups) &&
-                       (hd == 64 || hd == 128) && (n == 64 || n == 128) && a.conv_w.size(-1) == 4 && d % (a.norm_groups * hd) == 0;
-    Tensor rows = first;
-    if (residual.defined() && (in.x_kind == 0 || !fused))
-        rows = add_rmsnorm(residual, delta.defined() ? OptTensor(delta) : std::nullopt, block_norm, block_eps, act.dtype().toScalarType());
-    else if (delta.defined()) residual.add_(delta);
-    const Tensor result = residual.defined() && fused ? residual : at::empty({b, a.out_w.size(0)}, act);
+    const bool fused = linear_takes(a.in_w, a.in_b) && linear_takes(a.out_w, a.out_b) && (r || hidden.scalar_type() == at::kBFloat16) &&
+                       lib.m2_linear_small_fits(in.M, in.N, in.K, 1) && lib.m2_linear_small_fits(out.M, out.N, out.K, static_cast<int32_t>(a.norm_groups)) &&
+                       (hd == 64 || hd == 128) && (n == 64 || n == 128) && a.conv_w.size(-1) == 4 && h % a.norm_groups == 0;
     if (!fused) {
+        Tensor rows = hidden;
+        if (r) {
+            rows = add_rmsnorm(stream_rows(*r), r->delta.defined() ? OptTensor(r->delta) : std::nullopt, block_norm, block_eps, act_type);
+            r->x = r->sq = Tensor();
+        }
         const Tensor packed = linear_rows(rows, a.in_w, a.in_b, stream).unsqueeze(1);
         const int64_t cx = d + 2 * a.g * n;
         const Tensor y = std::get<0>(decode_step(packed.narrow(2, d, cx), a.conv_state, a.conv_w, a.conv_b.defined() ? OptTensor(a.conv_b) : std::nullopt,
                                                  a.ssm_state, packed.narrow(2, d + cx, h), a.A, a.D, a.g, M2_ACT_SILU, a.dt_bias, std::nullopt, false));
-        const Tensor normed = rmsnorm_forward(y.view({b, d}), packed.select(1, 0).narrow(1, 0, d), a.norm_w, a.norm_groups, a.eps, act.dtype().toScalarType());
-        return linear_rows(normed, a.out_w, a.out_b, stream);
+        const Tensor normed = rmsnorm_forward(y.view({b, d}), packed.select(1, 0).narrow(1, 0, d), a.norm_w, a.norm_groups, a.eps, act_type);
+        const Tensor o = linear_rows(normed, a.out_w, a.out_b, stream);
+        if (r) r->delta = o;
+        return o;
     }
+    const Tensor zx = at::empty({b, a.in_w.size(0)}, act);
     const Tensor conv_w = a.conv_w.contiguous(), conv_b = a.conv_b.defined() ? a.conv_b.contiguous() : a.conv_b;
-    const Tensor mid = at::empty({b * (d * 2 + h * 4)}, act.dtype(at::kByte));          // h rows (bf16), then the head sums (fp32)
-    in.x = ptr(rows); in.x_stride_row = rows.stride(0); in.out = ptr(zx); in.out_stride_row = zx.size(1);
-    in.norm_weight = in.x_kind ? ptr<float>(block_norm) : nullptr; in.eps = static_cast<float>(block_eps);
-    out.x = ptr(mid); out.x_stride_row = d; out.head_sq = reinterpret_cast<float*>(at_column(mid, b * d * 2));
-    out.out = ptr(result); out.out_stride_row = result.stride(0); out.out_kind = residual.defined() ? 2 : 0;
+    const Tensor mid = at::empty({b * (d * 2 + h * 4)}, act.dtype(at::kByte));          // gated rows (bf16), then the head sums (fp32)
+    const Tensor x = r ? Tensor() : aligned(hidden);
+    Tensor result, next_x, next_sq;
+    if (r) {
+        stream_heads(*r, block_norm, stream);
+        set_rows(in, r->x, r->sq, block_eps);
+        out.out = ptr(r->rows); out.out_kind = 2;
+        if (next_norm.defined()) {
+            next_x = at::empty({b, out.N}, act);
+            next_sq = at::empty({b, (out.N + 15) / 16}, r->rows.options());
+            out.next_weight = ptr<float>(next_norm); out.next_x = ptr(next_x); out.next_sq = ptr<float>(next_sq);
+        }
+    } else {
+        set_rows(in, x, Tensor(), 0.0);
+        result = at::empty({b, out.N}, act);
+        out.out = ptr(result);
+    }
+    in.out = ptr(zx); in.out_stride_row = in.N;
+    out.x = ptr(mid); out.x_stride_row = d; out.sq = reinterpret_cast<float*>(at_column(mid, b * d * 2)); out.nsq = h;
+    out.groups = static_cast<int32_t>(a.norm_groups); out.eps = static_cast<float>(a.eps); out.out_stride_row = out.N;
     m2_decode_params p{};
     p.conv_state = ptr(a.conv_state); p.conv_w = ptr(conv_w); p.conv_b = ptr(conv_b); p.S = ptr<float>(a.ssm_state);
     p.A = ptr<float>(a.A); p.D = ptr<float>(a.D); p.dt_bias = ptr<float>(a.dt_bias);
     p.batch = b; p.nheads = h; p.headdim = hd; p.dstate = n; p.ngroups = a.g; p.k = 4; p.W = static_cast<int32_t>(a.conv_state.size(2));
     p.dtype = M2_BF16; p.param_dtype = dtype_code(conv_w); p.activation = M2_ACT_SILU;
-    check(lib.m2_decode_layer(&in, &p, &out, ptr(mid), reinterpret_cast<float*>(at_column(mid, b * d * 2)), stream), "m2_decode_layer");
-    return residual.defined() ? Tensor() : result;
+    check(lib.m2_decode_layer(&in, &p, ptr<float>(a.norm_w), &out, stream), "m2_decode_layer");
+    if (r) { r->x = next_x; r->sq = next_sq; }
+    return result;
 }
 
-// A, D, dt_bias, norm weights: fp32 (the caller keeps them)
-Tensor mixer_step(const OptTensor& hidden_, const OptTensor& residual_, const OptTensor& delta_, const OptTensor& block_norm_, double block_eps, const Tensor& in_w, const OptTensor& in_b,
-                      const Tensor& conv_w, const OptTensor& conv_b, const Tensor& A, const Tensor& D, const Tensor& dt_bias, const Tensor& norm_w, double eps,
-                      int64_t norm_groups, const Tensor& out_w, const OptTensor& out_b, const Tensor& conv_state, const Tensor& ssm_state, int64_t g) {
-    const Tensor &hidden = or_none(hidden_), &residual = or_none(residual_), &delta = or_none(delta_), &block_norm = or_none(block_norm_);
-    const Tensor& x = residual.defined() ? residual : hidden;
-    TORCH_CHECK_VALUE(x.defined() && x.dim() == 3 && x.size(1) == 1, "hidden_states must be (batch, 1, hidden_size)");
-    const int64_t b = x.size(0);
+void check_fp32(std::initializer_list<const Tensor*> tensors, const char* what) {
+    for (const Tensor* t : tensors)
+        TORCH_CHECK_VALUE(!t->defined() || (t->scalar_type() == at::kFloat && t->is_contiguous()), what, " must be contiguous float32");
+}
+
+// A, D, dt_bias, norm weights: fp32 (the caller keeps them).  Either hidden (b, 1, hidden) -> output, or a stream with the norms.
+Tensor mixer_step(const OptTensor& hidden_, ResidualStream* r, const OptTensor& block_norm_, double block_eps, const OptTensor& next_norm_, const Tensor& in_w,
+                  const OptTensor& in_b, const Tensor& conv_w, const OptTensor& conv_b, const Tensor& A, const Tensor& D, const Tensor& dt_bias, const Tensor& norm_w,
+                  double eps, int64_t norm_groups, const Tensor& out_w, const OptTensor& out_b, const Tensor& conv_state, const Tensor& ssm_state, int64_t g) {
+    const Tensor &hidden = or_none(hidden_), &block_norm = or_none(block_norm_), &next_norm = or_none(next_norm_);
+    const Tensor& x = r ? (r->first.defined() ? r->first : r->rows) : hidden;
+    TORCH_CHECK_VALUE(x.defined() && (r ? x.dim() == 2 : x.dim() == 3 && x.size(1) == 1), "hidden_states must be (batch, 1, hidden_size)");
+    const int64_t b = x.size(0), width = x.size(-1);
     require_gpu({&x, &in_w, &conv_w, &A, &D, &dt_bias, &norm_w, &out_w, &conv_state, &ssm_state});
     TORCH_CHECK_VALUE(ssm_state.dim() == 4 && ssm_state.size(0) == b && ssm_state.scalar_type() == at::kFloat && ssm_state.is_contiguous(),
                       "the SSM state must be float32 (batch, heads, headdim, state), contiguous");
@@ -863,43 +916,64 @@ Tensor mixer_step(const OptTensor& hidden_, const OptTensor& residual_, const Op
     TORCH_CHECK_VALUE(conv_state.dim() == 3 && conv_state.size(0) == b && conv_state.size(1) == cx && conv_state.size(2) >= conv_w.size(-1) - 1 &&
                           conv_state.scalar_type() == in_w.scalar_type() && conv_state.is_contiguous(),
                       "the conv state must be (batch, ", cx, ", W >= k-1), contiguous, in the dtype of the projections");
-    TORCH_CHECK_VALUE(in_w.dim() == 2 && in_w.size(0) == d + cx + h && in_w.size(1) == x.size(2) && out_w.dim() == 2 && out_w.size(1) == d,
+    TORCH_CHECK_VALUE(in_w.dim() == 2 && in_w.size(0) == d + cx + h && in_w.size(1) == width && out_w.dim() == 2 && out_w.size(1) == d,
                       "the projections do not match the states");
     TORCH_CHECK_VALUE(g > 0 && h % g == 0 && conv_w.numel() == cx * conv_w.size(-1) && A.numel() == h && D.numel() == h && dt_bias.numel() == h && norm_w.numel() == d,
                       "parameter shapes do not match the states");
-    for (const Tensor* t : {&A, &D, &dt_bias, &norm_w})
-        TORCH_CHECK_VALUE(t->scalar_type() == at::kFloat && t->is_contiguous(), "A, D, dt_bias and the norm weight must be contiguous float32");
-    if (residual.defined())
-        TORCH_CHECK_VALUE(residual.scalar_type() == at::kFloat && residual.is_contiguous() && block_norm.defined() && block_norm.scalar_type() == at::kFloat &&
-                              block_norm.is_contiguous() && block_norm.numel() == x.size(2) && out_w.size(0) == x.size(2),
-                          "the residual stream must be contiguous float32 with a float32 norm weight of its width");
+    check_fp32({&A, &D, &dt_bias, &norm_w, &block_norm, &next_norm}, "A, D, dt_bias and the norm weights");
+    TORCH_CHECK_VALUE(!r || (block_norm.defined() && block_norm.numel() == width && out_w.size(0) == width && (!next_norm.defined() || next_norm.numel() == width)),
+                      "the norm weights must have the width of the residual stream");
     Scope scope(x);
     const StepArgs a{in_w, or_none(in_b), conv_w, or_none(conv_b), A, D, dt_bias, norm_w, out_w, or_none(out_b), conv_state, ssm_state, g, norm_groups, eps};
-    const Tensor o = residual.defined() ? step_rows(Tensor(), residual.view({b, x.size(2)}), delta.defined() ? delta.view({b, x.size(2)}) : delta, block_norm,
-                                                    block_eps, a, scope.stream)
-                                        : step_rows(hidden.reshape({b, hidden.size(2)}), Tensor(), Tensor(), Tensor(), 0.0, a, scope.stream);
-    return o.defined() ? o.view({b, 1, out_w.size(0)}) : o;
+    if (r) {
+        step_rows(Tensor(), r, block_norm, block_eps, next_norm, a, scope.stream);
+        return Tensor();
+    }
+    return step_rows(hidden.reshape({b, width}), nullptr, Tensor(), 0.0, Tensor(), a, scope.stream).view({b, 1, out_w.size(0)});
 }
 
-// fp32 logits of the normalised residual rows: norm_f and the LM head (modeling_mamba2.py:350, 489-490)
-Tensor norm_linear(const Tensor& residual, const OptTensor& delta, const Tensor& norm_w, double eps, const Tensor& w, const OptTensor& bias_) {
-    require_gpu({&residual, &norm_w, &w});
-    TORCH_CHECK_VALUE(residual.scalar_type() == at::kFloat && residual.is_contiguous() && residual.size(-1) == w.size(1) && norm_w.numel() == w.size(1) &&
-                          norm_w.scalar_type() == at::kFloat && norm_w.is_contiguous(), "norm_linear: fp32 residual rows and norm weight of the product's width");
-    Scope scope(residual);
+ResidualStream residual_stream(const Tensor& embedded) {
+    require_gpu({&embedded});
+    dtype_code(embedded);
+    ResidualStream r;
+    r.first = embedded.reshape({-1, embedded.size(-1)});
+    return r;
+}
+
+// the stream's rows as they are, everything added
+Tensor stream_sum(ResidualStream& r) {
+    const Tensor& any = r.first.defined() ? r.first : r.rows;
+    Scope scope(any);
+    const Tensor& rows = stream_rows(r);
+    if (r.delta.defined()) { rows.add_(r.delta); r.delta = Tensor(); }
+    return rows;
+}
+
+// the stream's rows after its last norm, in out_dtype
+Tensor stream_norm(ResidualStream& r, const Tensor& norm_w, double eps, at::ScalarType out_dtype) {
+    check_fp32({&norm_w}, "the norm weight");
+    Scope scope(norm_w);
+    const Tensor& rows = stream_rows(r);
+    const Tensor out = add_rmsnorm(rows, r.delta.defined() ? OptTensor(r.delta) : std::nullopt, norm_w, eps, out_dtype);
+    r.delta = r.x = r.sq = Tensor();
+    return out;
+}
+
+// fp32 product of the normalised rows: norm_f and the LM head (modeling_mamba2.py:350, 489-490)
+Tensor stream_norm_linear(ResidualStream& r, const Tensor& norm_w, double eps, const Tensor& w, const OptTensor& bias_) {
     const Tensor& bias = or_none(bias_);
-    std::vector<int64_t> shape = residual.sizes().vec();
-    shape.back() = w.size(0);
-    const Tensor x = residual.view({-1, w.size(1)});
-    m2_linear_params p = linear_params(w, bias, x.size(0));
-    p.x_kind = 1; p.out_kind = 1;
-    if (delta || !linear_takes(w, w, bias) || !lib.m2_linear_small_fits(p.M, p.N, p.K, 1, 1)) {
-        const Tensor rows = add_rmsnorm(x, delta ? OptTensor(delta->view(x.sizes())) : std::nullopt, norm_w, eps, w.scalar_type());
-        return linear_rows(rows, w, bias, scope.stream).to(at::kFloat).view(shape);
-    }
-    Tensor out = at::empty(shape, residual.options());
-    p.x = ptr(x); p.x_stride_row = p.K; p.norm_weight = ptr<float>(norm_w); p.eps = static_cast<float>(eps);
-    p.out = ptr(out); p.out_stride_row = p.N;
+    require_gpu({&norm_w, &w, &bias});
+    check_fp32({&norm_w}, "the norm weight");
+    const Tensor& any = r.first.defined() ? r.first : r.rows;
+    TORCH_CHECK_VALUE(w.dim() == 2 && any.size(1) == w.size(1) && norm_w.numel() == w.size(1), "the norm weight and the product must have the width of the residual stream");
+    Scope scope(w);
+    m2_linear_params p = linear_params(w, bias, any.size(0));
+    if (!linear_takes(w, bias) || !lib.m2_linear_small_fits(p.M, p.N, p.K, 1))
+        return linear_rows(stream_norm(r, norm_w, eps, w.scalar_type()), w, bias, scope.stream).to(at::kFloat);
+    stream_heads(r, norm_w, scope.stream);
+    const Tensor out = at::empty({p.M, p.N}, r.rows.options());
+    set_rows(p, r.x, r.sq, eps);
+    p.out = ptr(out); p.out_stride_row = p.N; p.out_kind = 1;
     check(lib.m2_linear_small(&p, scope.stream), "m2_linear_small");
     return out;
 }
@@ -907,6 +981,7 @@ Tensor norm_linear(const Tensor& residual, const OptTensor& delta, const Tensor&
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    py::class_<ResidualStream>(m, "ResidualStream");
     m.def("bound_names", &bound_names);
     m.def("bind", &bind);
     m.def("conv1d_forward", &conv1d_forward);
@@ -926,6 +1001,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("mixer", &mixer);
     m.def("fused_prefill", &fused_prefill);
     m.def("mixer_step", &mixer_step);
-    m.def("norm_linear", &norm_linear);
+    m.def("residual_stream", &residual_stream);
+    m.def("stream_sum", &stream_sum);
+    m.def("stream_norm", &stream_norm);
+    m.def("stream_norm_linear", &stream_norm_linear);
     m.def("decode_step", &decode_step);
 }

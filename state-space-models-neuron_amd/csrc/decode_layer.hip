@@ -1,172 +1,212 @@
 // One decode step of a whole mixer layer for few sequences: three launches (mamba2/mamba2_mixer.py:243-282 step, and around it
 // modeling_mamba2.py:94-103, 133-140, the block's norm and residual add).
 //
-//   linear_small (in_proj)     [norm of the residual row ->] zxBCdt = W x
-//   decode_gated               conv + SiLU of the token, S' = S exp(A dt) + dt x (x) B, h = (S' C + D x) silu(z), sum of h^2 per head
-//   linear_small (out_proj)    h scaled to the gated RMSNorm -> W h [+ residual]; shifts the B/C conv states on the side
+//   linear_small (in_proj)     zxBCdt = W x, scaled by the row's 1 / rms when x comes from the residual stream
+//   decode_gated               conv + SiLU of the token, S' = S exp(A dt) + dt x (x) B, h = (S' C + D x) silu(z): w h and sum of h^2 per head
+//   linear_small (out_proj)    W (w h), scaled by the groups' 1 / rms [+ residual: the new residual times the next norm's weight
+//                              and its sums of squares]; shifts the B/C conv states on the side
 //
 // At this size a step is bound by its launches and by latency: the same layer as separate kernels is seven of 4.6-11 us each
-// (two library products, conv, scan, norm, add + norm), most of them idle, and 2.3x the host work.  Folding every row-wise
-// operation into the product that reads its result leaves three launches whose time is the weights' and states' way from HBM.
-#include "common.hpp"
+// (two library products, conv, scan, norm, add + norm), most of them idle, and 2.3x the host work.  An RMS norm in front of a
+// product costs nothing when it is taken apart: the weight is applied by whoever writes the row, the sum of squares is left
+// beside it, and 1 / rms scales the finished product (a common factor of the row, or of the K range of one wave for grouped
+// norms).  Normalising the rows inside the product instead (once per workgroup, through LDS) made it 7.9 us where the plain
+// product takes 5.3 (8 rows of 1024, 4384 outputs), and a kernel of its own is 4.7 us.
+#include <initializer_list>
+
+#include "ssd_host.hpp"
+#include "ssd_y.hpp"
 
 namespace m2 {
 namespace {
 
 // ------------------------------------------------------------------------------------------ small products
-// out[m][n] = sum_k X[m][k] W[n][k] for m < M <= 32, bf16 operands, fp32 accumulation.
+// out[m][n] = scale[m] * sum_k X[m][k] W[n][k] for m < M <= 32, bf16 operands, fp32 accumulation.
 //
-// A workgroup owns 16 rows of W at a time; its NW waves split K, each with v_mfma_f32_16x16x32_bf16 whose A operand is the
-// weights (16 bytes per lane straight from HBM, UN loads ahead) and whose B operand is the activations, and the NW partial
-// tiles meet in LDS.  16 rows rather than 32 because the narrow products have few of them (1024 outputs: 64 workgroups) and
-// what counts is the number of loads in flight over the chip.  X kinds:
-//   plain   bf16 rows read where they lie (L2 hits: every workgroup reads all of them)
-//   norm    fp32 residual rows -> w x rsqrt(mean(x^2) + eps), formed once per workgroup into LDS as bf16
-//   gated   bf16 h rows and per-head sums of squares -> w h rsqrt(group mean + eps), likewise
-// The weights of the first tile are on their way before the rows are normalised.
-enum { kPlain = 0, kNorm = 1, kGated = 2 };
+// A workgroup owns 16 rows of W at a time; its NW waves split K, each with v_mfma_f32_16x16x32_bf16 (A = weights, B = x), and
+// the NW partial tiles meet in LDS.  16 rows rather than 32 because the narrow products have few of them (1024 outputs: 64
+// workgroups) and what counts is the number of loads in flight over the chip.
+// Both operands come through LDS by asynchronous copies of whole 128-byte lines (8 rows x 128 bytes per wave-wide copy), each
+// wave in a ring of its own that runs D - 1 steps ahead, also into the workgroup's next tile: no barrier but the one around a
+// tile's sum.  Loading the fragments straight into registers touches 16 rows, 64 bytes each, per instruction, and the L1 then
+// delivers 12 bytes per clock: 18 us for 10576 x 2560 at 16 rows and 26 at 32 with the weights in the memory-side cache.
+// Slots of 16 bytes are swizzled by the row so that the 16 rows of a fragment read spread over all banks.
 enum { kOutBf16 = 0, kOutF32 = 1, kOutAdd = 2 };
-constexpr int kUN = 8;           // k steps of 32 in flight per wave
 
 struct LinearArgs {
     const bf16_t* w; const bf16_t* bias;
-    const void* x; int64_t x_sr;
-    const float* norm_w; const float* head_sq;
+    const bf16_t* x; int64_t x_sr;
+    const float* sq;                        // (M, nsq) sums of squares of the unscaled rows, or null: no scale
     void* out; int64_t out_sr;
-    int M, N, K, tiles, nheads, norm_groups;
+    const float* next_w; bf16_t* next_x; float* next_sq;      // kOutAdd: next norm's weight -> rows (M, N) and sums (M, tiles)
+    int M, N, K, tiles, nsq, groups;
     float eps;
     // conv states of the B and C channels, shifted here because every head of the scan in front of this reads them whole
     bf16_t* conv_state; const bf16_t* conv_in; int64_t conv_in_sb; int conv_c0, conv_cx, conv_W;
 };
 
-__device__ __forceinline__ bf16x8 as_frag(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
-__device__ __forceinline__ uint4 pack8(const float (&v)[8]) {
-    bf16x8 r;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = (bf16_t)v[e];
-    return __builtin_bit_cast(uint4, r);
+// Barrier for LDS traffic alone: the copies in flight stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
 }
 
-template <int XK, int NW>
-__device__ __forceinline__ void stage_rows(const LinearArgs& a, bf16_t* xs, float (*rs)[8], int ld) {
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    if constexpr (XK == kNorm) {
-        for (int m = wave; m < a.M; m += NW) {
-            const float* xr = static_cast<const float*>(a.x) + m * a.x_sr;
-            float ss = 0.f;
-            for (int k = lane * 4; k < a.K; k += 256) {
-                const floatx4 v = *reinterpret_cast<const floatx4*>(xr + k);
-                ss += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
-            }
-            const float rinv = rsqrtf(warp_sum(ss) / (float)a.K + a.eps);
-            for (int k = lane * 4; k < a.K; k += 256) {
-                const floatx4 v = *reinterpret_cast<const floatx4*>(xr + k), w = *reinterpret_cast<const floatx4*>(a.norm_w + k);
-                bf16x4 o;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = (bf16_t)(w[e] * (v[e] * rinv));
-                *reinterpret_cast<bf16x4*>(xs + m * ld + k) = o;
-            }
-        }
-        __syncthreads();
-    } else if constexpr (XK == kGated) {
-        const int hpg = a.nheads / a.norm_groups, gw = a.K / a.norm_groups;
-        for (int i = wave; i < a.M * a.norm_groups; i += NW) {
-            const int m = i / a.norm_groups, g = i - m * a.norm_groups;
-            float ss = 0.f;
-            for (int h = lane; h < hpg; h += 64) ss += a.head_sq[(int64_t)m * a.nheads + g * hpg + h];
-            ss = warp_sum(ss);
-            if (lane == 0) rs[m][g] = rsqrtf(ss / (float)gw + a.eps);
-        }
-        __syncthreads();
-        const int vecs = a.K / 8;
-        for (int i = tid; i < a.M * vecs; i += NW * 64) {
-            const int m = i / vecs, k = (i - m * vecs) * 8;
-            const float r = rs[m][k / gw];
-            float h[8], o[8];
-            cvt16<bf16_t>(*reinterpret_cast<const uint4*>(static_cast<const bf16_t*>(a.x) + m * a.x_sr + k), h);
-            const floatx4 w0 = *reinterpret_cast<const floatx4*>(a.norm_w + k), w1 = *reinterpret_cast<const floatx4*>(a.norm_w + k + 4);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] = (e < 4 ? w0[e & 3] : w1[e & 3]) * (h[e] * r);
-            *reinterpret_cast<uint4*>(xs + m * ld + k) = pack8(o);
-        }
-        __syncthreads();
-    }
-}
-
-template <int XK, int OK, int MT, int NW>
+template <int OK, int XR, int NW, int D>
 __global__ void __launch_bounds__(NW * 64)
 linear_small_kernel(const LinearArgs a) {
-    extern __shared__ __align__(16) char smem[];
-    __shared__ float red[NW][MT][256];
-    __shared__ float rs[XK == kGated ? 32 : 1][8];
-    bf16_t* xs = reinterpret_cast<bf16_t*>(smem);
-    const int ld = a.K + 8;                                  // rows 16 bytes apart in the banks
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r16 = lane & 15, kq = (lane >> 4) * 8;
-    const int steps = a.K / 32, s0 = steps * wave / NW, s1 = steps * (wave + 1) / NW;
-    const bf16_t* xrow[MT];
+    constexpr int MT = (XR + 1) / 2, SLOT = (2 + XR) * 1024, PER = 2 + XR;     // column tiles; bytes and copies of a step of 64 k
+    extern __shared__ __align__(1024) char ring_mem[];
+    __shared__ __align__(16) float red[NW][MT][256];
+    __shared__ float rs[32][8];
+    const int tid = threadIdx.x, wave = (int)uniform(tid >> 6), lane = tid & 63, r16 = lane & 15, q4 = lane >> 4;
+    const int steps = a.K / 64, s0 = steps * wave / NW, mine = steps * (wave + 1) / NW - s0;
+    const char* ring = ring_mem + wave * (D * SLOT);
+    const uint32_t ring_addr = uniform(lds_addr_of(ring));
+    // copies: lane i fills slot i & 7 of row i >> 3 with the row's chunk (slot ^ swizzle)
+    const int crow = lane >> 3;
+    auto chunk_off = [&](int row) { return (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) * 16); };
+    uint32_t xoff[XR];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        const int m = t * 16 + r16 < a.M ? t * 16 + r16 : 0;     // columns past M repeat a row and are not stored
-        xrow[t] = XK == kPlain ? static_cast<const bf16_t*>(a.x) + m * a.x_sr + kq : xs + m * ld + kq;
+    for (int j = 0; j < XR; ++j) {
+        const int row = j * 8 + crow;
+        xoff[j] = (uint32_t)((row < a.M ? row : a.M - 1) * a.x_sr * 2) + chunk_off(row);
     }
-    uint4 wa[kUN];
-    auto wrow = [&](int tile) {
-        const int n = tile * 16 + r16;
-        return a.w + (int64_t)(n < a.N ? n : a.N - 1) * a.K + kq;
-    };
-    const bf16_t* wp = wrow(blockIdx.x);
+    int itile = blockIdx.x, is = 0, islot = 0;               // the next step to issue
+    uint32_t woff[2];
+    auto tile_rows = [&](int tile) {
 #pragma unroll
-    for (int u = 0; u < kUN; ++u)
-        if (s0 + u < s1) wa[u] = *reinterpret_cast<const uint4*>(wp + (s0 + u) * 32);
-    stage_rows<XK, NW>(a, xs, rs, ld);
+        for (int j = 0; j < 2; ++j) {
+            const int row = j * 8 + crow, n = tile * 16 + row;
+            woff[j] = (uint32_t)((n < a.N ? row : a.N - 1 - tile * 16) * (int64_t)a.K * 2) + chunk_off(row);
+        }
+    };
+    tile_rows(itile);
+    auto issue = [&] {
+        const int64_t k0 = (int64_t)(s0 + is) * 64;
+        const bf16_t* wp = a.w + (int64_t)itile * 16 * a.K + k0;
+        const uint32_t dst = ring_addr + islot * SLOT;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) async_copy16(wp, woff[j], dst + j * 1024);
+#pragma unroll
+        for (int j = 0; j < XR; ++j) async_copy16(a.x + k0, xoff[j], dst + (2 + j) * 1024);
+        islot = islot + 1 == D ? 0 : islot + 1;
+        if (++is == mine) {
+            is = 0;
+            itile += gridDim.x;
+            if (itile < a.tiles) tile_rows(itile);
+        }
+    };
+    // the row scales: this wave's rows, their partial sums asked for ahead of everything and added up behind the first tile
+    constexpr int RU = 4, RV = 3;
+    const int per = a.sq ? a.nsq / a.groups : 0, nrs = a.sq ? a.M * a.groups : 0;
+    const bool early = nrs <= RU * NW && per <= RV * 64;
+    float part[RU][RV];
+#pragma unroll
+    for (int u = 0; u < RU; ++u)
+#pragma unroll
+        for (int v = 0; v < RV; ++v) {
+            const int i = wave + u * NW, q = v * 64 + lane;
+            part[u][v] = early && i < nrs && q < per ? a.sq[(int64_t)i * per + q] : 0.f;
+        }
+    // old values of the outputs that a thread adds to
+    constexpr int NO = (MT * 256 + NW * 64 - 1) / (NW * 64);
+    float old[NO], nw[NO];
+    auto fetch_old = [&](int tile) {
+        if constexpr (OK == kOutAdd) {
+#pragma unroll
+            for (int j = 0; j < NO; ++j) {
+                const int i = j * NW * 64 + tid, m = i >> 4, n = tile * 16 + (i & 15);
+                const bool own = i < MT * 256 && m < a.M && n < a.N;
+                old[j] = own ? static_cast<const float*>(a.out)[m * a.out_sr + n] : 0.f;
+                nw[j] = own && a.next_w ? a.next_w[n] : 0.f;
+            }
+        }
+    };
+    fetch_old(blockIdx.x);
+    const int total = mine * ((a.tiles - 1 - (int)blockIdx.x) / (int)gridDim.x + 1);
+    for (int j = 0; j < D - 1 && j < total; ++j) issue();
 
+    int done = 0, slot = 0;
     for (int tile = blockIdx.x; tile < a.tiles; tile += gridDim.x) {
         floatx4 acc[MT];
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-        const int next = tile + (int)gridDim.x;
-        const bf16_t* np = wrow(next < a.tiles ? next : tile);
-        for (int s = s0; s < s1; s += kUN) {
-            uint4 cur[kUN];
+        for (int s = 0; s < mine; ++s, ++done) {
+            // the slot that is filled now was read in the step before, whose products have its values
+            if (done + D - 1 < total) issue();
+            wait_vmem_keep<PER>(total - 1 - done < D - 1 ? total - 1 - done : D - 1);
+            const char* base = ring + slot * SLOT;
+            slot = slot + 1 == D ? 0 : slot + 1;
 #pragma unroll
-            for (int u = 0; u < kUN; ++u) cur[u] = wa[u];
-            // the next kUN steps of this tile, or the first ones of the workgroup's next tile
-            const bool more = s + kUN < s1;
-            const bf16_t* p = more ? wp : np;
-            const int f = more ? s + kUN : s0;
-            if (more || next < a.tiles) {
+            for (int kk = 0; kk < 2; ++kk) {
+                const int c = kk * 4 + q4;
+                const bf16x8 wf = *reinterpret_cast<const bf16x8*>(base + r16 * 128 + ((c ^ ((r16 >> 1) & 7)) * 16));
 #pragma unroll
-                for (int u = 0; u < kUN; ++u)
-                    if (f + u < s1) wa[u] = *reinterpret_cast<const uint4*>(p + (f + u) * 32);
-            }
-#pragma unroll
-            for (int u = 0; u < kUN; ++u) {
-                if (s + u >= s1) break;
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(cur[u]), as_frag(*reinterpret_cast<const uint4*>(xrow[t] + (s + u) * 32)),
-                                                                     acc[t], 0, 0, 0);
+                for (int t = 0; t < MT; ++t) {
+                    const int m = XR == 1 ? r16 & 7 : t * 16 + r16;
+                    const bf16x8 xf = *reinterpret_cast<const bf16x8*>(base + 2048 + m * 128 + ((c ^ ((m >> 1) & 7)) * 16));
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf, acc[t], 0, 0, 0);
+                }
             }
         }
-        wp = np;
+        const int next = tile + (int)gridDim.x;
         // lane: column m = lane & 15, rows n = 4 (lane >> 4) + 0..3
 #pragma unroll
-        for (int t = 0; t < MT; ++t) *reinterpret_cast<floatx4*>(&red[wave][t][r16 * 16 + (lane >> 4) * 4]) = acc[t];
-        __syncthreads();
-        for (int i = tid; i < MT * 256; i += NW * 64) {
-            const int m = i >> 4, n = tile * 16 + (i & 15);
-            float v = 0.f;
+        for (int t = 0; t < MT; ++t) *reinterpret_cast<floatx4*>(&red[wave][t][r16 * 16 + q4 * 4]) = acc[t];
+        if (a.sq && tile == (int)blockIdx.x) {
 #pragma unroll
-            for (int q = 0; q < NW; ++q) v += red[q][i >> 8][i & 255];
-            if (m < a.M && n < a.N) {
-                if (a.bias) v += to_f32(a.bias[n]);
-                const int64_t o = m * a.out_sr + n;
-                if (OK == kOutBf16) static_cast<bf16_t*>(a.out)[o] = (bf16_t)v;
-                else if (OK == kOutF32) static_cast<float*>(a.out)[o] = v;
-                else static_cast<float*>(a.out)[o] += v;
+            for (int u = 0; u < RU; ++u) {
+                const int i = wave + u * NW;
+                if (early && i < nrs) {
+                    const float v = warp_sum(part[u][0] + part[u][1] + part[u][2]);
+                    if (lane == 0) rs[i / a.groups][i % a.groups] = rsqrtf(v * (float)a.groups / (float)a.K + a.eps);
+                }
+            }
+            if (!early)
+                for (int i = wave; i < nrs; i += NW) {
+                    float v = 0.f;
+                    for (int q = lane; q < per; q += 64) v += a.sq[(int64_t)i * per + q];
+                    v = warp_sum(v);
+                    if (lane == 0) rs[i / a.groups][i % a.groups] = rsqrtf(v * (float)a.groups / (float)a.K + a.eps);
+                }
+        }
+        lds_barrier();
+#pragma unroll
+        for (int j = 0; j < NO; ++j) {
+            const int i = j * NW * 64 + tid, m = i >> 4, n = tile * 16 + (i & 15);
+            if (i >= MT * 256) break;                        // whole waves
+            const bool own = m < a.M && n < a.N;
+            float v = 0.f;
+            if (a.sq) {
+                const int wpg = NW / a.groups;               // waves per norm group: their K ranges lie inside one
+#pragma unroll
+                for (int q = 0; q < NW; ++q) v += red[q][i >> 8][i & 255] * rs[m][a.groups == 1 ? 0 : q / wpg];
+            } else {
+#pragma unroll
+                for (int q = 0; q < NW; ++q) v += red[q][i >> 8][i & 255];
+            }
+            const int64_t o = m * a.out_sr + n;
+            if (own && a.bias) v += to_f32(a.bias[n]);
+            if (OK == kOutBf16) {
+                if (own) static_cast<bf16_t*>(a.out)[o] = (bf16_t)v;
+            } else if (OK == kOutF32) {
+                if (own) static_cast<float*>(a.out)[o] = v;
+            } else {
+                v = own ? v + old[j] : 0.f;
+                if (own) static_cast<float*>(a.out)[o] = v;
+                if (a.next_w) {
+                    if (own) a.next_x[(int64_t)m * a.N + n] = (bf16_t)(v * nw[j]);
+                    float s = v * v;
+                    s = lane_xor_add<1>(s); s = lane_xor_add<2>(s); s = lane_xor_add<4>(s); s = lane_xor_add<8>(s);
+                    if ((i & 15) == 0 && m < a.M) a.next_sq[(int64_t)m * a.tiles + tile] = s;
+                }
             }
         }
-        __syncthreads();
+        if (next < a.tiles) {
+            fetch_old(next);
+            lds_barrier();
+        }
     }
     if (a.conv_state) {
         const int nch = a.conv_cx - a.conv_c0;
@@ -179,25 +219,65 @@ linear_small_kernel(const LinearArgs a) {
     }
 }
 
-constexpr size_t kLdsRows = 40 * 1024;       // normalised rows that fit beside the partial tiles in the 64 KB a launch may ask for
+// Waves per tile: eight where the tiles do not fill the chip by themselves, and for more than 16 rows, whose ring leaves room
+// for one workgroup per CU; else four.  A grouped norm needs every wave's share of K inside one group (0: no such split).
+int linear_waves(int64_t M, int64_t N, int64_t K, int64_t groups) {
+    const int64_t steps = K / 64;
+    const int want = (ceil_div(N, (int64_t)16) <= device_cus() || M > 16) && steps >= 8 ? 8 : 4;
+    if (groups == 1) return steps >= want ? want : (steps >= 4 ? 4 : 1);
+    for (const int nw : {want, 8, 4})
+        if (nw % groups == 0 && steps % nw == 0) return nw;
+    return 0;
+}
 
-template <int XK, int OK>
+template <int OK>
 int launch_linear(LinearArgs a, hipStream_t st) {
     a.tiles = (int)ceil_div(a.N, 16);
-    // eight waves per tile where the tiles do not fill the chip by themselves, four otherwise; workgroups that normalise
-    // rows take several tiles each once there are more than two per CU
-    const int64_t cus = device_cus();
-    const bool wide = a.tiles < 2 * cus && a.K >= 1024;
-    const int64_t most = XK == kPlain ? 4 * cus : 2 * cus;
-    const unsigned grid = (unsigned)(a.tiles < most ? a.tiles : most);
-    const size_t lds = XK == kPlain ? 0 : (size_t)a.M * (a.K + 8) * sizeof(bf16_t);
-    auto go = [&](auto mt) {
-        constexpr int MT = decltype(mt)::value;
-        if (wide) linear_small_kernel<XK, OK, MT, 8><<<grid, 512, lds, st>>>(a);
-        else linear_small_kernel<XK, OK, MT, 4><<<grid, 256, lds, st>>>(a);
+    const int nw = linear_waves(a.M, a.N, a.K, a.sq ? a.groups : 1);
+    int rc = M2_OK;
+    auto go = [&](auto xr, auto waves) {
+        constexpr int XR = decltype(xr)::value, NW = decltype(waves)::value, D = XR == 4 && NW == 8 ? 2 : 4;
+        constexpr size_t lds = (size_t)NW * D * (2 + XR) * 1024;
+        static_assert(lds + NW * ((XR + 1) / 2) * 1024 + 1024 <= 160 * 1024, "ring and partial tiles within the LDS of a CU");
+        // Two workgroups of four waves, or one of eight, per CU; each goes on to its next tile without draining its ring.
+        // (10576 x 2560, 1 / 8 / 16 rows, four waves: 12.1 / 12.9 / 14.8 us with 512 workgroups, 13.7 / 14.5 / 16.6 with one per
+        // tile; 32 rows, eight waves: 20.4 with 256, 23.8 with one per tile.)
+        const int64_t most = (NW == 8 ? 1 : 2) * device_cus();
+        const unsigned grid = (unsigned)(a.tiles < most ? a.tiles : most);
+        rc = allow_smem(linear_small_kernel<OK, XR, NW, D>, lds);
+        if (rc == M2_OK) linear_small_kernel<OK, XR, NW, D><<<grid, NW * 64, lds, st>>>(a);
     };
-    if (a.M <= 16) go(std::integral_constant<int, 1>{}); else go(std::integral_constant<int, 2>{});
-    return check_launch("linear_small_kernel");
+    auto rows = [&](auto waves) {
+        if (a.M <= 8) go(std::integral_constant<int, 1>{}, waves);
+        else if (a.M <= 16) go(std::integral_constant<int, 2>{}, waves);
+        else go(std::integral_constant<int, 4>{}, waves);
+    };
+    if (nw == 8) rows(std::integral_constant<int, 8>{});
+    else if (nw == 4) rows(std::integral_constant<int, 4>{});
+    else rows(std::integral_constant<int, 1>{});
+    return rc ? rc : check_launch("linear_small_kernel");
+}
+
+// The head of the chain: residual [+= delta], and the rows (residual times the norm's weight) with their sums of squares, as
+// linear_small leaves them behind a layer.  One workgroup per row.
+template <typename T>
+__global__ void __launch_bounds__(256)
+decode_rows_kernel(float* __restrict__ res, const T* __restrict__ add, int set, const float* __restrict__ w, bf16_t* __restrict__ x,
+                   float* __restrict__ sq, int64_t K) {
+    __shared__ float red[4];
+    const int64_t row = (int64_t)blockIdx.x * K;
+    float s = 0.f;
+    for (int64_t k = threadIdx.x; k < K; k += 256) {
+        float v = set ? 0.f : res[row + k];
+        if (add) v += to_f32(add[row + k]);
+        res[row + k] = v;
+        x[row + k] = (bf16_t)(v * w[k]);
+        s += v * v;
+    }
+    s = warp_sum(s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) sq[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // ------------------------------------------------------------------------------------------ conv + scan + gate
@@ -208,8 +288,8 @@ int launch_linear(LinearArgs a, hipStream_t st) {
 struct GatedArgs {
     float* S; const bf16_t* zx; int64_t zx_sb;            // [z | x | B | C | dt] row of a sequence
     bf16_t* conv_state; const void* conv_w; const void* conv_b;
-    const float *A, *D, *dt_bias;
-    bf16_t* h; float* head_sq;
+    const float *A, *D, *dt_bias, *norm_w;
+    bf16_t* h; float* head_sq;                            // w h (batch, heads * P) and sum of h^2 (batch, heads)
     int nheads, ngroups, conv_cx, W;
 };
 template <typename WT, int P, int N>
@@ -217,33 +297,52 @@ __global__ void __launch_bounds__(256)
 decode_gated_kernel(const GatedArgs a) {
     constexpr int GL = N / 4, ROWS = 256 / GL, UP = P / ROWS < 8 ? P / ROWS : 8, NCH = P + 2 * N;
     static_assert(P % (ROWS * UP) == 0, "whole passes over the state rows");
-    __shared__ float xa[P], za[P], Ba[N], Ca[N], ha[P], red[4];
+    constexpr int NI = (NCH + 255) / 256;
+    __shared__ __align__(16) float xa[P], za[P], Ba[N], Ca[N], ha[P], red[4];
     const int tid = threadIdx.x, h = blockIdx.x, b = blockIdx.y;
     const int g = h / (a.nheads / a.ngroups), d = a.nheads * P;
     const bf16_t* row = a.zx + b * a.zx_sb;
     float* Sp = a.S + ((int64_t)b * a.nheads + h) * (P * N);
     const int sub = tid % GL, rowi = tid / GL;
+    // all loads go out in the order in which they are used: the conv's, then the states
+    bf16_t hist[NI][3], in[NI], zin = (bf16_t)0.f;
+    float taps[NI][4], bias[NI];
+    auto channel = [&](int i) { return i < P ? h * P + i : (i < P + N ? d + g * N + (i - P) : d + (a.ngroups + g) * N + (i - P - N)); };
+#pragma unroll
+    for (int q = 0; q < NI; ++q) {
+        const int i = q * 256 + tid;
+        if (i < NCH) {
+            const int c = channel(i);
+            const bf16_t* cs = a.conv_state + ((int64_t)b * a.conv_cx + c) * a.W + a.W - 3;
+#pragma unroll
+            for (int j = 0; j < 3; ++j) hist[q][j] = cs[j];
+            in[q] = row[d + c];
+            loadv<WT, 4>(static_cast<const WT*>(a.conv_w) + c * 4, taps[q]);
+            bias[q] = a.conv_b ? to_f32(static_cast<const WT*>(a.conv_b)[c]) : 0.f;
+        }
+    }
+    float nw = 0.f;
+    if (tid < P) { zin = row[h * P + tid]; nw = a.norm_w[h * P + tid]; }
+    const float dtr = to_f32(row[d + a.conv_cx + h]) + (a.dt_bias ? a.dt_bias[h] : 0.f), Ah = a.A[h], Dh = a.D ? a.D[h] : 0.f;
     floatx4 sv[UP];
 #pragma unroll
     for (int u = 0; u < UP; ++u) sv[u] = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(Sp + (u * ROWS + rowi) * N + sub * 4));
-    const float dtv = softplus_f(to_f32(row[d + a.conv_cx + h]) + (a.dt_bias ? a.dt_bias[h] : 0.f));
-    const float dA = __expf(a.A[h] * dtv), Dh = a.D ? a.D[h] : 0.f;
-    for (int i = tid; i < NCH; i += 256) {
-        const int c = i < P ? h * P + i : (i < P + N ? d + g * N + (i - P) : d + (a.ngroups + g) * N + (i - P - N));
-        bf16_t* cs = a.conv_state + ((int64_t)b * a.conv_cx + c) * a.W;
-        const bf16_t in = row[d + c];
-        const WT* w = static_cast<const WT*>(a.conv_w) + c * 4;
-        const bf16_t o1 = cs[a.W - 3], o2 = cs[a.W - 2], o3 = cs[a.W - 1];
-        float z = a.conv_b ? to_f32(static_cast<const WT*>(a.conv_b)[c]) : 0.f;
-        z += to_f32(w[0]) * to_f32(o1) + to_f32(w[1]) * to_f32(o2) + to_f32(w[2]) * to_f32(o3) + to_f32(w[3]) * to_f32(in);
-        const float v = silu_f(z);
-        if (i < P) {
-            xa[i] = v;
-            za[i] = silu_f(to_f32(row[h * P + i]));
-            for (int j = 0; j + 1 < a.W; ++j) cs[j] = cs[j + 1];
-            cs[a.W - 1] = in;
-        } else if (i < P + N) Ba[i - P] = v;
-        else Ca[i - P - N] = v;
+    const float dtv = softplus_f(dtr), dA = __expf(Ah * dtv);
+#pragma unroll
+    for (int q = 0; q < NI; ++q) {
+        const int i = q * 256 + tid;
+        if (i < NCH) {
+            const float z = bias[q] + taps[q][0] * to_f32(hist[q][0]) + taps[q][1] * to_f32(hist[q][1]) + taps[q][2] * to_f32(hist[q][2]) + taps[q][3] * to_f32(in[q]);
+            const float v = silu_f(z);
+            if (i < P) {
+                xa[i] = v;
+                za[i] = silu_f(to_f32(zin));
+                bf16_t* cs = a.conv_state + ((int64_t)b * a.conv_cx + h * P + i) * a.W;
+                for (int j = 0; j < a.W - 3; ++j) cs[j] = cs[j + 1];
+                cs[a.W - 3] = hist[q][1]; cs[a.W - 2] = hist[q][2]; cs[a.W - 1] = in[q];
+            } else if (i < P + N) Ba[i - P] = v;
+            else Ca[i - P - N] = v;
+        }
     }
     __syncthreads();
     const floatx4 bv = *reinterpret_cast<const floatx4*>(Ba + sub * 4), cv = *reinterpret_cast<const floatx4*>(Ca + sub * 4);
@@ -270,7 +369,7 @@ decode_gated_kernel(const GatedArgs a) {
     float sq = 0.f;
     if (tid < P) {
         sq = ha[tid] * ha[tid];
-        a.h[(int64_t)b * d + h * P + tid] = (bf16_t)ha[tid];
+        a.h[(int64_t)b * d + h * P + tid] = (bf16_t)(ha[tid] * nw);
     }
     sq = warp_sum(sq);
     if ((tid & 63) == 0) red[tid >> 6] = sq;
@@ -281,17 +380,15 @@ decode_gated_kernel(const GatedArgs a) {
 int check_linear(const m2_linear_params* p) {
     M2_REQUIRE(p, M2_ERR_NULL, "linear_small: params is NULL");
     M2_REQUIRE(p->M >= 0 && p->N > 0 && p->K > 0, M2_ERR_SHAPE, "linear_small: M %lld, N %lld, K %lld", (long long)p->M, (long long)p->N, (long long)p->K);
-    M2_REQUIRE(m2_linear_small_fits(p->M, p->N, p->K, p->x_kind, p->norm_groups), M2_ERR_SHAPE,
-               "linear_small: M %lld, N %lld, K %lld, x kind %d: at most 32 rows, K a multiple of 32, normalised rows within 40 KB",
-               (long long)p->M, (long long)p->N, (long long)p->K, (int)p->x_kind);
+    M2_REQUIRE(m2_linear_small_fits(p->M, p->N, p->K, p->sq ? p->groups : 1), M2_ERR_SHAPE,
+               "linear_small: M %lld, N %lld, K %lld, %d groups: at most 32 rows, K a multiple of 64, whole K ranges per group",
+               (long long)p->M, (long long)p->N, (long long)p->K, (int)p->groups);
     if (p->M == 0) return M2_OK;
     M2_REQUIRE(p->x && p->w && p->out, M2_ERR_NULL, "linear_small: x, w and out are required");
-    M2_REQUIRE(p->x_kind == kPlain || p->norm_weight, M2_ERR_NULL, "linear_small: norm_weight is required");
-    M2_REQUIRE(p->x_kind != kGated || (p->head_sq && p->nheads > 0 && p->nheads % p->norm_groups == 0 && p->K % p->norm_groups == 0), M2_ERR_SHAPE,
-               "linear_small: gated rows need head_sq and whole heads per norm group");
-    const int64_t xv = p->x_kind == kNorm ? 4 : 8;
-    M2_REQUIRE(aligned16(p->x) && aligned16(p->w) && p->x_stride_row % xv == 0 && (!p->norm_weight || aligned16(p->norm_weight)), M2_ERR_ALIGN,
-               "linear_small: x rows, w and norm_weight must be 16-byte aligned");
+    M2_REQUIRE(!p->sq || (p->nsq > 0 && p->nsq % p->groups == 0), M2_ERR_SHAPE, "linear_small: %lld sums do not divide into %d groups", (long long)p->nsq, (int)p->groups);
+    M2_REQUIRE(p->out_kind >= kOutBf16 && p->out_kind <= kOutAdd && (!p->next_weight || (p->out_kind == kOutAdd && p->next_x && p->next_sq)), M2_ERR_NULL,
+               "linear_small: next_weight goes with out_kind 2, next_x and next_sq");
+    M2_REQUIRE(aligned16(p->x) && aligned16(p->w) && p->x_stride_row % 8 == 0, M2_ERR_ALIGN, "linear_small: x rows and w must be 16-byte aligned");
     return M2_OK;
 }
 
@@ -300,34 +397,40 @@ int launch_linear_params(const m2_linear_params* p, const LinearArgs& conv, hipS
     if (rc || p->M == 0) return rc;
     LinearArgs a = conv;
     a.w = static_cast<const bf16_t*>(p->w); a.bias = static_cast<const bf16_t*>(p->bias);
-    a.x = p->x; a.x_sr = p->x_stride_row; a.norm_w = p->norm_weight; a.head_sq = p->head_sq;
+    a.x = static_cast<const bf16_t*>(p->x); a.x_sr = p->x_stride_row; a.sq = p->sq; a.nsq = (int)p->nsq; a.groups = p->groups; a.eps = p->eps;
     a.out = p->out; a.out_sr = p->out_stride_row;
-    a.M = (int)p->M; a.N = (int)p->N; a.K = (int)p->K; a.nheads = (int)p->nheads; a.norm_groups = p->norm_groups; a.eps = p->eps;
-    auto out = [&](auto xk) {
-        constexpr int XK = decltype(xk)::value;
-        if (p->out_kind == kOutBf16) return launch_linear<XK, kOutBf16>(a, st);
-        if (p->out_kind == kOutF32) return launch_linear<XK, kOutF32>(a, st);
-        return launch_linear<XK, kOutAdd>(a, st);
-    };
-    if (p->x_kind == kPlain) return out(std::integral_constant<int, kPlain>{});
-    if (p->x_kind == kNorm) return out(std::integral_constant<int, kNorm>{});
-    return out(std::integral_constant<int, kGated>{});
+    a.next_w = p->next_weight; a.next_x = static_cast<bf16_t*>(p->next_x); a.next_sq = p->next_sq;
+    a.M = (int)p->M; a.N = (int)p->N; a.K = (int)p->K;
+    if (p->out_kind == kOutBf16) return launch_linear<kOutBf16>(a, st);
+    if (p->out_kind == kOutF32) return launch_linear<kOutF32>(a, st);
+    return launch_linear<kOutAdd>(a, st);
 }
 
 }  // namespace
 }  // namespace m2
 
-extern "C" int m2_linear_small_fits(int64_t M, int64_t N, int64_t K, int32_t x_kind, int32_t norm_groups) {
+extern "C" int m2_linear_small_fits(int64_t M, int64_t N, int64_t K, int32_t groups) {
     using namespace m2;
-    return M >= 0 && M <= 32 && N > 0 && N < (int64_t(1) << 30) && K > 0 && K % 32 == 0 && K <= (1 << 20) && x_kind >= kPlain && x_kind <= kGated &&
-           (x_kind == kPlain || (size_t)M * (K + 8) * sizeof(bf16_t) <= kLdsRows) && (x_kind != kGated || (norm_groups >= 1 && norm_groups <= 8 && K / norm_groups % 8 == 0));
+    return M >= 0 && M <= 32 && N > 0 && N < (int64_t(1) << 30) && K > 0 && K % 64 == 0 && K <= (1 << 20) && groups >= 1 && groups <= 8 &&
+           linear_waves(M, N, K, groups) > 0;
 }
 
 extern "C" int m2_linear_small(const m2_linear_params* p, void* stream) {
     return m2::launch_linear_params(p, m2::LinearArgs{}, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int m2_decode_layer(const m2_linear_params* in, const m2_decode_params* dec, const m2_linear_params* out, void* h, float* head_sq, void* stream) {
+extern "C" int m2_decode_rows(float* residual, const void* delta, int32_t delta_dtype, int32_t set, const float* weight, void* x, float* sq, int64_t rows,
+                              int64_t channels, void* stream) {
+    using namespace m2;
+    M2_REQUIRE(rows >= 0 && rows <= 65535 && channels > 0, M2_ERR_SHAPE, "decode_rows: rows %lld, channels %lld", (long long)rows, (long long)channels);
+    if (rows == 0) return M2_OK;
+    M2_REQUIRE(residual && weight && x && sq && (delta || !set), M2_ERR_NULL, "decode_rows: residual, weight, x and sq are required");
+    M2_DISPATCH_DTYPE(delta_dtype, T, (decode_rows_kernel<T><<<(unsigned)rows, 256, 0, static_cast<hipStream_t>(stream)>>>(
+                                          residual, static_cast<const T*>(delta), set, weight, static_cast<bf16_t*>(x), sq, channels)));
+    return check_launch("decode_rows_kernel");
+}
+
+extern "C" int m2_decode_layer(const m2_linear_params* in, const m2_decode_params* dec, const float* norm_weight, const m2_linear_params* out, void* stream) {
     using namespace m2;
     M2_REQUIRE(in && dec && out, M2_ERR_NULL, "decode_layer: params is NULL");
     const int64_t P = dec->headdim, N = dec->dstate, d = dec->nheads * P, cx = d + 2 * dec->ngroups * N;
@@ -336,11 +439,11 @@ extern "C" int m2_decode_layer(const m2_linear_params* in, const m2_decode_param
                "decode_layer: headdim %lld and dstate %lld must be 64 or 128, the conv 4 wide, the heads whole per group", (long long)P, (long long)N);
     M2_REQUIRE(dec->dtype == M2_BF16 && dec->activation == M2_ACT_SILU && (dec->param_dtype == M2_F32 || dec->param_dtype == M2_BF16), M2_ERR_DTYPE,
                "decode_layer: bf16 activations with SiLU only");
-    M2_REQUIRE(in->M == dec->batch && out->M == dec->batch && in->N == d + cx + dec->nheads && out->K == d && out->x_kind == kGated && in->out_kind == kOutBf16,
-               M2_ERR_SHAPE, "decode_layer: the projections do not match the layer");
+    M2_REQUIRE(in->M == dec->batch && out->M == dec->batch && in->N == d + cx + dec->nheads && out->K == d && in->out_kind == kOutBf16 && out->nsq == dec->nheads &&
+                   dec->batch <= 65535, M2_ERR_SHAPE, "decode_layer: the projections do not match the layer");
     if (dec->batch == 0) return M2_OK;
-    M2_REQUIRE(dec->conv_state && dec->conv_w && dec->S && dec->A && dec->dt_bias && h && head_sq, M2_ERR_NULL,
-               "decode_layer: conv_state, conv_w, S, A, dt_bias, h and head_sq are required");
+    M2_REQUIRE(dec->conv_state && dec->conv_w && dec->S && dec->A && dec->dt_bias && norm_weight && out->sq && out->x, M2_ERR_NULL,
+               "decode_layer: conv_state, conv_w, S, A, dt_bias, norm_weight, and the scratch behind out->x and out->sq are required");
     M2_REQUIRE(aligned16(dec->S), M2_ERR_ALIGN, "decode_layer: S must be 16-byte aligned");
     hipStream_t st = static_cast<hipStream_t>(stream);
     int rc = check_linear(out);
@@ -350,8 +453,8 @@ extern "C" int m2_decode_layer(const m2_linear_params* in, const m2_decode_param
     const bf16_t* zx = static_cast<const bf16_t*>(in->out);
     GatedArgs g{};
     g.S = dec->S; g.zx = zx; g.zx_sb = in->out_stride_row; g.conv_state = static_cast<bf16_t*>(dec->conv_state);
-    g.conv_w = dec->conv_w; g.conv_b = dec->conv_b; g.A = dec->A; g.D = dec->D; g.dt_bias = dec->dt_bias;
-    g.h = static_cast<bf16_t*>(h); g.head_sq = head_sq;
+    g.conv_w = dec->conv_w; g.conv_b = dec->conv_b; g.A = dec->A; g.D = dec->D; g.dt_bias = dec->dt_bias; g.norm_w = norm_weight;
+    g.h = static_cast<bf16_t*>(const_cast<void*>(out->x)); g.head_sq = const_cast<float*>(out->sq);
     g.nheads = (int)dec->nheads; g.ngroups = (int)dec->ngroups; g.conv_cx = (int)cx; g.W = dec->W;
     const dim3 grid((unsigned)dec->nheads, (unsigned)dec->batch);
     auto go = [&](auto wt, auto p, auto n) {

@@ -71,9 +71,9 @@ class RmsnormParams(C.Structure):
 
 
 class LinearParams(C.Structure):
-    _fields_ = [("x", _vp), ("w", _vp), ("bias", _vp), ("norm_weight", _vp), ("head_sq", _vp), ("out", _vp),
-                ("M", _i64), ("N", _i64), ("K", _i64), ("nheads", _i64), ("x_stride_row", _i64), ("out_stride_row", _i64),
-                ("x_kind", _i32), ("out_kind", _i32), ("norm_groups", _i32), ("eps", C.c_float)]
+    _fields_ = [("x", _vp), ("w", _vp), ("bias", _vp), ("sq", _vp), ("out", _vp), ("next_weight", _vp), ("next_x", _vp), ("next_sq", _vp),
+                ("M", _i64), ("N", _i64), ("K", _i64), ("nsq", _i64), ("x_stride_row", _i64), ("out_stride_row", _i64),
+                ("out_kind", _i32), ("groups", _i32), ("eps", C.c_float)]
 
 
 # name -> (restype, argtypes); every symbol the header declares
@@ -99,9 +99,10 @@ SYMBOLS = {
     "m2_rmsnorm_gated_bwd_workspace_bytes": (_sz, [_i64, _i64, _i32, _i32]),
     "m2_rmsnorm_gated_bwd": (C.c_int, [C.POINTER(RmsnormParams), _vp]),
     "m2_add_rmsnorm": (C.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, C.c_float, _i32, _vp]),
-    "m2_linear_small_fits": (C.c_int, [_i64, _i64, _i64, _i32, _i32]),
+    "m2_linear_small_fits": (C.c_int, [_i64, _i64, _i64, _i32]),
     "m2_linear_small": (C.c_int, [C.POINTER(LinearParams), _vp]),
-    "m2_decode_layer": (C.c_int, [C.POINTER(LinearParams), C.POINTER(DecodeParams), C.POINTER(LinearParams), _vp, _vp, _vp]),
+    "m2_decode_rows": (C.c_int, [_vp, _vp, _i32, _i32, _vp, _vp, _vp, _i64, _i64, _vp]),
+    "m2_decode_layer": (C.c_int, [C.POINTER(LinearParams), C.POINTER(DecodeParams), _vp, C.POINTER(LinearParams), _vp]),
     "m2_mixer_params": (C.c_int, [_vp, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _vp, _i64, _i64, _vp]),
     "m2_mixer_params_grads": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _i64, _i64, _vp]),
     "m2_mfma_selftest": (C.c_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp]),

@@ -181,16 +181,16 @@ class Mamba2Mixer(nn.Module):
         return (not torch.is_grad_enabled() and _plain_linear(self.in_proj) and _plain_linear(self.out_proj)
                 and type(self.norm) is MambaRMSNormGated and not torch.is_autocast_enabled())
 
-    def _step(self, cache_params, hidden=None, residual=None, delta=None, block_norm=None):
-        """One token through the layer: ``hidden`` (b, 1, D) -> the layer's output; or, with ``residual`` (fp32, in place), what is
-        still to be added to it and ``block_norm``, the whole block: residual += delta; mixer(norm(residual)) is added to the
-        residual as well (returns None) or comes back to be added."""
+    def _step(self, cache_params, hidden=None, stream=None, block_norm=None, next_norm=None):
+        """One token through the layer: ``hidden`` (b, 1, D) -> the layer's output; or, with a native residual ``stream``, the block
+        in it: stream += mixer(block_norm(stream)).  ``next_norm``: the norm module that reads the stream next."""
         A, D, dt_bias = self._inference_params()
         conv, norm, i = self.conv1d, self.norm, self.layer_idx
         weight, eps = (None, 0.0) if block_norm is None else (_lib.f32_param(block_norm.weight), block_norm.variance_epsilon)
-        return _lib.native().mixer_step(hidden, residual, delta, weight, eps, self.in_proj.weight, self.in_proj.bias, conv.weight, conv.bias, A, D, dt_bias,
-                                        _lib.f32_param(norm.weight), norm.eps, norm.n_groups if norm.rmsnorm_within_groups else 1, self.out_proj.weight,
-                                        self.out_proj.bias, cache_params.conv_states[i], cache_params.ssm_states[i], self.n_groups_tp)
+        return _lib.native().mixer_step(hidden, stream, weight, eps, None if next_norm is None else _lib.f32_param(next_norm.weight), self.in_proj.weight,
+                                        self.in_proj.bias, conv.weight, conv.bias, A, D, dt_bias, _lib.f32_param(norm.weight), norm.eps,
+                                        norm.n_groups if norm.rmsnorm_within_groups else 1, self.out_proj.weight, self.out_proj.bias,
+                                        cache_params.conv_states[i], cache_params.ssm_states[i], self.n_groups_tp)
 
     def step(self, hidden_states, cache_params: Optional[Mamba2Cache] = None):
         """hidden_states: (B, 1, D) -> same shape; updates the layer's conv and SSM state."""

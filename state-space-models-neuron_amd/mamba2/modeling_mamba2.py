@@ -58,7 +58,17 @@ class Mamba2Block(nn.Module):
                                    attention_mask=attention_mask)
         return residual + hidden_states
 
+    def _native_step(self):
+        """True if the block's step runs in a native fp32 residual stream."""
+        weight = self.norm.weight
+        return (self.residual_in_fp32 and type(self.norm) is Mamba2RMSNorm and self.mixer._native_step() and weight.is_cuda
+                and glue.add_rmsnorm_ok(weight.shape[0], self.mixer.in_proj.weight.dtype))
+
     def step(self, x, cache_params: Optional[Mamba2Cache] = None):
+        if self._native_step() and x.dtype in (torch.float32, torch.bfloat16):
+            stream = _lib.native().residual_stream(x)
+            self.mixer._step(cache_params, stream=stream, block_norm=self.norm)
+            return _lib.native().stream_sum(stream).view(x.shape)
         residual = x
         if self.residual_in_fp32:
             residual = residual.to(torch.float32)
@@ -170,28 +180,27 @@ class Mamba2Model(Mamba2PreTrainedModel):
     def step(self, input_ids, cache_params: Optional[Mamba2Cache] = None):
         """input_ids: int64 (batch, 1), one token per sequence -> hidden states (batch, 1, hidden) after the final norm.
         The caller advances ``cache_params.seqlen_offset`` (a host integer, so that a captured step stays replayable)."""
-        residual, delta = self._step_residual(input_ids, cache_params)
-        if residual is not None:
-            return glue.add_rmsnorm_(residual, delta, self.norm_f.weight, self.norm_f.variance_epsilon, self.layers[0].mixer.in_proj.weight.dtype)
+        stream = self._step_stream(input_ids, cache_params)
+        if stream is not None:
+            act = self.layers[0].mixer.in_proj.weight.dtype
+            rows = _lib.native().stream_norm(stream, _lib.f32_param(self.norm_f.weight), self.norm_f.variance_epsilon, act)
+            return rows.view(input_ids.shape[0], 1, -1)
         x = self.embeddings(input_ids)
         for mixer_block in self.layers:
             x = mixer_block.step(x, cache_params=cache_params)
         return self.norm_f(x)
 
-    def _step_residual(self, input_ids, cache_params):
-        """The fp32 residual stream (batch, 1, hidden) behind the last block and what is still to be added to it (or None), for
-        inference with ``residual_in_fp32``: each block's norm and residual add are part of its kernels or of one pass between
-        them (the same arithmetic as Mamba2Block.step, fp32 sums and norm).  (None, None) where the blocks have to be called one
-        by one."""
-        if not (self.config.residual_in_fp32 and len(self.layers) and all(blk.mixer._native_step() and type(blk.norm) is Mamba2RMSNorm for blk in self.layers)):
-            return None, None
-        x = self.embeddings(input_ids)
-        if not (x.is_cuda and glue.add_rmsnorm_ok(x.shape[-1], self.layers[0].mixer.in_proj.weight.dtype)):
-            return None, None
-        residual, delta = x.to(torch.float32, copy=True, memory_format=torch.contiguous_format), None
-        for mixer_block in self.layers:
-            delta = mixer_block.mixer._step(cache_params, residual=residual, delta=delta, block_norm=mixer_block.norm)
-        return residual, delta
+    def _step_stream(self, input_ids, cache_params):
+        """The native fp32 residual stream behind the last block, for inference with ``residual_in_fp32``: each block's norm and
+        residual add are part of its kernels or of one pass between them (the arithmetic of Mamba2Block.step: fp32 sums and
+        norm).  None where the blocks have to be called one by one."""
+        if not (len(self.layers) and type(self.norm_f) is Mamba2RMSNorm and all(blk._native_step() for blk in self.layers)):
+            return None
+        norms = [blk.norm for blk in self.layers] + [self.norm_f]
+        stream = _lib.native().residual_stream(self.embeddings(input_ids))
+        for i, mixer_block in enumerate(self.layers):
+            mixer_block.mixer._step(cache_params, stream=stream, block_norm=norms[i], next_norm=norms[i + 1])
+        return stream
 
 
 class Mamba2ForCausalLM(Mamba2PreTrainedModel):
@@ -241,10 +250,11 @@ class Mamba2ForCausalLM(Mamba2PreTrainedModel):
 
     def step(self, idx, cache_params: Optional[Mamba2Cache] = None):
         """idx: int64 (batch, 1) -> logits (batch, 1, vocab) fp32; the layers' states in ``cache_params`` advance by one token."""
-        residual, delta = self.backbone._step_residual(idx, cache_params) if _plain_linear(self.lm_head) else (None, None)
-        if residual is not None:
+        stream = self.backbone._step_stream(idx, cache_params) if _plain_linear(self.lm_head) and not torch.is_grad_enabled() else None
+        if stream is not None:
             norm_f = self.backbone.norm_f
-            return _lib.native().norm_linear(residual, delta, _lib.f32_param(norm_f.weight), norm_f.variance_epsilon, self.lm_head.weight, self.lm_head.bias)
+            logits = _lib.native().stream_norm_linear(stream, _lib.f32_param(norm_f.weight), norm_f.variance_epsilon, self.lm_head.weight, self.lm_head.bias)
+            return logits.view(idx.shape[0], 1, -1)
         hidden_states = self.backbone.step(idx, cache_params=cache_params)
         return self.lm_head(hidden_states.to(self.lm_head.weight.dtype)).float()
 

@@ -14,31 +14,37 @@ def _rel(got, ref):
     return ((got.double().cpu() - ref).norm() / ref.norm()).item()
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 5, 32), (3, 16, 96), (16, 33, 1024), (17, 100, 2560), (32, 4384, 1024), (8, 20000, 256)])
-@pytest.mark.parametrize("x_kind,out_kind", [(0, 0), (1, 1), (0, 2)])
-def test_linear_small(M, N, K, x_kind, out_kind):
+@pytest.mark.parametrize("M,N,K,groups", [(1, 5, 64, 1), (3, 16, 192, 1), (9, 40, 320, 1), (16, 33, 1024, 4), (17, 100, 2560, 8), (32, 4384, 1024, 1), (8, 20000, 256, 2),
+                                          (2, 256, 5120, 8)])
+@pytest.mark.parametrize("normed,out_kind", [(False, 0), (True, 1), (True, 2)])
+def test_linear_small(M, N, K, groups, normed, out_kind):
     from mamba2 import _lib
     lib = _lib.load()
-    if not lib.m2_linear_small_fits(M, N, K, x_kind, 1):
-        pytest.skip("normalised rows beyond the LDS limit take the separate norm")
+    assert lib.m2_linear_small_fits(M, N, K, groups)
     gen = torch.Generator().manual_seed(M + N)
     w = (torch.randn(N, K, generator=gen) / K ** 0.5).bfloat16().to(DEV)
     bias = torch.randn(N, generator=gen).bfloat16().to(DEV)
-    nw = (1 + 0.1 * torch.randn(K, generator=gen)).to(DEV)
-    x = torch.randn(M, K, generator=gen).to(DEV)
-    x = x if x_kind == 1 else x.bfloat16()
+    next_w = (1 + 0.1 * torch.randn(N, generator=gen)).to(DEV)
+    x = torch.randn(M, K, generator=gen).bfloat16().to(DEV)
+    sq = torch.rand(M, groups * 3, generator=gen).to(DEV) * K / 3 / groups
     base = torch.randn(M, N, generator=gen)
     out = base.bfloat16().to(DEV) if out_kind == 0 else base.to(DEV)
+    nx, nsq = torch.empty(M, N, dtype=torch.bfloat16, device=DEV), torch.empty(M, -(-N // 16), device=DEV)
     p = _lib.LinearParams()
-    p.x, p.w, p.bias, p.norm_weight, p.out = (_lib.ptr(t) for t in (x, w, bias, nw, out))
-    p.M, p.N, p.K, p.x_stride_row, p.out_stride_row, p.nheads, p.norm_groups = M, N, K, K, N, 1, 1
-    p.x_kind, p.out_kind, p.eps = x_kind, out_kind, 1e-5
+    p.x, p.w, p.bias, p.out = (_lib.ptr(t) for t in (x, w, bias, out))
+    p.M, p.N, p.K, p.x_stride_row, p.out_stride_row, p.groups, p.out_kind, p.eps = M, N, K, K, N, groups, out_kind, 1e-5
+    if normed:
+        p.sq, p.nsq = _lib.ptr(sq), groups * 3
+    if out_kind == 2:
+        p.next_weight, p.next_x, p.next_sq = _lib.ptr(next_w), _lib.ptr(nx), _lib.ptr(nsq)
     _lib.check(lib.m2_linear_small(p, _lib.stream_ptr()), "m2_linear_small")
-    xd = x.double().cpu()
-    if x_kind == 1:
-        xd = nw.double().cpu() * xd * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + 1e-5)
-    ref = xd @ w.double().cpu().T + bias.double().cpu() + (base.double() if out_kind == 2 else 0)
+    xd = x.double().cpu().view(M, groups, K // groups)
+    if normed:
+        xd = xd * torch.rsqrt(sq.double().cpu().view(M, groups, 3).sum(-1, keepdim=True) * groups / K + 1e-5)
+    ref = xd.reshape(M, K) @ w.double().cpu().T + bias.double().cpu() + (base.double() if out_kind == 2 else 0)
     assert _rel(out, ref) < 5e-3
+    if out_kind == 2:
+        assert _rel(nx, ref * next_w.double().cpu()) < 5e-3 and _rel(nsq.sum(1), ref.pow(2).sum(1)) < 1e-3
 
 
 @pytest.mark.parametrize("b,h,p,n,g,W,groups_norm", [(1, 8, 64, 128, 1, 4, True), (3, 6, 64, 64, 2, 3, True), (16, 4, 128, 64, 1, 4, False),
@@ -69,16 +75,15 @@ def test_layer_step_against_oracle(b, h, p, n, g, W, groups_norm, block):
         got = blk.step(x, cache_params=cache) if block else m.step(x.bfloat16(), cache_params=cache)
     assert _rel(got, ref + xin if block else ref) < 2e-2
     assert _rel(cache.conv_states[0], cs) < 5e-3 and _rel(cache.ssm_states[0], S) < 1e-2
-    # the residual form: the block inside Mamba2Model.step
+    # the same block inside a model's residual stream, chained into itself
     if block:
-        for t, r in ((cache.conv_states[0], cs), (cache.ssm_states[0], S)):
-            assert torch.isfinite(t).all()
-        c2 = Mamba2Cache(cfg, b, dtype=torch.bfloat16, device=DEV, conv_width=W)
-        c3 = Mamba2Cache(cfg, b, dtype=torch.bfloat16, device=DEV, conv_width=W)
+        from mamba2 import _lib
+        c2, c3 = (Mamba2Cache(cfg, b, dtype=torch.bfloat16, device=DEV, conv_width=W) for _ in range(2))
         with torch.no_grad():
-            res = x.clone()
-            delta = m._step(c2, residual=res, block_norm=blk.norm)
-            want = blk.step(x, cache_params=c3)
-        res = res if delta is None else res + delta
-        assert _rel(res, want.double().cpu()) < 5e-3
+            stream = _lib.native().residual_stream(x)
+            for _ in range(2):
+                m._step(c2, stream=stream, block_norm=blk.norm, next_norm=blk.norm)
+            got = _lib.native().stream_norm(stream, _lib.f32_param(blk.norm.weight), blk.norm.variance_epsilon, torch.bfloat16)
+            want = blk.norm(blk.step(blk.step(x, cache_params=c3), cache_params=c3))
+        assert _rel(got.view(b, 1, hidden), want.double().cpu()) < 1e-2
         assert _rel(c2.ssm_states[0], c3.ssm_states[0].double().cpu()) < 1e-2
