@@ -14,6 +14,15 @@
 namespace m2 {
 
 constexpr int kQ = M2_CHUNK;   // 128 tokens per chunk
+constexpr int kP = 64;         // channels of a head as the SSD kernels see it
+
+// A head of 128 channels is two kernel heads of 64 (HS = 1): they share dt, A, D, B and C, their states and channels lie one
+// behind the other, and every per-head sum is linear in the channels, so only the final sums (da_body) know of the pair.
+// Element offset of kernel head h in a tensor whose true heads are `sh` elements apart.  (A template argument, not a value:
+// one more scalar per tensor in the head loops sends kernel arguments back to memory, and their reloads wait for the LDS
+// traffic around them: 340 -> 347 us for forward + backward at b4 l2048 h80.)
+template <int HS>
+__device__ __forceinline__ int64_t head_off(int64_t h, int64_t sh) { return HS ? (h >> 1) * sh + (h & 1) * kP : h * sh; }
 
 template <typename T> struct MmaTraits;
 template <> struct MmaTraits<bf16_t> { static constexpr int kPad = 8; };

@@ -52,7 +52,7 @@ namespace {
 template <typename T, int P>
 constexpr bool dg_g_in_lds() { return (size_t)14 * kQ * sizeof(float) + ((size_t)2 * kQ * lds_ld<T>(P) + (size_t)kQ * lds_ld<T>(kQ)) * sizeof(T) <= 150 * 1024; }
 
-template <typename T, int P>
+template <typename T, int P, int HS>
 __global__ void __launch_bounds__(512, 2)
 dg_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
           const T* __restrict__ dY, const T* __restrict__ Gm, float* __restrict__ dGp, float* __restrict__ dl_diag,
@@ -93,8 +93,8 @@ dg_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
     static_assert((kQ * VPR) % 512 == 0, "tile does not divide over the workgroup");
     uint4 pdy[NV], pxx[NV];
     auto prefetch = [&](int64_t h) {
-        const T* gy = dY + b * dYsb + t0 * dYsl + h * dYsh;
-        const T* gx = X + b * Xsb + t0 * Xsl + h * Xsh;
+        const T* gy = dY + b * dYsb + t0 * dYsl + head_off<HS>(h, dYsh);
+        const T* gx = X + b * Xsb + t0 * Xsl + head_off<HS>(h, Xsh);
 #pragma unroll
         for (int it = 0; it < NV; ++it) {
             const int e = it * 512 + tid, rr = e / VPR, cv = e % VPR;
@@ -194,7 +194,7 @@ dg_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
 template <typename T, int P, int N>
 constexpr bool off_c_in_lds() { return (size_t)10 * kQ * sizeof(float) + ((size_t)(kQ + N) * lds_ld<T>(P) + (size_t)kQ * lds_ld<T>(N)) * sizeof(T) <= 150 * 1024; }
 
-template <typename T, int P, int N, bool SIDE_C>
+template <typename T, int P, int N, bool SIDE_C, int HS>
 __global__ void __launch_bounds__(512, SIDE_C ? 2 : 4)
 off_kernel(const T* __restrict__ Arow, int64_t Asb, int64_t Asl, int64_t Ash,      // dY (C side) or X (B side)
            const float* __restrict__ ldtab,
@@ -235,7 +235,7 @@ off_kernel(const T* __restrict__ Arow, int64_t Asb, int64_t Asl, int64_t Ash,   
     static_assert((kQ * VPR) % 512 == 0 && (P * VPS) % 512 == 0, "tile does not divide over the workgroup");
     uint4 pa[NVA], ps[NVS];
     auto prefetch = [&](int64_t h) {
-        const T* ga = Arow + b * Asb + t0 * Asl + h * Ash;
+        const T* ga = Arow + b * Asb + t0 * Asl + head_off<HS>(h, Ash);
 #pragma unroll
         for (int it = 0; it < NVA; ++it) {
             const int e = it * 512 + tid, rr = e / VPR, cv = e % VPR;
@@ -330,8 +330,6 @@ __device__ __forceinline__ void slice_sum_body(const SliceSumArgs& a, int64_t bl
     for (int64_t sl = 0; sl < sg.nslices; ++sl) s += *reinterpret_cast<const floatx4*>(sg.part + (grp * sg.nslices + sl) * sg.tile + e);
     *reinterpret_cast<floatx4*>(sg.out + grp * sg.tile + e) = s;
 }
-__global__ void __launch_bounds__(256)
-slice_sum_kernel(const SliceSumArgs a) { slice_sum_body<256>(a, blockIdx.x); }
 // The slice sums and the per-chunk decay-gradient scan (da_body) in one launch: they are independent, and both are short.
 template <typename T>
 __global__ void __launch_bounds__(kDaHeads * 64)
@@ -595,8 +593,8 @@ size_t off_smem(bool side_c) { return (size_t)(8 * kQ + 2 * kQ) * sizeof(float) 
 template <typename T, int N>
 size_t bcf_smem() { return sizeof(T) == 2 ? (size_t)2 * kQ * kQ * sizeof(T) : (size_t)(kQ + N) * lds_ld<T>(kQ) * sizeof(T); }
 
-template <typename T, int P, int N>
-int ssd_bwd_impl(const m2_ssd_params* p, hipStream_t st) {
+template <typename T, int P, int N, int HS>
+int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
     const int64_t nc = ceil_div(p->seqlen, (int64_t)kQ);
     const SsdWorkspace w = ssd_carve(p, p->workspace, true);
     const int dt_f32 = p->dt_dtype == M2_F32;
@@ -609,24 +607,22 @@ int ssd_bwd_impl(const m2_ssd_params* p, hipStream_t st) {
     M2_REQUIRE(p->nheads <= 65535, M2_ERR_SHAPE, "ssd_bwd: too many group slices");
     int rc;
     // decay tables, G (+ operand tiles) and the state entering each chunk, unless the caller kept the forward's
-    if (!p->chunk_states && (rc = ssd_launch_states<T, P, N>(p, w, nullptr, st))) return rc;
+    if (!p->chunk_states && (rc = ssd_launch_states<T, P, N, HS>(p, w, nullptr, st))) return rc;
     // gradient of the state leaving each chunk (reverse recurrence over the chunks' own contributions)
     if constexpr (sizeof(T) == 2) {
-        // the main backward kernel forms dlam itself when it runs; otherwise this pass does (and reads the forward states for it)
         constexpr int SPLIT = kStatePassSplit;
-        auto k = state_pass16_kernel<T, P, N, true, !bwd16_ok<T, P, N>(), false, SPLIT>;
+        auto k = state_pass16_kernel<T, P, N, true, HS, false, SPLIT>;
         const size_t sm = state_pass_smem<P, N, false, SPLIT>();
         if ((rc = allow_smem(k, sm))) return rc;
         StatePassArgs sa;
         sa.X = dy; sa.X_sb = p->dy_stride_b; sa.X_sl = p->dy_stride_l; sa.X_sh = p->dy_stride_h;
         sa.ldtab = w.ldtab; sa.Mt = w.Ct; sa.init = p->d_final_state; sa.prev = w.dprev; sa.final_out = p->d_initial_state;
-        sa.sprev = w.prev; sa.dlam = w.dlam;
         sa.seqlen = p->seqlen; sa.nheads = p->nheads; sa.ngroups = p->ngroups; sa.nchunks = nc;
         k<<<dim3((unsigned)(p->nheads * SPLIT), (unsigned)p->batch), state_pass_threads<N>(), sm, st>>>(sa);
         if ((rc = check_launch("ssd state_pass16_kernel<reverse>"))) return rc;
     } else
     {   // fp32: local dS contributions (reuses the `local` region), then the reverse recurrence
-        auto k = chunk_state_kernel<T, P, N, true>;
+        auto k = chunk_state_kernel<T, P, N, true, HS>;
         const size_t sm = state_smem<T, P, N>();
         if ((rc = allow_smem(k, sm))) return rc;
         int64_t ns, hps;
@@ -641,8 +637,8 @@ int ssd_bwd_impl(const m2_ssd_params* p, hipStream_t st) {
         if ((rc = check_launch("ssd state_scan_kernel<reverse>"))) return rc;
     }
     {
-        if constexpr (sizeof(T) == 2 && dg16_smem<P>() <= 160 * 1024) {
-            auto k = dg16_kernel<T, P>;
+        if constexpr (sizeof(T) == 2) {
+            auto k = dg16_kernel<T, P, HS>;
             const size_t sm = dg16_smem<P>();
             if ((rc = allow_smem(k, sm))) return rc;
             k<<<grid_g, kDgWaves * 64, sm, st>>>(x, w.ldtab, dy, w.G, w.dGp, w.dl,
@@ -650,7 +646,7 @@ int ssd_bwd_impl(const m2_ssd_params* p, hipStream_t st) {
                                        p->x_stride_b, p->x_stride_l, p->x_stride_h,
                                        p->dy_stride_b, p->dy_stride_l, p->dy_stride_h);
         } else {
-            auto k = dg_kernel<T, P>;
+            auto k = dg_kernel<T, P, HS>;
             const size_t sm = dg_smem<T, P>();
             if ((rc = allow_smem(k, sm))) return rc;
             k<<<grid_g, 512, sm, st>>>(x, w.ldtab, dy, static_cast<const T*>(w.Gm), w.dGp, w.dl,
@@ -660,12 +656,26 @@ int ssd_bwd_impl(const m2_ssd_params* p, hipStream_t st) {
         }
         if ((rc = check_launch("ssd dg_kernel"))) return rc;
     }
-    DaArgs da{};
-    bool have_da = false;
-    {
-        if constexpr (!bwd16_ok<T, P, N>()) {
-        auto kc = off_kernel<T, P, N, true>;
-        auto kb = off_kernel<T, P, N, false>;
+    if constexpr (sizeof(T) == 2) {
+        Bwd16Args m{};
+        m.ldtab = w.ldtab; m.D = p->D;
+        m.Bm = p->B; m.B_sb = p->B_stride_b; m.B_sl = p->B_stride_l; m.B_sg = p->B_stride_g;
+        m.Cm = p->C; m.C_sb = p->C_stride_b; m.C_sl = p->C_stride_l; m.C_sg = p->C_stride_g;
+        m.Gmt = w.Gmt; m.dS = w.dprev; m.Sprev = w.prev;
+        m.dy = p->dy; m.dy_sb = p->dy_stride_b; m.dy_sl = p->dy_stride_l; m.dy_sh = p->dy_stride_h;
+        m.x = p->x; m.x_sb = p->x_stride_b; m.x_sl = p->x_stride_l; m.x_sh = p->x_stride_h;
+        m.dx = p->dx; m.dx_sb = p->dx_stride_b; m.dx_sl = p->dx_stride_l; m.dx_sh = p->dx_stride_h;
+        m.dirp = w.dirp; m.rbp = w.rbp; m.dlc = w.dlc; m.dDp8 = w.dDp8; m.dlam = w.dlam; m.dBp = w.dBp; m.dCp = w.dCp;
+        m.seqlen = p->seqlen; m.nheads = p->nheads; m.ngroups = p->ngroups; m.nchunks = nc;
+        m.nslices = w.ns_b; m.hps = w.hps_b;
+        auto k = ssd_bwd16_kernel<T, P, N, HS>;
+        const size_t sm = bwd16_smem<P, N>();
+        if ((rc = allow_smem(k, sm))) return rc;
+        k<<<grid_b, 512, sm, st>>>(m);
+        if ((rc = check_launch("ssd_bwd16_kernel"))) return rc;
+    } else {
+        auto kc = off_kernel<T, P, N, true, HS>;
+        auto kb = off_kernel<T, P, N, false, HS>;
         const size_t smc = off_smem<T, P, N>(true), sm = off_smem<T, P, N>(false);
         if ((rc = allow_smem(kc, smc))) return rc;
         if ((rc = allow_smem(kb, sm))) return rc;
@@ -677,56 +687,30 @@ int ssd_bwd_impl(const m2_ssd_params* p, hipStream_t st) {
                                     static_cast<const T*>(w.dprev), nullptr, 0, 0, 0,
                                     w.dBp, nullptr, p->seqlen, p->nheads, p->ngroups, nc, w.ns_b, w.hps_b);
         if ((rc = check_launch("ssd off_kernel<B>"))) return rc;
-        }
-    }
-    {
         DiagArgs a{};
-        a.dt = p->dt; a.dt_f32 = dt_f32; a.A = p->A; a.D = p->D;
+        a.D = p->D;
         a.Aoff = p->B; a.Ao_sb = p->B_stride_b; a.Ao_sl = p->B_stride_l; a.Ao_sg = p->B_stride_g;
         a.Gd = w.Gmt; a.S = w.dprev;
         a.Z = p->dy; a.Z_sb = p->dy_stride_b; a.Z_sl = p->dy_stride_l; a.Z_sh = p->dy_stride_h;
-        a.dt_sb = p->dt_stride_b; a.dt_sl = p->dt_stride_l;
         a.seqlen = p->seqlen; a.nheads = p->nheads; a.ngroups = p->ngroups; a.nchunks = nc;
         ssd_slicing(p, 2, &a.nslices, &a.hps);
         a.X = p->x; a.X_sb = p->x_stride_b; a.X_sl = p->x_stride_l; a.X_sh = p->x_stride_h;
         a.dX = p->dx; a.dX_sb = p->dx_stride_b; a.dX_sl = p->dx_stride_l; a.dX_sh = p->dx_stride_h;
-        a.ddt = p->ddt; a.ddt_sb = p->ddt_stride_b; a.ddt_sl = p->ddt_stride_l;
         a.ldtab = w.ldtab;
-        a.dl_diag = w.dl; a.dl_c = w.dlc; a.dlam = w.dlam; a.dAp = w.dAp; a.dDp = w.dDp;
-        a.dbp = p->dt_bias ? w.dbp : nullptr;
-        const dim3 grid((unsigned)nc, (unsigned)(p->ngroups * a.nslices), (unsigned)p->batch);
-        if constexpr (bwd16_ok<T, P, N>()) {
-            Bwd16Args m{};
-            m.ldtab = w.ldtab; m.D = p->D;
-            m.Bm = p->B; m.B_sb = p->B_stride_b; m.B_sl = p->B_stride_l; m.B_sg = p->B_stride_g;
-            m.Cm = p->C; m.C_sb = p->C_stride_b; m.C_sl = p->C_stride_l; m.C_sg = p->C_stride_g;
-            m.Gmt = w.Gmt; m.dS = w.dprev; m.Sprev = w.prev;
-            m.dy = p->dy; m.dy_sb = p->dy_stride_b; m.dy_sl = p->dy_stride_l; m.dy_sh = p->dy_stride_h;
-            m.x = p->x; m.x_sb = p->x_stride_b; m.x_sl = p->x_stride_l; m.x_sh = p->x_stride_h;
-            m.dx = p->dx; m.dx_sb = p->dx_stride_b; m.dx_sl = p->dx_stride_l; m.dx_sh = p->dx_stride_h;
-            m.dirp = w.dirp; m.rbp = w.rbp; m.dlc = w.dlc; m.dDp8 = w.dDp8; m.dlam = w.dlam; m.dBp = w.dBp; m.dCp = w.dCp;
-            m.seqlen = p->seqlen; m.nheads = p->nheads; m.ngroups = p->ngroups; m.nchunks = nc;
-            m.nslices = w.ns_b; m.hps = w.hps_b;
-            auto k = ssd_bwd16_kernel<T, P, N>;
-            const size_t sm = bwd16_smem<P, N>();
-            if ((rc = allow_smem(k, sm))) return rc;
-            k<<<grid_b, 512, sm, st>>>(m);
-            if ((rc = check_launch("ssd_bwd16_kernel"))) return rc;
-            // the per-chunk scan that turns these per-token terms into ddt and dA partials runs with the slice sums below
-            have_da = true;
-            da.ldtab = w.ldtab; da.A = p->A; da.dl_diag = w.dl; da.dl_c = w.dlc; da.dlam = w.dlam;
-            da.dirp = w.dirp; da.rbp = w.rbp; da.dDp8 = w.dDp8;
-            da.ddt = p->ddt; da.dt_f32 = dt_f32; da.ddt_sb = p->ddt_stride_b; da.ddt_sl = p->ddt_stride_l; da.dAp = w.dAp; da.dDp = w.dDp;
-            da.dbp = p->dt_bias ? w.dbp : nullptr;
-            da.seqlen = p->seqlen; da.nheads = p->nheads; da.nchunks = nc; da.batch = p->batch;
-        } else {
-            auto k = diag_off_kernel<T, P, N, true>;
-            const size_t sm = diag_smem<T, P, N, true>();
-            if ((rc = allow_smem(k, sm))) return rc;
-            k<<<grid, 256, sm, st>>>(a);
-        }
+        a.dirp = w.dirp; a.rbp = w.rbp; a.dDp8 = w.dDp8;
+        auto k = diag_off_kernel<T, P, N, true, HS>;
+        const size_t smd = diag_smem<T, P, N, true>();
+        if ((rc = allow_smem(k, smd))) return rc;
+        k<<<dim3((unsigned)nc, (unsigned)(p->ngroups * a.nslices), (unsigned)p->batch), 256, smd, st>>>(a);
         if ((rc = check_launch("ssd diag_off_kernel<bwd>"))) return rc;
     }
+    // the per-chunk scan that turns the per-token terms into ddt and dA partials runs with the slice sums below
+    DaArgs da{};
+    da.ldtab = w.ldtab; da.A = p->A; da.dl_diag = w.dl; da.dl_c = w.dlc; da.dlam = w.dlam;
+    da.dirp = w.dirp; da.rbp = w.rbp; da.dDp8 = w.dDp8;
+    da.ddt = p->ddt; da.dt_f32 = dt_f32; da.ddt_sb = p->ddt_stride_b; da.ddt_sl = p->ddt_stride_l; da.dAp = w.dAp; da.dDp = w.dDp;
+    da.dbp = p->dt_bias ? w.dbp : nullptr;
+    da.seqlen = p->seqlen; da.nheads = p->true_heads; da.nchunks = nc; da.batch = p->batch; da.hs = p->hs;
     {
         const int64_t ngrp = p->batch * nc * p->ngroups;
         const float *gs = w.dGp, *cs = w.dCp, *bs = w.dBp;
@@ -743,12 +727,8 @@ int ssd_bwd_impl(const m2_ssd_params* p, hipStream_t st) {
             add(w.dCp, w.dCs, w.ns_c, (int64_t)kQ * N, &cs);
             add(w.dBp, w.dBs, w.ns_b, (int64_t)kQ * N, &bs);
             sa.total = first;
-            if (have_da) {
-                const int64_t n_da = da_blocks(da), n_ss = ceil_div(first, (int64_t)(kDaHeads * 64));
-                tail1_kernel<T><<<(unsigned)(n_da + n_ss), kDaHeads * 64, 0, st>>>(da, n_da, sa);
-            } else if (first > 0) {
-                slice_sum_kernel<<<(unsigned)ceil_div(first, (int64_t)256), 256, 0, st>>>(sa);
-            }
+            const int64_t n_da = da_blocks(da), n_ss = ceil_div(first, (int64_t)(kDaHeads * 64));
+            tail1_kernel<T><<<(unsigned)(n_da + n_ss), kDaHeads * 64, 0, st>>>(da, n_da, sa);
         }
         if ((rc = check_launch("ssd tail1_kernel"))) return rc;
         // 16-bit operands: one workgroup per (batch, chunk, group) once those alone fill the chip, one per side below that
@@ -763,8 +743,8 @@ int ssd_bwd_impl(const m2_ssd_params* p, hipStream_t st) {
         ta.dCsb = p->dC_stride_b; ta.dCsl = p->dC_stride_l; ta.dCsg = p->dC_stride_g;
         ta.dAp = w.dAp; ta.dDp = w.dDp; ta.dbp = w.dbp; ta.dA = p->dA; ta.dD = p->D ? p->dD : nullptr;
         ta.dbias = p->dt_bias ? p->d_dt_bias : nullptr;
-        ta.seqlen = p->seqlen; ta.ngroups = p->ngroups; ta.nchunks = nc; ta.batch = p->batch; ta.nheads = p->nheads; ta.n_bc = ngrp;
-        k<<<(unsigned)((both ? 1 : 2) * ngrp + p->nheads), 512, sm, st>>>(ta);
+        ta.seqlen = p->seqlen; ta.ngroups = p->ngroups; ta.nchunks = nc; ta.batch = p->batch; ta.nheads = p->true_heads; ta.n_bc = ngrp;
+        k<<<(unsigned)((both ? 1 : 2) * ngrp + p->true_heads), 512, sm, st>>>(ta);
         if ((rc = check_launch("ssd tail2_kernel"))) return rc;
     }
     return M2_OK;
@@ -775,7 +755,8 @@ int ssd_bwd_impl(const m2_ssd_params* p, hipStream_t st) {
 
 extern "C" size_t m2_ssd_bwd_workspace_bytes(const m2_ssd_params* p) {
     if (!p || p->batch <= 0 || p->seqlen <= 0 || p->nheads <= 0) return 256;
-    return m2::ssd_carve(p, nullptr, true).bytes;
+    const m2::SsdCall q(p);
+    return m2::ssd_carve(&q, nullptr, true).bytes;
 }
 
 extern "C" int m2_ssd_bwd(const m2_ssd_params* p, void* stream) {
@@ -812,6 +793,7 @@ extern "C" int m2_ssd_bwd(const m2_ssd_params* p, void* stream) {
     M2_REQUIRE(p->workspace && p->workspace_bytes >= need, M2_ERR_WORKSPACE, "ssd_bwd: workspace %zu bytes < %zu needed",
                p->workspace_bytes, need);
     M2_REQUIRE((reinterpret_cast<uintptr_t>(p->workspace) & 255u) == 0, M2_ERR_ALIGN, "ssd_bwd: workspace must be 256-byte aligned");
-    M2_DISPATCH_DTYPE(p->dtype, T, M2_DISPATCH_PN(p, P, N, return (ssd_bwd_impl<T, P, N>(p, st))));
+    const SsdCall q(p);
+    M2_DISPATCH_DTYPE(p->dtype, T, M2_DISPATCH_N_HS(&q, N, HS, return (ssd_bwd_impl<T, kP, N, HS>(&q, st))));
     return M2_OK;
 }

@@ -35,8 +35,6 @@ constexpr size_t bwd16_smem() {
     return (size_t)2 * ((2 * P * N + 2 * kQ * P) * 2 + 2 * kQ * sizeof(float)) + (size_t)4 * (kQ + 32) * sizeof(float) +
            (size_t)4 * bwd16_clds<N>() * 4 * 64 * sizeof(uint2);
 }
-template <typename T, int P, int N>
-constexpr bool bwd16_ok() { return sizeof(T) == 2 && bwd16_smem<P, N>() <= 160 * 1024; }
 
 struct Bwd16Args {
     const float* ldtab;                                   // [b][h][c][ l kQ | dt kQ ]
@@ -55,7 +53,7 @@ struct Bwd16Args {
     int64_t seqlen, nheads, ngroups, nchunks, nslices, hps;
 };
 
-template <typename T, int P, int N>
+template <typename T, int P, int N, int HS>
 __global__ void __launch_bounds__(512, 1)
 ssd_bwd16_kernel(const Bwd16Args a) {
     static_assert(sizeof(T) == 2, "16-bit operands only");
@@ -111,8 +109,8 @@ ssd_bwd16_kernel(const Bwd16Args a) {
             async_copy16(Sp, off, dst + ch * 1024u);
             async_copy16(Pp, off, dst + (uint32_t)(P * N * 2) + ch * 1024u);
         }
-        const T* Yp = static_cast<const T*>(a.dy) + b * a.dy_sb + t0 * a.dy_sl + h * a.dy_sh;
-        const T* Xp = static_cast<const T*>(a.x) + b * a.x_sb + t0 * a.x_sl + h * a.x_sh;
+        const T* Yp = static_cast<const T*>(a.dy) + b * a.dy_sb + t0 * a.dy_sl + head_off<HS>(h, a.dy_sh);
+        const T* Xp = static_cast<const T*>(a.x) + b * a.x_sb + t0 * a.x_sl + head_off<HS>(h, a.x_sh);
         const uint32_t ypitch = uniform((uint32_t)a.dy_sl * 2u), xpitch = uniform((uint32_t)a.x_sl * 2u), last = (uint32_t)(valid - 1);
 #pragma unroll
         for (int it = 0; it < NX; ++it) {
@@ -172,7 +170,7 @@ ssd_bwd16_kernel(const Bwd16Args a) {
             const int64_t h = h_first + hh;
             const int buf = (int)(hh & 1);
             const int64_t bhc = (b * a.nheads + h) * a.nchunks + c;
-            const float Dh = a.D ? a.D[h] : 0.f;
+            const float Dh = a.D ? a.D[h >> HS] : 0.f;
 
             wait_vmem_all();          // this wave's share of the tiles of head hh, and the whole [ l | dt ] table, have landed
             const float* sl = sLD + buf * 2 * kQ;
@@ -277,7 +275,7 @@ ssd_bwd16_kernel(const Bwd16Args a) {
             // ---- epilogue: dx = dt_j dxd + D dy, dir_j = sum_p dxd x, dD partial = sum dy x.  One lane-pair swap per
             //      4-channel group leaves every lane with whole groups of 8 consecutive channels of its token: 16-byte
             //      reads of x and dy, 16-byte stores of dx, no pass through LDS
-            T* dXp = static_cast<T*>(a.dx) + b * a.dx_sb + t0 * a.dx_sl + h * a.dx_sh + (int64_t)tok * a.dx_sl;
+            T* dXp = static_cast<T*>(a.dx) + b * a.dx_sb + t0 * a.dx_sl + head_off<HS>(h, a.dx_sh) + (int64_t)tok * a.dx_sl;
             const float dts = sd[tok] * fin_sc;      // the block's final scale rides on dt here and on the finished row sum below
             float dir = 0.f, dd = 0.f;
 #pragma unroll
@@ -441,7 +439,8 @@ struct DaArgs {
     const float* dirp; const float* rbp; const float* dDp8;
     void* ddt; int dt_f32; int64_t ddt_sb, ddt_sl; float* dAp; float* dDp;
     float* dbp;            // with softplus folded into the scan: [b][h][c] partials of d_dt_bias, and ddt is w.r.t. the raw dt; else null
-    int64_t seqlen, nheads, nchunks, batch;
+    int64_t seqlen, nheads, nchunks, batch;      // nheads: true heads, each the sum of its 1 << hs kernel heads
+    int hs;
 };
 inline int64_t da_blocks(const DaArgs& q) { return q.batch * q.nchunks * ((q.nheads + kDaHeads - 1) / kDaHeads); }
 template <typename T>
@@ -463,14 +462,21 @@ __device__ __forceinline__ void da_body(const DaArgs& q, int64_t blk) {
     if (h < nheads) {      // wave-uniform
         const int64_t bhc = (b * nheads + h) * nchunks + c;
         const float Ah = A[h];
-        float xa = dl_diag[bhc * kQ + ta] + dl_c[bhc * kQ + ta];
-        float xb = dl_diag[bhc * kQ + tb] + dl_c[bhc * kQ + tb];
-        const float ra = rbp[bhc * kQ + ta], rbv = rbp[bhc * kQ + tb];
-        const float dira = dirp[bhc * kQ + ta], dirb = dirp[bhc * kQ + tb];
-        const float dta = ldtab[bhc * 2 * kQ + kQ + ta], dtb = ldtab[bhc * 2 * kQ + kQ + tb];     // 0 past the end of the sequence
-        float dlm = 0.f;
+        float xa = 0.f, xb = 0.f, ra = 0.f, rbv = 0.f, dira = 0.f, dirb = 0.f, dlm = 0.f, dDs = 0.f;
+        const int nv = 1 << q.hs;
+        for (int v = 0; v < nv; ++v) {
+            const int64_t k = ((b * nheads + h) * nv + v) * nchunks + c;
+            xa += dl_diag[k * kQ + ta] + dl_c[k * kQ + ta];
+            xb += dl_diag[k * kQ + tb] + dl_c[k * kQ + tb];
+            ra += rbp[k * kQ + ta]; rbv += rbp[k * kQ + tb];
+            dira += dirp[k * kQ + ta]; dirb += dirp[k * kQ + tb];
 #pragma unroll
-        for (int sp = 0; sp < kDlamParts; ++sp) dlm += dlam[bhc * kDlamParts + sp];
+            for (int sp = 0; sp < kDlamParts; ++sp) dlm += dlam[k * kDlamParts + sp];
+#pragma unroll
+            for (int w = 0; w < 8; ++w) dDs += dDp8[k * 8 + w];
+        }
+        const float* tab = ldtab + ((b * nheads + h) * nv * nchunks + c) * (2 * kQ) + kQ;
+        const float dta = tab[ta], dtb = tab[tb];     // 0 past the end of the sequence
         float ya = ra, yb = rbv;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -502,10 +508,7 @@ __device__ __forceinline__ void da_body(const DaArgs& q, int64_t blk) {
         if (lane == 0) {
             dAp[bhc] = dAl;
             if (dbp) dbp[bhc] = dbl;
-            float s = 0.f;
-#pragma unroll
-            for (int w = 0; w < 8; ++w) s += dDp8[bhc * 8 + w];
-            dDp[bhc] = s;
+            dDp[bhc] = dDs;
         }
     }
     __syncthreads();

@@ -23,7 +23,7 @@ constexpr int dg16_ring() { return (size_t)4 * (2 * kQ * P * 2 + 1024) + 8 * 102
 template <int P>
 constexpr size_t dg16_smem() { return (size_t)dg16_ring<P>() * (2 * kQ * P * 2 + 2 * kQ * sizeof(float)) + (size_t)(2 * 8 * kQ + kDgWaves * 32) * sizeof(float); }
 
-template <typename T, int P>
+template <typename T, int P, int HS>
 __global__ void __launch_bounds__(kDgWaves * 64)
 dg16_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
             const T* __restrict__ dY, const float* __restrict__ Gf, float* __restrict__ dGp, float* __restrict__ dl_diag,
@@ -69,8 +69,8 @@ dg16_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
     }
     auto issue_tiles = [&](int64_t h, int buf) {
         if (copier) {
-            const T* gy = dY + b * dYsb + t0 * dYsl + h * dYsh;
-            const T* gx = X + b * Xsb + t0 * Xsl + h * Xsh;
+            const T* gy = dY + b * dYsb + t0 * dYsl + head_off<HS>(h, dYsh);
+            const T* gx = X + b * Xsb + t0 * Xsl + head_off<HS>(h, Xsh);
             const uint32_t dst = lds_T + (uint32_t)(buf * 2 * TILE * 2);
 #pragma unroll
             for (int it = 0; it < NX; ++it) {

@@ -28,7 +28,7 @@ constexpr float kMaxRange = 80.f;
 
 struct DiagArgs {
     // common
-    const void* dt; int dt_f32; const float* A; const float* D;
+    const float* D;
     const float* ldtab;         // [b][h][c][ l kQ | dt kQ ]
     const void* Aoff;           // C (fwd) or B (bwd): [b][l][g][N]
     int64_t Ao_sb, Ao_sl, Ao_sg;
@@ -36,32 +36,29 @@ struct DiagArgs {
     const void* S;              // [b][c][h][P][N]
     const void* Z;              // x (fwd) or dy (bwd): [b][l][h][P]
     int64_t Z_sb, Z_sl, Z_sh;
-    int64_t dt_sb, dt_sl;
     int64_t seqlen, nheads, ngroups, nchunks, nslices, hps;
     // forward
     void* Y; int64_t Y_sb, Y_sl, Y_sh;
     // backward
     const void* X; int64_t X_sb, X_sl, X_sh;
     void* dX; int64_t dX_sb, dX_sl, dX_sh;
-    void* ddt; int64_t ddt_sb, ddt_sl;
-    const float* dl_diag; const float* dl_c; const float* dlam;   // [b][h][c][kQ], [b][h][c][kQ], [b][h][c]
-    float* dAp; float* dDp;                                       // [b][h][c]
-    float* dbp;            // softplus folded into the scan: [b][h][c] partials of d_dt_bias (ddt is then w.r.t. the raw dt), else null
+    float* dirp; float* rbp;                        // [b][h][c][kQ]: dxd . x;  B . dBoff
+    float* dDp8;                                    // [b][h][c][8]
 };
 
 // The backward keeps a transposed copy of x in LDS for its epilogue when that fits (always for bf16);
 // otherwise it reads x from global memory there.
 template <typename T, int P, int N>
 constexpr bool diag_xt_in_lds() {
-    return (size_t)(4 * 4 * kQ + 2 * kQ + 8) * sizeof(float) + ((size_t)P * lds_ld<T>(N) + (size_t)2 * P * lds_ld<T>(kQ)) * sizeof(T) <= 150 * 1024;
+    return (size_t)(4 * 4 * kQ) * sizeof(float) + ((size_t)P * lds_ld<T>(N) + (size_t)2 * P * lds_ld<T>(kQ)) * sizeof(T) <= 150 * 1024;
 }
 template <typename T, int P, int N, bool BWD>
 constexpr size_t diag_smem() {
-    return (size_t)(4 * 4 * kQ + (BWD ? 2 * kQ + 8 : 0)) * sizeof(float) +
+    return (size_t)(4 * 4 * kQ) * sizeof(float) +
            ((size_t)P * lds_ld<T>(N) + (size_t)((BWD && diag_xt_in_lds<T, P, N>()) ? 2 : 1) * P * lds_ld<T>(kQ)) * sizeof(T);
 }
 
-template <typename T, int P, int N, bool BWD>
+template <typename T, int P, int N, bool BWD, int HS>
 __global__ void __launch_bounds__(256, 2)
 diag_off_kernel(const DiagArgs a) {
     constexpr int LDN = lds_ld<T>(N), LDQ = lds_ld<T>(kQ);
@@ -69,10 +66,7 @@ diag_off_kernel(const DiagArgs a) {
     constexpr bool XT = BWD && diag_xt_in_lds<T, P, N>();
     extern __shared__ __align__(16) unsigned char smem_raw[];
     float* wt_all = reinterpret_cast<float*>(smem_raw);              // [4 waves][4 tables][kQ]
-    float* s_dir = wt_all + 4 * 4 * kQ;                              // BWD: [kQ] dxd . x
-    float* s_rb = s_dir + (BWD ? kQ : 0);                            // BWD: [kQ] B . dBoff
-    float* s_red = s_rb + (BWD ? kQ : 0);                            // BWD: [8]
-    T* sS = reinterpret_cast<T*>(s_red + (BWD ? 8 : 0));             // [P][LDN]
+    T* sS = reinterpret_cast<T*>(wt_all + 4 * 4 * kQ);               // [P][LDN]
     T* sZt = sS + P * LDN;                                           // [P][LDQ]
     T* sXt = sZt + P * LDQ;                                          // BWD: [P][LDQ]
 
@@ -106,12 +100,12 @@ diag_off_kernel(const DiagArgs a) {
 
     for (int64_t hh = 0; hh < a.hps; ++hh) {
         const int64_t h = g * hpg + slice * a.hps + hh;
-        const float Ah = a.A[h];
-        const float Dh = a.D ? a.D[h] : 0.f;
+        const float Dh = a.D ? a.D[h >> HS] : 0.f;
+        const int64_t bhc = (b * a.nheads + h) * a.nchunks + c;
 
         // ---- wave-private cumulative sum and decay tables
         float l0, l1, d0, d1;
-        wave_ld_load(a.ldtab, (b * a.nheads + h) * a.nchunks + c, l0, l1, d0, d1);
+        wave_ld_load(a.ldtab, bhc, l0, l1, d0, d1);
         // l at the first / last token of this wave's row block (tokens 32w, 32w+31) and at the chunk end
         const float l_first = wave < 2 ? __shfl(l0, row0, 64) : __shfl(l1, row0 - 64, 64);
         const float l_last = wave < 2 ? __shfl(l0, row0 + 31, 64) : __shfl(l1, row0 + 31 - 64, 64);
@@ -141,13 +135,13 @@ diag_off_kernel(const DiagArgs a) {
         const int64_t tile = ((b * a.nchunks + c) * a.nheads + h) * (int64_t)(P * N);
         __syncthreads();          // every wave is done with the previous head's tiles
         stage_rows<T, P, N, 256, false>(sS, LDN, static_cast<const T*>(a.S) + tile, N, P, nullptr, tid);
-        stage_transposed<T, kQ, P, 256, false>(sZt, LDQ, static_cast<const T*>(a.Z) + b * a.Z_sb + t0 * a.Z_sl + h * a.Z_sh, a.Z_sl,
+        stage_transposed<T, kQ, P, 256, false>(sZt, LDQ, static_cast<const T*>(a.Z) + b * a.Z_sb + t0 * a.Z_sl + head_off<HS>(h, a.Z_sh), a.Z_sl,
                                                valid, nullptr, tid);
         if (XT)
-            stage_transposed<T, kQ, P, 256, false>(sXt, LDQ, static_cast<const T*>(a.X) + b * a.X_sb + t0 * a.X_sl + h * a.X_sh,
+            stage_transposed<T, kQ, P, 256, false>(sXt, LDQ, static_cast<const T*>(a.X) + b * a.X_sb + t0 * a.X_sl + head_off<HS>(h, a.X_sh),
                                                    a.X_sl, valid, nullptr, tid);
         __syncthreads();
-        const T* Xg = BWD ? static_cast<const T*>(a.X) + b * a.X_sb + t0 * a.X_sl + h * a.X_sh : nullptr;
+        const T* Xg = BWD ? static_cast<const T*>(a.X) + b * a.X_sb + t0 * a.X_sl + head_off<HS>(h, a.X_sh) : nullptr;
         // x[row0 + 8q + 4 half + e][col], e = 0..3, at this lane's accumulator positions
         auto load_x4 = [&](int q, int col, T (&xv)[4]) {
             if (XT) *reinterpret_cast<RawVec<T, 4>*>(xv) = *reinterpret_cast<const RawVec<T, 4>*>(sXt + col * LDQ + row0 + 8 * q + 4 * half);
@@ -213,7 +207,7 @@ diag_off_kernel(const DiagArgs a) {
             int ri;
             const float tot = half_wave_reduce16(rbv, &ri);
             const int row = row0 + acc_row(lane, ri);
-            if ((lane & 1) == 0) s_rb[row] = tot * wd[row];
+            if ((lane & 1) == 0) a.rbp[bhc * kQ + row] = tot * wd[row];
         }
 
         // ---- diagonal term: A fragment = masked CB^T fragment scaled by the decay table along k
@@ -247,7 +241,7 @@ diag_off_kernel(const DiagArgs a) {
 
         // ---- epilogue
         if (!BWD) {
-            T* Yp = static_cast<T*>(a.Y) + b * a.Y_sb + t0 * a.Y_sl + h * a.Y_sh;
+            T* Yp = static_cast<T*>(a.Y) + b * a.Y_sb + t0 * a.Y_sl + head_off<HS>(h, a.Y_sh);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
 #pragma unroll
@@ -264,7 +258,7 @@ diag_off_kernel(const DiagArgs a) {
                 }
             }
         } else {
-            T* dXp = static_cast<T*>(a.dX) + b * a.dX_sb + t0 * a.dX_sl + h * a.dX_sh;
+            T* dXp = static_cast<T*>(a.dX) + b * a.dX_sb + t0 * a.dX_sl + head_off<HS>(h, a.dX_sh);
             float dirv[16];
             float dD_loc = 0.f;
 #pragma unroll
@@ -291,57 +285,9 @@ diag_off_kernel(const DiagArgs a) {
             }
             int ri;
             const float tot = half_wave_reduce16(dirv, &ri);
-            if ((lane & 1) == 0) s_dir[row0 + acc_row(lane, ri)] = tot;
+            if ((lane & 1) == 0) a.dirp[bhc * kQ + row0 + acc_row(lane, ri)] = tot;
             dD_loc = warp_sum(dD_loc);
-            if (lane == 0) s_red[wave] = dD_loc;
-            __syncthreads();      // s_dir, s_rb, s_red complete; also the "tiles are free" barrier for the next head
-            if (wave == 0) {
-                // da_t = sum_{i>=t} (dl_diag_i + dl_c_i) + sum_{j<t} rb_j + dlam;  lanes hold the tokens in reverse
-                // order (127-lane, 63-lane), so the suffix over tokens is an inclusive prefix over lanes and the
-                // exclusive prefix over tokens an exclusive suffix over lanes.
-                const int64_t bhc = (b * a.nheads + h) * a.nchunks + c;
-                const int ta = kQ - 1 - lane, tb = 63 - lane;
-                float xa = a.dl_diag[bhc * kQ + ta] + a.dl_c[bhc * kQ + ta];
-                float xb = a.dl_diag[bhc * kQ + tb] + a.dl_c[bhc * kQ + tb];
-                const float ra = s_rb[ta], rbv = s_rb[tb];
-                float ya = ra, yb = rbv;
-#pragma unroll
-                for (int o = 1; o < 64; o <<= 1) {
-                    const float na = __shfl_up(xa, o, 64), nb = __shfl_up(xb, o, 64);
-                    const float ma = __shfl_down(ya, o, 64), mb = __shfl_down(yb, o, 64);
-                    if (lane >= o) { xa += na; xb += nb; }
-                    if (lane + o < 64) { ya += ma; yb += mb; }
-                }
-                xb += __shfl(xa, 63, 64);
-                xa += (ya - ra) + __shfl(yb, 0, 64);
-                xb += yb - rbv;
-                float dlm = 0.f;
-#pragma unroll
-                for (int sp = 0; sp < kDlamParts; ++sp) dlm += a.dlam[bhc * kDlamParts + sp];
-                const float da_a = xa + dlm, da_b = xb + dlm;
-                float dAl = 0.f, dbl = 0.f;
-                if (ta < valid) {
-                    float val = Ah * da_a + s_dir[ta];
-                    if (a.dbp) { val *= softplus_grad_of_value(wd[ta]); dbl += val; }      // wd = softplus(raw dt + bias)
-                    const int64_t o = b * a.ddt_sb + (t0 + ta) * a.ddt_sl + h;
-                    if (a.dt_f32) static_cast<float*>(a.ddt)[o] = val; else static_cast<T*>(a.ddt)[o] = from_f32<T>(val);
-                    dAl += da_a * wd[ta];
-                }
-                if (tb < valid) {
-                    float val = Ah * da_b + s_dir[tb];
-                    if (a.dbp) { val *= softplus_grad_of_value(wd[tb]); dbl += val; }
-                    const int64_t o = b * a.ddt_sb + (t0 + tb) * a.ddt_sl + h;
-                    if (a.dt_f32) static_cast<float*>(a.ddt)[o] = val; else static_cast<T*>(a.ddt)[o] = from_f32<T>(val);
-                    dAl += da_b * wd[tb];
-                }
-                dAl = warp_sum(dAl);
-                if (a.dbp) dbl = warp_sum(dbl);
-                if (lane == 0) {
-                    if (a.dbp) a.dbp[bhc] = dbl;
-                    a.dAp[bhc] = dAl;
-                    a.dDp[bhc] = s_red[0] + s_red[1] + s_red[2] + s_red[3];
-                }
-            }
+            if (lane == 0) { a.dDp8[bhc * 8 + wave] = dD_loc; a.dDp8[bhc * 8 + wave + 4] = 0.f; }
         }
     }
 }

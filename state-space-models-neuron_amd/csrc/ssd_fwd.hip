@@ -25,35 +25,35 @@ __global__ void copy_or_zero_kernel(const float* __restrict__ src, float* __rest
     if (i < n) dst[i] = src ? src[i] : 0.f;
 }
 
-template <typename T, int P, int N>
-int ssd_fwd_impl(const m2_ssd_params* p, hipStream_t st) {
+template <typename T, int P, int N, int HS>
+int ssd_fwd_impl(const SsdCall* p, hipStream_t st) {
     const int64_t nc = ceil_div(p->seqlen, (int64_t)kQ);
     const SsdWorkspace w = ssd_carve(p, p->workspace, false);
     int rc;
-    if ((rc = ssd_launch_states<T, P, N>(p, w, p->final_state, st))) return rc;
+    if ((rc = ssd_launch_states<T, P, N, HS>(p, w, p->final_state, st))) return rc;
     DiagArgs a{};
-    a.dt = p->dt; a.dt_f32 = p->dt_dtype == M2_F32; a.A = p->A; a.D = p->D;
+    a.D = p->D;
     a.Aoff = p->C; a.Ao_sb = p->C_stride_b; a.Ao_sl = p->C_stride_l; a.Ao_sg = p->C_stride_g;
     a.Gd = w.Gm; a.S = w.prev; a.ldtab = w.ldtab;
     a.Z = p->x; a.Z_sb = p->x_stride_b; a.Z_sl = p->x_stride_l; a.Z_sh = p->x_stride_h;
-    a.dt_sb = p->dt_stride_b; a.dt_sl = p->dt_stride_l;
     a.seqlen = p->seqlen; a.nheads = p->nheads; a.ngroups = p->ngroups; a.nchunks = nc;
     ssd_slicing(p, kWgsY, &a.nslices, &a.hps);
     a.Y = p->y; a.Y_sb = p->y_stride_b; a.Y_sl = p->y_stride_l; a.Y_sh = p->y_stride_h;
     M2_REQUIRE(p->ngroups * a.nslices <= 65535, M2_ERR_SHAPE, "ssd_fwd: too many group slices");
     const dim3 grid((unsigned)nc, (unsigned)(p->ngroups * a.nslices), (unsigned)p->batch);
-    if constexpr (sizeof(T) == 2 && y16_smem<P, N>() <= 160 * 1024) {
-        auto k = ssd_y16_kernel<T, P, N>;
+    if constexpr (sizeof(T) == 2) {
+        auto k = ssd_y16_kernel<T, P, N, HS>;
         const size_t sm = y16_smem<P, N>();
         if ((rc = allow_smem(k, sm))) return rc;
         k<<<grid, 256, sm, st>>>(a);
         return check_launch("ssd_y16_kernel");
-    }
-    auto k = diag_off_kernel<T, P, N, false>;
+    } else {
+    auto k = diag_off_kernel<T, P, N, false, HS>;
     const size_t sm = diag_smem<T, P, N, false>();
     if ((rc = allow_smem(k, sm))) return rc;
     k<<<grid, 256, sm, st>>>(a);
     return check_launch("ssd diag_off_kernel<fwd>");
+    }
 }
 
 }  // namespace
@@ -61,12 +61,14 @@ int ssd_fwd_impl(const m2_ssd_params* p, hipStream_t st) {
 
 extern "C" size_t m2_ssd_chunk_states_bytes(const m2_ssd_params* p) {
     if (!p || p->batch <= 0 || p->seqlen <= 0 || p->nheads <= 0) return 0;
-    return m2::ssd_carve(p, nullptr, false, true).kept_bytes;
+    const m2::SsdCall q(p);
+    return m2::ssd_carve(&q, nullptr, false, true).kept_bytes;
 }
 
 extern "C" size_t m2_ssd_fwd_workspace_bytes(const m2_ssd_params* p) {
     if (!p || p->batch <= 0 || p->seqlen <= 0 || p->nheads <= 0) return 256;
-    return m2::ssd_carve(p, nullptr, false).bytes;
+    const m2::SsdCall q(p);
+    return m2::ssd_carve(&q, nullptr, false).bytes;
 }
 
 extern "C" int m2_ssd_fwd(const m2_ssd_params* p, void* stream) {
@@ -93,6 +95,7 @@ extern "C" int m2_ssd_fwd(const m2_ssd_params* p, void* stream) {
     M2_REQUIRE(p->workspace && p->workspace_bytes >= need, M2_ERR_WORKSPACE, "ssd_fwd: workspace %zu bytes < %zu needed",
                p->workspace_bytes, need);
     M2_REQUIRE((reinterpret_cast<uintptr_t>(p->workspace) & 255u) == 0, M2_ERR_ALIGN, "ssd_fwd: workspace must be 256-byte aligned");
-    M2_DISPATCH_DTYPE(p->dtype, T, M2_DISPATCH_PN(p, P, N, return (ssd_fwd_impl<T, P, N>(p, st))));
+    const SsdCall q(p);
+    M2_DISPATCH_DTYPE(p->dtype, T, M2_DISPATCH_N_HS(&q, N, HS, return (ssd_fwd_impl<T, kP, N, HS>(&q, st))));
     return M2_OK;
 }

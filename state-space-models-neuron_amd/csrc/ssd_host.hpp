@@ -8,6 +8,16 @@
 
 namespace m2 {
 
+// A call as the kernels see it: heads of kP channels, hs = 1 where a true head is two of them (see head_off; the HS of the kernels).
+struct SsdCall : m2_ssd_params {
+    int hs;
+    int64_t true_heads;
+    explicit SsdCall(const m2_ssd_params* p) : m2_ssd_params(*p), hs(p->headdim > kP ? 1 : 0), true_heads(p->nheads) {
+        nheads <<= hs;
+        headdim = kP;
+    }
+};
+
 // Workspace regions.  Forward uses G, local, prev, lam.  Backward additionally uses
 // dprev (gradient w.r.t. the state leaving each chunk, operand type), dlam, dl (per-token gradient of the in-chunk cumulative
 // sum, per head), per-(b,h,chunk) partials of dA and dD, and
@@ -30,7 +40,7 @@ struct SsdWorkspace {
 // group stay on chip, group-level reductions happen in registers).  The slice count is the smallest divisor of
 // heads-per-group that gives at least `wgs_per_cu` workgroups per compute unit: the grid then fills the GPU in one
 // round of long-running workgroups (measured: fewer, longer workgroups beat more, shorter ones for every kernel).
-inline void ssd_slicing(const m2_ssd_params* p, int wgs_per_cu, int64_t* nslices, int64_t* hps) {
+inline void ssd_slicing(const SsdCall* p, int wgs_per_cu, int64_t* nslices, int64_t* hps) {
     const int64_t nc = ceil_div(p->seqlen, (int64_t)kQ);
     const int64_t hpg = p->nheads / p->ngroups;
     const int64_t base = p->batch * nc * p->ngroups;
@@ -46,7 +56,7 @@ inline void ssd_slicing(const m2_ssd_params* p, int wgs_per_cu, int64_t* nslices
 }
 constexpr int kWgsChunkState = 2, kWgsY = 2, kWgsDx = 1, kWgsDg = 1, kWgsOffC = 1, kWgsOffB = 2;
 
-inline SsdWorkspace ssd_carve(const m2_ssd_params* p, void* base, bool bwd, bool kept_only = false) {
+inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_only = false) {
     const int64_t nc = ceil_div(p->seqlen, (int64_t)kQ);
     const size_t esz = p->dtype == M2_F32 ? 4 : 2;
     const size_t tiles = (size_t)p->batch * nc * p->nheads * p->headdim * p->dstate;
@@ -84,7 +94,7 @@ inline SsdWorkspace ssd_carve(const m2_ssd_params* p, void* base, bool bwd, bool
         ssd_slicing(p, kWgsDg, &w.ns_g, &w.hps_g);
         ssd_slicing(p, kWgsOffC, &w.ns_c, &w.hps_c);
         ssd_slicing(p, kWgsOffB, &w.ns_b, &w.hps_b);
-        if (p->dtype != M2_F32 && p->headdim == 64) {       // the main backward kernel produces both state parts there
+        if (p->dtype != M2_F32) {       // the main backward kernel produces both state parts there
             ssd_slicing(p, kWgsDx, &w.ns_b, &w.hps_b);
             w.ns_c = w.ns_b; w.hps_c = w.hps_b;
         }
@@ -157,8 +167,8 @@ inline size_t cb_smem(int n) { return (size_t)2 * 64 * lds_ld<T>(n) * sizeof(T);
 
 // Decay tables, G = C B^T (+ operand tiles), local chunk states, forward state scan.  Used by the forward and, when the
 // caller did not keep the forward's chunk_states buffer, by the backward (recompute).
-template <typename T, int P, int N>
-inline int ssd_launch_states(const m2_ssd_params* p, const SsdWorkspace& w, float* final_out, hipStream_t st) {
+template <typename T, int P, int N, int HS>
+inline int ssd_launch_states(const SsdCall* p, const SsdWorkspace& w, float* final_out, hipStream_t st) {
     const int64_t nc = ceil_div(p->seqlen, (int64_t)kQ);
     const T* x = static_cast<const T*>(p->x);
     const T* Bm = static_cast<const T*>(p->B);
@@ -176,9 +186,9 @@ inline int ssd_launch_states(const m2_ssd_params* p, const SsdWorkspace& w, floa
         pa.Csb = p->C_stride_b; pa.Csl = p->C_stride_l; pa.Csg = p->C_stride_g;
         pa.dt = p->dt; pa.dt_f32 = dt_f32; pa.dt_bias = p->dt_bias; pa.A = p->A; pa.ldtab = w.ldtab; pa.lam = w.lam;
         pa.dtsb = p->dt_stride_b; pa.dtsl = p->dt_stride_l;
-        pa.seqlen = p->seqlen; pa.nheads = p->nheads; pa.ngroups = p->ngroups; pa.nchunks = nc;
+        pa.seqlen = p->seqlen; pa.nheads = p->true_heads; pa.hs = p->hs; pa.ngroups = p->ngroups; pa.nchunks = nc;
         pa.n_cb = nc * p->ngroups * p->batch;
-        const int64_t blocks = kCbParts * pa.n_cb + ld_table_blocks(p->batch, p->nheads, nc);
+        const int64_t blocks = kCbParts * pa.n_cb + ld_table_blocks(p->batch, p->true_heads, nc);
         M2_REQUIRE(blocks < ((int64_t)1 << 31), M2_ERR_SHAPE, "ssd: too many workgroups");
         k<<<(unsigned)blocks, 256, sm, st>>>(pa);
         if ((rc = check_launch("ssd prep_kernel"))) return rc;
@@ -190,19 +200,18 @@ inline int ssd_launch_states(const m2_ssd_params* p, const SsdWorkspace& w, floa
         // differs from the one-tile form in the last bit here and there)
         const bool hilo = final_out != nullptr;
         constexpr int SPLIT = kStatePassSplit;
-        auto k = hilo ? state_pass16_kernel<T, P, N, false, false, true, SPLIT> : state_pass16_kernel<T, P, N, false, false, false, SPLIT>;
+        auto k = hilo ? state_pass16_kernel<T, P, N, false, HS, true, SPLIT> : state_pass16_kernel<T, P, N, false, HS, false, SPLIT>;
         const size_t sm = hilo ? state_pass_smem<P, N, true, SPLIT>() : state_pass_smem<P, N, false, SPLIT>();
         if ((rc = allow_smem(k, sm))) return rc;
         StatePassArgs sa;
         sa.X = x; sa.X_sb = p->x_stride_b; sa.X_sl = p->x_stride_l; sa.X_sh = p->x_stride_h;
         sa.ldtab = w.ldtab; sa.Mt = w.Bt; sa.init = p->initial_state; sa.prev = w.prev; sa.final_out = final_out;
-        sa.sprev = nullptr; sa.dlam = nullptr;
         sa.seqlen = p->seqlen; sa.nheads = p->nheads; sa.ngroups = p->ngroups; sa.nchunks = nc;
         k<<<dim3((unsigned)(p->nheads * SPLIT), (unsigned)p->batch), state_pass_threads<N>(), sm, st>>>(sa);
         return check_launch("ssd state_pass16_kernel");
     } else {
         // fp32 operands: per-chunk contributions (fp32, workspace), then the recurrence over the chunks
-        auto k = chunk_state_kernel<T, P, N, false>;
+        auto k = chunk_state_kernel<T, P, N, false, HS>;
         const size_t sm = state_smem<T, P, N>();
         if ((rc = allow_smem(k, sm))) return rc;
         int64_t ns, hps;
@@ -219,12 +228,12 @@ inline int ssd_launch_states(const m2_ssd_params* p, const SsdWorkspace& w, floa
     }
 }
 
-#define M2_DISPATCH_PN(p, P, N, ...)                                                     \
-    do {                                                                                 \
-        if ((p)->headdim == 64 && (p)->dstate == 64) { constexpr int P = 64, N = 64; __VA_ARGS__; }        \
-        else if ((p)->headdim == 64 && (p)->dstate == 128) { constexpr int P = 64, N = 128; __VA_ARGS__; } \
-        else if ((p)->headdim == 128 && (p)->dstate == 64) { constexpr int P = 128, N = 64; __VA_ARGS__; } \
-        else { constexpr int P = 128, N = 128; __VA_ARGS__; }                            \
+#define M2_DISPATCH_N_HS(p, N, HS, ...)                                                                                   \
+    do {                                                                                                                  \
+        if ((p)->dstate == 64 && (p)->hs == 0) { constexpr int N = 64, HS = 0; __VA_ARGS__; }                             \
+        else if ((p)->dstate == 64) { constexpr int N = 64, HS = 1; __VA_ARGS__; }                                        \
+        else if ((p)->hs == 0) { constexpr int N = 128, HS = 0; __VA_ARGS__; }                                            \
+        else { constexpr int N = 128, HS = 1; __VA_ARGS__; }                                                              \
     } while (0)
 
 }  // namespace m2

@@ -127,7 +127,7 @@ template <typename T>
 __device__ __forceinline__ void
 ld_table_body(const void* __restrict__ dt, int dt_f32, const float* __restrict__ dt_bias, const float* __restrict__ A, float* __restrict__ ldtab,
               float* __restrict__ lam, int64_t seqlen, int64_t nheads, int64_t nchunks,
-              int64_t dtsb, int64_t dtsl, int64_t blk) {
+              int64_t dtsb, int64_t dtsl, int hs, int64_t blk) {
     __shared__ float sdt[kLdHeads][kQ];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t hgroups = (nheads + kLdHeads - 1) / kLdHeads;
@@ -167,7 +167,6 @@ ld_table_body(const void* __restrict__ dt, int dt_f32, const float* __restrict__
     }
     __syncthreads();
     if (h >= nheads) return;      // wave-uniform, behind the only barrier
-    const int64_t bhc = (b * nheads + h) * nchunks + c;
     float l0, l1, d0 = sdt[wave][lane], d1 = sdt[wave][lane + 64];
     if (dt_bias) {
         // dt holds the raw projection: the step size is softplus(dt + dt_bias) (0 stays 0 past the end of the sequence)
@@ -176,9 +175,12 @@ ld_table_body(const void* __restrict__ dt, int dt_f32, const float* __restrict__
         if (lane + 64 < valid) d1 = softplus_f(d1 + bh);
     }
     wave_cumsum_from(A[h], d0, d1, l0, l1);
-    float* p = ldtab + bhc * (2 * kQ);
-    p[lane] = l0; p[lane + 64] = l1; p[kQ + lane] = d0; p[kQ + lane + 64] = d1;
-    if (lane == 63) lam[bhc] = l1;
+    for (int v = 0; v < (1 << hs); ++v) {      // one table per kernel head
+        const int64_t bhc = (((b * nheads + h) << hs) + v) * nchunks + c;
+        float* p = ldtab + bhc * (2 * kQ);
+        p[lane] = l0; p[lane + 64] = l1; p[kQ + lane] = d0; p[kQ + lane + 64] = d1;
+        if (lane == 63) lam[bhc] = l1;
+    }
 }
 
 // Both preparations in one launch (they are independent, and either alone leaves most of the GPU idle): the first
@@ -187,7 +189,8 @@ struct PrepArgs {
     const void* Bm; const void* Cm; float* Gf; void* Gm; void* Gmt; void* Bt; void* Ct;
     int64_t Bsb, Bsl, Bsg, Csb, Csl, Csg;
     const void* dt; int dt_f32; const float* dt_bias; const float* A; float* ldtab; float* lam; int64_t dtsb, dtsl;
-    int64_t seqlen, nheads, ngroups, nchunks, n_cb;
+    int64_t seqlen, nheads, ngroups, nchunks, n_cb;      // nheads: true heads
+    int hs;
 };
 template <typename T, int N>
 __global__ void __launch_bounds__(256)
@@ -200,7 +203,7 @@ prep_kernel(const PrepArgs a) {
                       static_cast<T*>(a.Bt), static_cast<T*>(a.Ct), a.seqlen, a.ngroups, a.nchunks,
                       a.Bsb, a.Bsl, a.Bsg, a.Csb, a.Csl, a.Csg, c, g, b, (int)(blk % kCbParts));
     } else {
-        ld_table_body<T>(a.dt, a.dt_f32, a.dt_bias, a.A, a.ldtab, a.lam, a.seqlen, a.nheads, a.nchunks, a.dtsb, a.dtsl, blk - kCbParts * a.n_cb);
+        ld_table_body<T>(a.dt, a.dt_f32, a.dt_bias, a.A, a.ldtab, a.lam, a.seqlen, a.nheads, a.nchunks, a.dtsb, a.dtsl, a.hs, blk - kCbParts * a.n_cb);
     }
 }
 
@@ -212,7 +215,7 @@ prep_kernel(const PrepArgs a) {
 // `X` is x or dy; `Mt` is the group's B or C tile already transposed to [N][kQ] (tokens contiguous) by cb_body (prep_kernel),
 // staged into LDS once per workgroup.  Per head only the x tile moves: it is loaded 16 bytes at a time, scaled in
 // fp32 and written transposed; the next head's tile is prefetched into registers while the MFMAs run.
-template <typename T, int P, int N, bool DSTATE>
+template <typename T, int P, int N, bool DSTATE, int HS>
 __global__ void __launch_bounds__(256)
 chunk_state_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
                    const T* __restrict__ Mt, float* __restrict__ out,
@@ -238,7 +241,7 @@ chunk_state_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
     const int wm = wave >> 1, wn = wave & 1;
     uint4 pre[NIT];
     auto prefetch = [&](int64_t h) {
-        const T* xp = X + b * Xsb + (t0 + tok) * Xsl + h * Xsh;
+        const T* xp = X + b * Xsb + (t0 + tok) * Xsl + head_off<HS>(h, Xsh);
 #pragma unroll
         for (int it = 0; it < NIT; ++it)
             pre[it] = tok < valid ? *reinterpret_cast<const uint4*>(xp + (it * 2 + cvh) * V) : uint4{0u, 0u, 0u, 0u};

@@ -2,11 +2,7 @@
 // with the running state in registers (fp32), so that no per-chunk contribution is ever written to memory.
 //
 //   forward:  S = init;   for c = 0 .. nc-1:   prev[c] = T(S);   S = e^{Lam_c} S + sum_j (dt_j e^{Lam_c - l_j}) x_j (x) B_j;   final = S
-//   reverse:  R = dfinal; for c = nc-1 .. 0:   prev[c] = T(R);   dlam[c] = e^{Lam_c} <T(R), sprev[c]>;
-//                                              R = e^{Lam_c} R + sum_i e^{l_i} dy_i (x) C_i;   dinit = R
-// (dlam is the part of dL/dLam_c that flows through the carried state; sprev[c] = the forward state entering chunk c.
-//  With DLAM == false the reverse pass leaves dlam to ssd_bwd16_kernel, which has both tiles in LDS anyway, and does
-//  not read sprev at all.)
+//   reverse:  R = dfinal; for c = nc-1 .. 0:   prev[c] = T(R);   R = e^{Lam_c} R + sum_i e^{l_i} dy_i (x) C_i;   dinit = R
 //
 // grid (nheads * 2, batch), N / 32 waves; a workgroup owns one half of the ROWS of the [P][N] state (P / 2 head channels, all
 // N columns), wave w the columns [32 w, +32) of them, as 32x32 MFMA accumulator blocks: only that half of the x / dy columns
@@ -32,8 +28,6 @@ struct StatePassArgs {
     const float* init;                             // fp32 [b][h][P][N]: initial state / gradient of the final state, or null
     void* prev;                                    // out [b][c][h][P][N], operand type
     float* final_out;                              // out fp32 [b][h][P][N]: final state / gradient of the initial state, or null
-    const void* sprev;                             // reverse: [b][c][h][P][N] forward states entering the chunks
-    float* dlam;                                   // reverse: out [b][h][c][kDlamParts]
     int64_t seqlen, nheads, ngroups, nchunks;
 };
 
@@ -52,14 +46,13 @@ constexpr size_t state_pass_smem() {
 // HILO: the scaled rows are staged as TWO 16-bit tiles, the rounded value and the rounded remainder, and each k step takes
 // two products, so that the fp32 scale dt e^{Lam - l} reaches the accumulators with 16 significand bits instead of 8 (the
 // final state is an fp32 output; with one tile its error is that of the operand rounding, 2^-9 of every term).
-template <typename T, int P, int N, bool REVERSE, bool DLAM = REVERSE, bool HILO = false, int SPLIT = kStatePassSplit>
-__global__ void __launch_bounds__(state_pass_threads<N>(), (SPLIT == 1 ? (P == 64 ? 2 : 1) : (P == 64 ? (DLAM ? 2 : 3) : (DLAM ? 1 : 2))))
+template <typename T, int P, int N, bool REVERSE, int HS, bool HILO = false, int SPLIT = kStatePassSplit>
+__global__ void __launch_bounds__(state_pass_threads<N>(), SPLIT == 1 ? 2 : 3)
 state_pass16_kernel(const StatePassArgs a) {
     static_assert(sizeof(T) == 2, "16-bit operands only");
     constexpr int NWAVES = N / 32, THREADS = state_pass_threads<N>();
     constexpr int PH = P / SPLIT;                      // state rows (head channels) of this workgroup
     constexpr int NW = 32;                             // state columns per wave
-    static_assert(SPLIT * NWAVES <= kDlamParts, "dlam slots");
     constexpr int PBW = PH / 32, NBW = 1;              // 32x32 blocks per wave
     constexpr int SPR_X = PH / 8;                      // 16-byte slots per staged x row
     constexpr int NXR = kQ * SPR_X / THREADS;              // x pieces per thread per chunk
@@ -118,7 +111,7 @@ state_pass16_kernel(const StatePassArgs a) {
     auto load_ahead = [&](int64_t c, Ahead& s) {
         const int64_t t0 = c * kQ;
         const uint32_t last = (uint32_t)(((a.seqlen - t0) < kQ ? (a.seqlen - t0) : kQ) - 1);      // last valid row
-        const char* xp = reinterpret_cast<const char*>(static_cast<const T*>(a.X) + b * a.X_sb + t0 * a.X_sl + h * a.X_sh + pw * PH);
+        const char* xp = reinterpret_cast<const char*>(static_cast<const T*>(a.X) + b * a.X_sb + t0 * a.X_sl + head_off<HS>(h, a.X_sh) + pw * PH);
         const float* tab = a.ldtab + (bh * nc + c) * (2 * kQ);
         s.lam = tab[kQ - 1];
 #pragma unroll
@@ -131,11 +124,8 @@ state_pass16_kernel(const StatePassArgs a) {
         }
     };
     // loaded at the top of the iteration that consumes them (so that the wait in front of their use can be counted
-    // exactly and leaves the next chunk's rows, issued behind them, in flight): the group's B^T / C^T fragments (L2) and,
-    // for the reverse pass, this lane's pieces of the forward state
+    // exactly and leaves the next chunk's rows, issued behind them, in flight): the group's B^T / C^T fragments (L2)
     Frag<T> bf[NBW][8];
-    static_assert(REVERSE || !DLAM, "dlam belongs to the reverse pass");
-    u32x4 spr[DLAM ? NSP : 1];
     const uint32_t st_off = (uint32_t)(((pw * PH + wave * RW + lane / LPR) * N + (lane % LPR) * 8) * 2);      // pass ps: + ps * RPP * N * 2
     auto load_same = [&](int64_t c) {
         const char* mp = reinterpret_cast<const char*>(static_cast<const T*>(a.Mt) + ((b * nc + c) * a.ngroups + g) * (int64_t)(N * kQ));
@@ -144,11 +134,6 @@ state_pass16_kernel(const StatePassArgs a) {
 #pragma unroll
             for (int ks = 0; ks < 8; ++ks)      // see mt_offset
                 bf[j][ks].v = *reinterpret_cast<const bf16x8*>(mp + ((uint32_t)lane * 16u + (uint32_t)((((n0 >> 5) + j) * 8 + ks) * 1024)));
-        if (DLAM) {
-            const char* sp = reinterpret_cast<const char*>(static_cast<const T*>(a.sprev) + ((b * nc + c) * a.nheads + h) * (int64_t)(P * N));
-#pragma unroll
-            for (int ps = 0; ps < NSP; ++ps) spr[ps] = *reinterpret_cast<const u32x4*>(sp + (st_off + (uint32_t)(ps * RPP * N * 2)));
-        }
     };
 
     auto step = [&](int64_t cc, Ahead& s) {
@@ -219,25 +204,11 @@ state_pass16_kernel(const StatePassArgs a) {
 
         // ---- the state entering (forward) / the gradient leaving (reverse) this chunk: whole rows of the workgroup's slab
         char* op = reinterpret_cast<char*>(static_cast<T*>(a.prev) + ((b * nc + c) * a.nheads + h) * (int64_t)(P * N));
-        float dot = 0.f;
 #pragma unroll
         for (int ps = 0; ps < NSP; ++ps) {
             const int rl = wave * RW + ps * RPP + lane / LPR, cv = lane % LPR;
             const u32x4 o = *reinterpret_cast<const u32x4*>(cO + rl * LDO + cv * 8);
             *reinterpret_cast<u32x4*>(op + (st_off + (uint32_t)(ps * RPP * N * 2))) = o;
-            if (DLAM) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    dot = dot2_acc<T>(o[q], spr[ps][q], dot);
-            }
-        }
-        if (DLAM) {
-            dot = warp_sum(dot);
-            if (lane == 0) {
-                const int slot = pw * NWAVES + wave;
-                a.dlam[(bh * nc + c) * kDlamParts + slot] = dec * dot;
-                for (int s2 = slot + SPLIT * NWAVES; s2 < kDlamParts; s2 += SPLIT * NWAVES) a.dlam[(bh * nc + c) * kDlamParts + s2] = 0.f;
-            }
         }
 
         // ---- S = e^{Lam} S + X_scaled^T M  (accumulated as its transpose M^T X_scaled)

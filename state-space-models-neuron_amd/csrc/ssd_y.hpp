@@ -115,7 +115,7 @@ constexpr size_t y16_smem() {
     return (size_t)2 * ((P * N + kQ * P) * 2 + 2 * kQ * sizeof(float)) + (size_t)4 * (kQ + 32) * sizeof(float);
 }
 
-template <typename T, int P, int N>
+template <typename T, int P, int N, int HS>
 __global__ void __launch_bounds__(256, (y16_smem<P, N>() <= 80 * 1024 ? 2 : 1))
 ssd_y16_kernel(const DiagArgs a) {
     static_assert(sizeof(T) == 2, "16-bit operands only");
@@ -166,7 +166,7 @@ ssd_y16_kernel(const DiagArgs a) {
         const T* Sp = static_cast<const T*>(a.S) + ((b * a.nchunks + c) * a.nheads + h) * (int64_t)(P * N);
 #pragma unroll
         for (int it = 0; it < NS; ++it) async_copy16(Sp, offS[it], lds_S + (uint32_t)(buf * (P * N) * 2) + (wave_u * NS + it) * 1024u);
-        const T* Xp = static_cast<const T*>(a.Z) + b * a.Z_sb + t0 * a.Z_sl + h * a.Z_sh;
+        const T* Xp = static_cast<const T*>(a.Z) + b * a.Z_sb + t0 * a.Z_sl + head_off<HS>(h, a.Z_sh);
 #pragma unroll
         for (int it = 0; it < NX; ++it) async_copy16(Xp, offX[it], lds_X + (uint32_t)(buf * (kQ * P) * 2) + (wave_u * NX + it) * 1024u);
         async_copy_ldtab(a.ldtab, (b * a.nheads + h) * a.nchunks + c, lds_LD + (uint32_t)(buf * 2 * kQ * 4));
@@ -197,7 +197,7 @@ ssd_y16_kernel(const DiagArgs a) {
     for (int64_t hh = 0; hh < a.hps; ++hh) {
         const int64_t h = h_first + hh;
         const int buf = (int)(hh & 1);
-        const float Dh = a.D ? load_uniform_f32(a.D + h) : 0.f;
+        const float Dh = a.D ? load_uniform_f32(a.D + (h >> HS)) : 0.f;
 
         // this wave's share of the tiles of head hh, and the whole [ l | dt ] table, have landed.  The y stores of the head
         // before were issued behind these copies and vector-memory operations retire in issue order, so in a full chunk
@@ -286,7 +286,7 @@ ssd_y16_kernel(const DiagArgs a) {
         //      whole groups of 8 consecutive channels: 16-byte stores without a pass through LDS
         const int tok = row0 + r;
         const float fs = fast ? wu[r] : 1.f;
-        T* Yp = static_cast<T*>(a.Y) + b * a.Y_sb + t0 * a.Y_sl + h * a.Y_sh + (int64_t)tok * a.Y_sl;
+        T* Yp = static_cast<T*>(a.Y) + b * a.Y_sb + t0 * a.Y_sl + head_off<HS>(h, a.Y_sh) + (int64_t)tok * a.Y_sl;
 #pragma unroll
         for (int j = 0; j < BN; ++j) {
 #pragma unroll
