@@ -86,6 +86,9 @@ typedef struct m2_conv1d_params {
 } m2_conv1d_params;
 
 int m2_conv1d_fwd(const m2_conv1d_params* p, void* stream);
+/* Forward of a prompt into the decode cache conv_state (b, C, W >= k-1) of the activation type, contiguous, oldest input
+ * first: with `continuing` its contents precede the sequence, and on return it holds the last W inputs. */
+int m2_conv1d_prefill(const m2_conv1d_params* p, void* conv_state, int32_t W, int32_t continuing, void* stream);
 size_t m2_conv1d_bwd_workspace_bytes(int64_t batch, int64_t seqlen, int64_t channels, int32_t k);
 int m2_conv1d_bwd(const m2_conv1d_params* p, void* stream);
 

@@ -27,7 +27,7 @@ using torch::autograd::variable_list;
 
 // ----------------------------------------------------------------------------------------------- the library
 #define M2_BOUND(F) \
-    F(m2_last_error) F(m2_conv1d_fwd) F(m2_conv1d_bwd_workspace_bytes) F(m2_conv1d_bwd) F(m2_ssd_chunk_states_bytes) \
+    F(m2_last_error) F(m2_conv1d_fwd) F(m2_conv1d_prefill) F(m2_conv1d_bwd_workspace_bytes) F(m2_conv1d_bwd) F(m2_ssd_chunk_states_bytes) \
     F(m2_ssd_fwd_workspace_bytes) F(m2_ssd_fwd) F(m2_ssd_bwd_workspace_bytes) F(m2_ssd_bwd) F(m2_decode_workspace_bytes) \
     F(m2_decode_step) F(m2_decode_step_static) F(m2_rmsnorm_gated_fwd) F(m2_rmsnorm_gated_bwd_workspace_bytes) \
     F(m2_rmsnorm_gated_bwd) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_rows) F(m2_decode_layer) F(m2_mixer_params) F(m2_mixer_params_grads)
@@ -713,27 +713,22 @@ Tensor fused_prefill(const Tensor& zx, const Tensor& A, const OptTensor& D, cons
     TORCH_CHECK_VALUE(ssm_state.dim() == 4 && ssm_state.size(0) == k.b && ssm_state.size(1) == k.h && ssm_state.size(2) == hd && ssm_state.size(3) == n &&
                           ssm_state.scalar_type() == at::kFloat, "ssm_state must be (b, h, p, n) float32");
     if (k.l == 0) return at::empty({k.b, 0, d}, zx.options());
-    const int64_t W = conv_state.size(2);
-    const Tensor xBC = k.zx.narrow(2, d, k.conv);
-    Tensor conv_out, tail;
-    if (continuing) {
-        // the cached inputs go in front of the new ones; the outputs for them are dropped
-        const Tensor hist = at::cat({conv_state.transpose(1, 2).to(xBC.scalar_type()), xBC}, 1);
-        conv_out = conv1d_forward(hist, conv_w, conv_b_, M2_ACT_SILU, true, std::nullopt).narrow(1, W, k.l);
-        tail = hist.narrow(1, k.l, W);
-    } else {
-        conv_out = conv1d_forward(xBC, conv_w, conv_b_, M2_ACT_SILU, true, std::nullopt);
-        tail = k.l >= W ? xBC.narrow(1, k.l - W, W) : at::cat({at::zeros({k.b, W - k.l, k.conv}, xBC.options()), xBC}, 1);
-    }
+    // the kernels work in the caller's cache tensors where those are contiguous and of the kernels' types
+    const bool own_conv = conv_state.is_contiguous() && conv_state.scalar_type() == zx.scalar_type(), own_ssm = ssm_state.is_contiguous();
+    const Tensor cs = own_conv ? conv_state : conv_state.to(zx.options(), false, true).contiguous(), S = own_ssm ? ssm_state : ssm_state.contiguous();
+    const Tensor w = conv_w.contiguous(), bi = conv_b.defined() ? conv_b.contiguous() : conv_b;
+    const Tensor conv_out = at::empty({k.b, k.l, k.conv}, zx.options());
+    m2_conv1d_params c = conv_params(k.xBC(), w, bi, {ptr(conv_out), k.l * k.conv, k.conv, 1}, k.b, k.l, k.conv, dtype_code(k.zx), M2_ACT_SILU);
+    c.y = ptr(conv_out);
+    check(lib.m2_conv1d_prefill(&c, ptr(cs), static_cast<int32_t>(cs.size(2)), continuing, scope.stream), "m2_conv1d_prefill");
     const Tensor A32 = f32(A), D32 = f32(or_none(D)), bias = f32(dt_bias);
     m2_ssd_params p = core_ssd_params(k, conv_out, A32, D32, bias);
-    const Tensor y = at::empty({k.b, k.l, d}, zx.options()), S = at::empty_like(ssm_state, at::MemoryFormat::Contiguous);
-    const Tensor S0 = continuing ? ssm_state.contiguous() : Tensor();
-    p.initial_state = ptr<float>(S0); p.final_state = ptr<float>(S);
+    const Tensor y = at::empty({k.b, k.l, d}, zx.options());
+    p.initial_state = continuing ? ptr<float>(S) : nullptr; p.final_state = ptr<float>(S);
     p.y = ptr(y); p.y_stride_b = k.l * d; p.y_stride_l = d; p.y_stride_h = hd;
     launch_ssd_fwd(p, zx, scope.stream);
-    ssm_state.copy_(S);
-    conv_state.copy_(tail.transpose(1, 2));
+    if (!own_conv) conv_state.copy_(cs);
+    if (!own_ssm) ssm_state.copy_(S);
     return rmsnorm_forward(y, k.z(), norm_w, g, kNormEps, zx.scalar_type());
 }
 

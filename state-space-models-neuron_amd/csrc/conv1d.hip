@@ -141,7 +141,7 @@ __device__ __forceinline__ void load_taps(const void* __restrict__ w, const void
 // grid: x = ceil(CV / kCVT), y = ceil(nseg / kSEG), z = batch; block (kCVT, kSEG).
 template <typename T, typename WT, int V, int ACT>
 __global__ void __launch_bounds__(kCVT * kSEG)
-conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias,
+conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias, const T* __restrict__ hist, int W,
                    T* __restrict__ y, int64_t l, int64_t C, int64_t xsb, int64_t xsl, int64_t ysb, int64_t ysl) {
     const int64_t cv = (int64_t)blockIdx.x * kCVT + threadIdx.x;
     const int64_t seg = (int64_t)blockIdx.y * kSEG + threadIdx.y;
@@ -160,6 +160,15 @@ conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     if (t0 - 3 >= 0) ld_elems<T, V>(xp + (t0 - 3) * xsl, h0);
     if (t0 - 2 >= 0) ld_elems<T, V>(xp + (t0 - 2) * xsl, h1);
     if (t0 - 1 >= 0) ld_elems<T, V>(xp + (t0 - 1) * xsl, h2);
+    if (hist && t0 == 0) {
+        // the inputs in front of the sequence come out of the decode cache (three short reads per channel in the first
+        // segment only; putting cache and sequence behind one another in memory first took 35 us of 145 at b8 l333 C5376)
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            const T* hp = hist + (b * C + c0 + j) * W + (W - 3);
+            h0[j] = to_f32(hp[0]); h1[j] = to_f32(hp[1]); h2[j] = to_f32(hp[2]);
+        }
+    }
     auto step = [&](const RawVec<T, V>& r, T* __restrict__ yq) {
         float out[V], cur[V];
         cvtv<T, V>(r, cur);
@@ -507,7 +516,7 @@ conv_bwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
 // Generic path: any strides / layout, k <= 8, one thread per output element.
 template <typename T>
 __global__ void conv_fwd_generic_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias,
-                                        T* __restrict__ y, int64_t nb, int64_t l, int64_t C, int k,
+                                        const T* __restrict__ hist, int W, T* __restrict__ y, int64_t nb, int64_t l, int64_t C, int k,
                                         int64_t xsb, int64_t xsl, int64_t xsc, int64_t ysb, int64_t ysl, int64_t ysc,
                                         int pd, int act, int t_fastest) {
     const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -519,9 +528,25 @@ __global__ void conv_fwd_generic_kernel(const T* __restrict__ x, const void* __r
     for (int i = 0; i < k; ++i) {
         const int64_t tt = t - (k - 1) + i;
         if (tt >= 0) z += ld_param(w, pd, c * k + i) * to_f32(x[b * xsb + tt * xsl + c * xsc]);
+        else if (hist) z += ld_param(w, pd, c * k + i) * to_f32(hist[(b * C + c) * W + W + tt]);
     }
     const float o = act == M2_ACT_SILU ? silu_f(z) : (act == M2_ACT_RELU ? (z > 0.f ? z : 0.f) : z);
     y[b * ysb + t * ysl + c * ysc] = from_f32<T>(o);
+}
+
+// The last W inputs of a sequence into the decode cache [b][C][W], oldest first; one thread per channel.  Where the sequence
+// is shorter than W, what is left of the cache (or zeros) moves up; a thread reads ahead of what it writes.
+template <typename T>
+__global__ void __launch_bounds__(256)
+conv_tail_kernel(const T* __restrict__ x, T* state, int W, int keep, int64_t nb, int64_t l, int64_t C, int64_t xsb, int64_t xsl, int64_t xsc) {
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= nb * C) return;
+    const int64_t b = idx / C, c = idx % C;
+    T* sp = state + idx * W;
+    for (int w = 0; w < W; ++w) {
+        const int64_t t = l - W + w;
+        sp[w] = t >= 0 ? x[b * xsb + t * xsl + c * xsc] : (keep ? sp[w + l] : from_f32<T>(0.f));
+    }
 }
 
 template <typename T>
@@ -636,8 +661,10 @@ int check_common(const m2_conv1d_params* p) {
     return M2_OK;
 }
 
+// hist: null, or the W >= k - 1 inputs in front of the sequence, [b][C][W], oldest first
 template <typename T>
-int launch_fwd(const m2_conv1d_params* p, hipStream_t st) {
+int launch_fwd(const m2_conv1d_params* p, const void* hist_, int W, hipStream_t st) {
+    const T* hist = static_cast<const T*>(hist_);
     const int64_t nb = p->batch, l = p->seqlen, C = p->channels;
     const T* x = static_cast<const T*>(p->x);
     T* y = static_cast<T*>(p->y);
@@ -648,9 +675,9 @@ int launch_fwd(const m2_conv1d_params* p, hipStream_t st) {
         M2_REQUIRE(grid.y <= 65535, M2_ERR_SHAPE, "conv1d: sequence too long for the grid");
         conv_dispatch(p, [&](auto wt, auto act) {
             conv_fwd_cl_kernel<T, decltype(wt), V, decltype(act)::value><<<grid, block, 0, st>>>(
-                x, p->w, p->bias, y, l, C, p->x_stride_b, p->x_stride_l, p->y_stride_b, p->y_stride_l);
+                x, p->w, p->bias, hist, W, y, l, C, p->x_stride_b, p->x_stride_l, p->y_stride_b, p->y_stride_l);
         });
-    } else if (channel_major_ok(p, false)) {
+    } else if (!hist && channel_major_ok(p, false)) {
         const int64_t pieces = ceil_div(l, (int64_t)VecTraits<T>::kVec), total = nb * C * pieces;
         conv_dispatch(p, [&](auto wt, auto act) {
             conv_fwd_cm_kernel<T, decltype(wt), decltype(act)::value><<<(unsigned)ceil_div(total, (int64_t)256), 256, 0, st>>>(
@@ -660,7 +687,7 @@ int launch_fwd(const m2_conv1d_params* p, hipStream_t st) {
         const int64_t total = nb * l * C;
         const int tf = (p->x_stride_l == 1 && p->x_stride_c != 1) ? 1 : 0;
         conv_fwd_generic_kernel<T><<<(unsigned)ceil_div(total, 256), 256, 0, st>>>(
-            x, p->w, p->bias, y, nb, l, C, p->k, p->x_stride_b, p->x_stride_l, p->x_stride_c,
+            x, p->w, p->bias, hist, W, y, nb, l, C, p->k, p->x_stride_b, p->x_stride_l, p->x_stride_c,
             p->y_stride_b, p->y_stride_l, p->y_stride_c, p->param_dtype, p->activation, tf);
     }
     return check_launch("conv1d_fwd");
@@ -736,7 +763,25 @@ extern "C" int m2_conv1d_fwd(const m2_conv1d_params* p, void* stream) {
     if (rc) return rc;
     if (p->batch == 0 || p->seqlen == 0 || p->channels == 0) return M2_OK;
     M2_REQUIRE(p->x && p->w && p->y, M2_ERR_NULL, "conv1d_fwd: x, w and y are required");
-    M2_DISPATCH_DTYPE(p->dtype, T, return launch_fwd<T>(p, static_cast<hipStream_t>(stream)));
+    M2_DISPATCH_DTYPE(p->dtype, T, return launch_fwd<T>(p, nullptr, 0, static_cast<hipStream_t>(stream)));
+    return M2_OK;
+}
+
+extern "C" int m2_conv1d_prefill(const m2_conv1d_params* p, void* conv_state, int32_t W, int32_t continuing, void* stream) {
+    using namespace m2;
+    int rc = check_common(p);
+    if (rc) return rc;
+    if (p->batch == 0 || p->seqlen == 0 || p->channels == 0) return M2_OK;
+    M2_REQUIRE(p->x && p->w && p->y && conv_state, M2_ERR_NULL, "conv1d_prefill: x, w, y and conv_state are required");
+    M2_REQUIRE(W >= p->k - 1, M2_ERR_SHAPE, "conv1d_prefill: the cache holds %d inputs, needs %d", W, p->k - 1);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    M2_DISPATCH_DTYPE(p->dtype, T, {
+        if ((rc = launch_fwd<T>(p, continuing ? conv_state : nullptr, W, st))) return rc;
+        conv_tail_kernel<T><<<(unsigned)ceil_div(p->batch * p->channels, (int64_t)256), 256, 0, st>>>(
+            static_cast<const T*>(p->x), static_cast<T*>(conv_state), W, continuing, p->batch, p->seqlen, p->channels,
+            p->x_stride_b, p->x_stride_l, p->x_stride_c);
+        return check_launch("conv1d_tail");
+    });
     return M2_OK;
 }
 

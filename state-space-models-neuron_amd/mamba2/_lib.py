@@ -82,6 +82,7 @@ SYMBOLS = {
     "m2_last_error": (C.c_char_p, []),
     "m2_struct_layout": (C.c_int, [_i32, C.POINTER(_i64), _i32]),
     "m2_conv1d_fwd": (C.c_int, [C.POINTER(Conv1dParams), _vp]),
+    "m2_conv1d_prefill": (C.c_int, [C.POINTER(Conv1dParams), _vp, _i32, _i32, _vp]),
     "m2_conv1d_bwd_workspace_bytes": (_sz, [_i64, _i64, _i64, _i32]),
     "m2_conv1d_bwd": (C.c_int, [C.POINTER(Conv1dParams), _vp]),
     "m2_ssd_chunk_states_bytes": (_sz, [C.POINTER(SsdParams)]),

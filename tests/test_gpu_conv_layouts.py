@@ -27,3 +27,35 @@ def test_conv_layout_edges(dtype, channels_last, b, l, C, act):
     tol, metric = (1e-4, rel_err) if dtype == torch.float32 else (2e-2, rel_rms_err)
     for name, a, r in zip(("y", "dx", "dw", "db"), got, ref):
         assert metric(a, r) < tol, name
+
+
+@pytest.mark.parametrize("l1,l2,k,W", [(5, 1, 4, 4), (1, 2, 4, 3), (16, 17, 4, 4), (130, 3, 4, 4), (7, 40, 2, 3), (2, 1, 3, 5)])
+@pytest.mark.parametrize("dtype,state_dtype", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("strided", [False, True])
+def test_prefill_in_two_pieces(l1, l2, k, W, dtype, state_dtype, strided):
+    """The conv with the cache in front of it, and what it leaves there, against one pass over the whole sequence."""
+    from mamba2.fused_kernel import mamba2_fused_prefill
+    torch.manual_seed(l1 * 100 + l2)
+    b, h, p, n, g = 2, 8, 64, 64, 1
+    d, c, l = h * p, h * p + 2 * g * n, l1 + l2
+    zx = (torch.randn(b, l, d + c + h, device="cuda") * 0.5).to(dtype)
+    A, D, dt_bias = -torch.rand(h, device="cuda") - 0.5, torch.randn(h, device="cuda"), torch.randn(h, device="cuda")
+    conv_w, conv_b = (torch.randn(c, 1, k, device="cuda") * 0.3).to(dtype), torch.randn(c, device="cuda").to(dtype)
+    norm_w = torch.rand(d, device="cuda") + 0.5
+
+    def states():
+        if strided:
+            return (torch.empty(b, c, 2 * W, device="cuda", dtype=state_dtype)[..., ::2], torch.empty(b, h, n, p, device="cuda").transpose(2, 3))
+        return torch.empty(b, c, W, device="cuda", dtype=state_dtype), torch.empty(b, h, p, n, device="cuda")
+
+    def run(part, st, continuing):
+        return mamba2_fused_prefill(part, A, D, conv_w, conv_b, dt_bias, norm_w, g, n, d, p, *st, continuing=continuing)
+
+    one, two = states(), states()
+    whole = run(zx, one, False)
+    pieces = torch.cat([run(zx[:, :l1], two, False), run(zx[:, l1:], two, True)], 1)
+    tail = torch.nn.functional.pad(zx[:, :, d:d + c], (0, 0, W, 0))[:, l:].transpose(1, 2)
+    assert torch.equal(one[0].float(), tail.float()) and torch.equal(two[0].float(), tail.float())
+    tol = 2e-2 if dtype == torch.bfloat16 else 2e-4
+    torch.testing.assert_close(pieces.float(), whole.float(), rtol=tol, atol=tol)
+    torch.testing.assert_close(two[1], one[1], rtol=tol, atol=tol)
