@@ -165,6 +165,20 @@ inline size_t state_smem() { return (size_t)(P + N) * lds_ld<T>(kQ) * sizeof(T);
 template <typename T>
 inline size_t cb_smem(int n) { return (size_t)2 * 64 * lds_ld<T>(n) * sizeof(T); }
 
+template <typename T, int P, int N, bool REVERSE, int HS, bool HILO>
+inline int launch_state_pass16(const StatePassArgs& a, int64_t batch, hipStream_t st) {
+    auto launch = [&](auto k, size_t sm, int split) -> int {
+        if (const int rc = allow_smem(k, sm)) return rc;
+        k<<<dim3((unsigned)(a.nheads * split), (unsigned)batch), state_pass_threads<N>(), sm, st>>>(a);
+        return M2_OK;
+    };
+    if constexpr (N == 128 && !HILO)
+        if (state_pass_split(batch * a.nheads, N) == 1)
+            return launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, 1>, state_pass_smem<P, N, HILO, 1>(), 1);
+    constexpr int SPLIT = kStatePassSplit;
+    return launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, SPLIT>, state_pass_smem<P, N, HILO, SPLIT>(), SPLIT);
+}
+
 // Decay tables, G = C B^T (+ operand tiles), local chunk states, forward state scan.  Used by the forward and, when the
 // caller did not keep the forward's chunk_states buffer, by the backward (recompute).
 template <typename T, int P, int N, int HS>
@@ -199,15 +213,11 @@ inline int ssd_launch_states(const SsdCall* p, const SsdWorkspace& w, float* fin
         // (3.7 us more per pass at b4 l2048 h80; the states entering the chunks come out of the same accumulators, so y
         // differs from the one-tile form in the last bit here and there)
         const bool hilo = final_out != nullptr;
-        constexpr int SPLIT = kStatePassSplit;
-        auto k = hilo ? state_pass16_kernel<T, P, N, false, HS, true, SPLIT> : state_pass16_kernel<T, P, N, false, HS, false, SPLIT>;
-        const size_t sm = hilo ? state_pass_smem<P, N, true, SPLIT>() : state_pass_smem<P, N, false, SPLIT>();
-        if ((rc = allow_smem(k, sm))) return rc;
         StatePassArgs sa;
         sa.X = x; sa.X_sb = p->x_stride_b; sa.X_sl = p->x_stride_l; sa.X_sh = p->x_stride_h;
         sa.ldtab = w.ldtab; sa.Mt = w.Bt; sa.init = p->initial_state; sa.prev = w.prev; sa.final_out = final_out;
         sa.seqlen = p->seqlen; sa.nheads = p->nheads; sa.ngroups = p->ngroups; sa.nchunks = nc;
-        k<<<dim3((unsigned)(p->nheads * SPLIT), (unsigned)p->batch), state_pass_threads<N>(), sm, st>>>(sa);
+        if ((rc = hilo ? launch_state_pass16<T, P, N, false, HS, true>(sa, p->batch, st) : launch_state_pass16<T, P, N, false, HS, false>(sa, p->batch, st))) return rc;
         return check_launch("ssd state_pass16_kernel");
     } else {
         // fp32 operands: per-chunk contributions (fp32, workspace), then the recurrence over the chunks

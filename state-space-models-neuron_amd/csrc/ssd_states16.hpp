@@ -4,9 +4,9 @@
 //   forward:  S = init;   for c = 0 .. nc-1:   prev[c] = T(S);   S = e^{Lam_c} S + sum_j (dt_j e^{Lam_c - l_j}) x_j (x) B_j;   final = S
 //   reverse:  R = dfinal; for c = nc-1 .. 0:   prev[c] = T(R);   R = e^{Lam_c} R + sum_i e^{l_i} dy_i (x) C_i;   dinit = R
 //
-// grid (nheads * 2, batch), N / 32 waves; a workgroup owns one half of the ROWS of the [P][N] state (P / 2 head channels, all
-// N columns), wave w the columns [32 w, +32) of them, as 32x32 MFMA accumulator blocks: only that half of the x / dy columns
-// is loaded, scaled and staged, so the two workgroups of a head share no work.  Per chunk the MFMA computes
+// grid (nheads * SPLIT, batch), N / 32 waves; a workgroup owns 1 / SPLIT of the ROWS of the [P][N] state (head channels; all N
+// columns), wave w the columns [32 w, +32) of them, as 32x32 MFMA accumulator blocks: only that part of the x / dy columns
+// is loaded, scaled and staged, so the workgroups of a head share no work.  Per chunk the MFMA computes
 // X_scaled^T [P/2 x kQ] * M [kQ x N]:
 //   * M (B or C of the group) comes from the transposed tiles that prep_kernel wrote in MFMA operand order: a wave's
 //     B-operand fragment is one contiguous KiB of global memory, loaded straight into registers at the top of the
@@ -31,11 +31,22 @@ struct StatePassArgs {
     int64_t seqlen, nheads, ngroups, nchunks;
 };
 
-// workgroups per (batch, head): each takes half of the state rows (more, smaller workgroups: the chunk loop is a chain of
-// dependent memory round trips, and only other resident waves can fill its gaps).  One workgroup per head (SPLIT = 1: whole
-// 128-byte x rows, each operand fragment feeding two products, half the fragment traffic) is slower: reverse pass 52 -> 57 us,
-// forward pass with the two-tile operands 56 -> 79 us at b4 l2048 h80.
+// What bounds the pass: a CU's vector-memory path.  Its loads retire in order, so the operand fragments (which come from L2)
+// queue behind the x rows (which come from HBM), and the bytes that one step takes through it decide the step's time: x and
+// dy 8 KiB, fragments 32 KiB and states 8 KiB for half a head, whose stores and loads each cost their own time at b4 l2048
+// h80 (57 us; 42 without the stores, 41 without the x rows, 46 without the fragments, 16 without any).
+// SPLIT = 2, half a head per workgroup, spreads few heads over more CUs and fills the last round of many better.  SPLIT = 1
+// feeds two products from each fragment, 48 KiB a step for a whole head where two halves take 80, and reads whole 128-byte
+// lines of x: state_pass_split says where that wins.
 constexpr int kStatePassSplit = 2;
+// SPLIT = 1 only with 128 state columns (with 64 there are two waves of 256 registers, and they spill), only for the one-tile
+// form, and only where whole heads fill the CUs in nearly whole rounds (the last one idle by a fifth at most).  Forward at
+// l 4096 (b h up to 256) or 2048: b h 192 136 -> 132 us, 224 162 -> 152, 256 177 -> 163, 448 157 -> 150, 512 178 -> 163,
+// 768 252 -> 247, 1024 367 -> 355; below the line 80 63 -> 79, 160 98 -> 100, 288 88 -> 91, 320 98 -> 101, 384 124 -> 126.
+inline int state_pass_split(int64_t heads, int n) {
+    const int64_t cus = device_cus(), rounds = ceil_div(heads, cus);
+    return n == 128 && heads * 5 >= rounds * cus * 4 ? 1 : kStatePassSplit;
+}
 // one wave per 32 state columns
 template <int N> constexpr int state_pass_threads() { return (N / 32) * 64; }
 template <int P, int N, bool HILO = false, int SPLIT = kStatePassSplit>
@@ -69,17 +80,20 @@ state_pass16_kernel(const StatePassArgs a) {
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int r = lane & 31, half = lane >> 5;
-    const int pw = (int)(blockIdx.x / a.nheads);       // which half of the rows
+    const int pw = (int)(blockIdx.x / a.nheads);       // which part of the rows
     // the workgroups of one head are nheads apart in the grid: with a head count that is a multiple of 8 they land on the
     // same XCD and share the head's rows in its L2
     const int64_t h = blockIdx.x % a.nheads, b = blockIdx.y;
-    const int n0 = wave * NW;                          // first state column of this wave
+    const int wave_u = (int)uniform((uint32_t)wave), n0 = wave_u * NW;      // first state column of this wave
     const int64_t g = h / (a.nheads / a.ngroups);
     const int64_t bh = b * a.nheads + h;
     const int64_t nc = a.nchunks;
     const int tr_tok = 8 * half + ((lane >> 2) & 3);
     const int tr_col = ((lane >> 4) & 1) * 16 + 4 * (lane & 3);
     typedef T tvec4 __attribute__((ext_vector_type(4)));
+    // element offsets of this lane's transpose reads of k step 0 (a step is 16 rows, and tile_swz looks at the row modulo 16)
+    const int tr_lo = (tr_tok * SPR_X + ((tr_col >> 3) ^ tile_swz<SPR_X>(tr_tok))) * 8 + (tr_col & 7);
+    const int tr_hi = ((tr_tok + 4) * SPR_X + ((tr_col >> 3) ^ tile_swz<SPR_X>(tr_tok + 4))) * 8 + (tr_col & 7);
 
     // The MFMAs are issued with swapped operands: acc[i][j][v] is the state at row pw P/2 + 32 i + r, column
     // n0 + 32 j + acc_row(lane, v), i.e. a lane holds groups of 4 consecutive columns of ONE row (8-byte staging writes).
@@ -99,58 +113,71 @@ state_pass16_kernel(const StatePassArgs a) {
     // is loaded with chunk cc + 2, so that a load has two iterations to land.
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     struct Ahead { u32x4 x[NXR]; float l[NXR], d[NXR], lam; };
-    auto chunk_of = [&](int64_t cc) -> int64_t {       // cc-th chunk in processing order, clamped to the last one
-        const int64_t k = cc < nc ? cc : nc - 1;
-        return REVERSE ? nc - 1 - k : k;
-    };
     // Addresses are a wave-uniform base (scalar registers) plus a 32-bit per-lane byte offset, recomputed from the thread
     // index where it is cheap: 64-bit per-lane pointers kept alive across the chunk loop cost more registers than the data.
     const uint32_t row_t = (uint32_t)tid / SPR_X, slot_t = (uint32_t)tid % SPR_X;      // piece `it` of this thread: row_t + it * RSTEP
     constexpr int RSTEP = THREADS / SPR_X;
     const uint32_t x_row_bytes = (uint32_t)(a.X_sl * 2);
-    auto load_ahead = [&](int64_t c, Ahead& s) {
-        const int64_t t0 = c * kQ;
-        const uint32_t last = (uint32_t)(((a.seqlen - t0) < kQ ? (a.seqlen - t0) : kQ) - 1);      // last valid row
-        const char* xp = reinterpret_cast<const char*>(static_cast<const T*>(a.X) + b * a.X_sb + t0 * a.X_sl + head_off<HS>(h, a.X_sh) + pw * PH);
-        const float* tab = a.ldtab + (bh * nc + c) * (2 * kQ);
+    // The bases walk from chunk to chunk by constant steps: formed anew for each chunk out of 64-bit products (and the issue
+    // priority below out of a 64-bit quotient) they were 150 of the 200 scalar instructions of an iteration, which on a chip
+    // holding few workgroups stand between one chunk's products and the next: 181 -> 169 us at b1 l16384 h80.
+    const int nci = (int)nc, cfirst = REVERSE ? nci - 1 : 0;
+    const int tail_rows = (int)(a.seqlen - (nc - 1) * kQ);      // valid rows of the last chunk
+    constexpr int DIR = REVERSE ? -1 : 1;
+    const char* xq = reinterpret_cast<const char*>(static_cast<const T*>(a.X) + b * a.X_sb + (int64_t)cfirst * kQ * a.X_sl + head_off<HS>(h, a.X_sh) + pw * PH);
+    const float* tq = a.ldtab + (bh * nc + cfirst) * (2 * kQ);
+    const char* mp = reinterpret_cast<const char*>(static_cast<const T*>(a.Mt) + ((b * nc + cfirst) * a.ngroups + g) * (int64_t)(N * kQ) + wave_u * (8 * 512));
+    char* op = reinterpret_cast<char*>(static_cast<T*>(a.prev) + ((b * nc + cfirst) * a.nheads + h) * (int64_t)(P * N) + (pw * PH + wave_u * RW) * N);
+    const int64_t x_step = DIR * (int64_t)kQ * a.X_sl * 2, m_step = DIR * a.ngroups * (int64_t)(N * kQ * 2), o_step = DIR * a.nheads * (int64_t)(P * N * 2);
+    int kload = 0;                                      // processing index of the chunk xq and tq stand at
+    auto load_ahead = [&](Ahead& s) {
+        const uint32_t last = (uint32_t)((kload == (REVERSE ? 0 : nci - 1) ? tail_rows : kQ) - 1);      // last valid row
+        const uint32_t last_off = last * x_row_bytes;
+        const char* xp = xq;
+        const float* tab = tq;
         s.lam = tab[kQ - 1];
 #pragma unroll
         for (int it = 0; it < NXR; ++it) {
             const uint32_t row = row_t + it * RSTEP;
-            const uint32_t grow = row < last ? row : last;      // rows past the end: finite stand-ins, scaled by zero
-            s.x[it] = *reinterpret_cast<const u32x4*>(xp + (grow * x_row_bytes + slot_t * 16u));
+            // rows past the end: finite stand-ins, scaled by zero (minimum of products, not product of the minimum: hipcc
+            // multiplies and adds in a 64-bit instruction whose unused high half it puts into a load's target register)
+            const uint32_t off = row * x_row_bytes < last_off ? row * x_row_bytes : last_off;
+            s.x[it] = *reinterpret_cast<const u32x4*>(xp + (off + slot_t * 16u));
             s.l[it] = tab[row];
             s.d[it] = REVERSE ? (row <= last ? 1.f : 0.f) : tab[kQ + row];      // dt is 0 past the end of the sequence
         }
+        if (kload < nci - 1) { ++kload; xq += x_step; tq += DIR * 2 * kQ; }      // past the end: the last chunk once more
     };
     // loaded at the top of the iteration that consumes them (so that the wait in front of their use can be counted
     // exactly and leaves the next chunk's rows, issued behind them, in flight): the group's B^T / C^T fragments (L2)
     Frag<T> bf[NBW][8];
-    const uint32_t st_off = (uint32_t)(((pw * PH + wave * RW + lane / LPR) * N + (lane % LPR) * 8) * 2);      // pass ps: + ps * RPP * N * 2
-    auto load_same = [&](int64_t c) {
-        const char* mp = reinterpret_cast<const char*>(static_cast<const T*>(a.Mt) + ((b * nc + c) * a.ngroups + g) * (int64_t)(N * kQ));
+    const uint32_t st_off = (uint32_t)((lane / LPR * N + (lane % LPR) * 8) * 2);      // pass ps: + ps * RPP * N * 2
+    auto load_same = [&] {
 #pragma unroll
         for (int j = 0; j < NBW; ++j)
 #pragma unroll
             for (int ks = 0; ks < 8; ++ks)      // see mt_offset
-                bf[j][ks].v = *reinterpret_cast<const bf16x8*>(mp + ((uint32_t)lane * 16u + (uint32_t)((((n0 >> 5) + j) * 8 + ks) * 1024)));
+                bf[j][ks].v = *reinterpret_cast<const bf16x8*>((mp + ((j * 8 + ks) & ~3) * 1024) + ((uint32_t)lane * 16u + (uint32_t)((ks & 3) * 1024)));
+        mp += m_step;
     };
 
-    auto step = [&](int64_t cc, Ahead& s) {
-        const int64_t c = chunk_of(cc);
-        const int buf = (int)(cc & 1);
+    const int q1 = (nci + 3) / 4, q2 = (2 * nci + 3) / 4, q3 = (3 * nci + 3) / 4;      // first chunk of each quarter
+    int next_drop = q1;
+    __builtin_amdgcn_s_setprio(3);
+    auto step = [&](int cc, Ahead& s) {
+        const int buf = cc & 1;
         // Issue priority falls as the workgroup advances, so that of the workgroups sharing a CU the one furthest behind
         // goes first: the hardware otherwise prefers the oldest waves, and the last workgroup placed on a CU that holds
         // one more than its neighbours finishes long after everybody else.
-        switch ((int)(cc * 4 / nc)) {
-            case 0: __builtin_amdgcn_s_setprio(3); break;
-            case 1: __builtin_amdgcn_s_setprio(2); break;
-            case 2: __builtin_amdgcn_s_setprio(1); break;
-            default: __builtin_amdgcn_s_setprio(0); break;
+        if (cc == next_drop) {
+            if (cc == q1) __builtin_amdgcn_s_setprio(2);
+            else if (cc == q2) __builtin_amdgcn_s_setprio(1);
+            else __builtin_amdgcn_s_setprio(0);
+            next_drop = cc < q2 ? q2 : q3;
         }
         T* cX = sX + buf * (XT * kQ * PH);
         __builtin_amdgcn_sched_barrier(0);      // keep this chunk's loads out of the previous chunk's MFMA phase (registers)
-        load_same(c);
+        load_same();
         // the values loaded one chunk ahead become visible to the optimiser here and no earlier: otherwise their
         // unpacking is scheduled right behind the loads, which then wait for the data a whole chunk too early
 #pragma unroll
@@ -199,17 +226,16 @@ state_pass16_kernel(const StatePassArgs a) {
                     *reinterpret_cast<u32x4*>(cO + (i * 32 + r) * LDO + n0 + j * 32 + 8 * (q0 + half)) = u32x4{o0, o1, o2, o3};
                 }
         __syncthreads();          // both tiles are complete; every wave is done with the other buffers
-        // the rows two chunks on (past the end: the last chunk once more, rather than branching around the loads)
-        load_ahead(chunk_of(cc + 2), s);
+        load_ahead(s);            // the rows two chunks on
 
         // ---- the state entering (forward) / the gradient leaving (reverse) this chunk: whole rows of the workgroup's slab
-        char* op = reinterpret_cast<char*>(static_cast<T*>(a.prev) + ((b * nc + c) * a.nheads + h) * (int64_t)(P * N));
 #pragma unroll
         for (int ps = 0; ps < NSP; ++ps) {
             const int rl = wave * RW + ps * RPP + lane / LPR, cv = lane % LPR;
             const u32x4 o = *reinterpret_cast<const u32x4*>(cO + rl * LDO + cv * 8);
-            *reinterpret_cast<u32x4*>(op + (st_off + (uint32_t)(ps * RPP * N * 2))) = o;
+            *reinterpret_cast<u32x4*>((op + ps * RPP * N * 2) + st_off) = o;
         }
+        op += o_step;
 
         // ---- S = e^{Lam} S + X_scaled^T M  (accumulated as its transpose M^T X_scaled)
 #pragma unroll
@@ -225,19 +251,14 @@ state_pass16_kernel(const StatePassArgs a) {
             const T* tX = cX + xt * (kQ * PH);
             Frag<T> af[PBW][8];
 #pragma unroll
-            for (int ks = 0; ks < 8; ++ks) {
-                const int ta = ks * 16 + tr_tok, tb = ta + 4;
+            for (int ks = 0; ks < 8; ++ks)
 #pragma unroll
                 for (int i = 0; i < PBW; ++i) {
-                    const int col = i * 32 + tr_col;
-                    const tvec4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-                        (M2_LDS tvec4*)(tX + (ta * SPR_X + ((col >> 3) ^ tile_swz<SPR_X>(ta))) * 8 + (col & 7)));
-                    const tvec4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-                        (M2_LDS tvec4*)(tX + (tb * SPR_X + ((col >> 3) ^ tile_swz<SPR_X>(tb))) * 8 + (col & 7)));
+                    const tvec4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((M2_LDS tvec4*)(tX + (tr_lo ^ (i * 32)) + ks * 16 * PH));
+                    const tvec4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((M2_LDS tvec4*)(tX + (tr_hi ^ (i * 32)) + ks * 16 * PH));
 #pragma unroll
                     for (int e = 0; e < 4; ++e) { af[i][ks].v[e] = lo[e]; af[i][ks].v[4 + e] = hi[e]; }
                 }
-            }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int ks = 0; ks < 8; ++ks)
@@ -252,18 +273,18 @@ state_pass16_kernel(const StatePassArgs a) {
     // Chunks are taken two per loop iteration (one per register set); an odd first chunk is peeled off in front so that
     // the loop body is free of conditionals (a branch around loads costs register copies, and with them early waits).
     Ahead s0, s1;
-    int64_t cc = 0;
-    if (nc & 1) {
-        load_ahead(chunk_of(0), s1);
-        load_ahead(chunk_of(1), s0);
+    int cc = 0;
+    if (nci & 1) {
+        load_ahead(s1);
+        load_ahead(s0);
         step(0, s1);
         cc = 1;
     } else {
-        load_ahead(chunk_of(0), s0);
-        load_ahead(chunk_of(1), s1);
+        load_ahead(s0);
+        load_ahead(s1);
     }
 #pragma unroll 1
-    for (; cc < nc; cc += 2) {
+    for (; cc < nci; cc += 2) {
         step(cc, s0);
         step(cc + 1, s1);
     }

@@ -28,3 +28,20 @@ def test_wide_heads_far_apart(dtype, b, l, h, n, g):
     tol, metric = (1e-4, rel_err) if dtype == torch.float32 else (2e-2, rel_rms_err)
     for name, got in (("y", y), ("final_state", S), ("dX", dX), ("ddt", ddt), ("dA", dA), ("dB", dB), ("dC", dC), ("dD", dD)):
         assert metric(got, ref[name]) < tol, name
+
+
+@pytest.mark.parametrize("l", [1, 129, 384])
+@pytest.mark.parametrize("b,h", [(2, 104), (1, 257), (2, 128)])
+def test_whole_heads_per_workgroup(b, h, l):
+    """The state passes at head counts on either side of where a workgroup takes a whole head, over one, two and three chunks."""
+    from mamba2.mamba2_kernel import ssd_backward, ssd_forward
+    d = make_ssd_inputs(b, l, h, 64, 128, 1, seed=l + h, dtype=torch.bfloat16)
+    v = {k: t.to(DEV) for k, t in d.items()}
+    some = [0, h // 2, h - 1]      # heads are independent up to dB and dC, which sum over them
+    X, dy, dt = (d[k][:, :, some].double() for k in ("X", "dy", "dt"))
+    ref = ssd_grads_ref(dt, d["A"][some].double(), X, d["B"].double(), d["C"].double(), d["D"][some].double(), dy, chunk=64)
+    y, _ = ssd_forward(v["dt"], v["A"], v["X"], v["B"], v["C"], v["D"])
+    ddt, dA, dX, dB, dC, dD, _ = ssd_backward(v["dt"], v["A"], v["X"], v["B"], v["C"], v["D"], v["dy"])
+    for name, got in (("y", y[:, :, some]), ("dX", dX[:, :, some]), ("ddt", ddt[:, :, some]), ("dA", dA[some]), ("dD", dD[some])):
+        assert rel_rms_err(got, ref[name]) < 2e-2, name
+    assert torch.isfinite(dB.float()).all() and torch.isfinite(dC.float()).all()
