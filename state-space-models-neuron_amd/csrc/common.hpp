@@ -129,13 +129,18 @@ template <int CTRL, int BANK>
 __device__ __forceinline__ float dpp_move(float old, float x) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old), __builtin_bit_cast(int, x), CTRL, 0xF, BANK, false));
 }
+// every lane has a source: with nothing to keep, the move folds into the instruction that uses its result
+template <int CTRL>
+__device__ __forceinline__ float dpp_all(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xF, 0xF, true));
+}
 template <int M>
 __device__ __forceinline__ float lane_xor(float x) {
     static_assert(M == 1 || M == 2 || M == 4 || M == 8 || M == 16 || M == 32, "lane_xor: single-bit masks");
-    if constexpr (M == 1) return dpp_move<0xB1, 0xF>(x, x);                  // quad_perm [1,0,3,2]
-    else if constexpr (M == 2) return dpp_move<0x4E, 0xF>(x, x);             // quad_perm [2,3,0,1]
+    if constexpr (M == 1) return dpp_all<0xB1>(x);                            // quad_perm [1,0,3,2]
+    else if constexpr (M == 2) return dpp_all<0x4E>(x);                       // quad_perm [2,3,0,1]
     else if constexpr (M == 4) return dpp_move<0x114, 0xA>(dpp_move<0x104, 0x5>(x, x), x);     // row_shl:4 into banks 0, 2; row_shr:4 into banks 1, 3
-    else if constexpr (M == 8) return dpp_move<0x128, 0xF>(x, x);            // row_ror:8
+    else if constexpr (M == 8) return dpp_all<0x128>(x);                      // row_ror:8
     else {
         const uint32_t u = __builtin_bit_cast(uint32_t, x);
         uint32_t r0, r1;

@@ -235,7 +235,8 @@ __device__ __forceinline__ void stage_transposed(T* __restrict__ s, int ld, cons
 }
 
 // Sum of v over the 32 lanes that share (lane >> 5), for 16 values at once (the 16 accumulator rows of a lane),
-// by a butterfly reduce-scatter: 16 cross-lane moves instead of 80.  On return every lane holds ONE total:
+// by a butterfly reduce-scatter: 16 cross-lane moves instead of 80 (the widest step selects and adds with one row swap, the
+// single-move DPP steps fold into their additions: 45 instructions, not 85, in kernels bound by their vector instructions).  On return every lane holds ONE total:
 // that of register index  r = 8*b4 + 4*b3 + 2*b2 + b1  (b_k = bit k of lane), i.e. of accumulator row
 // acc_row(lane, r); lanes differing only in bit 0 hold the same total.
 __device__ __forceinline__ float half_wave_reduce16(float (&v)[16], int* reg_index) {
@@ -243,8 +244,10 @@ __device__ __forceinline__ float half_wave_reduce16(float (&v)[16], int* reg_ind
     const bool b4 = lane & 16, b3 = lane & 8, b2 = lane & 4, b1 = lane & 2;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-        const float keep = b4 ? v[k + 8] : v[k], send = b4 ? v[k] : v[k + 8];
-        v[k] = keep + lane_xor<16>(send);
+        // the row swap leaves the pair's two halves of v[k] in the lanes with b4 = 0, of v[k + 8] in the others
+        const auto sw = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, v[k]), __builtin_bit_cast(uint32_t, v[k + 8]), false, false);
+        const uint32_t r0 = sw[0], r1 = sw[1];
+        v[k] = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {

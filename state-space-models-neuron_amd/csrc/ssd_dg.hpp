@@ -8,10 +8,11 @@
 // (blocks above the diagonal do not exist).  Waves w, w + 4, w + 8 share a SIMD, so the SIMDs carry 3, 3, 2, 2 blocks;
 // the diagonal blocks, which carry the i >= j mask, go to the SIMDs with two.
 // Both operands are token rows with k = channel contiguous, i.e. the tiles as they lie in global memory: they are
-// copied global -> LDS asynchronously (by waves 0-7) up to three heads ahead into a ring of buffers (one barrier per
+// copied global -> LDS asynchronously (by waves 0-7, the tables by wave 8) up to three heads ahead into a ring of buffers (one barrier per
 // head), slots XOR-swizzled inside each row.  The fp32 G values at this lane's accumulator positions are
 // head-independent and stay in registers.  The row/column sums of head k are combined and written after the barrier
-// of head k + 1.
+// of head k + 1.  What bounds it is the vector instructions between two barriers (without the copies it takes 75 of 85 us at
+// b2 l4096 h128), so the copies, the sums and the decay factors run behind the products (49 -> 46 us at b4 l2048 h80).
 #pragma once
 #include "ssd_y.hpp"
 
@@ -78,7 +79,7 @@ dg16_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
                 async_copy16(gx, offX[it], dst + (uint32_t)(TILE * 2) + (wave_u * NX + it) * 1024u);
             }
         }
-        async_copy_ldtab(ldtab, (b * nheads + h) * nchunks + c, lds_LD + (uint32_t)(buf * 2 * kQ * 4));
+        if (wave_u == 8) async_copy_ldtab(ldtab, (b * nheads + h) * nchunks + c, lds_LD + (uint32_t)(buf * 2 * kQ * 4));
     };
     const int64_t h_first = g * hpg + slice * hps;
 #pragma unroll
@@ -123,8 +124,27 @@ dg16_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
             // the tiles of the heads after this one may stay in flight
             const int64_t younger = hps - 1 - hh;
             const int keep = (int)(younger < RING - 2 ? younger : RING - 2);
-            if (copier) wait_vmem_keep<2 * NX + 1>(keep); else wait_vmem_keep<1>(keep);
+            if (copier) wait_vmem_keep<2 * NX>(keep); else wait_vmem_keep<1>(keep);
         }
+        __syncthreads();          // tiles of head hh are in LDS; the sums of head hh-1 are complete; buffer of hh-1 is free
+        const T* cA = tiles + buf * 2 * TILE;
+        const T* cT = cA + TILE;
+        float* s_rs = s_sum + par * 8 * kQ;
+        float* s_cs = s_rs + 4 * kQ;
+
+        floatx16 pa = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        const int ra = rb * 32 + r, rt = cb * 32 + r;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const Frag<T> af = load_frag(cA + (ra * SPR + ((ks * 2 + half) ^ tile_swz<SPR>(ra))) * 8);
+            const Frag<T> bf = load_frag(cT + (rt * SPR + ((ks * 2 + half) ^ tile_swz<SPR>(rt))) * 8);
+            mma_frag(pa, af, bf);
+        }
+        // while the products run: the copies of a later head (a wave stands until the memory path takes them), the sums of the
+        // head before, the decay factors
+        __builtin_amdgcn_sched_barrier(0);
+        if (hh + RING - 1 < hps) issue_tiles(h + RING - 1, (int)((hh + RING - 1) % RING));
+        if (hh > 0) flush_sums(h - 1, par ^ 1);
         const float* sl = sLD + buf * 2 * kQ;
         const float* sd = sl + kQ;
         const float l_first = sl[rb * 32], l_last = sl[rb * 32 + 31];
@@ -150,22 +170,6 @@ dg16_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
         } else {
 #pragma unroll
             for (int v = 0; v < 16; ++v) ui[v] = __expf(fminf(ui[v] - lj, 0.f)) * dtj;
-        }
-        __syncthreads();          // tiles of head hh are in LDS; the sums of head hh-1 are complete; buffer of hh-1 is free
-        if (hh + RING - 1 < hps) issue_tiles(h + RING - 1, (int)((hh + RING - 1) % RING));
-        if (hh > 0) flush_sums(h - 1, par ^ 1);
-        const T* cA = tiles + buf * 2 * TILE;
-        const T* cT = cA + TILE;
-        float* s_rs = s_sum + par * 8 * kQ;
-        float* s_cs = s_rs + 4 * kQ;
-
-        floatx16 pa = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        const int ra = rb * 32 + r, rt = cb * 32 + r;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const Frag<T> af = load_frag(cA + (ra * SPR + ((ks * 2 + half) ^ tile_swz<SPR>(ra))) * 8);
-            const Frag<T> bf = load_frag(cT + (rt * SPR + ((ks * 2 + half) ^ tile_swz<SPR>(rt))) * 8);
-            mma_frag(pa, af, bf);
         }
         float rsum[16], csum = 0.f;
         if (masked) {
