@@ -129,6 +129,11 @@ template <int CTRL, int BANK>
 __device__ __forceinline__ float dpp_move(float old, float x) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old), __builtin_bit_cast(int, x), CTRL, 0xF, BANK, false));
 }
+// zero where there is no source (or the lane's row is masked out)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_from(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, ROWS, 0xF, false));
+}
 // every lane has a source: with nothing to keep, the move folds into the instruction that uses its result
 template <int CTRL>
 __device__ __forceinline__ float dpp_all(float x) {

@@ -268,68 +268,18 @@ __device__ __forceinline__ float half_wave_reduce16(float (&v)[16], int* reg_ind
     return v[0];
 }
 
-// Wave-private chunk cumulative sum: every wave computes l for all 128 tokens by itself (lane holds tokens
-// `lane` and `lane + 64`), so no block barrier is needed.  Tokens >= valid behave as dt = 0.
-// Split in two so that the loads of the next head's dt can be issued long before they are needed.
-template <typename T>
-__device__ __forceinline__ void wave_dt_load(const void* __restrict__ dt, int dt_f32, int64_t off, int64_t stride_l,
-                                             int valid, float& d0, float& d1) {
-    const int lane = threadIdx.x & 63;
-    d0 = 0.f; d1 = 0.f;
-    if (dt_f32) {
-        const float* p = static_cast<const float*>(dt) + off;
-        if (lane < valid) d0 = p[(int64_t)lane * stride_l];
-        if (lane + 64 < valid) d1 = p[(int64_t)(lane + 64) * stride_l];
-    } else {
-        const T* p = static_cast<const T*>(dt) + off;
-        if (lane < valid) d0 = to_f32(p[(int64_t)lane * stride_l]);
-        if (lane + 64 < valid) d1 = to_f32(p[(int64_t)(lane + 64) * stride_l]);
-    }
+// Inclusive sum over the lanes of a wave in six DPP additions: row shifts inside the rows of 16 lanes, then the last lane of
+// row 0 (2) broadcast to row 1 (3), and lane 31 to the upper half.  All 64 lanes must be active.
+__device__ __forceinline__ float wave_scan(float x) {
+    x += dpp_from<0x111, 0xF>(x); x += dpp_from<0x112, 0xF>(x); x += dpp_from<0x114, 0xF>(x); x += dpp_from<0x118, 0xF>(x);      // row_shr
+    x += dpp_from<0x142, 0xA>(x);      // row_bcast:15
+    x += dpp_from<0x143, 0xC>(x);      // row_bcast:31
+    return x;
 }
-// The same loads without conversion or divergent branches (addresses of tokens >= valid are clamped), so that
-// nothing forces a wait for them where they are issued; wave_dt_cvt turns them into dt values where they are used.
-template <typename T>
-__device__ __forceinline__ void wave_dt_load_raw(const void* __restrict__ dt, int dt_f32, int64_t off, int64_t stride_l,
-                                                 int valid, uint32_t& r0, uint32_t& r1) {
-    const int lane = threadIdx.x & 63;
-    const int t0 = lane < valid ? lane : valid - 1, t1 = lane + 64 < valid ? lane + 64 : valid - 1;
-    if (dt_f32) {
-        const uint32_t* p = static_cast<const uint32_t*>(dt) + off;
-        r0 = p[(int64_t)t0 * stride_l]; r1 = p[(int64_t)t1 * stride_l];
-    } else {
-        static_assert(sizeof(T) == 2 || sizeof(T) == 4, "dt element size");
-        if (sizeof(T) == 2) {
-            const uint16_t* p = static_cast<const uint16_t*>(dt) + off;
-            r0 = p[(int64_t)t0 * stride_l]; r1 = p[(int64_t)t1 * stride_l];
-        } else {
-            const uint32_t* p = static_cast<const uint32_t*>(dt) + off;
-            r0 = p[(int64_t)t0 * stride_l]; r1 = p[(int64_t)t1 * stride_l];
-        }
-    }
-}
-template <typename T>
-__device__ __forceinline__ void wave_dt_cvt(int dt_f32, int valid, uint32_t r0, uint32_t r1, float& d0, float& d1) {
-    const int lane = threadIdx.x & 63;
-    if (dt_f32 || sizeof(T) == 4) { d0 = __uint_as_float(r0); d1 = __uint_as_float(r1); }
-    else { d0 = __uint_as_float(r0 << 16); d1 = __uint_as_float(r1 << 16); }      // bf16 bits -> fp32
-    if (lane >= valid) d0 = 0.f;
-    if (lane + 64 >= valid) d1 = 0.f;
-}
+// l[t] = sum_{s <= t} A d[s] over a chunk, lane holding tokens `lane` and `lane + 64`
 __device__ __forceinline__ void wave_cumsum_from(float A, float d0, float d1, float& l0, float& l1) {
-    const int lane = threadIdx.x & 63;
-    l0 = A * d0; l1 = A * d1;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const float n0 = __shfl_up(l0, o, 64), n1 = __shfl_up(l1, o, 64);
-        if (lane >= o) { l0 += n0; l1 += n1; }
-    }
+    l0 = wave_scan(A * d0); l1 = wave_scan(A * d1);
     l1 += __shfl(l0, 63, 64);
-}
-template <typename T>
-__device__ __forceinline__ void wave_chunk_cumsum(const void* __restrict__ dt, int dt_f32, int64_t off, int64_t stride_l,
-                                                  int valid, float A, float& l0, float& l1, float& d0, float& d1) {
-    wave_dt_load<T>(dt, dt_f32, off, stride_l, valid, d0, d1);
-    wave_cumsum_from(A, d0, d1, l0, l1);
 }
 
 // Per (batch, head, chunk) the cumulative log-decay and dt are computed once (ld_table_body, prep_kernel) into a table of
@@ -348,43 +298,6 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Inclusive cumulative sum l[t] = sum_{s<=t} A * dt[s] over one chunk (kQ = 128 tokens), in fp32.
-// Tokens >= valid behave as dt = 0 (no decay, no input).  Results in LDS: s_l[kQ], s_dt[kQ].
-// Must be called by all threads of the block (contains barriers); blockDim.x >= 128.
-template <typename DT>
-__device__ __forceinline__ void chunk_cumsum(const DT* __restrict__ dt, int64_t stride_l, int valid, float A,
-                                             float* __restrict__ s_l, float* __restrict__ s_dt,
-                                             float* __restrict__ s_tmp, int tid) {
-    float a = 0.f, d = 0.f;
-    if (tid < kQ) {
-        if (tid < valid) d = to_f32(dt[(int64_t)tid * stride_l]);
-        a = A * d;
-        const int lane = tid & 63;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const float nb = __shfl_up(a, off, 64);
-            if (lane >= off) a += nb;
-        }
-        if (tid == 63) s_tmp[0] = a;
-    }
-    __syncthreads();
-    if (tid < kQ) {
-        if (tid >= 64) a += s_tmp[0];
-        s_l[tid] = a;
-        s_dt[tid] = d;
-    }
-    __syncthreads();
-}
-
-// dt is stored either as fp32 or in the activation type T; `off` is the element offset of token 0.
-template <typename T>
-__device__ __forceinline__ void chunk_cumsum_any(const void* __restrict__ dt, int dt_f32, int64_t off, int64_t stride_l,
-                                                 int valid, float A, float* __restrict__ s_l, float* __restrict__ s_dt,
-                                                 float* __restrict__ s_tmp, int tid) {
-    if (dt_f32) chunk_cumsum<float>(static_cast<const float*>(dt) + off, stride_l, valid, A, s_l, s_dt, s_tmp, tid);
-    else chunk_cumsum<T>(static_cast<const T*>(dt) + off, stride_l, valid, A, s_l, s_dt, s_tmp, tid);
 }
 
 }  // namespace m2

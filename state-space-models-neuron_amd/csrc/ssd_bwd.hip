@@ -607,7 +607,7 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
     M2_REQUIRE(p->nheads <= 65535, M2_ERR_SHAPE, "ssd_bwd: too many group slices");
     int rc;
     // decay tables, G (+ operand tiles) and the state entering each chunk, unless the caller kept the forward's
-    if (!p->chunk_states && (rc = ssd_launch_states<T, P, N, HS>(p, w, nullptr, st))) return rc;
+    if (!p->chunk_states && (rc = ssd_launch_states<T, P, N, HS>(p, w, nullptr, false, true, st))) return rc;
     // gradient of the state leaving each chunk (reverse recurrence over the chunks' own contributions)
     if constexpr (sizeof(T) == 2) {
         StatePassArgs sa;

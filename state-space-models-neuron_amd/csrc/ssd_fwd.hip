@@ -30,7 +30,7 @@ int ssd_fwd_impl(const SsdCall* p, hipStream_t st) {
     const int64_t nc = ceil_div(p->seqlen, (int64_t)kQ);
     const SsdWorkspace w = ssd_carve(p, p->workspace, false);
     int rc;
-    if ((rc = ssd_launch_states<T, P, N, HS>(p, w, p->final_state, st))) return rc;
+    if ((rc = ssd_launch_states<T, P, N, HS>(p, w, p->final_state, true, p->chunk_states != nullptr, st))) return rc;
     DiagArgs a{};
     a.D = p->D;
     a.Aoff = p->C; a.Ao_sb = p->C_stride_b; a.Ao_sl = p->C_stride_l; a.Ao_sg = p->C_stride_g;

@@ -83,7 +83,7 @@ inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_
         w.prev = keep(tiles * esz);
         w.lam = reinterpret_cast<float*>(keep(bhc * 4));
         w.ldtab = reinterpret_cast<float*>(keep(bhc * 2 * kQ * 4));
-        w.G = reinterpret_cast<float*>(keep(grp * kQ * kQ * 4));
+        if (p->dtype != M2_F32) w.G = reinterpret_cast<float*>(keep(grp * kQ * kQ * 4));      // fp32 operands: Gm is G already
         w.Gm = keep(grp * kQ * kQ * esz);
         w.Gmt = keep(grp * kQ * kQ * esz);
         w.Bt = keep(grp * p->dstate * kQ * esz);
@@ -163,7 +163,10 @@ inline int allow_smem(K kernel, size_t bytes) {
 template <typename T, int P, int N>
 inline size_t state_smem() { return (size_t)(P + N) * lds_ld<T>(kQ) * sizeof(T); }
 template <typename T>
-inline size_t cb_smem(int n) { return (size_t)2 * 64 * lds_ld<T>(n) * sizeof(T); }
+inline size_t cb_smem(int n) {      // operand rows; 32 tokens of both to transpose; the waves' blocks on their way out
+    const size_t a = (size_t)2 * 64 * lds_ld<T>(cb_kh<T>(n)) * sizeof(T), b = (size_t)2 * 32 * lds_ld<T>(n) * sizeof(T), o = (size_t)4 * 32 * 36 * 4;
+    return a > b ? (a > o ? a : o) : (b > o ? b : o);
+}
 
 template <typename T, int P, int N, bool REVERSE, int HS, bool HILO>
 inline int launch_state_pass16(const StatePassArgs& a, int64_t batch, hipStream_t st) {
@@ -180,9 +183,10 @@ inline int launch_state_pass16(const StatePassArgs& a, int64_t batch, hipStream_
 }
 
 // Decay tables, G = C B^T (+ operand tiles), local chunk states, forward state scan.  Used by the forward and, when the
-// caller did not keep the forward's chunk_states buffer, by the backward (recompute).
+// caller did not keep the forward's chunk_states buffer, by the backward (recompute).  for_fwd, for_bwd: which of the operand
+// tiles will be read.
 template <typename T, int P, int N, int HS>
-inline int ssd_launch_states(const SsdCall* p, const SsdWorkspace& w, float* final_out, hipStream_t st) {
+inline int ssd_launch_states(const SsdCall* p, const SsdWorkspace& w, float* final_out, bool for_fwd, bool for_bwd, hipStream_t st) {
     const int64_t nc = ceil_div(p->seqlen, (int64_t)kQ);
     const T* x = static_cast<const T*>(p->x);
     const T* Bm = static_cast<const T*>(p->B);
@@ -195,14 +199,16 @@ inline int ssd_launch_states(const SsdCall* p, const SsdWorkspace& w, float* fin
         const size_t sm = cb_smem<T>(N);
         if ((rc = allow_smem(k, sm))) return rc;
         PrepArgs pa;
-        pa.Bm = Bm; pa.Cm = Cm; pa.Gf = w.G; pa.Gm = w.Gm; pa.Gmt = w.Gmt; pa.Bt = w.Bt; pa.Ct = w.Ct;
+        pa.Bm = Bm; pa.Cm = Cm; pa.Bt = w.Bt;
+        pa.Gf = for_bwd ? w.G : nullptr; pa.Gmt = for_bwd ? w.Gmt : nullptr; pa.Ct = for_bwd ? w.Ct : nullptr;
+        pa.Gm = for_fwd || sizeof(T) == 4 ? w.Gm : nullptr;
         pa.Bsb = p->B_stride_b; pa.Bsl = p->B_stride_l; pa.Bsg = p->B_stride_g;
         pa.Csb = p->C_stride_b; pa.Csl = p->C_stride_l; pa.Csg = p->C_stride_g;
         pa.dt = p->dt; pa.dt_f32 = dt_f32; pa.dt_bias = p->dt_bias; pa.A = p->A; pa.ldtab = w.ldtab; pa.lam = w.lam;
         pa.dtsb = p->dt_stride_b; pa.dtsl = p->dt_stride_l;
         pa.seqlen = p->seqlen; pa.nheads = p->true_heads; pa.hs = p->hs; pa.ngroups = p->ngroups; pa.nchunks = nc;
         pa.n_cb = nc * p->ngroups * p->batch;
-        const int64_t blocks = kCbParts * pa.n_cb + ld_table_blocks(p->batch, p->true_heads, nc);
+        const int64_t blocks = cb_blocks(pa.n_cb) + ld_table_blocks(p->batch, p->true_heads, nc);
         M2_REQUIRE(blocks < ((int64_t)1 << 31), M2_ERR_SHAPE, "ssd: too many workgroups");
         k<<<(unsigned)blocks, 256, sm, st>>>(pa);
         if ((rc = check_launch("ssd prep_kernel"))) return rc;

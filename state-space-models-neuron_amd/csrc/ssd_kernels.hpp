@@ -20,6 +20,8 @@
 //                      (REVERSE variant: gradient recurrence + <dS, S> per chunk)
 // The last two serve fp32 operands; for 16-bit operands ssd_states16.hpp does both in one pass.
 #pragma once
+#include <type_traits>
+
 #include "mma.hpp"
 
 namespace m2 {
@@ -30,6 +32,7 @@ namespace m2 {
 //   Gf  [kQ][kQ] fp32            G[i][j] (all blocks with block-row >= block-col)
 //   Gm  [kQ][kQ] T               causal G:  G[i][j] for i >= j, else 0         (forward diagonal term, rows i)
 //   Gmt [kQ][kQ] T               its transpose: Gmt[j][i] = G[i][j] for i >= j (backward dx term, rows j)
+//   (each of Gf, Gm, Gmt and Ct only where it is not null: the forward alone reads Gm and Bt)
 //   Bt, Ct N x kQ T              B and C transposed (tokens contiguous), laid out by mt_offset: MFMA operands of the
 //                                chunk-state products
 // kCbParts workgroups of 256 threads per (chunk, group, batch), see cb_body.  The upper-right 64x64 quadrant of G is
@@ -48,6 +51,11 @@ __device__ __forceinline__ int64_t mt_offset(int n, int s0) {
 // Workgroups per (chunk, group, batch): three for the 64x64 quadrants of G on and below the diagonal, four for the
 // transposed tiles (32 tokens each) -- seven short independent pieces rather than two long ones.
 constexpr int kCbParts = 7;
+constexpr int kXcds = 8;
+__host__ __device__ inline int64_t cb_blocks(int64_t n_cb) { return (n_cb + kXcds - 1) / kXcds * kXcds * kCbParts; }
+// Contraction length staged at once: all of it (one staging phase, one barrier), but fp32 rows of 128 in two halves, so that
+// four workgroups fit a CU and not two (66 -> 51 us at b3 l2048 h32 g8).
+template <typename T> __host__ __device__ constexpr int cb_kh(int n) { return sizeof(T) == 4 && n > 64 ? n / 2 : n; }
 template <typename T, int N>
 __device__ __forceinline__ void
 cb_body(const T* __restrict__ Bm, const T* __restrict__ Cm, float* __restrict__ Gf, T* __restrict__ Gm, T* __restrict__ Gmt,
@@ -55,11 +63,11 @@ cb_body(const T* __restrict__ Bm, const T* __restrict__ Cm, float* __restrict__ 
         int64_t seqlen, int64_t ngroups, int64_t nchunks,
         int64_t Bsb, int64_t Bsl, int64_t Bsg, int64_t Csb, int64_t Csl, int64_t Csg, int64_t c, int64_t g, int64_t b,
         const int part) {
-    constexpr int LD = lds_ld<T>(N);      // the whole contraction length at once: one staging phase, one barrier
+    constexpr int KH = cb_kh<T>(N), LD = lds_ld<T>(KH);
     constexpr int V = VecTraits<T>::kVec;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T* sC = reinterpret_cast<T*>(smem_raw);      // [64][LD]
-    T* sB = sC + 64 * LD;                        // [64][LD]
+    T* sB = sC + 64 * LD;                        // [64][LD], the transposing parts: behind [32][LDT]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int64_t t0 = c * kQ;
     const int valid = (int)((seqlen - t0) < kQ ? (seqlen - t0) : kQ);
@@ -69,122 +77,157 @@ cb_body(const T* __restrict__ Bm, const T* __restrict__ Cm, float* __restrict__ 
     if (part >= 3) {
         // transposed copies of tokens [tk0, tk0 + 32): thread -> (state column n, group of V tokens)
         const int tk0 = (part - 3) * 32;
+        constexpr int LDT = lds_ld<T>(N);
+        T* sBt = sC + 32 * LDT;
         T* Btp = Bt + grp * (int64_t)(N * kQ);
-        T* Ctp = Ct + grp * (int64_t)(N * kQ);
-        stage_rows<T, 32, N, 256, false>(sC, LD, Cp + (int64_t)tk0 * Csl, Csl, valid - tk0, nullptr, tid);
-        stage_rows<T, 32, N, 256, false>(sB, LD, Bp + (int64_t)tk0 * Bsl, Bsl, valid - tk0, nullptr, tid);
+        T* Ctp = Ct ? Ct + grp * (int64_t)(N * kQ) : nullptr;
+        if (Ct) stage_rows<T, 32, N, 256, false>(sC, LDT, Cp + (int64_t)tk0 * Csl, Csl, valid - tk0, nullptr, tid);
+        stage_rows<T, 32, N, 256, false>(sBt, LDT, Bp + (int64_t)tk0 * Bsl, Bsl, valid - tk0, nullptr, tid);
         __syncthreads();
         for (int e = tid; e < N * (32 / V); e += 256) {
             const int n = e % N, s0 = (e / N) * V;
-            T vb[V], vc[V];
+            T v[V];
 #pragma unroll
-            for (int q = 0; q < V; ++q) { vb[q] = sB[(s0 + q) * LD + n]; vc[q] = sC[(s0 + q) * LD + n]; }
-            *reinterpret_cast<uint4*>(Btp + mt_offset<T>(n, tk0 + s0)) = *reinterpret_cast<const uint4*>(vb);
-            *reinterpret_cast<uint4*>(Ctp + mt_offset<T>(n, tk0 + s0)) = *reinterpret_cast<const uint4*>(vc);
+            for (int q = 0; q < V; ++q) v[q] = sBt[(s0 + q) * LDT + n];
+            *reinterpret_cast<uint4*>(Btp + mt_offset<T>(n, tk0 + s0)) = *reinterpret_cast<const uint4*>(v);
+            if (Ct) {
+#pragma unroll
+                for (int q = 0; q < V; ++q) v[q] = sC[(s0 + q) * LDT + n];
+                *reinterpret_cast<uint4*>(Ctp + mt_offset<T>(n, tk0 + s0)) = *reinterpret_cast<const uint4*>(v);
+            }
         }
         return;
     }
     // quadrant (wm, wn) of G = C B^T; wave (wi, wj) takes one 32x32 block of it
     const int wm = part == 0 ? 0 : 1, wn = part == 2 ? 1 : 0;
     const int wi = wave >> 1, wj = wave & 1;
-    stage_rows<T, 64, N, 256, false>(sC, LD, Cp + (int64_t)(wm * 64) * Csl, Csl, valid - wm * 64, nullptr, tid);
-    stage_rows<T, 64, N, 256, false>(sB, LD, Bp + (int64_t)(wn * 64) * Bsl, Bsl, valid - wn * 64, nullptr, tid);
-    __syncthreads();
-    if (wm * 2 + wi < wn * 2 + wj) return;          // block above the diagonal
+    const bool live = wm * 2 + wi >= wn * 2 + wj;   // else a block above the diagonal
     floatx16 acc[1][1];
     acc_zero(acc);
-    wave_mma<1, 1>(acc, sC + wi * 32 * LD, LD, sB + wj * 32 * LD, LD, 0, N);
-    float* Gfp = Gf + grp * (int64_t)(kQ * kQ);
-    T* Gmp = Gm + grp * (int64_t)(kQ * kQ);
-    T* Gmtp = Gmt + grp * (int64_t)(kQ * kQ);
-    const int col = wn * 64 + wj * 32 + acc_col(lane);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int rowq = wm * 64 + wi * 32 + 8 * q + 4 * (lane >> 5);
-        T mt[4];
+    for (int n0 = 0; n0 < N; n0 += KH) {
+        if (n0) __syncthreads();
+        stage_rows<T, 64, KH, 256, false>(sC, LD, Cp + (int64_t)(wm * 64) * Csl + n0, Csl, valid - wm * 64, nullptr, tid);
+        stage_rows<T, 64, KH, 256, false>(sB, LD, Bp + (int64_t)(wn * 64) * Bsl + n0, Bsl, valid - wn * 64, nullptr, tid);
+        __syncthreads();
+        if (live) wave_mma<1, 1>(acc, sC + wi * 32 * LD, LD, sB + wj * 32 * LD, LD, 0, KH);
+    }
+    __syncthreads();                                // the operand tiles give way to the four waves' blocks
+    if (!live) return;
+    // The block leaves through LDS: eight lanes store a row (of G, or of its transpose) of 32 elements, where accumulator
+    // registers would go out one element (or four of a column) at a time -- 36 store instructions per wave instead of 12.
+    constexpr int LDG = 36;                         // 4 rows on: 16 banks on
+    float* blk = reinterpret_cast<float*>(smem_raw) + wave * (32 * LDG);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int row = rowq + e;
-            const float gv = acc[0][0][4 * q + e];
-            const float gm = row >= col ? gv : 0.f;
-            Gfp[row * kQ + col] = gv;
-            Gmp[row * kQ + col] = from_f32<T>(gm);
-            mt[e] = from_f32<T>(gm);
+    for (int v = 0; v < 16; ++v) blk[acc_row(lane, v) * LDG + acc_col(lane)] = acc[0][0][v];
+    wave_lds_sync();
+    const int i0 = wm * 64 + wi * 32, j0 = wn * 64 + wj * 32;      // first row, first column of the block
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+        const int a = it * 8 + (lane >> 3), k0 = (lane & 7) * 4;   // row of the output, first of its four elements
+        const floatx4 v = *reinterpret_cast<const floatx4*>(blk + a * LDG + k0);
+        if (Gf) *reinterpret_cast<floatx4*>(Gf + grp * (int64_t)(kQ * kQ) + (i0 + a) * kQ + j0 + k0) = v;
+        if (Gm) {
+            T o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = from_f32<T>(i0 + a >= j0 + k0 + e ? v[e] : 0.f);
+            *reinterpret_cast<RawVec<T, 4>*>(Gm + grp * (int64_t)(kQ * kQ) + (i0 + a) * kQ + j0 + k0) = *reinterpret_cast<const RawVec<T, 4>*>(o);
         }
-        *reinterpret_cast<RawVec<T, 4>*>(Gmtp + col * kQ + rowq) = *reinterpret_cast<const RawVec<T, 4>*>(mt);
+        if (Gmt) {
+            T o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = from_f32<T>(i0 + k0 + e >= j0 + a ? blk[(k0 + e) * LDG + a] : 0.f);
+            *reinterpret_cast<RawVec<T, 4>*>(Gmt + grp * (int64_t)(kQ * kQ) + (j0 + a) * kQ + i0 + k0) = *reinterpret_cast<const RawVec<T, 4>*>(o);
+        }
     }
 }
 
 // ------------------------------------------------------------------------------------------
-// Cumulative log-decay table: one wave per (batch, head, chunk); ldtab[bhc] = [ l[0..kQ) | dt[0..kQ) ] in fp32,
+// Cumulative log-decay table per (batch, head, chunk): ldtab[bhc] = [ l[0..kQ) | dt[0..kQ) ] in fp32,
 // l = inclusive cumsum of A_h dt within the chunk, lam[bhc] = l[kQ-1].  Every other kernel reads this table instead
-// of gathering dt (stride = nheads elements) and scanning it again per head.  The four waves of a workgroup take four
-// consecutive heads of one (batch, chunk): dt is [b][l][h], so a token's four values are 8 (fp32: 16) consecutive bytes
-// and are fetched by one thread per token and handed to the waves through LDS, instead of 128 two-byte gathers per wave.
-constexpr int kLdHeads = 4;
+// of gathering dt (stride = nheads elements) and scanning it again per head.  A workgroup takes eight consecutive heads of
+// one (batch, chunk), two per wave: dt is [b][l][h], so two threads per token fetch 8 (fp32: 16) bytes each and hand them
+// to the waves through LDS.  These workgroups are chains of latencies that hold the shared memory of a cb_body workgroup, so
+// fewer of them with interleaved scans beat more with one (alone, four / eight / sixteen heads: 14.8 / 12.4 / 12.8 us at b2
+// l4096 h128; b1 l200 h80, where a handful of workgroups take the softplus of everything: 5.7 / 6.2 / 8.9).
+constexpr int kLdHeads = 8;
 inline int64_t ld_table_blocks(int64_t batch, int64_t nheads, int64_t nchunks) { return batch * nchunks * ((nheads + kLdHeads - 1) / kLdHeads); }
 template <typename T>
 __device__ __forceinline__ void
 ld_table_body(const void* __restrict__ dt, int dt_f32, const float* __restrict__ dt_bias, const float* __restrict__ A, float* __restrict__ ldtab,
               float* __restrict__ lam, int64_t seqlen, int64_t nheads, int64_t nchunks,
               int64_t dtsb, int64_t dtsl, int hs, int64_t blk) {
-    __shared__ float sdt[kLdHeads][kQ];
+    constexpr int kPer = kLdHeads / 2, kHW = kLdHeads / 4;      // heads per loading thread, per wave
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    float (*sdt)[kQ] = reinterpret_cast<float (*)[kQ]>(smem_raw);      // [kLdHeads][kQ], in what cb_body would use
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t hgroups = (nheads + kLdHeads - 1) / kLdHeads;
     const int64_t hg = blk % hgroups, c = (blk / hgroups) % nchunks, b = blk / (hgroups * nchunks);
-    const int64_t h0 = hg * kLdHeads, h = h0 + wave;
+    const int64_t h0 = hg * kLdHeads;
     const int64_t t0 = c * kQ;
     const int valid = (int)((seqlen - t0) < kQ ? (seqlen - t0) : kQ);
-    const int hc = (int)(nheads - h0 < kLdHeads ? nheads - h0 : kLdHeads);
-    if (threadIdx.x < kQ) {
-        const int t = threadIdx.x;
-        float v[kLdHeads] = {0.f, 0.f, 0.f, 0.f};      // tokens past the end of the sequence behave as dt = 0
-        if (t < valid) {
-            const int64_t off = b * dtsb + (t0 + t) * dtsl + h0;
-            if (dt_f32) {
-                const float* p = static_cast<const float*>(dt) + off;
-                if (hc == kLdHeads && (reinterpret_cast<uintptr_t>(p) & 15) == 0) {
-                    const floatx4 q = *reinterpret_cast<const floatx4*>(p);
+    float Ah[kHW], bh[kHW];      // fetched along with dt: one latency, not one per head
 #pragma unroll
-                    for (int k = 0; k < kLdHeads; ++k) v[k] = q[k];
-                } else {
-                    for (int k = 0; k < hc; ++k) v[k] = p[k];
-                }
+    for (int k = 0; k < kHW; ++k) {
+        const int64_t h = h0 + wave * kHW + k < nheads ? h0 + wave * kHW + k : nheads - 1;
+        Ah[k] = A[h];
+        bh[k] = dt_bias ? dt_bias[h] : 0.f;
+    }
+    {
+        const int t = threadIdx.x & (kQ - 1), k0 = (threadIdx.x >> 7) * kPer;
+        const int64_t left = nheads - h0 - k0;
+        const int hc = (int)(left < kPer ? left : kPer);
+        float v[kPer];      // tokens past the end of the sequence behave as dt = 0
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) v[k] = 0.f;
+        auto fetch = [&](auto* p) {
+            using E = std::remove_const_t<std::remove_pointer_t<decltype(p)>>;
+            if (hc == kPer && (reinterpret_cast<uintptr_t>(p) & (kPer * sizeof(E) - 1)) == 0) {
+                const RawVec<E, kPer> raw = *reinterpret_cast<const RawVec<E, kPer>*>(p);
+                const E* e = reinterpret_cast<const E*>(&raw);
+#pragma unroll
+                for (int k = 0; k < kPer; ++k) v[k] = to_f32(e[k]);
             } else {
-                const T* p = static_cast<const T*>(dt) + off;
-                if (hc == kLdHeads && (reinterpret_cast<uintptr_t>(p) & (kLdHeads * sizeof(T) - 1)) == 0) {
-                    const RawVec<T, kLdHeads> q = *reinterpret_cast<const RawVec<T, kLdHeads>*>(p);
-                    const T* e = reinterpret_cast<const T*>(&q);
 #pragma unroll
-                    for (int k = 0; k < kLdHeads; ++k) v[k] = to_f32(e[k]);
-                } else {
-                    for (int k = 0; k < hc; ++k) v[k] = to_f32(p[k]);
-                }
+                for (int k = 0; k < kPer; ++k)
+                    if (k < hc) v[k] = to_f32(p[k]);
             }
+        };
+        if (t < valid) {
+            const int64_t off = b * dtsb + (t0 + t) * dtsl + h0 + k0;
+            if (dt_f32) fetch(static_cast<const float*>(dt) + off);
+            else fetch(static_cast<const T*>(dt) + off);
         }
 #pragma unroll
-        for (int k = 0; k < kLdHeads; ++k) sdt[k][t] = v[k];
+        for (int k = 0; k < kPer; ++k) sdt[k0 + k][t] = v[k];
     }
     __syncthreads();
-    if (h >= nheads) return;      // wave-uniform, behind the only barrier
-    float l0, l1, d0 = sdt[wave][lane], d1 = sdt[wave][lane + 64];
-    if (dt_bias) {
-        // dt holds the raw projection: the step size is softplus(dt + dt_bias) (0 stays 0 past the end of the sequence)
-        const float bh = dt_bias[h];
-        if (lane < valid) d0 = softplus_f(d0 + bh);
-        if (lane + 64 < valid) d1 = softplus_f(d1 + bh);
+    float l0[kHW], l1[kHW], d0[kHW], d1[kHW];
+#pragma unroll
+    for (int k = 0; k < kHW; ++k) {      // past the last head: its values once more, not stored
+        d0[k] = sdt[wave * kHW + k][lane]; d1[k] = sdt[wave * kHW + k][lane + 64];
+        if (dt_bias) {
+            // dt holds the raw projection: the step size is softplus(dt + dt_bias) (0 stays 0 past the end of the sequence)
+            d0[k] = lane < valid ? softplus_f(d0[k] + bh[k]) : 0.f;
+            d1[k] = lane + 64 < valid ? softplus_f(d1[k] + bh[k]) : 0.f;
+        }
+        wave_cumsum_from(Ah[k], d0[k], d1[k], l0[k], l1[k]);
     }
-    wave_cumsum_from(A[h], d0, d1, l0, l1);
-    for (int v = 0; v < (1 << hs); ++v) {      // one table per kernel head
-        const int64_t bhc = (((b * nheads + h) << hs) + v) * nchunks + c;
-        float* p = ldtab + bhc * (2 * kQ);
-        p[lane] = l0; p[lane + 64] = l1; p[kQ + lane] = d0; p[kQ + lane + 64] = d1;
-        if (lane == 63) lam[bhc] = l1;
+#pragma unroll
+    for (int k = 0; k < kHW; ++k) {
+        const int64_t h = h0 + wave * kHW + k;
+        if (h >= nheads) return;
+        for (int v = 0; v < (1 << hs); ++v) {      // one table per kernel head
+            const int64_t bhc = (((b * nheads + h) << hs) + v) * nchunks + c;
+            float* p = ldtab + bhc * (2 * kQ);
+            p[lane] = l0[k]; p[lane + 64] = l1[k]; p[kQ + lane] = d0[k]; p[kQ + lane + 64] = d1[k];
+            if (lane == 63) lam[bhc] = l1[k];
+        }
     }
 }
 
 // Both preparations in one launch (they are independent, and either alone leaves most of the GPU idle): the first
-// kCbParts n_cb workgroups run cb_body for (part, chunk, group, batch) = the index split in that order, the others ld_table_body.
+// cb_blocks(n_cb) workgroups run cb_body, the others ld_table_body.
 struct PrepArgs {
     const void* Bm; const void* Cm; float* Gf; void* Gm; void* Gmt; void* Bt; void* Ct;
     int64_t Bsb, Bsl, Bsg, Csb, Csl, Csg;
@@ -196,14 +239,17 @@ template <typename T, int N>
 __global__ void __launch_bounds__(256)
 prep_kernel(const PrepArgs a) {
     const int64_t blk = blockIdx.x;
-    if (blk < kCbParts * a.n_cb) {
-        const int64_t q = blk / kCbParts;
+    if (blk < cb_blocks(a.n_cb)) {
+        // The parts of one (chunk, group, batch) read the same rows.  Workgroups are dealt round-robin to the XCDs, so the
+        // parts are kXcds apart: one L2 then fetches those rows once, where seven neighbours would each fetch their own.
+        const int64_t u = blk / kXcds, q = u / kCbParts * kXcds + blk % kXcds;
+        if (q >= a.n_cb) return;
         const int64_t c = q % a.nchunks, g = (q / a.nchunks) % a.ngroups, b = q / (a.nchunks * a.ngroups);
         cb_body<T, N>(static_cast<const T*>(a.Bm), static_cast<const T*>(a.Cm), a.Gf, static_cast<T*>(a.Gm), static_cast<T*>(a.Gmt),
                       static_cast<T*>(a.Bt), static_cast<T*>(a.Ct), a.seqlen, a.ngroups, a.nchunks,
-                      a.Bsb, a.Bsl, a.Bsg, a.Csb, a.Csl, a.Csg, c, g, b, (int)(blk % kCbParts));
+                      a.Bsb, a.Bsl, a.Bsg, a.Csb, a.Csl, a.Csg, c, g, b, (int)(u % kCbParts));
     } else {
-        ld_table_body<T>(a.dt, a.dt_f32, a.dt_bias, a.A, a.ldtab, a.lam, a.seqlen, a.nheads, a.nchunks, a.dtsb, a.dtsl, a.hs, blk - kCbParts * a.n_cb);
+        ld_table_body<T>(a.dt, a.dt_f32, a.dt_bias, a.A, a.ldtab, a.lam, a.seqlen, a.nheads, a.nchunks, a.dtsb, a.dtsl, a.hs, blk - cb_blocks(a.n_cb));
     }
 }
 
