@@ -272,6 +272,22 @@ int m2_decode_rows(float* residual, const void* delta, int32_t delta_dtype, int3
                    int64_t channels, void* stream);
 int m2_decode_layer(const m2_linear_params* in, const m2_decode_params* dec, const float* norm_weight, const m2_linear_params* out, void* stream);
 
+/* A linear layer's products on few tokens, bf16 operands and result, fp32 accumulation:
+ *   out[m][n] = bias[n] + sum_k A(m, k) B(n, k),   A = a[m * lda + k] (a_k != 0) or a[k * lda + m], B = b[n * ldb + k] (b_k != 0) or
+ *   b[k * ldb + n];  bias (N) bf16 or NULL.
+ * N, the contiguous extent of each operand, lda, ldb and ldo multiples of 8, pointers 16-byte aligned (m2_product_fits: the
+ * shape is taken; m2_product_pays: it is also the faster choice over a general library's product); workspace as m2_product_workspace_bytes says (0: none). */
+typedef struct m2_product_params {
+    const void* a; const void* b; const void* bias; void* out; void* workspace; size_t workspace_bytes;
+    int64_t M, N, K, lda, ldb, ldo;
+    int32_t a_k, b_k;
+} m2_product_params;
+
+int m2_product_fits(int64_t M, int64_t N, int64_t K, int32_t a_k, int32_t b_k);
+int m2_product_pays(int64_t M, int64_t N, int64_t K, int32_t a_k, int32_t b_k);
+size_t m2_product_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int m2_product(const m2_product_params* p, void* stream);
+
 /* The small parameters of a mixer layer as the kernels take them, and their gradients back, in one launch each
  * (mamba2/mamba2_mixer.py:225-236: A = -exp(A_log.float()) and the casts around it).
  * m2_mixer_params:       out (3 * nheads + channels) fp32 = [ -exp(A_log) | D | dt_bias | norm_weight ].

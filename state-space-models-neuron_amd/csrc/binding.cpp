@@ -30,7 +30,8 @@ using torch::autograd::variable_list;
     F(m2_last_error) F(m2_conv1d_fwd) F(m2_conv1d_prefill) F(m2_conv1d_bwd_workspace_bytes) F(m2_conv1d_bwd) F(m2_ssd_chunk_states_bytes) \
     F(m2_ssd_fwd_workspace_bytes) F(m2_ssd_fwd) F(m2_ssd_bwd_workspace_bytes) F(m2_ssd_bwd) F(m2_decode_workspace_bytes) \
     F(m2_decode_step) F(m2_decode_step_static) F(m2_rmsnorm_gated_fwd) F(m2_rmsnorm_gated_bwd_workspace_bytes) \
-    F(m2_rmsnorm_gated_bwd) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_rows) F(m2_decode_layer) F(m2_mixer_params) F(m2_mixer_params_grads)
+    F(m2_rmsnorm_gated_bwd) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_rows) F(m2_decode_layer) F(m2_mixer_params) F(m2_mixer_params_grads) \
+    F(m2_product_pays) F(m2_product_workspace_bytes) F(m2_product)
 struct Lib {
 #define M2_FIELD(name) decltype(&::name) name = nullptr;
     M2_BOUND(M2_FIELD)
@@ -625,10 +626,41 @@ Tensor fused_core(const Tensor& zx, const Tensor& A, const OptTensor& D, const T
 }
 
 // ----------------------------------------------------------------------------------------------- whole mixer layer
-// mamba2_mixer.py:213-240: in_proj -> core -> out_proj as one node, the plain products by the library that torch uses, the
-// small parameters cast (and A = -exp(A_log) formed) by one kernel and their gradients cast back by one.
-Tensor project(const Tensor& x, const Tensor& w, const Tensor& bias) {
-    return bias.defined() ? at::addmm(bias, x, w.t()) : at::mm(x, w.t());
+// mamba2_mixer.py:213-240: in_proj -> core -> out_proj as one node, the products on few tokens by the kernel for them and the
+// large ones by the library that torch uses, the small parameters cast (and A = -exp(A_log) formed) by one kernel and their
+// gradients cast back by one.
+
+// out (M, N) = A B (+ bias): `a` is A or, if !a_k, A^T (K, M); `b` is B^T (N, K) or, if !b_k, B
+Tensor product(const Tensor& a, bool a_k, const Tensor& b, bool b_k, const Tensor& bias, void* stream) {
+    m2_product_params p{};
+    p.M = a.size(a_k ? 0 : 1); p.K = a.size(a_k ? 1 : 0); p.N = b.size(b_k ? 0 : 1);
+    p.lda = a.stride(0); p.ldb = b.stride(0); p.ldo = p.N; p.a_k = a_k; p.b_k = b_k;
+    auto rows = [](const Tensor& t) {
+        return t.scalar_type() == at::kBFloat16 && t.stride(1) == 1 && t.stride(0) % 8 == 0 && t.stride(0) >= t.size(1) &&
+               t.size(0) * t.stride(0) < (int64_t{1} << 31) && reinterpret_cast<uintptr_t>(ptr(t)) % 16 == 0;
+    };
+    const bool plain_bias = !bias.defined() || (bias.scalar_type() == at::kBFloat16 && bias.is_contiguous());
+    if (!plain_bias || !rows(a) || !rows(b) || b.size(b_k ? 1 : 0) != p.K || !lib.m2_product_pays(p.M, p.N, p.K, a_k, b_k)) {
+        const Tensor at_ = a_k ? a : a.t(), bt = b_k ? b.t() : b;
+        return bias.defined() ? at::addmm(bias, at_, bt) : at::mm(at_, bt);
+    }
+    const Tensor out = at::empty({p.M, p.N}, a.options());
+    p.workspace_bytes = lib.m2_product_workspace_bytes(p.M, p.N, p.K);
+    const Tensor ws = p.workspace_bytes ? at::empty({static_cast<int64_t>(p.workspace_bytes)}, a.options().dtype(at::kByte)) : Tensor();
+    p.a = ptr(a); p.b = ptr(b); p.bias = ptr(bias); p.out = ptr(out); p.workspace = ptr(ws);
+    check(lib.m2_product(&p, stream), "m2_product");
+    return out;
+}
+Tensor project(const Tensor& x, const Tensor& w, const Tensor& bias, void* stream) { return product(x, true, w, true, bias, stream); }
+
+// a linear layer outside autograd
+Tensor linear(const Tensor& x, const Tensor& w, const OptTensor& bias) {
+    require_gpu({&x, &w});
+    TORCH_CHECK_VALUE(x.dim() >= 1 && w.dim() == 2 && x.size(-1) == w.size(1), "linear: x (..., in) and weight (out, in) are required");
+    Scope scope(x);
+    std::vector<int64_t> shape = x.sizes().vec();
+    shape.back() = w.size(0);
+    return project(x.reshape({-1, w.size(1)}), w, or_none(bias), scope.stream).view(shape);
 }
 
 struct MixerFn : torch::autograd::Function<MixerFn> {
@@ -639,7 +671,7 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
         Scope scope(hidden);
         const int64_t b = hidden.size(0), l = hidden.size(1), h = d / hd;
         const Tensor x = hidden.reshape({b * l, hidden.size(2)});
-        const Tensor zx = project(x, in_w, or_none(in_b)).view({b, l, in_w.size(0)});
+        const Tensor zx = project(x, in_w, or_none(in_b), scope.stream).view({b, l, in_w.size(0)});
         const Packed k(zx, g, n, d, hd);
         check_core(k, A_log, D, conv_w, or_none(conv_b), dt_bias, norm_w);
         const Tensor small = empty_f32({3 * h + d}, zx);
@@ -655,7 +687,7 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
             ctx->save_for_backward(std::move(saved));
             ctx->saved_data["dims"] = std::vector<int64_t>{g, n, d, hd};
         }
-        return project(y, out_w, or_none(out_b)).view({b, l, out_w.size(0)});
+        return project(y, out_w, or_none(out_b), scope.stream).view({b, l, out_w.size(0)});
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const variable_list s = ctx->get_saved_variables();
@@ -668,9 +700,9 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
         const Tensor A = small.narrow(0, 0, k.h), D = small.narrow(0, k.h, k.h), dt_bias = small.narrow(0, 2 * k.h, k.h), norm_w = small.narrow(0, 3 * k.h, k.d);
         variable_list out(17);
         const Tensor dy = grads[0].reshape({rows, s[kOutW].size(0)});
-        if (ctx->needs_input_grad(kOutW)) out[kOutW] = at::mm(dy.t(), s[kNormOut]);
+        if (ctx->needs_input_grad(kOutW)) out[kOutW] = product(dy, false, s[kNormOut], false, Tensor(), scope.stream);
         if (s[kOutB].defined()) out[kOutB] = dy.sum(0);
-        const Tensor d_core = at::mm(dy, s[kOutW]).view({k.b, k.l, k.d});
+        const Tensor d_core = product(dy, true, s[kOutW], false, Tensor(), scope.stream).view({k.b, k.l, k.d});
         CoreOut f;
         if (s.size() > kConvOut) { f.conv_out = s[kConvOut]; f.scan_out = s[kScanOut]; f.states = s[kStates]; }
         else f = core_forward(k, A, D, s[kConvW], s[kConvB], dt_bias, norm_w, true, false, scope.stream);
@@ -681,8 +713,8 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
                                         dtype_code(s[kNormW]), k.h, k.d, scope.stream), "m2_mixer_params_grads");
         out[kConvW] = r.conv_w; out[kConvB] = r.conv_b;
         const Tensor d_zx = r.zx.view({rows, zx.size(2)});
-        if (ctx->needs_input_grad(kHidden)) out[kHidden] = at::mm(d_zx, s[kInW]).view(s[kHidden].sizes());
-        if (ctx->needs_input_grad(kInW)) out[kInW] = at::mm(d_zx.t(), s[kHidden].reshape({rows, s[kHidden].size(2)}));
+        if (ctx->needs_input_grad(kHidden)) out[kHidden] = product(d_zx, true, s[kInW], false, Tensor(), scope.stream).view(s[kHidden].sizes());
+        if (ctx->needs_input_grad(kInW)) out[kInW] = product(d_zx, false, s[kHidden].reshape({rows, s[kHidden].size(2)}), false, Tensor(), scope.stream);
         if (s[kInB].defined()) out[kInB] = d_zx.sum(0);
         return out;
     }
@@ -800,7 +832,7 @@ m2_linear_params linear_params(const Tensor& w, const Tensor& bias, int64_t rows
 // out = x w^T + bias for a few bf16 rows; the library's product where the kernel does not take the shape
 Tensor linear_rows(const Tensor& x, const Tensor& w, const Tensor& bias, void* stream) {
     m2_linear_params p = linear_params(w, bias, x.size(0));
-    if (x.scalar_type() != at::kBFloat16 || !linear_takes(w, bias) || !lib.m2_linear_small_fits(p.M, p.N, p.K, 1)) return project(x, w, bias);
+    if (x.scalar_type() != at::kBFloat16 || !linear_takes(w, bias) || !lib.m2_linear_small_fits(p.M, p.N, p.K, 1)) return project(x, w, bias, stream);
     const Tensor xr = aligned(x);
     Tensor out = at::empty({p.M, p.N}, x.options());
     p.x = ptr(xr); p.x_stride_row = xr.stride(0); p.out = ptr(out); p.out_stride_row = p.N;
@@ -999,6 +1031,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("residual_stream", &residual_stream);
     m.def("stream_sum", &stream_sum);
     m.def("stream_norm", &stream_norm);
+    m.def("linear", &linear);
     m.def("stream_norm_linear", &stream_norm_linear);
     m.def("decode_step", &decode_step);
 }

@@ -189,6 +189,16 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
+template <typename K>
+inline int allow_smem(K kernel, size_t bytes) {
+    if (bytes > 160 * 1024) return fail(M2_ERR_SHAPE, "kernel needs %zu bytes of LDS (> 160 KiB)", bytes);
+    if (bytes > 48 * 1024) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
+            return fail(M2_ERR_LAUNCH, "hipFuncSetAttribute(%zu bytes of LDS) failed: %s", bytes, hipGetErrorString(hipGetLastError()));
+    }
+    return M2_OK;
+}
+
 // Dispatch a runtime dtype to a template type.
 #define M2_DISPATCH_DTYPE(dtype, T, ...)                                  \
     do {                                                                  \

@@ -150,16 +150,6 @@ inline int ssd_check(const m2_ssd_params* p, const char* who) {
     return M2_OK;
 }
 
-template <typename K>
-inline int allow_smem(K kernel, size_t bytes) {
-    if (bytes > 160 * 1024) return fail(M2_ERR_SHAPE, "kernel needs %zu bytes of LDS (> 160 KiB)", bytes);
-    if (bytes > 48 * 1024) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
-            return fail(M2_ERR_LAUNCH, "hipFuncSetAttribute(%zu bytes of LDS) failed: %s", bytes, hipGetErrorString(hipGetLastError()));
-    }
-    return M2_OK;
-}
-
 template <typename T, int P, int N>
 inline size_t state_smem() { return (size_t)(P + N) * lds_ld<T>(kQ) * sizeof(T); }
 template <typename T>

@@ -76,6 +76,11 @@ class LinearParams(C.Structure):
                 ("out_kind", _i32), ("groups", _i32), ("eps", C.c_float)]
 
 
+class ProductParams(C.Structure):
+    _fields_ = [("a", _vp), ("b", _vp), ("bias", _vp), ("out", _vp), ("workspace", _vp), ("workspace_bytes", _sz),
+                ("M", _i64), ("N", _i64), ("K", _i64), ("lda", _i64), ("ldb", _i64), ("ldo", _i64), ("a_k", _i32), ("b_k", _i32)]
+
+
 # name -> (restype, argtypes); every symbol the header declares
 SYMBOLS = {
     "m2_abi_version": (C.c_int, []),
@@ -104,6 +109,10 @@ SYMBOLS = {
     "m2_linear_small": (C.c_int, [C.POINTER(LinearParams), _vp]),
     "m2_decode_rows": (C.c_int, [_vp, _vp, _i32, _i32, _vp, _vp, _vp, _i64, _i64, _vp]),
     "m2_decode_layer": (C.c_int, [C.POINTER(LinearParams), C.POINTER(DecodeParams), _vp, C.POINTER(LinearParams), _vp]),
+    "m2_product_fits": (C.c_int, [_i64, _i64, _i64, _i32, _i32]),
+    "m2_product_pays": (C.c_int, [_i64, _i64, _i64, _i32, _i32]),
+    "m2_product_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "m2_product": (C.c_int, [C.POINTER(ProductParams), _vp]),
     "m2_mixer_params": (C.c_int, [_vp, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _vp, _i64, _i64, _vp]),
     "m2_mixer_params_grads": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _i64, _i64, _vp]),
     "m2_mfma_selftest": (C.c_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp]),

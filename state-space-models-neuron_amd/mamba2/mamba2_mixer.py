@@ -33,6 +33,13 @@ def _plain_linear(m):
                                          or nn.modules.module._has_any_global_hook())
 
 
+def _inference_linear(m, x):
+    """``m(x)`` outside autograd; a plain product on few rows by this library's kernel."""
+    if _plain_linear(m) and not torch.is_autocast_enabled():
+        return _lib.native().linear(x, m.weight, m.bias)
+    return m(x)
+
+
 class Mamba2Cache:
     """Minimal decode cache: per-layer ``conv_states[i]`` (b, conv_dim, W) and ``ssm_states[i]`` (b, h, p, n) fp32,
     plus ``seqlen_offset`` (the fields the reference touches, ``mamba2_mixer.py:270-276``, ``modeling_mamba2.py:321``)."""
@@ -154,12 +161,12 @@ class Mamba2Mixer(nn.Module):
         if cache_params is not None:
             assert not torch.is_grad_enabled(), "forward with a cache is the inference prefill: call it under torch.no_grad()"
             A, D, dt_bias = self._inference_params()
-            zxBCdt = self.in_proj(hidden_states)
+            zxBCdt = _inference_linear(self.in_proj, hidden_states)
             scan_output = mamba2_fused_prefill(zxBCdt, A, D, self.conv1d.weight, self.conv1d.bias, dt_bias, self.norm.weight,
                                                self.n_groups_tp, self.ssm_state_size, self.intermediate_size_tp, self.head_dim,
                                                cache_params.conv_states[self.layer_idx], cache_params.ssm_states[self.layer_idx],
                                                continuing=cache_params.seqlen_offset > 0)
-            return self.out_proj(scan_output)
+            return _inference_linear(self.out_proj, scan_output)
         if _plain_linear(self.in_proj) and _plain_linear(self.out_proj) and not torch.is_autocast_enabled():
             # one native node for the layer: the projections' products, the core, and the small parameters' casts
             return _lib.native().mixer(hidden_states, self.in_proj.weight, self.A_log, self.D, self.dt_bias, self.conv1d.weight, self.norm.weight,

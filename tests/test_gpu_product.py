@@ -1,0 +1,39 @@
+"""GPU: the products of a layer's projections on few tokens, in the storage forms of a linear layer's forward and backward, at the
+edges of their tiles and k splits, against fp64 on the CPU."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (8, 8, 1), (64, 64, 64), (65, 72, 72), (72, 200, 1000), (40, 64, 5), (200, 2560, 520), (136, 264, 2056), (1000, 1544, 136)])
+@pytest.mark.parametrize("a_k,b_k", [(1, 1), (1, 0), (0, 0), (0, 1)])
+@pytest.mark.parametrize("pad", [0, 8])
+def test_product(M, N, K, a_k, b_k, pad):
+    from mamba2 import _lib
+    lib = _lib.load()
+    if not lib.m2_product_fits(M, N, K, a_k, b_k):
+        assert (a_k or b_k) and K % 8 or not a_k and M % 8
+        return
+    gen = torch.Generator().manual_seed(M + N + K)
+    a, b = (torch.randn(r, K, generator=gen).bfloat16() for r in (M, N))
+    bias = torch.randn(N, generator=gen).bfloat16()
+    ref = a.double() @ b.double().T + bias.double()
+
+    def stored(t, k):      # rows of the operand as it lies in memory, NaN behind their ends
+        t = t if k else t.T
+        buf = torch.full((t.shape[0], -(-t.shape[1] // 8) * 8 + pad), float("nan"), dtype=t.dtype)
+        buf[:, :t.shape[1]] = t
+        return buf.to(DEV)
+
+    ad, bd, biasd = stored(a, a_k), stored(b, b_k), bias.to(DEV)
+    out = torch.full((M, N + pad), 7.0, dtype=torch.bfloat16, device=DEV)
+    n = lib.m2_product_workspace_bytes(M, N, K)
+    ws = torch.empty(max(n, 1), dtype=torch.uint8, device=DEV)
+    p = _lib.ProductParams(a=_lib.ptr(ad), b=_lib.ptr(bd), bias=_lib.ptr(biasd), out=_lib.ptr(out), workspace=_lib.ptr(ws), workspace_bytes=n, M=M, N=N, K=K,
+                           lda=ad.stride(0), ldb=bd.stride(0), ldo=N + pad, a_k=a_k, b_k=b_k)
+    _lib.check(lib.m2_product(p, _lib.stream_ptr()), "m2_product")
+    got = out.double().cpu()
+    assert ((got[:, :N] - ref).norm() / ref.norm()).item() < 4e-3
+    assert (got[:, N:] == 7.0).all()
