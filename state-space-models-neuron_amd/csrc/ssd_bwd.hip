@@ -314,7 +314,7 @@ off_kernel(const T* __restrict__ Arow, int64_t Asb, int64_t Asl, int64_t Ash,   
 
 // Sum of the per-slice partials (fixed order) of up to three arrays in one launch.  One thread per float4;
 // `tile` floats per (group, slice) tile; segment k covers threads [first_k, first_{k+1}).
-struct SliceSumSeg { const float* part; float* out; int64_t nslices, tile, first; };
+struct SliceSumSeg { const float* part; float* out; int64_t nslices, tile, first; int lower; };      // lower: kQ x kQ, blocks above the diagonal unused
 struct SliceSumArgs { SliceSumSeg seg[3]; int nseg; int64_t total; };
 template <int THREADS>
 __device__ __forceinline__ void slice_sum_body(const SliceSumArgs& a, int64_t blk) {
@@ -326,7 +326,9 @@ __device__ __forceinline__ void slice_sum_body(const SliceSumArgs& a, int64_t bl
     const SliceSumSeg sg = a.seg[k];
     const int64_t per = sg.tile / 4, loc = idx - sg.first;
     const int64_t grp = loc / per, e = (loc % per) * 4;
+    if (sg.lower && ((e % kQ) >> 5) > e / (32 * kQ)) return;
     floatx4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
     for (int64_t sl = 0; sl < sg.nslices; ++sl) s += *reinterpret_cast<const floatx4*>(sg.part + (grp * sg.nslices + sl) * sg.tile + e);
     *reinterpret_cast<floatx4*>(sg.out + grp * sg.tile + e) = s;
 }
@@ -622,7 +624,7 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
         const size_t sm = state_smem<T, P, N>();
         if ((rc = allow_smem(k, sm))) return rc;
         int64_t ns, hps;
-        ssd_slicing(p, kWgsChunkState, &ns, &hps);
+        ssd_slicing(p, kWgsChunkState, false, &ns, &hps);
         k<<<dim3((unsigned)nc, (unsigned)(p->ngroups * ns), (unsigned)p->batch), 256, sm, st>>>(
             dy, w.ldtab, static_cast<const T*>(w.Ct), w.local, p->seqlen, p->nheads, p->ngroups, nc, ns, hps,
             p->dy_stride_b, p->dy_stride_l, p->dy_stride_h);
@@ -689,7 +691,7 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
         a.Gd = w.Gmt; a.S = w.dprev;
         a.Z = p->dy; a.Z_sb = p->dy_stride_b; a.Z_sl = p->dy_stride_l; a.Z_sh = p->dy_stride_h;
         a.seqlen = p->seqlen; a.nheads = p->nheads; a.ngroups = p->ngroups; a.nchunks = nc;
-        ssd_slicing(p, 2, &a.nslices, &a.hps);
+        ssd_slicing(p, 2, false, &a.nslices, &a.hps);
         a.X = p->x; a.X_sb = p->x_stride_b; a.X_sl = p->x_stride_l; a.X_sh = p->x_stride_h;
         a.dX = p->dx; a.dX_sb = p->dx_stride_b; a.dX_sl = p->dx_stride_l; a.dX_sh = p->dx_stride_h;
         a.ldtab = w.ldtab;
@@ -713,15 +715,15 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
         {
             SliceSumArgs sa{};
             int64_t first = 0;
-            auto add = [&](const float* part, float* out, int64_t ns, int64_t tile, const float** use) {
+            auto add = [&](const float* part, float* out, int64_t ns, int64_t tile, int lower, const float** use) {
                 if (ns <= 1) return;
-                sa.seg[sa.nseg++] = SliceSumSeg{part, out, ns, tile, first};
+                sa.seg[sa.nseg++] = SliceSumSeg{part, out, ns, tile, first, lower};
                 first += ngrp * tile / 4;
                 *use = out;
             };
-            add(w.dGp, w.dGs, w.ns_g, (int64_t)kQ * kQ, &gs);
-            add(w.dCp, w.dCs, w.ns_c, (int64_t)kQ * N, &cs);
-            add(w.dBp, w.dBs, w.ns_b, (int64_t)kQ * N, &bs);
+            add(w.dGp, w.dGs, w.ns_g, (int64_t)kQ * kQ, 1, &gs);
+            add(w.dCp, w.dCs, w.ns_c, (int64_t)kQ * N, 0, &cs);
+            add(w.dBp, w.dBs, w.ns_b, (int64_t)kQ * N, 0, &bs);
             sa.total = first;
             const int64_t n_da = da_blocks(da), n_ss = ceil_div(first, (int64_t)(kDaHeads * 64));
             tail1_kernel<T><<<(unsigned)(n_da + n_ss), kDaHeads * 64, 0, st>>>(da, n_da, sa);

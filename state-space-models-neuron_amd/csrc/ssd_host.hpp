@@ -37,19 +37,24 @@ struct SsdWorkspace {
 };
 
 // A workgroup owns one chunk of one group and loops over a slice of that group's heads (operands shared by the
-// group stay on chip, group-level reductions happen in registers).  The slice count is the smallest divisor of
-// heads-per-group that gives at least `wgs_per_cu` workgroups per compute unit: the grid then fills the GPU in one
-// round of long-running workgroups (measured: fewer, longer workgroups beat more, shorter ones for every kernel).
-inline void ssd_slicing(const SsdCall* p, int wgs_per_cu, int64_t* nslices, int64_t* hps) {
+// group stay on chip, group-level reductions happen in registers).  The slice count is the divisor of heads-per-group with the
+// least of: workgroups on the busiest CU times heads per slice -- a CU that could hold two (`wgs_per_cu`) and has one takes three
+// quarters of two's time --, 1.5 heads' worth for filling and draining each of them, and, `partials`, what the slices' partial
+// sums cost on their way out and back (128 KiB each: a head's worth per 110 workgroups).  Taking whatever first filled the chip
+// instead left a nearly empty last round and twice the partials at b3 l1111 h32: main backward kernel 41 -> 31 us, dG 17.7 ->
+// 14.2, slice sums 17.9 -> 10.1, y 17.4 -> 15.4; y at b8 l333 h80 25.9 -> 22.1.
+inline void ssd_slicing(const SsdCall* p, int wgs_per_cu, bool partials, int64_t* nslices, int64_t* hps) {
     const int64_t nc = ceil_div(p->seqlen, (int64_t)kQ);
     const int64_t hpg = p->nheads / p->ngroups;
     const int64_t base = p->batch * nc * p->ngroups;
-    const int64_t target = device_cus() * wgs_per_cu;
+    const int64_t cus = device_cus();
     int64_t best = 1;
+    float least = 1e30f;
     for (int64_t s = 1; s <= hpg; ++s) {
         if (hpg % s) continue;
-        best = s;
-        if (base * s >= target) break;
+        const float n = (float)ceil_div(base * s, cus), busy = n < (float)wgs_per_cu ? 0.75f * (float)wgs_per_cu : n;
+        const float cost = busy * (float)(hpg / s) + 1.5f * n + (partials ? 0.009f * (float)(base * s) : 0.f);
+        if (cost < least) { least = cost; best = s; }
     }
     *nslices = best;
     *hps = hpg / best;
@@ -91,11 +96,11 @@ inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_
         w.kept_bytes = koff;
     }
     if (bwd) {
-        ssd_slicing(p, kWgsDg, &w.ns_g, &w.hps_g);
-        ssd_slicing(p, kWgsOffC, &w.ns_c, &w.hps_c);
-        ssd_slicing(p, kWgsOffB, &w.ns_b, &w.hps_b);
+        ssd_slicing(p, kWgsDg, true, &w.ns_g, &w.hps_g);
+        ssd_slicing(p, kWgsOffC, true, &w.ns_c, &w.hps_c);
+        ssd_slicing(p, kWgsOffB, true, &w.ns_b, &w.hps_b);
         if (p->dtype != M2_F32) {       // the main backward kernel produces both state parts there
-            ssd_slicing(p, kWgsDx, &w.ns_b, &w.hps_b);
+            ssd_slicing(p, kWgsDx, true, &w.ns_b, &w.hps_b);
             w.ns_c = w.ns_b; w.hps_c = w.hps_b;
         }
         w.dprev = take(tiles * esz);
@@ -221,7 +226,7 @@ inline int ssd_launch_states(const SsdCall* p, const SsdWorkspace& w, float* fin
         const size_t sm = state_smem<T, P, N>();
         if ((rc = allow_smem(k, sm))) return rc;
         int64_t ns, hps;
-        ssd_slicing(p, kWgsChunkState, &ns, &hps);
+        ssd_slicing(p, kWgsChunkState, false, &ns, &hps);
         M2_REQUIRE(p->ngroups * ns <= 65535, M2_ERR_SHAPE, "ssd: too many group slices");
         k<<<dim3((unsigned)nc, (unsigned)(p->ngroups * ns), (unsigned)p->batch), 256, sm, st>>>(
             x, w.ldtab, static_cast<const T*>(w.Bt), w.local, p->seqlen, p->nheads, p->ngroups, nc, ns, hps,
