@@ -561,9 +561,13 @@ extern "C" int m2_rmsnorm_gated_fwd(const m2_rmsnorm_params* p, void* stream) {
 
 extern "C" size_t m2_rmsnorm_gated_bwd_workspace_bytes(int64_t rows, int64_t channels, int32_t n_groups, int32_t dtype) {
     if (rows <= 0 || channels <= 0 || n_groups <= 0) return 256;
+    // A partial row per workgroup.  Where one workgroup per compute unit runs, room for the general rule's count (about 512) is
+    // asked for all the same: a size that followed the units would depend on the device that is current when it is asked for, and
+    // a caller may size its scratch without one.
     const int64_t nvec = channels / n_groups / (dtype == M2_F32 ? 4 : 8);
-    const int64_t nrb = m2::ceil_div(rows, m2::norm_rows_per_block_bwd(rows, n_groups, nvec));
-    return m2::align_up((size_t)nrb * (size_t)channels * sizeof(float), 256);      // a partial row per workgroup
+    const int64_t used = m2::ceil_div(rows, m2::norm_rows_per_block_bwd(rows, n_groups, nvec));
+    const int64_t most = m2::ceil_div(rows, m2::norm_rows_per_block(rows, n_groups, true));
+    return m2::align_up((size_t)(used > most ? used : most) * (size_t)channels * sizeof(float), 256);
 }
 
 extern "C" int m2_rmsnorm_gated_bwd(const m2_rmsnorm_params* p, void* stream) {
