@@ -198,7 +198,7 @@ void check_ssd(const Tensor& dt, const Tensor& A, const Tensor& X, const Tensor&
     const int64_t b = X.size(0), l = X.size(1), h = X.size(2);
     TORCH_CHECK_VALUE(dt.size(0) == b && dt.size(1) == l && dt.size(2) == h, "dt shape ", dt.sizes(), " != (", b, ", ", l, ", ", h, ")");
     TORCH_CHECK_VALUE(B.sizes() == C.sizes() && B.size(0) == b && B.size(1) == l, "B ", B.sizes(), " / C ", C.sizes(), " do not match X ", X.sizes());
-    TORCH_CHECK_VALUE(h % B.size(2) == 0, "n_heads ", h, " not divisible by n_groups ", B.size(2));
+    TORCH_CHECK_VALUE(B.size(2) > 0 && h % B.size(2) == 0, "n_heads ", h, " not divisible by n_groups ", B.size(2));
     TORCH_CHECK_VALUE(A.dim() == 1 && A.size(0) == h && (!D.defined() || (D.dim() == 1 && D.size(0) == h)), "A and D must have shape (n_heads,)");
     TORCH_CHECK_VALUE(B.scalar_type() == X.scalar_type() && C.scalar_type() == X.scalar_type(), "X, B and C must share one dtype");
     TORCH_CHECK_VALUE(dt.scalar_type() == X.scalar_type() || dt.scalar_type() == at::kFloat, "dt must be float32 or have the dtype of X");
@@ -469,13 +469,22 @@ Tensor add_rmsnorm(const Tensor& residual, const OptTensor& delta_, const Tensor
 // ----------------------------------------------------------------------------------------------- fused mixer core
 constexpr double kNormEps = 1e-5;      // fixed in the reference's fused kernel (fused_kernel.py:254)
 
+// Heads of a core of d channels.  The scan writes whole heads only: channels past the last one would stay as they were allocated.
+int64_t core_heads(int64_t g, int64_t n, int64_t d, int64_t p) {
+    TORCH_CHECK_VALUE(p > 0 && d >= 0 && d % p == 0, "intermediate_size ", d, " is not a multiple of head_dim ", p);
+    const int64_t h = d / p;
+    TORCH_CHECK_VALUE(g > 0 && h % g == 0, "n_heads ", h, " not divisible by n_groups ", g);
+    TORCH_CHECK_VALUE(n > 0, "ssm_state_size ", n, " must be positive");
+    return h;
+}
+
 // [z | xBC | dt] columns of the packed projection output; the kernels read them where they lie
 struct Packed {
     Tensor zx;
     int64_t b, l, h, g, n, d, p, conv, sb, sl;
     Packed(const Tensor& t, int64_t g_, int64_t n_, int64_t d_, int64_t p_) : g(g_), n(n_), d(d_), p(p_) {
         TORCH_CHECK_VALUE(t.dim() == 3, "zxBCdt must be (b, l, width)");
-        h = d / p; conv = d + 2 * g * n;
+        h = core_heads(g, n, d, p); conv = d + 2 * g * n;
         TORCH_CHECK_VALUE(t.size(2) == d + conv + h, "zxBCdt width ", t.size(2), " != 2*d_inner + 2*g*n + h = ", d + conv + h);
         const bool even = t.stride(2) == 1 && (t.size(0) <= 1 || t.stride(0) == t.size(1) * t.stride(1));
         zx = even ? t : t.contiguous();
@@ -503,7 +512,6 @@ m2_ssd_params core_ssd_params(const Packed& k, const Tensor& conv_out, const Ten
 
 void check_core(const Packed& k, const Tensor& A, const Tensor& D, const Tensor& conv_w, const Tensor& conv_b, const Tensor& dt_bias, const Tensor& norm_w) {
     require_gpu({&k.zx, &A, &D, &conv_w, &conv_b, &dt_bias, &norm_w});
-    TORCH_CHECK_VALUE(k.g > 0 && k.h % k.g == 0, "n_heads ", k.h, " not divisible by n_groups ", k.g);
     TORCH_CHECK_VALUE(A.dim() == 1 && A.size(0) == k.h && (!D.defined() || (D.dim() == 1 && D.size(0) == k.h)), "A and D must have shape (n_heads,)");
     TORCH_CHECK_VALUE(dt_bias.dim() == 1 && dt_bias.size(0) == k.h, "dt_bias must have shape (n_heads,)");
     TORCH_CHECK_VALUE(norm_w.dim() == 1 && norm_w.size(0) == k.d, "norm_weight must have shape (d_inner,)");
@@ -620,6 +628,7 @@ struct CoreFn : torch::autograd::Function<CoreFn> {
 };
 Tensor fused_core(const Tensor& zx, const Tensor& A, const OptTensor& D, const Tensor& conv_w, const OptTensor& conv_b, const Tensor& dt_bias,
                   const Tensor& norm_w, int64_t g, int64_t n, int64_t d, int64_t hd, bool caching) {
+    core_heads(g, n, d, hd);
     require_gpu({&zx});
     bool keep = caching && at::GradMode::is_enabled();
     return CoreFn::apply(zx, A, D, conv_w, conv_b, dt_bias, norm_w, g, n, d, hd, keep);
@@ -669,7 +678,7 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
                           const Tensor& conv_w, const Tensor& norm_w, const Tensor& out_w, const OptTensor& conv_b, const OptTensor& in_b,
                           const OptTensor& out_b, int64_t g, int64_t n, int64_t d, int64_t hd, bool differentiable, bool recompute) {
         Scope scope(hidden);
-        const int64_t b = hidden.size(0), l = hidden.size(1), h = d / hd;
+        const int64_t b = hidden.size(0), l = hidden.size(1), h = core_heads(g, n, d, hd);
         const Tensor x = hidden.reshape({b * l, hidden.size(2)});
         const Tensor zx = project(x, in_w, or_none(in_b), scope.stream).view({b, l, in_w.size(0)});
         const Packed k(zx, g, n, d, hd);
@@ -722,6 +731,7 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
 Tensor mixer(const Tensor& hidden, const Tensor& in_w, const Tensor& A_log, const Tensor& D, const Tensor& dt_bias, const Tensor& conv_w, const Tensor& norm_w,
              const Tensor& out_w, const OptTensor& conv_b, const OptTensor& in_b, const OptTensor& out_b, int64_t g, int64_t n, int64_t d, int64_t hd,
              bool recompute) {
+    core_heads(g, n, d, hd);
     require_gpu({&hidden, &in_w, &out_w});
     TORCH_CHECK_VALUE(hidden.dim() == 3, "hidden_states must be (batch, seqlen, hidden_size)");
     bool differentiable = false;
@@ -734,6 +744,7 @@ Tensor mixer(const Tensor& hidden, const Tensor& in_w, const Tensor& A_log, cons
 // Inference forward that hands the sequence over to the decode step: final SSM state and last W conv inputs into the cache.
 Tensor fused_prefill(const Tensor& zx, const Tensor& A, const OptTensor& D, const Tensor& conv_w, const OptTensor& conv_b_, const Tensor& dt_bias,
                      const Tensor& norm_w, int64_t g, int64_t n, int64_t d, int64_t hd, const Tensor& conv_state, const Tensor& ssm_state, bool continuing) {
+    core_heads(g, n, d, hd);
     require_gpu({&zx, &conv_state, &ssm_state});
     Scope scope(zx);
     const Packed k(zx, g, n, d, hd);

@@ -752,7 +752,7 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
 }  // namespace m2
 
 extern "C" size_t m2_ssd_bwd_workspace_bytes(const m2_ssd_params* p) {
-    if (!p || p->batch <= 0 || p->seqlen <= 0 || p->nheads <= 0) return 256;
+    if (!p || p->batch <= 0 || p->seqlen <= 0 || p->nheads <= 0 || p->ngroups <= 0) return 256;
     const m2::SsdCall q(p);
     return m2::ssd_carve(&q, nullptr, true).bytes;
 }

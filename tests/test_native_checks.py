@@ -1,0 +1,41 @@
+"""CPU: what the operators' host code refuses before it looks at a device: sizes that do not fit together are a ValueError, whatever
+the tensors' device, and never an end of the process."""
+import ctypes
+
+import pytest
+import torch
+
+
+def _core_args(h, d, g, n, l=8):
+    conv = d + 2 * g * n
+    return (torch.zeros(1, l, d + conv + h), -torch.ones(h), torch.ones(h), torch.zeros(conv, 1, 4), torch.zeros(conv), torch.zeros(h), torch.ones(d))
+
+
+@pytest.mark.parametrize("d,head_dim,g,message", [(96, 64, 1, "not a multiple of head_dim"), (64, 0, 1, "not a multiple of head_dim"),
+                                                  (64, -64, 1, "not a multiple of head_dim"), (128, 64, 0, "not divisible by n_groups"),
+                                                  (128, 64, 3, "not divisible by n_groups")])
+def test_core_refuses_channels_that_are_no_whole_heads(d, head_dim, g, message):
+    from mamba2 import _lib
+    from mamba2.fused_kernel import mamba2_fused_kernel, mamba2_fused_kernel_with_caching, mamba2_fused_prefill
+    h, n = d // head_dim if head_dim > 0 else 1, 64
+    args = _core_args(h, d, g, n)
+    for core in (mamba2_fused_kernel, mamba2_fused_kernel_with_caching):
+        with pytest.raises(ValueError, match=message):
+            core(*args, g, n, d, head_dim)
+    with pytest.raises(ValueError, match=message):
+        mamba2_fused_prefill(*args, g, n, d, head_dim, torch.zeros(1, d + 2 * g * n, 3), torch.zeros(1, h, 64, n))
+    hidden, width = torch.zeros(1, 8, 32), 2 * d + 2 * g * n + h
+    with pytest.raises(ValueError, match=message):
+        _lib.native().mixer(hidden, torch.zeros(width, 32), args[1], args[2], args[5], args[3], args[6], torch.zeros(32, d), args[4], None, None,
+                            g, n, d, head_dim, False)
+
+
+def test_no_groups_is_an_error_and_not_a_division(lib):
+    from mamba2 import _lib
+    from mamba2.mamba2_kernel import mamba2_kernel
+    with pytest.raises(ValueError, match="not divisible by n_groups"):
+        mamba2_kernel(torch.zeros(1, 128, 2), torch.zeros(2), torch.zeros(1, 128, 2, 64), torch.zeros(1, 128, 0, 64), torch.zeros(1, 128, 0, 64), torch.zeros(2))
+    p = _lib.SsdParams()
+    p.batch, p.seqlen, p.nheads, p.headdim, p.dstate, p.ngroups = 1, 128, 2, 64, 64, 0
+    assert lib.m2_ssd_bwd_workspace_bytes(ctypes.byref(p)) > 0
+    assert lib.m2_ssd_bwd(ctypes.byref(p), None) == -1
