@@ -860,6 +860,19 @@ const Tensor& stream_rows(ResidualStream& r) {
     return r.rows;
 }
 
+// The stream's rows, everything added, after a norm, in out_dtype: one kernel, or where what is left to add is of another type (a
+// head or a layer of its own precision behind it) that sum first.
+Tensor stream_add_norm(ResidualStream& r, const Tensor& norm_w, double eps, at::ScalarType out_dtype) {
+    const Tensor& rows = stream_rows(r);
+    if (r.delta.defined() && r.delta.scalar_type() != out_dtype) {
+        rows.add_(r.delta);
+        r.delta = Tensor();
+    }
+    const Tensor out = add_rmsnorm(rows, r.delta.defined() ? OptTensor(r.delta) : std::nullopt, norm_w, eps, out_dtype);
+    r.delta = r.x = r.sq = Tensor();
+    return out;
+}
+
 // x and sq of the stream for a norm weight
 void stream_heads(ResidualStream& r, const Tensor& norm_w, void* stream) {
     if (r.x.defined()) return;
@@ -888,11 +901,7 @@ Tensor step_rows(const Tensor& hidden, ResidualStream* r, const Tensor& block_no
                        lib.m2_linear_small_fits(in.M, in.N, in.K, 1) && lib.m2_linear_small_fits(out.M, out.N, out.K, static_cast<int32_t>(a.norm_groups)) &&
                        (hd == 64 || hd == 128) && (n == 64 || n == 128) && a.conv_w.size(-1) == 4 && h % a.norm_groups == 0;
     if (!fused) {
-        Tensor rows = hidden;
-        if (r) {
-            rows = add_rmsnorm(stream_rows(*r), r->delta.defined() ? OptTensor(r->delta) : std::nullopt, block_norm, block_eps, act_type);
-            r->x = r->sq = Tensor();
-        }
+        const Tensor rows = r ? stream_add_norm(*r, block_norm, block_eps, act_type) : hidden;
         const Tensor packed = linear_rows(rows, a.in_w, a.in_b, stream).unsqueeze(1);
         const int64_t cx = d + 2 * a.g * n;
         const Tensor y = std::get<0>(decode_step(packed.narrow(2, d, cx), a.conv_state, a.conv_w, a.conv_b.defined() ? OptTensor(a.conv_b) : std::nullopt,
@@ -972,9 +981,9 @@ Tensor mixer_step(const OptTensor& hidden_, ResidualStream* r, const OptTensor& 
 
 ResidualStream residual_stream(const Tensor& embedded) {
     require_gpu({&embedded});
-    dtype_code(embedded);
+    const bool read = embedded.scalar_type() == at::kFloat || embedded.scalar_type() == at::kBFloat16;      // as the kernels read it
     ResidualStream r;
-    r.first = embedded.reshape({-1, embedded.size(-1)});
+    r.first = (read ? embedded : embedded.to(at::kFloat)).reshape({-1, embedded.size(-1)});
     return r;
 }
 
@@ -991,10 +1000,7 @@ Tensor stream_sum(ResidualStream& r) {
 Tensor stream_norm(ResidualStream& r, const Tensor& norm_w, double eps, at::ScalarType out_dtype) {
     check_fp32({&norm_w}, "the norm weight");
     Scope scope(norm_w);
-    const Tensor& rows = stream_rows(r);
-    const Tensor out = add_rmsnorm(rows, r.delta.defined() ? OptTensor(r.delta) : std::nullopt, norm_w, eps, out_dtype);
-    r.delta = r.x = r.sq = Tensor();
-    return out;
+    return stream_add_norm(r, norm_w, eps, out_dtype);
 }
 
 // fp32 product of the normalised rows: norm_f and the LM head (modeling_mamba2.py:350, 489-490)
@@ -1006,8 +1012,10 @@ Tensor stream_norm_linear(ResidualStream& r, const Tensor& norm_w, double eps, c
     TORCH_CHECK_VALUE(w.dim() == 2 && any.size(1) == w.size(1) && norm_w.numel() == w.size(1), "the norm weight and the product must have the width of the residual stream");
     Scope scope(w);
     m2_linear_params p = linear_params(w, bias, any.size(0));
-    if (!linear_takes(w, bias) || !lib.m2_linear_small_fits(p.M, p.N, p.K, 1))
-        return linear_rows(stream_norm(r, norm_w, eps, w.scalar_type()), w, bias, scope.stream).to(at::kFloat);
+    if (!linear_takes(w, bias) || !lib.m2_linear_small_fits(p.M, p.N, p.K, 1)) {
+        const at::ScalarType normed = w.scalar_type() == at::kBFloat16 ? at::kBFloat16 : at::kFloat;      // the norm's output types
+        return linear_rows(stream_add_norm(r, norm_w, eps, normed).to(w.scalar_type()), w, bias, scope.stream).to(at::kFloat);
+    }
     stream_heads(r, norm_w, scope.stream);
     const Tensor out = at::empty({p.M, p.N}, r.rows.options());
     set_rows(p, r.x, r.sq, eps);

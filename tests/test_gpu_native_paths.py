@@ -1,0 +1,78 @@
+"""GPU: calls that the native step and layer take or leave to the modules: parameters of other types and alignments, hooks and
+overrides, a prefill that fails.  The reference is the same work block by block, module by module."""
+import pytest
+import torch
+
+from conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _rel(got, ref):
+    return ((got.double() - ref.double()).norm() / ref.double().norm()).item()
+
+
+def _model(layers=2, dtype=torch.bfloat16, **kw):
+    from mamba2.configuration_mamba2 import Mamba2Config
+    from mamba2.modeling_mamba2 import Mamba2ForCausalLM
+    cfg = Mamba2Config(num_heads=8, head_dim=64, hidden_size=256, state_size=64, n_groups=2, num_hidden_layers=layers, vocab_size=320, expand=2,
+                       residual_in_fp32=True, **kw)
+    torch.manual_seed(0)
+    return cfg, Mamba2ForCausalLM(cfg).to(DEV).to(dtype).eval()
+
+
+def _cache(cfg, b, dtype=torch.bfloat16, seed=1):
+    from mamba2.mamba2_mixer import Mamba2Cache
+    cache = Mamba2Cache(cfg, b, dtype=dtype, device=DEV)
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    for t in cache.conv_states + cache.ssm_states:
+        t.normal_(0, 0.3, generator=gen)
+    return cache
+
+
+@torch.no_grad()
+def _blockwise(m, ids, cache):
+    x = m.backbone.embeddings(ids).float()
+    for blk in m.backbone.layers:
+        x = x + blk.mixer.step(blk.norm(x).to(blk.mixer.in_proj.weight.dtype), cache)
+    return m.backbone.norm_f(x).double() @ m.lm_head.weight.double().T
+
+
+@pytest.mark.parametrize("b", [5, 33])
+@pytest.mark.parametrize("layers,head,table", [("bfloat16", "float32", "bfloat16"), ("float32", "bfloat16", "float32"), ("bfloat16", "float16", "bfloat16"),
+                                               ("bfloat16", "bfloat16", "float16")])
+def test_step_of_a_model_with_a_head_of_another_dtype(b, layers, head, table):
+    cfg, m = _model(dtype=getattr(torch, layers))
+    m.lm_head.to(getattr(torch, head))
+    m.backbone.embeddings.to(getattr(torch, table))
+    ids = torch.randint(0, cfg.vocab_size, (b, 1), generator=torch.Generator().manual_seed(2)).to(DEV)
+    c1, c2 = (_cache(cfg, b, getattr(torch, layers)) for _ in range(2))
+    for _ in range(2):
+        with torch.no_grad():
+            got = m.step(ids, c1)
+        assert got.dtype == torch.float32 and _rel(got, _blockwise(m, ids, c2)) < 1e-2      # bf16 rows and layers
+    assert _rel(c1.ssm_states[1], c2.ssm_states[1]) < 1e-2
+
+
+@pytest.mark.parametrize("b", [5, 33])
+def test_step_through_layers_of_two_dtypes(b):
+    """What a bf16 layer leaves to be added in front of an fp32 one goes into the stream as it is."""
+    from mamba2 import _lib
+    cfg, m = _model()
+    blocks = list(m.backbone.layers)
+    blocks[1].float()
+    c = _cache(cfg, b)
+    c.conv_states[1] = c.conv_states[1].float()
+    c2 = _cache(cfg, b)
+    c2.conv_states[1] = c2.conv_states[1].float()
+    x = torch.randn(b, 1, cfg.hidden_size, generator=torch.Generator().manual_seed(3)).to(DEV)
+    with torch.no_grad():
+        stream = _lib.native().residual_stream(x)
+        for i, blk in enumerate(blocks):
+            blk.mixer._step(c, stream=stream, block_norm=blk.norm)
+        got = _lib.native().stream_sum(stream).view(x.shape)
+        want = x
+        for blk in blocks:
+            want = want + blk.mixer.step(blk.norm(want).to(blk.mixer.in_proj.weight.dtype), c2)
+    assert rel_err(got, want) < 1e-2
