@@ -830,8 +830,18 @@ struct ResidualStream {
     Tensor first;                  // embedding rows that `rows` is yet to be set to
 };
 
+bool starts_at(const Tensor& t, size_t bytes) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % bytes == 0; }
+
+// the small product's kernel copies 16 bytes at a time (a view into a flat buffer of parameters may start anywhere)
 bool linear_takes(const Tensor& w, const Tensor& bias) {
-    return w.scalar_type() == at::kBFloat16 && w.is_contiguous() && (!bias.defined() || (bias.is_contiguous() && bias.scalar_type() == at::kBFloat16));
+    return w.scalar_type() == at::kBFloat16 && w.is_contiguous() && starts_at(w, 16) &&
+           (!bias.defined() || (bias.is_contiguous() && bias.scalar_type() == at::kBFloat16));
+}
+
+// rows as that kernel reads them: 16-byte pieces at 32-bit byte offsets from the first row; others are copied once
+Tensor linear_input(const Tensor& x) {
+    const bool fits = x.stride(1) == 1 && starts_at(x, 16) && x.stride(0) % 8 == 0 && x.stride(0) < (int64_t{1} << 26);
+    return fits ? x : x.clone(at::MemoryFormat::Contiguous);
 }
 
 m2_linear_params linear_params(const Tensor& w, const Tensor& bias, int64_t rows) {
@@ -844,7 +854,7 @@ m2_linear_params linear_params(const Tensor& w, const Tensor& bias, int64_t rows
 Tensor linear_rows(const Tensor& x, const Tensor& w, const Tensor& bias, void* stream) {
     m2_linear_params p = linear_params(w, bias, x.size(0));
     if (x.scalar_type() != at::kBFloat16 || !linear_takes(w, bias) || !lib.m2_linear_small_fits(p.M, p.N, p.K, 1)) return project(x, w, bias, stream);
-    const Tensor xr = aligned(x);
+    const Tensor xr = linear_input(x);
     Tensor out = at::empty({p.M, p.N}, x.options());
     p.x = ptr(xr); p.x_stride_row = xr.stride(0); p.out = ptr(out); p.out_stride_row = p.N;
     check(lib.m2_linear_small(&p, stream), "m2_linear_small");
@@ -868,7 +878,8 @@ Tensor stream_add_norm(ResidualStream& r, const Tensor& norm_w, double eps, at::
         rows.add_(r.delta);
         r.delta = Tensor();
     }
-    const Tensor out = add_rmsnorm(rows, r.delta.defined() ? OptTensor(r.delta) : std::nullopt, norm_w, eps, out_dtype);
+    const Tensor w = starts_at(norm_w, 16) ? norm_w : norm_w.clone();
+    const Tensor out = add_rmsnorm(rows, r.delta.defined() ? OptTensor(r.delta) : std::nullopt, w, eps, out_dtype);
     r.delta = r.x = r.sq = Tensor();
     return out;
 }
@@ -912,9 +923,10 @@ Tensor step_rows(const Tensor& hidden, ResidualStream* r, const Tensor& block_no
         return o;
     }
     const Tensor zx = at::empty({b, a.in_w.size(0)}, act);
-    const Tensor conv_w = a.conv_w.contiguous(), conv_b = a.conv_b.defined() ? a.conv_b.contiguous() : a.conv_b;
+    const Tensor conv_c = a.conv_w.contiguous(), conv_b = a.conv_b.defined() ? a.conv_b.contiguous() : a.conv_b;
+    const Tensor conv_w = starts_at(conv_c, 4 * conv_c.element_size()) ? conv_c : conv_c.clone();      // a channel's four taps in one load
     const Tensor mid = at::empty({b * (d * 2 + h * 4)}, act.dtype(at::kByte));          // gated rows (bf16), then the head sums (fp32)
-    const Tensor x = r ? Tensor() : aligned(hidden);
+    const Tensor x = r ? Tensor() : linear_input(hidden);
     Tensor result, next_x, next_sq;
     if (r) {
         stream_heads(*r, block_norm, stream);

@@ -389,6 +389,8 @@ int check_linear(const m2_linear_params* p) {
     M2_REQUIRE(p->out_kind >= kOutBf16 && p->out_kind <= kOutAdd && (!p->next_weight || (p->out_kind == kOutAdd && p->next_x && p->next_sq)), M2_ERR_NULL,
                "linear_small: next_weight goes with out_kind 2, next_x and next_sq");
     M2_REQUIRE(aligned16(p->x) && aligned16(p->w) && p->x_stride_row % 8 == 0, M2_ERR_ALIGN, "linear_small: x rows and w must be 16-byte aligned");
+    M2_REQUIRE(p->x_stride_row >= 0 && p->M * p->x_stride_row < ((int64_t)1 << 31), M2_ERR_SHAPE,
+               "linear_small: %lld rows %lld elements apart are out of reach of 32-bit byte offsets", (long long)p->M, (long long)p->x_stride_row);
     return M2_OK;
 }
 
@@ -444,7 +446,8 @@ extern "C" int m2_decode_layer(const m2_linear_params* in, const m2_decode_param
     if (dec->batch == 0) return M2_OK;
     M2_REQUIRE(dec->conv_state && dec->conv_w && dec->S && dec->A && dec->dt_bias && norm_weight && out->sq && out->x, M2_ERR_NULL,
                "decode_layer: conv_state, conv_w, S, A, dt_bias, norm_weight, and the scratch behind out->x and out->sq are required");
-    M2_REQUIRE(aligned16(dec->S), M2_ERR_ALIGN, "decode_layer: S must be 16-byte aligned");
+    M2_REQUIRE(aligned16(dec->S) && (uintptr_t)dec->conv_w % (dec->param_dtype == M2_F32 ? 16 : 8) == 0, M2_ERR_ALIGN,
+               "decode_layer: S must be 16-byte aligned, the conv weight on four of its elements");
     hipStream_t st = static_cast<hipStream_t>(stream);
     int rc = check_linear(out);
     if (rc) return rc;

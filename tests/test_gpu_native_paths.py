@@ -76,3 +76,58 @@ def test_step_through_layers_of_two_dtypes(b):
         for blk in blocks:
             want = want + blk.mixer.step(blk.norm(want).to(blk.mixer.in_proj.weight.dtype), c2)
     assert rel_err(got, want) < 1e-2
+
+
+def _views_of_one_buffer(module, offset):
+    """Every parameter a contiguous view into one flat buffer per dtype, `offset` elements off the allocation's alignment."""
+    for dtype in {p.dtype for p in module.parameters()}:
+        ps = [p for p in module.parameters() if p.dtype == dtype]
+        flat = torch.empty(sum(p.numel() + 8 for p in ps) + offset, dtype=dtype, device=DEV)
+        at = offset
+        for p in ps:
+            p.data = flat[at:at + p.numel()].copy_(p.detach().reshape(-1)).view(p.shape)
+            at += -(-p.numel() // 8) * 8
+    return module
+
+
+@pytest.mark.parametrize("b", [3, 33])
+@pytest.mark.parametrize("offset", [1, 4])
+def test_weights_that_start_anywhere(b, offset):
+    """Views into a flat buffer of parameters: contiguous, but on no 16-byte boundary."""
+    cfg, m = _model()
+    ids = torch.randint(0, cfg.vocab_size, (b, 1), generator=torch.Generator().manual_seed(2)).to(DEV)
+    c1, c2, c3 = (_cache(cfg, b) for _ in range(3))
+    with torch.no_grad():
+        want = m.step(ids, c1)
+        for block in m.backbone.layers:
+            block.norm.float()
+        _views_of_one_buffer(m, offset)
+        assert m.lm_head.weight.data_ptr() % 16 and m.lm_head.weight.is_contiguous()
+        got = m.step(ids, c2)
+        x = m.backbone.embeddings(ids).float()
+        block = m.backbone.layers[0]
+        assert _rel(block.step(x, c3), x + block.mixer.step(block.norm(x).bfloat16(), _cache(cfg, b))) < 1e-2
+    assert _rel(got, want) < 1e-2 and _rel(c2.ssm_states[1], c1.ssm_states[1]) < 1e-2
+    assert torch.equal(c2.conv_states[0][..., :-1], c1.conv_states[0][..., :-1])
+
+
+@pytest.mark.parametrize("b", [3, 33])
+def test_layer_step_on_rows_of_any_stride(b):
+    """The last token of a longer tensor, a column slice that starts anywhere, a transposed and an expanded one."""
+    cfg, m = _model(1)
+    mixer, d = m.backbone.layers[0].mixer, cfg.hidden_size
+    gen = torch.Generator().manual_seed(4)
+    x = torch.randn(b, 1, d, generator=gen).bfloat16().to(DEV)
+    long, wide = torch.zeros(b, 7, d, dtype=x.dtype, device=DEV), torch.zeros(b, 1, d + 5, dtype=x.dtype, device=DEV)
+    long[:, -1:], wide[..., 3:3 + d] = x, x
+    far = torch.empty(b, (1 << 26) // d + 1, d, dtype=x.dtype, device=DEV)[:, -1:]      # rows more than 2^26 elements apart
+    far.copy_(x)
+    forms = {"last": long[:, -1:], "columns": wide[..., 3:3 + d], "transposed": x[:, 0].T.contiguous().T[:, None], "far": far}
+    forms["expanded"] = x[:1].expand(b, 1, d)
+    for name, form in forms.items():
+        c1, c2 = (_cache(cfg, b) for _ in range(2))
+        with torch.no_grad():
+            want, got = mixer.step(form.contiguous(), c1), mixer.step(form, c2)
+        # up to 32 rows one kernel takes them all; above, some forms go to the library's product, which sums in another order
+        for a, e in ((got, want), (c2.ssm_states[0], c1.ssm_states[0])):
+            assert torch.equal(a, e) if b <= 32 else _rel(a, e) < 1e-2, name

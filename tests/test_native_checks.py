@@ -39,3 +39,11 @@ def test_no_groups_is_an_error_and_not_a_division(lib):
     p.batch, p.seqlen, p.nheads, p.headdim, p.dstate, p.ngroups = 1, 128, 2, 64, 64, 0
     assert lib.m2_ssd_bwd_workspace_bytes(ctypes.byref(p)) > 0
     assert lib.m2_ssd_bwd(ctypes.byref(p), None) == -1
+
+
+def test_small_products_refuse_what_their_addressing_does_not_reach(lib):
+    from mamba2 import _lib
+    p = _lib.LinearParams(x=16, w=16, out=16, M=32, N=64, K=64, x_stride_row=1 << 26, out_stride_row=64, groups=1)
+    assert lib.m2_linear_small(ctypes.byref(p), None) == -1 and b"32-bit" in lib.m2_last_error()
+    p.x_stride_row, p.w = 64, 24
+    assert lib.m2_linear_small(ctypes.byref(p), None) == -3
