@@ -448,7 +448,7 @@ def bench_model_step(steps, warmup, tune_gemms=True):
                 config={"workload": "Mamba2ForCausalLM.step, d_model 2560, 64 layers, h80 p64 n128 g1, vocab 50288, b128, conv state W3"},
                 roofline={"bound": "hbm", "achieved": bytes_ / (ms_g * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                           "frac": bytes_ / (ms_g * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": None, "algorithmic_bytes_per_step": bytes_,
-                          "kernels": "one graph replay: projections (" + ("rocBLAS / hipBLASLt solutions chosen by torch TunableOp during the graph's warm-up; the eager figure uses the libraries' defaults" if tune_gemms else "the BLAS libraries' default solutions") + ") + decode_conv/decode_ssm/rmsnorm_gated kernels + torch elementwise"})
+                          "kernels": "one graph replay: projections (" + ("rocBLAS / hipBLASLt solutions chosen by torch TunableOp during the graph's warm-up; the eager figure uses product_kernel" if tune_gemms else "product_kernel, LM head by the BLAS library's default solution") + ") + decode_conv/decode_ssm/rmsnorm_gated/add_rmsnorm kernels"})
 
 
 def bench_copy(steps, warmup):

@@ -131,3 +131,31 @@ def test_layer_step_on_rows_of_any_stride(b):
         # up to 32 rows one kernel takes them all; above, some forms go to the library's product, which sums in another order
         for a, e in ((got, want), (c2.ssm_states[0], c1.ssm_states[0])):
             assert torch.equal(a, e) if b <= 32 else _rel(a, e) < 1e-2, name
+
+
+def test_tuned_step_lets_the_library_try_the_projections():
+    """GraphedStep(tune_gemms=True) above 32 sequences: the projections' shapes are among those that TunableOp timed, and while it is
+    off they run in this library's kernel (bit for bit the untuned step's logits)."""
+    import torch.cuda.tunable as tunable
+    from mamba2.modeling_mamba2 import GraphedStep
+    cfg, m = _model()
+    b = 56
+    ids = torch.randint(0, cfg.vocab_size, (b, 1), generator=torch.Generator().manual_seed(2)).to(DEV)
+    c1, c2, c3 = (_cache(cfg, b) for _ in range(3))
+    with torch.no_grad():
+        before = m.step(ids, c1)
+    limits = tunable.get_max_tuning_duration(), tunable.get_max_tuning_iterations()
+    try:
+        tunable.set_max_tuning_duration(1)
+        tunable.set_max_tuning_iterations(1)
+        step = GraphedStep(m, c2, b, tune_gemms=True)
+    finally:
+        tunable.set_max_tuning_duration(limits[0])
+        tunable.set_max_tuning_iterations(limits[1])
+    shapes = " ".join(r[1] for r in tunable.get_results())
+    mixer = m.backbone.layers[0].mixer
+    for proj in (mixer.in_proj, mixer.out_proj):
+        assert f"{proj.out_features}_{b}_{proj.in_features}" in shapes, shapes
+    assert _rel(step(ids), before) < 1e-2
+    with torch.no_grad():
+        assert torch.equal(m.step(ids, c3), before)
