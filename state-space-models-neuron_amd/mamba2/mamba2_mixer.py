@@ -27,10 +27,27 @@ def softplus(x, threshold=10):
     return torch.where(x < threshold, torch.log1p(torch.exp(torch.clamp(x, max=threshold))), x)
 
 
+_PLAIN_TENSORS = (nn.Parameter, torch.Tensor, type(None))
+
+
+def _plain(m, cls):
+    """True if calling ``m`` is nothing but ``cls.forward`` on parameters of its own: ``cls`` itself and no subclass or wrapper, no
+    hooks, no ``forward`` put on the instance, not compiled, no parametrization and no parameter of a tensor subclass."""
+    d = m.__dict__
+    if type(m) is not cls or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] or "forward" in d:
+        return False
+    params = d["_parameters"]
+    return ("weight" in params and all(type(p) in _PLAIN_TENSORS for p in params.values()) and m._compiled_call_impl is None
+            and not nn.modules.module._has_any_global_hook())
+
+
 def _plain_linear(m):
-    """True if calling ``m`` is nothing but its product: an ``nn.Linear`` itself, no subclass or wrapper, no hooks."""
-    return type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                                         or nn.modules.module._has_any_global_hook())
+    return _plain(m, nn.Linear)
+
+
+def _own_step(m, cls):
+    """True if ``m.step`` is ``cls.step``: neither a subclass nor the instance has one of its own (nor is ``m`` another module)."""
+    return getattr(type(m), "step", None) is cls.step and "step" not in m.__dict__
 
 
 def _inference_linear(m, x):
@@ -186,7 +203,7 @@ class Mamba2Mixer(nn.Module):
     def _native_step(self):
         """True if the step is the native one: inference on plain projections and norm (no wrappers, hooks or autocast)."""
         return (not torch.is_grad_enabled() and _plain_linear(self.in_proj) and _plain_linear(self.out_proj)
-                and type(self.norm) is MambaRMSNormGated and not torch.is_autocast_enabled())
+                and _plain(self.norm, MambaRMSNormGated) and not torch.is_autocast_enabled())
 
     def _step(self, cache_params, hidden=None, stream=None, block_norm=None, next_norm=None):
         """One token through the layer: ``hidden`` (b, 1, D) -> the layer's output; or, with a native residual ``stream``, the block

@@ -20,7 +20,7 @@ from torch import nn
 
 from . import _lib, glue
 from .configuration_mamba2 import Mamba2Config
-from .mamba2_mixer import Mamba2Cache, Mamba2Mixer, _plain_linear
+from .mamba2_mixer import Mamba2Cache, Mamba2Mixer, _own_step, _plain, _plain_linear
 
 
 class Mamba2RMSNorm(nn.Module):
@@ -59,10 +59,11 @@ class Mamba2Block(nn.Module):
         return residual + hidden_states
 
     def _native_step(self):
-        """True if the block's step runs in a native fp32 residual stream."""
+        """True if the block's step runs in a native fp32 residual stream (which calls neither the norm nor ``mixer.step``)."""
+        if not (self.residual_in_fp32 and _plain(self.norm, Mamba2RMSNorm) and _own_step(self.mixer, Mamba2Mixer) and self.mixer._native_step()):
+            return False
         weight = self.norm.weight
-        return (self.residual_in_fp32 and type(self.norm) is Mamba2RMSNorm and self.mixer._native_step() and weight.is_cuda
-                and glue.add_rmsnorm_ok(weight.shape[0], self.mixer.in_proj.weight.dtype))
+        return weight.is_cuda and glue.add_rmsnorm_ok(weight.shape[0], self.mixer.in_proj.weight.dtype)
 
     def step(self, x, cache_params: Optional[Mamba2Cache] = None):
         if self._native_step() and x.dtype in (torch.float32, torch.bfloat16):
@@ -194,7 +195,7 @@ class Mamba2Model(Mamba2PreTrainedModel):
         """The native fp32 residual stream behind the last block, for inference with ``residual_in_fp32``: each block's norm and
         residual add are part of its kernels or of one pass between them (the arithmetic of Mamba2Block.step: fp32 sums and
         norm).  None where the blocks have to be called one by one."""
-        if not (len(self.layers) and type(self.norm_f) is Mamba2RMSNorm and all(blk._native_step() for blk in self.layers)):
+        if not (len(self.layers) and _plain(self.norm_f, Mamba2RMSNorm) and all(_own_step(blk, Mamba2Block) and blk._native_step() for blk in self.layers)):
             return None
         norms = [blk.norm for blk in self.layers] + [self.norm_f]
         stream = _lib.native().residual_stream(self.embeddings(input_ids))
@@ -250,7 +251,8 @@ class Mamba2ForCausalLM(Mamba2PreTrainedModel):
 
     def step(self, idx, cache_params: Optional[Mamba2Cache] = None):
         """idx: int64 (batch, 1) -> logits (batch, 1, vocab) fp32; the layers' states in ``cache_params`` advance by one token."""
-        stream = self.backbone._step_stream(idx, cache_params) if _plain_linear(self.lm_head) and not torch.is_grad_enabled() else None
+        native = _own_step(self.backbone, Mamba2Model) and _plain_linear(self.lm_head) and not torch.is_grad_enabled()
+        stream = self.backbone._step_stream(idx, cache_params) if native else None
         if stream is not None:
             norm_f = self.backbone.norm_f
             logits = _lib.native().stream_norm_linear(stream, _lib.f32_param(norm_f.weight), norm_f.variance_epsilon, self.lm_head.weight, self.lm_head.bias)

@@ -159,3 +159,100 @@ def test_tuned_step_lets_the_library_try_the_projections():
     assert _rel(step(ids), before) < 1e-2
     with torch.no_grad():
         assert torch.equal(m.step(ids, c3), before)
+
+
+def _hook(m, calls):
+    m.register_forward_hook(lambda *_: calls.append(1))
+
+
+def _replaced(m, calls):
+    forward = m.forward
+
+    def wrapper(*args, **kwargs):
+        calls.append(1)
+        return forward(*args, **kwargs)
+
+    m.forward = wrapper
+
+
+def _own_step(m, calls):
+    class Other(type(m)):
+        def step(self, *args, **kwargs):
+            calls.append(1)
+            return super().step(*args, **kwargs)
+
+    m.__class__ = Other
+
+
+@pytest.mark.parametrize("change,where", [(c, w) for c in (_hook, _replaced) for w in ("norm", "mixer.norm", "mixer.in_proj", "mixer.out_proj")]
+                         + [(_own_step, "mixer"), (_own_step, "")])
+def test_step_calls_what_a_user_put_there(change, where):
+    """A hook, a replaced forward and a step of one's own run once per token, in a layer's, a block's and a model's step, and change
+    nothing else."""
+    cfg, m = _model()
+    b = 3
+    ids = torch.randint(0, cfg.vocab_size, (b, 1), generator=torch.Generator().manual_seed(2)).to(DEV)
+    calls = []
+    block = m.backbone.layers[1]
+    with torch.no_grad():
+        x = m.backbone.embeddings(ids)
+        want = m.step(ids, _cache(cfg, b)), block.step(x.float(), _cache(cfg, b)), block.mixer.step(x, _cache(cfg, b))
+        change(block.get_submodule(where), calls)
+        got = m.step(ids, _cache(cfg, b)), block.step(x.float(), _cache(cfg, b))
+        assert len(calls) == 2
+        if where.startswith("mixer"):
+            got += (block.mixer.step(x, _cache(cfg, b)),)
+            assert len(calls) == 3
+    for g, w in zip(got, want):
+        assert _rel(g, w) < 1e-2
+
+
+@pytest.mark.parametrize("change,where", [(_hook, "backbone.norm_f"), (_replaced, "backbone.norm_f"), (_hook, "lm_head"), (_replaced, "lm_head"), (_own_step, "backbone")])
+def test_model_step_calls_what_a_user_put_there(change, where):
+    cfg, m = _model()
+    ids = torch.randint(0, cfg.vocab_size, (3, 1), generator=torch.Generator().manual_seed(2)).to(DEV)
+    calls = []
+    with torch.no_grad():
+        want = m.step(ids, _cache(cfg, 3))
+        change(m.get_submodule(where), calls)
+        assert _rel(m.step(ids, _cache(cfg, 3)), want) < 1e-2 and len(calls) == 1
+
+
+@pytest.mark.parametrize("change", [_hook, _replaced])
+@pytest.mark.parametrize("where", ["in_proj", "out_proj"])
+def test_forward_and_prefill_call_what_a_user_put_there(change, where):
+    cfg, m = _model(1)
+    mixer, calls = m.backbone.layers[0].mixer, []
+    x = torch.randn(2, 40, cfg.hidden_size, generator=torch.Generator().manual_seed(5)).bfloat16().to(DEV)
+
+    def passes():
+        out = mixer(x)
+        grad, = torch.autograd.grad(out.float().pow(2).sum(), mixer.A_log)
+        with torch.no_grad():
+            return out.detach(), grad, mixer(x, cache_params=_cache(cfg, 2))
+
+    want = passes()
+    change(mixer.get_submodule(where), calls)
+    for g, w in zip(passes(), want):
+        assert _rel(g, w) < 2e-2
+    assert len(calls) == 2
+
+
+def test_model_of_other_blocks_is_stepped_through_their_own_step():
+    class Own(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def step(self, *args, **kwargs):
+            return self.inner.step(*args, **kwargs)
+
+    cfg, m = _model()
+    ids = torch.randint(0, cfg.vocab_size, (3, 1), generator=torch.Generator().manual_seed(2)).to(DEV)
+    with torch.no_grad():
+        want = m.step(ids, _cache(cfg, 3))
+        m.backbone.layers[0].mixer = Own(m.backbone.layers[0].mixer)
+        m.backbone.layers[0].mixer.in_proj = m.backbone.layers[0].mixer.inner.in_proj      # whose dtype the block's norm is cast to
+        m.backbone.layers[1] = Own(m.backbone.layers[1])
+        m.backbone.layers[0].mixer.inner.norm.register_forward_hook(lambda *_: None)
+        assert _rel(m.step(ids, _cache(cfg, 3)), want) < 1e-2
