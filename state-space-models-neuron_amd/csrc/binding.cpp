@@ -678,6 +678,10 @@ Tensor linear(const Tensor& x, const Tensor& w, const OptTensor& bias) {
     return project(x.reshape({-1, w.size(1)}), w, or_none(bias), scope.stream).view(shape);
 }
 
+bool casts(const Tensor& t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16; }
+// a small parameter as the casting kernel reads it; types that it does not take come as fp32
+Tensor small_param(const Tensor& t) { return (casts(t) ? t : t.to(at::kFloat)).contiguous(); }
+
 struct MixerFn : torch::autograd::Function<MixerFn> {
     enum { kHidden, kInW, kALog, kD, kDtBias, kConvW, kNormW, kOutW, kConvB, kInB, kOutB, kSmall, kZx, kNormOut, kConvOut, kScanOut, kStates };
     static Tensor forward(AutogradContext* ctx, const Tensor& hidden, const Tensor& in_w, const Tensor& A_log, const Tensor& D, const Tensor& dt_bias,
@@ -690,7 +694,7 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
         const Packed k(zx, g, n, d, hd);
         check_core(k, A_log, D, conv_w, or_none(conv_b), dt_bias, norm_w);
         const Tensor small = empty_f32({3 * h + d}, zx);
-        const Tensor a = A_log.contiguous(), dd = D.contiguous(), tb = dt_bias.contiguous(), nw = norm_w.contiguous();
+        const Tensor a = small_param(A_log), dd = small_param(D), tb = small_param(dt_bias), nw = small_param(norm_w);
         check(lib.m2_mixer_params(ptr(a), dtype_code(a), ptr(dd), dtype_code(dd), ptr(tb), dtype_code(tb), ptr(nw), dtype_code(nw), ptr<float>(small),
                                   h, d, scope.stream), "m2_mixer_params");
         const CoreOut r = core_forward(k, small.narrow(0, 0, h), small.narrow(0, h, h), conv_w, or_none(conv_b), small.narrow(0, 2 * h, h),
@@ -722,10 +726,12 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
         if (s.size() > kConvOut) { f.conv_out = s[kConvOut]; f.scan_out = s[kScanOut]; f.states = s[kStates]; }
         else f = core_forward(k, A, D, s[kConvW], s[kConvB], dt_bias, norm_w, true, false, scope.stream);
         const CoreGrads r = core_backward(k, d_core, A, D, s[kConvW], s[kConvB], dt_bias, norm_w, f.conv_out, f.scan_out, f.states, scope.stream);
-        for (const int i : {kALog, kD, kDtBias, kNormW}) out[i] = at::empty(s[i].sizes(), s[i].options());
+        for (const int i : {kALog, kD, kDtBias, kNormW}) out[i] = at::empty(s[i].sizes(), casts(s[i]) ? s[i].options() : s[i].options().dtype(at::kFloat));
         check(lib.m2_mixer_params_grads(ptr<float>(A), ptr<float>(r.A), ptr<float>(r.D), ptr<float>(r.dt_bias), ptr<float>(r.norm_w), ptr(out[kALog]),
-                                        dtype_code(s[kALog]), ptr(out[kD]), dtype_code(s[kD]), ptr(out[kDtBias]), dtype_code(s[kDtBias]), ptr(out[kNormW]),
-                                        dtype_code(s[kNormW]), k.h, k.d, scope.stream), "m2_mixer_params_grads");
+                                        dtype_code(out[kALog]), ptr(out[kD]), dtype_code(out[kD]), ptr(out[kDtBias]), dtype_code(out[kDtBias]), ptr(out[kNormW]),
+                                        dtype_code(out[kNormW]), k.h, k.d, scope.stream), "m2_mixer_params_grads");
+        for (const int i : {kALog, kD, kDtBias, kNormW})
+            if (!casts(s[i])) out[i] = out[i].to(s[i].scalar_type());
         out[kConvW] = r.conv_w; out[kConvB] = r.conv_b;
         const Tensor d_zx = r.zx.view({rows, zx.size(2)});
         if (ctx->needs_input_grad(kHidden)) out[kHidden] = product(d_zx, true, s[kInW], false, Tensor(), scope.stream).view(s[kHidden].sizes());

@@ -256,3 +256,28 @@ def test_model_of_other_blocks_is_stepped_through_their_own_step():
         m.backbone.layers[1] = Own(m.backbone.layers[1])
         m.backbone.layers[0].mixer.inner.norm.register_forward_hook(lambda *_: None)
         assert _rel(m.step(ids, _cache(cfg, 3)), want) < 1e-2
+
+
+@pytest.mark.parametrize("types", [(torch.float64, torch.float16, torch.float64, torch.float16), (torch.float16, torch.float32, torch.bfloat16, torch.float64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_layer_takes_small_parameters_of_any_type(types, dtype):
+    """A_log, D, dt_bias and the norm's weight in types that the casting kernel does not read: as the modules one by one take them."""
+    cfg, m = _model(1, dtype)
+    mixer = m.backbone.layers[0].mixer
+    for owner, name, t in zip((mixer, mixer, mixer, mixer.norm), ("A_log", "D", "dt_bias", "weight"), types):
+        setattr(owner, name, torch.nn.Parameter(getattr(owner, name).detach().to(t)))
+    x = torch.randn(2, 140, cfg.hidden_size, generator=torch.Generator().manual_seed(5)).to(dtype).to(DEV)
+
+    def passes():
+        mixer.zero_grad()
+        out = mixer(x)
+        out.float().pow(2).sum().backward()
+        return out.detach(), {k: p.grad.clone() for k, p in mixer.named_parameters()}
+
+    got = passes()
+    _hook(mixer.in_proj, [])          # the same layer, module by module
+    want = passes()
+    bar = 1e-2 if dtype == torch.bfloat16 else 2e-3          # fp16 gradients of the small parameters: 2^-11 each
+    assert _rel(got[0], want[0]) < bar
+    for k, p in mixer.named_parameters():
+        assert got[1][k].dtype == p.dtype and _rel(got[1][k], want[1][k]) < bar, k
