@@ -150,6 +150,9 @@ typedef struct m2_ssd_params {
 size_t m2_ssd_chunk_states_bytes(const m2_ssd_params* p);
 size_t m2_ssd_fwd_workspace_bytes(const m2_ssd_params* p);
 int m2_ssd_fwd(const m2_ssd_params* p, void* stream);
+/* what m2_ssd_fwd would refuse, without the work: a caller that launches something else first (the conv, into its own decode
+ * cache) asks before it does */
+int m2_ssd_fwd_check(const m2_ssd_params* p);
 size_t m2_ssd_bwd_workspace_bytes(const m2_ssd_params* p);
 int m2_ssd_bwd(const m2_ssd_params* p, void* stream);
 
@@ -229,6 +232,7 @@ typedef struct m2_rmsnorm_params {
 } m2_rmsnorm_params;
 
 int m2_rmsnorm_gated_fwd(const m2_rmsnorm_params* p, void* stream);
+int m2_rmsnorm_gated_fwd_check(const m2_rmsnorm_params* p);      /* what it would refuse, without the work */
 size_t m2_rmsnorm_gated_bwd_workspace_bytes(int64_t rows, int64_t channels, int32_t n_groups, int32_t dtype);
 int m2_rmsnorm_gated_bwd(const m2_rmsnorm_params* p, void* stream);
 

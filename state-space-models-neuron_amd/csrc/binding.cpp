@@ -29,8 +29,8 @@ using torch::autograd::variable_list;
 // ----------------------------------------------------------------------------------------------- the library
 #define M2_BOUND(F) \
     F(m2_last_error) F(m2_conv1d_fwd) F(m2_conv1d_prefill) F(m2_conv1d_bwd_workspace_bytes) F(m2_conv1d_bwd) F(m2_ssd_chunk_states_bytes) \
-    F(m2_ssd_fwd_workspace_bytes) F(m2_ssd_fwd) F(m2_ssd_bwd_workspace_bytes) F(m2_ssd_bwd) F(m2_decode_workspace_bytes) \
-    F(m2_decode_step) F(m2_decode_step_static) F(m2_rmsnorm_gated_fwd) F(m2_rmsnorm_gated_bwd_workspace_bytes) \
+    F(m2_ssd_fwd_workspace_bytes) F(m2_ssd_fwd_check) F(m2_ssd_fwd) F(m2_ssd_bwd_workspace_bytes) F(m2_ssd_bwd) F(m2_decode_workspace_bytes) \
+    F(m2_decode_step) F(m2_decode_step_static) F(m2_rmsnorm_gated_fwd_check) F(m2_rmsnorm_gated_fwd) F(m2_rmsnorm_gated_bwd_workspace_bytes) \
     F(m2_rmsnorm_gated_bwd) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_rows) F(m2_decode_layer) F(m2_mixer_params) F(m2_mixer_params_grads) \
     F(m2_product_pays) F(m2_product_workspace_bytes) F(m2_product)
 struct Lib {
@@ -390,17 +390,28 @@ void check_norm(const Tensor& x, const Tensor& z) {
     TORCH_CHECK_VALUE(!z.defined() || (z.sizes() == x.sizes() && z.scalar_type() == x.scalar_type()), "rmsnorm_gated: z must have the shape and dtype of x");
 }
 
-Tensor rmsnorm_forward(const Tensor& x_, const OptTensor& z_, const Tensor& weight, int64_t n_groups, double eps, at::ScalarType out_dtype) {
-    require_gpu({&x_, &or_none(z_), &weight});
-    check_norm(x_, or_none(z_));
-    TORCH_CHECK_VALUE(out_dtype == at::kFloat || out_dtype == x_.scalar_type(), "rmsnorm_gated: out_dtype must be float32 or the dtype of x");
-    Scope scope(x_);
-    const Tensor x = aligned(x_), z = z_ ? aligned(*z_) : Tensor(), w32 = f32(weight);
-    m2_rmsnorm_params p = norm_params(x, z, w32, n_groups, eps);
-    Tensor out = at::empty(x.sizes(), x.options().dtype(out_dtype));
-    p.out = ptr(out); p.out_stride_row = x.size(-1); p.out_f32 = out_dtype == at::kFloat;
-    check(lib.m2_rmsnorm_gated_fwd(&p, scope.stream), "m2_rmsnorm_gated_fwd");
-    return out;
+// A norm that is ready to run: its operands (rows that the kernel does not read where they lie copied) and its output.
+struct NormCall {
+    Tensor x, z, w32, out;
+    m2_rmsnorm_params p;
+    NormCall(const Tensor& x_, const OptTensor& z_, const Tensor& weight, int64_t n_groups, double eps, at::ScalarType out_dtype) {
+        require_gpu({&x_, &or_none(z_), &weight});
+        check_norm(x_, or_none(z_));
+        TORCH_CHECK_VALUE(out_dtype == at::kFloat || out_dtype == x_.scalar_type(), "rmsnorm_gated: out_dtype must be float32 or the dtype of x");
+        x = aligned(x_); z = z_ ? aligned(*z_) : Tensor(); w32 = f32(weight);
+        p = norm_params(x, z, w32, n_groups, eps);
+        out = at::empty(x.sizes(), x.options().dtype(out_dtype));
+        p.out = ptr(out); p.out_stride_row = x.size(-1); p.out_f32 = out_dtype == at::kFloat;
+    }
+    void run(void* stream) { check(lib.m2_rmsnorm_gated_fwd(&p, stream), "m2_rmsnorm_gated_fwd"); }
+};
+
+Tensor rmsnorm_forward(const Tensor& x, const OptTensor& z, const Tensor& weight, int64_t n_groups, double eps, at::ScalarType out_dtype) {
+    require_gpu({&x});
+    Scope scope(x);
+    NormCall norm(x, z, weight, n_groups, eps, out_dtype);
+    norm.run(scope.stream);
+    return norm.out;
 }
 
 std::tuple<Tensor, Tensor, Tensor> rmsnorm_backward(const Tensor& x_, const OptTensor& z_, const Tensor& weight, const Tensor& d_out, int64_t n_groups,
@@ -775,16 +786,25 @@ Tensor fused_prefill(const Tensor& zx, const Tensor& A, const OptTensor& D, cons
     const Tensor conv_out = at::empty({k.b, k.l, k.conv}, zx.options());
     m2_conv1d_params c = conv_params(k.xBC(), w, bi, {ptr(conv_out), k.l * k.conv, k.conv, 1}, k.b, k.l, k.conv, dtype_code(k.zx), M2_ACT_SILU);
     c.y = ptr(conv_out);
-    check(lib.m2_conv1d_prefill(&c, ptr(cs), static_cast<int32_t>(cs.size(2)), continuing, scope.stream), "m2_conv1d_prefill");
+    // The conv moves the cache on, so everything behind it is allocated and checked first: a call that is refused leaves the cache
+    // as it was.
     const Tensor A32 = f32(A), D32 = f32(or_none(D)), bias = f32(dt_bias);
     m2_ssd_params p = core_ssd_params(k, conv_out, A32, D32, bias);
     const Tensor y = at::empty({k.b, k.l, d}, zx.options());
     p.initial_state = continuing ? ptr<float>(S) : nullptr; p.final_state = ptr<float>(S);
     p.y = ptr(y); p.y_stride_b = k.l * d; p.y_stride_l = d; p.y_stride_h = hd;
-    launch_ssd_fwd(p, zx, scope.stream);
+    p.workspace_bytes = lib.m2_ssd_fwd_workspace_bytes(&p);
+    const Tensor ws = scratch(p.workspace_bytes, zx);
+    p.workspace = ptr(ws);
+    check(lib.m2_ssd_fwd_check(&p), "m2_ssd_fwd");
+    NormCall norm(y, k.z(), norm_w, g, kNormEps, zx.scalar_type());
+    check(lib.m2_rmsnorm_gated_fwd_check(&norm.p), "m2_rmsnorm_gated_fwd");
+    check(lib.m2_conv1d_prefill(&c, ptr(cs), static_cast<int32_t>(cs.size(2)), continuing, scope.stream), "m2_conv1d_prefill");
+    check(lib.m2_ssd_fwd(&p, scope.stream), "m2_ssd_fwd");
     if (!own_conv) conv_state.copy_(cs);
     if (!own_ssm) ssm_state.copy_(S);
-    return rmsnorm_forward(y, k.z(), norm_w, g, kNormEps, zx.scalar_type());
+    norm.run(scope.stream);
+    return norm.out;
 }
 
 // ----------------------------------------------------------------------------------------------- decode step

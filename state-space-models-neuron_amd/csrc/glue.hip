@@ -539,16 +539,26 @@ extern "C" int m2_softplus_bias_bwd(const void* dt, int64_t dt_stride_row, const
     return launch_column_sum(static_cast<const float*>(workspace), d_bias, nblk, nheads, st);
 }
 
-extern "C" int m2_rmsnorm_gated_fwd(const m2_rmsnorm_params* p, void* stream) {
+extern "C" int m2_rmsnorm_gated_fwd_check(const m2_rmsnorm_params* p) {
     using namespace m2;
-    int rc = check_norm_common(p, "rmsnorm_gated_fwd");
-    if (rc) return rc;
-    if (p->rows == 0) return M2_OK;
+    const int rc = check_norm_common(p, "rmsnorm_gated_fwd");
+    if (rc || p->rows == 0) return rc;
     M2_REQUIRE(p->x && p->weight && p->out, M2_ERR_NULL, "rmsnorm_gated_fwd: x, weight and out are required");
     const int V = p->dtype == M2_F32 ? 4 : 8;
     M2_REQUIRE(aligned16(p->x) && aligned16(p->out) && (!p->z || aligned16(p->z)) && p->x_stride_row % V == 0 && p->out_stride_row % 4 == 0 &&
                    (p->out_f32 || p->out_stride_row % V == 0) && (!p->z || p->z_stride_row % V == 0),
                M2_ERR_ALIGN, "rmsnorm_gated_fwd: pointers must be 16-byte aligned and row strides multiples of %d elements", V);
+    int wpg = 0, nv = 0;
+    const int64_t gw = p->channels / p->n_groups;
+    M2_REQUIRE(norm_shape(gw / V, V, &wpg, &nv), M2_ERR_SHAPE, "rmsnorm_gated: %lld channels per group exceed the supported 8192", (long long)gw);
+    return M2_OK;
+}
+
+extern "C" int m2_rmsnorm_gated_fwd(const m2_rmsnorm_params* p, void* stream) {
+    using namespace m2;
+    const int rc = m2_rmsnorm_gated_fwd_check(p);
+    if (rc || p->rows == 0) return rc;
+    const int V = p->dtype == M2_F32 ? 4 : 8;
     NormArgs a{};
     a.x = p->x; a.x_sr = p->x_stride_row; a.z = p->z; a.z_sr = p->z_stride_row; a.w = p->weight;
     a.out = p->out; a.out_sr = p->out_stride_row; a.out_f32 = p->out_f32 || p->dtype == M2_F32;

@@ -71,9 +71,27 @@ extern "C" size_t m2_ssd_fwd_workspace_bytes(const m2_ssd_params* p) {
     return m2::ssd_carve(&q, nullptr, false).bytes;
 }
 
+extern "C" int m2_ssd_fwd_check(const m2_ssd_params* p) {
+    using namespace m2;
+    const int rc = ssd_check(p, "ssd_fwd");
+    if (rc) return rc;
+    if (p->batch == 0 || p->nheads == 0 || p->seqlen == 0) return M2_OK;
+    M2_REQUIRE(p->x && p->dt && p->A && p->B && p->C && p->y, M2_ERR_NULL, "ssd_fwd: x, dt, A, B, C, y are required");
+    {
+        const int V = p->dtype == M2_F32 ? 4 : 8;
+        M2_REQUIRE(aligned16(p->y) && p->y_stride_b % V == 0 && p->y_stride_l % V == 0 && p->y_stride_h % V == 0, M2_ERR_ALIGN,
+                   "ssd_fwd: y and its strides must be 16-byte aligned (multiples of %d elements)", V);
+    }
+    const size_t need = m2_ssd_fwd_workspace_bytes(p);
+    M2_REQUIRE(p->workspace && p->workspace_bytes >= need, M2_ERR_WORKSPACE, "ssd_fwd: workspace %zu bytes < %zu needed",
+               p->workspace_bytes, need);
+    M2_REQUIRE((reinterpret_cast<uintptr_t>(p->workspace) & 255u) == 0, M2_ERR_ALIGN, "ssd_fwd: workspace must be 256-byte aligned");
+    return M2_OK;
+}
+
 extern "C" int m2_ssd_fwd(const m2_ssd_params* p, void* stream) {
     using namespace m2;
-    int rc = ssd_check(p, "ssd_fwd");
+    const int rc = m2_ssd_fwd_check(p);
     if (rc) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (p->batch == 0 || p->nheads == 0) return M2_OK;
@@ -85,16 +103,6 @@ extern "C" int m2_ssd_fwd(const m2_ssd_params* p, void* stream) {
         }
         return M2_OK;
     }
-    M2_REQUIRE(p->x && p->dt && p->A && p->B && p->C && p->y, M2_ERR_NULL, "ssd_fwd: x, dt, A, B, C, y are required");
-    {
-        const int V = p->dtype == M2_F32 ? 4 : 8;
-        M2_REQUIRE(aligned16(p->y) && p->y_stride_b % V == 0 && p->y_stride_l % V == 0 && p->y_stride_h % V == 0, M2_ERR_ALIGN,
-                   "ssd_fwd: y and its strides must be 16-byte aligned (multiples of %d elements)", V);
-    }
-    const size_t need = m2_ssd_fwd_workspace_bytes(p);
-    M2_REQUIRE(p->workspace && p->workspace_bytes >= need, M2_ERR_WORKSPACE, "ssd_fwd: workspace %zu bytes < %zu needed",
-               p->workspace_bytes, need);
-    M2_REQUIRE((reinterpret_cast<uintptr_t>(p->workspace) & 255u) == 0, M2_ERR_ALIGN, "ssd_fwd: workspace must be 256-byte aligned");
     const SsdCall q(p);
     M2_DISPATCH_DTYPE(p->dtype, T, M2_DISPATCH_N_HS(&q, N, HS, return (ssd_fwd_impl<T, kP, N, HS>(&q, st))));
     return M2_OK;

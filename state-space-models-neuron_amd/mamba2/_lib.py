@@ -93,6 +93,7 @@ SYMBOLS = {
     "m2_ssd_chunk_states_bytes": (_sz, [C.POINTER(SsdParams)]),
     "m2_ssd_fwd_workspace_bytes": (_sz, [C.POINTER(SsdParams)]),
     "m2_ssd_fwd": (C.c_int, [C.POINTER(SsdParams), _vp]),
+    "m2_ssd_fwd_check": (C.c_int, [C.POINTER(SsdParams)]),
     "m2_ssd_bwd_workspace_bytes": (_sz, [C.POINTER(SsdParams)]),
     "m2_ssd_bwd": (C.c_int, [C.POINTER(SsdParams), _vp]),
     "m2_decode_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
@@ -102,6 +103,7 @@ SYMBOLS = {
     "m2_softplus_bias_bwd_workspace_bytes": (_sz, [_i64, _i64]),
     "m2_softplus_bias_bwd": (C.c_int, [_vp, _i64, _vp, _vp, _i64, _vp, _i64, _vp, _vp, _sz, _i64, _i64, _i32, _vp]),
     "m2_rmsnorm_gated_fwd": (C.c_int, [C.POINTER(RmsnormParams), _vp]),
+    "m2_rmsnorm_gated_fwd_check": (C.c_int, [C.POINTER(RmsnormParams)]),
     "m2_rmsnorm_gated_bwd_workspace_bytes": (_sz, [_i64, _i64, _i32, _i32]),
     "m2_rmsnorm_gated_bwd": (C.c_int, [C.POINTER(RmsnormParams), _vp]),
     "m2_add_rmsnorm": (C.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, C.c_float, _i32, _vp]),

@@ -281,3 +281,20 @@ def test_layer_takes_small_parameters_of_any_type(types, dtype):
     assert _rel(got[0], want[0]) < bar
     for k, p in mixer.named_parameters():
         assert got[1][k].dtype == p.dtype and _rel(got[1][k], want[1][k]) < bar, k
+
+
+@pytest.mark.parametrize("continuing", [False, True])
+@pytest.mark.parametrize("h,head_dim,n,message", [(4, 32, 64, "headdim"), (4, 64, 32, "dstate"), (136, 64, 64, "8192")])
+def test_prefill_that_is_refused_leaves_the_cache(continuing, h, head_dim, n, message):
+    """Heads or states that the scan does not take, a group wider than the norm takes: neither state has moved."""
+    from mamba2.fused_kernel import mamba2_fused_prefill
+    d, g, b, l = h * head_dim, 1, 2, 40
+    cx = d + 2 * g * n
+    gen = torch.Generator(device=DEV).manual_seed(6)
+    rand = lambda *s: torch.randn(*s, device=DEV, generator=gen)
+    conv_state, ssm_state = rand(b, cx, 4).bfloat16(), rand(b, h, head_dim, n)
+    before = conv_state.clone(), ssm_state.clone()
+    with pytest.raises(ValueError, match=message):
+        mamba2_fused_prefill(rand(b, l, d + cx + h).bfloat16(), -torch.ones(h, device=DEV), torch.ones(h, device=DEV), rand(cx, 1, 4).bfloat16(),
+                             rand(cx).bfloat16(), rand(h), torch.ones(d, device=DEV), g, n, d, head_dim, conv_state, ssm_state, continuing=continuing)
+    assert torch.equal(conv_state, before[0]) and torch.equal(ssm_state, before[1])
