@@ -45,9 +45,11 @@ struct LinearArgs {
     bf16_t* conv_state; const bf16_t* conv_in; int64_t conv_in_sb; int conv_c0, conv_cx, conv_W;
 };
 
+// Every LDS read that this wave has issued has returned its data.
+__device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 // Barrier for LDS traffic alone: the copies in flight stay in flight.
 __device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    lds_reads_done();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
@@ -133,8 +135,13 @@ linear_small_kernel(const LinearArgs a) {
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
         for (int s = 0; s < mine; ++s, ++done) {
-            // the slot that is filled now was read in the step before, whose products have its values
-            if (done + D - 1 < total) issue();
+            // The slot that is filled now was read in the step before.  Those reads have to have returned before a copy is issued on
+            // top of them: nothing orders an LDS read against the LDS write of a copy but this wait (the step's products wait for
+            // most of them anyway; asked for here, it holds however the compiler schedules them).
+            if (done + D - 1 < total) {
+                lds_reads_done();
+                issue();
+            }
             wait_vmem_keep<PER>(total - 1 - done < D - 1 ? total - 1 - done : D - 1);
             const char* base = ring + slot * SLOT;
             slot = slot + 1 == D ? 0 : slot + 1;
