@@ -60,8 +60,9 @@ extern "C" {
 int m2_abi_version(void);
 const char* m2_last_error(void);
 /* Layout of a parameter structure as THIS library was compiled: out[0] = sizeof, out[1..] = offsetof each field in
- * declaration order.  which: 0 m2_conv1d_params, 1 m2_ssd_params, 2 m2_decode_params, 3 m2_rmsnorm_params.  Returns the
- * number of entries (only the first `capacity` are written); a binding compares them with its own mirror of the structs. */
+ * declaration order.  which: 0 m2_conv1d_params, 1 m2_ssd_params, 2 m2_decode_params, 3 m2_rmsnorm_params,
+ * 4 m2_linear_params, 5 m2_product_params.  Returns the number of entries (only the first `capacity` are written); a
+ * binding compares them with its own mirror of the structs. */
 int m2_struct_layout(int32_t which, int64_t* out, int32_t capacity);
 
 /* ------------------------------------------------------------------ conv1d

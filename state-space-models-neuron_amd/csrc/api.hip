@@ -164,6 +164,17 @@ static const int64_t k_layout_3[] = {(int64_t)sizeof(m2_rmsnorm_params),
     M2_OFF(m2_rmsnorm_params, d_out_stride_row), M2_OFF(m2_rmsnorm_params, dx_stride_row),
     M2_OFF(m2_rmsnorm_params, dz_stride_row), M2_OFF(m2_rmsnorm_params, n_groups), M2_OFF(m2_rmsnorm_params, dtype),
     M2_OFF(m2_rmsnorm_params, out_f32), M2_OFF(m2_rmsnorm_params, eps),};
+static const int64_t k_layout_4[] = {(int64_t)sizeof(m2_linear_params),
+    M2_OFF(m2_linear_params, x), M2_OFF(m2_linear_params, w), M2_OFF(m2_linear_params, bias), M2_OFF(m2_linear_params, sq),
+    M2_OFF(m2_linear_params, out), M2_OFF(m2_linear_params, next_weight), M2_OFF(m2_linear_params, next_x),
+    M2_OFF(m2_linear_params, next_sq), M2_OFF(m2_linear_params, M), M2_OFF(m2_linear_params, N), M2_OFF(m2_linear_params, K),
+    M2_OFF(m2_linear_params, nsq), M2_OFF(m2_linear_params, x_stride_row), M2_OFF(m2_linear_params, out_stride_row),
+    M2_OFF(m2_linear_params, out_kind), M2_OFF(m2_linear_params, groups), M2_OFF(m2_linear_params, eps),};
+static const int64_t k_layout_5[] = {(int64_t)sizeof(m2_product_params),
+    M2_OFF(m2_product_params, a), M2_OFF(m2_product_params, b), M2_OFF(m2_product_params, bias), M2_OFF(m2_product_params, out),
+    M2_OFF(m2_product_params, workspace), M2_OFF(m2_product_params, workspace_bytes), M2_OFF(m2_product_params, M),
+    M2_OFF(m2_product_params, N), M2_OFF(m2_product_params, K), M2_OFF(m2_product_params, lda), M2_OFF(m2_product_params, ldb),
+    M2_OFF(m2_product_params, ldo), M2_OFF(m2_product_params, a_k), M2_OFF(m2_product_params, b_k),};
 #undef M2_OFF
 
 }  // namespace
@@ -180,6 +191,8 @@ extern "C" int m2_struct_layout(int32_t which, int64_t* out, int32_t capacity) {
         case 1: tab = k_layout_1; n = (int)(sizeof(k_layout_1) / sizeof(int64_t)); break;
         case 2: tab = k_layout_2; n = (int)(sizeof(k_layout_2) / sizeof(int64_t)); break;
         case 3: tab = k_layout_3; n = (int)(sizeof(k_layout_3) / sizeof(int64_t)); break;
+        case 4: tab = k_layout_4; n = (int)(sizeof(k_layout_4) / sizeof(int64_t)); break;
+        case 5: tab = k_layout_5; n = (int)(sizeof(k_layout_5) / sizeof(int64_t)); break;
         default: return fail(M2_ERR_SHAPE, "struct_layout: unknown structure %d", (int)which);
     }
     for (int i = 0; i < n && i < capacity; ++i) out[i] = tab[i];

@@ -47,3 +47,25 @@ def test_small_products_refuse_what_their_addressing_does_not_reach(lib):
     assert lib.m2_linear_small(ctypes.byref(p), None) == -1 and b"32-bit" in lib.m2_last_error()
     p.x_stride_row, p.w = 64, 24
     assert lib.m2_linear_small(ctypes.byref(p), None) == -3
+
+
+def test_every_struct_of_the_header_is_mirrored_and_reported(lib):
+    """Each parameter struct that the header declares: its fields in the ctypes mirror, its size and offsets as the library was built."""
+    import os
+    import re
+
+    from mamba2 import _lib
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(root, "include", "mamba2_hip.h")).read(), flags=re.S)
+    declared = re.findall(r"typedef struct (m2_\w+) \{(.*?)\} \1;", text, flags=re.S)
+    mirrors = {"m2_conv1d_params": _lib.Conv1dParams, "m2_ssd_params": _lib.SsdParams, "m2_decode_params": _lib.DecodeParams,
+               "m2_rmsnorm_params": _lib.RmsnormParams, "m2_linear_params": _lib.LinearParams, "m2_product_params": _lib.ProductParams}
+    assert [name for name, _ in declared] == list(mirrors)
+    for which, (name, body) in enumerate(declared):
+        fields = [re.split(r"[\s*]+", f.strip())[-1] for decl in body.split(";") if decl.strip() for f in decl.split(",")]
+        mirror = mirrors[name]
+        assert fields == [f[0] for f in mirror._fields_], name
+        buf = (ctypes.c_int64 * 128)()
+        assert lib.m2_struct_layout(which, buf, 128) == 1 + len(fields), name
+        assert buf[0] == ctypes.sizeof(mirror) and list(buf[1:1 + len(fields)]) == [getattr(mirror, f).offset for f in fields], name
+    assert lib.m2_struct_layout(len(declared), (ctypes.c_int64 * 4)(), 4) == -1
