@@ -7,15 +7,21 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (8, 8, 1), (64, 64, 64), (65, 72, 72), (72, 200, 1000), (40, 64, 5), (200, 2560, 520), (136, 264, 2056), (1000, 1544, 136)])
-@pytest.mark.parametrize("a_k,b_k", [(1, 1), (1, 0), (0, 0), (0, 1)])
+def _taken(M, K, a_k, b_k):
+    """What the storage asks for: the contiguous extent of each operand (k, or the rows of a transposed A) in eights."""
+    return not ((a_k or b_k) and K % 8) and (a_k or not M % 8)
+
+
+SIZES = [(1, 8, 8), (8, 8, 1), (64, 64, 64), (65, 72, 72), (72, 200, 1000), (40, 64, 5), (200, 2560, 520), (136, 264, 2056), (1000, 1544, 136)]
+FORMS = [(*s, *f) for s in SIZES for f in ((1, 1), (1, 0), (0, 0), (0, 1))]
+
+
+@pytest.mark.parametrize("M,N,K,a_k,b_k", [f for f in FORMS if _taken(f[0], f[2], f[3], f[4])])
 @pytest.mark.parametrize("pad", [0, 8])
 def test_product(M, N, K, a_k, b_k, pad):
     from mamba2 import _lib
     lib = _lib.load()
-    if not lib.m2_product_fits(M, N, K, a_k, b_k):
-        assert (a_k or b_k) and K % 8 or not a_k and M % 8
-        return
+    assert lib.m2_product_fits(M, N, K, a_k, b_k)
     gen = torch.Generator().manual_seed(M + N + K)
     a, b = (torch.randn(r, K, generator=gen).bfloat16() for r in (M, N))
     bias = torch.randn(N, generator=gen).bfloat16()
@@ -37,3 +43,14 @@ def test_product(M, N, K, a_k, b_k, pad):
     got = out.double().cpu()
     assert ((got[:, :N] - ref).norm() / ref.norm()).item() < 4e-3
     assert (got[:, N:] == 7.0).all()
+
+
+@pytest.mark.parametrize("M,N,K,a_k,b_k", [f for f in FORMS if not _taken(f[0], f[2], f[3], f[4])] + [(64, 12, 64, 1, 1), (0, 64, 64, 1, 1)])
+def test_product_refuses_other_storage(M, N, K, a_k, b_k):
+    from mamba2 import _lib
+    lib = _lib.load()
+    assert not lib.m2_product_fits(M, N, K, a_k, b_k)
+    t = torch.zeros(1 << 14, dtype=torch.bfloat16, device=DEV)          # refused before any of it is read
+    p = _lib.ProductParams(a=_lib.ptr(t), b=_lib.ptr(t), out=_lib.ptr(t), M=M, N=N, K=K, lda=8, ldb=8, ldo=8, a_k=a_k, b_k=b_k)
+    with pytest.raises(ValueError, match="is not taken"):
+        _lib.check(lib.m2_product(p, _lib.stream_ptr()), "m2_product")
