@@ -28,12 +28,11 @@
 // Launch sequence (16-bit operands; fp32 operands take the kernels named in brackets):
 //   prep_kernel, state_pass16_kernel [chunk_state + state_scan]   recompute G, tables, S_prev (skipped if the caller kept them)
 //   state_pass16_kernel<REVERSE> [chunk_state<DSTATE> + state_scan<REVERSE>]
-//                                                              dS per chunk, d initial state (and e^{Lam} <dS, S_prev> when
-//                                                              ssd_bwd16_kernel does not run)
+//                                                              dS per chunk, d initial state [, e^{Lam} <dS, S_prev>]
 //   dg16_kernel [dg_kernel]   per (b, chunk, group, head slice)  partial dG (heads reduced in registers), dl_diag per head
 //   ssd_bwd16_kernel [off_kernel<C>, <B>, diag_off_kernel<bwd>]
-//                             per (b, chunk, group, head slice)  dx, per-token decay-gradient terms, e^{Lam} <dS, S_prev>,
-//                                                                dD partials, partial state parts of dB / dC
+//                             per (b, chunk, group, head slice)  dx, per-token decay-gradient terms, dD partials, partial state parts
+//                                                                of dB / dC, and with 16-bit operands e^{Lam} <dS, S_prev>
 //   tail1_kernel              da_body: ddt, dA partials per (b, head, chunk);  slice_sum_body: partials over the head slices
 //   tail2_kernel              bc_final16_body [bc_final_body] per (b, chunk, group): dC = dG B + dCoff, dB = dG^T C + dBoff;
 //                             ad_reduce_body per head: dA, dD (fixed order, no atomics)
@@ -43,21 +42,19 @@ namespace m2 {
 namespace {
 
 // ------------------------------------------------------------------------------------------
-// dG partial and the diagonal part of the decay gradient.
+// dG partial and the diagonal part of the decay gradient, fp32 operands (16-bit ones: dg16_kernel).
 // grid (nchunks, ngroups * nslices, batch), 512 threads (8 waves).  Wave w owns the 32x32 blocks of the
 // [kQ][kQ] tile with block-row rb = w >> 1 and block-columns cb0 = 2 (w & 1), cb0 + 1.
 //   per head:  P = dY X^T  (MFMA, K = headdim);   dG^h[i][j] = e^{l_i - l_j} dt_j P[i][j]   (i >= j)
 //              dG += dG^h;    pr = dG^h o G;   dl_diag[i] = sum_j pr[i][j] - sum_i' pr[i'][i]
 // Row and column sums come from the same fp32 products, so pairs inside a suffix cancel exactly.
-template <typename T, int P>
-constexpr bool dg_g_in_lds() { return (size_t)14 * kQ * sizeof(float) + ((size_t)2 * kQ * lds_ld<T>(P) + (size_t)kQ * lds_ld<T>(kQ)) * sizeof(T) <= 150 * 1024; }
-
 template <typename T, int P, int HS>
 __global__ void __launch_bounds__(512, 2)
 dg_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
           const T* __restrict__ dY, const T* __restrict__ Gm, float* __restrict__ dGp, float* __restrict__ dl_diag,
           int64_t seqlen, int64_t nheads, int64_t ngroups, int64_t nchunks, int64_t nslices, int64_t hps,
           int64_t Xsb, int64_t Xsl, int64_t Xsh, int64_t dYsb, int64_t dYsl, int64_t dYsh) {
+    static_assert(sizeof(T) == 4, "16-bit operands take dg16_kernel");
     constexpr int LDP = lds_ld<T>(P);
     constexpr int LDQ = lds_ld<T>(kQ);
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -80,9 +77,7 @@ dg_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
     float* wl = wtab + wave * kQ;
 
     // causal-masked G of this (chunk, group), shared by all heads: staged once
-    constexpr bool G_LDS = dg_g_in_lds<T, P>();
-    const T* Gg = Gm + ((b * nchunks + c) * ngroups + g) * (int64_t)(kQ * kQ);
-    if (G_LDS) stage_rows<T, kQ, kQ, 512, false>(sG, LDQ, Gg, kQ, kQ, nullptr, tid);
+    stage_rows<T, kQ, kQ, 512, false>(sG, LDQ, Gm + ((b * nchunks + c) * ngroups + g) * (int64_t)(kQ * kQ), kQ, kQ, nullptr, tid);
     floatx16 dG[1][2];
     acc_zero(dG);
 
@@ -152,7 +147,7 @@ dg_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
                     else w = __expf(fminf(wl[i] - lj[jb], 0.f)) * dtj[jb];
                     const float dgh = (i >= j) ? w * pa[0][0][v] : 0.f;
                     dG[0][jb][v] += dgh;
-                    const float pr = dgh * to_f32(G_LDS ? sG[i * LDQ + j] : Gg[i * kQ + j]);
+                    const float pr = dgh * to_f32(sG[i * LDQ + j]);
                     rsum[v] += pr;
                     csum[jb] += pr;
                 }
@@ -185,15 +180,12 @@ dg_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
 }
 
 // ------------------------------------------------------------------------------------------
-// Off-diagonal (state) parts of dC and dB, heads of a slice reduced in registers.
+// Off-diagonal (state) parts of dC and dB, heads of a slice reduced in registers, fp32 operands (16-bit ones: ssd_bwd16_kernel).
 // grid (nchunks, ngroups * nslices, batch), 512 threads.  Wave w owns rows rb = w >> 1 and state-column blocks
 // nb0 = (w & 1) * NB .. + NB - 1 of the [kQ][N] tile.
 //   SIDE_C:  dC[i][n] += e^{l_i} sum_p dy[i][p] S_prev[p][n];   dl_c[i] = C_i . (that head's contribution)
 //   SIDE_B:  dB[j][n] += dt_j e^{Lam - l_j} sum_p x[j][p] dS[p][n]
 // The row scale is applied in fp32 after the MFMA, so both operands are exact copies of the inputs.
-template <typename T, int P, int N>
-constexpr bool off_c_in_lds() { return (size_t)10 * kQ * sizeof(float) + ((size_t)(kQ + N) * lds_ld<T>(P) + (size_t)kQ * lds_ld<T>(N)) * sizeof(T) <= 150 * 1024; }
-
 template <typename T, int P, int N, bool SIDE_C, int HS>
 __global__ void __launch_bounds__(512, SIDE_C ? 2 : 4)
 off_kernel(const T* __restrict__ Arow, int64_t Asb, int64_t Asl, int64_t Ash,      // dY (C side) or X (B side)
@@ -202,6 +194,7 @@ off_kernel(const T* __restrict__ Arow, int64_t Asb, int64_t Asl, int64_t Ash,   
            const T* __restrict__ Cm, int64_t Csb, int64_t Csl, int64_t Csg,        // C side only
            float* __restrict__ outp, float* __restrict__ dl_c,
            int64_t seqlen, int64_t nheads, int64_t ngroups, int64_t nchunks, int64_t nslices, int64_t hps) {
+    static_assert(sizeof(T) == 4, "16-bit operands take ssd_bwd16_kernel");
     constexpr int LDP = lds_ld<T>(P);
     constexpr int NB = N / 64;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -222,9 +215,7 @@ off_kernel(const T* __restrict__ Arow, int64_t Asb, int64_t Asl, int64_t Ash,   
 
     constexpr int LDN = lds_ld<T>(N);
     T* sC = sT + N * LDP;                                  // C side: C [kQ][LDN], staged once for all heads
-    constexpr bool C_LDS = off_c_in_lds<T, P, N>();
-    const T* Cgl = SIDE_C ? Cm + b * Csb + t0 * Csl + g * Csg : nullptr;
-    if (SIDE_C && C_LDS) stage_rows<T, kQ, N, 512, false>(sC, LDN, Cgl, Csl, valid, nullptr, tid);
+    if (SIDE_C) stage_rows<T, kQ, N, 512, false>(sC, LDN, Cm + b * Csb + t0 * Csl + g * Csg, Csl, valid, nullptr, tid);
     floatx16 acc[1][NB];
     acc_zero(acc);
 
@@ -291,8 +282,7 @@ off_kernel(const T* __restrict__ Arow, int64_t Asb, int64_t Asl, int64_t Ash,   
                 acc[0][jn][v] += t;
                 if (SIDE_C) {
                     const int i = rb * 32 + acc_row(lane, v), n = (nb0 + jn) * 32 + r;
-                    const T cval = C_LDS ? sC[i * LDN + n] : (i < valid ? Cgl[(int64_t)i * Csl + n] : (T)0.f);
-                    rcv[v] += t * to_f32(cval);
+                    rcv[v] += t * to_f32(sC[i * LDN + n]);
                 }
             }
         }
@@ -589,9 +579,9 @@ __global__ void copy_f32_kernel(const float* __restrict__ src, float* __restrict
 }
 
 template <typename T, int P>
-size_t dg_smem() { return (size_t)(8 * kQ + 2 * kQ + 4 * kQ) * sizeof(float) + ((size_t)2 * kQ * lds_ld<T>(P) + (dg_g_in_lds<T, P>() ? (size_t)kQ * lds_ld<T>(kQ) : 0)) * sizeof(T); }
+size_t dg_smem() { return (size_t)(8 * kQ + 2 * kQ + 4 * kQ) * sizeof(float) + ((size_t)2 * kQ * lds_ld<T>(P) + (size_t)kQ * lds_ld<T>(kQ)) * sizeof(T); }
 template <typename T, int P, int N>
-size_t off_smem(bool side_c) { return (size_t)(8 * kQ + 2 * kQ) * sizeof(float) + ((size_t)(kQ + N) * lds_ld<T>(P) + ((side_c && off_c_in_lds<T, P, N>()) ? (size_t)kQ * lds_ld<T>(N) : 0)) * sizeof(T); }
+size_t off_smem(bool side_c) { return (size_t)(8 * kQ + 2 * kQ) * sizeof(float) + ((size_t)(kQ + N) * lds_ld<T>(P) + (side_c ? (size_t)kQ * lds_ld<T>(N) : 0)) * sizeof(T); }
 template <typename T, int N>
 size_t bcf_smem() { return sizeof(T) == 2 ? (size_t)2 * kQ * kQ * sizeof(T) : (size_t)(kQ + N) * lds_ld<T>(kQ) * sizeof(T); }
 

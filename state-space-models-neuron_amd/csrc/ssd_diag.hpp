@@ -1,11 +1,12 @@
-// The two "diagonal + off-diagonal" SSD kernels (forward output, backward dx/ddt) share one structure.
+// The two "diagonal + off-diagonal" SSD kernels for fp32 operands (forward: y; backward: dx, and the per-token and per-chunk terms that
+// ddt, dA and dD are formed from afterwards) share one structure.  16-bit operands take ssd_y16_kernel and ssd_bwd16_kernel.
 //
 // Per (batch, chunk, head) the result is a [kQ tokens][P] tile
 //     OUT[r][p] = final_r * ( off_r * sum_n Aoff[r][n] * S[p][n]   +   sum_k (Gd[r][k] * tab_w[k]) * Z[k][p] )
 //   forward : Aoff = C,  S = state entering the chunk,  Gd = causal C B^T (rows i, k = j <= i),  Z = x
 //             y = OUT + D x
 //   backward: Aoff = B,  S = gradient of the state leaving the chunk,  Gd = (causal C B^T)^T (rows j, k = i >= j),
-//             Z = dy;    dxd = OUT,  dx = dt dxd + D dy,  ddt = A da + dxd . x
+//             Z = dy;    dxd = OUT,  dx = dt dxd + D dy;  per token dxd . x and its state part (dirp, rbp), per chunk dy . x (dDp8)
 //
 // A workgroup owns one chunk of one group and loops over `hps` heads of that group.  What does not depend on the
 // head -- the MFMA A-operand fragments of C (or B) and of the masked C B^T tile -- is loaded ONCE into registers;
@@ -46,24 +47,18 @@ struct DiagArgs {
     float* dDp8;                                    // [b][h][c][8]
 };
 
-// The backward keeps a transposed copy of x in LDS for its epilogue when that fits (always for bf16);
-// otherwise it reads x from global memory there.
-template <typename T, int P, int N>
-constexpr bool diag_xt_in_lds() {
-    return (size_t)(4 * 4 * kQ) * sizeof(float) + ((size_t)P * lds_ld<T>(N) + (size_t)2 * P * lds_ld<T>(kQ)) * sizeof(T) <= 150 * 1024;
-}
+// The backward keeps a transposed copy of x in LDS for its epilogue beside that of dy.
 template <typename T, int P, int N, bool BWD>
 constexpr size_t diag_smem() {
-    return (size_t)(4 * 4 * kQ) * sizeof(float) +
-           ((size_t)P * lds_ld<T>(N) + (size_t)((BWD && diag_xt_in_lds<T, P, N>()) ? 2 : 1) * P * lds_ld<T>(kQ)) * sizeof(T);
+    return (size_t)(4 * 4 * kQ) * sizeof(float) + ((size_t)P * lds_ld<T>(N) + (size_t)(BWD ? 2 : 1) * P * lds_ld<T>(kQ)) * sizeof(T);
 }
 
 template <typename T, int P, int N, bool BWD, int HS>
 __global__ void __launch_bounds__(256, 2)
 diag_off_kernel(const DiagArgs a) {
+    static_assert(sizeof(T) == 4, "16-bit operands take ssd_y16_kernel and ssd_bwd16_kernel");
     constexpr int LDN = lds_ld<T>(N), LDQ = lds_ld<T>(kQ);
     constexpr int BN = P / 32, KSN = N / 16;
-    constexpr bool XT = BWD && diag_xt_in_lds<T, P, N>();
     extern __shared__ __align__(16) unsigned char smem_raw[];
     float* wt_all = reinterpret_cast<float*>(smem_raw);              // [4 waves][4 tables][kQ]
     T* sS = reinterpret_cast<T*>(wt_all + 4 * 4 * kQ);               // [P][LDN]
@@ -137,21 +132,13 @@ diag_off_kernel(const DiagArgs a) {
         stage_rows<T, P, N, 256, false>(sS, LDN, static_cast<const T*>(a.S) + tile, N, P, nullptr, tid);
         stage_transposed<T, kQ, P, 256, false>(sZt, LDQ, static_cast<const T*>(a.Z) + b * a.Z_sb + t0 * a.Z_sl + head_off<HS>(h, a.Z_sh), a.Z_sl,
                                                valid, nullptr, tid);
-        if (XT)
+        if (BWD)
             stage_transposed<T, kQ, P, 256, false>(sXt, LDQ, static_cast<const T*>(a.X) + b * a.X_sb + t0 * a.X_sl + head_off<HS>(h, a.X_sh),
                                                    a.X_sl, valid, nullptr, tid);
         __syncthreads();
-        const T* Xg = BWD ? static_cast<const T*>(a.X) + b * a.X_sb + t0 * a.X_sl + head_off<HS>(h, a.X_sh) : nullptr;
         // x[row0 + 8q + 4 half + e][col], e = 0..3, at this lane's accumulator positions
         auto load_x4 = [&](int q, int col, T (&xv)[4]) {
-            if (XT) *reinterpret_cast<RawVec<T, 4>*>(xv) = *reinterpret_cast<const RawVec<T, 4>*>(sXt + col * LDQ + row0 + 8 * q + 4 * half);
-            else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int row = row0 + 8 * q + 4 * half + e;
-                    xv[e] = row < valid ? Xg[(int64_t)row * a.X_sl + col] : (T)0.f;
-                }
-            }
+            *reinterpret_cast<RawVec<T, 4>*>(xv) = *reinterpret_cast<const RawVec<T, 4>*>(sXt + col * LDQ + row0 + 8 * q + 4 * half);
         };
 
         // per-row scales: off-diagonal prescale and final row scale (recomputed where used to keep registers free)

@@ -12,7 +12,7 @@
 // Kernels here (all launched with the chunk index in blockIdx.x so consecutive workgroups,
 // which the hardware deals round-robin to the 8 XCDs, still share B/C/G tiles of one batch
 // row through the MALL, and each XCD's L2 sees whole (head, chunk) tiles):
-//   cb_kernel          G = C B^T per (batch, chunk, group)          -> workspace, fp32
+//   prep_kernel        decay tables per (batch, head, chunk); G = C B^T and the operand tiles per (batch, chunk, group)
 //   chunk_state_kernel local chunk state  sum_j scale_j x_j (x) B_j -> workspace, fp32
 //                      (DSTATE variant: sum_i e^{l_i} dy_i (x) C_i for the backward)
 //   state_scan_kernel  sequential-in-chunks, parallel-in-(b,h,p,n) fp32 recurrence; writes the
