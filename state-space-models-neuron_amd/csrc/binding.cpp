@@ -59,10 +59,15 @@ void check(int rc, const char* what) {
 }
 
 // ----------------------------------------------------------------------------------------------- small helpers
+// all on the one GPU whose stream the kernels go to
 void require_gpu(std::initializer_list<const Tensor*> tensors) {
-    for (const Tensor* t : tensors)
-        TORCH_CHECK(!t || !t->defined() || t->is_cuda(), "mamba2 HIP kernels need tensors on a GPU device (got ",
-                    t ? t->device().str() : "", "); there is no CPU path");
+    const Tensor* first = nullptr;
+    for (const Tensor* t : tensors) {
+        if (!t || !t->defined()) continue;
+        TORCH_CHECK(t->is_cuda(), "mamba2 HIP kernels need tensors on a GPU device (got ", t->device().str(), "); there is no CPU path");
+        if (!first) first = t;
+        TORCH_CHECK(t->device() == first->device(), "expected all tensors on one device, got ", first->device().str(), " and ", t->device().str());
+    }
 }
 
 int dtype_code(const Tensor& t) {
@@ -665,7 +670,7 @@ Tensor product(const Tensor& a, bool a_k, const Tensor& b, bool b_k, const Tenso
         return t.scalar_type() == at::kBFloat16 && t.stride(1) == 1 && t.stride(0) % 8 == 0 && t.stride(0) >= t.size(1) &&
                t.size(0) * t.stride(0) < (int64_t{1} << 31) && reinterpret_cast<uintptr_t>(ptr(t)) % 16 == 0;
     };
-    const bool plain_bias = !bias.defined() || (bias.scalar_type() == at::kBFloat16 && bias.is_contiguous());
+    const bool plain_bias = !bias.defined() || (bias.scalar_type() == at::kBFloat16 && bias.is_contiguous() && bias.dim() == 1 && bias.size(0) == p.N);
     if (!plain_bias || !rows(a) || !rows(b) || b.size(b_k ? 1 : 0) != p.K || !lib.m2_product_pays(p.M, p.N, p.K, a_k, b_k) || library_is_tuned()) {
         const Tensor at_ = a_k ? a : a.t(), bt = b_k ? b.t() : b;
         return bias.defined() ? at::addmm(bias, at_, bt) : at::mm(at_, bt);
@@ -681,7 +686,7 @@ Tensor project(const Tensor& x, const Tensor& w, const Tensor& bias, void* strea
 
 // a linear layer outside autograd
 Tensor linear(const Tensor& x, const Tensor& w, const OptTensor& bias) {
-    require_gpu({&x, &w});
+    require_gpu({&x, &w, &or_none(bias)});
     TORCH_CHECK_VALUE(x.dim() >= 1 && w.dim() == 2 && x.size(-1) == w.size(1), "linear: x (..., in) and weight (out, in) are required");
     Scope scope(x);
     std::vector<int64_t> shape = x.sizes().vec();
@@ -755,7 +760,7 @@ Tensor mixer(const Tensor& hidden, const Tensor& in_w, const Tensor& A_log, cons
              const Tensor& out_w, const OptTensor& conv_b, const OptTensor& in_b, const OptTensor& out_b, int64_t g, int64_t n, int64_t d, int64_t hd,
              bool recompute) {
     core_heads(g, n, d, hd);
-    require_gpu({&hidden, &in_w, &out_w});
+    require_gpu({&hidden, &in_w, &out_w, &or_none(in_b), &or_none(out_b)});
     TORCH_CHECK_VALUE(hidden.dim() == 3, "hidden_states must be (batch, seqlen, hidden_size)");
     bool differentiable = false;
     if (at::GradMode::is_enabled())
@@ -808,6 +813,11 @@ Tensor fused_prefill(const Tensor& zx, const Tensor& A, const OptTensor& D, cons
 }
 
 // ----------------------------------------------------------------------------------------------- decode step
+void check_conv_bias(const Tensor& conv_w, const Tensor& conv_b, int64_t channels) {
+    TORCH_CHECK_VALUE(!conv_b.defined() || (conv_b.numel() == channels && conv_b.scalar_type() == conv_w.scalar_type()),
+                      "the conv bias must have ", channels, " values in the dtype of the conv weight");
+}
+
 std::tuple<Tensor, Tensor, Tensor> decode_step(const Tensor& xBC, const Tensor& conv_state, const Tensor& conv_w, const OptTensor& conv_b_, const Tensor& S,
                                                const Tensor& dt, const Tensor& A_, const OptTensor& D_, int64_t g, int64_t activation,
                                                const OptTensor& dt_bias_, const OptTensor& out, bool static_scratch) {
@@ -832,6 +842,8 @@ std::tuple<Tensor, Tensor, Tensor> decode_step(const Tensor& xBC, const Tensor& 
     p.S = ptr<float>(S); p.dt = ptr(dt); p.A = ptr<float>(A); p.D = ptr<float>(D); p.y = ptr(Y); p.dt_bias = ptr<float>(bias);
     p.batch = b; p.nheads = h; p.headdim = p_; p.dstate = n; p.ngroups = g;
     p.k = static_cast<int32_t>(w.size(-1)); p.W = static_cast<int32_t>(conv_state.size(2));
+    check_conv_bias(w, bi, cx);
+    TORCH_CHECK_VALUE(A.numel() == h && (!D.defined() || D.numel() == h), "A and D must have shape (n_heads,)");
     TORCH_CHECK_VALUE(w.numel() == cx * p.k && conv_state.size(0) == b && conv_state.size(1) == cx, "conv weight and state must have ", cx, " channels");
     p.xBC_stride_b = xBC.stride(0); p.dt_stride_b = dt.stride(0); p.y_stride_b = Y.stride(0);
     p.dtype = dtype_code(xBC); p.param_dtype = dtype_code(w); p.activation = static_cast<int32_t>(activation);
@@ -867,7 +879,7 @@ bool starts_at(const Tensor& t, size_t bytes) { return reinterpret_cast<uintptr_
 // the small product's kernel copies 16 bytes at a time (a view into a flat buffer of parameters may start anywhere)
 bool linear_takes(const Tensor& w, const Tensor& bias) {
     return w.scalar_type() == at::kBFloat16 && w.is_contiguous() && starts_at(w, 16) &&
-           (!bias.defined() || (bias.is_contiguous() && bias.scalar_type() == at::kBFloat16));
+           (!bias.defined() || (bias.is_contiguous() && bias.scalar_type() == at::kBFloat16 && bias.dim() == 1 && bias.size(0) == w.size(0)));
 }
 
 // rows as that kernel reads them: 16-byte pieces at 32-bit byte offsets from the first row; others are copied once
@@ -1000,7 +1012,8 @@ Tensor mixer_step(const OptTensor& hidden_, ResidualStream* r, const OptTensor& 
     const Tensor& x = r ? (r->first.defined() ? r->first : r->rows) : hidden;
     TORCH_CHECK_VALUE(x.defined() && (r ? x.dim() == 2 : x.dim() == 3 && x.size(1) == 1), "hidden_states must be (batch, 1, hidden_size)");
     const int64_t b = x.size(0), width = x.size(-1);
-    require_gpu({&x, &in_w, &conv_w, &A, &D, &dt_bias, &norm_w, &out_w, &conv_state, &ssm_state});
+    require_gpu({&x, &in_w, &or_none(in_b), &conv_w, &or_none(conv_b), &A, &D, &dt_bias, &norm_w, &block_norm, &next_norm, &out_w, &or_none(out_b),
+                 &conv_state, &ssm_state});
     TORCH_CHECK_VALUE(ssm_state.dim() == 4 && ssm_state.size(0) == b && ssm_state.scalar_type() == at::kFloat && ssm_state.is_contiguous(),
                       "the SSM state must be float32 (batch, heads, headdim, state), contiguous");
     const int64_t h = ssm_state.size(1), d = h * ssm_state.size(2), cx = d + 2 * g * ssm_state.size(3);
@@ -1011,6 +1024,7 @@ Tensor mixer_step(const OptTensor& hidden_, ResidualStream* r, const OptTensor& 
                       "the projections do not match the states");
     TORCH_CHECK_VALUE(g > 0 && h % g == 0 && conv_w.numel() == cx * conv_w.size(-1) && A.numel() == h && D.numel() == h && dt_bias.numel() == h && norm_w.numel() == d,
                       "parameter shapes do not match the states");
+    check_conv_bias(conv_w, or_none(conv_b), cx);
     check_fp32({&A, &D, &dt_bias, &norm_w, &block_norm, &next_norm}, "A, D, dt_bias and the norm weights");
     TORCH_CHECK_VALUE(!r || (block_norm.defined() && block_norm.numel() == width && out_w.size(0) == width && (!next_norm.defined() || next_norm.numel() == width)),
                       "the norm weights must have the width of the residual stream");
@@ -1053,6 +1067,7 @@ Tensor stream_norm_linear(ResidualStream& r, const Tensor& norm_w, double eps, c
     require_gpu({&norm_w, &w, &bias});
     check_fp32({&norm_w}, "the norm weight");
     const Tensor& any = r.first.defined() ? r.first : r.rows;
+    require_gpu({&any, &w});
     TORCH_CHECK_VALUE(w.dim() == 2 && any.size(1) == w.size(1) && norm_w.numel() == w.size(1), "the norm weight and the product must have the width of the residual stream");
     Scope scope(w);
     m2_linear_params p = linear_params(w, bias, any.size(0));

@@ -298,3 +298,36 @@ def test_prefill_that_is_refused_leaves_the_cache(continuing, h, head_dim, n, me
         mamba2_fused_prefill(rand(b, l, d + cx + h).bfloat16(), -torch.ones(h, device=DEV), torch.ones(h, device=DEV), rand(cx, 1, 4).bfloat16(),
                              rand(cx).bfloat16(), rand(h), torch.ones(d, device=DEV), g, n, d, head_dim, conv_state, ssm_state, continuing=continuing)
     assert torch.equal(conv_state, before[0]) and torch.equal(ssm_state, before[1])
+
+
+@pytest.mark.parametrize("b", [3, 33])
+def test_biases_that_broadcast_and_biases_that_do_not_fit(b):
+    """A bias of one value is added to every output, as nn.Linear does; one of another length or on the host is an error."""
+    cfg, m = _model(1, use_bias=True)
+    mixer = m.backbone.layers[0].mixer
+    x = torch.randn(b, 1, cfg.hidden_size, generator=torch.Generator().manual_seed(4)).bfloat16().to(DEV)
+    long = torch.randn(2, 20, cfg.hidden_size, generator=torch.Generator().manual_seed(5)).bfloat16().to(DEV)
+
+    def passes():
+        with torch.no_grad():
+            return mixer.step(x, _cache(cfg, b)), mixer(long), mixer(long, cache_params=_cache(cfg, 2)), m.lm_head(x)
+
+    full = {}
+    for p in (mixer.in_proj, mixer.out_proj):
+        p.bias = torch.nn.Parameter(torch.full((1,), 0.25, dtype=torch.bfloat16, device=DEV))
+        full[p] = torch.nn.Parameter(p.bias.detach().repeat(p.out_features))
+    got = passes()
+    for p, bias in full.items():
+        p.bias = bias
+    for g, w in zip(got, passes()):
+        assert _rel(g, w) < 1e-2
+    for bias in (torch.zeros(mixer.out_proj.out_features - 1, dtype=torch.bfloat16, device=DEV), torch.zeros(mixer.out_proj.out_features, dtype=torch.bfloat16)):
+        mixer.out_proj.bias = torch.nn.Parameter(bias)
+        for call in (lambda: mixer.step(x, _cache(cfg, b)), lambda: mixer(long), lambda: mixer(long, cache_params=_cache(cfg, 2))):
+            with torch.no_grad(), pytest.raises(RuntimeError):
+                call()
+    mixer.out_proj.bias = full[mixer.out_proj]
+    for bias in (torch.zeros(8, dtype=torch.bfloat16, device=DEV), torch.zeros(mixer.conv_dim, device=DEV)):
+        mixer.conv1d.bias = torch.nn.Parameter(bias)
+        with torch.no_grad(), pytest.raises(ValueError, match="conv bias"):
+            mixer.step(x, _cache(cfg, b))
