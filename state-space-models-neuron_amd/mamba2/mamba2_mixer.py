@@ -160,12 +160,12 @@ class Mamba2Mixer(nn.Module):
         self.recompute_core = bool(getattr(config, "recompute_core", False))
 
     def _inference_params(self):
-        """fp32 (A, D, dt_bias) as the decode kernel takes them, rebuilt only when a parameter changed."""
+        """Contiguous fp32 (A, D, dt_bias) as the decode kernels take them, rebuilt only when a parameter changed."""
         ps = (self.A_log, self.D, self.dt_bias)
         key = tuple((p.data_ptr(), p._version, p.dtype) for p in ps)
         if self._fp32_params is None or self._fp32_params[0] != key:
             with torch.no_grad():
-                self._fp32_params = (key, -torch.exp(self.A_log.float()), self.D.float(), self.dt_bias.float())
+                self._fp32_params = (key, -torch.exp(self.A_log.float().contiguous()), self.D.float().contiguous(), self.dt_bias.float().contiguous())
         return self._fp32_params[1:]
 
     def nki_kernels_forward(self, hidden_states, cache_params: Optional[Mamba2Cache] = None,

@@ -331,3 +331,29 @@ def test_biases_that_broadcast_and_biases_that_do_not_fit(b):
         mixer.conv1d.bias = torch.nn.Parameter(bias)
         with torch.no_grad(), pytest.raises(ValueError, match="conv bias"):
             mixer.step(x, _cache(cfg, b))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("b", [3, 33])
+def test_layer_takes_parameters_that_are_strided_views(b, dtype):
+    """Every parameter a view with a stride of two into a wider one: step, training pass and prefill as with parameters of their own."""
+    cfg, m = _model(1, dtype)
+    mixer = m.backbone.layers[0].mixer
+    x = torch.randn(b, 1, cfg.hidden_size, generator=torch.Generator().manual_seed(4)).to(dtype).to(DEV)
+    long = torch.randn(2, 40, cfg.hidden_size, generator=torch.Generator().manual_seed(5)).to(dtype).to(DEV)
+
+    def passes():
+        out = mixer(long)
+        grads = torch.autograd.grad(out.float().pow(2).sum(), list(mixer.parameters()))
+        with torch.no_grad():
+            return [mixer.step(x, _cache(cfg, b, dtype)), mixer(long, cache_params=_cache(cfg, 2, dtype)), out.detach(), *grads]
+
+    want = passes()
+    for owner in (mixer, mixer.conv1d, mixer.norm, mixer.in_proj, mixer.out_proj):
+        for name, p in list(owner._parameters.items()):
+            if p is not None:
+                wide = torch.stack((p.detach(), torch.full_like(p, float("nan"))), dim=-1)
+                setattr(owner, name, torch.nn.Parameter(wide[..., 0]))
+    assert not mixer.D.is_contiguous() and not mixer.in_proj.weight.is_contiguous()
+    for g, w in zip(passes(), want):
+        assert _rel(g, w) < 2e-2
