@@ -29,10 +29,10 @@ HBM_PEAK_GBS = 8000.0              # MI355X HBM3E
 # HBM bytes per step as PROFILED (two rocprofv3 --pmc runs of this file, FETCH_SIZE then WRITE_SIZE, each scaled by what
 # the same counter reads for the 1 GiB copy kernel in the same run; summaries under profiles/).  They are constants of
 # the kernels as last profiled, not measurements of this run: `traffic_source` in the JSON says so.
-SSD_TRAFFIC_BYTES = 1.460e9
+SSD_TRAFFIC_BYTES = 1.445e9
 CONV_TRAFFIC_BYTES = 489.3e6
 DECODE_TRAFFIC_BYTES = 64 * 689.2e6
-GLUE_TRAFFIC_BYTES = 710.5e6
+GLUE_TRAFFIC_BYTES = 705.6e6
 TRAFFIC_SOURCE = "profiled constant: rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of this workload, scaled by the 1 GiB copy kernel; not measured in this run"
 
 SSD_CFG = dict(b=4, l=2048, h=80, p=64, n=128, g=1)
@@ -356,7 +356,7 @@ def bench_layer_c3(steps, warmup):
                 wall_ms_per_step=wall_ms, ms_per_step_recompute_core=ms_recompute, dtype="bf16",
                 config={"workload": "Mamba2Mixer fwd+bwd, b2 l4096 d_model4096 d_inner8192 h128 p64 n128 g8 chunk128: in_proj, conv1d+SiLU, SSD, grouped gated RMSNorm, out_proj; core activations kept for the backward"},
                 parity={"against": "oracle.mixer.fused_core_ref (fp64), fused core at this width, b1 l512, checked before timing", "tensors": parity},
-                projections={"gemm_flops_per_step": gemm_flops, "library": "hipBLASLt behind nn.Linear (outside the hot path)"},
+                projections={"gemm_flops_per_step": gemm_flops, "library": "hipBLASLt behind torch.mm (outside the hot path)"},
                 ssd_part={"ms_per_step": ms_ssd, "algorithmic_flops_per_step": ssd_flops,
                           "roofline": {"bound": "mfma", "achieved": ssd_flops / (ms_ssd * 1e-3) / 1e12, "peak": MFMA_BF16_PEAK_TFLOPS,
                                        "unit": "TFLOP/s", "frac": ssd_flops / (ms_ssd * 1e-3) / 1e12 / MFMA_BF16_PEAK_TFLOPS, "traffic": None}},

@@ -658,7 +658,8 @@ Tensor fused_core(const Tensor& zx, const Tensor& A, const OptTensor& D, const T
 
 // A program that has torch's TunableOp on wants the general library's solutions timed and the best one taken: its products go there.
 // At 128 rows of a 2560-channel layer the best ones beat this library's kernel, which beats the library's default choice (64-layer
-// step, replayed: 11.28 ms with the kernel, 11.11 with the chosen solutions, 11.8 with the default ones).  Asking costs 2 ns.
+// step, replayed: 11.18 to 11.29 ms with the kernel; 10.98 to 11.13 with the chosen solutions in five of seven graphs and 11.28 in
+// two, by what the tuner's own timing preferred; 11.8 with the default ones).  Asking costs 2 ns.
 bool library_is_tuned() { return at::cuda::tunable::getTuningContext()->IsTunableOpEnabled(); }
 
 // out (M, N) = A B (+ bias): `a` is A or, if !a_k, A^T (K, M); `b` is B^T (N, K) or, if !b_k, B

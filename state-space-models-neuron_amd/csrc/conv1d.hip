@@ -5,9 +5,9 @@
 //
 // The op is HBM-bandwidth bound (8 FLOP + one SiLU per element), so the fast path is a
 // streaming kernel on the channels-last (b, l, C) layout the mixer uses: one thread owns
-// one 16-byte channel vector and walks TL consecutive tokens with the k-1 token history in
-// registers, so every element is loaded once (plus a (k-1)/TL halo) and all global accesses
-// are 16-byte, lane-contiguous along channels.  No transposes (the reference needs two per
+// a short vector of channels (8 bytes forward, 4 backward in bf16) and walks TL consecutive tokens
+// with the k-1 token history in registers, so every element is loaded once (plus a (k-1)/TL halo)
+// and all global accesses are lane-contiguous along channels.  No transposes (the reference needs two per
 // tile because its engine wants channels on partitions).
 //
 // The backward recomputes the pre-activation, forms g = dy * act'(z) and emits dx with a

@@ -8,8 +8,8 @@
 //              backward (fused_kernel.py:159-171):  var = mean(h^2) + eps, r = rsqrt(var), gw = g w,
 //              cf = mean(h gw) / var,  d_h = r (gw - cf h),  dx = d_h silu(z),  dz = d_h x silu'(z),  dw = sum_rows g h r
 //
-// A (row, group) is handled by one wave (groups of up to 2048 channels) or by the four waves of a workgroup (up to
-// 8192), its channels in registers as 16-byte vectors; a workgroup walks a block of rows, so the per-channel weight
+// A (row, group) is handled by one wave (groups of up to 2048 channels) or by the four or five waves of a workgroup (up
+// to 8192), its channels in registers as 16-byte vectors; a workgroup takes many rows, so the per-channel weight
 // and -- in the backward -- the dw accumulators stay in registers across rows.  dw and d_bias leave as per-block
 // partials in a caller-owned workspace and are summed in a fixed order by a second small kernel (no atomics).
 #include <initializer_list>

@@ -240,7 +240,9 @@ extern "C" int m2_product_fits(int64_t M, int64_t N, int64_t K, int32_t a_k, int
     return 1;
 }
 
-// Where these kernels are ahead of the general library's product (bf16, by size; its call also costs the host 18 us to their 4):
+// Where these kernels are ahead of the general library's product with its default solution (bf16, by size; its call also costs the
+// host 18 us to their 4).  Solutions chosen by timing are another matter: at 128 rows of a 2560-channel layer they are ahead, so a
+// program that has them chosen keeps its products there (library_is_tuned in binding.cpp).
 //   weight gradients (k = tokens) with few outputs -- 500 x 3352 x 768: 14.4 -> 11.1 us, 2000: 39 -> 27; with ten million outputs
 //   the stores bound both and the library's are better (200 tokens, 10576 x 2560: 34 us to 51);
 //   other products up to 4e9 multiply-adds -- 200 x 2560 x 5120: 25.8 -> 21.3 us, 500 x 3352 x 768: 10.0 -> 8.5; beyond, its larger

@@ -4,7 +4,9 @@ Parameter names and shapes are the reference's (and HF / state-spaces'): ``in_pr
 ``conv1d.bias``, ``dt_bias``, ``A_log``, ``D``, ``norm.weight``, ``out_proj``.  The tensor-parallel linears of the
 reference become ``nn.Linear`` (tp = 1) and its XLA-device assert is dropped.  ``forward`` = in_proj ->
 ``mamba2_fused_kernel`` -> out_proj; ``step`` = in_proj -> ``mamba2_kernel_inference`` on the [xBC | dt] columns
-(softplus applied inside) -> gated norm -> out_proj: two projections and three kernels of this library per token.
+(softplus applied inside) -> gated norm -> out_proj.  Where calling the projections (and in ``step`` the norm) does nothing
+but their own arithmetic, both run as one native call: ``forward`` as one autograd node, ``step`` for up to 32 bf16 sequences
+as three launches; else module by module.
 
 ``forward`` with ``cache_params`` (inference only) is the prefill that hands over to ``step``: it leaves the layer's
 SSM and conv state in the cache, and continues from them when ``cache_params.seqlen_offset > 0``.  The reference

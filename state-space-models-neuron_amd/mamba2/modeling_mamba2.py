@@ -320,7 +320,7 @@ class GraphedStep:
 
     ``tune_gemms=True`` lets torch's TunableOp time the BLAS libraries' solutions for the step's projection shapes (in_proj,
     out_proj, LM head) during the warm-up and captures the chosen ones in place of this library's kernel for few rows (64 layers
-    of 2560 channels, batch 128: 11.28 -> 11.11 ms); the process-wide TunableOp switches are put back afterwards, the graph keeps
+    of 2560 channels, batch 128: 11.2 -> 11.0 to 11.1 ms in most graphs); the process-wide TunableOp switches are put back afterwards, the graph keeps
     the kernels it captured.  Up to 32 sequences there is nothing to choose: the projections are part of the layer's own
     launches.  The chosen solutions may round differently, so replays then agree with the eager step to bf16 accuracy, not bit
     for bit.
