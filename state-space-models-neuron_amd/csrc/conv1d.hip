@@ -139,9 +139,14 @@ __device__ __forceinline__ void load_taps(const void* __restrict__ w, const void
 // ------------------------------------------------------------------------------------------
 // Fast path, channels-last, k == 4.
 // grid: x = ceil(CV / kCVT), y = ceil(nseg / kSEG), z = batch; block (kCVT, kSEG).
-template <typename T, typename WT, int V, int ACT>
+// PREFILL: the decode cache `state` ([b][C][W], oldest first) holds the inputs in front of the sequence (kContinuing) and takes
+// its last W ones (kTail).  The thread of a strip's first segment does both, so nobody reads a cache entry that another thread
+// has renewed; a kernel of its own behind this one took 4-5 us of every prefill (77 -> 73 us for 200 tokens of a 2560-channel
+// layer).  Only where no two threads share channels (C a multiple of V), else conv_tail_kernel follows.
+constexpr int kContinuing = 1, kTail = 2;
+template <typename T, typename WT, int V, int ACT, bool PREFILL>
 __global__ void __launch_bounds__(kCVT * kSEG)
-conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias, const T* __restrict__ hist, int W,
+conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias, T* state, int W, int flags,
                    T* __restrict__ y, int64_t l, int64_t C, int64_t xsb, int64_t xsl, int64_t ysb, int64_t ysl) {
     const int64_t cv = (int64_t)blockIdx.x * kCVT + threadIdx.x;
     const int64_t seg = (int64_t)blockIdx.y * kSEG + threadIdx.y;
@@ -160,15 +165,43 @@ conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     if (t0 - 3 >= 0) ld_elems<T, V>(xp + (t0 - 3) * xsl, h0);
     if (t0 - 2 >= 0) ld_elems<T, V>(xp + (t0 - 2) * xsl, h1);
     if (t0 - 1 >= 0) ld_elems<T, V>(xp + (t0 - 1) * xsl, h2);
-    if (hist && t0 == 0) {
+    if (PREFILL && (flags & kContinuing) && t0 == 0) {
         // the inputs in front of the sequence come out of the decode cache (three short reads per channel in the first
         // segment only; putting cache and sequence behind one another in memory first took 35 us of 145 at b8 l333 C5376)
 #pragma unroll
         for (int j = 0; j < V; ++j) {
-            const T* hp = hist + (b * C + c0 + j) * W + (W - 3);
+            const T* hp = state + (b * C + c0 + j) * W + (W - 3);
             h0[j] = to_f32(hp[0]); h1[j] = to_f32(hp[1]); h2[j] = to_f32(hp[2]);
         }
     }
+    // the last W inputs, four columns at a time; where the sequence is shorter, what is left of the cache (or zeros) moves up
+    auto leave_tail = [&] {
+        if (!PREFILL || !(flags & kTail) || t0 != 0) return;
+        T* sp = state + (b * C + c0) * W;
+        for (int w0 = 0; w0 < W; w0 += 4) {
+            T v[4][V];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int wq = w0 + q < W ? w0 + q : W - 1;
+                const int64_t t = l - W + wq;
+                if (t >= 0) {
+                    const RawVec<T, V> r = ld_stream<T, V>(xp + t * xsl);
+                    const T* e = reinterpret_cast<const T*>(&r);
+#pragma unroll
+                    for (int j = 0; j < V; ++j) v[q][j] = e[j];
+                } else {
+#pragma unroll
+                    for (int j = 0; j < V; ++j) v[q][j] = flags & kContinuing ? sp[j * W + wq + l] : from_f32<T>(0.f);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (w0 + q < W) {
+#pragma unroll
+                    for (int j = 0; j < V; ++j) sp[j * W + w0 + q] = v[q][j];
+                }
+        }
+    };
     auto step = [&](const RawVec<T, V>& r, T* __restrict__ yq) {
         float out[V], cur[V];
         cvtv<T, V>(r, cur);
@@ -200,6 +233,7 @@ conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
         }
 #pragma unroll
         for (int u = 0; u < kUNR; ++u) step(nxt[u], yq + u * ysl);
+        leave_tail();
         return;
     }
     const int64_t t1 = l;
@@ -217,6 +251,7 @@ conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
         for (int u = 0; u < kUNR; ++u)
             if (tg + u < t1) step(raw[u], yp + (tg + u) * ysl);
     }
+    leave_tail();
 }
 
 // Backward fast path.  Each thread marches t over [t0, t0+TL+3): at step t it forms g[t] and
@@ -661,10 +696,13 @@ int check_common(const m2_conv1d_params* p) {
     return M2_OK;
 }
 
-// hist: null, or the W >= k - 1 inputs in front of the sequence, [b][C][W], oldest first
+// state: null, or the decode cache of W >= k - 1 inputs, [b][C][W], oldest first: in front of the sequence where `continuing`,
+// and its last ones afterwards
 template <typename T>
-int launch_fwd(const m2_conv1d_params* p, const void* hist_, int W, hipStream_t st) {
-    const T* hist = static_cast<const T*>(hist_);
+int launch_fwd(const m2_conv1d_params* p, void* state_, int W, bool continuing, hipStream_t st) {
+    T* state = static_cast<T*>(state_);
+    const T* hist = continuing ? state : nullptr;
+    bool tail = state != nullptr;      // still to be left by conv_tail_kernel
     const int64_t nb = p->batch, l = p->seqlen, C = p->channels;
     const T* x = static_cast<const T*>(p->x);
     T* y = static_cast<T*>(p->y);
@@ -673,10 +711,14 @@ int launch_fwd(const m2_conv1d_params* p, const void* hist_, int W, hipStream_t 
         const int64_t CV = ceil_div(C, (int64_t)V), nseg = ceil_div(l, kTLF);
         dim3 grid((unsigned)ceil_div(CV, kCVT), (unsigned)ceil_div(nseg, kSEG), (unsigned)nb), block(kCVT, kSEG);
         M2_REQUIRE(grid.y <= 65535, M2_ERR_SHAPE, "conv1d: sequence too long for the grid");
+        const bool fold = tail && C % V == 0;
+        const int flags = (continuing ? kContinuing : 0) | (fold ? kTail : 0);
         conv_dispatch(p, [&](auto wt, auto act) {
-            conv_fwd_cl_kernel<T, decltype(wt), V, decltype(act)::value><<<grid, block, 0, st>>>(
-                x, p->w, p->bias, hist, W, y, l, C, p->x_stride_b, p->x_stride_l, p->y_stride_b, p->y_stride_l);
+            auto k = state ? conv_fwd_cl_kernel<T, decltype(wt), V, decltype(act)::value, true>
+                           : conv_fwd_cl_kernel<T, decltype(wt), V, decltype(act)::value, false>;
+            k<<<grid, block, 0, st>>>(x, p->w, p->bias, state, W, flags, y, l, C, p->x_stride_b, p->x_stride_l, p->y_stride_b, p->y_stride_l);
         });
+        tail = tail && !fold;
     } else if (!hist && channel_major_ok(p, false)) {
         const int64_t pieces = ceil_div(l, (int64_t)VecTraits<T>::kVec), total = nb * C * pieces;
         conv_dispatch(p, [&](auto wt, auto act) {
@@ -690,7 +732,10 @@ int launch_fwd(const m2_conv1d_params* p, const void* hist_, int W, hipStream_t 
             x, p->w, p->bias, hist, W, y, nb, l, C, p->k, p->x_stride_b, p->x_stride_l, p->x_stride_c,
             p->y_stride_b, p->y_stride_l, p->y_stride_c, p->param_dtype, p->activation, tf);
     }
-    return check_launch("conv1d_fwd");
+    const int rc = check_launch("conv1d_fwd");
+    if (rc || !tail) return rc;
+    conv_tail_kernel<T><<<(unsigned)ceil_div(nb * C, (int64_t)256), 256, 0, st>>>(x, state, W, continuing, nb, l, C, p->x_stride_b, p->x_stride_l, p->x_stride_c);
+    return check_launch("conv1d_tail");
 }
 
 template <typename T>
@@ -763,7 +808,7 @@ extern "C" int m2_conv1d_fwd(const m2_conv1d_params* p, void* stream) {
     if (rc) return rc;
     if (p->batch == 0 || p->seqlen == 0 || p->channels == 0) return M2_OK;
     M2_REQUIRE(p->x && p->w && p->y, M2_ERR_NULL, "conv1d_fwd: x, w and y are required");
-    M2_DISPATCH_DTYPE(p->dtype, T, return launch_fwd<T>(p, nullptr, 0, static_cast<hipStream_t>(stream)));
+    M2_DISPATCH_DTYPE(p->dtype, T, return launch_fwd<T>(p, nullptr, 0, false, static_cast<hipStream_t>(stream)));
     return M2_OK;
 }
 
@@ -774,14 +819,7 @@ extern "C" int m2_conv1d_prefill(const m2_conv1d_params* p, void* conv_state, in
     if (p->batch == 0 || p->seqlen == 0 || p->channels == 0) return M2_OK;
     M2_REQUIRE(p->x && p->w && p->y && conv_state, M2_ERR_NULL, "conv1d_prefill: x, w, y and conv_state are required");
     M2_REQUIRE(W >= p->k - 1, M2_ERR_SHAPE, "conv1d_prefill: the cache holds %d inputs, needs %d", W, p->k - 1);
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    M2_DISPATCH_DTYPE(p->dtype, T, {
-        if ((rc = launch_fwd<T>(p, continuing ? conv_state : nullptr, W, st))) return rc;
-        conv_tail_kernel<T><<<(unsigned)ceil_div(p->batch * p->channels, (int64_t)256), 256, 0, st>>>(
-            static_cast<const T*>(p->x), static_cast<T*>(conv_state), W, continuing, p->batch, p->seqlen, p->channels,
-            p->x_stride_b, p->x_stride_l, p->x_stride_c);
-        return check_launch("conv1d_tail");
-    });
+    M2_DISPATCH_DTYPE(p->dtype, T, return launch_fwd<T>(p, conv_state, W, continuing != 0, static_cast<hipStream_t>(stream)));
     return M2_OK;
 }
 

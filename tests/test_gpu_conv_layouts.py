@@ -59,3 +59,29 @@ def test_prefill_in_two_pieces(l1, l2, k, W, dtype, state_dtype, strided):
     tol = 2e-2 if dtype == torch.bfloat16 else 2e-4
     torch.testing.assert_close(pieces.float(), whole.float(), rtol=tol, atol=tol)
     torch.testing.assert_close(two[1], one[1], rtol=tol, atol=tol)
+
+
+@pytest.mark.parametrize("C", [8, 12, 9, 64, 257, 260])                     # whole vectors, shared last vectors, more than one block
+@pytest.mark.parametrize("W,l", [(3, 1), (3, 2), (4, 3), (5, 4), (5, 1), (8, 3), (8, 6), (11, 40), (4, 16), (4, 129)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("continuing", [0, 1])
+def test_prefill_leaves_the_last_inputs(C, W, l, dtype, continuing):
+    """The cache after a prefill is, bit for bit, the end of (what it held | the sequence); the outputs those of the conv over both."""
+    import ctypes
+    from mamba2 import _lib
+    from mamba2.conv1d_grouped import conv1d_forward
+    lib, b = _lib.load(), 2
+    torch.manual_seed(C * 100 + W * 10 + l)
+    x = torch.randn(b, l, C, device=DEV).to(dtype)
+    w, bias = torch.randn(C, 1, 4, device=DEV).to(dtype), torch.randn(C, device=DEV).to(dtype)
+    state = torch.randn(b, C, W, device=DEV).to(dtype)
+    before = state.clone() if continuing else torch.zeros_like(state)
+    joined = torch.cat([before, x.transpose(1, 2)], 2)
+    y = torch.empty_like(x)
+    p = _lib.Conv1dParams(x=x.data_ptr(), w=w.data_ptr(), bias=bias.data_ptr(), y=y.data_ptr(), batch=b, seqlen=l, channels=C, k=4,
+                          x_stride_b=l * C, x_stride_l=C, x_stride_c=1, y_stride_b=l * C, y_stride_l=C, y_stride_c=1,
+                          dtype=_lib.dtype_code(dtype), param_dtype=_lib.dtype_code(dtype), activation=1)
+    _lib.check(lib.m2_conv1d_prefill(ctypes.byref(p), _lib.ptr(state), W, continuing, _lib.stream_ptr()), "prefill")
+    assert torch.equal(state, joined[:, :, -W:])
+    ref = conv1d_forward(joined.transpose(1, 2).contiguous(), w, bias, "silu", channels_last=True)[:, W:]
+    assert torch.equal(y, ref)      # the same sums in the same order
