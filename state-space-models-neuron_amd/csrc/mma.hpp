@@ -81,12 +81,6 @@ __device__ __forceinline__ Frag<bf16_t> scale_frag(const Frag<bf16_t>& a, const 
     for (int i = 0; i < 8; ++i) r.v[i] = (bf16_t)((float)a.v[i] * f[i]);
     return r;
 }
-__device__ __forceinline__ Frag<float> scale_frag(const Frag<float>& a, const float (&f)[8]) {
-    Frag<float> r;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) r.v[i] = a.v[i] * f[i];
-    return r;
-}
 
 // the two 16-bit elements of a 32-bit word as fp32, and back (round to nearest even)
 template <typename T> __device__ __forceinline__ float unpack_lo(uint32_t w);
@@ -132,7 +126,6 @@ __device__ __forceinline__ void keep_packed(Frag<bf16_t>& f) {
     asm volatile("" : "+v"(raw));
     f.v = __builtin_bit_cast(bf16x8, raw);
 }
-__device__ __forceinline__ void keep_packed(Frag<float>&) {}
 
 // One wave: acc[i][j] (32x32 blocks) += A[rows i*32.., k0:k1] * Bt[rows j*32.., k0:k1]^T, operands in LDS.
 // A points at the first of this wave's BM*32 rows, Bt at the first of its BN*32 rows.  k0, k1 multiples of 16.
@@ -195,45 +188,6 @@ __device__ __forceinline__ void stage_rows(T* __restrict__ s, int ld, const T* _
     }
 }
 
-// stage_transposed: global tile [ROWS][COLS] (COLS contiguous) -> LDS [COLS][ld], element (c, r).
-// Global reads stay 16-byte and coalesced; the transpose happens in the (2- or 4-byte) LDS writes.
-template <typename T, int ROWS, int COLS, int NT, bool SCALE>
-__device__ __forceinline__ void stage_transposed(T* __restrict__ s, int ld, const T* __restrict__ g, int64_t gstride,
-                                                 int valid, const float* __restrict__ rowscale, int tid) {
-    constexpr int V = VecTraits<T>::kVec;
-    constexpr int VPR = COLS / V;
-    constexpr int TOTAL = ROWS * VPR;
-    static_assert(COLS % V == 0, "tile width must be a multiple of the vector width");
-    if (!SCALE) {
-#pragma unroll 4
-        for (int e = tid; e < TOTAL; e += NT) {
-            const int cv = e / ROWS, r = e % ROWS;
-            uint4 raw = uint4{0u, 0u, 0u, 0u};
-            if (r < valid) raw = *reinterpret_cast<const uint4*>(g + (int64_t)r * gstride + cv * V);
-            const T* el = reinterpret_cast<const T*>(&raw);
-#pragma unroll
-            for (int i = 0; i < V; ++i) s[(cv * V + i) * ld + r] = el[i];
-        }
-        return;
-    }
-#pragma unroll 4
-    for (int e = tid; e < TOTAL; e += NT) {
-        // consecutive threads take consecutive tokens of the same channel vector: the LDS writes of a
-        // wave then fall into consecutive addresses of V rows (few bank conflicts), while the global
-        // reads of a wave are 64 rows x 16 bytes.
-        const int cv = e / ROWS, r = e % ROWS;
-        float v[V];
-        if (r < valid) load16(g + (int64_t)r * gstride + cv * V, v);
-        else {
-#pragma unroll
-            for (int i = 0; i < V; ++i) v[i] = 0.f;
-        }
-        const float sc = SCALE ? rowscale[r] : 1.f;
-#pragma unroll
-        for (int i = 0; i < V; ++i) s[(cv * V + i) * ld + r] = from_f32<T>(SCALE ? v[i] * sc : v[i]);
-    }
-}
-
 // Sum of v over the 32 lanes that share (lane >> 5), for 16 values at once (the 16 accumulator rows of a lane),
 // by a butterfly reduce-scatter: 16 cross-lane moves instead of 80 (the widest step selects and adds with one row swap, the
 // single-move DPP steps fold into their additions: 45 instructions, not 85, in kernels bound by their vector instructions).  On return every lane holds ONE total:
@@ -276,19 +230,16 @@ __device__ __forceinline__ float wave_scan(float x) {
     x += dpp_from<0x143, 0xC>(x);      // row_bcast:31
     return x;
 }
+// The same over each half of a wave
+__device__ __forceinline__ float half_wave_scan(float x) {
+    x += dpp_from<0x111, 0xF>(x); x += dpp_from<0x112, 0xF>(x); x += dpp_from<0x114, 0xF>(x); x += dpp_from<0x118, 0xF>(x);      // row_shr
+    x += dpp_from<0x142, 0xA>(x);      // row_bcast:15
+    return x;
+}
 // l[t] = sum_{s <= t} A d[s] over a chunk, lane holding tokens `lane` and `lane + 64`
 __device__ __forceinline__ void wave_cumsum_from(float A, float d0, float d1, float& l0, float& l1) {
     l0 = wave_scan(A * d0); l1 = wave_scan(A * d1);
     l1 += __shfl(l0, 63, 64);
-}
-
-// Per (batch, head, chunk) the cumulative log-decay and dt are computed once (ld_table_body, prep_kernel) into a table of
-// 2 * kQ floats, [ l[0..kQ) | dt[0..kQ) ], tokens past the end of the sequence holding dt = 0 and the last l.
-// Lane holds tokens `lane` and `lane + 64`.
-__device__ __forceinline__ void wave_ld_load(const float* __restrict__ ldtab, int64_t bhc, float& l0, float& l1, float& d0, float& d1) {
-    const int lane = threadIdx.x & 63;
-    const float* p = ldtab + bhc * (2 * kQ);
-    l0 = p[lane]; l1 = p[lane + 64]; d0 = p[kQ + lane]; d1 = p[kQ + lane + 64];
 }
 
 // Orders this wave's LDS writes before its later LDS reads of what OTHER lanes of the same wave wrote

@@ -27,280 +27,19 @@
 //
 // Launch sequence (16-bit operands; fp32 operands take the kernels named in brackets):
 //   prep_kernel, state_pass16_kernel [chunk_state + state_scan]   recompute G, tables, S_prev (skipped if the caller kept them)
-//   state_pass16_kernel<REVERSE> [chunk_state<DSTATE> + state_scan<REVERSE>]
-//                                                              dS per chunk, d initial state [, e^{Lam} <dS, S_prev>]
-//   dg16_kernel [dg_kernel]   per (b, chunk, group, head slice)  partial dG (heads reduced in registers), dl_diag per head
-//   ssd_bwd16_kernel [off_kernel<C>, <B>, diag_off_kernel<bwd>]
-//                             per (b, chunk, group, head slice)  dx, per-token decay-gradient terms, dD partials, partial state parts
-//                                                                of dB / dC, and with 16-bit operands e^{Lam} <dS, S_prev>
+//   state_pass16_kernel<REVERSE> [chunk_state32<DSTATE> + state_scan<REVERSE>]
+//                                                              dS per chunk, d initial state
+//   dg16_kernel               per (b, chunk, group, head slice)  partial dG (heads reduced in registers), dl_diag per head
+//   ssd_bwd16_kernel          per (b, chunk, group, head slice)  dx, per-token decay-gradient terms, dD and e^{Lam} <dS, S_prev> partials,
+//                                                                partial state parts of dB / dC
+//   [ssd_bwd32_kernel         what those two do in one pass; dB and dC too where a workgroup has all heads of its group]
 //   tail1_kernel              da_body: ddt, dA partials per (b, head, chunk);  slice_sum_body: partials over the head slices
-//   tail2_kernel              bc_final16_body [bc_final_body] per (b, chunk, group): dC = dG B + dCoff, dB = dG^T C + dBoff;
+//   tail2_kernel              bc_final16_body [bc_final32_body] per (b, chunk, group): dC = dG B + dCoff, dB = dG^T C + dBoff;
 //                             ad_reduce_body per head: dA, dD (fixed order, no atomics)
 #include "ssd_host.hpp"
 
 namespace m2 {
 namespace {
-
-// ------------------------------------------------------------------------------------------
-// dG partial and the diagonal part of the decay gradient, fp32 operands (16-bit ones: dg16_kernel).
-// grid (nchunks, ngroups * nslices, batch), 512 threads (8 waves).  Wave w owns the 32x32 blocks of the
-// [kQ][kQ] tile with block-row rb = w >> 1 and block-columns cb0 = 2 (w & 1), cb0 + 1.
-//   per head:  P = dY X^T  (MFMA, K = headdim);   dG^h[i][j] = e^{l_i - l_j} dt_j P[i][j]   (i >= j)
-//              dG += dG^h;    pr = dG^h o G;   dl_diag[i] = sum_j pr[i][j] - sum_i' pr[i'][i]
-// Row and column sums come from the same fp32 products, so pairs inside a suffix cancel exactly.
-template <typename T, int P, int HS>
-__global__ void __launch_bounds__(512, 2)
-dg_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
-          const T* __restrict__ dY, const T* __restrict__ Gm, float* __restrict__ dGp, float* __restrict__ dl_diag,
-          int64_t seqlen, int64_t nheads, int64_t ngroups, int64_t nchunks, int64_t nslices, int64_t hps,
-          int64_t Xsb, int64_t Xsl, int64_t Xsh, int64_t dYsb, int64_t dYsl, int64_t dYsh) {
-    static_assert(sizeof(T) == 4, "16-bit operands take dg16_kernel");
-    constexpr int LDP = lds_ld<T>(P);
-    constexpr int LDQ = lds_ld<T>(kQ);
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    float* wtab = reinterpret_cast<float*>(smem_raw);      // [8 waves][kQ]  l (wave-private)
-    float* s_rs = wtab + 8 * kQ;                           // [2][kQ]
-    float* s_cs = s_rs + 2 * kQ;                           // [4][kQ]
-    T* sA = reinterpret_cast<T*>(s_cs + 4 * kQ);           // dY [kQ][LDP]
-    T* sT = sA + kQ * LDP;                                 // X  [kQ][LDP]
-    T* sG = sT + kQ * LDP;                                 // G  [kQ][LDQ]  (blocks above the diagonal are never read)
-
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int r = lane & 31;
-    const int64_t c = blockIdx.x, b = blockIdx.z;
-    const int64_t g = blockIdx.y / nslices, slice = blockIdx.y % nslices;
-    const int64_t hpg = nheads / ngroups;
-    const int64_t t0 = c * kQ;
-    const int valid = (int)((seqlen - t0) < kQ ? (seqlen - t0) : kQ);
-    const int rb = wave >> 1, cb0 = (wave & 1) * 2;
-    const bool active = cb0 <= rb;
-    float* wl = wtab + wave * kQ;
-
-    // causal-masked G of this (chunk, group), shared by all heads: staged once
-    stage_rows<T, kQ, kQ, 512, false>(sG, LDQ, Gm + ((b * nchunks + c) * ngroups + g) * (int64_t)(kQ * kQ), kQ, kQ, nullptr, tid);
-    floatx16 dG[1][2];
-    acc_zero(dG);
-
-    // the next head's dY and X tiles travel global -> registers while the current head is computed
-    constexpr int V = VecTraits<T>::kVec;
-    constexpr int VPR = P / V;                     // 16-byte vectors per token row
-    constexpr int NV = kQ * VPR / 512;             // vectors per thread per tile
-    static_assert((kQ * VPR) % 512 == 0, "tile does not divide over the workgroup");
-    uint4 pdy[NV], pxx[NV];
-    auto prefetch = [&](int64_t h) {
-        const T* gy = dY + b * dYsb + t0 * dYsl + head_off<HS>(h, dYsh);
-        const T* gx = X + b * Xsb + t0 * Xsl + head_off<HS>(h, Xsh);
-#pragma unroll
-        for (int it = 0; it < NV; ++it) {
-            const int e = it * 512 + tid, rr = e / VPR, cv = e % VPR;
-            const bool ok = rr < valid;
-            pdy[it] = ok ? *reinterpret_cast<const uint4*>(gy + (int64_t)rr * dYsl + cv * V) : uint4{0u, 0u, 0u, 0u};
-            pxx[it] = ok ? *reinterpret_cast<const uint4*>(gx + (int64_t)rr * Xsl + cv * V) : uint4{0u, 0u, 0u, 0u};
-        }
-    };
-    prefetch(g * hpg + slice * hps);
-
-    for (int64_t hh = 0; hh < hps; ++hh) {
-        const int64_t h = g * hpg + slice * hps + hh;
-        float l0, l1, d0, d1;
-        wave_ld_load(ldtab, (b * nheads + h) * nchunks + c, l0, l1, d0, d1);
-        wl[lane] = l0; wl[lane + 64] = l1;
-        const float l_first = rb < 2 ? __shfl(l0, rb * 32, 64) : __shfl(l1, rb * 32 - 64, 64);
-        const float l_last = rb < 2 ? __shfl(l0, rb * 32 + 31, 64) : __shfl(l1, rb * 32 + 31 - 64, 64);
-        const bool fast = (l_first - l_last) < kMaxRange;
-        // column-side values of this lane's two columns j = (cb0 + jb) * 32 + r
-        float lj[2], dtj[2], vj[2];
-#pragma unroll
-        for (int jb = 0; jb < 2; ++jb) {
-            const int src = jb * 32 + r;
-            lj[jb] = cb0 == 0 ? __shfl(l0, src, 64) : __shfl(l1, src, 64);
-            dtj[jb] = cb0 == 0 ? __shfl(d0, src, 64) : __shfl(d1, src, 64);
-            vj[jb] = (cb0 + jb <= rb) ? __expf(fminf(l_first - lj[jb], kMaxRange)) * dtj[jb] : 0.f;
-        }
-
-        __syncthreads();      // previous head: tiles consumed, s_rs / s_cs consumed
-#pragma unroll
-        for (int it = 0; it < NV; ++it) {
-            const int e = it * 512 + tid, rr = e / VPR, cv = e % VPR;
-            *reinterpret_cast<uint4*>(sA + rr * LDP + cv * V) = pdy[it];
-            *reinterpret_cast<uint4*>(sT + rr * LDP + cv * V) = pxx[it];
-        }
-        __syncthreads();
-        if (hh + 1 < hps) prefetch(h + 1);
-
-        float rsum[16], csum[2] = {0.f, 0.f};
-#pragma unroll
-        for (int v = 0; v < 16; ++v) rsum[v] = 0.f;
-        if (active) {
-#pragma unroll
-            for (int jb = 0; jb < 2; ++jb) {
-                if (cb0 + jb > rb) continue;
-                floatx16 pa[1][1];
-                acc_zero(pa);
-                wave_mma<1, 1>(pa, sA + rb * 32 * LDP, LDP, sT + (cb0 + jb) * 32 * LDP, LDP, 0, P);
-                const int j = (cb0 + jb) * 32 + r;
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int i = rb * 32 + acc_row(lane, v);
-                    float w;
-                    if (fast) w = __expf(wl[i] - l_first) * vj[jb];            // u_i * v_j
-                    else w = __expf(fminf(wl[i] - lj[jb], 0.f)) * dtj[jb];
-                    const float dgh = (i >= j) ? w * pa[0][0][v] : 0.f;
-                    dG[0][jb][v] += dgh;
-                    const float pr = dgh * to_f32(sG[i * LDQ + j]);
-                    rsum[v] += pr;
-                    csum[jb] += pr;
-                }
-            }
-        }
-        int ri;
-        const float rtot = half_wave_reduce16(rsum, &ri);
-        if ((lane & 1) == 0) s_rs[(wave & 1) * kQ + rb * 32 + acc_row(lane, ri)] = rtot;
-#pragma unroll
-        for (int jb = 0; jb < 2; ++jb) {
-            const float cs = lane_xor_add<32>(csum[jb]);
-            if (lane < 32) s_cs[rb * kQ + (cb0 + jb) * 32 + lane] = cs;
-        }
-        __syncthreads();
-        if (tid < kQ) {
-            const float rs = s_rs[tid] + s_rs[kQ + tid];
-            const float cs = s_cs[tid] + s_cs[kQ + tid] + s_cs[2 * kQ + tid] + s_cs[3 * kQ + tid];
-            dl_diag[((b * nheads + h) * nchunks + c) * kQ + tid] = rs - cs;
-        }
-    }
-    if (!active) return;
-    float* out = dGp + (((b * nchunks + c) * ngroups + g) * nslices + slice) * (int64_t)(kQ * kQ);
-#pragma unroll
-    for (int jb = 0; jb < 2; ++jb) {
-        if (cb0 + jb > rb) continue;
-#pragma unroll
-        for (int v = 0; v < 16; ++v)
-            out[(rb * 32 + acc_row(lane, v)) * kQ + (cb0 + jb) * 32 + r] = dG[0][jb][v];
-    }
-}
-
-// ------------------------------------------------------------------------------------------
-// Off-diagonal (state) parts of dC and dB, heads of a slice reduced in registers, fp32 operands (16-bit ones: ssd_bwd16_kernel).
-// grid (nchunks, ngroups * nslices, batch), 512 threads.  Wave w owns rows rb = w >> 1 and state-column blocks
-// nb0 = (w & 1) * NB .. + NB - 1 of the [kQ][N] tile.
-//   SIDE_C:  dC[i][n] += e^{l_i} sum_p dy[i][p] S_prev[p][n];   dl_c[i] = C_i . (that head's contribution)
-//   SIDE_B:  dB[j][n] += dt_j e^{Lam - l_j} sum_p x[j][p] dS[p][n]
-// The row scale is applied in fp32 after the MFMA, so both operands are exact copies of the inputs.
-template <typename T, int P, int N, bool SIDE_C, int HS>
-__global__ void __launch_bounds__(512, SIDE_C ? 2 : 4)
-off_kernel(const T* __restrict__ Arow, int64_t Asb, int64_t Asl, int64_t Ash,      // dY (C side) or X (B side)
-           const float* __restrict__ ldtab,
-           const T* __restrict__ St,                                               // S_prev (C side) or dS (B side): [b][c][h][P][N]
-           const T* __restrict__ Cm, int64_t Csb, int64_t Csl, int64_t Csg,        // C side only
-           float* __restrict__ outp, float* __restrict__ dl_c,
-           int64_t seqlen, int64_t nheads, int64_t ngroups, int64_t nchunks, int64_t nslices, int64_t hps) {
-    static_assert(sizeof(T) == 4, "16-bit operands take ssd_bwd16_kernel");
-    constexpr int LDP = lds_ld<T>(P);
-    constexpr int NB = N / 64;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    float* wtab = reinterpret_cast<float*>(smem_raw);      // [8 waves][kQ]  row scale (wave-private)
-    float* s_rc = wtab + 8 * kQ;                           // [2][kQ]
-    T* sA = reinterpret_cast<T*>(s_rc + 2 * kQ);           // [kQ][LDP]
-    T* sT = sA + kQ * LDP;                                 // [N][LDP]   state tile transposed
-
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int r = lane & 31;
-    const int64_t c = blockIdx.x, b = blockIdx.z;
-    const int64_t g = blockIdx.y / nslices, slice = blockIdx.y % nslices;
-    const int64_t hpg = nheads / ngroups;
-    const int64_t t0 = c * kQ;
-    const int valid = (int)((seqlen - t0) < kQ ? (seqlen - t0) : kQ);
-    const int rb = wave >> 1, nb0 = (wave & 1) * NB;
-    float* ws = wtab + wave * kQ;
-
-    constexpr int LDN = lds_ld<T>(N);
-    T* sC = sT + N * LDP;                                  // C side: C [kQ][LDN], staged once for all heads
-    if (SIDE_C) stage_rows<T, kQ, N, 512, false>(sC, LDN, Cm + b * Csb + t0 * Csl + g * Csg, Csl, valid, nullptr, tid);
-    floatx16 acc[1][NB];
-    acc_zero(acc);
-
-    // the next head's row tile and state tile travel global -> registers while the current head is computed
-    constexpr int V = VecTraits<T>::kVec;
-    constexpr int VPR = P / V, NVA = kQ * VPR / 512;      // row tile: vectors per token row / per thread
-    constexpr int VPS = N / V, NVS = P * VPS / 512;       // state tile [P][N]: vectors per row / per thread
-    static_assert((kQ * VPR) % 512 == 0 && (P * VPS) % 512 == 0, "tile does not divide over the workgroup");
-    uint4 pa[NVA], ps[NVS];
-    auto prefetch = [&](int64_t h) {
-        const T* ga = Arow + b * Asb + t0 * Asl + head_off<HS>(h, Ash);
-#pragma unroll
-        for (int it = 0; it < NVA; ++it) {
-            const int e = it * 512 + tid, rr = e / VPR, cv = e % VPR;
-            pa[it] = rr < valid ? *reinterpret_cast<const uint4*>(ga + (int64_t)rr * Asl + cv * V) : uint4{0u, 0u, 0u, 0u};
-        }
-        const T* gs = St + ((b * nchunks + c) * nheads + h) * (int64_t)(P * N);
-#pragma unroll
-        for (int it = 0; it < NVS; ++it) {
-            // consecutive threads take consecutive state rows p of the same 16-byte column vector (see stage_transposed)
-            const int e = it * 512 + tid, cv = e / P, pr = e % P;
-            ps[it] = *reinterpret_cast<const uint4*>(gs + (int64_t)pr * N + cv * V);
-        }
-    };
-    constexpr bool PREFETCH = SIDE_C;
-    if (PREFETCH) prefetch(g * hpg + slice * hps);
-
-    for (int64_t hh = 0; hh < hps; ++hh) {
-        const int64_t h = g * hpg + slice * hps + hh;
-        float l0, l1, d0, d1;
-        wave_ld_load(ldtab, (b * nheads + h) * nchunks + c, l0, l1, d0, d1);
-        if (SIDE_C) { ws[lane] = __expf(l0); ws[lane + 64] = __expf(l1); }
-        else {
-            const float Lam = __shfl(l1, 63, 64);
-            ws[lane] = d0 * __expf(Lam - l0); ws[lane + 64] = d1 * __expf(Lam - l1);
-        }
-        __syncthreads();
-        if (!PREFETCH) prefetch(h);
-#pragma unroll
-        for (int it = 0; it < NVA; ++it) {
-            const int e = it * 512 + tid, rr = e / VPR, cv = e % VPR;
-            *reinterpret_cast<uint4*>(sA + rr * LDP + cv * V) = pa[it];
-        }
-#pragma unroll
-        for (int it = 0; it < NVS; ++it) {
-            const int e = it * 512 + tid, cv = e / P, pr = e % P;
-            const T* el = reinterpret_cast<const T*>(&ps[it]);
-#pragma unroll
-            for (int i = 0; i < V; ++i) sT[(cv * V + i) * LDP + pr] = el[i];
-        }
-        __syncthreads();
-        if (PREFETCH && hh + 1 < hps) prefetch(h + 1);
-        float rcv[16];
-#pragma unroll
-        for (int v = 0; v < 16; ++v) rcv[v] = 0.f;
-#pragma unroll
-        for (int jn = 0; jn < NB; ++jn) {
-            floatx16 tc[1][1];
-            acc_zero(tc);
-            wave_mma<1, 1>(tc, sA + rb * 32 * LDP, LDP, sT + (nb0 + jn) * 32 * LDP, LDP, 0, P);
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const float t = tc[0][0][v] * ws[rb * 32 + acc_row(lane, v)];
-                acc[0][jn][v] += t;
-                if (SIDE_C) {
-                    const int i = rb * 32 + acc_row(lane, v), n = (nb0 + jn) * 32 + r;
-                    rcv[v] += t * to_f32(sC[i * LDN + n]);
-                }
-            }
-        }
-        if (SIDE_C) {
-            int ri;
-            const float tot = half_wave_reduce16(rcv, &ri);
-            if ((lane & 1) == 0) s_rc[(wave & 1) * kQ + rb * 32 + acc_row(lane, ri)] = tot;
-            __syncthreads();
-            if (tid < kQ) dl_c[((b * nheads + h) * nchunks + c) * kQ + tid] = s_rc[tid] + s_rc[kQ + tid];
-        }
-    }
-    float* out = outp + (((b * nchunks + c) * ngroups + g) * nslices + slice) * (int64_t)(kQ * N);
-#pragma unroll
-    for (int jn = 0; jn < NB; ++jn)
-#pragma unroll
-        for (int v = 0; v < 16; ++v)
-            out[(rb * 32 + acc_row(lane, v)) * N + (nb0 + jn) * 32 + r] = acc[0][jn][v];
-}
 
 // Sum of the per-slice partials (fixed order) of up to three arrays in one launch.  One thread per float4;
 // `tile` floats per (group, slice) tile; segment k covers threads [first_k, first_{k+1}).
@@ -332,69 +71,6 @@ tail1_kernel(const DaArgs d, const int64_t n_da, const SliceSumArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------
-// Group-level finish for fp32 operands, one side per workgroup of 512 threads:  dC = dG B + sum dCoff  or
-// dB = dG^T C + sum dBoff  (dG and the off parts already summed over the head slices).
-template <typename T, int N>
-__device__ __forceinline__ void
-bc_final_body(const float* __restrict__ dGp, const float* __restrict__ dCp, const float* __restrict__ dBp,
-              const T* __restrict__ Bt, const T* __restrict__ Ct, T* __restrict__ dB, T* __restrict__ dC,
-              int64_t seqlen, int64_t ngroups, int64_t nchunks,
-              int64_t dBsb, int64_t dBsl, int64_t dBsg, int64_t dCsb, int64_t dCsl, int64_t dCsg, int64_t c, int64_t g, int64_t b,
-              const bool side_b) {
-    static_assert(sizeof(T) == 4, "16-bit operands take bc_final16_body");
-    constexpr int LDQ = lds_ld<T>(kQ);
-    constexpr int NB = N / 64;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    T* sA2 = reinterpret_cast<T*>(smem_raw);       // [kQ][LDQ]  dG (dC side) or its transpose (dB side)
-    T* sT2 = sA2 + kQ * LDQ;                       // [N][LDQ]   Bt or Ct
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int r = lane & 31;
-    const int64_t t0 = c * kQ;
-    const int valid = (int)((seqlen - t0) < kQ ? (seqlen - t0) : kQ);
-    const int rb = wave >> 1, cb0 = (wave & 1) * 2, nb0 = (wave & 1) * NB;
-    const int64_t grp = (b * nchunks + c) * ngroups + g;
-
-    // inputs are already summed over the head slices (slice_sum_body)
-    floatx16 dG[1][2], acc[1][NB];
-    acc_zero(dG);
-    {
-        const float* gp = dGp + grp * (int64_t)(kQ * kQ);
-        const float* op = (side_b ? dBp : dCp) + grp * (int64_t)(kQ * N);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int row = rb * 32 + acc_row(lane, v);
-#pragma unroll
-            for (int jb = 0; jb < 2; ++jb)
-                if (cb0 + jb <= rb) dG[0][jb][v] = gp[row * kQ + (cb0 + jb) * 32 + r];
-#pragma unroll
-            for (int jn = 0; jn < NB; ++jn) acc[0][jn][v] = op[row * N + (nb0 + jn) * 32 + r];
-        }
-    }
-    //   dC[i][n] += sum_{j<=i} dG[i][j] B[j][n]      (A = dG,   k = j in [0, 32 (rb + 1)) )
-    //   dB[j][n] += sum_{i>=j} dG[i][j] C[i][n]      (A = dG^T, k = i in [32 rb, kQ) )
-    const T* tile = (side_b ? Ct : Bt) + grp * (int64_t)(N * kQ);
-    stage_rows<T, N, kQ, 512, false>(sT2, LDQ, tile, kQ, N, nullptr, tid);
-    const int k0 = side_b ? rb * 32 : 0, k1 = side_b ? kQ : (rb + 1) * 32;
-#pragma unroll
-    for (int jb = 0; jb < 2; ++jb)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int i = rb * 32 + acc_row(lane, v), j = (cb0 + jb) * 32 + r;
-            sA2[side_b ? j * LDQ + i : i * LDQ + j] = dG[0][jb][v];
-        }
-    __syncthreads();
-    wave_mma<1, NB>(acc, sA2 + rb * 32 * LDQ, LDQ, sT2 + nb0 * 32 * LDQ, LDQ, k0, k1);
-    T* out = side_b ? dB + b * dBsb + t0 * dBsl + g * dBsg : dC + b * dCsb + t0 * dCsl + g * dCsg;
-    const int64_t osl = side_b ? dBsl : dCsl;
-#pragma unroll
-    for (int jn = 0; jn < NB; ++jn)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int row = rb * 32 + acc_row(lane, v), col = (nb0 + jn) * 32 + r;
-            if (row < valid) out[(int64_t)row * osl + col] = from_f32<T>(acc[0][jn][v]);
-        }
-}
-
 // Group-level finish for 16-bit operands, both sides in one workgroup of 8 waves, so that the head-summed dG is read once:
 //   waves 0-3 (row block w):      dC[i][n] = sum_{j<=i} dG[i][j] B[j][n] + dCoff[i][n]
 //   waves 4-7 (row block w - 4):  dB[j][n] = sum_{i>=j} dG[i][j] C[i][n] + dBoff[j][n]
@@ -537,8 +213,8 @@ __device__ __forceinline__ void ad_reduce_body(const float* __restrict__ dAp, co
 }
 
 // The group-level finish and the per-head reductions in one launch: the first workgroups run the group finish for
-// ([side,] chunk, group, batch) = the index split in that order (fp32 operands: side 0 dC, side 1 dB, one workgroup each;
-// 16-bit operands with BOTH: both sides in one workgroup), the others ad_reduce_body for one head each.
+// ([side,] chunk, group, batch) = the index split in that order (16-bit operands without BOTH: side 0 dC, side 1 dB, one workgroup
+// each), the others ad_reduce_body for one head each.
 constexpr int64_t kTail2BothFrom = 256;      // (batch, chunk, group) triples from which a workgroup takes both sides: one per CU
 struct Tail2Args {
     const float* dGp; const float* dCp; const float* dBp; const void* Bt; const void* Ct; void* dB; void* dC;
@@ -546,26 +222,35 @@ struct Tail2Args {
     const float* dAp; const float* dDp; const float* dbp; float* dA; float* dD; float* dbias;
     int64_t seqlen, ngroups, nchunks, batch, nheads, n_bc;
 };
+struct Tail2Args32 : Tail2Args {      // Bt, Ct: B and C as they lie
+    int64_t Bsb, Bsl, Bsg, Csb, Csl, Csg;
+};
 template <typename T, int N, bool BOTH>
 __global__ void __launch_bounds__(512)
 tail2_kernel(const Tail2Args a) {
     const int64_t blk = blockIdx.x;
     constexpr int SIDES = BOTH ? 1 : 2;
-    static_assert(!BOTH || sizeof(T) == 2, "both sides in one workgroup: 16-bit operands only");
     if (blk < SIDES * a.n_bc) {
         const int64_t q = blk / SIDES;
         const int64_t c = q % a.nchunks, g = (q / a.nchunks) % a.ngroups, b = q / (a.nchunks * a.ngroups);
-        if constexpr (sizeof(T) == 2) {
-            bc_final16_body<T, N, BOTH>(a.dGp, a.dCp, a.dBp, static_cast<const T*>(a.Bt), static_cast<const T*>(a.Ct), static_cast<T*>(a.dB),
-                                        static_cast<T*>(a.dC), a.seqlen, a.ngroups, a.nchunks, a.dBsb, a.dBsl, a.dBsg, a.dCsb, a.dCsl, a.dCsg, c, g,
-                                        b, (blk & 1) != 0);
-        } else {
-            bc_final_body<T, N>(a.dGp, a.dCp, a.dBp, static_cast<const T*>(a.Bt), static_cast<const T*>(a.Ct), static_cast<T*>(a.dB),
-                                static_cast<T*>(a.dC), a.seqlen, a.ngroups, a.nchunks, a.dBsb, a.dBsl, a.dBsg, a.dCsb, a.dCsl, a.dCsg, c, g, b,
-                                (blk & 1) != 0);
-        }
+        bc_final16_body<T, N, BOTH>(a.dGp, a.dCp, a.dBp, static_cast<const T*>(a.Bt), static_cast<const T*>(a.Ct), static_cast<T*>(a.dB),
+                                    static_cast<T*>(a.dC), a.seqlen, a.ngroups, a.nchunks, a.dBsb, a.dBsl, a.dBsg, a.dCsb, a.dCsl, a.dCsg, c, g,
+                                    b, (blk & 1) != 0);
     } else {
         ad_reduce_body(a.dAp, a.dDp, a.dbp, a.dA, a.dD, a.dbias, a.batch, a.nheads, a.nchunks, blk - SIDES * a.n_bc);
+    }
+}
+template <int N>
+__global__ void __launch_bounds__(512)
+tail2_32_kernel(const Tail2Args32 a) {
+    const int64_t blk = blockIdx.x;
+    if (blk < a.n_bc) {
+        const int64_t c = blk % a.nchunks, g = (blk / a.nchunks) % a.ngroups, b = blk / (a.nchunks * a.ngroups);
+        bc_final32_body<N>(a.dGp, a.dCp, a.dBp, static_cast<const float*>(a.Bt), a.Bsb, a.Bsl, a.Bsg, static_cast<const float*>(a.Ct), a.Csb, a.Csl, a.Csg,
+                           static_cast<float*>(a.dB), a.dBsb, a.dBsl, a.dBsg, static_cast<float*>(a.dC), a.dCsb, a.dCsl, a.dCsg, a.seqlen, a.ngroups,
+                           a.nchunks, c, g, b);
+    } else {
+        ad_reduce_body(a.dAp, a.dDp, a.dbp, a.dA, a.dD, a.dbias, a.batch, a.nheads, a.nchunks, blk - a.n_bc);
     }
 }
 
@@ -578,12 +263,8 @@ __global__ void copy_f32_kernel(const float* __restrict__ src, float* __restrict
     if (i < n) dst[i] = src ? src[i] : 0.f;
 }
 
-template <typename T, int P>
-size_t dg_smem() { return (size_t)(8 * kQ + 2 * kQ + 4 * kQ) * sizeof(float) + ((size_t)2 * kQ * lds_ld<T>(P) + (size_t)kQ * lds_ld<T>(kQ)) * sizeof(T); }
-template <typename T, int P, int N>
-size_t off_smem(bool side_c) { return (size_t)(8 * kQ + 2 * kQ) * sizeof(float) + ((size_t)(kQ + N) * lds_ld<T>(P) + (side_c ? (size_t)kQ * lds_ld<T>(N) : 0)) * sizeof(T); }
 template <typename T, int N>
-size_t bcf_smem() { return sizeof(T) == 2 ? (size_t)2 * kQ * kQ * sizeof(T) : (size_t)(kQ + N) * lds_ld<T>(kQ) * sizeof(T); }
+size_t bcf_smem() { return sizeof(T) == 2 ? (size_t)2 * kQ * kQ * sizeof(T) : finish32_smem<N>(); }
 
 template <typename T, int P, int N, int HS>
 int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
@@ -591,10 +272,8 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
     const SsdWorkspace w = ssd_carve(p, p->workspace, true);
     const int dt_f32 = p->dt_dtype == M2_F32;
     const T* x = static_cast<const T*>(p->x);
-    const T* Cm = static_cast<const T*>(p->C);
     const T* dy = static_cast<const T*>(p->dy);
     const dim3 grid_g((unsigned)nc, (unsigned)(p->ngroups * w.ns_g), (unsigned)p->batch);
-    const dim3 grid_c((unsigned)nc, (unsigned)(p->ngroups * w.ns_c), (unsigned)p->batch);
     const dim3 grid_b((unsigned)nc, (unsigned)(p->ngroups * w.ns_b), (unsigned)p->batch);
     M2_REQUIRE(p->nheads <= 65535, M2_ERR_SHAPE, "ssd_bwd: too many group slices");
     int rc;
@@ -610,22 +289,13 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
         if ((rc = check_launch("ssd state_pass16_kernel<reverse>"))) return rc;
     } else
     {   // fp32: local dS contributions (reuses the `local` region), then the reverse recurrence
-        auto k = chunk_state_kernel<T, P, N, true, HS>;
-        const size_t sm = state_smem<T, P, N>();
-        if ((rc = allow_smem(k, sm))) return rc;
-        int64_t ns, hps;
-        ssd_slicing(p, kWgsChunkState, false, &ns, &hps);
-        k<<<dim3((unsigned)nc, (unsigned)(p->ngroups * ns), (unsigned)p->batch), 256, sm, st>>>(
-            dy, w.ldtab, static_cast<const T*>(w.Ct), w.local, p->seqlen, p->nheads, p->ngroups, nc, ns, hps,
-            p->dy_stride_b, p->dy_stride_l, p->dy_stride_h);
-        if ((rc = check_launch("ssd chunk_state_kernel<dstate>"))) return rc;
-        state_scan_kernel<T, P * N, true><<<dim3((unsigned)p->nheads, (unsigned)p->batch, kScanSplit), 256, 0, st>>>(
-            w.local, w.lam, p->d_final_state, static_cast<T*>(w.dprev), p->d_initial_state,
-            static_cast<const T*>(w.prev), w.dlam, p->nheads, nc);
+        if ((rc = launch_chunk_state32<N, true, HS>(p, w, dy, p->dy_stride_b, p->dy_stride_l, p->dy_stride_h, p->C, p->C_stride_b, p->C_stride_l, p->C_stride_g, st))) return rc;
+        state_scan_kernel<P * N, true><<<dim3((unsigned)p->nheads, (unsigned)p->batch, kScanSplit), 256, 0, st>>>(
+            w.local, w.lam, p->d_final_state, static_cast<float*>(w.dprev), p->d_initial_state, p->nheads, nc);
         if ((rc = check_launch("ssd state_scan_kernel<reverse>"))) return rc;
     }
-    {
-        if constexpr (sizeof(T) == 2) {
+    if constexpr (sizeof(T) == 2) {
+        {
             auto k = dg16_kernel<T, P, HS>;
             const size_t sm = dg16_smem<P>();
             if ((rc = allow_smem(k, sm))) return rc;
@@ -633,18 +303,8 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
                                        p->seqlen, p->nheads, p->ngroups, nc, w.ns_g, w.hps_g,
                                        p->x_stride_b, p->x_stride_l, p->x_stride_h,
                                        p->dy_stride_b, p->dy_stride_l, p->dy_stride_h);
-        } else {
-            auto k = dg_kernel<T, P, HS>;
-            const size_t sm = dg_smem<T, P>();
-            if ((rc = allow_smem(k, sm))) return rc;
-            k<<<grid_g, 512, sm, st>>>(x, w.ldtab, dy, static_cast<const T*>(w.Gm), w.dGp, w.dl,
-                                       p->seqlen, p->nheads, p->ngroups, nc, w.ns_g, w.hps_g,
-                                       p->x_stride_b, p->x_stride_l, p->x_stride_h,
-                                       p->dy_stride_b, p->dy_stride_l, p->dy_stride_h);
+            if ((rc = check_launch("ssd dg16_kernel"))) return rc;
         }
-        if ((rc = check_launch("ssd dg_kernel"))) return rc;
-    }
-    if constexpr (sizeof(T) == 2) {
         Bwd16Args m{};
         m.ldtab = w.ldtab; m.D = p->D;
         m.Bm = p->B; m.B_sb = p->B_stride_b; m.B_sl = p->B_stride_l; m.B_sg = p->B_stride_g;
@@ -662,35 +322,24 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
         k<<<grid_b, 512, sm, st>>>(m);
         if ((rc = check_launch("ssd_bwd16_kernel"))) return rc;
     } else {
-        auto kc = off_kernel<T, P, N, true, HS>;
-        auto kb = off_kernel<T, P, N, false, HS>;
-        const size_t smc = off_smem<T, P, N>(true), sm = off_smem<T, P, N>(false);
-        if ((rc = allow_smem(kc, smc))) return rc;
-        if ((rc = allow_smem(kb, sm))) return rc;
-        kc<<<grid_c, 512, smc, st>>>(dy, p->dy_stride_b, p->dy_stride_l, p->dy_stride_h, w.ldtab,
-                                    static_cast<const T*>(w.prev), Cm, p->C_stride_b, p->C_stride_l, p->C_stride_g,
-                                    w.dCp, w.dlc, p->seqlen, p->nheads, p->ngroups, nc, w.ns_c, w.hps_c);
-        if ((rc = check_launch("ssd off_kernel<C>"))) return rc;
-        kb<<<grid_b, 512, sm, st>>>(x, p->x_stride_b, p->x_stride_l, p->x_stride_h, w.ldtab,
-                                    static_cast<const T*>(w.dprev), nullptr, 0, 0, 0,
-                                    w.dBp, nullptr, p->seqlen, p->nheads, p->ngroups, nc, w.ns_b, w.hps_b);
-        if ((rc = check_launch("ssd off_kernel<B>"))) return rc;
-        DiagArgs a{};
-        a.D = p->D;
-        a.Aoff = p->B; a.Ao_sb = p->B_stride_b; a.Ao_sl = p->B_stride_l; a.Ao_sg = p->B_stride_g;
-        a.Gd = w.Gmt; a.S = w.dprev;
-        a.Z = p->dy; a.Z_sb = p->dy_stride_b; a.Z_sl = p->dy_stride_l; a.Z_sh = p->dy_stride_h;
-        a.seqlen = p->seqlen; a.nheads = p->nheads; a.ngroups = p->ngroups; a.nchunks = nc;
-        ssd_slicing(p, 2, false, &a.nslices, &a.hps);
-        a.X = p->x; a.X_sb = p->x_stride_b; a.X_sl = p->x_stride_l; a.X_sh = p->x_stride_h;
-        a.dX = p->dx; a.dX_sb = p->dx_stride_b; a.dX_sl = p->dx_stride_l; a.dX_sh = p->dx_stride_h;
-        a.ldtab = w.ldtab;
-        a.dirp = w.dirp; a.rbp = w.rbp; a.dDp8 = w.dDp8;
-        auto k = diag_off_kernel<T, P, N, true, HS>;
-        const size_t smd = diag_smem<T, P, N, true>();
-        if ((rc = allow_smem(k, smd))) return rc;
-        k<<<dim3((unsigned)nc, (unsigned)(p->ngroups * a.nslices), (unsigned)p->batch), 256, smd, st>>>(a);
-        if ((rc = check_launch("ssd diag_off_kernel<bwd>"))) return rc;
+        Bwd32Args m{};
+        m.ldtab = w.ldtab; m.D = p->D;
+        m.Bm = static_cast<const float*>(p->B); m.B_sb = p->B_stride_b; m.B_sl = p->B_stride_l; m.B_sg = p->B_stride_g;
+        m.Cm = static_cast<const float*>(p->C); m.C_sb = p->C_stride_b; m.C_sl = p->C_stride_l; m.C_sg = p->C_stride_g;
+        m.Bt = static_cast<const float*>(w.Bt); m.Gm = static_cast<const float*>(w.Gm); m.Gmt = static_cast<const float*>(w.Gmt);
+        m.dS = static_cast<const float*>(w.dprev); m.Sprev = static_cast<const float*>(w.prev);
+        m.dy = dy; m.dy_sb = p->dy_stride_b; m.dy_sl = p->dy_stride_l; m.dy_sh = p->dy_stride_h;
+        m.x = x; m.x_sb = p->x_stride_b; m.x_sl = p->x_stride_l; m.x_sh = p->x_stride_h;
+        m.dx = static_cast<float*>(p->dx); m.dx_sb = p->dx_stride_b; m.dx_sl = p->dx_stride_l; m.dx_sh = p->dx_stride_h;
+        m.dB = static_cast<float*>(p->dB); m.dB_sb = p->dB_stride_b; m.dB_sl = p->dB_stride_l; m.dB_sg = p->dB_stride_g;
+        m.dC = static_cast<float*>(p->dC); m.dC_sb = p->dC_stride_b; m.dC_sl = p->dC_stride_l; m.dC_sg = p->dC_stride_g;
+        m.dGp = w.dGp; m.dBp = w.dBp; m.dCp = w.dCp; m.dirp = w.dirp; m.rbp = w.rbp; m.dl = w.dl; m.dlc = w.dlc; m.dDp8 = w.dDp8; m.dlam = w.dlam;
+        m.seqlen = p->seqlen; m.nheads = p->nheads; m.ngroups = p->ngroups; m.nchunks = nc; m.nslices = w.ns_b; m.hps = w.hps_b;
+        auto k = ssd_bwd32_kernel<N, HS>;
+        const size_t sm = bwd32_smem<N>();
+        if ((rc = allow_smem(k, sm))) return rc;
+        k<<<grid_b, 512, sm, st>>>(m);
+        if ((rc = check_launch("ssd_bwd32_kernel"))) return rc;
     }
     // the per-chunk scan that turns the per-token terms into ddt and dA partials runs with the slice sums below
     DaArgs da{};
@@ -712,27 +361,36 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
                 *use = out;
             };
             add(w.dGp, w.dGs, w.ns_g, (int64_t)kQ * kQ, 1, &gs);
-            add(w.dCp, w.dCs, w.ns_c, (int64_t)kQ * N, 0, &cs);
+            add(w.dCp, w.dCs, w.ns_b, (int64_t)kQ * N, 0, &cs);
             add(w.dBp, w.dBs, w.ns_b, (int64_t)kQ * N, 0, &bs);
             sa.total = first;
             const int64_t n_da = da_blocks(da), n_ss = ceil_div(first, (int64_t)(kDaHeads * 64));
             tail1_kernel<T><<<(unsigned)(n_da + n_ss), kDaHeads * 64, 0, st>>>(da, n_da, sa);
         }
         if ((rc = check_launch("ssd tail1_kernel"))) return rc;
-        // 16-bit operands: one workgroup per (batch, chunk, group) once those alone fill the chip, one per side below that
-        const bool both = sizeof(T) == 2 && ngrp >= kTail2BothFrom;
-        auto k = tail2_kernel<T, N, false>;
-        if constexpr (sizeof(T) == 2) { if (both) k = tail2_kernel<T, N, true>; }
-        const size_t sm = bcf_smem<T, N>();
-        if ((rc = allow_smem(k, sm))) return rc;
-        Tail2Args ta;
-        ta.dGp = gs; ta.dCp = cs; ta.dBp = bs; ta.Bt = w.Bt; ta.Ct = w.Ct; ta.dB = p->dB; ta.dC = p->dC;
+        // 16-bit operands: one workgroup per (batch, chunk, group) once those alone fill the chip, one per side below that; fp32
+        // operands: none where the main kernel has finished dB and dC
+        const bool both = sizeof(T) == 4 || ngrp >= kTail2BothFrom;
+        Tail2Args32 ta;
+        ta.dGp = gs; ta.dCp = cs; ta.dBp = bs; ta.Bt = sizeof(T) == 2 ? w.Bt : p->B; ta.Ct = sizeof(T) == 2 ? w.Ct : p->C; ta.dB = p->dB; ta.dC = p->dC;
+        ta.Bsb = p->B_stride_b; ta.Bsl = p->B_stride_l; ta.Bsg = p->B_stride_g; ta.Csb = p->C_stride_b; ta.Csl = p->C_stride_l; ta.Csg = p->C_stride_g;
         ta.dBsb = p->dB_stride_b; ta.dBsl = p->dB_stride_l; ta.dBsg = p->dB_stride_g;
         ta.dCsb = p->dC_stride_b; ta.dCsl = p->dC_stride_l; ta.dCsg = p->dC_stride_g;
         ta.dAp = w.dAp; ta.dDp = w.dDp; ta.dbp = w.dbp; ta.dA = p->dA; ta.dD = p->D ? p->dD : nullptr;
         ta.dbias = p->dt_bias ? p->d_dt_bias : nullptr;
-        ta.seqlen = p->seqlen; ta.ngroups = p->ngroups; ta.nchunks = nc; ta.batch = p->batch; ta.nheads = p->true_heads; ta.n_bc = ngrp;
-        k<<<(unsigned)((both ? 1 : 2) * ngrp + p->true_heads), 512, sm, st>>>(ta);
+        ta.seqlen = p->seqlen; ta.ngroups = p->ngroups; ta.nchunks = nc; ta.batch = p->batch; ta.nheads = p->true_heads;
+        ta.n_bc = sizeof(T) == 4 && w.ns_b == 1 ? 0 : ngrp;
+        const unsigned grid = (unsigned)((both ? 1 : 2) * ta.n_bc + p->true_heads);
+        const size_t sm = bcf_smem<T, N>();
+        if constexpr (sizeof(T) == 2) {
+            auto k = both ? tail2_kernel<T, N, true> : tail2_kernel<T, N, false>;
+            if ((rc = allow_smem(k, sm))) return rc;
+            k<<<grid, 512, sm, st>>>(ta);
+        } else {
+            auto k = tail2_32_kernel<N>;
+            if ((rc = allow_smem(k, sm))) return rc;
+            k<<<grid, 512, sm, st>>>(ta);
+        }
         if ((rc = check_launch("ssd tail2_kernel"))) return rc;
     }
     return M2_OK;

@@ -21,7 +21,7 @@
 // lane-pair swap per 4-channel group, without a pass through LDS.
 // All eight waves also form   dlam[c] = e^{Lam_c} <dS, S_prev>   (the part of dL/dLam_c that flows through the carried
 // state) from the two tiles as they lie in LDS, one partial per wave.
-// The decay is factorised per row block around its LAST token (see ssd_diag.hpp), with the exact per-element
+// The decay is factorised per row block around its LAST token (see ssd_y.hpp), with the exact per-element
 // fallback when the block's range exceeds kMaxRange.  ddt and dA need a scan over the chunk and are left to da_body (tail1_kernel).
 #pragma once
 #include "ssd_y.hpp"
@@ -462,12 +462,18 @@ __device__ __forceinline__ void da_body(const DaArgs& q, int64_t blk) {
     if (h < nheads) {      // wave-uniform
         const int64_t bhc = (b * nheads + h) * nchunks + c;
         const float Ah = A[h];
-        float xa = 0.f, xb = 0.f, ra = 0.f, rbv = 0.f, dira = 0.f, dirb = 0.f, dlm = 0.f, dDs = 0.f;
+        constexpr bool SCANNED = sizeof(T) == 4;      // dl_diag comes scanned from ssd_bwd32_kernel
+        float xa = 0.f, xb = 0.f, ga = 0.f, gb = 0.f, ra = 0.f, rbv = 0.f, dira = 0.f, dirb = 0.f, dlm = 0.f, dDs = 0.f;
         const int nv = 1 << q.hs;
         for (int v = 0; v < nv; ++v) {
             const int64_t k = ((b * nheads + h) * nv + v) * nchunks + c;
-            xa += dl_diag[k * kQ + ta] + dl_c[k * kQ + ta];
-            xb += dl_diag[k * kQ + tb] + dl_c[k * kQ + tb];
+            if constexpr (SCANNED) {
+                ga += dl_diag[k * kQ + ta]; gb += dl_diag[k * kQ + tb];
+                xa += dl_c[k * kQ + ta]; xb += dl_c[k * kQ + tb];
+            } else {
+                xa += dl_diag[k * kQ + ta] + dl_c[k * kQ + ta];
+                xb += dl_diag[k * kQ + tb] + dl_c[k * kQ + tb];
+            }
             ra += rbp[k * kQ + ta]; rbv += rbp[k * kQ + tb];
             dira += dirp[k * kQ + ta]; dirb += dirp[k * kQ + tb];
 #pragma unroll
@@ -488,7 +494,7 @@ __device__ __forceinline__ void da_body(const DaArgs& q, int64_t blk) {
         xb += __shfl(xa, 63, 64);
         xa += (ya - ra) + __shfl(yb, 0, 64);
         xb += yb - rbv;
-        const float da_a = xa + dlm, da_b = xb + dlm;
+        const float da_a = SCANNED ? xa + ga + dlm : xa + dlm, da_b = SCANNED ? xb + gb + dlm : xb + dlm;
         float dAl = 0.f, dbl = 0.f;
         float va = 0.f, vb = 0.f;
         if (ta < valid) {

@@ -8,8 +8,8 @@
 //   1. prep_kernel         l = cumsum(A dt) per (b, head, chunk);  G = C B^T (+ operand tiles) per (b, chunk, group)
 //   2. states entering the chunks, final state
 //        16-bit: state_pass16_kernel   contributions B^T (decay o dt o X) and recurrence fused, per (b, head)
-//        fp32  : chunk_state_kernel + state_scan_kernel
-//   3. ssd_y16_kernel (16-bit) / diag_off_kernel<false>      Y = (L o G)(dt o X) + e^l C S_prev + D X   MFMA
+//        fp32  : chunk_state32_kernel + state_scan_kernel
+//   3. ssd_y16_kernel / ssd_y32_kernel      Y = (L o G)(dt o X) + e^l C S_prev + D X   MFMA
 //
 // Extensions over the reference kernel: optional initial state, final-state output, any batch,
 // ragged sequence length (tokens past the end behave as dt = 0 and are never written).
@@ -31,13 +31,13 @@ int ssd_fwd_impl(const SsdCall* p, hipStream_t st) {
     const SsdWorkspace w = ssd_carve(p, p->workspace, false);
     int rc;
     if ((rc = ssd_launch_states<T, P, N, HS>(p, w, p->final_state, true, p->chunk_states != nullptr, st))) return rc;
-    DiagArgs a{};
+    YArgs a{};
     a.D = p->D;
     a.Aoff = p->C; a.Ao_sb = p->C_stride_b; a.Ao_sl = p->C_stride_l; a.Ao_sg = p->C_stride_g;
     a.Gd = w.Gm; a.S = w.prev; a.ldtab = w.ldtab;
     a.Z = p->x; a.Z_sb = p->x_stride_b; a.Z_sl = p->x_stride_l; a.Z_sh = p->x_stride_h;
     a.seqlen = p->seqlen; a.nheads = p->nheads; a.ngroups = p->ngroups; a.nchunks = nc;
-    ssd_slicing(p, kWgsY, false, &a.nslices, &a.hps);
+    ssd_slicing(p, sizeof(T) == 2 ? kWgsY : kWgsY32, false, &a.nslices, &a.hps);
     a.Y = p->y; a.Y_sb = p->y_stride_b; a.Y_sl = p->y_stride_l; a.Y_sh = p->y_stride_h;
     M2_REQUIRE(p->ngroups * a.nslices <= 65535, M2_ERR_SHAPE, "ssd_fwd: too many group slices");
     const dim3 grid((unsigned)nc, (unsigned)(p->ngroups * a.nslices), (unsigned)p->batch);
@@ -48,11 +48,11 @@ int ssd_fwd_impl(const SsdCall* p, hipStream_t st) {
         k<<<grid, 256, sm, st>>>(a);
         return check_launch("ssd_y16_kernel");
     } else {
-    auto k = diag_off_kernel<T, P, N, false, HS>;
-    const size_t sm = diag_smem<T, P, N, false>();
-    if ((rc = allow_smem(k, sm))) return rc;
-    k<<<grid, 256, sm, st>>>(a);
-    return check_launch("ssd diag_off_kernel<fwd>");
+        auto k = ssd_y32_kernel<N, HS>;
+        const size_t sm = y32_smem<N>();
+        if ((rc = allow_smem(k, sm))) return rc;
+        k<<<grid, 512, sm, st>>>(a);
+        return check_launch("ssd_y32_kernel");
     }
 }
 

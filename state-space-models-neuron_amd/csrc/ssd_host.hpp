@@ -1,10 +1,10 @@
 // Host-side helpers shared by the SSD forward and backward launchers.
 #pragma once
 #include "ssd_kernels.hpp"
-#include "ssd_diag.hpp"
 #include "ssd_bwd_main.hpp"
 #include "ssd_dg.hpp"
 #include "ssd_states16.hpp"
+#include "ssd_f32.hpp"
 
 namespace m2 {
 
@@ -31,7 +31,7 @@ struct SsdWorkspace {
     float* dAp = nullptr; float* dDp = nullptr; float* dBp = nullptr; float* dCp = nullptr; float* dl = nullptr; float* dlc = nullptr; float* dGp = nullptr;
     float* dGs = nullptr; float* dBs = nullptr; float* dCs = nullptr;   // partials summed over the head slices
     float* dirp = nullptr; float* rbp = nullptr; float* dDp8 = nullptr; // per channel-half / per-wave partials of the dx kernel
-    int64_t ns_g = 1, hps_g = 1, ns_c = 1, hps_c = 1, ns_b = 1, hps_b = 1;   // head slicing of the dg / off<C> / off<B> kernels
+    int64_t ns_g = 1, hps_g = 1, ns_b = 1, hps_b = 1;   // head slicing of dg16 and of the main backward kernel
     size_t bytes = 0;
     size_t kept_bytes = 0;              // size of the forward -> backward carry-over (chunk_states buffer)
 };
@@ -59,7 +59,23 @@ inline void ssd_slicing(const SsdCall* p, int wgs_per_cu, bool partials, int64_t
     *nslices = best;
     *hps = hpg / best;
 }
-constexpr int kWgsChunkState = 2, kWgsY = 2, kWgsDx = 1, kWgsDg = 1, kWgsOffC = 1, kWgsOffB = 2;
+constexpr int kWgsChunkState32 = 2, kWgsY = 2, kWgsY32 = 1, kWgsDx = 1, kWgsDg = 1;
+
+// The same for the backward of fp32 operands, whose heads take four times as long (15 us): in heads, rounds of workgroups x (heads
+// per slice + one for the way in and the finish), and for more than one slice the partials' way out, back and through kernels of
+// their own.
+inline void ssd_slicing32(const SsdCall* p, int64_t* nslices, int64_t* hps) {
+    const int64_t hpg = p->nheads / p->ngroups, base = p->batch * ceil_div(p->seqlen, (int64_t)kQ) * p->ngroups;
+    int64_t best = 1;
+    float least = 1e30f;
+    for (int64_t s = 1; s <= hpg; ++s) {
+        if (hpg % s) continue;
+        const float cost = (float)ceil_div(base * s, device_cus()) * ((float)(hpg / s) + 1.f) + (s > 1 ? 1.f + 0.007f * (float)(base * s) : 0.f);
+        if (cost < least) { least = cost; best = s; }
+    }
+    *nslices = best;
+    *hps = hpg / best;
+}
 
 inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_only = false) {
     const int64_t nc = ceil_div(p->seqlen, (int64_t)kQ);
@@ -92,17 +108,13 @@ inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_
         w.Gm = keep(grp * kQ * kQ * esz);
         w.Gmt = keep(grp * kQ * kQ * esz);
         w.Bt = keep(grp * p->dstate * kQ * esz);
-        w.Ct = keep(grp * p->dstate * kQ * esz);
+        if (p->dtype != M2_F32) w.Ct = keep(grp * p->dstate * kQ * esz);
         w.kept_bytes = koff;
     }
     if (bwd) {
         ssd_slicing(p, kWgsDg, true, &w.ns_g, &w.hps_g);
-        ssd_slicing(p, kWgsOffC, true, &w.ns_c, &w.hps_c);
-        ssd_slicing(p, kWgsOffB, true, &w.ns_b, &w.hps_b);
-        if (p->dtype != M2_F32) {       // the main backward kernel produces both state parts there
-            ssd_slicing(p, kWgsDx, true, &w.ns_b, &w.hps_b);
-            w.ns_c = w.ns_b; w.hps_c = w.hps_b;
-        }
+        ssd_slicing(p, kWgsDx, true, &w.ns_b, &w.hps_b);
+        if (p->dtype == M2_F32) { ssd_slicing32(p, &w.ns_b, &w.hps_b); w.ns_g = w.ns_b; w.hps_g = w.hps_b; }      // one kernel for all three
         w.dprev = take(tiles * esz);
         w.dlam = reinterpret_cast<float*>(take(bhc * 4 * kDlamParts));
         w.dAp = reinterpret_cast<float*>(take(bhc * 4));
@@ -116,7 +128,7 @@ inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_
         w.dGp = reinterpret_cast<float*>(take((size_t)p->batch * nc * p->ngroups * w.ns_g * kQ * kQ * 4));
         const size_t part = (size_t)p->batch * nc * p->ngroups * kQ * p->dstate * 4;
         w.dBp = reinterpret_cast<float*>(take(part * w.ns_b));
-        w.dCp = reinterpret_cast<float*>(take(part * w.ns_c));
+        w.dCp = reinterpret_cast<float*>(take(part * w.ns_b));
         w.dGs = reinterpret_cast<float*>(take((size_t)p->batch * nc * p->ngroups * kQ * kQ * 4));
         w.dBs = reinterpret_cast<float*>(take((size_t)p->batch * nc * p->ngroups * kQ * p->dstate * 4));
         w.dCs = reinterpret_cast<float*>(take((size_t)p->batch * nc * p->ngroups * kQ * p->dstate * 4));
@@ -155,8 +167,6 @@ inline int ssd_check(const m2_ssd_params* p, const char* who) {
     return M2_OK;
 }
 
-template <typename T, int P, int N>
-inline size_t state_smem() { return (size_t)(P + N) * lds_ld<T>(kQ) * sizeof(T); }
 template <typename T>
 inline size_t cb_smem(int n) {      // operand rows; 32 tokens of both to transpose; the waves' blocks on their way out
     const size_t a = (size_t)2 * 64 * lds_ld<T>(cb_kh<T>(n)) * sizeof(T), b = (size_t)2 * 32 * lds_ld<T>(n) * sizeof(T), o = (size_t)4 * 32 * 36 * 4;
@@ -177,6 +187,23 @@ inline int launch_state_pass16(const StatePassArgs& a, int64_t batch, hipStream_
     return launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, SPLIT>, state_pass_smem<P, N, HILO, SPLIT>(), SPLIT);
 }
 
+// Local chunk states of fp32 operands: X = x, M = B, or (DSTATE) dy and C.
+template <int N, bool DSTATE, int HS>
+inline int launch_chunk_state32(const SsdCall* p, const SsdWorkspace& w, const void* X, int64_t X_sb, int64_t X_sl, int64_t X_sh, const void* M, int64_t M_sb,
+                                int64_t M_sl, int64_t M_sg, hipStream_t st) {
+    auto k = chunk_state32_kernel<N, DSTATE, HS>;
+    if (const int rc = allow_smem(k, chunk_state32_smem<N>())) return rc;
+    ChunkState32Args a;
+    a.X = static_cast<const float*>(X); a.X_sb = X_sb; a.X_sl = X_sl; a.X_sh = X_sh;
+    a.M = static_cast<const float*>(M); a.M_sb = M_sb; a.M_sl = M_sl; a.M_sg = M_sg;
+    a.ldtab = w.ldtab; a.out = w.local;
+    a.seqlen = p->seqlen; a.nheads = p->nheads; a.ngroups = p->ngroups; a.nchunks = ceil_div(p->seqlen, (int64_t)kQ);
+    ssd_slicing(p, kWgsChunkState32, false, &a.nslices, &a.hps);
+    M2_REQUIRE(p->ngroups * a.nslices <= 65535, M2_ERR_SHAPE, "ssd: too many group slices");
+    k<<<dim3((unsigned)a.nchunks, (unsigned)(p->ngroups * a.nslices), (unsigned)p->batch), chunk_state32_threads<N>(), chunk_state32_smem<N>(), st>>>(a);
+    return check_launch("ssd chunk_state32_kernel");
+}
+
 // Decay tables, G = C B^T (+ operand tiles), local chunk states, forward state scan.  Used by the forward and, when the
 // caller did not keep the forward's chunk_states buffer, by the backward (recompute).  for_fwd, for_bwd: which of the operand
 // tiles will be read.
@@ -194,8 +221,8 @@ inline int ssd_launch_states(const SsdCall* p, const SsdWorkspace& w, float* fin
         const size_t sm = cb_smem<T>(N);
         if ((rc = allow_smem(k, sm))) return rc;
         PrepArgs pa;
-        pa.Bm = Bm; pa.Cm = Cm; pa.Bt = w.Bt;
-        pa.Gf = for_bwd ? w.G : nullptr; pa.Gmt = for_bwd ? w.Gmt : nullptr; pa.Ct = for_bwd ? w.Ct : nullptr;
+        pa.Bm = Bm; pa.Cm = Cm; pa.Bt = sizeof(T) == 2 || for_bwd ? w.Bt : nullptr; pa.parts = pa.Bt ? kCbParts : kCbGParts;
+        pa.Gf = for_bwd ? w.G : nullptr; pa.Gmt = for_bwd ? w.Gmt : nullptr; pa.Ct = for_bwd && sizeof(T) == 2 ? w.Ct : nullptr;
         pa.Gm = for_fwd || sizeof(T) == 4 ? w.Gm : nullptr;
         pa.Bsb = p->B_stride_b; pa.Bsl = p->B_stride_l; pa.Bsg = p->B_stride_g;
         pa.Csb = p->C_stride_b; pa.Csl = p->C_stride_l; pa.Csg = p->C_stride_g;
@@ -203,7 +230,7 @@ inline int ssd_launch_states(const SsdCall* p, const SsdWorkspace& w, float* fin
         pa.dtsb = p->dt_stride_b; pa.dtsl = p->dt_stride_l;
         pa.seqlen = p->seqlen; pa.nheads = p->true_heads; pa.hs = p->hs; pa.ngroups = p->ngroups; pa.nchunks = nc;
         pa.n_cb = nc * p->ngroups * p->batch;
-        const int64_t blocks = cb_blocks(pa.n_cb) + ld_table_blocks(p->batch, p->true_heads, nc);
+        const int64_t blocks = cb_blocks(pa.n_cb, pa.parts) + ld_table_blocks(p->batch, p->true_heads, nc);
         M2_REQUIRE(blocks < ((int64_t)1 << 31), M2_ERR_SHAPE, "ssd: too many workgroups");
         k<<<(unsigned)blocks, 256, sm, st>>>(pa);
         if ((rc = check_launch("ssd prep_kernel"))) return rc;
@@ -221,19 +248,10 @@ inline int ssd_launch_states(const SsdCall* p, const SsdWorkspace& w, float* fin
         if ((rc = hilo ? launch_state_pass16<T, P, N, false, HS, true>(sa, p->batch, st) : launch_state_pass16<T, P, N, false, HS, false>(sa, p->batch, st))) return rc;
         return check_launch("ssd state_pass16_kernel");
     } else {
-        // fp32 operands: per-chunk contributions (fp32, workspace), then the recurrence over the chunks
-        auto k = chunk_state_kernel<T, P, N, false, HS>;
-        const size_t sm = state_smem<T, P, N>();
-        if ((rc = allow_smem(k, sm))) return rc;
-        int64_t ns, hps;
-        ssd_slicing(p, kWgsChunkState, false, &ns, &hps);
-        M2_REQUIRE(p->ngroups * ns <= 65535, M2_ERR_SHAPE, "ssd: too many group slices");
-        k<<<dim3((unsigned)nc, (unsigned)(p->ngroups * ns), (unsigned)p->batch), 256, sm, st>>>(
-            x, w.ldtab, static_cast<const T*>(w.Bt), w.local, p->seqlen, p->nheads, p->ngroups, nc, ns, hps,
-            p->x_stride_b, p->x_stride_l, p->x_stride_h);
-        if ((rc = check_launch("ssd chunk_state_kernel"))) return rc;
-        state_scan_kernel<T, P * N, false><<<dim3((unsigned)p->nheads, (unsigned)p->batch, kScanSplit), 256, 0, st>>>(
-            w.local, w.lam, p->initial_state, static_cast<T*>(w.prev), final_out, nullptr, nullptr, p->nheads, nc);
+        // fp32 operands: per-chunk contributions (workspace), then the recurrence over the chunks
+        if ((rc = launch_chunk_state32<N, false, HS>(p, w, p->x, p->x_stride_b, p->x_stride_l, p->x_stride_h, Bm, p->B_stride_b, p->B_stride_l, p->B_stride_g, st))) return rc;
+        state_scan_kernel<P * N, false><<<dim3((unsigned)p->nheads, (unsigned)p->batch, kScanSplit), 256, 0, st>>>(
+            w.local, w.lam, p->initial_state, static_cast<float*>(w.prev), final_out, p->nheads, nc);
         if ((rc = check_launch("ssd state_scan_kernel"))) return rc;
         return M2_OK;
     }

@@ -13,12 +13,10 @@
 // which the hardware deals round-robin to the 8 XCDs, still share B/C/G tiles of one batch
 // row through the MALL, and each XCD's L2 sees whole (head, chunk) tiles):
 //   prep_kernel        decay tables per (batch, head, chunk); G = C B^T and the operand tiles per (batch, chunk, group)
-//   chunk_state_kernel local chunk state  sum_j scale_j x_j (x) B_j -> workspace, fp32
-//                      (DSTATE variant: sum_i e^{l_i} dy_i (x) C_i for the backward)
-//   state_scan_kernel  sequential-in-chunks, parallel-in-(b,h,p,n) fp32 recurrence; writes the
-//                      state ENTERING each chunk in the MFMA operand type, and the final state
-//                      (REVERSE variant: gradient recurrence + <dS, S> per chunk)
-// The last two serve fp32 operands; for 16-bit operands ssd_states16.hpp does both in one pass.
+//   state_scan_kernel  sequential-in-chunks, parallel-in-(b,h,p,n) fp32 recurrence over the chunks' own contributions
+//                      (chunk_state32_kernel); writes the state ENTERING each chunk, and the final state
+//                      (REVERSE variant: the gradient recurrence).  fp32 operands only; for 16-bit operands
+//                      ssd_states16.hpp forms the contributions and the recurrence in one pass.
 #pragma once
 #include <type_traits>
 
@@ -33,26 +31,30 @@ namespace m2 {
 //   Gm  [kQ][kQ] T               causal G:  G[i][j] for i >= j, else 0         (forward diagonal term, rows i)
 //   Gmt [kQ][kQ] T               its transpose: Gmt[j][i] = G[i][j] for i >= j (backward dx term, rows j)
 //   (each of Gf, Gm, Gmt and Ct only where it is not null: the forward alone reads Gm and Bt)
-//   Bt, Ct N x kQ T              B and C transposed (tokens contiguous), laid out by mt_offset: MFMA operands of the
-//                                chunk-state products
+//   Bt, Ct N x kQ T              (16-bit) B and C transposed, laid out by mt_offset: MFMA operands of the chunk-state products
+// fp32 operands: Gm and Gmt (and, where the backward will run, a copy of B in Bt) in the order in which a wave takes its operand
+// rows, op32_offset; no Gf, Ct.
 // kCbParts workgroups of 256 threads per (chunk, group, batch), see cb_body.  The upper-right 64x64 quadrant of G is
 // never consumed and is neither computed nor written.
-// Element offset of the 8 tokens s0 .. s0 + 7 (s0 a multiple of 8) of state column n inside a transposed B / C tile.
-//   fp32   : [N][kQ], tokens contiguous (rows staged into LDS by chunk_state_kernel);
-//   16-bit : MFMA operand order [N / 32][kQ / 16][64 lanes][8]: the B-operand fragment of a wave for column block n / 32
-//            and k-step s0 / 16 is one contiguous KiB, lane = 32 ((s0 / 8) & 1) + n % 32 (read by state_pass16_kernel
-//            straight into registers, eight full cache lines per load instruction).
-template <typename T>
+// Element offset of the 8 tokens s0 .. s0 + 7 (s0 a multiple of 8) of state column n inside a transposed B / C tile: MFMA operand
+// order [N / 32][kQ / 16][64 lanes][8], so that the B-operand fragment of a wave for column block n / 32 and k-step s0 / 16 is one
+// contiguous KiB, lane = 32 ((s0 / 8) & 1) + n % 32 (read by state_pass16_kernel straight into registers, eight full cache lines
+// per load instruction).
 __device__ __forceinline__ int64_t mt_offset(int n, int s0) {
-    if (sizeof(T) == 2) return ((int64_t)((n >> 5) * (kQ / 16) + (s0 >> 4)) * 64 + ((s0 >> 3) & 1) * 32 + (n & 31)) * 8;
-    return (int64_t)n * kQ + s0;
+    return ((int64_t)((n >> 5) * (kQ / 16) + (s0 >> 4)) * 64 + ((s0 >> 3) & 1) * 32 + (n & 31)) * 8;
 }
 
+// The four elements k = 16 (u / 2) + 8 half + 4 (u % 2) + 0..3 of operand row 32 rb + r, fp32: step u of row block rb is one contiguous
+// KiB, lane 32 half + r (a step straight from rows touches 32 of them, 2 x 16 bytes each: the loads of B and of C B^T then held the
+// phase of ssd_bwd32_kernel that needs them for 23 k cycles instead of 13).
+template <int STEPS>
+__device__ __forceinline__ int op32_offset(int rb, int u, int lane) { return ((rb * STEPS + u) * 64 + lane) * 4; }
+
 // Workgroups per (chunk, group, batch): three for the 64x64 quadrants of G on and below the diagonal, four for the
-// transposed tiles (32 tokens each) -- seven short independent pieces rather than two long ones.
-constexpr int kCbParts = 7;
+// transposed tiles or the copy of B (32 tokens each; none without Bt) -- seven short independent pieces rather than two long ones.
+constexpr int kCbParts = 7, kCbGParts = 3;
 constexpr int kXcds = 8;
-__host__ __device__ inline int64_t cb_blocks(int64_t n_cb) { return (n_cb + kXcds - 1) / kXcds * kXcds * kCbParts; }
+__host__ __device__ inline int64_t cb_blocks(int64_t n_cb, int parts) { return (n_cb + kXcds - 1) / kXcds * kXcds * parts; }
 // Contraction length staged at once: all of it (one staging phase, one barrier), but fp32 rows of 128 in two halves, so that
 // four workgroups fit a CU and not two (66 -> 51 us at b3 l2048 h32 g8).
 template <typename T> __host__ __device__ constexpr int cb_kh(int n) { return sizeof(T) == 4 && n > 64 ? n / 2 : n; }
@@ -74,9 +76,22 @@ cb_body(const T* __restrict__ Bm, const T* __restrict__ Cm, float* __restrict__ 
     const T* Bp = Bm + b * Bsb + t0 * Bsl + g * Bsg;
     const T* Cp = Cm + b * Csb + t0 * Csl + g * Csg;
     const int64_t grp = (b * nchunks + c) * ngroups + g;
-    if (part >= 3) {
+    if constexpr (sizeof(T) == 4) {
+        if (part >= kCbGParts) {
+            const int rb = part - kCbGParts, r = lane & 31, row = rb * 32 + r;
+            const T* src = Bp + (int64_t)(row < valid ? row : valid - 1) * Bsl + 8 * (lane >> 5);
+#pragma unroll
+            for (int it = 0; it < N / 32; ++it) {
+                const int u = it * 4 + wave;
+                *reinterpret_cast<floatx4*>(Bt + grp * (int64_t)(N * kQ) + op32_offset<N / 8>(rb, u, lane)) =
+                    *reinterpret_cast<const floatx4*>(src + (u >> 1) * 16 + 4 * (u & 1));
+            }
+            return;
+        }
+    }
+    if (sizeof(T) == 2 && part >= kCbGParts) {
         // transposed copies of tokens [tk0, tk0 + 32): thread -> (state column n, group of V tokens)
-        const int tk0 = (part - 3) * 32;
+        const int tk0 = (part - kCbGParts) * 32;
         constexpr int LDT = lds_ld<T>(N);
         T* sBt = sC + 32 * LDT;
         T* Btp = Bt + grp * (int64_t)(N * kQ);
@@ -89,11 +104,11 @@ cb_body(const T* __restrict__ Bm, const T* __restrict__ Cm, float* __restrict__ 
             T v[V];
 #pragma unroll
             for (int q = 0; q < V; ++q) v[q] = sBt[(s0 + q) * LDT + n];
-            *reinterpret_cast<uint4*>(Btp + mt_offset<T>(n, tk0 + s0)) = *reinterpret_cast<const uint4*>(v);
+            *reinterpret_cast<uint4*>(Btp + mt_offset(n, tk0 + s0)) = *reinterpret_cast<const uint4*>(v);
             if (Ct) {
 #pragma unroll
                 for (int q = 0; q < V; ++q) v[q] = sC[(s0 + q) * LDT + n];
-                *reinterpret_cast<uint4*>(Ctp + mt_offset<T>(n, tk0 + s0)) = *reinterpret_cast<const uint4*>(v);
+                *reinterpret_cast<uint4*>(Ctp + mt_offset(n, tk0 + s0)) = *reinterpret_cast<const uint4*>(v);
             }
         }
         return;
@@ -122,6 +137,26 @@ cb_body(const T* __restrict__ Bm, const T* __restrict__ Cm, float* __restrict__ 
     for (int v = 0; v < 16; ++v) blk[acc_row(lane, v) * LDG + acc_col(lane)] = acc[0][0][v];
     wave_lds_sync();
     const int i0 = wm * 64 + wi * 32, j0 = wn * 64 + wj * 32;      // first row, first column of the block
+    if constexpr (sizeof(T) == 4) {
+        const int r = lane & 31, k8 = 8 * (lane >> 5), I = i0 / 32, J = j0 / 32;
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+            const int k = 16 * (it >> 1) + k8 + 4 * (it & 1);
+            if (Gm) {
+                floatx4 v = *reinterpret_cast<const floatx4*>(blk + r * LDG + k);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = i0 + r >= j0 + k + e ? v[e] : 0.f;
+                *reinterpret_cast<floatx4*>(Gm + grp * (int64_t)(kQ * kQ) + op32_offset<16>(I, 4 * J + it, lane)) = v;
+            }
+            if (Gmt) {
+                floatx4 v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = i0 + k + e >= j0 + r ? blk[(k + e) * LDG + r] : 0.f;
+                *reinterpret_cast<floatx4*>(Gmt + grp * (int64_t)(kQ * kQ) + op32_offset<16>(J, 4 * I + it, lane)) = v;
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
         const int a = it * 8 + (lane >> 3), k0 = (lane & 7) * 4;   // row of the output, first of its four elements
@@ -144,7 +179,8 @@ cb_body(const T* __restrict__ Bm, const T* __restrict__ Cm, float* __restrict__ 
 
 // ------------------------------------------------------------------------------------------
 // Cumulative log-decay table per (batch, head, chunk): ldtab[bhc] = [ l[0..kQ) | dt[0..kQ) ] in fp32,
-// l = inclusive cumsum of A_h dt within the chunk, lam[bhc] = l[kQ-1].  Every other kernel reads this table instead
+// l = inclusive cumsum of A_h dt within the chunk, lam[bhc] = l[kQ-1]; tokens past the end of the sequence hold dt = 0 and the last
+// l.  Every other kernel reads this table instead
 // of gathering dt (stride = nheads elements) and scanning it again per head.  A workgroup takes eight consecutive heads of
 // one (batch, chunk), two per wave: dt is [b][l][h], so two threads per token fetch 8 (fp32: 16) bytes each and hand them
 // to the waves through LDS.  These workgroups are chains of latencies that hold the shared memory of a cb_body workgroup, so
@@ -227,140 +263,54 @@ ld_table_body(const void* __restrict__ dt, int dt_f32, const float* __restrict__
 }
 
 // Both preparations in one launch (they are independent, and either alone leaves most of the GPU idle): the first
-// cb_blocks(n_cb) workgroups run cb_body, the others ld_table_body.
+// cb_blocks workgroups run cb_body, the others ld_table_body.
 struct PrepArgs {
     const void* Bm; const void* Cm; float* Gf; void* Gm; void* Gmt; void* Bt; void* Ct;
     int64_t Bsb, Bsl, Bsg, Csb, Csl, Csg;
     const void* dt; int dt_f32; const float* dt_bias; const float* A; float* ldtab; float* lam; int64_t dtsb, dtsl;
     int64_t seqlen, nheads, ngroups, nchunks, n_cb;      // nheads: true heads
-    int hs;
+    int hs, parts;                                       // parts: kCbParts, or kCbGParts without Bt
 };
 template <typename T, int N>
 __global__ void __launch_bounds__(256)
 prep_kernel(const PrepArgs a) {
     const int64_t blk = blockIdx.x;
-    if (blk < cb_blocks(a.n_cb)) {
+    const int parts = sizeof(T) == 2 ? kCbParts : a.parts;
+    if (blk < cb_blocks(a.n_cb, parts)) {
         // The parts of one (chunk, group, batch) read the same rows.  Workgroups are dealt round-robin to the XCDs, so the
         // parts are kXcds apart: one L2 then fetches those rows once, where seven neighbours would each fetch their own.
-        const int64_t u = blk / kXcds, q = u / kCbParts * kXcds + blk % kXcds;
+        const uint32_t u = (uint32_t)blk / kXcds;
+        const int64_t q = (int64_t)(u / parts) * kXcds + blk % kXcds;
         if (q >= a.n_cb) return;
         const int64_t c = q % a.nchunks, g = (q / a.nchunks) % a.ngroups, b = q / (a.nchunks * a.ngroups);
         cb_body<T, N>(static_cast<const T*>(a.Bm), static_cast<const T*>(a.Cm), a.Gf, static_cast<T*>(a.Gm), static_cast<T*>(a.Gmt),
                       static_cast<T*>(a.Bt), static_cast<T*>(a.Ct), a.seqlen, a.ngroups, a.nchunks,
-                      a.Bsb, a.Bsl, a.Bsg, a.Csb, a.Csl, a.Csg, c, g, b, (int)(u % kCbParts));
+                      a.Bsb, a.Bsl, a.Bsg, a.Csb, a.Csl, a.Csg, c, g, b, (int)(u % parts));
     } else {
-        ld_table_body<T>(a.dt, a.dt_f32, a.dt_bias, a.A, a.ldtab, a.lam, a.seqlen, a.nheads, a.nchunks, a.dtsb, a.dtsl, a.hs, blk - cb_blocks(a.n_cb));
+        ld_table_body<T>(a.dt, a.dt_f32, a.dt_bias, a.A, a.ldtab, a.lam, a.seqlen, a.nheads, a.nchunks, a.dtsb, a.dtsl, a.hs, blk - cb_blocks(a.n_cb, parts));
     }
 }
 
 // ------------------------------------------------------------------------------------------
-// Local chunk state.  grid (nchunks, ngroups * nslices, batch), 256 threads; a workgroup loops over `hps` heads.
-//   DSTATE == false:  out[p][n] = sum_j (dt_j e^{Lam-l_j}) x[j][p] * B[j][n]      (forward)
-//   DSTATE == true :  out[p][n] = sum_i e^{l_i} dy[i][p] * C[i][n]                (backward)
-// Used for fp32 operands (16-bit operands take state_pass16_kernel, which fuses this with the recurrence); `out` is fp32.
-// `X` is x or dy; `Mt` is the group's B or C tile already transposed to [N][kQ] (tokens contiguous) by cb_body (prep_kernel),
-// staged into LDS once per workgroup.  Per head only the x tile moves: it is loaded 16 bytes at a time, scaled in
-// fp32 and written transposed; the next head's tile is prefetched into registers while the MFMAs run.
-template <typename T, int P, int N, bool DSTATE, int HS>
-__global__ void __launch_bounds__(256)
-chunk_state_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
-                   const T* __restrict__ Mt, float* __restrict__ out,
-                   int64_t seqlen, int64_t nheads, int64_t ngroups, int64_t nchunks, int64_t nslices, int64_t hps,
-                   int64_t Xsb, int64_t Xsl, int64_t Xsh) {
-    constexpr int LD = lds_ld<T>(kQ);
-    constexpr int V = VecTraits<T>::kVec;
-    constexpr int NIT = (P / V) / 2;              // 16-byte vectors per thread per head (thread <-> fixed token)
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    T* sX = reinterpret_cast<T*>(smem_raw);        // [P][LD]   x^T scaled
-    T* sM = sX + P * LD;                           // [N][LD]   B^T or C^T
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int64_t c = blockIdx.x, b = blockIdx.z;
-    const int64_t g = blockIdx.y / nslices, slice = blockIdx.y % nslices;
-    const int64_t hpg = nheads / ngroups;
-    const int64_t t0 = c * kQ;
-    const int valid = (int)((seqlen - t0) < kQ ? (seqlen - t0) : kQ);
-    const int tok = tid & (kQ - 1), cvh = tid >> 7;       // this thread's token and channel-vector parity
-
-    stage_rows<T, N, kQ, 256, false>(sM, LD, Mt + ((b * nchunks + c) * ngroups + g) * (int64_t)(N * kQ), kQ, N, nullptr, tid);
-
-    constexpr int BM = P / 64, BN = N / 64;
-    const int wm = wave >> 1, wn = wave & 1;
-    uint4 pre[NIT];
-    auto prefetch = [&](int64_t h) {
-        const T* xp = X + b * Xsb + (t0 + tok) * Xsl + head_off<HS>(h, Xsh);
-#pragma unroll
-        for (int it = 0; it < NIT; ++it)
-            pre[it] = tok < valid ? *reinterpret_cast<const uint4*>(xp + (it * 2 + cvh) * V) : uint4{0u, 0u, 0u, 0u};
-    };
-    prefetch(g * hpg + slice * hps);
-
-    for (int64_t hh = 0; hh < hps; ++hh) {
-        const int64_t h = g * hpg + slice * hps + hh;
-        float l0, l1, d0, d1;
-        wave_ld_load(ldtab, (b * nheads + h) * nchunks + c, l0, l1, d0, d1);
-        const float Lam = __shfl(l1, 63, 64);
-        // scale of this thread's token (token = lane + 64 * (wave & 1))
-        const float lt = (wave & 1) ? l1 : l0, dtt = (wave & 1) ? d1 : d0;
-        const float sc = DSTATE ? __expf(lt) : dtt * __expf(Lam - lt);
-        __syncthreads();                     // previous head's MFMAs are done with sX
-#pragma unroll
-        for (int it = 0; it < NIT; ++it) {
-            const T* el = reinterpret_cast<const T*>(&pre[it]);
-#pragma unroll
-            for (int i = 0; i < V; ++i) sX[((it * 2 + cvh) * V + i) * LD + tok] = from_f32<T>(to_f32(el[i]) * sc);
-        }
-        __syncthreads();
-        if (hh + 1 < hps) prefetch(h + 1);
-
-        floatx16 acc[BM][BN];
-        acc_zero(acc);
-        wave_mma<BM, BN>(acc, sX + wm * (P / 2) * LD, LD, sM + wn * (N / 2) * LD, LD, 0, kQ);
-        float* op = out + ((b * nchunks + c) * nheads + h) * (int64_t)(P * N);
-#pragma unroll
-        for (int i = 0; i < BM; ++i)
-#pragma unroll
-            for (int j = 0; j < BN; ++j)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int row = wm * (P / 2) + i * 32 + acc_row(lane, v);
-                    const int col = wn * (N / 2) + j * 32 + acc_col(lane);
-                    op[row * N + col] = acc[i][j][v];
-                }
-    }
-}
-
-// ------------------------------------------------------------------------------------------
-// Inter-chunk recurrence.  grid (nheads, batch, kScanSplit), 256 threads; a workgroup owns 1/kScanSplit of the
+// Inter-chunk recurrence, fp32 operands.  grid (nheads, batch, kScanSplit), 256 threads; a workgroup owns 1/kScanSplit of the
 // [p][n] state of one (batch, head), each thread EPT float4 slices of it, and walks the chunks with the running
-// state in registers (fp32).  The split only exists to put enough waves on the GPU to hide memory latency.
+// state in registers.  The split only exists to put enough waves on the GPU to hide memory latency.
 //
 // forward (REVERSE == false):
-//     run = init;  for c = 0..nc-1:  prev[c] = T(run);  run = e^{lam_c} run + local[c];  final = run
+//     run = init;  for c = 0..nc-1:  prev[c] = run;  run = e^{lam_c} run + local[c];  final = run
 // reverse (REVERSE == true), the gradient recurrence:
-//     run = dfinal;  for c = nc-1..0:  prev[c] = T(run)   (= dL/dS_new(c));
-//                                      dlam[c][split] = e^{lam_c} <run, sprev[c]> over this workgroup's part
-//                                      (sprev[c] = the forward state entering chunk c);
-//                                      run = e^{lam_c} run + local[c]
-//     dinit = run.
-// dlam is the part of dL/dLam_c that flows through the carried state only.  The part through the chunk's own
-// tokens is added by the consumer as a PREFIX sum of per-token terms; forming it here as <run, S_new(c)> and
-// subtracting a suffix sum there would cancel two large numbers rounded differently (operand-type copies of
-// the states), leaving an error that is constant over the chunk and accumulates in dA.
+//     run = dfinal;  for c = nc-1..0:  prev[c] = run   (= dL/dS_new(c));  run = e^{lam_c} run + local[c];  dinit = run.
 constexpr int kScanSplit = 4;
-constexpr int kDlamParts = 8;     // partial sums of dlam per (batch, head, chunk): every producer fills all of them
+constexpr int kDlamParts = 8;     // partial sums of dlam per (batch, head, chunk), one per wave of the main backward kernel
 
-template <typename T, int PN, bool REVERSE>
+template <int PN, bool REVERSE>
 __global__ void __launch_bounds__(256)
 state_scan_kernel(const float* __restrict__ local, const float* __restrict__ lam, const float* __restrict__ init,
-                  T* __restrict__ prev, float* __restrict__ final_out,
-                  const T* __restrict__ sprev, float* __restrict__ dlam,
-                  int64_t nheads, int64_t nchunks) {
+                  float* __restrict__ prev, float* __restrict__ final_out, int64_t nheads, int64_t nchunks) {
     constexpr int EPT = PN / 4 / 256 / kScanSplit;
     static_assert(PN % (1024 * kScanSplit) == 0, "state size must be a multiple of 4096 elements");
     const int part0 = blockIdx.z * (PN / kScanSplit);      // first element of this workgroup's part
-    constexpr int kRedBatch = 64;
-    __shared__ float red[kRedBatch * 4];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x;
     const int64_t h = blockIdx.x, b = blockIdx.y;
     const int64_t bh = b * nheads + h;
     floatx4 run[EPT];
@@ -374,46 +324,13 @@ state_scan_kernel(const float* __restrict__ local, const float* __restrict__ lam
         const int64_t c = REVERSE ? nchunks - 1 - cc : cc;
         const int64_t tile = ((b * nchunks + c) * nheads + h) * (int64_t)PN;
         const float dec = __expf(lam[bh * nchunks + c]);
-        float dot = 0.f;
 #pragma unroll
         for (int e = 0; e < EPT; ++e) {
             const int off = part0 + (e * 256 + tid) * 4;
-            float loc[4];
-            loadv<float, 4>(local + tile + off, loc);
-            // store the state entering (forward) / the gradient leaving (reverse) this chunk
-            T o[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) o[q] = from_f32<T>(run[e][q]);
-            if (sizeof(T) == 2) *reinterpret_cast<uint2*>(prev + tile + off) = *reinterpret_cast<const uint2*>(o);
-            else *reinterpret_cast<uint4*>(prev + tile + off) = *reinterpret_cast<const uint4*>(o);
-            if (REVERSE) {
-                // state that ENTERED this chunk in the forward pass (operand type, as the other kernels consume it)
-                T tv[4];
-                if (sizeof(T) == 2) *reinterpret_cast<uint2*>(tv) = *reinterpret_cast<const uint2*>(sprev + tile + off);
-                else *reinterpret_cast<uint4*>(tv) = *reinterpret_cast<const uint4*>(sprev + tile + off);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) dot += run[e][q] * to_f32(tv[q]);
-            }
+            const floatx4 loc = *reinterpret_cast<const floatx4*>(local + tile + off);
+            *reinterpret_cast<floatx4*>(prev + tile + off) = run[e];
 #pragma unroll
             for (int q = 0; q < 4; ++q) run[e][q] = dec * run[e][q] + loc[q];
-        }
-        if (REVERSE) {
-            // per-wave partial of e^{Lam} <dS, S_prev>; the four partials are combined once per kRedBatch chunks so
-            // the streaming loop has no barrier
-            dot = warp_sum(dot) * dec;
-            if (lane == 0) red[(cc % kRedBatch) * 4 + wave] = dot;
-            if ((cc % kRedBatch) == kRedBatch - 1 || cc == nchunks - 1) {
-                __syncthreads();
-                const int64_t first = cc - (cc % kRedBatch);
-                if (tid <= cc - first) {
-                    const int64_t c2 = REVERSE ? nchunks - 1 - (first + tid) : first + tid;
-                    {
-                        dlam[(bh * nchunks + c2) * kDlamParts + blockIdx.z] = red[tid * 4] + red[tid * 4 + 1] + red[tid * 4 + 2] + red[tid * 4 + 3];
-                        dlam[(bh * nchunks + c2) * kDlamParts + kScanSplit + blockIdx.z] = 0.f;
-                    }
-                }
-                __syncthreads();
-            }
         }
     }
     if (final_out) {

@@ -2,8 +2,14 @@
 //
 //     y[i][p] = u_i * ( e^{l_ref} sum_n C[i][n] S_prev[p][n]  +  sum_{j<=i} (G[i][j] v_j) x[j][p] )  +  D x[i][p]
 //
-// (same factorised decay as ssd_diag.hpp: u_i = e^{l_i - l_ref}, v_j = e^{l_ref - l_j} dt_j per 32-token row block,
-// exact per-element fallback when a block's range exceeds kMaxRange).
+// Decay.  e^{l_i - l_j} is factorised per 32-token row block around a reference token inside the block:
+//   forward  (ref = first token of the block):  e^{l_i-l_j} dt_j = u_i * v_j,   u_i = e^{l_i-l_ref} <= 1,
+//             v_j = e^{l_ref-l_j} dt_j;   for j inside the block v_j <= e^{R}, R = l_first - l_last of the block
+//   backward (ref = last token of the block):   e^{l_i-l_j} = v_i * u_j,        u_j = e^{l_ref-l_j} <= 1, v_i = e^{l_i-l_ref}
+// so the decay costs ONE multiply per operand element (v, applied to the register fragment) plus one per output
+// row (u) instead of an exp per element.  R <= 32 * max|A dt| (51 for A = -16, dt = 0.1); if a block's range
+// exceeds kMaxRange the wave falls back to evaluating e^{l_i-l_j} on the difference, element by element,
+// which cannot overflow (the reference always does that, mamba2/mamba2_kernel.py:32-33).
 //
 // A workgroup (4 waves, wave w owns token rows 32w..32w+31) handles one chunk of one group and loops over `hps`
 // heads.  The two tiles a head needs -- S_prev [P][N] and x [128][P] -- are copied global -> LDS by the
@@ -21,9 +27,24 @@
 // output block): decay scales and the D x term are lane-local, and after one lane-pair swap per 4-channel group
 // (v_permlane32_swap) y leaves in 16-byte row-contiguous stores, rounded once, without a pass through LDS.
 #pragma once
-#include "ssd_diag.hpp"
+#include "ssd_kernels.hpp"
 
 namespace m2 {
+
+constexpr float kMaxRange = 80.f;
+
+struct YArgs {
+    const float* D;
+    const float* ldtab;         // [b][h][c][ l kQ | dt kQ ]
+    const void* Aoff;           // C: [b][l][g][N]
+    int64_t Ao_sb, Ao_sl, Ao_sg;
+    const void* Gd;             // causal C B^T: [b][c][g][kQ][kQ]
+    const void* S;              // states entering the chunks: [b][c][h][P][N]
+    const void* Z;              // x: [b][l][h][P]
+    int64_t Z_sb, Z_sl, Z_sh;
+    int64_t seqlen, nheads, ngroups, nchunks, nslices, hps;
+    void* Y; int64_t Y_sb, Y_sl, Y_sh;
+};
 
 #define M2_LDS __attribute__((address_space(3)))
 #define M2_GLB __attribute__((address_space(1)))
@@ -117,7 +138,7 @@ constexpr size_t y16_smem() {
 
 template <typename T, int P, int N, int HS>
 __global__ void __launch_bounds__(256, (y16_smem<P, N>() <= 80 * 1024 ? 2 : 1))
-ssd_y16_kernel(const DiagArgs a) {
+ssd_y16_kernel(const YArgs a) {
     static_assert(sizeof(T) == 2, "16-bit operands only");
     constexpr int BN = P / 32, KSN = N / 16;
     constexpr int SPR_S = N / 8, SPR_X = P / 8;            // 16-byte slots per row

@@ -294,3 +294,26 @@ def test_ssd_softplus_folded_into_scan(dtype, b, l, h, p, n, g):
         # dA, like d_dt_bias, is a signed sum over all tokens (here with step sizes from 1e-2 up to 11, beyond the threshold)
         assert err(dA.cpu(), lv["A"].grad) < (5e-4 if dtype == torch.float32 else tol)
         assert torch.equal(gbuf[..., :24], torch.full((b, l, 24), 5.0, dtype=dtype, device=DEV))
+
+
+@pytest.mark.parametrize("steps", ["usual", "long"])
+@pytest.mark.parametrize("b,l,h,p,n,g", [
+    (16, 129, 16, 64, 128, 4),     # four heads one after the other in a workgroup, which finishes dB and dC itself; one token in the last chunk
+    (16, 130, 32, 64, 64, 4),      # two slices of four heads: partial sums and the separate finish
+    (1, 161, 3, 64, 128, 1),       # slices of a single head
+    (16, 160, 8, 128, 64, 4)])     # wide heads as pairs; a row block that is exactly full
+def test_ssd_fp32_heads_in_sequence(b, l, h, p, n, g, steps):
+    """fp32 kernels: several heads per workgroup, both ways to finish dB and dC, and (long steps) decay ranges beyond the factorised form."""
+    from mamba2.mamba2_kernel import alloc_chunk_states, ssd_backward, ssd_forward
+    d = make_ssd_inputs(b, l, h, p, n, g, seed=l + h)
+    if steps == "long":
+        d["dt"][..., ::3] *= 40.0          # A dt down to -64 per token: past kMaxRange within a row block
+    r = ssd_grads_ref(*(_f64(d)[k] for k in ("dt", "A", "X", "B", "C", "D", "dy")), chunk=64)
+    dd = _dev(d)
+    st = alloc_chunk_states(dd["dt"], dd["A"], dd["X"], dd["B"], dd["C"])
+    y, _ = ssd_forward(dd["dt"], dd["A"], dd["X"], dd["B"], dd["C"], dd["D"], chunk_states=st)
+    assert rel_err(y, r["y"]) < 1e-4
+    for states in (st, None):
+        out = ssd_backward(dd["dt"], dd["A"], dd["X"], dd["B"], dd["C"], dd["D"], dd["dy"], chunk_states=states)
+        for name, v in zip(("ddt", "dA", "dX", "dB", "dC", "dD"), out):
+            assert rel_err(v, r[name]) < 1e-4, name
