@@ -92,6 +92,9 @@ int m2_conv1d_fwd(const m2_conv1d_params* p, void* stream);
 int m2_conv1d_prefill(const m2_conv1d_params* p, void* conv_state, int32_t W, int32_t continuing, void* stream);
 size_t m2_conv1d_bwd_workspace_bytes(int64_t batch, int64_t seqlen, int64_t channels, int32_t k);
 int m2_conv1d_bwd(const m2_conv1d_params* p, void* stream);
+/* The same without its last sum where the kernel leaves partials: *slots > 0 rows of channels x (4 + 1) floats at the start of the
+ * workspace, which m2_param_sums adds up into dw and db; *slots == 0: dw and db are complete. */
+int m2_conv1d_bwd_partial(const m2_conv1d_params* p, int64_t* slots, void* stream);
 
 /* ------------------------------------------------------------------ SSD scan
  * dt (b,l,h), A (h) fp32, x (b,l,h,p), B,C (b,l,g,n), D (h) fp32 or NULL,
@@ -236,6 +239,8 @@ int m2_rmsnorm_gated_fwd(const m2_rmsnorm_params* p, void* stream);
 int m2_rmsnorm_gated_fwd_check(const m2_rmsnorm_params* p);      /* what it would refuse, without the work */
 size_t m2_rmsnorm_gated_bwd_workspace_bytes(int64_t rows, int64_t channels, int32_t n_groups, int32_t dtype);
 int m2_rmsnorm_gated_bwd(const m2_rmsnorm_params* p, void* stream);
+/* The same without the sum of d_weight: *rows partial rows of `channels` floats are left at the start of the workspace. */
+int m2_rmsnorm_gated_bwd_partial(const m2_rmsnorm_params* p, int64_t* rows, void* stream);
 
 /* Block boundary of the token-by-token loop (mamba2/modeling_mamba2.py:133-140 Mamba2Block.step's residual add,
  * followed by the next block's -- or the final -- Mamba2RMSNorm, :94-103), in one pass over the rows:
@@ -298,12 +303,20 @@ int m2_product(const m2_product_params* p, void* stream);
  * m2_mixer_params:       out (3 * nheads + channels) fp32 = [ -exp(A_log) | D | dt_bias | norm_weight ].
  * m2_mixer_params_grads: dA, dD, d_dt_bias (nheads) and d_norm_weight (channels) fp32 into the parameters' own types;
  *                        the gradient of A_log is dA * A with A the first nheads values of m2_mixer_params' out.
+ * m2_param_sums:         the sums behind a backward, in one launch: `norm_rows` partial rows of `channels` floats
+ *                        (m2_rmsnorm_gated_bwd_partial) into d_norm, the conv's partials (m2_conv1d_bwd_partial) into dw and db,
+ *                        dA (times A, if A is given), dD and d_dt_bias into their parameters' types.  channels == 0,
+ *                        conv_slots == 0, nheads == 0: without that part.
  * D may be NULL (then so is its gradient, and out's second part is unset).  *_dtype: M2_F32 or M2_BF16. */
 int m2_mixer_params(const void* A_log, int32_t A_dtype, const void* D, int32_t D_dtype, const void* dt_bias, int32_t dt_bias_dtype,
                     const void* norm_weight, int32_t norm_dtype, float* out, int64_t nheads, int64_t channels, void* stream);
 int m2_mixer_params_grads(const float* A, const float* dA, const float* dD, const float* d_dt_bias, const float* d_norm_weight,
                           void* dA_log, int32_t A_dtype, void* dD_out, int32_t D_dtype, void* d_dt_bias_out, int32_t dt_bias_dtype,
                           void* d_norm_out, int32_t norm_dtype, int64_t nheads, int64_t channels, void* stream);
+int m2_param_sums(const float* norm_partial, int64_t norm_rows, int64_t channels, void* d_norm, int32_t norm_dtype, const float* conv_partial,
+                  int64_t conv_slots, int64_t conv_channels, void* dw, void* db, int32_t conv_dtype, int64_t nheads, const float* A,
+                  const float* dA, const float* dD, const float* d_dt_bias, void* dA_out, int32_t A_dtype, void* dD_out, int32_t D_dtype,
+                  void* d_dt_bias_out, int32_t dt_bias_dtype, void* stream);
 
 /* ------------------------------------------------------------------ self tests / probes
  * m2_mfma_selftest: C (M x N fp32, row-major) = A (M x K) * Bt (N x K)^T through the same

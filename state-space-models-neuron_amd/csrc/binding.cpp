@@ -28,10 +28,10 @@ using torch::autograd::variable_list;
 
 // ----------------------------------------------------------------------------------------------- the library
 #define M2_BOUND(F) \
-    F(m2_last_error) F(m2_conv1d_fwd) F(m2_conv1d_prefill) F(m2_conv1d_bwd_workspace_bytes) F(m2_conv1d_bwd) F(m2_ssd_chunk_states_bytes) \
+    F(m2_last_error) F(m2_conv1d_fwd) F(m2_conv1d_prefill) F(m2_conv1d_bwd_workspace_bytes) F(m2_conv1d_bwd) F(m2_conv1d_bwd_partial) F(m2_ssd_chunk_states_bytes) \
     F(m2_ssd_fwd_workspace_bytes) F(m2_ssd_fwd_check) F(m2_ssd_fwd) F(m2_ssd_bwd_workspace_bytes) F(m2_ssd_bwd) F(m2_decode_workspace_bytes) \
     F(m2_decode_step) F(m2_decode_step_static) F(m2_rmsnorm_gated_fwd_check) F(m2_rmsnorm_gated_fwd) F(m2_rmsnorm_gated_bwd_workspace_bytes) \
-    F(m2_rmsnorm_gated_bwd) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_rows) F(m2_decode_layer) F(m2_mixer_params) F(m2_mixer_params_grads) \
+    F(m2_rmsnorm_gated_bwd) F(m2_rmsnorm_gated_bwd_partial) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_rows) F(m2_decode_layer) F(m2_mixer_params) F(m2_param_sums) \
     F(m2_product_pays) F(m2_product_workspace_bytes) F(m2_product)
 struct Lib {
 #define M2_FIELD(name) decltype(&::name) name = nullptr;
@@ -145,9 +145,12 @@ Tensor conv1d_forward(const Tensor& input, const Tensor& weight, const OptTensor
     return y;
 }
 
-// the launch shared by the operator and the fused core; returns (dw, db)
+// Partial rows of a parameter's gradient, to be summed by a later launch (count == 0: there are none)
+struct Partials { Tensor rows; int64_t count = 0; };
+
+// the launch shared by the operator and the fused core; returns (dw, db).  later: where partials go that the caller will have summed
 std::pair<Tensor, Tensor> launch_conv_bwd(const Strided& x, const Tensor& weight, const Tensor& bias, const Strided& dy, const Strided& dx,
-                                          int64_t b, int64_t l, int64_t c, const Tensor& like, int activation, void* stream) {
+                                          int64_t b, int64_t l, int64_t c, const Tensor& like, int activation, void* stream, Partials* later = nullptr) {
     const Tensor w = weight.contiguous(), bi = bias.defined() ? bias.contiguous() : bias;
     Tensor dw = at::empty(w.sizes(), w.options()), db = bi.defined() ? at::empty(bi.sizes(), bi.options()) : Tensor();
     m2_conv1d_params p = conv_params(x, w, bi, dy, b, l, c, dtype_code(like), activation);
@@ -156,7 +159,10 @@ std::pair<Tensor, Tensor> launch_conv_bwd(const Strided& x, const Tensor& weight
     p.workspace_bytes = lib.m2_conv1d_bwd_workspace_bytes(b, l, c, p.k);
     const Tensor ws = scratch(p.workspace_bytes, like);
     p.workspace = ptr(ws);
-    check(lib.m2_conv1d_bwd(&p, stream), "m2_conv1d_bwd");
+    if (later) {
+        check(lib.m2_conv1d_bwd_partial(&p, &later->count, stream), "m2_conv1d_bwd");
+        later->rows = ws;
+    } else check(lib.m2_conv1d_bwd(&p, stream), "m2_conv1d_bwd");
     return {dw, db};
 }
 
@@ -419,8 +425,9 @@ Tensor rmsnorm_forward(const Tensor& x, const OptTensor& z, const Tensor& weight
     return norm.out;
 }
 
-std::tuple<Tensor, Tensor, Tensor> rmsnorm_backward(const Tensor& x_, const OptTensor& z_, const Tensor& weight, const Tensor& d_out, int64_t n_groups,
-                                                    double eps, const OptTensor& out_dz) {
+// later: where the partial rows of dw go that the caller will have summed (dw is then undefined)
+std::tuple<Tensor, Tensor, Tensor> launch_norm_bwd(const Tensor& x_, const OptTensor& z_, const Tensor& weight, const Tensor& d_out, int64_t n_groups,
+                                                   double eps, const OptTensor& out_dz, Partials* later) {
     require_gpu({&x_, &or_none(z_), &weight, &d_out});
     check_norm(x_, or_none(z_));
     Scope scope(x_);
@@ -437,17 +444,24 @@ std::tuple<Tensor, Tensor, Tensor> rmsnorm_backward(const Tensor& x_, const OptT
         dz = out_dz && vec_ok(*out_dz) ? *out_dz : at::empty(x.sizes(), x.options());
         p.dz = ptr(dz); p.dz_stride_row = rows2d(dz, "out_dz").stride;
     }
-    Tensor dw = empty_f32({x.size(-1)}, x);
-    p.d_weight = ptr<float>(dw);
+    Tensor dw;
+    if (!later) { dw = empty_f32({x.size(-1)}, x); p.d_weight = ptr<float>(dw); }
     p.workspace_bytes = lib.m2_rmsnorm_gated_bwd_workspace_bytes(p.rows, p.channels, p.n_groups, p.dtype);
     const Tensor ws = scratch(p.workspace_bytes, x);
     p.workspace = ptr(ws);
-    check(lib.m2_rmsnorm_gated_bwd(&p, scope.stream), "m2_rmsnorm_gated_bwd");
+    if (later) {
+        check(lib.m2_rmsnorm_gated_bwd_partial(&p, &later->count, scope.stream), "m2_rmsnorm_gated_bwd");
+        later->rows = ws;
+    } else check(lib.m2_rmsnorm_gated_bwd(&p, scope.stream), "m2_rmsnorm_gated_bwd");
     if (z.defined() && out_dz && !dz.is_same(*out_dz)) {
         out_dz->copy_(dz);
         dz = *out_dz;
     }
     return {dx, dw, dz};
+}
+std::tuple<Tensor, Tensor, Tensor> rmsnorm_backward(const Tensor& x, const OptTensor& z, const Tensor& weight, const Tensor& d_out, int64_t n_groups,
+                                                    double eps, const OptTensor& out_dz) {
+    return launch_norm_bwd(x, z, weight, d_out, n_groups, eps, out_dz, nullptr);
 }
 
 struct NormFn : torch::autograd::Function<NormFn> {
@@ -559,18 +573,24 @@ CoreOut core_forward(const Packed& k, const Tensor& A, const Tensor& D, const Te
     return r;
 }
 
+// types that the kernels for the small parameters read and write
+bool casts(const Tensor& t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16; }
+
 struct CoreGrads { Tensor zx, A, D, conv_w, conv_b, dt_bias, norm_w; };
 // The packed gradient has rows of whole 128-byte cache lines (10576 columns of bf16 are 165.25 lines, and every wave-wide
 // access to a column slice of such a buffer straddles two lines in three rows out of four); its consumers take a leading
 // dimension.
+// The sums of the norm weight's and the conv's partials run in one launch at the end, the former into norm_param's type; with
+// head_grads (of A_log, D and dt_bias, in their types) it also leaves those.
 CoreGrads core_backward(const Packed& k, const Tensor& d_out, const Tensor& A, const Tensor& D, const Tensor& conv_w, const Tensor& conv_b,
-                        const Tensor& dt_bias, const Tensor& norm_w, const Tensor& conv_out, const Tensor& scan_out, const Tensor& states, void* stream) {
+                        const Tensor& dt_bias, const Tensor& norm_w, const Tensor& conv_out, const Tensor& scan_out, const Tensor& states,
+                        const Tensor& norm_param, const variable_list& head_grads, void* stream) {
     CoreGrads r;
+    Partials norm_rows, conv_rows;
     const int64_t width = k.zx.size(2), per_line = 128 / k.zx.element_size(), pitch = (width + per_line - 1) / per_line * per_line;
     r.zx = at::empty({k.b, k.l, pitch}, k.zx.options());
     if (pitch != width) r.zx = r.zx.narrow(2, 0, width);
-    auto [d_scan, d_norm_w, dz] = rmsnorm_backward(scan_out, k.z(), norm_w, d_out, k.g, kNormEps, r.zx.narrow(2, 0, k.d));
-    r.norm_w = d_norm_w;
+    const Tensor d_scan = std::get<0>(launch_norm_bwd(scan_out, k.z(), norm_w, d_out, k.g, kNormEps, r.zx.narrow(2, 0, k.d), &norm_rows));
     // the scan's gradients leave as one packed [dx | dB | dC] buffer, that of the raw dt in its columns of r.zx
     const Tensor d_conv = at::empty({k.b, k.l, k.conv}, k.zx.options());
     m2_ssd_params p = core_ssd_params(k, conv_out, A, D, dt_bias);
@@ -587,7 +607,15 @@ CoreGrads core_backward(const Packed& k, const Tensor& d_out, const Tensor& A, c
     p.dA = ptr<float>(r.A); p.dD = ptr<float>(r.D); p.d_dt_bias = ptr<float>(r.dt_bias);
     launch_ssd_bwd(p, k.zx, stream);
     std::tie(r.conv_w, r.conv_b) = launch_conv_bwd(k.xBC(), conv_w, conv_b, {ptr(d_conv), k.l * k.conv, k.conv, 1},
-                                                   {at_column(r.zx, k.d), r.zx.stride(0), r.zx.stride(1), 1}, k.b, k.l, k.conv, k.zx, M2_ACT_SILU, stream);
+                                                   {at_column(r.zx, k.d), r.zx.stride(0), r.zx.stride(1), 1}, k.b, k.l, k.conv, k.zx, M2_ACT_SILU, stream, &conv_rows);
+    r.norm_w = at::empty({k.d}, casts(norm_param) ? norm_param.options() : norm_param.options().dtype(at::kFloat));
+    const bool to_heads = !head_grads.empty();
+    auto head = [&](size_t i) { return to_heads && head_grads[i].defined() ? ptr(head_grads[i]) : nullptr; };
+    auto head_type = [&](size_t i) { return to_heads && head_grads[i].defined() ? dtype_code(head_grads[i]) : M2_F32; };
+    check(lib.m2_param_sums(ptr<float>(norm_rows.rows), norm_rows.count, k.d, ptr(r.norm_w), dtype_code(r.norm_w), ptr<float>(conv_rows.rows),
+                            conv_rows.count, k.conv, ptr(r.conv_w), ptr(r.conv_b), dtype_code(r.conv_w), to_heads ? k.h : 0, ptr<float>(A), ptr<float>(r.A),
+                            ptr<float>(r.D), ptr<float>(r.dt_bias), head(0), head_type(0), head(1), head_type(1), head(2), head_type(2), stream),
+          "m2_param_sums");
     return r;
 }
 
@@ -606,7 +634,7 @@ py::tuple backward_parts(const Tensor& d_out, const Tensor& zx, const Tensor& A,
     const Packed k(zx, g, n, d, hd);
     check_core(k, A, or_none(D), conv_w, or_none(conv_b), dt_bias, norm_w);
     const CoreGrads r = core_backward(k, d_out, f32(A), f32(or_none(D)), conv_w, or_none(conv_b), f32(dt_bias), norm_w, conv_out, scan_out,
-                                      or_none(states), scope.stream);
+                                      or_none(states), norm_w, {}, scope.stream);
     return py::make_tuple(r.zx, r.A.to(A.scalar_type()), D ? r.D.to(D->scalar_type()) : Tensor(), r.conv_w, r.conv_b, r.dt_bias.to(dt_bias.scalar_type()),
                           r.norm_w.to(norm_w.scalar_type()));
 }
@@ -635,7 +663,7 @@ struct CoreFn : torch::autograd::Function<CoreFn> {
         CoreOut f;
         if (s.size() > 7) { f.conv_out = s[7]; f.scan_out = s[8]; f.states = s[9]; }
         else f = core_forward(k, A, D, s[3], s[4], dt_bias, norm_w, true, false, scope.stream);
-        const CoreGrads r = core_backward(k, grads[0], A, D, s[3], s[4], dt_bias, norm_w, f.conv_out, f.scan_out, f.states, scope.stream);
+        const CoreGrads r = core_backward(k, grads[0], A, D, s[3], s[4], dt_bias, norm_w, f.conv_out, f.scan_out, f.states, s[6], {}, scope.stream);
         variable_list out(12);
         out[0] = r.zx; out[1] = r.A.to(s[1].scalar_type());
         if (s[2].defined()) out[2] = r.D.to(s[2].scalar_type());
@@ -695,7 +723,6 @@ Tensor linear(const Tensor& x, const Tensor& w, const OptTensor& bias) {
     return project(x.reshape({-1, w.size(1)}), w, or_none(bias), scope.stream).view(shape);
 }
 
-bool casts(const Tensor& t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16; }
 // a small parameter as the casting kernel reads it; types that it does not take come as fp32
 Tensor small_param(const Tensor& t) { return (casts(t) ? t : t.to(at::kFloat)).contiguous(); }
 
@@ -742,11 +769,10 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
         CoreOut f;
         if (s.size() > kConvOut) { f.conv_out = s[kConvOut]; f.scan_out = s[kScanOut]; f.states = s[kStates]; }
         else f = core_forward(k, A, D, s[kConvW], s[kConvB], dt_bias, norm_w, true, false, scope.stream);
-        const CoreGrads r = core_backward(k, d_core, A, D, s[kConvW], s[kConvB], dt_bias, norm_w, f.conv_out, f.scan_out, f.states, scope.stream);
-        for (const int i : {kALog, kD, kDtBias, kNormW}) out[i] = at::empty(s[i].sizes(), casts(s[i]) ? s[i].options() : s[i].options().dtype(at::kFloat));
-        check(lib.m2_mixer_params_grads(ptr<float>(A), ptr<float>(r.A), ptr<float>(r.D), ptr<float>(r.dt_bias), ptr<float>(r.norm_w), ptr(out[kALog]),
-                                        dtype_code(out[kALog]), ptr(out[kD]), dtype_code(out[kD]), ptr(out[kDtBias]), dtype_code(out[kDtBias]), ptr(out[kNormW]),
-                                        dtype_code(out[kNormW]), k.h, k.d, scope.stream), "m2_mixer_params_grads");
+        for (const int i : {kALog, kD, kDtBias}) out[i] = at::empty(s[i].sizes(), casts(s[i]) ? s[i].options() : s[i].options().dtype(at::kFloat));
+        const CoreGrads r = core_backward(k, d_core, A, D, s[kConvW], s[kConvB], dt_bias, norm_w, f.conv_out, f.scan_out, f.states, s[kNormW],
+                                          {out[kALog], out[kD], out[kDtBias]}, scope.stream);
+        out[kNormW] = r.norm_w.view(s[kNormW].sizes());
         for (const int i : {kALog, kD, kDtBias, kNormW})
             if (!casts(s[i])) out[i] = out[i].to(s[i].scalar_type());
         out[kConvW] = r.conv_w; out[kConvB] = r.conv_b;

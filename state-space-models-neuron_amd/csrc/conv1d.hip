@@ -19,7 +19,7 @@
 // of one row, so the taps of an output come from the lane's own window and nothing is loaded per tap.
 //
 // A generic path (any strides, k <= 8) covers the rest with one thread per output element.
-#include "common.hpp"
+#include "sums.hpp"
 
 namespace m2 {
 namespace {
@@ -97,11 +97,6 @@ __device__ __forceinline__ void ld_elems(const T* __restrict__ p, float (&out)[V
 __device__ __forceinline__ float ld_param(const void* p, int pd, int64_t i) {
     return pd == M2_F32 ? reinterpret_cast<const float*>(p)[i] : to_f32(reinterpret_cast<const bf16_t*>(p)[i]);
 }
-__device__ __forceinline__ void st_param(void* p, int pd, int64_t i, float v) {
-    if (pd == M2_F32) reinterpret_cast<float*>(p)[i] = v;
-    else reinterpret_cast<bf16_t*>(p)[i] = from_f32<bf16_t>(v);
-}
-
 // The 4 taps and the bias of V consecutive channels with 16-byte loads, all in flight together (w is (C, 4) contiguous).
 template <typename WT, int V>
 __device__ __forceinline__ void load_taps(const void* __restrict__ w, const void* __restrict__ bias, int64_t c0,
@@ -398,28 +393,11 @@ __global__ void conv_zero_kernel(uint16_t* __restrict__ p, int64_t n) {
     if (i < n) p[i] = 0;
 }
 
-// Second stage: sum the per-block partials.  Four adjacent lanes per (channel, tap-or-bias), each a quarter of the
-// slots (fixed order), combined by two shuffles.
+// Second stage: sum the per-block partials.
 __global__ void __launch_bounds__(256)
 conv_reduce_partials_kernel(const float* __restrict__ part, int64_t nslots, int64_t C, int k,
                             void* __restrict__ dw, void* __restrict__ db, int pd) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t e = t >> 2;
-    const int q = (int)(t & 3);
-    const int kk = k + 1;
-    const bool live = e < C * kk;
-    const int64_t c = live ? e / kk : 0;
-    const int i = live ? (int)(e % kk) : 0;
-    float s = 0.f;
-    if (live) {
-#pragma unroll 4
-        for (int64_t r = q; r < nslots; r += 4) s += part[(r * C + c) * kk + i];
-    }
-    s = lane_xor_add<1>(s);
-    s = lane_xor_add<2>(s);
-    if (!live || q != 0) return;
-    if (i < k) st_param(dw, pd, c * k + i, s);
-    else if (db) st_param(db, pd, c, s);
+    conv_sum_body(part, nslots, C, k, dw, db, pd, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -738,8 +716,9 @@ int launch_fwd(const m2_conv1d_params* p, void* state_, int W, bool continuing, 
     return check_launch("conv1d_tail");
 }
 
+// slots: null, or where the number of partial rows goes that are left in the workspace instead of summed (0: dw and db are there)
 template <typename T>
-int launch_bwd(const m2_conv1d_params* p, hipStream_t st) {
+int launch_bwd(const m2_conv1d_params* p, int64_t* slots, hipStream_t st) {
     const int64_t nb = p->batch, l = p->seqlen, C = p->channels;
     const T* x = static_cast<const T*>(p->x);
     const T* dy = static_cast<const T*>(p->dy);
@@ -760,6 +739,7 @@ int launch_bwd(const m2_conv1d_params* p, hipStream_t st) {
         });
         int rc = check_launch("conv1d_bwd");
         if (rc) return rc;
+        if (slots) { *slots = nslots; return M2_OK; }
         conv_reduce_partials_kernel<<<(unsigned)ceil_div(C * 5 * 4, (int64_t)256), 256, 0, st>>>(part, nslots, C, 4, p->dw, p->db, p->param_dtype);
         return check_launch("conv1d_bwd_reduce");
     }
@@ -830,8 +810,9 @@ extern "C" size_t m2_conv1d_bwd_workspace_bytes(int64_t batch, int64_t seqlen, i
     return (size_t)(ceil_div(nseg, kSEG) * batch * channels * 5) * sizeof(float) + 16;
 }
 
-extern "C" int m2_conv1d_bwd(const m2_conv1d_params* p, void* stream) {
-    using namespace m2;
+namespace m2 {
+namespace {
+int conv1d_bwd(const m2_conv1d_params* p, int64_t* slots, void* stream) {
     int rc = check_common(p);
     if (rc) return rc;
     M2_REQUIRE(p->dw, M2_ERR_NULL, "conv1d_bwd: dw is required");
@@ -846,6 +827,17 @@ extern "C" int m2_conv1d_bwd(const m2_conv1d_params* p, void* stream) {
         return check_launch("conv1d_bwd_zero");
     }
     M2_REQUIRE(p->x && p->w && p->dy && p->dx, M2_ERR_NULL, "conv1d_bwd: x, w, dy, dx are required");
-    M2_DISPATCH_DTYPE(p->dtype, T, return launch_bwd<T>(p, static_cast<hipStream_t>(stream)));
+    M2_DISPATCH_DTYPE(p->dtype, T, return launch_bwd<T>(p, slots, static_cast<hipStream_t>(stream)));
     return M2_OK;
+}
+}  // namespace
+}  // namespace m2
+
+extern "C" int m2_conv1d_bwd(const m2_conv1d_params* p, void* stream) { return m2::conv1d_bwd(p, nullptr, stream); }
+
+extern "C" int m2_conv1d_bwd_partial(const m2_conv1d_params* p, int64_t* slots, void* stream) {
+    using namespace m2;
+    M2_REQUIRE(slots, M2_ERR_NULL, "conv1d_bwd_partial: slots is required");
+    *slots = 0;
+    return conv1d_bwd(p, slots, stream);
 }

@@ -14,7 +14,7 @@
 // partials in a caller-owned workspace and are summed in a fixed order by a second small kernel (no atomics).
 #include <initializer_list>
 
-#include "common.hpp"
+#include "sums.hpp"
 
 namespace m2 {
 namespace {
@@ -61,43 +61,10 @@ softplus_bwd_kernel(const T* __restrict__ dt, int64_t dt_sr, const float* __rest
     }
 }
 
-// out[c] = sum over the partial rows of partial[row][c] in a fixed order: 32 channels (one cache line of a row) per workgroup, V to
-// a lane, 32 V row phases whose sums meet in LDS.  Few workgroups read little each: what bounds the kernel is the chain of
-// loads of one thread, hence many phases with wide loads (32 phases of one channel per thread: 11.2 us at 1668 rows of 2048).
-constexpr int kSumCols = 32;
 template <int V>
 __global__ void __launch_bounds__(1024)
 column_sum_kernel(const float* __restrict__ partial, float* __restrict__ out, int64_t nrows, int64_t ncols) {
-    constexpr int LANES = kSumCols / V, PHASES = 1024 / LANES;
-    typedef float vec __attribute__((ext_vector_type(V)));
-    __shared__ float red[PHASES][kSumCols + 4];
-    const int l = threadIdx.x % LANES, ph = threadIdx.x / LANES;
-    const int64_t col = (int64_t)blockIdx.x * kSumCols + l * V;
-    vec s = 0.f;
-    if (col < ncols) {
-#pragma unroll 4
-        for (int64_t r = ph; r < nrows; r += PHASES) s += *reinterpret_cast<const vec*>(partial + r * ncols + col);
-    }
-    *reinterpret_cast<vec*>(&red[ph][l * V]) = s;
-    __syncthreads();
-    // 32 threads per channel, then one
-    const int c = threadIdx.x & 31, q = threadIdx.x >> 5;
-    float t = 0.f;
-#pragma unroll
-    for (int k = 0; k < PHASES / 32; ++k) t += red[q * (PHASES / 32) + k][c];
-    __syncthreads();
-    red[q][c] = t;
-    __syncthreads();
-    if (q == 0 && (int64_t)blockIdx.x * kSumCols + c < ncols) {
-        float u[32];
-#pragma unroll
-        for (int k = 0; k < 32; ++k) u[k] = red[k][c];
-#pragma unroll
-        for (int w = 16; w >= 1; w >>= 1)
-#pragma unroll
-            for (int k = 0; k < w; ++k) u[k] += u[k + w];
-        out[(int64_t)blockIdx.x * kSumCols + c] = u[0];
-    }
+    column_sum_body<V>(partial, nrows, ncols, blockIdx.x, [&](int64_t c, float v) { out[c] = v; });
 }
 int launch_column_sum(const float* partial, float* out, int64_t nrows, int64_t ncols, hipStream_t st) {
     const unsigned blocks = (unsigned)ceil_div(ncols, (int64_t)kSumCols);
@@ -458,10 +425,6 @@ add_rmsnorm_kernel(float* __restrict__ res, int64_t res_sr, const T* __restrict_
 __device__ __forceinline__ float ld_as_f32(const void* p, int dt, int64_t i) {
     return dt == M2_F32 ? static_cast<const float*>(p)[i] : to_f32(static_cast<const bf16_t*>(p)[i]);
 }
-__device__ __forceinline__ void st_from_f32(void* p, int dt, int64_t i, float v) {
-    if (dt == M2_F32) static_cast<float*>(p)[i] = v;
-    else static_cast<bf16_t*>(p)[i] = from_f32<bf16_t>(v);
-}
 struct MixerParams { const void *A_log, *D, *dt_bias, *norm; int a, d, b, w; };
 __global__ void __launch_bounds__(256)
 mixer_params_kernel(const MixerParams p, float* __restrict__ out, int64_t nheads, int64_t channels) {
@@ -473,16 +436,29 @@ mixer_params_kernel(const MixerParams p, float* __restrict__ out, int64_t nheads
     }
     if (i < channels) out[3 * nheads + i] = ld_as_f32(p.norm, p.w, i);
 }
-struct MixerGrads { const float *A, *dA, *dD, *db, *dw; void *A_log, *D, *dt_bias, *norm; int a, d, b, w; };
-__global__ void __launch_bounds__(256)
-mixer_params_grads_kernel(const MixerGrads p, int64_t nheads, int64_t channels) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < nheads) {
-        st_from_f32(p.A_log, p.a, i, p.dA[i] * p.A[i]);
-        if (p.D) st_from_f32(p.D, p.d, i, p.dD[i]);
-        st_from_f32(p.dt_bias, p.b, i, p.db[i]);
+// The sums behind a layer's backward in one launch: the norm weight's partial rows, the conv's partials, and the per-head gradients
+// in their parameters' types (dA_log = dA A where A is given).  Each of them had been a launch of its own, 3-5 us plus the gap in front
+// of it for a few hundred kilobytes (training step of a 768-channel layer on 500 tokens: 23 launches 210 us, 21 launches 202; b3 l1111 h32 with recompute 217 -> 214).
+struct ParamSums {
+    const float* norm; int64_t norm_rows, channels; void* d_norm; int norm_dtype;
+    const float* conv; int64_t conv_slots, conv_channels; void *dw, *db; int conv_dtype;
+    int64_t nheads; const float *A, *dA, *dD, *d_dt_bias; void *o_A, *o_D, *o_dt_bias; int a, d, b;
+    unsigned n_norm, n_conv;      // workgroups of the first two parts
+};
+template <int V>
+__global__ void __launch_bounds__(1024)
+param_sums_kernel(const ParamSums p) {
+    if (blockIdx.x < p.n_norm) {
+        column_sum_body<V>(p.norm, p.norm_rows, p.channels, blockIdx.x, [&](int64_t c, float v) { st_param(p.d_norm, p.norm_dtype, c, v); });
+    } else if (blockIdx.x < p.n_norm + p.n_conv) {
+        conv_sum_body(p.conv, p.conv_slots, p.conv_channels, 4, p.dw, p.db, p.conv_dtype, (int64_t)(blockIdx.x - p.n_norm) * 1024 + threadIdx.x);
+    } else {
+        const int64_t i = (int64_t)(blockIdx.x - p.n_norm - p.n_conv) * 1024 + threadIdx.x;
+        if (i >= p.nheads) return;
+        st_param(p.o_A, p.a, i, p.A ? p.dA[i] * p.A[i] : p.dA[i]);
+        if (p.o_D) st_param(p.o_D, p.d, i, p.dD[i]);
+        st_param(p.o_dt_bias, p.b, i, p.d_dt_bias[i]);
     }
-    if (i < channels) st_from_f32(p.norm, p.w, i, p.dw[i]);
 }
 
 int check_norm_common(const m2_rmsnorm_params* p, const char* what) {
@@ -580,11 +556,11 @@ extern "C" size_t m2_rmsnorm_gated_bwd_workspace_bytes(int64_t rows, int64_t cha
     return m2::align_up((size_t)(used > most ? used : most) * (size_t)channels * sizeof(float), 256);
 }
 
-extern "C" int m2_rmsnorm_gated_bwd(const m2_rmsnorm_params* p, void* stream) {
+extern "C" int m2_rmsnorm_gated_bwd_partial(const m2_rmsnorm_params* p, int64_t* rows, void* stream) {
     using namespace m2;
     int rc = check_norm_common(p, "rmsnorm_gated_bwd");
     if (rc) return rc;
-    M2_REQUIRE(p->d_weight, M2_ERR_NULL, "rmsnorm_gated_bwd: d_weight is required");
+    M2_REQUIRE(rows, M2_ERR_NULL, "rmsnorm_gated_bwd_partial: rows is required");
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int V = p->dtype == M2_F32 ? 4 : 8;
     int64_t prows = 0;
@@ -612,7 +588,18 @@ extern "C" int m2_rmsnorm_gated_bwd(const m2_rmsnorm_params* p, void* stream) {
         M2_DISPATCH_DTYPE(p->dtype, T, rc = (launch_norm<T, true>(a, p->n_groups, st)));
         if (rc) return rc;
     }
-    return launch_column_sum(static_cast<const float*>(p->workspace), p->d_weight, prows, p->channels, st);
+    *rows = prows;
+    return M2_OK;
+}
+
+extern "C" int m2_rmsnorm_gated_bwd(const m2_rmsnorm_params* p, void* stream) {
+    using namespace m2;
+    int rc = check_norm_common(p, "rmsnorm_gated_bwd");
+    if (rc) return rc;
+    M2_REQUIRE(p->d_weight, M2_ERR_NULL, "rmsnorm_gated_bwd: d_weight is required");
+    int64_t prows = 0;
+    if ((rc = m2_rmsnorm_gated_bwd_partial(p, &prows, stream))) return rc;
+    return launch_column_sum(static_cast<const float*>(p->workspace), p->d_weight, prows, p->channels, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int m2_add_rmsnorm(float* residual, int64_t residual_stride_row, const void* delta, int64_t delta_stride_row,
@@ -650,6 +637,30 @@ extern "C" int m2_mixer_params(const void* A_log, int32_t A_dtype, const void* D
     return check_launch("mixer_params_kernel");
 }
 
+extern "C" int m2_param_sums(const float* norm_partial, int64_t norm_rows, int64_t channels, void* d_norm, int32_t norm_dtype, const float* conv_partial,
+                             int64_t conv_slots, int64_t conv_channels, void* dw, void* db, int32_t conv_dtype, int64_t nheads, const float* A,
+                             const float* dA, const float* dD, const float* d_dt_bias, void* dA_out, int32_t A_dtype, void* dD_out, int32_t D_dtype,
+                             void* d_dt_bias_out, int32_t dt_bias_dtype, void* stream) {
+    using namespace m2;
+    M2_REQUIRE(norm_rows >= 0 && channels >= 0 && conv_slots >= 0 && conv_channels >= 0 && nheads >= 0, M2_ERR_SHAPE, "param_sums: negative size");
+    M2_REQUIRE(channels == 0 || (d_norm && (norm_partial || norm_rows == 0)), M2_ERR_NULL, "param_sums: the norm's partial rows and gradient are required");
+    M2_REQUIRE(conv_slots == 0 || conv_channels == 0 || (conv_partial && dw), M2_ERR_NULL, "param_sums: the conv's partials and gradient are required");
+    M2_REQUIRE(nheads == 0 || (dA && d_dt_bias && dA_out && d_dt_bias_out && (!dD_out || dD)), M2_ERR_NULL, "param_sums: a gradient or its destination is missing");
+    for (const int32_t dt : {norm_dtype, conv_dtype, A_dtype, D_dtype, dt_bias_dtype})
+        M2_REQUIRE(dt == M2_F32 || dt == M2_BF16, M2_ERR_DTYPE, "param_sums: unsupported dtype %d", (int)dt);
+    ParamSums p{norm_partial, norm_rows, channels, d_norm, norm_dtype, conv_partial, conv_slots, conv_channels, dw, db, conv_dtype,
+                nheads, A, dA, dD, d_dt_bias, dA_out, dD_out, d_dt_bias_out, A_dtype, D_dtype, dt_bias_dtype, 0, 0};
+    const int64_t n_norm = ceil_div(channels, (int64_t)kSumCols), n_conv = conv_slots ? ceil_div(conv_channels * 5 * 4, (int64_t)1024) : 0;
+    const int64_t blocks = n_norm + n_conv + ceil_div(nheads, (int64_t)1024);
+    M2_REQUIRE(blocks < ((int64_t)1 << 31), M2_ERR_SHAPE, "param_sums: too many workgroups");
+    if (blocks == 0) return M2_OK;
+    p.n_norm = (unsigned)n_norm; p.n_conv = (unsigned)n_conv;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (channels % 4 == 0 && aligned16(norm_partial)) param_sums_kernel<4><<<(unsigned)blocks, 1024, 0, st>>>(p);
+    else param_sums_kernel<1><<<(unsigned)blocks, 1024, 0, st>>>(p);
+    return check_launch("param_sums_kernel");
+}
+
 extern "C" int m2_mixer_params_grads(const float* A, const float* dA, const float* dD, const float* d_dt_bias, const float* d_norm_weight,
                                      void* dA_log, int32_t A_dtype, void* dD_out, int32_t D_dtype, void* d_dt_bias_out, int32_t dt_bias_dtype,
                                      void* d_norm_out, int32_t norm_dtype, int64_t nheads, int64_t channels, void* stream) {
@@ -657,11 +668,7 @@ extern "C" int m2_mixer_params_grads(const float* A, const float* dA, const floa
     M2_REQUIRE(nheads > 0 && channels > 0, M2_ERR_SHAPE, "mixer_params_grads: heads %lld, channels %lld", (long long)nheads, (long long)channels);
     M2_REQUIRE(A && dA && d_dt_bias && d_norm_weight && dA_log && d_dt_bias_out && d_norm_out && (!dD_out || dD), M2_ERR_NULL,
                "mixer_params_grads: a gradient or its destination is missing");
-    for (const int32_t dt : {A_dtype, D_dtype, dt_bias_dtype, norm_dtype})
-        M2_REQUIRE(dt == M2_F32 || dt == M2_BF16, M2_ERR_DTYPE, "mixer_params_grads: unsupported dtype %d", (int)dt);
-    const int64_t n = nheads > channels ? nheads : channels;
-    mixer_params_grads_kernel<<<(unsigned)ceil_div(n, (int64_t)256), 256, 0, static_cast<hipStream_t>(stream)>>>(
-        MixerGrads{A, dA, dD, d_dt_bias, d_norm_weight, dA_log, dD_out, d_dt_bias_out, d_norm_out, A_dtype, D_dtype, dt_bias_dtype, norm_dtype},
-        nheads, channels);
-    return check_launch("mixer_params_grads_kernel");
+    // the finished gradient of the norm weight is a single partial row
+    return m2_param_sums(d_norm_weight, 1, channels, d_norm_out, norm_dtype, nullptr, 0, 0, nullptr, nullptr, M2_F32, nheads, A, dA, dD, d_dt_bias, dA_log,
+                         A_dtype, dD_out, D_dtype, d_dt_bias_out, dt_bias_dtype, stream);
 }

@@ -90,6 +90,7 @@ SYMBOLS = {
     "m2_conv1d_prefill": (C.c_int, [C.POINTER(Conv1dParams), _vp, _i32, _i32, _vp]),
     "m2_conv1d_bwd_workspace_bytes": (_sz, [_i64, _i64, _i64, _i32]),
     "m2_conv1d_bwd": (C.c_int, [C.POINTER(Conv1dParams), _vp]),
+    "m2_conv1d_bwd_partial": (C.c_int, [C.POINTER(Conv1dParams), C.POINTER(_i64), _vp]),
     "m2_ssd_chunk_states_bytes": (_sz, [C.POINTER(SsdParams)]),
     "m2_ssd_fwd_workspace_bytes": (_sz, [C.POINTER(SsdParams)]),
     "m2_ssd_fwd": (C.c_int, [C.POINTER(SsdParams), _vp]),
@@ -106,6 +107,7 @@ SYMBOLS = {
     "m2_rmsnorm_gated_fwd_check": (C.c_int, [C.POINTER(RmsnormParams)]),
     "m2_rmsnorm_gated_bwd_workspace_bytes": (_sz, [_i64, _i64, _i32, _i32]),
     "m2_rmsnorm_gated_bwd": (C.c_int, [C.POINTER(RmsnormParams), _vp]),
+    "m2_rmsnorm_gated_bwd_partial": (C.c_int, [C.POINTER(RmsnormParams), C.POINTER(_i64), _vp]),
     "m2_add_rmsnorm": (C.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, C.c_float, _i32, _vp]),
     "m2_linear_small_fits": (C.c_int, [_i64, _i64, _i64, _i32]),
     "m2_linear_small": (C.c_int, [C.POINTER(LinearParams), _vp]),
@@ -117,6 +119,8 @@ SYMBOLS = {
     "m2_product": (C.c_int, [C.POINTER(ProductParams), _vp]),
     "m2_mixer_params": (C.c_int, [_vp, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _vp, _i64, _i64, _vp]),
     "m2_mixer_params_grads": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _i64, _i64, _vp]),
+    "m2_param_sums": (C.c_int, [_vp, _i64, _i64, _vp, _i32, _vp, _i64, _i64, _vp, _vp, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _i32,
+                                _vp, _i32, _vp]),
     "m2_mfma_selftest": (C.c_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp]),
     "m2_stream_copy": (C.c_int, [_vp, _vp, _sz, _vp]),
     "m2_tile_walk": (C.c_int, [_vp, _vp, _i64, _i64, _i64, _i64, C.c_int32, _vp]),

@@ -158,3 +158,43 @@ def test_glue_empty_and_errors():
         glue.rmsnorm_gated_hip(torch.zeros(2, 36, dtype=torch.bfloat16, device=DEV), None, torch.ones(36, device=DEV), 3, 1e-5)
     with pytest.raises(RuntimeError):    # no CPU path
         glue.rmsnorm_gated_hip(torch.zeros(2, 64), None, torch.ones(64), 1, 1e-5)
+
+
+@pytest.mark.parametrize("norm_rows,channels,norm_dtype", [(0, 40, torch.float32), (1, 33, torch.bfloat16), (3, 64, torch.float32), (257, 132, torch.bfloat16), (5, 0, torch.float32)])
+@pytest.mark.parametrize("slots,conv_channels,conv_dtype", [(0, 7, torch.float32), (1, 9, torch.bfloat16), (6, 130, torch.float32)])
+@pytest.mark.parametrize("heads,times_A,dtypes", [(0, True, (torch.float32,) * 3), (5, False, (torch.bfloat16, torch.float32, torch.bfloat16)), (1500, True, (torch.float32, torch.bfloat16, torch.float32))])
+def test_param_sums(norm_rows, channels, norm_dtype, slots, conv_channels, conv_dtype, heads, times_A, dtypes):
+    """Each part of the joint launch against fp64 sums of the same partials, at the edges of its workgroups; parts that are absent."""
+    from mamba2 import _lib
+    lib = _lib.load()
+    torch.manual_seed(norm_rows + slots + heads)
+    r = lambda *shape: torch.randn(*shape, device="cuda")
+    rows, conv = r(max(norm_rows, 1), max(channels, 1)), r(max(slots, 1), conv_channels, 5)
+    A, dA, dD, db = (r(max(heads, 1)) for _ in range(4))
+    new = lambda n, dtype: torch.full((max(n, 1),), 7.0, device="cuda", dtype=dtype)
+    o_norm, o_w, o_b = new(channels, norm_dtype), new(conv_channels * 4, conv_dtype), new(conv_channels, conv_dtype)
+    o_A, o_D, o_db = (new(heads, t) for t in dtypes)
+    code, ptr = _lib.dtype_code, _lib.ptr
+    _lib.check(lib.m2_param_sums(ptr(rows), norm_rows, channels, ptr(o_norm), code(norm_dtype), ptr(conv), slots, conv_channels, ptr(o_w), ptr(o_b),
+                                 code(conv_dtype), heads, ptr(A) if times_A else None, ptr(dA), ptr(dD), ptr(db), ptr(o_A), code(dtypes[0]), ptr(o_D),
+                                 code(dtypes[1]), ptr(o_db), code(dtypes[2]), _lib.stream_ptr()), "param_sums")
+
+    def close(got, want, terms):
+        # fp32 sums: half an ulp of the largest partial sum per addition; bf16 results: half an ulp of the value on top
+        bound = terms * 2.0 ** -24 * (want.abs().max() + 4 * terms ** 0.5) + (2.0 ** -8 * want.abs() if got.dtype == torch.bfloat16 else 0.0)
+        assert ((got.double() - want).abs() <= bound).all()
+
+    if channels:
+        close(o_norm[:channels], rows[:norm_rows].double().sum(0), max(norm_rows, 1))
+    if slots:
+        s = conv.double().sum(0)
+        close(o_w, s[:, :4].reshape(-1), slots)
+        close(o_b, s[:, 4], slots)
+    else:
+        assert (o_w == 7).all() and (o_b == 7).all()
+    if heads:
+        close(o_A, dA.double() * (A.double() if times_A else 1.0), 1)
+        close(o_D, dD.double(), 1)
+        close(o_db, db.double(), 1)
+    else:
+        assert (o_A == 7).all()
