@@ -25,12 +25,6 @@ namespace m2 {
 namespace {
 
 constexpr int kMaxK = 8;
-#ifndef M2_CONV_TLF
-#define M2_CONV_TLF 16
-#endif
-#ifndef M2_CONV_TLB
-#define M2_CONV_TLB 32
-#endif
 #ifndef M2_CONV_UNR
 #define M2_CONV_UNR 4
 #endif
@@ -40,12 +34,9 @@ constexpr int kMaxK = 8;
 #ifndef M2_CONV_VB
 #define M2_CONV_VB 4
 #endif
-// Tokens per thread in the fast path, and bytes of channels per thread (VF forward, VB backward; at least two channels).
-// Both directions are short on loads in flight, so they take short segments (many threads).  The backward carries five
+// Bytes of channels per thread in the fast path (VF forward, VB backward; at least two channels).  The backward carries five
 // sums, two 3-token windows and the taps per channel: with two channels per thread it needs 96 registers (five waves per
 // SIMD), with four 160 (three waves), and the narrower form is the faster one although its loads are 4-byte ones.
-constexpr int kTLF = M2_CONV_TLF;
-constexpr int kTLB = M2_CONV_TLB;
 constexpr int kUNR = M2_CONV_UNR;    // tokens whose loads are in flight together
 #ifndef M2_CONV_CVT
 #define M2_CONV_CVT 64
@@ -58,7 +49,36 @@ constexpr int kUNR = M2_CONV_UNR;    // tokens whose loads are in flight togethe
 #endif
 constexpr int kCVT = M2_CONV_CVT;    // channel vectors per block (x dimension)
 constexpr int kSEG = M2_CONV_SEG;    // token segments per block (y dimension)
-static_assert(kTLF % kUNR == 0 && kTLB % kUNR == 0 && kUNR >= 3, "segments are whole load groups; the dx lag fits one group");
+static_assert(kUNR >= 3, "the dx lag fits one load group");
+
+// Tokens per thread.  A thread is a chain of load groups, so where the threads do not fill the chip short segments win, and their
+// halo (three tokens more read; six in the backward, and three more activations) and, in the backward, their partial rows only count
+// once it is full.  Kernel times in us (backward with its sum) at 4 | 8 | 16 and 8 | 16 | 32 tokens, bf16:
+//   b1 l200 C5376    3.1 |  3.2 |  4.5      9.4 |   8.6 |  11.2        b1 l2048 C10240  19.2 | 17.1 | 17.4     36.7 |  33.8 |  37.2
+//   b1 l500 C1792    3.1 |  3.4 |  4.5      7.4 |   8.4 |  11.8        b4 l2048 C5376   37.6 | 30.4 | 31.6     71.2 |  59.9 |  60.2
+//   b3 l1111 C2304   9.2 |  8.3 |  8.1     20.1 |  17.3 |  18.3        b2 l4096 C10240  69.3 | 56.4 | 58.8    136.9 | 115.9 | 114.0
+//   b8 l333 C5376   14.2 | 12.8 | 13.2     28.4 |  26.7 |  24.7        b1 l16384 C5376  70.4 | 56.1 | 58.9    143.4 | 119.7 | 119.0
+constexpr int64_t kMaxSegs = (int64_t)65535 * kSEG;      // what the grid holds: the longest sequences keep the longest segments
+int64_t conv_fwd_tokens(int64_t batch, int64_t seqlen, int64_t vectors) {
+    const int64_t threads = batch * ceil_div(seqlen, (int64_t)16) * vectors;
+    return threads <= 48 * 1024 ? 4 : (threads <= 192 * 1024 || ceil_div(seqlen, (int64_t)8) > kMaxSegs ? 16 : 8);
+}
+int64_t conv_bwd_tokens(int64_t batch, int64_t seqlen, int64_t channels) {
+    const int64_t threads = batch * ceil_div(seqlen, (int64_t)32) * ceil_div(channels, (int64_t)2);
+    const int64_t tl = threads <= 16 * 1024 ? 8 : (threads <= 1024 * 1024 ? 16 : 32);
+    return ceil_div(seqlen, tl) > kMaxSegs ? 32 : tl;
+}
+// f<tokens per thread>
+template <typename F> void with_fwd_tokens(int64_t tl, F&& f) {
+    if (tl == 4) f(std::integral_constant<int, 4>{});
+    else if (tl == 8) f(std::integral_constant<int, 8>{});
+    else f(std::integral_constant<int, 16>{});
+}
+template <typename F> void with_bwd_tokens(int64_t tl, F&& f) {
+    if (tl == 8) f(std::integral_constant<int, 8>{});
+    else if (tl == 16) f(std::integral_constant<int, 16>{});
+    else f(std::integral_constant<int, 32>{});
+}
 
 // streaming loads/stores of the activations (optionally non-temporal: nothing is re-read soon enough to be worth caching)
 // The vectors promise the alignment of an element only: gfx950 issues the same wide access either way, so rows that start
@@ -139,14 +159,15 @@ __device__ __forceinline__ void load_taps(const void* __restrict__ w, const void
 // has renewed; a kernel of its own behind this one took 4-5 us of every prefill (77 -> 73 us for 200 tokens of a 2560-channel
 // layer).  Only where no two threads share channels (C a multiple of V), else conv_tail_kernel follows.
 constexpr int kContinuing = 1, kTail = 2;
-template <typename T, typename WT, int V, int ACT, bool PREFILL>
+template <typename T, typename WT, int V, int ACT, bool PREFILL, int TL>
 __global__ void __launch_bounds__(kCVT * kSEG)
 conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias, T* state, int W, int flags,
                    T* __restrict__ y, int64_t l, int64_t C, int64_t xsb, int64_t xsl, int64_t ysb, int64_t ysl) {
+    static_assert(TL % kUNR == 0, "segments are whole load groups");
     const int64_t cv = (int64_t)blockIdx.x * kCVT + threadIdx.x;
     const int64_t seg = (int64_t)blockIdx.y * kSEG + threadIdx.y;
     const int64_t b = blockIdx.z;
-    const int64_t t0 = seg * kTLF;
+    const int64_t t0 = seg * TL;
     if (cv * V >= C || t0 >= l) return;
     const int64_t c0 = cv * V < C - V ? cv * V : C - V;     // the last vector ends with the row (it may repeat channels: same values)
 
@@ -210,14 +231,14 @@ conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     };
     // software pipeline: the loads of group g+1 are issued before group g is computed and stored
     RawVec<T, V> nxt[kUNR];
-    if (t0 + kTLF <= l) {
+    if (t0 + TL <= l) {
         // whole segment inside the sequence: no per-token predicates, so the wait before a group's compute can leave
         // the previous group's stores in flight
         const T* xq = xp + t0 * xsl;
         T* yq = yp + t0 * ysl;
 #pragma unroll
         for (int u = 0; u < kUNR; ++u) nxt[u] = ld_stream<T, V>(xq + u * xsl);
-        for (int g = 0; g < kTLF / kUNR - 1; ++g) {
+        for (int g = 0; g < TL / kUNR - 1; ++g) {
             RawVec<T, V> raw[kUNR];
             xq += kUNR * xsl;
 #pragma unroll
@@ -252,18 +273,19 @@ conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
 // Backward fast path.  Each thread marches t over [t0, t0+TL+3): at step t it forms g[t] and
 // emits dx[t-3] = w3 g[t-3] + w2 g[t-2] + w1 g[t-1] + w0 g[t]  (dx[s] = sum_i w[i] g[s+3-i]).
 // Partials: part[(blockIdx.z * gridDim.y + blockIdx.y)][c][0..4] = (dw0..dw3, db).
-template <typename T, typename WT, int V, int ACT>
+template <typename T, typename WT, int V, int ACT, int TL>
 __global__ void __launch_bounds__(kCVT * kSEG)
 conv_bwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias,
                    const T* __restrict__ dy, T* __restrict__ dx, float* __restrict__ part,
                    int64_t l, int64_t C, int64_t xsb, int64_t xsl, int64_t gsb, int64_t gsl,
                    int64_t dsb, int64_t dsl) {
+    static_assert(TL % kUNR == 0, "segments are whole load groups");
     __shared__ float red[kSEG][5][kCVT * V + 1];
     const int64_t cv = (int64_t)blockIdx.x * kCVT + threadIdx.x;
     const int64_t seg = (int64_t)blockIdx.y * kSEG + threadIdx.y;
     const int64_t b = blockIdx.z;
     const int64_t c0 = cv * V < C - V ? cv * V : C - V;     // the last vector ends with the row (it may repeat channels: same values)
-    const int64_t t0 = seg * kTLB;
+    const int64_t t0 = seg * TL;
     const bool active = (cv * V < C) && (t0 < l);
 
     float acc[5][V];
@@ -317,14 +339,14 @@ conv_bwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
         };
         // software pipeline: the loads of group g+1 are issued before group g is computed and stored
         RawVec<T, V> nx[kUNR], ng[kUNR];
-        if (t0 + kTLB + kUNR <= l) {
+        if (t0 + TL + kUNR <= l) {
             // the segment and its 3 lag tokens lie inside the sequence: no per-token predicates
             const T* xq = xp + t0 * xsl;
             const T* gq = gp + t0 * gsl;
             T* dq = dp + (t0 - 3) * dsl;
 #pragma unroll
             for (int u = 0; u < kUNR; ++u) { nx[u] = ld_stream<T, V>(xq + u * xsl); ng[u] = ld_stream<T, V>(gq + u * gsl); }
-            for (int grp = 0; grp < kTLB / kUNR; ++grp) {
+            for (int grp = 0; grp < TL / kUNR; ++grp) {
                 RawVec<T, V> rawx[kUNR], rawg[kUNR];
                 xq += kUNR * xsl;
                 gq += kUNR * gsl;
@@ -340,7 +362,7 @@ conv_bwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
 #pragma unroll
             for (int u = 0; u < 3; ++u) step(nx[u], ng[u], false, true, dq + u * dsl);
         } else {
-            const int64_t tseg = (t0 + kTLB < l) ? t0 + kTLB : l;      // end of this thread's own tokens
+            const int64_t tseg = (t0 + TL < l) ? t0 + TL : l;      // end of this thread's own tokens
             const int64_t tend = tseg + 3;                            // march 3 further for the dx lag
 #pragma unroll
             for (int u = 0; u < kUNR; ++u) {
@@ -686,15 +708,17 @@ int launch_fwd(const m2_conv1d_params* p, void* state_, int W, bool continuing, 
     T* y = static_cast<T*>(p->y);
     constexpr int V = conv_vec<T>(false);
     if (channels_last_ok<V>(p, false)) {
-        const int64_t CV = ceil_div(C, (int64_t)V), nseg = ceil_div(l, kTLF);
+        const int64_t CV = ceil_div(C, (int64_t)V), tl = conv_fwd_tokens(nb, l, CV), nseg = ceil_div(l, tl);
         dim3 grid((unsigned)ceil_div(CV, kCVT), (unsigned)ceil_div(nseg, kSEG), (unsigned)nb), block(kCVT, kSEG);
         M2_REQUIRE(grid.y <= 65535, M2_ERR_SHAPE, "conv1d: sequence too long for the grid");
         const bool fold = tail && C % V == 0;
         const int flags = (continuing ? kContinuing : 0) | (fold ? kTail : 0);
         conv_dispatch(p, [&](auto wt, auto act) {
-            auto k = state ? conv_fwd_cl_kernel<T, decltype(wt), V, decltype(act)::value, true>
-                           : conv_fwd_cl_kernel<T, decltype(wt), V, decltype(act)::value, false>;
-            k<<<grid, block, 0, st>>>(x, p->w, p->bias, state, W, flags, y, l, C, p->x_stride_b, p->x_stride_l, p->y_stride_b, p->y_stride_l);
+            with_fwd_tokens(tl, [&](auto t) {
+                auto k = state ? conv_fwd_cl_kernel<T, decltype(wt), V, decltype(act)::value, true, decltype(t)::value>
+                               : conv_fwd_cl_kernel<T, decltype(wt), V, decltype(act)::value, false, decltype(t)::value>;
+                k<<<grid, block, 0, st>>>(x, p->w, p->bias, state, W, flags, y, l, C, p->x_stride_b, p->x_stride_l, p->y_stride_b, p->y_stride_l);
+            });
         });
         tail = tail && !fold;
     } else if (!hist && channel_major_ok(p, false)) {
@@ -725,7 +749,7 @@ int launch_bwd(const m2_conv1d_params* p, int64_t* slots, hipStream_t st) {
     T* dx = static_cast<T*>(p->dx);
     constexpr int V = conv_vec<T>(true);
     if (channels_last_ok<V>(p, true)) {
-        const int64_t CV = ceil_div(C, (int64_t)V), nseg = ceil_div(l, kTLB);
+        const int64_t CV = ceil_div(C, (int64_t)V), tl = conv_bwd_tokens(nb, l, C), nseg = ceil_div(l, tl);
         dim3 grid((unsigned)ceil_div(CV, kCVT), (unsigned)ceil_div(nseg, kSEG), (unsigned)nb), block(kCVT, kSEG);
         M2_REQUIRE(grid.y <= 65535, M2_ERR_SHAPE, "conv1d: sequence too long for the grid");
         const int64_t nslots = (int64_t)grid.y * grid.z;
@@ -734,8 +758,10 @@ int launch_bwd(const m2_conv1d_params* p, int64_t* slots, hipStream_t st) {
                    "conv1d_bwd: workspace %zu bytes < %zu needed", p->workspace_bytes, need);
         float* part = static_cast<float*>(p->workspace);
         conv_dispatch(p, [&](auto wt, auto act) {
-            conv_bwd_cl_kernel<T, decltype(wt), V, decltype(act)::value><<<grid, block, 0, st>>>(
-                x, p->w, p->bias, dy, dx, part, l, C, p->x_stride_b, p->x_stride_l, p->y_stride_b, p->y_stride_l, p->dx_stride_b, p->dx_stride_l);
+            with_bwd_tokens(tl, [&](auto t) {
+                conv_bwd_cl_kernel<T, decltype(wt), V, decltype(act)::value, decltype(t)::value><<<grid, block, 0, st>>>(
+                    x, p->w, p->bias, dy, dx, part, l, C, p->x_stride_b, p->x_stride_l, p->y_stride_b, p->y_stride_l, p->dx_stride_b, p->dx_stride_l);
+            });
         });
         int rc = check_launch("conv1d_bwd");
         if (rc) return rc;
@@ -806,7 +832,7 @@ extern "C" int m2_conv1d_prefill(const m2_conv1d_params* p, void* conv_state, in
 extern "C" size_t m2_conv1d_bwd_workspace_bytes(int64_t batch, int64_t seqlen, int64_t channels, int32_t k) {
     using namespace m2;
     (void)k;
-    const int64_t nseg = ceil_div(seqlen, kTLB);
+    const int64_t nseg = ceil_div(seqlen, conv_bwd_tokens(batch, seqlen, channels));
     return (size_t)(ceil_div(nseg, kSEG) * batch * channels * 5) * sizeof(float) + 16;
 }
 

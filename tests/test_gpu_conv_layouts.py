@@ -85,3 +85,19 @@ def test_prefill_leaves_the_last_inputs(C, W, l, dtype, continuing):
     assert torch.equal(state, joined[:, :, -W:])
     ref = conv1d_forward(joined.transpose(1, 2).contiguous(), w, bias, "silu", channels_last=True)[:, W:]
     assert torch.equal(y, ref)      # the same sums in the same order
+
+
+@pytest.mark.parametrize("b,l,C", [(1, 3, 64), (1, 9, 130), (1, 800, 1024), (1, 3000, 1024), (2, 4090, 1024), (1, 2060, 4100), (3, 4100, 6000)])
+def test_conv_segment_lengths(b, l, C):
+    """Sizes on both sides of the rules for the tokens per thread (4, 16, 8 forward; 8, 16, 32 backward), ends inside a segment."""
+    from mamba2.conv1d_grouped import conv1d_backward, conv1d_forward
+    torch.manual_seed(l)
+    x, dy = (torch.randn(b, l, C, device=DEV).bfloat16() for _ in range(2))
+    w, bias = torch.randn(C, 1, 4, device=DEV).bfloat16(), torch.randn(C, device=DEV).bfloat16()
+    xd, wd, bd = (t.float().requires_grad_(True) for t in (x, w, bias))
+    ref = torch.nn.functional.silu(torch.nn.functional.conv1d(xd.transpose(1, 2), wd, bd, padding=3, groups=C)[..., :l]).transpose(1, 2)
+    grads = torch.autograd.grad(ref, (xd, wd, bd), dy.float())
+    got = (conv1d_forward(x, w, bias, "silu", channels_last=True), *conv1d_backward(x, w, bias, dy, "silu", channels_last=True))
+    for name, a, r in zip(("y", "dx", "dw", "db"), got, (ref.detach(), *grads)):
+        # one bf16 rounding of the result (2^-9 of it; heavy tails count against the tensor's norm) behind fp32 sums
+        assert (a.float() - r).norm() / r.norm() < 2.0 ** -8, name
