@@ -31,6 +31,14 @@ namespace {
 // tile's sum.  Loading the fragments straight into registers touches 16 rows, 64 bytes each, per instruction, and the L1 then
 // delivers 12 bytes per clock: 18 us for 10576 x 2560 at 16 rows and 26 at 32 with the weights in the memory-side cache.
 // Slots of 16 bytes are swizzled by the row so that the 16 rows of a fragment read spread over all banks.
+// What bounds the larger products is a CU's path to memory (10576 x 2560 with the weights in the memory-side cache: 10.6 us of the
+// 12.1 with cold ones), and of the ring's three copies per step one is x, however few its rows.  Up to four rows (XM < 8, padded to
+// 1, 2 or 4) therefore come ahead of the ring and stay, 8 rows-times-steps per copy, where they fit beside it: 10576 x 2560 and
+// 2560 x 5120 at 4 rows 12.9 + 9.5 -> 12.1 + 8.5 us, at 1 row 12.0 + 8.7 -> 11.9 + 8.4.  The LDS they free is not for a deeper
+// ring: 6 or 8 steps give nothing there and 5.7 -> 6.3 / 6.4 us at 4384 x 1024.
+// The small products wait for memory once.  The ring's copies go out first and everything else that a workgroup will need (sums,
+// old values, the conv states it shifts) right behind them: shifted behind the last tile the states were a second wait, and with
+// the sums in front the weights came 0.5 us later (24 layers of 1024 channels, 8 rows: 487 -> 476 us a step; 1 row 436 -> 399).
 enum { kOutBf16 = 0, kOutF32 = 1, kOutAdd = 2 };
 
 struct LinearArgs {
@@ -54,20 +62,26 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
-template <int OK, int XR, int NW, int D>
+// Bytes of a wave's share of the resident rows
+template <int XM>
+__host__ __device__ constexpr int linear_resident(int steps, int nw) { return XM < 8 ? ((steps + nw - 1) / nw * XM + 7) / 8 * 1024 : 0; }
+
+template <int OK, int XM, int NW, int D>
 __global__ void __launch_bounds__(NW * 64)
 linear_small_kernel(const LinearArgs a) {
-    constexpr int MT = (XR + 1) / 2, SLOT = (2 + XR) * 1024, PER = 2 + XR;     // column tiles; bytes and copies of a step of 64 k
+    constexpr bool RESIDENT = XM < 8;
+    constexpr int MT = (XM + 15) / 16, PER = 2 + (RESIDENT ? 0 : XM / 8), SLOT = PER * 1024;     // column tiles; copies and bytes of a step of 64 k
     extern __shared__ __align__(1024) char ring_mem[];
     __shared__ __align__(16) float red[NW][MT][256];
     __shared__ float rs[32][8];
     const int tid = threadIdx.x, wave = (int)uniform(tid >> 6), lane = tid & 63, r16 = lane & 15, q4 = lane >> 4;
     const int steps = a.K / 64, s0 = steps * wave / NW, mine = steps * (wave + 1) / NW - s0;
-    const char* ring = ring_mem + wave * (D * SLOT);
+    const char* ring = ring_mem + wave * (D * SLOT + linear_resident<XM>(steps, NW));
     const uint32_t ring_addr = uniform(lds_addr_of(ring));
     // copies: lane i fills slot i & 7 of row i >> 3 with the row's chunk (slot ^ swizzle)
     const int crow = lane >> 3;
     auto chunk_off = [&](int row) { return (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) * 16); };
+    constexpr int XR = RESIDENT ? 1 : XM / 8;
     uint32_t xoff[XR];
 #pragma unroll
     for (int j = 0; j < XR; ++j) {
@@ -90,8 +104,10 @@ linear_small_kernel(const LinearArgs a) {
         const uint32_t dst = ring_addr + islot * SLOT;
 #pragma unroll
         for (int j = 0; j < 2; ++j) async_copy16(wp, woff[j], dst + j * 1024);
+        if constexpr (!RESIDENT) {
 #pragma unroll
-        for (int j = 0; j < XR; ++j) async_copy16(a.x + k0, xoff[j], dst + (2 + j) * 1024);
+            for (int j = 0; j < XR; ++j) async_copy16(a.x + k0, xoff[j], dst + (2 + j) * 1024);
+        }
         islot = islot + 1 == D ? 0 : islot + 1;
         if (++is == mine) {
             is = 0;
@@ -99,6 +115,15 @@ linear_small_kernel(const LinearArgs a) {
             if (itile < a.tiles) tile_rows(itile);
         }
     };
+    if constexpr (RESIDENT) {
+        for (int j = 0; j * 8 < mine * XM; ++j) {            // 8 rows of 64 k, row % XM of step row / XM
+            const int row = j * 8 + crow, m = row % XM, step = row / XM < mine ? row / XM : mine - 1;
+            async_copy16(a.x + (int64_t)s0 * 64, (uint32_t)((m < a.M ? m : a.M - 1) * a.x_sr * 2) + (uint32_t)(step * 128) + chunk_off(m),
+                         ring_addr + D * SLOT + j * 1024);
+        }
+    }
+    const int total = mine * ((a.tiles - 1 - (int)blockIdx.x) / (int)gridDim.x + 1);
+    for (int j = 0; j < D - 1 && j < total; ++j) issue();
     // the row scales: this wave's rows, their partial sums asked for ahead of everything and added up behind the first tile
     constexpr int RU = 4, RV = 3;
     const int per = a.sq ? a.nsq / a.groups : 0, nrs = a.sq ? a.M * a.groups : 0;
@@ -126,9 +151,24 @@ linear_small_kernel(const LinearArgs a) {
         }
     };
     fetch_old(blockIdx.x);
-    const int total = mine * ((a.tiles - 1 - (int)blockIdx.x) / (int)gridDim.x + 1);
-    for (int j = 0; j < D - 1 && j < total; ++j) issue();
-
+    // the first conv state that this thread shifts
+    constexpr int CW = 8;                                    // widest
+    const int nch = a.conv_cx - a.conv_c0, conv_n = a.conv_state ? a.M * nch : 0, conv_i = blockIdx.x * NW * 64 + tid;
+    bf16_t* conv_at = nullptr;
+    bf16_t conv_v[CW];
+    auto conv_fetch = [&](int i) {
+        const int b = i / nch, c = a.conv_c0 + i - b * nch;
+        conv_at = a.conv_state + ((int64_t)b * a.conv_cx + c) * a.conv_W;
+#pragma unroll
+        for (int j = 1; j < CW; ++j) if (j < a.conv_W) conv_v[j - 1] = conv_at[j];
+        conv_v[CW - 1] = a.conv_in[b * a.conv_in_sb + c];
+    };
+    auto conv_store = [&] {
+#pragma unroll
+        for (int j = 0; j < CW - 1; ++j) if (j + 1 < a.conv_W) conv_at[j] = conv_v[j];
+        conv_at[a.conv_W - 1] = conv_v[CW - 1];
+    };
+    if (conv_i < conv_n) conv_fetch(conv_i);
     int done = 0, slot = 0;
     for (int tile = blockIdx.x; tile < a.tiles; tile += gridDim.x) {
         floatx4 acc[MT];
@@ -144,6 +184,7 @@ linear_small_kernel(const LinearArgs a) {
             }
             wait_vmem_keep<PER>(total - 1 - done < D - 1 ? total - 1 - done : D - 1);
             const char* base = ring + slot * SLOT;
+            const char* xbase = RESIDENT ? ring + D * SLOT + s * (XM * 128) : base + 2048;
             slot = slot + 1 == D ? 0 : slot + 1;
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk) {
@@ -151,8 +192,8 @@ linear_small_kernel(const LinearArgs a) {
                 const bf16x8 wf = *reinterpret_cast<const bf16x8*>(base + r16 * 128 + ((c ^ ((r16 >> 1) & 7)) * 16));
 #pragma unroll
                 for (int t = 0; t < MT; ++t) {
-                    const int m = XR == 1 ? r16 & 7 : t * 16 + r16;
-                    const bf16x8 xf = *reinterpret_cast<const bf16x8*>(base + 2048 + m * 128 + ((c ^ ((m >> 1) & 7)) * 16));
+                    const int m = XM <= 8 ? r16 & (XM - 1) : t * 16 + r16;
+                    const bf16x8 xf = *reinterpret_cast<const bf16x8*>(xbase + m * 128 + ((c ^ ((m >> 1) & 7)) * 16));
                     acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf, acc[t], 0, 0, 0);
                 }
             }
@@ -215,14 +256,9 @@ linear_small_kernel(const LinearArgs a) {
             lds_barrier();
         }
     }
-    if (a.conv_state) {
-        const int nch = a.conv_cx - a.conv_c0;
-        for (int i = blockIdx.x * NW * 64 + tid; i < a.M * nch; i += gridDim.x * NW * 64) {
-            const int b = i / nch, c = a.conv_c0 + i - b * nch;
-            bf16_t* cs = a.conv_state + ((int64_t)b * a.conv_cx + c) * a.conv_W;
-            for (int j = 0; j + 1 < a.conv_W; ++j) cs[j] = cs[j + 1];
-            cs[a.conv_W - 1] = a.conv_in[b * a.conv_in_sb + c];
-        }
+    if (conv_i < conv_n) {
+        conv_store();
+        for (int i = conv_i + (int)gridDim.x * NW * 64; i < conv_n; i += gridDim.x * NW * 64) { conv_fetch(i); conv_store(); }
     }
 }
 
@@ -242,22 +278,28 @@ int launch_linear(LinearArgs a, hipStream_t st) {
     a.tiles = (int)ceil_div(a.N, 16);
     const int nw = linear_waves(a.M, a.N, a.K, a.sq ? a.groups : 1);
     int rc = M2_OK;
-    auto go = [&](auto xr, auto waves) {
-        constexpr int XR = decltype(xr)::value, NW = decltype(waves)::value, D = XR == 4 && NW == 8 ? 2 : 4;
-        constexpr size_t lds = (size_t)NW * D * (2 + XR) * 1024;
-        static_assert(lds + NW * ((XR + 1) / 2) * 1024 + 1024 <= 160 * 1024, "ring and partial tiles within the LDS of a CU");
+    auto go = [&](auto xm, auto waves) {
+        constexpr int XM = decltype(xm)::value, NW = decltype(waves)::value, D = XM == 32 && NW == 8 ? 2 : 4;
+        constexpr size_t ring = (size_t)NW * D * (XM < 8 ? 2 : 2 + XM / 8) * 1024, room = (NW == 8 ? 160 : 80) * 1024 - NW * ((XM + 15) / 16) * 1024 - 1024;
+        static_assert(ring <= room || (XM == 32 && NW == 4), "ring and partial tiles within a workgroup's share of the LDS of a CU");
+        const size_t lds = ring + (size_t)NW * linear_resident<XM>(a.K / 64, NW);
+        if (XM < 8 && lds > room) return false;
         // Two workgroups of four waves, or one of eight, per CU; each goes on to its next tile without draining its ring.
         // (10576 x 2560, 1 / 8 / 16 rows, four waves: 12.1 / 12.9 / 14.8 us with 512 workgroups, 13.7 / 14.5 / 16.6 with one per
         // tile; 32 rows, eight waves: 20.4 with 256, 23.8 with one per tile.)
         const int64_t most = (NW == 8 ? 1 : 2) * device_cus();
         const unsigned grid = (unsigned)(a.tiles < most ? a.tiles : most);
-        rc = allow_smem(linear_small_kernel<OK, XR, NW, D>, lds);
-        if (rc == M2_OK) linear_small_kernel<OK, XR, NW, D><<<grid, NW * 64, lds, st>>>(a);
+        rc = allow_smem(linear_small_kernel<OK, XM, NW, D>, lds > 48 * 1024 && XM < 8 ? room : lds);      // one value per kernel: threads may launch side by side
+        if (rc == M2_OK) linear_small_kernel<OK, XM, NW, D><<<grid, NW * 64, lds, st>>>(a);
+        return true;
     };
     auto rows = [&](auto waves) {
-        if (a.M <= 8) go(std::integral_constant<int, 1>{}, waves);
-        else if (a.M <= 16) go(std::integral_constant<int, 2>{}, waves);
-        else go(std::integral_constant<int, 4>{}, waves);
+        if (a.M <= 1 && go(std::integral_constant<int, 1>{}, waves)) return;
+        if (a.M <= 2 && go(std::integral_constant<int, 2>{}, waves)) return;
+        if (a.M <= 4 && go(std::integral_constant<int, 4>{}, waves)) return;
+        if (a.M <= 8) go(std::integral_constant<int, 8>{}, waves);
+        else if (a.M <= 16) go(std::integral_constant<int, 16>{}, waves);
+        else go(std::integral_constant<int, 32>{}, waves);
     };
     if (nw == 8) rows(std::integral_constant<int, 8>{});
     else if (nw == 4) rows(std::integral_constant<int, 4>{});

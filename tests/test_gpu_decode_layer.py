@@ -87,3 +87,16 @@ def test_layer_step_against_oracle(b, h, p, n, g, W, groups_norm, block):
             want = blk.norm(blk.step(blk.step(x, cache_params=c3), cache_params=c3))
         assert _rel(got.view(b, 1, hidden), want.double().cpu()) < 1e-2
         assert _rel(c2.ssm_states[0], c3.ssm_states[0].double().cpu()) < 1e-2
+
+
+# few rows kept in LDS beside the ring: padded to 1, 2 or 4, step counts that do not divide by the waves, one and several tiles per workgroup,
+# and rows too long for that
+@pytest.mark.parametrize("M,N,K,groups", [(1, 33, 128, 1), (2, 16, 64, 1), (3, 4100, 320, 1), (4, 20000, 256, 2), (3, 50, 1088, 1), (4, 40, 16384, 1), (1, 9000, 2560, 4)])
+def test_linear_small_few_rows(M, N, K, groups):
+    for normed, out_kind in ((False, 0), (True, 2)):
+        test_linear_small(M, N, K, groups, normed, out_kind)
+
+
+@pytest.mark.parametrize("W", [5, 8])
+def test_layer_step_conv_widths(W):
+    test_layer_step_against_oracle(3, 8, 64, 64, 1, W, True, False)
