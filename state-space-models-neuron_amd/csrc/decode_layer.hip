@@ -341,7 +341,11 @@ struct GatedArgs {
     bf16_t* h; float* head_sq;                            // w h (batch, heads * P) and sum of h^2 (batch, heads)
     int nheads, ngroups, conv_cx, W;
 };
-template <typename WT, int P, int N>
+// STATES_FIRST: which loads go out first, the states' or the conv's dozen small ones per lane.  With more workgroups than CUs the
+// memory has to be kept busy: 8 sequences of 80 heads 10.3 -> 8.9 us, 4 of 128 8.7 -> 7.8, 32 of 32 13.3 -> 12.7 (a whole layer, 12 of
+// 32: 20.2 -> 19.3, 4 of 80: 28.5 -> 27.4).  Below that a workgroup's own chain counts too, and the conv is at its head: a layer of 8
+// of 32 17.5 us, 17.6 with the states first; 1 and 4 the same.
+template <typename WT, int P, int N, bool STATES_FIRST>
 __global__ void __launch_bounds__(256)
 decode_gated_kernel(const GatedArgs a) {
     constexpr int GL = N / 4, ROWS = 256 / GL, UP = P / ROWS < 8 ? P / ROWS : 8, NCH = P + 2 * N;
@@ -353,7 +357,12 @@ decode_gated_kernel(const GatedArgs a) {
     const bf16_t* row = a.zx + b * a.zx_sb;
     float* Sp = a.S + ((int64_t)b * a.nheads + h) * (P * N);
     const int sub = tid % GL, rowi = tid / GL;
-    // all loads go out in the order in which they are used: the conv's, then the states
+    floatx4 sv[UP];
+    auto load_states = [&] {
+#pragma unroll
+        for (int u = 0; u < UP; ++u) sv[u] = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(Sp + (u * ROWS + rowi) * N + sub * 4));
+    };
+    if constexpr (STATES_FIRST) load_states();
     bf16_t hist[NI][3], in[NI], zin = (bf16_t)0.f;
     float taps[NI][4], bias[NI];
     auto channel = [&](int i) { return i < P ? h * P + i : (i < P + N ? d + g * N + (i - P) : d + (a.ngroups + g) * N + (i - P - N)); };
@@ -373,9 +382,7 @@ decode_gated_kernel(const GatedArgs a) {
     float nw = 0.f;
     if (tid < P) { zin = row[h * P + tid]; nw = a.norm_w[h * P + tid]; }
     const float dtr = to_f32(row[d + a.conv_cx + h]) + (a.dt_bias ? a.dt_bias[h] : 0.f), Ah = a.A[h], Dh = a.D ? a.D[h] : 0.f;
-    floatx4 sv[UP];
-#pragma unroll
-    for (int u = 0; u < UP; ++u) sv[u] = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(Sp + (u * ROWS + rowi) * N + sub * 4));
+    if constexpr (!STATES_FIRST) load_states();
     const float dtv = softplus_f(dtr), dA = __expf(Ah * dtv);
 #pragma unroll
     for (int q = 0; q < NI; ++q) {
@@ -510,7 +517,8 @@ extern "C" int m2_decode_layer(const m2_linear_params* in, const m2_decode_param
     g.nheads = (int)dec->nheads; g.ngroups = (int)dec->ngroups; g.conv_cx = (int)cx; g.W = dec->W;
     const dim3 grid((unsigned)dec->nheads, (unsigned)dec->batch);
     auto go = [&](auto wt, auto p, auto n) {
-        decode_gated_kernel<decltype(wt), decltype(p)::value, decltype(n)::value><<<grid, 256, 0, st>>>(g);
+        if ((int64_t)grid.x * grid.y > device_cus()) decode_gated_kernel<decltype(wt), decltype(p)::value, decltype(n)::value, true><<<grid, 256, 0, st>>>(g);
+        else decode_gated_kernel<decltype(wt), decltype(p)::value, decltype(n)::value, false><<<grid, 256, 0, st>>>(g);
     };
     auto dims = [&](auto wt) {
         using c64 = std::integral_constant<int, 64>;
