@@ -316,7 +316,10 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
         m.dirp = w.dirp; m.rbp = w.rbp; m.dlc = w.dlc; m.dDp8 = w.dDp8; m.dlam = w.dlam; m.dBp = w.dBp; m.dCp = w.dCp;
         m.seqlen = p->seqlen; m.nheads = p->nheads; m.ngroups = p->ngroups; m.nchunks = nc;
         m.nslices = w.ns_b; m.hps = w.hps_b;
-        auto k = ssd_bwd16_kernel<T, P, N, HS>;
+        m.dG = w.dGp; m.Bt = w.Bt; m.Ct = w.Ct;
+        m.dB = p->dB; m.dB_sb = p->dB_stride_b; m.dB_sl = p->dB_stride_l; m.dB_sg = p->dB_stride_g;
+        m.dC = p->dC; m.dC_sb = p->dC_stride_b; m.dC_sl = p->dC_stride_l; m.dC_sg = p->dC_stride_g;
+        auto k = w.finished ? ssd_bwd16_kernel<T, P, N, HS, true> : ssd_bwd16_kernel<T, P, N, HS, false>;
         const size_t sm = bwd16_smem<P, N>();
         if ((rc = allow_smem(k, sm))) return rc;
         k<<<grid_b, 512, sm, st>>>(m);
@@ -368,8 +371,8 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
             tail1_kernel<T><<<(unsigned)(n_da + n_ss), kDaHeads * 64, 0, st>>>(da, n_da, sa);
         }
         if ((rc = check_launch("ssd tail1_kernel"))) return rc;
-        // 16-bit operands: one workgroup per (batch, chunk, group) once those alone fill the chip, one per side below that; fp32
-        // operands: none where the main kernel has finished dB and dC
+        // none where the main kernel has finished dB and dC; else, with 16-bit operands, one workgroup per (batch, chunk, group) once
+        // those alone fill the chip, one per side below that
         const bool both = sizeof(T) == 4 || ngrp >= kTail2BothFrom;
         Tail2Args32 ta;
         ta.dGp = gs; ta.dCp = cs; ta.dBp = bs; ta.Bt = sizeof(T) == 2 ? w.Bt : p->B; ta.Ct = sizeof(T) == 2 ? w.Ct : p->C; ta.dB = p->dB; ta.dC = p->dC;
@@ -379,9 +382,9 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
         ta.dAp = w.dAp; ta.dDp = w.dDp; ta.dbp = w.dbp; ta.dA = p->dA; ta.dD = p->D ? p->dD : nullptr;
         ta.dbias = p->dt_bias ? p->d_dt_bias : nullptr;
         ta.seqlen = p->seqlen; ta.ngroups = p->ngroups; ta.nchunks = nc; ta.batch = p->batch; ta.nheads = p->true_heads;
-        ta.n_bc = sizeof(T) == 4 && w.ns_b == 1 ? 0 : ngrp;
+        ta.n_bc = w.finished ? 0 : ngrp;
         const unsigned grid = (unsigned)((both ? 1 : 2) * ta.n_bc + p->true_heads);
-        const size_t sm = bcf_smem<T, N>();
+        const size_t sm = w.finished ? 0 : bcf_smem<T, N>();
         if constexpr (sizeof(T) == 2) {
             auto k = both ? tail2_kernel<T, N, true> : tail2_kernel<T, N, false>;
             if ((rc = allow_smem(k, sm))) return rc;

@@ -50,10 +50,20 @@ struct Bwd16Args {
     float* dDp8;                                          // [b][h][c][8]
     float* dlam;                                          // [b][h][c][kDlamParts]
     float* dBp; float* dCp;                               // [b][c][g][slice][kQ][N]
+    // FINISH: dG of the group and B^T, C^T tiles in operand order [b][c][g]; dB, dC [b][l][g][N]
+    const float* dG; const void* Bt; const void* Ct;
+    void* dB; int64_t dB_sb, dB_sl, dB_sg;
+    void* dC; int64_t dC_sb, dC_sl, dC_sg;
     int64_t seqlen, nheads, ngroups, nchunks, nslices, hps;
 };
 
-template <typename T, int P, int N, int HS>
+// FINISH: the workgroup has all heads of its group (nslices == 1) and dG is complete (dg16_kernel's slices too are one), so that role
+// B's accumulators are the whole state parts: it adds dG B and dG^T C to them and writes dB and dC, instead of leaving 128 KiB of
+// fp32 to be read again by bc_final16_body, with the same products in the same order.  dG (fp32, the ten 32x32 blocks of its lower
+// triangle) is copied into the free tile buffer while the last head is worked on, B^T and C^T into the other one behind it.
+// b2 l4096 h128 g8: this kernel 194 -> 201 us and the finish 39 -> 5 (its sums of dA and dD); b8 l2048 h8 g8 79 -> 89 and 78 -> 5.
+// With the operand fragments read from memory by each wave instead of through LDS: 207.
+template <typename T, int P, int N, int HS, bool FINISH>
 __global__ void __launch_bounds__(512, 1)
 ssd_bwd16_kernel(const Bwd16Args a) {
     static_assert(sizeof(T) == 2, "16-bit operands only");
@@ -123,6 +133,38 @@ ssd_bwd16_kernel(const Bwd16Args a) {
         }
         async_copy_ldtab(a.ldtab, (b * a.nheads + h) * a.nchunks + c, lds_LD + (uint32_t)(buf * 2 * kQ * 4));
     };
+    // the lower triangle's blocks of dG, row by row of blocks, each [32][32]: rows of eight 16-byte slots, slot ^ row
+    static_assert(TILES * 2 >= 10 * 4096, "dG's blocks fit a tile buffer");
+    auto issue_dg = [&](int buf) {
+        const float* Gp = a.dG + ((b * a.nchunks + c) * a.ngroups + g) * (int64_t)(kQ * kQ);
+        uint32_t ln = (uint32_t)lane;
+        asm volatile("" : "+v"(ln));
+#pragma unroll
+        for (int it = 0; it < 5; ++it) {
+            const uint32_t q = wave_u * 5 + it, blk = q >> 2;                           // 8 rows of a block per copy
+            const uint32_t bi = (uint32_t)(0x3333222110ull >> (4 * blk)) & 15, bj = (uint32_t)(0x3210210100ull >> (4 * blk)) & 15;
+            const uint32_t row = (q & 3) * 8 + (ln >> 3), slot = (ln ^ row) & 7;
+            async_copy16(Gp + (int)(bi * 32 * kQ + bj * 32), row * (uint32_t)(kQ * 4) + slot * 16u, lds_T + (uint32_t)(buf * TILES * 2) + q * 1024u);
+        }
+    };
+    // B^T and C^T of the group as they lie, one behind the other, into the buffer of the last head once everybody is done with it; complete
+    // with everything before it when this returns
+    static_assert(TILES >= 2 * N * kQ, "both operand tiles fit a tile buffer");
+    auto fetch_operands = [&] {
+        wait_vmem_all();              // this wave's blocks of dG have landed
+        __syncthreads();
+        const int64_t grp = ((b * a.nchunks + c) * a.ngroups + g) * (int64_t)(N * kQ);
+        const uint32_t dst = lds_T + (uint32_t)(((a.hps - 1) & 1) * TILES * 2);
+        constexpr int PIECES = N * kQ * 2 / 1024 / 8;                                   // per wave and tile
+#pragma unroll
+        for (int it = 0; it < PIECES; ++it) {
+            const uint32_t q = (wave_u * PIECES + it) * 1024u;
+            async_copy16(static_cast<const T*>(a.Bt) + grp, q + (uint32_t)lane * 16u, dst + q);
+            async_copy16(static_cast<const T*>(a.Ct) + grp, q + (uint32_t)lane * 16u, dst + (uint32_t)(N * kQ * 2) + q);
+        }
+        wait_vmem_all();
+        __syncthreads();
+    };
     // this wave's share of <dS, S_prev> over the two tiles of buffer `buf` (same slot order in both, so any order will do)
     auto tiles_dot = [&](int buf, int64_t bhc, float Lam) {
         const T* cS = tiles + buf * TILES;
@@ -183,6 +225,7 @@ ssd_bwd16_kernel(const Bwd16Args a) {
             if (lane < 32) wu[lane] = __expf(fminf(lref - sl[row0 + lane], 0.f));
             __syncthreads();
             if (hh + 1 < a.hps) issue_tiles(h + 1, buf ^ 1);
+            else if constexpr (FINISH) issue_dg(buf ^ 1);
             tiles_dot(buf, bhc, Lam);
             const T* cS = tiles + buf * TILES;
             const T* cP = cS + P * N;
@@ -308,6 +351,7 @@ ssd_bwd16_kernel(const Bwd16Args a) {
             float dD_loc = warp_sum(tok < valid ? dd : 0.f);
             if (lane == 0) { a.dDp8[bhc * 8 + wave] = dD_loc; a.dDp8[bhc * 8 + wave + 4] = 0.f; }
         }
+        if constexpr (FINISH) fetch_operands();
     } else {
         // =============================================================== role B: state parts of dB and dC, and dl_c
         // Operands swapped here too: lane (r, half) owns token row0 + r and, per 32-column block jn, the state columns
@@ -339,6 +383,7 @@ ssd_bwd16_kernel(const Bwd16Args a) {
             const float* sd = sl + kQ;
             __syncthreads();
             if (hh + 1 < a.hps) issue_tiles(h + 1, buf ^ 1);
+            else if constexpr (FINISH) issue_dg(buf ^ 1);
             // lane-dependent LDS offsets are rebuilt from the lane number for every head (a few integer instructions):
             // carried across the head loop they are spilled, and every reload waits for the tile copies in flight
             int ln = lane;
@@ -414,15 +459,69 @@ ssd_bwd16_kernel(const Bwd16Args a) {
             dlc = lane_xor_add<32>(dlc);
             if (half == 0) a.dlc[((b * a.nheads + h) * a.nchunks + c) * kQ + tok] = dlc * ws_c;
         }
-        const int64_t part = (((b * a.nchunks + c) * a.ngroups + g) * a.nslices + slice) * (int64_t)(kQ * N) + (int64_t)tok * N;
+        if constexpr (FINISH) {
+            fetch_operands();
+            const char* dg = reinterpret_cast<const char*>(tiles + (a.hps & 1) * TILES);
+            const char* ops = reinterpret_cast<const char*>(tiles + ((a.hps - 1) & 1) * TILES);
+            // acc[tok][n] += sum_k dG[tok][k] B[k][n], or dG[k][tok] C[k][n]
+            auto finish = [&](floatx16 (&acc)[1][NBN], auto side, const char* tile, T* out) {
+                constexpr bool SIDE_B = decltype(side)::value;
 #pragma unroll
-        for (int jn = 0; jn < NBN; ++jn)
+                for (int ks = 0; ks < 8; ++ks) {
+                    if (SIDE_B ? ks < 2 * rbk : ks >= 2 * rbk + 2) continue;      // wave-uniform
+                    Frag<T> xf[NBN];      // see mt_offset
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int64_t o = part + jn * 32 + 8 * q + 4 * half;
-                *reinterpret_cast<floatx4*>(a.dBp + o) = floatx4{accB[0][jn][4 * q], accB[0][jn][4 * q + 1], accB[0][jn][4 * q + 2], accB[0][jn][4 * q + 3]};
-                *reinterpret_cast<floatx4*>(a.dCp + o) = floatx4{accC[0][jn][4 * q], accC[0][jn][4 * q + 1], accC[0][jn][4 * q + 2], accC[0][jn][4 * q + 3]};
-            }
+                    for (int nb = 0; nb < NBN; ++nb) xf[nb].v = *reinterpret_cast<const bf16x8*>(tile + ((uint32_t)lane * 16u + (uint32_t)((nb * 8 + ks) * 1024)));
+                    const int bi = SIDE_B ? ks >> 1 : rbk, bj = SIDE_B ? rbk : ks >> 1, k0 = (ks & 1) * 16 + 8 * half;
+                    const char* blk = dg + (bi * (bi + 1) / 2 + bj) * 4096;
+                    float f[8];
+                    if constexpr (SIDE_B) {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) f[e] = *reinterpret_cast<const float*>(blk + (k0 + e) * 128 + (((r >> 2) ^ e) << 4) + (r & 3) * 4);
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < 2; ++q) {
+                            const floatx4 v = *reinterpret_cast<const floatx4*>(blk + r * 128 + (((k0 >> 2) + q) ^ (r & 7)) * 16);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) f[4 * q + e] = v[e];
+                        }
+                    }
+                    Frag<T> yh, yl;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        yh.v[e] = from_f32<T>(f[e]);
+                        yl.v[e] = from_f32<T>(f[e] - to_f32((T)yh.v[e]));
+                    }
+#pragma unroll
+                    for (int nb = 0; nb < NBN; ++nb) {
+                        mma_frag(acc[0][nb], xf[nb], yh);
+                        mma_frag(acc[0][nb], xf[nb], yl);
+                    }
+                }
+#pragma unroll
+                for (int nb = 0; nb < NBN; ++nb)
+#pragma unroll
+                    for (int qp = 0; qp < 2; ++qp) {
+                        float g8[8];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) pair_swap(acc[0][nb][8 * qp + e], acc[0][nb][8 * qp + 4 + e], g8[e], g8[4 + e]);
+                        const uint4 o = {pack2<T>(g8[0], g8[1]), pack2<T>(g8[2], g8[3]), pack2<T>(g8[4], g8[5]), pack2<T>(g8[6], g8[7])};
+                        if (tok < valid) *reinterpret_cast<uint4*>(out + nb * 32 + 8 * (2 * qp + half)) = o;
+                    }
+            };
+            finish(accC, std::false_type{}, ops, static_cast<T*>(a.dC) + b * a.dC_sb + (t0 + tok) * a.dC_sl + g * a.dC_sg);
+            finish(accB, std::true_type{}, ops + N * kQ * 2, static_cast<T*>(a.dB) + b * a.dB_sb + (t0 + tok) * a.dB_sl + g * a.dB_sg);
+        } else {
+            const int64_t part = (((b * a.nchunks + c) * a.ngroups + g) * a.nslices + slice) * (int64_t)(kQ * N) + (int64_t)tok * N;
+#pragma unroll
+            for (int jn = 0; jn < NBN; ++jn)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int64_t o = part + jn * 32 + 8 * q + 4 * half;
+                    *reinterpret_cast<floatx4*>(a.dBp + o) = floatx4{accB[0][jn][4 * q], accB[0][jn][4 * q + 1], accB[0][jn][4 * q + 2], accB[0][jn][4 * q + 3]};
+                    *reinterpret_cast<floatx4*>(a.dCp + o) = floatx4{accC[0][jn][4 * q], accC[0][jn][4 * q + 1], accC[0][jn][4 * q + 2], accC[0][jn][4 * q + 3]};
+                }
+        }
     }
 }
 

@@ -32,6 +32,7 @@ struct SsdWorkspace {
     float* dGs = nullptr; float* dBs = nullptr; float* dCs = nullptr;   // partials summed over the head slices
     float* dirp = nullptr; float* rbp = nullptr; float* dDp8 = nullptr; // per channel-half / per-wave partials of the dx kernel
     int64_t ns_g = 1, hps_g = 1, ns_b = 1, hps_b = 1;   // head slicing of dg16 and of the main backward kernel
+    bool finished = false;              // the main kernel's workgroups have whole groups and leave dB and dC: no partials of those
     size_t bytes = 0;
     size_t kept_bytes = 0;              // size of the forward -> backward carry-over (chunk_states buffer)
 };
@@ -127,8 +128,9 @@ inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_
         w.dDp8 = reinterpret_cast<float*>(take(bhc * 8 * 4));
         w.dGp = reinterpret_cast<float*>(take((size_t)p->batch * nc * p->ngroups * w.ns_g * kQ * kQ * 4));
         const size_t part = (size_t)p->batch * nc * p->ngroups * kQ * p->dstate * 4;
-        w.dBp = reinterpret_cast<float*>(take(part * w.ns_b));
-        w.dCp = reinterpret_cast<float*>(take(part * w.ns_b));
+        w.finished = w.ns_b == 1 && w.ns_g == 1;
+        w.dBp = reinterpret_cast<float*>(take(w.finished ? 0 : part * w.ns_b));
+        w.dCp = reinterpret_cast<float*>(take(w.finished ? 0 : part * w.ns_b));
         w.dGs = reinterpret_cast<float*>(take((size_t)p->batch * nc * p->ngroups * kQ * kQ * 4));
         w.dBs = reinterpret_cast<float*>(take((size_t)p->batch * nc * p->ngroups * kQ * p->dstate * 4));
         w.dCs = reinterpret_cast<float*>(take((size_t)p->batch * nc * p->ngroups * kQ * p->dstate * 4));

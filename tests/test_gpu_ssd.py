@@ -296,6 +296,28 @@ def test_ssd_softplus_folded_into_scan(dtype, b, l, h, p, n, g):
         assert torch.equal(gbuf[..., :24], torch.full((b, l, 24), 5.0, dtype=dtype, device=DEV))
 
 
+@pytest.mark.parametrize("b,l,h,p,n,g", [
+    (1, 300, 8, 64, 128, 8),       # one head per group; a partly filled last chunk
+    (16, 129, 16, 64, 128, 8),     # two heads one after the other; one token in the last chunk
+    (16, 130, 24, 64, 64, 8),      # three, 64 state columns
+    (16, 160, 8, 128, 128, 8)])    # a wide head as a pair; a row block that is exactly full
+def test_ssd_bf16_whole_groups(b, l, h, p, n, g):
+    """bf16 backward where a workgroup has all heads of its group and finishes dB and dC itself.  Bar: as above; a wrong 32x32 block of the ten
+    would show as more than 0.1 of its chunk."""
+    from mamba2.mamba2_kernel import alloc_chunk_states, ssd_backward, ssd_forward
+    d = make_ssd_inputs(b, l, h, p, n, g, seed=l + h, dtype=torch.bfloat16)
+    r = ssd_grads_ref(*(_f64(d)[k] for k in ("dt", "A", "X", "B", "C", "D", "dy")), chunk=64)
+    dd = _dev(d)
+    st = alloc_chunk_states(dd["dt"], dd["A"], dd["X"], dd["B"], dd["C"])
+    ssd_forward(dd["dt"], dd["A"], dd["X"], dd["B"], dd["C"], dd["D"], chunk_states=st)
+    out = ssd_backward(dd["dt"], dd["A"], dd["X"], dd["B"], dd["C"], dd["D"], dd["dy"], chunk_states=st)
+    for name, v in zip(("ddt", "dA", "dX", "dB", "dC", "dD"), out):
+        assert rel_rms_err(v, r[name]) < 2e-2, name
+    for name, v in (("dB", out[3]), ("dC", out[4])):
+        for t in range(0, l, 128):
+            assert rel_rms_err(v[:, t:t + 128], r[name][:, t:t + 128]) < 2e-2, (name, t)
+
+
 @pytest.mark.parametrize("steps", ["usual", "long"])
 @pytest.mark.parametrize("b,l,h,p,n,g", [
     (16, 129, 16, 64, 128, 4),     # four heads one after the other in a workgroup, which finishes dB and dC itself; one token in the last chunk
