@@ -25,7 +25,7 @@ constexpr int kK = 64, kRing = 4;      // k tile, tiles in the ring
 struct ProductArgs {
     const bf16_t* A; const bf16_t* B; const bf16_t* bias; bf16_t* out; float* part;
     int64_t lda, ldb, ldo;
-    int M, N, K, tiles_m, tiles_n, ksteps;      // ksteps: k tiles per split
+    int M, N, K, tiles_m, tiles_n, splits, ksteps;      // ksteps: k tiles per split
 };
 
 // Source of one wave-wide copy of an operand tile of R rows or columns: the 16-byte piece of lane s % 64 of 1 KiB chunk s / 64.
@@ -74,12 +74,15 @@ product_kernel(const ProductArgs p) {
     bf16_t* ring = reinterpret_cast<bf16_t*>(smem_raw);            // [kRing][ A tile | B tile ]
     float* red = reinterpret_cast<float*>(smem_raw);               // [KSPLIT ? 4 : 1][R][R], after the last k tile
     const int lane = threadIdx.x & 63, wave = (int)uniform(threadIdx.x >> 6), half = lane >> 5;
-    // the row tiles of one column of tiles follow one another on one XCD: its L2 then hands them the same rows of B
-    const int xcd = blockIdx.x & 7, u = blockIdx.x >> 3;
-    const int tn = u / p.tiles_m * 8 + xcd, tm = u % p.tiles_m;
-    if (tn >= p.tiles_n) return;
+    // Each XCD gets an eighth of the (split, column of tiles, row tile) triples in that order: the row tiles of one column follow one
+    // another on it, and its L2 hands them the same rows of B.  Whole columns dealt round the XCDs instead left some with half as much
+    // again as others, and two rounds where one would do (20 columns of 3 tiles, four splits: 36 workgroups on the 32 CUs of half of
+    // them): 257 x 2560 x 10576 63 -> 39 us, 737 x 1792 x 7480 65 -> 40, 1326 x 2560 x 10576 216 -> 120.
+    const int tiles = p.tiles_m * p.tiles_n, at = (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3));
+    if (at >= tiles * p.splits) return;
+    const int split = at / tiles, tn = (at - split * tiles) / p.tiles_m, tm = (at - split * tiles) % p.tiles_m;
     const int m0 = tm * R, n0 = tn * R;
-    const int k_first = blockIdx.y * p.ksteps * kK;
+    const int k_first = split * p.ksteps * kK;
     const int steps = min(p.ksteps, (p.K - k_first + kK - 1) / kK);
 
     Piece<AK, R> pa[NP];
@@ -172,7 +175,7 @@ product_kernel(const ProductArgs p) {
         const int row = m0 + m, col = n0 + c * 8;
         if (row >= p.M || col >= p.N) continue;
         if (p.part) {
-            float* o = p.part + ((int64_t)blockIdx.y * p.M + row) * p.N + col;
+            float* o = p.part + ((int64_t)split * p.M + row) * p.N + col;
             *reinterpret_cast<floatx4*>(o) = s0;
             *reinterpret_cast<floatx4*>(o + 4) = s1;
         } else {
@@ -209,21 +212,22 @@ product_sum_kernel(const float* __restrict__ part, const bf16_t* __restrict__ bi
     store16(out + row * ldo + col, v);
 }
 
-// Tile size and number of k splits: the cheapest of a count of k steps on the busiest CU, in microseconds as measured over tokens
-// 64 .. 2000 and layers of 768 and 2560 channels (the choice is within 2 % of the best one there on average).  Two workgroups of
-// the small tile share a CU and hide each other's waits; a split costs its second launch and the partials' way out and back.
+// Tile size and number of k splits: the cheapest of a count of k steps on the busiest CU (of the XCDs' equal shares), in microseconds as
+// fitted to 144 products of layers of 256 to 3072 channels over 33 to 2048 tokens, in all forms (the choice is within 1 % of the best of
+// tiles and one to six splits there on average, within 20 % for all).  Two workgroups of the small tile share a CU and hide each
+// other's waits; a split costs its second launch and the partials' way out and back.
 struct ProductPlan { int r, splits, ksteps; };
 ProductPlan product_plan(int64_t M, int64_t N, int64_t K) {
-    const int64_t cus = device_cus(), ktiles = ceil_div(K, (int64_t)kK);
+    const int64_t cus = device_cus() / 8, ktiles = ceil_div(K, (int64_t)kK);
     ProductPlan best{64, 1, (int)ktiles};
     float best_us = 1e30f;
     for (const int r : {64, 128}) {
         const int64_t tiles = ceil_div(M, (int64_t)r) * ceil_div(N, (int64_t)r);
-        for (int64_t want = 1; want <= 4 && (want == 1 || ktiles / want >= 4); ++want) {
-            const int64_t ks = ceil_div(ktiles, want), s = ceil_div(ktiles, ks), busiest = ceil_div(tiles * s, cus);
-            float us = r == 64 ? (float)ks * 0.33f * (1.3f * (busiest / 2) + busiest % 2) + 1.2f * ceil_div(busiest, (int64_t)2)
-                               : (float)busiest * (ks * 0.42f + 1.8f);
-            if (s > 1) us += 2.f + 5e-6f * s * M * N;
+        for (int64_t want = 1; want <= 6 && (want == 1 || ktiles / want >= 4); ++want) {
+            const int64_t ks = ceil_div(ktiles, want), s = ceil_div(ktiles, ks), busiest = ceil_div(ceil_div(tiles * s, (int64_t)8), cus);
+            float us = r == 64 ? (float)ks * 0.3f * (1.6f * (busiest / 2) + busiest % 2) + 1.2f * ceil_div(busiest, (int64_t)2)
+                               : (float)busiest * (ks * 0.54f + 1.8f);
+            if (s > 1) us += 1.6f + 3e-6f * s * M * N;
             if (us < best_us) { best_us = us; best = {r, (int)s, (int)ks}; }
         }
     }
@@ -243,11 +247,11 @@ extern "C" int m2_product_fits(int64_t M, int64_t N, int64_t K, int32_t a_k, int
 // Where these kernels are ahead of the general library's product with its default solution (bf16, by size; its call also costs the
 // host 18 us to their 4).  Solutions chosen by timing are another matter: at 128 rows of a 2560-channel layer they are ahead, so a
 // program that has them chosen keeps its products there (library_is_tuned in binding.cpp).
-//   weight gradients (k = tokens) with few outputs -- 500 x 3352 x 768: 14.4 -> 11.1 us, 2000: 39 -> 27; with ten million outputs
-//   the stores bound both and the library's are better (200 tokens, 10576 x 2560: 34 us to 51);
-//   other products up to 4e9 multiply-adds -- 200 x 2560 x 5120: 25.8 -> 21.3 us, 500 x 3352 x 768: 10.0 -> 8.5; beyond, its larger
-//   tiles reuse more (500 x 10576 x 2560: 40 us to 58);
-//   long sums for few outputs, where it does not split k -- 500 x 2560 x 10576: 110 -> 93 us, 64 tokens: 78 -> 28.
+//   weight gradients (k = tokens) with few outputs -- 768 x 3352 x 768: 13.7 -> 12.9 us, 1024 x 2048 x 1536: 16.5 -> 14.0; with ten
+//   million outputs the stores bound both and the library's are better (200 tokens, 10576 x 2560: 35 us to 46);
+//   other products up to 4e9 multiply-adds -- 200 x 2560 x 5120: 25.6 -> 20.1 us, 360 x 4384 x 1024: 11.4 -> 9.5; beyond, its larger
+//   tiles reuse more (512 x 10576 x 2560: 39 us to 57);
+//   long sums for few outputs, where it does not split k -- 512 x 2560 x 10576: 108 -> 52 us, 200 tokens: 69 -> 32.
 extern "C" int m2_product_pays(int64_t M, int64_t N, int64_t K, int32_t a_k, int32_t b_k) {
     if (!m2_product_fits(M, N, K, a_k, b_k)) return 0;
     const int64_t outputs = M * N, macs = outputs * K;
@@ -282,7 +286,8 @@ extern "C" int m2_product(const m2_product_params* p, void* stream) {
         M2_REQUIRE(p->workspace && p->workspace_bytes >= (size_t)splits * p->M * p->N * 4, M2_ERR_WORKSPACE, "product: workspace too small");
         a.part = static_cast<float*>(p->workspace);
     }
-    const dim3 grid((unsigned)(ceil_div(a.tiles_n, 8) * 8 * a.tiles_m), (unsigned)splits);
+    a.splits = splits;
+    const unsigned grid = (unsigned)(ceil_div((int64_t)a.tiles_m * a.tiles_n * splits, (int64_t)8) * 8);
     const size_t sm = (size_t)kRing * 2 * plan.r * kK * 2;
     auto launch = [&](auto k) -> int {
         if (const int rc = allow_smem(k, sm)) return rc;

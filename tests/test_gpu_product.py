@@ -45,6 +45,14 @@ def test_product(M, N, K, a_k, b_k, pad):
     assert (got[:, N:] == 7.0).all()
 
 
+# tiles and splits whose count is no multiple of the XCDs: six and five splits of the small tile, several of the large one
+@pytest.mark.parametrize("M,N,K", [(65, 136, 3200), (264, 1288, 3336), (136, 2568, 4104), (200, 2568, 5128), (192, 4104, 1032)])
+@pytest.mark.parametrize("a_k,b_k", [(1, 1), (1, 0), (0, 0)])
+def test_product_shares(M, N, K, a_k, b_k):
+    if _taken(M, K, a_k, b_k):
+        test_product(M, N, K, a_k, b_k, 0)
+
+
 @pytest.mark.parametrize("M,N,K,a_k,b_k", [f for f in FORMS if not _taken(f[0], f[2], f[3], f[4])] + [(64, 12, 64, 1, 1), (0, 64, 64, 1, 1)])
 def test_product_refuses_other_storage(M, N, K, a_k, b_k):
     from mamba2 import _lib
