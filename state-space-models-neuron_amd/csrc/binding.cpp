@@ -100,6 +100,20 @@ Tensor f32(const Tensor& t) { return t.defined() ? t.to(at::kFloat).contiguous()
 Tensor scratch(size_t bytes, const Tensor& like) {
     return at::empty({static_cast<int64_t>(bytes)}, like.options().dtype(at::kByte));
 }
+// Several pieces of one scratch allocation, each on a 256-byte boundary: sizes first, then the pieces in the same order.
+struct Pieces {
+    size_t total = 0, used = 0;
+    Tensor held;
+    static size_t rounded(size_t bytes) { return (bytes + 255) / 256 * 256; }
+    void want(size_t bytes) { total += rounded(bytes); }
+    void allocate(const Tensor& like) { held = scratch(total, like); }
+    void* take(size_t bytes) {
+        TORCH_INTERNAL_ASSERT(used + rounded(bytes) <= total);
+        char* at = static_cast<char*>(held.data_ptr()) + used;
+        used += rounded(bytes);
+        return at;
+    }
+};
 Tensor empty_f32(at::IntArrayRef shape, const Tensor& like) { return at::empty(shape, like.options().dtype(at::kFloat)); }
 
 // ----------------------------------------------------------------------------------------------- conv1d
@@ -146,22 +160,25 @@ Tensor conv1d_forward(const Tensor& input, const Tensor& weight, const OptTensor
 }
 
 // Partial rows of a parameter's gradient, to be summed by a later launch (count == 0: there are none)
-struct Partials { Tensor rows; int64_t count = 0; };
+struct Partials { const float* rows = nullptr; int64_t count = 0; };
 
-// the launch shared by the operator and the fused core; returns (dw, db).  later: where partials go that the caller will have summed
+// the launch shared by the operator and the fused core; returns (dw, db).  later: where partials go that the caller will have summed;
+// they lie in ws, of as many bytes as the library asks for
 std::pair<Tensor, Tensor> launch_conv_bwd(const Strided& x, const Tensor& weight, const Tensor& bias, const Strided& dy, const Strided& dx,
-                                          int64_t b, int64_t l, int64_t c, const Tensor& like, int activation, void* stream, Partials* later = nullptr) {
+                                          int64_t b, int64_t l, int64_t c, const Tensor& like, int activation, void* stream, Partials* later = nullptr,
+                                          void* ws = nullptr) {
     const Tensor w = weight.contiguous(), bi = bias.defined() ? bias.contiguous() : bias;
     Tensor dw = at::empty(w.sizes(), w.options()), db = bi.defined() ? at::empty(bi.sizes(), bi.options()) : Tensor();
     m2_conv1d_params p = conv_params(x, w, bi, dy, b, l, c, dtype_code(like), activation);
     p.dy = dy.p; p.dx = dx.p; p.dw = ptr(dw); p.db = ptr(db);
     p.dx_stride_b = dx.sb; p.dx_stride_l = dx.sl; p.dx_stride_c = dx.sc;
     p.workspace_bytes = lib.m2_conv1d_bwd_workspace_bytes(b, l, c, p.k);
-    const Tensor ws = scratch(p.workspace_bytes, like);
-    p.workspace = ptr(ws);
+    Tensor own;
+    if (!ws) { own = scratch(p.workspace_bytes, like); ws = ptr(own); }
+    p.workspace = ws;
     if (later) {
         check(lib.m2_conv1d_bwd_partial(&p, &later->count, stream), "m2_conv1d_bwd");
-        later->rows = ws;
+        later->rows = static_cast<const float*>(ws);
     } else check(lib.m2_conv1d_bwd(&p, stream), "m2_conv1d_bwd");
     return {dw, db};
 }
@@ -254,8 +271,7 @@ void launch_ssd_fwd(m2_ssd_params& p, const Tensor& like, void* stream) {
     check(lib.m2_ssd_fwd(&p, stream), "m2_ssd_fwd");
 }
 void launch_ssd_bwd(m2_ssd_params& p, const Tensor& like, void* stream) {
-    p.workspace_bytes = lib.m2_ssd_bwd_workspace_bytes(&p);
-    const Tensor ws = scratch(p.workspace_bytes, like);
+    const Tensor ws = scratch(p.workspace_bytes = lib.m2_ssd_bwd_workspace_bytes(&p), like);
     p.workspace = ptr(ws);
     check(lib.m2_ssd_bwd(&p, stream), "m2_ssd_bwd");
 }
@@ -425,14 +441,19 @@ Tensor rmsnorm_forward(const Tensor& x, const OptTensor& z, const Tensor& weight
     return norm.out;
 }
 
-// later: where the partial rows of dw go that the caller will have summed (dw is then undefined)
-std::tuple<Tensor, Tensor, Tensor> launch_norm_bwd(const Tensor& x_, const OptTensor& z_, const Tensor& weight, const Tensor& d_out, int64_t n_groups,
-                                                   double eps, const OptTensor& out_dz, Partials* later) {
+// the gradient of a norm's output as its kernel reads it
+Tensor norm_rows(const Tensor& d_out, at::ScalarType dtype) {
+    Tensor g = d_out.to(dtype);
+    if (g.stride(-1) != 1 || !vec_ok(g)) g = g.clone(at::MemoryFormat::Contiguous);
+    return g;
+}
+
+std::tuple<Tensor, Tensor, Tensor> rmsnorm_backward(const Tensor& x_, const OptTensor& z_, const Tensor& weight, const Tensor& d_out, int64_t n_groups,
+                                                    double eps, const OptTensor& out_dz) {
     require_gpu({&x_, &or_none(z_), &weight, &d_out});
     check_norm(x_, or_none(z_));
     Scope scope(x_);
-    Tensor g = d_out.to(x_.scalar_type());
-    if (g.stride(-1) != 1 || !vec_ok(g)) g = g.clone(at::MemoryFormat::Contiguous);
+    const Tensor g = norm_rows(d_out, x_.scalar_type());
     const Tensor x = aligned(x_), z = z_ ? aligned(*z_) : Tensor(), w32 = f32(weight);
     m2_rmsnorm_params p = norm_params(x, z, w32, n_groups, eps);
     p.d_out = ptr(g); p.d_out_stride_row = rows2d(g, "d_out").stride;
@@ -444,24 +465,17 @@ std::tuple<Tensor, Tensor, Tensor> launch_norm_bwd(const Tensor& x_, const OptTe
         dz = out_dz && vec_ok(*out_dz) ? *out_dz : at::empty(x.sizes(), x.options());
         p.dz = ptr(dz); p.dz_stride_row = rows2d(dz, "out_dz").stride;
     }
-    Tensor dw;
-    if (!later) { dw = empty_f32({x.size(-1)}, x); p.d_weight = ptr<float>(dw); }
+    Tensor dw = empty_f32({x.size(-1)}, x);
+    p.d_weight = ptr<float>(dw);
     p.workspace_bytes = lib.m2_rmsnorm_gated_bwd_workspace_bytes(p.rows, p.channels, p.n_groups, p.dtype);
     const Tensor ws = scratch(p.workspace_bytes, x);
     p.workspace = ptr(ws);
-    if (later) {
-        check(lib.m2_rmsnorm_gated_bwd_partial(&p, &later->count, scope.stream), "m2_rmsnorm_gated_bwd");
-        later->rows = ws;
-    } else check(lib.m2_rmsnorm_gated_bwd(&p, scope.stream), "m2_rmsnorm_gated_bwd");
+    check(lib.m2_rmsnorm_gated_bwd(&p, scope.stream), "m2_rmsnorm_gated_bwd");
     if (z.defined() && out_dz && !dz.is_same(*out_dz)) {
         out_dz->copy_(dz);
         dz = *out_dz;
     }
     return {dx, dw, dz};
-}
-std::tuple<Tensor, Tensor, Tensor> rmsnorm_backward(const Tensor& x, const OptTensor& z, const Tensor& weight, const Tensor& d_out, int64_t n_groups,
-                                                    double eps, const OptTensor& out_dz) {
-    return launch_norm_bwd(x, z, weight, d_out, n_groups, eps, out_dz, nullptr);
 }
 
 struct NormFn : torch::autograd::Function<NormFn> {
@@ -522,16 +536,37 @@ struct Packed {
         b = zx.size(0); l = zx.size(1); sb = zx.stride(0); sl = zx.stride(1);
     }
     Tensor z() const { return zx.narrow(2, 0, d); }
-    Tensor dt() const { return zx.narrow(2, d + conv, h); }
+    // z where the norm reads it: in zx if its rows lie on 16 bytes there, else a copy that `held` keeps
+    std::pair<const void*, int64_t> z_rows(Tensor& held) const {
+        if (reinterpret_cast<uintptr_t>(zx.data_ptr()) % 16 == 0 && (sl * zx.element_size()) % 16 == 0) return {zx.data_ptr(), sl};
+        held = z().clone(at::MemoryFormat::Contiguous);
+        return {ptr(held), d};
+    }
     Strided xBC() const { return {at_column(zx, d), sb, sl, 1}; }
 };
 
+// The per-head and per-channel parameters in fp32, contiguous.  As pointers: the whole layer holds them in one buffer, and a view of
+// a part of it costs the host more than a launch's arguments.
+struct CoreParams { const float *A, *D, *dt_bias, *norm_w; };
+CoreParams core_params(const Tensor& A, const Tensor& D, const Tensor& dt_bias, const Tensor& norm_w) {
+    return {ptr<float>(A), ptr<float>(D), ptr<float>(dt_bias), ptr<float>(norm_w)};
+}
+
+// the norm's parameters: the scan's output, gated by z, per group
+m2_rmsnorm_params core_norm_params(const Packed& k, const CoreParams& w, const void* scan_out, const std::pair<const void*, int64_t>& z) {
+    m2_rmsnorm_params p{};
+    p.x = scan_out; p.x_stride_row = k.d; p.z = z.first; p.z_stride_row = z.second;
+    p.rows = k.b * k.l; p.channels = k.d; p.n_groups = static_cast<int32_t>(k.g);
+    p.dtype = dtype_code(k.zx); p.eps = static_cast<float>(kNormEps); p.weight = w.norm_w;
+    return p;
+}
+
 // the scan's parameters with x, B and C as columns of the packed conv output
-m2_ssd_params core_ssd_params(const Packed& k, const Tensor& conv_out, const Tensor& A, const Tensor& D, const Tensor& dt_bias) {
+m2_ssd_params core_ssd_params(const Packed& k, const Tensor& conv_out, const CoreParams& w) {
     m2_ssd_params p{};
     const int64_t sb = conv_out.stride(0), sl = conv_out.stride(1);
     p.x = ptr(conv_out); p.B = at_column(conv_out, k.d); p.C = at_column(conv_out, k.d + k.g * k.n); p.dt = at_column(k.zx, k.d + k.conv);
-    p.A = ptr<float>(A); p.D = ptr<float>(D); p.dt_bias = ptr<float>(dt_bias);
+    p.A = w.A; p.D = w.D; p.dt_bias = w.dt_bias;
     p.batch = k.b; p.seqlen = k.l; p.nheads = k.h; p.headdim = k.p; p.dstate = k.n; p.ngroups = k.g;
     p.x_stride_b = p.B_stride_b = p.C_stride_b = sb;
     p.x_stride_l = p.B_stride_l = p.C_stride_l = sl;
@@ -552,16 +587,15 @@ void check_core(const Packed& k, const Tensor& A, const Tensor& D, const Tensor&
 }
 
 struct CoreOut { Tensor norm_out, conv_out, scan_out, states; };
-// A, D, dt_bias fp32.  want_norm false: only what the backward needs (conv output, scan output, chunk states).
-CoreOut core_forward(const Packed& k, const Tensor& A, const Tensor& D, const Tensor& conv_w, const Tensor& conv_b, const Tensor& dt_bias,
-                     const Tensor& norm_w, bool keep_states, bool want_norm, void* stream) {
+// want_norm false: only what the backward needs (conv output, scan output, chunk states).
+CoreOut core_forward(const Packed& k, const CoreParams& params, const Tensor& conv_w, const Tensor& conv_b, bool keep_states, bool want_norm, void* stream) {
     CoreOut r;
     r.conv_out = at::empty({k.b, k.l, k.conv}, k.zx.options());
     const Tensor w = conv_w.contiguous(), bi = conv_b.defined() ? conv_b.contiguous() : conv_b;
     m2_conv1d_params c = conv_params(k.xBC(), w, bi, {ptr(r.conv_out), k.l * k.conv, k.conv, 1}, k.b, k.l, k.conv, dtype_code(k.zx), M2_ACT_SILU);
     c.y = ptr(r.conv_out);
     check(lib.m2_conv1d_fwd(&c, stream), "m2_conv1d_fwd");
-    m2_ssd_params p = core_ssd_params(k, r.conv_out, A, D, dt_bias);
+    m2_ssd_params p = core_ssd_params(k, r.conv_out, params);
     if (keep_states && k.zx.numel() > 0) {
         r.states = scratch(lib.m2_ssd_chunk_states_bytes(&p), k.zx);
         p.chunk_states = ptr(r.states);
@@ -569,52 +603,83 @@ CoreOut core_forward(const Packed& k, const Tensor& A, const Tensor& D, const Te
     r.scan_out = at::empty({k.b, k.l, k.d}, k.zx.options());
     p.y = ptr(r.scan_out); p.y_stride_b = k.l * k.d; p.y_stride_l = k.d; p.y_stride_h = k.p;
     launch_ssd_fwd(p, k.zx, stream);
-    if (want_norm) r.norm_out = rmsnorm_forward(r.scan_out, k.z(), norm_w, k.g, kNormEps, k.zx.scalar_type());
+    if (want_norm) {
+        Tensor held;
+        m2_rmsnorm_params q = core_norm_params(k, params, ptr(r.scan_out), k.z_rows(held));
+        r.norm_out = at::empty({k.b, k.l, k.d}, k.zx.options());
+        q.out = ptr(r.norm_out); q.out_stride_row = k.d;
+        check(lib.m2_rmsnorm_gated_fwd(&q, stream), "m2_rmsnorm_gated_fwd");
+    }
     return r;
 }
 
 // types that the kernels for the small parameters read and write
 bool casts(const Tensor& t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16; }
 
-struct CoreGrads { Tensor zx, A, D, conv_w, conv_b, dt_bias, norm_w; };
+struct CoreGrads {
+    Tensor zx, heads, conv_w, conv_b, norm_w;      // heads: rows of A, dt_bias and D, unless they went into head_grads
+    Tensor head(int64_t row, const Tensor& param) const { return heads.select(0, row).to(param.scalar_type()); }
+};
 // The packed gradient has rows of whole 128-byte cache lines (10576 columns of bf16 are 165.25 lines, and every wave-wide
 // access to a column slice of such a buffer straddles two lines in three rows out of four); its consumers take a leading
 // dimension.
 // The sums of the norm weight's and the conv's partials run in one launch at the end, the former into norm_param's type; with
 // head_grads (of A_log, D and dt_bias, in their types) it also leaves those.
-CoreGrads core_backward(const Packed& k, const Tensor& d_out, const Tensor& A, const Tensor& D, const Tensor& conv_w, const Tensor& conv_b,
-                        const Tensor& dt_bias, const Tensor& norm_w, const Tensor& conv_out, const Tensor& scan_out, const Tensor& states,
-                        const Tensor& norm_param, const variable_list& head_grads, void* stream) {
+CoreGrads core_backward(const Packed& k, const Tensor& d_out_, const CoreParams& w, const Tensor& conv_w, const Tensor& conv_b, const Tensor& conv_out,
+                        const Tensor& scan_out, const Tensor& states, const Tensor& norm_param, const variable_list& head_grads, void* stream) {
     CoreGrads r;
-    Partials norm_rows, conv_rows;
+    Partials norm_sums, conv_rows;
     const int64_t width = k.zx.size(2), per_line = 128 / k.zx.element_size(), pitch = (width + per_line - 1) / per_line * per_line;
     r.zx = at::empty({k.b, k.l, pitch}, k.zx.options());
     if (pitch != width) r.zx = r.zx.narrow(2, 0, width);
-    const Tensor d_scan = std::get<0>(launch_norm_bwd(scan_out, k.z(), norm_w, d_out, k.g, kNormEps, r.zx.narrow(2, 0, k.d), &norm_rows));
-    // the scan's gradients leave as one packed [dx | dB | dC] buffer, that of the raw dt in its columns of r.zx
-    const Tensor d_conv = at::empty({k.b, k.l, k.conv}, k.zx.options());
-    m2_ssd_params p = core_ssd_params(k, conv_out, A, D, dt_bias);
+    char* const d_zx = static_cast<char*>(r.zx.data_ptr());
+    const Tensor d_out = norm_rows(d_out_, k.zx.scalar_type());
+    const bool to_heads = !head_grads.empty();
+    // everything that does not leave this function, in one allocation
+    Tensor held;
+    require_gpu({&d_out, &scan_out, &conv_out});
+    TORCH_CHECK_VALUE(scan_out.dim() == 3 && scan_out.size(0) == k.b && scan_out.size(1) == k.l && scan_out.size(2) == k.d &&
+                          scan_out.scalar_type() == k.zx.scalar_type(), "scan_out must be (b, l, d_inner) in the dtype of zxBCdt");
+    const Tensor scanned = aligned(scan_out);
+    m2_rmsnorm_params q = core_norm_params(k, w, ptr(scanned), k.z_rows(held));
+    q.x_stride_row = rows2d(scanned, "scan_out").stride;
+    m2_ssd_params p = core_ssd_params(k, conv_out, w);
     p.chunk_states = chunk_states_ptr(p, states);
-    p.dy = ptr(d_scan); p.dy_stride_b = k.l * k.d; p.dy_stride_l = k.d; p.dy_stride_h = k.p;
-    p.dx = ptr(d_conv); p.dB = at_column(d_conv, k.d); p.dC = at_column(d_conv, k.d + k.g * k.n);
+    p.dy_stride_b = k.l * k.d; p.dy_stride_l = k.d; p.dy_stride_h = k.p;
     p.dx_stride_b = p.dB_stride_b = p.dC_stride_b = k.l * k.conv;
     p.dx_stride_l = p.dB_stride_l = p.dC_stride_l = k.conv;
     p.dx_stride_h = k.p; p.dB_stride_g = p.dC_stride_g = k.n;
-    p.ddt = at_column(r.zx, k.d + k.conv); p.ddt_stride_b = r.zx.stride(0); p.ddt_stride_l = r.zx.stride(1);
-    const Tensor heads = empty_f32({3, k.h}, k.zx);
-    r.A = heads.select(0, 0); r.dt_bias = heads.select(0, 1);
-    if (D.defined()) r.D = heads.select(0, 2);
-    p.dA = ptr<float>(r.A); p.dD = ptr<float>(r.D); p.d_dt_bias = ptr<float>(r.dt_bias);
-    launch_ssd_bwd(p, k.zx, stream);
-    std::tie(r.conv_w, r.conv_b) = launch_conv_bwd(k.xBC(), conv_w, conv_b, {ptr(d_conv), k.l * k.conv, k.conv, 1},
-                                                   {at_column(r.zx, k.d), r.zx.stride(0), r.zx.stride(1), 1}, k.b, k.l, k.conv, k.zx, M2_ACT_SILU, stream, &conv_rows);
+    p.ddt_stride_b = k.l * pitch; p.ddt_stride_l = pitch;
+    const size_t es = k.zx.element_size(), d_scan_bytes = static_cast<size_t>(k.b * k.l * k.d) * es, d_conv_bytes = static_cast<size_t>(k.b * k.l * k.conv) * es,
+                 heads_bytes = to_heads ? static_cast<size_t>(3 * k.h) * 4 : 0, conv_bytes = lib.m2_conv1d_bwd_workspace_bytes(k.b, k.l, k.conv, conv_w.size(2));
+    q.workspace_bytes = lib.m2_rmsnorm_gated_bwd_workspace_bytes(q.rows, q.channels, q.n_groups, q.dtype);
+    p.workspace_bytes = lib.m2_ssd_bwd_workspace_bytes(&p);
+    Pieces pieces;
+    for (const size_t bytes : {d_scan_bytes, d_conv_bytes, heads_bytes, conv_bytes, q.workspace_bytes, p.workspace_bytes}) pieces.want(bytes);
+    pieces.allocate(k.zx);
+    void* const d_scan = pieces.take(d_scan_bytes);
+    char* const d_conv = static_cast<char*>(pieces.take(d_conv_bytes));
+    if (!to_heads) r.heads = empty_f32({3, k.h}, k.zx);
+    float* const heads = to_heads ? static_cast<float*>(pieces.take(heads_bytes)) : ptr<float>(r.heads);
+    void* const conv_ws = pieces.take(conv_bytes);
+    // norm: dz into its columns of r.zx
+    q.d_out = ptr(d_out); q.d_out_stride_row = rows2d(d_out, "d_out").stride;
+    q.dx = d_scan; q.dx_stride_row = k.d; q.dz = d_zx; q.dz_stride_row = pitch;
+    q.workspace = pieces.take(q.workspace_bytes);
+    check(lib.m2_rmsnorm_gated_bwd_partial(&q, &norm_sums.count, stream), "m2_rmsnorm_gated_bwd");
+    norm_sums.rows = static_cast<const float*>(q.workspace);
+    // the scan's gradients leave as one packed [dx | dB | dC] buffer, that of the raw dt in its columns of r.zx
+    p.dy = d_scan; p.dx = d_conv; p.dB = d_conv + k.d * es; p.dC = d_conv + (k.d + k.g * k.n) * es; p.ddt = d_zx + (k.d + k.conv) * es;
+    p.dA = heads; p.d_dt_bias = heads + k.h; p.dD = w.D ? heads + 2 * k.h : nullptr;
+    p.workspace = pieces.take(p.workspace_bytes);
+    check(lib.m2_ssd_bwd(&p, stream), "m2_ssd_bwd");
+    std::tie(r.conv_w, r.conv_b) = launch_conv_bwd(k.xBC(), conv_w, conv_b, {d_conv, k.l * k.conv, k.conv, 1}, {d_zx + k.d * es, k.l * pitch, pitch, 1}, k.b, k.l,
+                                                   k.conv, k.zx, M2_ACT_SILU, stream, &conv_rows, conv_ws);
     r.norm_w = at::empty({k.d}, casts(norm_param) ? norm_param.options() : norm_param.options().dtype(at::kFloat));
-    const bool to_heads = !head_grads.empty();
     auto head = [&](size_t i) { return to_heads && head_grads[i].defined() ? ptr(head_grads[i]) : nullptr; };
     auto head_type = [&](size_t i) { return to_heads && head_grads[i].defined() ? dtype_code(head_grads[i]) : M2_F32; };
-    check(lib.m2_param_sums(ptr<float>(norm_rows.rows), norm_rows.count, k.d, ptr(r.norm_w), dtype_code(r.norm_w), ptr<float>(conv_rows.rows),
-                            conv_rows.count, k.conv, ptr(r.conv_w), ptr(r.conv_b), dtype_code(r.conv_w), to_heads ? k.h : 0, ptr<float>(A), ptr<float>(r.A),
-                            ptr<float>(r.D), ptr<float>(r.dt_bias), head(0), head_type(0), head(1), head_type(1), head(2), head_type(2), stream),
+    check(lib.m2_param_sums(norm_sums.rows, norm_sums.count, k.d, ptr(r.norm_w), dtype_code(r.norm_w), conv_rows.rows, conv_rows.count, k.conv,
+                            ptr(r.conv_w), ptr(r.conv_b), dtype_code(r.conv_w), to_heads ? k.h : 0, w.A, p.dA, p.dD, p.d_dt_bias, head(0), head_type(0), head(1), head_type(1), head(2), head_type(2), stream),
           "m2_param_sums");
     return r;
 }
@@ -624,7 +689,8 @@ py::tuple forward_parts(const Tensor& zx, const Tensor& A, const OptTensor& D, c
     Scope scope(zx);
     const Packed k(zx, g, n, d, hd);
     check_core(k, A, or_none(D), conv_w, or_none(conv_b), dt_bias, norm_w);
-    const CoreOut r = core_forward(k, f32(A), f32(or_none(D)), conv_w, or_none(conv_b), f32(dt_bias), norm_w, keep_states, true, scope.stream);
+    const Tensor A32 = f32(A), D32 = f32(or_none(D)), bias = f32(dt_bias), norm32 = f32(norm_w);
+    const CoreOut r = core_forward(k, core_params(A32, D32, bias, norm32), conv_w, or_none(conv_b), keep_states, true, scope.stream);
     return py::make_tuple(r.norm_out, r.conv_out, r.scan_out, r.states);
 }
 py::tuple backward_parts(const Tensor& d_out, const Tensor& zx, const Tensor& A, const OptTensor& D, const Tensor& conv_w, const OptTensor& conv_b,
@@ -633,9 +699,10 @@ py::tuple backward_parts(const Tensor& d_out, const Tensor& zx, const Tensor& A,
     Scope scope(zx);
     const Packed k(zx, g, n, d, hd);
     check_core(k, A, or_none(D), conv_w, or_none(conv_b), dt_bias, norm_w);
-    const CoreGrads r = core_backward(k, d_out, f32(A), f32(or_none(D)), conv_w, or_none(conv_b), f32(dt_bias), norm_w, conv_out, scan_out,
-                                      or_none(states), norm_w, {}, scope.stream);
-    return py::make_tuple(r.zx, r.A.to(A.scalar_type()), D ? r.D.to(D->scalar_type()) : Tensor(), r.conv_w, r.conv_b, r.dt_bias.to(dt_bias.scalar_type()),
+    const Tensor A32 = f32(A), D32 = f32(or_none(D)), bias = f32(dt_bias), norm32 = f32(norm_w);
+    const CoreGrads r = core_backward(k, d_out, core_params(A32, D32, bias, norm32), conv_w, or_none(conv_b), conv_out, scan_out, or_none(states), norm_w, {},
+                                      scope.stream);
+    return py::make_tuple(r.zx, r.head(0, A), D ? r.head(2, *D) : Tensor(), r.conv_w, r.conv_b, r.head(1, dt_bias),
                           r.norm_w.to(norm_w.scalar_type()));
 }
 
@@ -647,7 +714,8 @@ struct CoreFn : torch::autograd::Function<CoreFn> {
         Scope scope(zx);
         const Packed k(zx, g, n, d, hd);
         check_core(k, A, or_none(D), conv_w, or_none(conv_b), dt_bias, norm_w);
-        const CoreOut r = core_forward(k, f32(A), f32(or_none(D)), conv_w, or_none(conv_b), f32(dt_bias), norm_w, keep, true, scope.stream);
+        const Tensor A32 = f32(A), D32 = f32(or_none(D)), bias = f32(dt_bias), norm32 = f32(norm_w);
+        const CoreOut r = core_forward(k, core_params(A32, D32, bias, norm32), conv_w, or_none(conv_b), keep, true, scope.stream);
         variable_list saved = {zx, A, or_none(D), conv_w, or_none(conv_b), dt_bias, norm_w};
         if (keep) { saved.push_back(r.conv_out); saved.push_back(r.scan_out); saved.push_back(r.states); }
         ctx->save_for_backward(std::move(saved));
@@ -660,14 +728,15 @@ struct CoreFn : torch::autograd::Function<CoreFn> {
         Scope scope(s[0]);
         const Packed k(s[0], dims[0], dims[1], dims[2], dims[3]);
         const Tensor A = f32(s[1]), D = f32(s[2]), dt_bias = f32(s[5]), norm_w = f32(s[6]);
+        const CoreParams params = core_params(A, D, dt_bias, norm_w);
         CoreOut f;
         if (s.size() > 7) { f.conv_out = s[7]; f.scan_out = s[8]; f.states = s[9]; }
-        else f = core_forward(k, A, D, s[3], s[4], dt_bias, norm_w, true, false, scope.stream);
-        const CoreGrads r = core_backward(k, grads[0], A, D, s[3], s[4], dt_bias, norm_w, f.conv_out, f.scan_out, f.states, s[6], {}, scope.stream);
+        else f = core_forward(k, params, s[3], s[4], true, false, scope.stream);
+        const CoreGrads r = core_backward(k, grads[0], params, s[3], s[4], f.conv_out, f.scan_out, f.states, s[6], {}, scope.stream);
         variable_list out(12);
-        out[0] = r.zx; out[1] = r.A.to(s[1].scalar_type());
-        if (s[2].defined()) out[2] = r.D.to(s[2].scalar_type());
-        out[3] = r.conv_w; out[4] = r.conv_b; out[5] = r.dt_bias.to(s[5].scalar_type()); out[6] = r.norm_w.to(s[6].scalar_type());
+        out[0] = r.zx; out[1] = r.head(0, s[1]);
+        if (s[2].defined()) out[2] = r.head(2, s[2]);
+        out[3] = r.conv_w; out[4] = r.conv_b; out[5] = r.head(1, s[5]); out[6] = r.norm_w.to(s[6].scalar_type());
         return out;
     }
 };
@@ -728,6 +797,11 @@ Tensor small_param(const Tensor& t) { return (casts(t) ? t : t.to(at::kFloat)).c
 
 struct MixerFn : torch::autograd::Function<MixerFn> {
     enum { kHidden, kInW, kALog, kD, kDtBias, kConvW, kNormW, kOutW, kConvB, kInB, kOutB, kSmall, kZx, kNormOut, kConvOut, kScanOut, kStates };
+    // the casting kernel leaves A, D and dt_bias (a value per head each) and the norm's weight one behind the other
+    static CoreParams params_in(const Tensor& small, int64_t h) {
+        const float* at = ptr<float>(small);
+        return {at, at + h, at + 2 * h, at + 3 * h};
+    }
     static Tensor forward(AutogradContext* ctx, const Tensor& hidden, const Tensor& in_w, const Tensor& A_log, const Tensor& D, const Tensor& dt_bias,
                           const Tensor& conv_w, const Tensor& norm_w, const Tensor& out_w, const OptTensor& conv_b, const OptTensor& in_b,
                           const OptTensor& out_b, int64_t g, int64_t n, int64_t d, int64_t hd, bool differentiable, bool recompute) {
@@ -741,8 +815,7 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
         const Tensor a = small_param(A_log), dd = small_param(D), tb = small_param(dt_bias), nw = small_param(norm_w);
         check(lib.m2_mixer_params(ptr(a), dtype_code(a), ptr(dd), dtype_code(dd), ptr(tb), dtype_code(tb), ptr(nw), dtype_code(nw), ptr<float>(small),
                                   h, d, scope.stream), "m2_mixer_params");
-        const CoreOut r = core_forward(k, small.narrow(0, 0, h), small.narrow(0, h, h), conv_w, or_none(conv_b), small.narrow(0, 2 * h, h),
-                                       small.narrow(0, 3 * h, d), differentiable && !recompute, true, scope.stream);
+        const CoreOut r = core_forward(k, params_in(small, h), conv_w, or_none(conv_b), differentiable && !recompute, true, scope.stream);
         const Tensor y = r.norm_out.view({b * l, d});
         if (differentiable) {
             variable_list saved = {hidden, in_w, A_log, D, dt_bias, conv_w, norm_w, out_w, or_none(conv_b), or_none(in_b), or_none(out_b), small, zx, y};
@@ -760,7 +833,7 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
         const Packed k(zx, dims[0], dims[1], dims[2], dims[3]);
         const int64_t rows = k.b * k.l;
         const Tensor& small = s[kSmall];
-        const Tensor A = small.narrow(0, 0, k.h), D = small.narrow(0, k.h, k.h), dt_bias = small.narrow(0, 2 * k.h, k.h), norm_w = small.narrow(0, 3 * k.h, k.d);
+        const CoreParams params = params_in(small, k.h);
         variable_list out(17);
         const Tensor dy = grads[0].reshape({rows, s[kOutW].size(0)});
         if (ctx->needs_input_grad(kOutW)) out[kOutW] = product(dy, false, s[kNormOut], false, Tensor(), scope.stream);
@@ -768,9 +841,9 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
         const Tensor d_core = product(dy, true, s[kOutW], false, Tensor(), scope.stream).view({k.b, k.l, k.d});
         CoreOut f;
         if (s.size() > kConvOut) { f.conv_out = s[kConvOut]; f.scan_out = s[kScanOut]; f.states = s[kStates]; }
-        else f = core_forward(k, A, D, s[kConvW], s[kConvB], dt_bias, norm_w, true, false, scope.stream);
+        else f = core_forward(k, params, s[kConvW], s[kConvB], true, false, scope.stream);
         for (const int i : {kALog, kD, kDtBias}) out[i] = at::empty(s[i].sizes(), casts(s[i]) ? s[i].options() : s[i].options().dtype(at::kFloat));
-        const CoreGrads r = core_backward(k, d_core, A, D, s[kConvW], s[kConvB], dt_bias, norm_w, f.conv_out, f.scan_out, f.states, s[kNormW],
+        const CoreGrads r = core_backward(k, d_core, params, s[kConvW], s[kConvB], f.conv_out, f.scan_out, f.states, s[kNormW],
                                           {out[kALog], out[kD], out[kDtBias]}, scope.stream);
         out[kNormW] = r.norm_w.view(s[kNormW].sizes());
         for (const int i : {kALog, kD, kDtBias, kNormW})
@@ -821,7 +894,7 @@ Tensor fused_prefill(const Tensor& zx, const Tensor& A, const OptTensor& D, cons
     // The conv moves the cache on, so everything behind it is allocated and checked first: a call that is refused leaves the cache
     // as it was.
     const Tensor A32 = f32(A), D32 = f32(or_none(D)), bias = f32(dt_bias);
-    m2_ssd_params p = core_ssd_params(k, conv_out, A32, D32, bias);
+    m2_ssd_params p = core_ssd_params(k, conv_out, core_params(A32, D32, bias, Tensor()));
     const Tensor y = at::empty({k.b, k.l, d}, zx.options());
     p.initial_state = continuing ? ptr<float>(S) : nullptr; p.final_state = ptr<float>(S);
     p.y = ptr(y); p.y_stride_b = k.l * d; p.y_stride_l = d; p.y_stride_h = hd;
