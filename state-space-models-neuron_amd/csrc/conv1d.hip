@@ -478,20 +478,24 @@ conv_fwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
 }
 
 // One wave per (channel, split): its lanes walk the channel's pieces of two vectors of tokens over all rows of the batch,
-// so the sums of dw and db stay in registers until the end and one wave's reduction finishes a channel (splits > 1: fp32
-// partials for conv_reduce_partials_kernel).  A lane recomputes the three tokens behind its own for the dx lag: 3 in 16
+// so the sums of dw and db stay in registers until the end.  The 1, 2 or 4 (`inner`) splits of a channel inside a workgroup meet in
+// LDS and finish it there; only with more of them (few channels) do fp32 partials go to conv_reduce_partials_kernel, whose launch
+// took 4.3 us beside the 70 of this kernel at b4 l2048 C5376 (two splits; forward and backward 125.7 -> 123.5 us in a stream of them; with
+// one split the chip is short of waves, 131 -> 141 in an eager loop).
+// A lane recomputes the three tokens behind its own for the dx lag: 3 in 16
 // (bf16) more activations, against a cross-lane exchange that would break at every row end.
 template <typename T, typename WT, int ACT>
 __global__ void __launch_bounds__(256)
 conv_bwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias, const T* __restrict__ dy,
                    T* __restrict__ dx, float* __restrict__ part, void* __restrict__ dw, void* __restrict__ db,
-                   int64_t l, uint32_t C, uint32_t splits, uint32_t pieces, uint32_t per_split, uint32_t total,
+                   int64_t l, uint32_t C, uint32_t inner, uint32_t outer, uint32_t pieces, uint32_t per_split, uint32_t total,
                    int64_t xsb, int64_t xsc, int64_t gsb, int64_t gsc, int64_t dsb, int64_t dsc) {
     constexpr int V = VecTraits<T>::kVec, N = 2 * V;
-    const uint32_t unit = blockIdx.x * 4u + (threadIdx.x >> 6);
-    if (unit >= C * splits) return;
-    const uint32_t split = unit / C, c = unit - split * C;
-    const uint32_t end = (split + 1) * per_split < total ? (split + 1) * per_split : total;
+    __shared__ float red[4][5];
+    const uint32_t wave = threadIdx.x >> 6, unit = (blockIdx.x * 4u + wave) / inner, sub = wave & (inner - 1);
+    const bool live = unit < C * outer;            // the last workgroup may have fewer channels
+    const uint32_t part_row = live ? unit / C : 0, c = live ? unit - part_row * C : 0, split = part_row * inner + sub;
+    const uint32_t end = !live ? 0 : (split + 1) * per_split < total ? (split + 1) * per_split : total;
     float wv[4], bv, acc[5];
     ld_row_taps<WT>(w, bias, c, wv, bv);
 #pragma unroll
@@ -537,13 +541,17 @@ conv_bwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
 #pragma unroll
     for (int k = 0; k < 5; ++k) acc[k] = warp_sum(acc[k]);
     if ((threadIdx.x & 63) == 0) {
-        constexpr int pd = std::is_same<WT, float>::value ? M2_F32 : M2_BF16;
 #pragma unroll
-        for (int k = 0; k < 5; ++k) {
-            if (splits > 1) part[((int64_t)split * C + c) * 5 + k] = acc[k];
-            else if (k < 4) st_param(dw, pd, (int64_t)c * 4 + k, acc[k]);
-            else if (db) st_param(db, pd, c, acc[k]);
-        }
+        for (int k = 0; k < 5; ++k) red[wave][k] = acc[k];
+    }
+    __syncthreads();
+    if (const uint32_t k = threadIdx.x & 63; live && sub == 0 && k < 5) {
+        constexpr int pd = std::is_same<WT, float>::value ? M2_F32 : M2_BF16;
+        float v = 0.f;
+        for (uint32_t q = 0; q < inner; ++q) v += red[wave + q][k];
+        if (outer > 1) part[((int64_t)part_row * C + c) * 5 + k] = v;
+        else if (k < 4) st_param(dw, pd, (int64_t)c * 4 + k, v);
+        else if (db) st_param(db, pd, c, v);
     }
 }
 
@@ -772,23 +780,22 @@ int launch_bwd(const m2_conv1d_params* p, int64_t* slots, hipStream_t st) {
     if (channel_major_ok(p, true)) {
         const int64_t pieces = ceil_div(l, (int64_t)(2 * VecTraits<T>::kVec)), total = nb * pieces;
         // enough waves to fill the chip (about 24 per CU), each with at least one whole round of its lanes; never more
-        // splits than the partial rows that m2_conv1d_bwd_workspace_bytes sizes
+        // partial rows than m2_conv1d_bwd_workspace_bytes sizes
         int64_t splits = ceil_div((int64_t)24 * device_cus(), C);
         if (splits > total / 64) splits = total / 64;
         if (splits < 1) splits = 1;
-        const int64_t per_split = ceil_div(total, splits);
-        splits = ceil_div(total, per_split);
+        const int64_t inner = splits > 2 ? 4 : splits, outer = ceil_div(splits, inner), per_split = ceil_div(total, inner * outer);
         float* part = static_cast<float*>(p->workspace);
-        M2_REQUIRE(splits == 1 || (part && p->workspace_bytes >= (size_t)(splits * C * 5) * sizeof(float)), M2_ERR_WORKSPACE,
-                   "conv1d_bwd: workspace %zu bytes < %zu needed", p->workspace_bytes, (size_t)(splits * C * 5) * sizeof(float));
+        M2_REQUIRE(outer == 1 || (part && p->workspace_bytes >= (size_t)(outer * C * 5) * sizeof(float)), M2_ERR_WORKSPACE,
+                   "conv1d_bwd: workspace %zu bytes < %zu needed", p->workspace_bytes, (size_t)(outer * C * 5) * sizeof(float));
         conv_dispatch(p, [&](auto wt, auto act) {
-            conv_bwd_cm_kernel<T, decltype(wt), decltype(act)::value><<<(unsigned)ceil_div(C * splits, (int64_t)4), 256, 0, st>>>(
-                x, p->w, p->bias, dy, dx, part, p->dw, p->db, l, (uint32_t)C, (uint32_t)splits, (uint32_t)pieces, (uint32_t)per_split,
+            conv_bwd_cm_kernel<T, decltype(wt), decltype(act)::value><<<(unsigned)ceil_div(C * outer * inner, (int64_t)4), 256, 0, st>>>(
+                x, p->w, p->bias, dy, dx, part, p->dw, p->db, l, (uint32_t)C, (uint32_t)inner, (uint32_t)outer, (uint32_t)pieces, (uint32_t)per_split,
                 (uint32_t)total, p->x_stride_b, p->x_stride_c, p->y_stride_b, p->y_stride_c, p->dx_stride_b, p->dx_stride_c);
         });
         int rc = check_launch("conv1d_bwd");
-        if (rc || splits == 1) return rc;
-        conv_reduce_partials_kernel<<<(unsigned)ceil_div(C * 5 * 4, (int64_t)256), 256, 0, st>>>(part, splits, C, 4, p->dw, p->db, p->param_dtype);
+        if (rc || outer == 1) return rc;
+        conv_reduce_partials_kernel<<<(unsigned)ceil_div(C * 5 * 4, (int64_t)256), 256, 0, st>>>(part, outer, C, 4, p->dw, p->db, p->param_dtype);
         return check_launch("conv1d_bwd_reduce");
     }
     const int64_t total = nb * l * C;

@@ -101,3 +101,10 @@ def test_conv_segment_lengths(b, l, C):
     for name, a, r in zip(("y", "dx", "dw", "db"), got, (ref.detach(), *grads)):
         # one bf16 rounding of the result (2^-9 of it; heavy tails count against the tensor's norm) behind fp32 sums
         assert (a.float() - r).norm() / r.norm() < 2.0 ** -8, name
+
+
+# channel-major backward: the splits of a channel inside a workgroup (two, four) and in several partial rows; a last workgroup that is not full
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,l,C,act", [(1, 2048, 3075, "silu"), (2, 2050, 2049, None), (2, 4100, 1023, "silu")])
+def test_conv_channel_major_splits(dtype, b, l, C, act):
+    test_conv_layout_edges(dtype, False, b, l, C, act)
