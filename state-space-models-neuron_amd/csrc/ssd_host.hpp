@@ -62,7 +62,7 @@ inline void ssd_slicing(const SsdCall* p, int wgs_per_cu, bool partials, int64_t
 }
 constexpr int kWgsChunkState32 = 2, kWgsY = 2, kWgsY32 = 1, kWgsDx = 1, kWgsDg = 1;
 
-// The same for the backward of fp32 operands, whose heads take four times as long (15 us): in heads, rounds of workgroups x (heads
+// The same for the backward of fp32 operands, whose heads take 61 k cycles: in heads, rounds of workgroups x (heads
 // per slice + one for the way in and the finish), and for more than one slice the partials' way out, back and through kernels of
 // their own.
 inline void ssd_slicing32(const SsdCall* p, int64_t* nslices, int64_t* hps) {

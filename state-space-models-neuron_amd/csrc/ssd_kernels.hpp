@@ -46,7 +46,7 @@ __device__ __forceinline__ int64_t mt_offset(int n, int s0) {
 
 // The four elements k = 16 (u / 2) + 8 half + 4 (u % 2) + 0..3 of operand row 32 rb + r, fp32: step u of row block rb is one contiguous
 // KiB, lane 32 half + r (a step straight from rows touches 32 of them, 2 x 16 bytes each: the loads of B and of C B^T then held the
-// phase of ssd_bwd32_kernel that needs them for 23 k cycles instead of 13).
+// phase of ssd_bwd32_kernel that needs them for 23.5 k cycles instead of 21.5).
 template <int STEPS>
 __device__ __forceinline__ int op32_offset(int rb, int u, int lane) { return ((rb * STEPS + u) * 64 + lane) * 4; }
 
@@ -56,7 +56,7 @@ constexpr int kCbParts = 7, kCbGParts = 3;
 constexpr int kXcds = 8;
 __host__ __device__ inline int64_t cb_blocks(int64_t n_cb, int parts) { return (n_cb + kXcds - 1) / kXcds * kXcds * parts; }
 // Contraction length staged at once: all of it (one staging phase, one barrier), but fp32 rows of 128 in two halves, so that
-// four workgroups fit a CU and not two (66 -> 51 us at b3 l2048 h32 g8).
+// four workgroups fit a CU and not two (66 -> 51 us at b3 l2048 h32 g8 with transposed tiles of B and C, 33 since B is copied as it lies).
 template <typename T> __host__ __device__ constexpr int cb_kh(int n) { return sizeof(T) == 4 && n > 64 ? n / 2 : n; }
 template <typename T, int N>
 __device__ __forceinline__ void
