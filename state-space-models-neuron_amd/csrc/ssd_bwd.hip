@@ -34,8 +34,8 @@
 //                                                                partial state parts of dB / dC
 //   [ssd_bwd32_kernel         what those two do in one pass; dB and dC too where a workgroup has all heads of its group]
 //   tail1_kernel              da_body: ddt, dA partials per (b, head, chunk);  slice_sum_body: partials over the head slices
-//   tail2_kernel              bc_final16_body [bc_final32_body] per (b, chunk, group): dC = dG B + dCoff, dB = dG^T C + dBoff;
-//                             ad_reduce_body per head: dA, dD (fixed order, no atomics)
+//   tail2_kernel              group_finish16_body per (b, chunk, group, token block) [bc_final32_body per (b, chunk, group)], unless done
+//                             already: dC = dG B + dCoff, dB = dG^T C + dBoff;  ad_reduce_body per head: dA, dD (fixed order, no atomics)
 #include "ssd_host.hpp"
 
 namespace m2 {
@@ -71,119 +71,92 @@ tail1_kernel(const DaArgs d, const int64_t n_da, const SliceSumArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------
-// Group-level finish for 16-bit operands, both sides in one workgroup of 8 waves, so that the head-summed dG is read once:
-//   waves 0-3 (row block w):      dC[i][n] = sum_{j<=i} dG[i][j] B[j][n] + dCoff[i][n]
-//   waves 4-7 (row block w - 4):  dB[j][n] = sum_{i>=j} dG[i][j] C[i][n] + dBoff[j][n]
-// (wave w and wave w + 4 share a SIMD: 2w + 2 and 8 - 2w k blocks, ten on every SIMD).  dG is split into hi + lo
-// operand-type tiles in LDS (row-major, 16-byte slots swizzled as everywhere), so the contractions see it at ~2^-17
-// relative: the dC side reads its fragments row-wise, the dB side, which needs dG^T, through LDS transpose reads.  B^T / C^T
-// fragments come straight from the operand-order tiles (one contiguous KiB per fragment), the MFMAs are issued with swapped
-// operands, so a lane owns one token: the accumulators start from 16-byte loads of the summed state parts and leave as
-// 16-byte stores after one lane-pair swap per 4-column group.  One barrier, no pass of the results through LDS.
-// With few (batch, chunk, group) triples the launch is latency-bound and more, shorter workgroups win: BOTH = false runs
-// one side per workgroup (`side_b`), wave w and w + 4 taking the two halves of the state columns of row block w & 3, with
-// all B^T / C^T fragments requested before the barrier.
-template <typename T, int N, bool BOTH>
-__device__ __forceinline__ void
-bc_final16_body(const float* __restrict__ dGs, const float* __restrict__ dCs, const float* __restrict__ dBs,
-                const T* __restrict__ Bt, const T* __restrict__ Ct, T* __restrict__ dB, T* __restrict__ dC,
-                int64_t seqlen, int64_t ngroups, int64_t nchunks,
-                int64_t dBsb, int64_t dBsl, int64_t dBsg, int64_t dCsb, int64_t dCsl, int64_t dCsg, int64_t c, int64_t g, int64_t b,
-                const bool wg_side_b) {
+// Group-level finish for 16-bit operands whose heads are cut into slices, from the summed partials:
+//   dC[i][n] = sum_{j<=i} dG[i][j] B[j][n] + dCoff[i][n],      dB[j][n] = sum_{i>=j} dG[i][j] C[i][n] + dBoff[j][n]
+// One workgroup of 8 waves per (batch, chunk, group) and block of 32 tokens, wave w the column block w & 3 of dC (w < 4) or dB.  The
+// token block meets four 32x32 blocks of dG, (rb, 0 .. rb) for dC and (rb .. 3, rb) for dB: they come through LDS, fp32, 16-byte slots
+// swizzled by the row, and a fragment is split into value and remainder in registers, so the contractions see dG at ~2^-17 relative.
+// The accumulators start from the summed state parts (16-byte loads), B^T / C^T fragments are contiguous KiB of the operand-order
+// tiles; everything is asked for in front of the one barrier, and a lane owns one token: 16-byte stores after one lane-pair swap per
+// 4-column group.
+// What bounds it is latency: hence the quarter of a triple per workgroup.  As one workgroup per side, which put all of dG through LDS in
+// two 16-bit tiles, the launch took 8.8 us at 27 triples, 8.6 at 4 and 10.4 at 64 (b4 l2048 h80); 6.7, 6.5 and 9.1 so.
+struct GroupFinishArgs {
+    const float* dG; const float* dCoff; const float* dBoff; const void* Bt; const void* Ct; void* dB; void* dC;
+    int64_t dBsb, dBsl, dBsg, dCsb, dCsl, dCsg, seqlen, ngroups, nchunks, n;      // n: workgroups
+};
+template <typename T, int N>
+__device__ __forceinline__ void group_finish16_body(const GroupFinishArgs& a, int64_t blk) {
     static_assert(sizeof(T) == 2, "16-bit operands only");
-    constexpr int NBN = BOTH ? N / 32 : N / 64, SPR = kQ / 8;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    T* sH = reinterpret_cast<T*>(smem_raw);      // [kQ][kQ] hi part of dG
-    T* sL = sH + kQ * kQ;                        // [kQ][kQ] lo part
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int r = lane & 31, half = lane >> 5;
-    const int64_t t0 = c * kQ;
-    const int valid = (int)((seqlen - t0) < kQ ? (seqlen - t0) : kQ);
-    const int64_t grp = (b * nchunks + c) * ngroups + g;
-    {
-        const float* gp = dGs + grp * (int64_t)(kQ * kQ);
+    __shared__ __align__(16) float sG[4][32 * 32];      // block q: (rb, q) up to the diagonal, (q, rb) behind it
+    const int tid = threadIdx.x, wave = (int)uniform(tid >> 6), lane = tid & 63, r = lane & 31, half = lane >> 5;
+    const int rb = (int)(blk & 3), tok = rb * 32 + r;
+    const int64_t grp = blk >> 2, g = grp % a.ngroups, c = grp / a.ngroups % a.nchunks, b = grp / (a.ngroups * a.nchunks), t0 = c * kQ;
+    const int valid = (int)((a.seqlen - t0) < kQ ? (a.seqlen - t0) : kQ);
+    const bool side_b = wave >= 4;
+    const int nb = wave & 3, row = (tid & 255) >> 3, slot = tid & 7;
+    const bool active = nb < N / 32;                    // with 64 state columns half of the waves only help to fetch dG
+    floatx4 v[2];
 #pragma unroll
-        for (int it = 0; it < kQ * kQ / 4 / 512; ++it) {
-            const int e = it * 512 + tid, i = e / (kQ / 4), j4 = (e % (kQ / 4)) * 4;
-            floatx4 v = floatx4{0.f, 0.f, 0.f, 0.f};
-            if ((j4 >> 5) <= (i >> 5)) v = *reinterpret_cast<const floatx4*>(gp + i * kQ + j4);      // blocks above the diagonal are never written
-            const T h0 = from_f32<T>(v[0]), h1 = from_f32<T>(v[1]), h2 = from_f32<T>(v[2]), h3 = from_f32<T>(v[3]);
-            const uint2 hw = {pack2<T>(to_f32(h0), to_f32(h1)), pack2<T>(to_f32(h2), to_f32(h3))};
-            const uint2 lw = {pack2<T>(v[0] - to_f32(h0), v[1] - to_f32(h1)), pack2<T>(v[2] - to_f32(h2), v[3] - to_f32(h3))};
-            const int at = (i * SPR + ((j4 >> 3) ^ tile_swz<SPR>(i))) * 8 + (j4 & 7);
-            *reinterpret_cast<uint2*>(sH + at) = hw;
-            *reinterpret_cast<uint2*>(sL + at) = lw;
-        }
+    for (int it = 0; it < 2; ++it) {
+        const int q = it * 2 + (wave >> 2), bi = q <= rb ? rb : q, bj = q <= rb ? q : rb;
+        v[it] = *reinterpret_cast<const floatx4*>(a.dG + grp * (int64_t)(kQ * kQ) + (bi * 32 + row) * kQ + bj * 32 + slot * 4);
     }
-    const bool side_b = BOTH ? wave >= 4 : wg_side_b;
-    const int rb = wave & 3, tok = rb * 32 + r;
-    const int n0 = BOTH ? 0 : (wave >> 2) * (N / 2);      // first state column of this wave
-    floatx16 acc[NBN];
-    {
-        const float* op = (side_b ? dBs : dCs) + grp * (int64_t)(kQ * N) + (int64_t)tok * N + n0;
-#pragma unroll
-        for (int nb = 0; nb < NBN; ++nb)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const floatx4 v = *reinterpret_cast<const floatx4*>(op + nb * 32 + 8 * q + 4 * half);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[nb][4 * q + e] = v[e];
-            }
-    }
-    const char* tile = reinterpret_cast<const char*>((side_b ? Ct : Bt) + grp * (int64_t)(N * kQ)) + (n0 / 32) * (8 * 1024);
+    floatx16 acc;
+    Frag<T> xf[8];
     const int ks0 = side_b ? 2 * rb : 0, ks1 = side_b ? 8 : 2 * rb + 2;      // 16-wide k blocks of this wave
-    Frag<T> xpre[BOTH ? 1 : 8][NBN];
-    if constexpr (!BOTH) {
+    if (active) {
+        const float* op = (side_b ? a.dBoff : a.dCoff) + grp * (int64_t)(kQ * N) + (int64_t)tok * N + nb * 32 + 4 * half;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const floatx4 o = *reinterpret_cast<const floatx4*>(op + 8 * q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[4 * q + e] = o[e];
+        }
+        const char* tile = static_cast<const char*>(side_b ? a.Ct : a.Bt) + grp * (int64_t)(N * kQ * 2) + nb * 8 * 1024;      // see mt_offset
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks)
-            if (ks >= ks0 && ks < ks1) {
-#pragma unroll
-                for (int nb = 0; nb < NBN; ++nb)
-                    xpre[ks][nb].v = *reinterpret_cast<const bf16x8*>(tile + ((uint32_t)lane * 16u + (uint32_t)((nb * 8 + ks) * 1024)));
-            }
+            if (ks >= ks0 && ks < ks1) xf[ks].v = *reinterpret_cast<const bf16x8*>(tile + ((uint32_t)lane * 16u + (uint32_t)(ks * 1024)));
     }
+#pragma unroll
+    for (int it = 0; it < 2; ++it) *reinterpret_cast<floatx4*>(&sG[it * 2 + (wave >> 2)][row * 32 + ((slot ^ (row & 7)) * 4)]) = v[it];
     __syncthreads();
-    const int tr_tok = 8 * half + ((lane >> 2) & 3), tr_col = rb * 32 + ((lane >> 4) & 1) * 16 + 4 * (lane & 3);
-    typedef T tvec4 __attribute__((ext_vector_type(4)));
+    if (!active) return;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
         if (ks < ks0 || ks >= ks1) continue;      // wave-uniform
-        Frag<T> yh, yl;
-        if (!side_b) {
-            const int at = (tok * SPR + ((ks * 2 + half) ^ tile_swz<SPR>(tok))) * 8;
-            yh = load_frag(sH + at);
-            yl = load_frag(sL + at);
+        const float* blk_g = sG[ks >> 1];
+        const int k0 = (ks & 1) * 16 + 8 * half;
+        float f[8];
+        if (side_b) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] = blk_g[(k0 + e) * 32 + (((r >> 2) ^ e) * 4) + (r & 3)];
         } else {
-            const int ta = ks * 16 + tr_tok, tb = ta + 4;
-            const int aa = (ta * SPR + ((tr_col >> 3) ^ tile_swz<SPR>(ta))) * 8 + (tr_col & 7);
-            const int ab = (tb * SPR + ((tr_col >> 3) ^ tile_swz<SPR>(tb))) * 8 + (tr_col & 7);
-            const tvec4 h0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((M2_LDS tvec4*)(sH + aa));
-            const tvec4 h1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((M2_LDS tvec4*)(sH + ab));
-            const tvec4 l0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((M2_LDS tvec4*)(sL + aa));
-            const tvec4 l1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((M2_LDS tvec4*)(sL + ab));
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { yh.v[e] = h0[e]; yh.v[4 + e] = h1[e]; yl.v[e] = l0[e]; yl.v[4 + e] = l1[e]; }
-        }
+            for (int q = 0; q < 2; ++q) {
+                const floatx4 o = *reinterpret_cast<const floatx4*>(blk_g + r * 32 + (((k0 >> 2) + q) ^ (r & 7)) * 4);
 #pragma unroll
-        for (int nb = 0; nb < NBN; ++nb) {
-            Frag<T> xf;      // see mt_offset
-            if constexpr (BOTH) xf.v = *reinterpret_cast<const bf16x8*>(tile + ((uint32_t)lane * 16u + (uint32_t)((nb * 8 + ks) * 1024)));
-            else xf = xpre[ks][nb];
-            mma_frag(acc[nb], xf, yh);
-            mma_frag(acc[nb], xf, yl);
+                for (int e = 0; e < 4; ++e) f[4 * q + e] = o[e];
+            }
         }
+        Frag<T> yh, yl;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            yh.v[e] = from_f32<T>(f[e]);
+            yl.v[e] = from_f32<T>(f[e] - to_f32((T)yh.v[e]));
+        }
+        mma_frag(acc, xf[ks], yh);
+        mma_frag(acc, xf[ks], yl);
     }
-    T* out = (side_b ? dB + b * dBsb + t0 * dBsl + g * dBsg : dC + b * dCsb + t0 * dCsl + g * dCsg) + (int64_t)tok * (side_b ? dBsl : dCsl) + n0;
+    T* out = side_b ? static_cast<T*>(a.dB) + b * a.dBsb + (t0 + tok) * a.dBsl + g * a.dBsg : static_cast<T*>(a.dC) + b * a.dCsb + (t0 + tok) * a.dCsl + g * a.dCsg;
 #pragma unroll
-    for (int nb = 0; nb < NBN; ++nb)
+    for (int qp = 0; qp < 2; ++qp) {
+        float g8[8];
 #pragma unroll
-        for (int qp = 0; qp < 2; ++qp) {
-            float g8[8];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) pair_swap(acc[nb][8 * qp + e], acc[nb][8 * qp + 4 + e], g8[e], g8[4 + e]);
-            const uint4 o = {pack2<T>(g8[0], g8[1]), pack2<T>(g8[2], g8[3]), pack2<T>(g8[4], g8[5]), pack2<T>(g8[6], g8[7])};
-            if (tok < valid) *reinterpret_cast<uint4*>(out + nb * 32 + 8 * (2 * qp + half)) = o;
-        }
+        for (int e = 0; e < 4; ++e) pair_swap(acc[8 * qp + e], acc[8 * qp + 4 + e], g8[e], g8[4 + e]);
+        const uint4 o = {pack2<T>(g8[0], g8[1]), pack2<T>(g8[2], g8[3]), pack2<T>(g8[4], g8[5]), pack2<T>(g8[6], g8[7])};
+        if (tok < valid) *reinterpret_cast<uint4*>(out + nb * 32 + 8 * (2 * qp + half)) = o;
+    }
 }
 
 // dA[h] = sum_{b,c} dAp[b][h][c], dD likewise (fixed order, no atomics).  One workgroup of 512 threads per head.
@@ -212,33 +185,22 @@ __device__ __forceinline__ void ad_reduce_body(const float* __restrict__ dAp, co
     }
 }
 
-// The group-level finish and the per-head reductions in one launch: the first workgroups run the group finish for
-// ([side,] chunk, group, batch) = the index split in that order (16-bit operands without BOTH: side 0 dC, side 1 dB, one workgroup
-// each), the others ad_reduce_body for one head each.
-constexpr int64_t kTail2BothFrom = 256;      // (batch, chunk, group) triples from which a workgroup takes both sides: one per CU
+// The group-level finish, where the main kernel has not done it, and behind its workgroups the per-head reductions, one workgroup each,
+// in one launch.
 struct Tail2Args {
-    const float* dGp; const float* dCp; const float* dBp; const void* Bt; const void* Ct; void* dB; void* dC;
-    int64_t dBsb, dBsl, dBsg, dCsb, dCsl, dCsg;
     const float* dAp; const float* dDp; const float* dbp; float* dA; float* dD; float* dbias;
-    int64_t seqlen, ngroups, nchunks, batch, nheads, n_bc;
+    int64_t seqlen, ngroups, nchunks, batch, nheads;
 };
-struct Tail2Args32 : Tail2Args {      // Bt, Ct: B and C as they lie
-    int64_t Bsb, Bsl, Bsg, Csb, Csl, Csg;
+struct Tail2Args32 : Tail2Args {
+    const float* dGp; const float* dCp; const float* dBp; const void* B; const void* C; void* dB; void* dC;
+    int64_t dBsb, dBsl, dBsg, dCsb, dCsl, dCsg, Bsb, Bsl, Bsg, Csb, Csl, Csg, n_bc;
 };
-template <typename T, int N, bool BOTH>
+template <typename T, int N>
 __global__ void __launch_bounds__(512)
-tail2_kernel(const Tail2Args a) {
+tail2_kernel(const Tail2Args a, const GroupFinishArgs f) {
     const int64_t blk = blockIdx.x;
-    constexpr int SIDES = BOTH ? 1 : 2;
-    if (blk < SIDES * a.n_bc) {
-        const int64_t q = blk / SIDES;
-        const int64_t c = q % a.nchunks, g = (q / a.nchunks) % a.ngroups, b = q / (a.nchunks * a.ngroups);
-        bc_final16_body<T, N, BOTH>(a.dGp, a.dCp, a.dBp, static_cast<const T*>(a.Bt), static_cast<const T*>(a.Ct), static_cast<T*>(a.dB),
-                                    static_cast<T*>(a.dC), a.seqlen, a.ngroups, a.nchunks, a.dBsb, a.dBsl, a.dBsg, a.dCsb, a.dCsl, a.dCsg, c, g,
-                                    b, (blk & 1) != 0);
-    } else {
-        ad_reduce_body(a.dAp, a.dDp, a.dbp, a.dA, a.dD, a.dbias, a.batch, a.nheads, a.nchunks, blk - SIDES * a.n_bc);
-    }
+    if (blk < f.n) group_finish16_body<T, N>(f, blk);
+    else ad_reduce_body(a.dAp, a.dDp, a.dbp, a.dA, a.dD, a.dbias, a.batch, a.nheads, a.nchunks, blk - f.n);
 }
 template <int N>
 __global__ void __launch_bounds__(512)
@@ -246,7 +208,7 @@ tail2_32_kernel(const Tail2Args32 a) {
     const int64_t blk = blockIdx.x;
     if (blk < a.n_bc) {
         const int64_t c = blk % a.nchunks, g = (blk / a.nchunks) % a.ngroups, b = blk / (a.nchunks * a.ngroups);
-        bc_final32_body<N>(a.dGp, a.dCp, a.dBp, static_cast<const float*>(a.Bt), a.Bsb, a.Bsl, a.Bsg, static_cast<const float*>(a.Ct), a.Csb, a.Csl, a.Csg,
+        bc_final32_body<N>(a.dGp, a.dCp, a.dBp, static_cast<const float*>(a.B), a.Bsb, a.Bsl, a.Bsg, static_cast<const float*>(a.C), a.Csb, a.Csl, a.Csg,
                            static_cast<float*>(a.dB), a.dBsb, a.dBsl, a.dBsg, static_cast<float*>(a.dC), a.dCsb, a.dCsl, a.dCsg, a.seqlen, a.ngroups,
                            a.nchunks, c, g, b);
     } else {
@@ -262,9 +224,6 @@ __global__ void copy_f32_kernel(const float* __restrict__ src, float* __restrict
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = src ? src[i] : 0.f;
 }
-
-template <typename T, int N>
-size_t bcf_smem() { return sizeof(T) == 2 ? (size_t)2 * kQ * kQ * sizeof(T) : finish32_smem<N>(); }
 
 template <typename T, int P, int N, int HS>
 int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
@@ -371,28 +330,27 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
             tail1_kernel<T><<<(unsigned)(n_da + n_ss), kDaHeads * 64, 0, st>>>(da, n_da, sa);
         }
         if ((rc = check_launch("ssd tail1_kernel"))) return rc;
-        // none where the main kernel has finished dB and dC; else, with 16-bit operands, one workgroup per (batch, chunk, group) once
-        // those alone fill the chip, one per side below that
-        const bool both = sizeof(T) == 4 || ngrp >= kTail2BothFrom;
-        Tail2Args32 ta;
-        ta.dGp = gs; ta.dCp = cs; ta.dBp = bs; ta.Bt = sizeof(T) == 2 ? w.Bt : p->B; ta.Ct = sizeof(T) == 2 ? w.Ct : p->C; ta.dB = p->dB; ta.dC = p->dC;
-        ta.Bsb = p->B_stride_b; ta.Bsl = p->B_stride_l; ta.Bsg = p->B_stride_g; ta.Csb = p->C_stride_b; ta.Csl = p->C_stride_l; ta.Csg = p->C_stride_g;
-        ta.dBsb = p->dB_stride_b; ta.dBsl = p->dB_stride_l; ta.dBsg = p->dB_stride_g;
-        ta.dCsb = p->dC_stride_b; ta.dCsl = p->dC_stride_l; ta.dCsg = p->dC_stride_g;
+        const int64_t n_bc = w.finished ? 0 : ngrp;
+        Tail2Args32 ta{};
         ta.dAp = w.dAp; ta.dDp = w.dDp; ta.dbp = w.dbp; ta.dA = p->dA; ta.dD = p->D ? p->dD : nullptr;
         ta.dbias = p->dt_bias ? p->d_dt_bias : nullptr;
         ta.seqlen = p->seqlen; ta.ngroups = p->ngroups; ta.nchunks = nc; ta.batch = p->batch; ta.nheads = p->true_heads;
-        ta.n_bc = w.finished ? 0 : ngrp;
-        const unsigned grid = (unsigned)((both ? 1 : 2) * ta.n_bc + p->true_heads);
-        const size_t sm = w.finished ? 0 : bcf_smem<T, N>();
         if constexpr (sizeof(T) == 2) {
-            auto k = both ? tail2_kernel<T, N, true> : tail2_kernel<T, N, false>;
-            if ((rc = allow_smem(k, sm))) return rc;
-            k<<<grid, 512, sm, st>>>(ta);
+            GroupFinishArgs f{};
+            f.dG = gs; f.dCoff = cs; f.dBoff = bs; f.Bt = w.Bt; f.Ct = w.Ct; f.dB = p->dB; f.dC = p->dC;
+            f.dBsb = p->dB_stride_b; f.dBsl = p->dB_stride_l; f.dBsg = p->dB_stride_g;
+            f.dCsb = p->dC_stride_b; f.dCsl = p->dC_stride_l; f.dCsg = p->dC_stride_g;
+            f.seqlen = p->seqlen; f.ngroups = p->ngroups; f.nchunks = nc; f.n = 4 * n_bc;
+            tail2_kernel<T, N><<<(unsigned)(f.n + p->true_heads), 512, 0, st>>>(ta, f);
         } else {
+            ta.dGp = gs; ta.dCp = cs; ta.dBp = bs; ta.B = p->B; ta.C = p->C; ta.dB = p->dB; ta.dC = p->dC;
+            ta.Bsb = p->B_stride_b; ta.Bsl = p->B_stride_l; ta.Bsg = p->B_stride_g; ta.Csb = p->C_stride_b; ta.Csl = p->C_stride_l; ta.Csg = p->C_stride_g;
+            ta.dBsb = p->dB_stride_b; ta.dBsl = p->dB_stride_l; ta.dBsg = p->dB_stride_g;
+            ta.dCsb = p->dC_stride_b; ta.dCsl = p->dC_stride_l; ta.dCsg = p->dC_stride_g;
+            ta.n_bc = n_bc;
             auto k = tail2_32_kernel<N>;
-            if ((rc = allow_smem(k, sm))) return rc;
-            k<<<grid, 512, sm, st>>>(ta);
+            if ((rc = allow_smem(k, finish32_smem<N>()))) return rc;
+            k<<<(unsigned)(n_bc + p->true_heads), 512, n_bc ? finish32_smem<N>() : 0, st>>>(ta);
         }
         if ((rc = check_launch("ssd tail2_kernel"))) return rc;
     }

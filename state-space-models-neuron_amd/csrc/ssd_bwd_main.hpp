@@ -59,7 +59,7 @@ struct Bwd16Args {
 
 // FINISH: the workgroup has all heads of its group (nslices == 1) and dG is complete (dg16_kernel's slices too are one), so that role
 // B's accumulators are the whole state parts: it adds dG B and dG^T C to them and writes dB and dC, instead of leaving 128 KiB of
-// fp32 to be read again by bc_final16_body, with the same products in the same order.  dG (fp32, the ten 32x32 blocks of its lower
+// fp32 to be read again by group_finish16_body, with the same products in the same order.  dG (fp32, the ten 32x32 blocks of its lower
 // triangle) is copied into the free tile buffer while the last head is worked on, B^T and C^T into the other one behind it.
 // b2 l4096 h128 g8: this kernel 194 -> 201 us and the finish 39 -> 5 (its sums of dA and dD); b8 l2048 h8 g8 79 -> 89 and 78 -> 5.
 // With the operand fragments read from memory by each wave instead of through LDS: 207.

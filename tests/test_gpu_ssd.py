@@ -318,6 +318,12 @@ def test_ssd_bf16_whole_groups(b, l, h, p, n, g):
             assert rel_rms_err(v[:, t:t + 128], r[name][:, t:t + 128]) < 2e-2, (name, t)
 
 
+# the group finish from slices' partials: 64 and 128 state columns, one token in a token block, a wide head, several groups
+@pytest.mark.parametrize("b,l,h,p,n,g", [(1, 97, 8, 64, 64, 1), (2, 225, 12, 64, 128, 2), (1, 300, 4, 128, 128, 1), (40, 129, 16, 64, 64, 4)])
+def test_ssd_bf16_cut_groups(b, l, h, p, n, g):
+    test_ssd_bf16_whole_groups(b, l, h, p, n, g)
+
+
 @pytest.mark.parametrize("steps", ["usual", "long"])
 @pytest.mark.parametrize("b,l,h,p,n,g", [
     (16, 129, 16, 64, 128, 4),     # four heads one after the other in a workgroup, which finishes dB and dC itself; one token in the last chunk
