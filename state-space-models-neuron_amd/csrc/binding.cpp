@@ -533,6 +533,9 @@ struct Packed {
         TORCH_CHECK_VALUE(t.size(2) == d + conv + h, "zxBCdt width ", t.size(2), " != 2*d_inner + 2*g*n + h = ", d + conv + h);
         const bool even = t.stride(2) == 1 && (t.size(0) <= 1 || t.stride(0) == t.size(1) * t.stride(1));
         zx = even ? t : t.contiguous();
+        // One token per sequence: contiguous() looks at no stride of a dimension of size one and returns a transposed time-first buffer,
+        // say, as it is.  Its rows are a width apart, and so is "the next token" to whoever takes the token stride for that of the rows.
+        if (!even && t.size(1) == 1) zx = zx.as_strided(zx.sizes(), {zx.size(2), zx.size(2), 1});
         b = zx.size(0); l = zx.size(1); sb = zx.stride(0); sl = zx.stride(1);
     }
     Tensor z() const { return zx.narrow(2, 0, d); }

@@ -357,3 +357,47 @@ def test_layer_takes_parameters_that_are_strided_views(b, dtype):
     assert not mixer.D.is_contiguous() and not mixer.in_proj.weight.is_contiguous()
     for g, w in zip(passes(), want):
         assert _rel(g, w) < 2e-2
+
+
+def _one_token(x, layout):
+    """x (b, 1, width), its values in another layout; every row lies inside the tensor's own memory."""
+    b, _, width = x.shape
+    if layout == "time first":
+        form = torch.empty(1, b, width, dtype=x.dtype, device=DEV).copy_(x.transpose(0, 1)).transpose(0, 1)
+        assert form.is_contiguous() and form.stride() == (width, b * width, 1)
+    elif layout == "last of five":
+        form = x.repeat(1, 5, 1)[:, -1:]
+    else:
+        form = torch.cat([x, x], 2)[..., :width]
+    return form
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("b,h", [(1, 8), (2, 8), (5, 8), (3, 5)])      # rows on 16 bytes and (5 heads) rows that are not
+@pytest.mark.parametrize("layout", ["time first", "last of five", "padded"])
+def test_core_on_one_token_of_any_layout(layout, b, h, dtype):
+    """The stride of the token dimension says nothing where that has one entry: forward, backward and prefill, bit for bit as on
+    contiguous rows."""
+    from mamba2.fused_kernel import mamba2_fused_kernel, mamba2_fused_kernel_with_caching, mamba2_fused_prefill
+    p, n, g = 64, 64, 1
+    d, c = h * p, h * p + 2 * g * n
+    gen = torch.Generator(device=DEV).manual_seed(7)
+    rand = lambda *s: torch.randn(*s, device=DEV, generator=gen)
+    x, dy = rand(b, 1, d + c + h).to(dtype), rand(b, 1, d).to(dtype)
+    params = [-rand(h).abs(), rand(h), rand(c, 1, 4).to(dtype), rand(c).to(dtype), rand(h), rand(d)]
+    states = rand(b, c, 4).to(dtype), rand(b, h, p, n)
+
+    def passes(form):
+        out = []
+        for core in (mamba2_fused_kernel, mamba2_fused_kernel_with_caching):
+            leaves = [t.detach().requires_grad_(True) for t in (form, *params)]
+            y = core(*leaves, g, n, d, p)
+            out += [y.detach(), *torch.autograd.grad(y, leaves, dy)]
+        for continuing in (False, True):
+            moved = [t.clone() for t in states]
+            with torch.no_grad():
+                out += [mamba2_fused_prefill(form, *params, g, n, d, p, *moved, continuing=continuing), *moved]
+        return out
+
+    for got, want in zip(passes(_one_token(x, layout)), passes(x)):
+        assert torch.equal(got, want)
