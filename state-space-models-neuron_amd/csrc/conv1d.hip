@@ -53,19 +53,31 @@ static_assert(kUNR >= 3, "the dx lag fits one load group");
 
 // Tokens per thread.  A thread is a chain of load groups, so where the threads do not fill the chip short segments win, and their
 // halo (three tokens more read; six in the backward, and three more activations) and, in the backward, their partial rows only count
-// once it is full.  Kernel times in us (backward with its sum) at 4 | 8 | 16 and 8 | 16 | 32 tokens, bf16:
-//   b1 l200 C5376    3.1 |  3.2 |  4.5      9.4 |   8.6 |  11.2        b1 l2048 C10240  19.2 | 17.1 | 17.4     36.7 |  33.8 |  37.2
-//   b1 l500 C1792    3.1 |  3.4 |  4.5      7.4 |   8.4 |  11.8        b4 l2048 C5376   37.6 | 30.4 | 31.6     71.2 |  59.9 |  60.2
-//   b3 l1111 C2304   9.2 |  8.3 |  8.1     20.1 |  17.3 |  18.3        b2 l4096 C10240  69.3 | 56.4 | 58.8    136.9 | 115.9 | 114.0
-//   b8 l333 C5376   14.2 | 12.8 | 13.2     28.4 |  26.7 |  24.7        b1 l16384 C5376  70.4 | 56.1 | 58.9    143.4 | 119.7 | 119.0
+// once it is full.  The lines below come from 389 timings (256 to 10240 channels, 24 to 18746 tokens, batches of 1 to 16, both types,
+// with the tensors in the caches and not); per band the geometric mean of the time over that of the best of the three forms, threads
+// counted at 16 tokens forward and at 32 backward:
+//   forward           4 |    8 |   16          backward (with its sum)             8 |   16 |   32
+//   to 24K         1.00 | 1.09 | 1.37          to 16K                           1.01 | 1.12 | 1.49
+//   24K to 48K     1.02 | 1.02 | 1.11          16K to 64K                       1.06 | 1.04 | 1.27
+//   48K to 96K     1.03 | 1.01 | 1.09          64K to 128K                      1.10 | 1.03 | 1.04
+//   96K to 192K    1.08 | 1.01 | 1.03          128K to 1M, to 2560 channels     1.15 | 1.05 | 1.01
+//   above          1.15 | 1.00 | 1.05          128K to 1M, more channels        1.09 | 1.01 | 1.05
+//                                              above                            1.21 | 1.03 | 1.00
+//                                              192 partial rows and more        1.32 | 1.07 | 1.00
+// Few channels and many partial rows want long segments for the sum's sake: it has a workgroup per 13 channels, and each of its
+// threads walks a quarter of the rows.  In us, sizes beside the lines: b3 l1111 C2304 forward 10.1 | 8.7 | 8.8, backward 21.9 | 20.4 |
+// 20.0; b6 l808 C2304 12.0 | 11.8 | 11.5 and 28.0 | 25.9 | 24.0; b12 l669 C4352 30.1 | 25.4 | 27.4 and 60.0 | 54.0 | 57.6; b4 l18746
+// C256 18.0 | 16.4 | 17.4 and 83.0 | 57.3 | 49.5; b2 l4096 C10240 68.7 | 57.3 | 59.8 and 135.4 | 115.6 | 112.9.  A size on the wrong
+// side of a line: b8 l333 C5376, backward 29.6 | 28.7 | 26.6.
 constexpr int64_t kMaxSegs = (int64_t)65535 * kSEG;      // what the grid holds: the longest sequences keep the longest segments
 int64_t conv_fwd_tokens(int64_t batch, int64_t seqlen, int64_t vectors) {
     const int64_t threads = batch * ceil_div(seqlen, (int64_t)16) * vectors;
-    return threads <= 48 * 1024 ? 4 : (threads <= 192 * 1024 || ceil_div(seqlen, (int64_t)8) > kMaxSegs ? 16 : 8);
+    return ceil_div(seqlen, (int64_t)8) > kMaxSegs ? 16 : (threads <= 48 * 1024 ? 4 : 8);
 }
 int64_t conv_bwd_tokens(int64_t batch, int64_t seqlen, int64_t channels) {
-    const int64_t threads = batch * ceil_div(seqlen, (int64_t)32) * ceil_div(channels, (int64_t)2);
-    const int64_t tl = threads <= 16 * 1024 ? 8 : (threads <= 1024 * 1024 ? 16 : 32);
+    const int64_t threads = batch * ceil_div(seqlen, (int64_t)32) * ceil_div(channels, (int64_t)2), rows16 = batch * ceil_div(seqlen, (int64_t)(16 * kSEG));
+    const bool long_ones = rows16 > 192 || threads > (channels <= 2560 ? 128 * 1024 : 1024 * 1024);
+    const int64_t tl = threads <= 16 * 1024 ? 8 : (long_ones ? 32 : 16);
     return ceil_div(seqlen, tl) > kMaxSegs ? 32 : tl;
 }
 // f<tokens per thread>

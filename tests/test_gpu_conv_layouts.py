@@ -87,9 +87,11 @@ def test_prefill_leaves_the_last_inputs(C, W, l, dtype, continuing):
     assert torch.equal(y, ref)      # the same sums in the same order
 
 
-@pytest.mark.parametrize("b,l,C", [(1, 3, 64), (1, 9, 130), (1, 800, 1024), (1, 3000, 1024), (2, 4090, 1024), (1, 2060, 4100), (3, 4100, 6000)])
+@pytest.mark.parametrize("b,l,C", [(1, 3, 64), (1, 9, 130), (1, 800, 1024), (1, 3000, 1024), (2, 4090, 1024), (1, 2060, 4100), (3, 4100, 6000),
+                                   (2, 4130, 1024), (1, 12299, 128), (1, 2097125, 4)])
 def test_conv_segment_lengths(b, l, C):
-    """Sizes on both sides of the rules for the tokens per thread (4, 16, 8 forward; 8, 16, 32 backward), ends inside a segment."""
+    """Sizes on both sides of the rules for the tokens per thread (4, 8, and 16 where the grid needs it, forward; 8, 16, 32 backward,
+    the last one also for few channels and for many partial rows), ends inside a segment."""
     from mamba2.conv1d_grouped import conv1d_backward, conv1d_forward
     torch.manual_seed(l)
     x, dy = (torch.randn(b, l, C, device=DEV).bfloat16() for _ in range(2))
