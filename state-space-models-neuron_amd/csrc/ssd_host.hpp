@@ -29,8 +29,8 @@ struct SsdWorkspace {
     void* dprev = nullptr; float* dlam = nullptr;
     float* dbp = nullptr;                                               // per (b, h, chunk) partials of d_dt_bias
     float* dAp = nullptr; float* dDp = nullptr; float* dBp = nullptr; float* dCp = nullptr; float* dl = nullptr; float* dlc = nullptr; float* dGp = nullptr;
-    float* dGs = nullptr; float* dBs = nullptr; float* dCs = nullptr;   // partials summed over the head slices
-    float* dirp = nullptr; float* rbp = nullptr; float* dDp8 = nullptr; // per channel-half / per-wave partials of the dx kernel
+    float* dGs = nullptr; float* dBs = nullptr; float* dCs = nullptr;   // partials summed over the head slices, where there are several
+    float* dirp = nullptr; float* rbp = nullptr; float* dDp8 = nullptr; // per token, per wave: what the main kernel leaves for ddt and dD
     int64_t ns_g = 1, hps_g = 1, ns_b = 1, hps_b = 1;   // head slicing of dg16 and of the main backward kernel
     bool finished = false;              // the main kernel's workgroups have whole groups and leave dB and dC: no partials of those
     size_t bytes = 0;
@@ -117,23 +117,26 @@ inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_
         ssd_slicing(p, kWgsDx, true, &w.ns_b, &w.hps_b);
         if (p->dtype == M2_F32) { ssd_slicing32(p, &w.ns_b, &w.hps_b); w.ns_g = w.ns_b; w.hps_g = w.hps_b; }      // one kernel for all three
         w.dprev = take(tiles * esz);
+        // Only what a kernel writes: the 16-bit main kernel reads a single slice's dG where dg16_kernel left it, the fp32 one keeps it on
+        // chip, and of one slice there is no sum (the 7B core, b2 l4096 h128 g8, had 100 MB for sums that nobody forms).
+        const size_t groups = (size_t)p->batch * nc * p->ngroups, g_tile = groups * kQ * kQ * 4, n_tile = groups * kQ * p->dstate * 4;
+        w.finished = w.ns_b == 1 && w.ns_g == 1;
+        auto part = [&](bool need, size_t n) { return need ? reinterpret_cast<float*>(take(n)) : nullptr; };
+        w.dGp = part(!w.finished || p->dtype != M2_F32, g_tile * w.ns_g);
+        w.dBp = part(!w.finished, n_tile * w.ns_b);
+        w.dCp = part(!w.finished, n_tile * w.ns_b);
+        w.dGs = part(w.ns_g > 1, g_tile);
+        w.dBs = part(w.ns_b > 1, n_tile);
+        w.dCs = part(w.ns_b > 1, n_tile);
         w.dlam = reinterpret_cast<float*>(take(bhc * 4 * kDlamParts));
         w.dAp = reinterpret_cast<float*>(take(bhc * 4));
         w.dDp = reinterpret_cast<float*>(take(bhc * 4));
         w.dbp = reinterpret_cast<float*>(take(bhc * 4));
         w.dl = reinterpret_cast<float*>(take(bhc * kQ * 4));
         w.dlc = reinterpret_cast<float*>(take(bhc * kQ * 4));
-        w.dirp = reinterpret_cast<float*>(take(bhc * 2 * kQ * 4));
-        w.rbp = reinterpret_cast<float*>(take(bhc * 2 * kQ * 4));
+        w.dirp = reinterpret_cast<float*>(take(bhc * kQ * 4));
+        w.rbp = reinterpret_cast<float*>(take(bhc * kQ * 4));
         w.dDp8 = reinterpret_cast<float*>(take(bhc * 8 * 4));
-        w.dGp = reinterpret_cast<float*>(take((size_t)p->batch * nc * p->ngroups * w.ns_g * kQ * kQ * 4));
-        const size_t part = (size_t)p->batch * nc * p->ngroups * kQ * p->dstate * 4;
-        w.finished = w.ns_b == 1 && w.ns_g == 1;
-        w.dBp = reinterpret_cast<float*>(take(w.finished ? 0 : part * w.ns_b));
-        w.dCp = reinterpret_cast<float*>(take(w.finished ? 0 : part * w.ns_b));
-        w.dGs = reinterpret_cast<float*>(take((size_t)p->batch * nc * p->ngroups * kQ * kQ * 4));
-        w.dBs = reinterpret_cast<float*>(take((size_t)p->batch * nc * p->ngroups * kQ * p->dstate * 4));
-        w.dCs = reinterpret_cast<float*>(take((size_t)p->batch * nc * p->ngroups * kQ * p->dstate * 4));
     }
     w.bytes = off + 256;
     return w;

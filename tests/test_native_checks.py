@@ -69,3 +69,20 @@ def test_every_struct_of_the_header_is_mirrored_and_reported(lib):
         assert lib.m2_struct_layout(which, buf, 128) == 1 + len(fields), name
         assert buf[0] == ctypes.sizeof(mirror) and list(buf[1:1 + len(fields)]) == [getattr(mirror, f).offset for f in fields], name
     assert lib.m2_struct_layout(len(declared), (ctypes.c_int64 * 4)(), 4) == -1
+
+
+@pytest.mark.parametrize("dtype,b,l,h,p,n,g,slices", [(1, 2, 4096, 128, 64, 128, 8, (1, 1)), (0, 3, 2048, 16, 128, 128, 8, (1, 1)), (1, 1, 17, 1, 64, 64, 1, (1, 1)),
+                                                      (1, 4, 2048, 80, 64, 128, 1, (4, 4)), (0, 1, 256, 8, 64, 64, 1, (8, 8))])
+def test_scan_backward_asks_for_what_its_kernels_write(lib, dtype, b, l, h, p, n, g, slices):
+    """Workspace beside the buffer that the forward left, counted from the kernels: state gradients, per-token and per-chunk rows, and
+    of dG, dB and dC a partial per slice and a sum only where there are several slices."""
+    from mamba2 import _lib
+    q = 128
+    params = _lib.SsdParams(batch=b, seqlen=l, nheads=h, headdim=p, dstate=n, ngroups=g, dtype=dtype, dt_dtype=dtype, chunk_states=256)
+    chunks, size, (s_g, s_b) = -(-l // q), 2 if dtype else 4, slices
+    bhc, groups = b * (h * p // 64) * chunks, b * chunks * g
+    want = bhc * 64 * n * size + bhc * 4 * (8 + 3 + 4 * q + 8) + (0 if dtype else bhc * 64 * n * 4)
+    done = s_g == s_b == 1
+    want += groups * q * q * 4 * ((0 if done and not dtype else s_g) + (s_g > 1)) + 2 * groups * q * n * 4 * ((0 if done else s_b) + (s_b > 1))
+    got = lib.m2_ssd_bwd_workspace_bytes(ctypes.byref(params))
+    assert want <= got <= want + 20 * 256, (got, want)
