@@ -198,3 +198,25 @@ def test_param_sums(norm_rows, channels, norm_dtype, slots, conv_channels, conv_
         close(o_db, db.double(), 1)
     else:
         assert (o_A == 7).all()
+
+
+@pytest.mark.parametrize("heads,channels,with_D,types", [(24, 1536, True, (torch.bfloat16,) * 4), (5, 33, False, (torch.float32, torch.bfloat16, torch.bfloat16, torch.float32))])
+def test_mixer_params_and_their_gradients(heads, channels, with_D, types):
+    """The small parameters into fp32 and their gradients back into the parameters' types: products and casts, one rounding each."""
+    from mamba2 import _lib
+    lib, code, ptr = _lib.load(), _lib.dtype_code, _lib.ptr
+    torch.manual_seed(heads)
+    A_log, D, dt_bias, norm = (torch.randn(n, device=DEV).to(t) for n, t in zip((heads, heads, heads, channels), types))
+    out = torch.full((3 * heads + channels,), 7.0, device=DEV)
+    _lib.check(lib.m2_mixer_params(ptr(A_log), code(types[0]), ptr(D) if with_D else None, code(types[1]), ptr(dt_bias), code(types[2]), ptr(norm),
+                                   code(types[3]), ptr(out), heads, channels, _lib.stream_ptr()), "mixer_params")
+    A, D32, bias32, norm32 = out.split((heads, heads, heads, channels))
+    assert ((A.double() + A_log.double().exp()).abs() <= 2.0 ** -21 * A.double().abs()).all()      # expf: a few ulp
+    assert torch.equal(bias32, dt_bias.float()) and torch.equal(norm32, norm.float())
+    assert torch.equal(D32, D.float()) if with_D else (D32 == 7).all()
+    dA, dD, db, dn = (torch.randn(n, device=DEV) for n in (heads, heads, heads, channels))
+    got = [torch.full((n,), 7.0, device=DEV, dtype=t) for n, t in zip((heads, heads, heads, channels), types)]
+    _lib.check(lib.m2_mixer_params_grads(ptr(A), ptr(dA), ptr(dD) if with_D else None, ptr(db), ptr(dn), ptr(got[0]), code(types[0]), ptr(got[1]) if with_D else None,
+                                         code(types[1]), ptr(got[2]), code(types[2]), ptr(got[3]), code(types[3]), heads, channels, _lib.stream_ptr()), "mixer_params_grads")
+    for name, a, want in zip(("A_log", "D", "dt_bias", "norm"), got, (A * dA, dD, db, dn)):
+        assert torch.equal(a, want.to(a.dtype)) if name != "D" or with_D else (a == 7).all(), name
