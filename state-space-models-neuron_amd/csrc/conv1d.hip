@@ -492,8 +492,8 @@ conv_fwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
 // One wave per (channel, split): its lanes walk the channel's pieces of two vectors of tokens over all rows of the batch,
 // so the sums of dw and db stay in registers until the end.  The 1, 2 or 4 (`inner`) splits of a channel inside a workgroup meet in
 // LDS and finish it there; only with more of them (few channels) do fp32 partials go to conv_reduce_partials_kernel, whose launch
-// took 4.3 us beside the 70 of this kernel at b4 l2048 C5376 (two splits; forward and backward 125.7 -> 123.5 us in a stream of them; with
-// one split the chip is short of waves, 131 -> 141 in an eager loop).
+// took 4.3 us beside the 70 of this kernel at b4 l2048 C5376 (two splits; forward and backward 125.0-126.1 -> 122.9-124.1 us in a stream of
+// them over eight sessions; with one split the chip is short of waves, 131 -> 141 in an eager loop).
 // A lane recomputes the three tokens behind its own for the dx lag: 3 in 16
 // (bf16) more activations, against a cross-lane exchange that would break at every row end.
 template <typename T, typename WT, int ACT>
