@@ -122,6 +122,10 @@ state_pass16_kernel(const StatePassArgs a) {
     // priority below out of a 64-bit quotient) they were 150 of the 200 scalar instructions of an iteration, which on a chip
     // holding few workgroups stand between one chunk's products and the next: 181 -> 169 us at b1 l16384 h80.
     const int nci = (int)nc, cfirst = REVERSE ? nci - 1 : 0;
+    // Steps of the recurrence: what the last chunk adds reaches only the state behind it, so without a reader of that the last
+    // chunk's state is stored and nothing of it is loaded or multiplied (forward and backward at b4 l2048 h80 335.5 -> 332.5 us; fp32
+    // operands, whose chunks are workgroups of part-filled rounds, gained nothing by the same).
+    const int nsteps = HILO || a.final_out ? nci : nci - 1;      // (two-tile operands are for a final state)
     const int tail_rows = (int)(a.seqlen - (nc - 1) * kQ);      // valid rows of the last chunk
     constexpr int DIR = REVERSE ? -1 : 1;
     const char* xq = reinterpret_cast<const char*>(static_cast<const T*>(a.X) + b * a.X_sb + (int64_t)cfirst * kQ * a.X_sl + head_off<HS>(h, a.X_sh) + pw * PH);
@@ -146,7 +150,7 @@ state_pass16_kernel(const StatePassArgs a) {
             s.l[it] = tab[row];
             s.d[it] = REVERSE ? (row <= last ? 1.f : 0.f) : tab[kQ + row];      // dt is 0 past the end of the sequence
         }
-        if (kload < nci - 1) { ++kload; xq += x_step; tq += DIR * 2 * kQ; }      // past the end: the last chunk once more
+        if (kload < nsteps - 1) { ++kload; xq += x_step; tq += DIR * 2 * kQ; }      // past the end: the last step's chunk once more
     };
     // loaded at the top of the iteration that consumes them (so that the wait in front of their use can be counted
     // exactly and leaves the next chunk's rows, issued behind them, in flight): the group's B^T / C^T fragments (L2)
@@ -161,7 +165,33 @@ state_pass16_kernel(const StatePassArgs a) {
         mp += m_step;
     };
 
-    const int q1 = (nci + 3) / 4, q2 = (2 * nci + 3) / 4, q3 = (3 * nci + 3) / 4;      // first chunk of each quarter
+    const int q1 = (nsteps + 3) / 4, q2 = (2 * nsteps + 3) / 4, q3 = (3 * nsteps + 3) / 4;      // first chunk of each quarter
+    auto put_state = [&](T* cO) {
+#pragma unroll
+        for (int i = 0; i < PBW; ++i)
+#pragma unroll
+            for (int j = 0; j < NBW; ++j)
+#pragma unroll
+                for (int qp = 0; qp < 2; ++qp) {
+                    // a lane and its partner (lane ^ 32) hold the two halves of every 8-column group: one exchange of the packed
+                    // words leaves each with a whole group, written as 16 bytes (8-byte writes of 32 rows at this pitch would
+                    // meet pairwise in the same banks)
+                    const int q0 = 2 * qp, q1 = q0 + 1;
+                    uint32_t o0, o1, o2, o3;
+                    pair_swap(pack2<T>(acc[i][j][4 * q0], acc[i][j][4 * q0 + 1]), pack2<T>(acc[i][j][4 * q1], acc[i][j][4 * q1 + 1]), o0, o2);
+                    pair_swap(pack2<T>(acc[i][j][4 * q0 + 2], acc[i][j][4 * q0 + 3]), pack2<T>(acc[i][j][4 * q1 + 2], acc[i][j][4 * q1 + 3]), o1, o3);
+                    *reinterpret_cast<u32x4*>(cO + (i * 32 + r) * LDO + n0 + j * 32 + 8 * (q0 + half)) = u32x4{o0, o1, o2, o3};
+                }
+    };
+    auto store_rows = [&](const T* cO) {      // whole rows of the workgroup's slab
+#pragma unroll
+        for (int ps = 0; ps < NSP; ++ps) {
+            const int rl = wave * RW + ps * RPP + lane / LPR, cv = lane % LPR;
+            const u32x4 o = *reinterpret_cast<const u32x4*>(cO + rl * LDO + cv * 8);
+            *reinterpret_cast<u32x4*>((op + ps * RPP * N * 2) + st_off) = o;
+        }
+        op += o_step;
+    };
     int next_drop = q1;
     __builtin_amdgcn_s_setprio(3);
     auto step = [&](int cc, Ahead& s) {
@@ -209,33 +239,12 @@ state_pass16_kernel(const StatePassArgs a) {
         const float dec = __expf(s.lam);
         // the state as it enters this chunk goes into the slab tile of this parity (the other one may still be read by a
         // wave that is behind: it was filled one barrier ago)
-        T* cO = sO + buf * (PH * LDO);
-#pragma unroll
-        for (int i = 0; i < PBW; ++i)
-#pragma unroll
-            for (int j = 0; j < NBW; ++j)
-#pragma unroll
-                for (int qp = 0; qp < 2; ++qp) {
-                    // a lane and its partner (lane ^ 32) hold the two halves of every 8-column group: one exchange of the packed
-                    // words leaves each with a whole group, written as 16 bytes (8-byte writes of 32 rows at this pitch would
-                    // meet pairwise in the same banks)
-                    const int q0 = 2 * qp, q1 = q0 + 1;
-                    uint32_t o0, o1, o2, o3;
-                    pair_swap(pack2<T>(acc[i][j][4 * q0], acc[i][j][4 * q0 + 1]), pack2<T>(acc[i][j][4 * q1], acc[i][j][4 * q1 + 1]), o0, o2);
-                    pair_swap(pack2<T>(acc[i][j][4 * q0 + 2], acc[i][j][4 * q0 + 3]), pack2<T>(acc[i][j][4 * q1 + 2], acc[i][j][4 * q1 + 3]), o1, o3);
-                    *reinterpret_cast<u32x4*>(cO + (i * 32 + r) * LDO + n0 + j * 32 + 8 * (q0 + half)) = u32x4{o0, o1, o2, o3};
-                }
+        put_state(sO + buf * (PH * LDO));
         __syncthreads();          // both tiles are complete; every wave is done with the other buffers
         load_ahead(s);            // the rows two chunks on
 
-        // ---- the state entering (forward) / the gradient leaving (reverse) this chunk: whole rows of the workgroup's slab
-#pragma unroll
-        for (int ps = 0; ps < NSP; ++ps) {
-            const int rl = wave * RW + ps * RPP + lane / LPR, cv = lane % LPR;
-            const u32x4 o = *reinterpret_cast<const u32x4*>(cO + rl * LDO + cv * 8);
-            *reinterpret_cast<u32x4*>((op + ps * RPP * N * 2) + st_off) = o;
-        }
-        op += o_step;
+        // ---- the state entering (forward) / the gradient leaving (reverse) this chunk
+        store_rows(sO + buf * (PH * LDO));
 
         // ---- S = e^{Lam} S + X_scaled^T M  (accumulated as its transpose M^T X_scaled)
 #pragma unroll
@@ -274,21 +283,21 @@ state_pass16_kernel(const StatePassArgs a) {
     // the loop body is free of conditionals (a branch around loads costs register copies, and with them early waits).
     Ahead s0, s1;
     int cc = 0;
-    if (nci & 1) {
+    if (nsteps & 1) {
         load_ahead(s1);
         load_ahead(s0);
         step(0, s1);
         cc = 1;
-    } else {
+    } else if (nsteps > 0) {
         load_ahead(s0);
         load_ahead(s1);
     }
 #pragma unroll 1
-    for (; cc < nci; cc += 2) {
+    for (; cc < nsteps; cc += 2) {
         step(cc, s0);
         step(cc + 1, s1);
     }
-    if (a.final_out) {
+    if (HILO || a.final_out) {
 #pragma unroll
         for (int i = 0; i < PBW; ++i)
 #pragma unroll
@@ -298,6 +307,11 @@ state_pass16_kernel(const StatePassArgs a) {
                     const int row = pw * PH + i * 32 + r, col = n0 + j * 32 + acc_row(lane, v);
                     a.final_out[bh * (P * N) + row * N + col] = acc[i][j][v];
                 }
+    } else {
+        T* cO = sO + (nsteps & 1) * (PH * LDO);
+        put_state(cO);
+        __syncthreads();
+        store_rows(cO);
     }
 }
 

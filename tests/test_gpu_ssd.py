@@ -345,3 +345,18 @@ def test_ssd_fp32_heads_in_sequence(b, l, h, p, n, g, steps):
         out = ssd_backward(dd["dt"], dd["A"], dd["X"], dd["B"], dd["C"], dd["D"], dd["dy"], chunk_states=states)
         for name, v in zip(("ddt", "dA", "dX", "dB", "dC", "dD"), out):
             assert rel_err(v, r[name]) < 1e-4, name
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,h,p,n", [(2, 6, 64, 64), (1, 3, 128, 128), (8, 32, 64, 128)])      # the last: whole heads in the state pass
+@pytest.mark.parametrize("l", [1, 128, 129, 385])
+def test_ssd_gradients_without_the_initial_states_own(l, b, h, p, n, dtype):
+    """Nobody reads what the last step of the state recurrence adds unless its final output is asked for: the same bits without it."""
+    from mamba2.mamba2_kernel import mamba2_kernel
+    d = _dev(make_ssd_inputs(b, l, h, p, n, 1, seed=l + h, dtype=dtype))
+    leaves = [d[k].requires_grad_(True) for k in ("dt", "A", "X", "B", "C", "D")]
+    zero = torch.zeros(b, h, p, n, device=DEV, requires_grad=True)
+    y1, y2 = mamba2_kernel(*leaves), mamba2_kernel(*leaves, initial_state=zero)
+    g1 = torch.autograd.grad(y1, leaves, d["dy"])
+    g2 = torch.autograd.grad(y2, leaves + [zero], d["dy"])
+    assert torch.equal(y1, y2) and all(torch.equal(a, c) for a, c in zip(g1, g2))
