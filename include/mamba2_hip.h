@@ -263,6 +263,8 @@ int m2_add_rmsnorm(float* residual, int64_t residual_stride_row, const void* del
  * m2_linear_small_fits() says whether a shape is taken.
  * m2_decode_rows: the head of such a chain: residual (rows, channels) fp32 += delta (set != 0: = delta; delta may be NULL
  * otherwise), x = bf16(residual * weight), sq (rows, 1).
+ * m2_embed_rows: the same with residual = table[ids], the embedding of a model's step: table (vocab, channels) fp32 or bf16, ids
+ * (rows) on the device; an id outside the table gives a row of NaN.
  * m2_decode_layer: one decode step of a whole mixer layer in three launches (mamba2/mamba2_mixer.py:243-282): `in` writes
  * zxBCdt (bf16 rows, in->out), the scan reads it and the states of `dec` (updated in place; dec's xBC, dt, y and workspace
  * are not used) and writes the gated rows times norm_weight to out->x (batch, nheads * headdim) bf16 and their sums to
@@ -280,6 +282,8 @@ int m2_linear_small_fits(int64_t M, int64_t N, int64_t K, int32_t groups);
 int m2_linear_small(const m2_linear_params* p, void* stream);
 int m2_decode_rows(float* residual, const void* delta, int32_t delta_dtype, int32_t set, const float* weight, void* x, float* sq, int64_t rows,
                    int64_t channels, void* stream);
+int m2_embed_rows(const void* table, int32_t table_dtype, int64_t vocab, const int64_t* ids, float* residual, const float* weight, void* x, float* sq,
+                  int64_t rows, int64_t channels, void* stream);
 int m2_decode_layer(const m2_linear_params* in, const m2_decode_params* dec, const float* norm_weight, const m2_linear_params* out, void* stream);
 
 /* A linear layer's products on few tokens, bf16 operands and result, fp32 accumulation:

@@ -31,7 +31,7 @@ using torch::autograd::variable_list;
     F(m2_last_error) F(m2_conv1d_fwd) F(m2_conv1d_prefill) F(m2_conv1d_bwd_workspace_bytes) F(m2_conv1d_bwd) F(m2_conv1d_bwd_partial) F(m2_ssd_chunk_states_bytes) \
     F(m2_ssd_fwd_workspace_bytes) F(m2_ssd_fwd_check) F(m2_ssd_fwd) F(m2_ssd_bwd_workspace_bytes) F(m2_ssd_bwd) F(m2_decode_workspace_bytes) \
     F(m2_decode_step) F(m2_decode_step_static) F(m2_rmsnorm_gated_fwd_check) F(m2_rmsnorm_gated_fwd) F(m2_rmsnorm_gated_bwd_workspace_bytes) \
-    F(m2_rmsnorm_gated_bwd) F(m2_rmsnorm_gated_bwd_partial) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_rows) F(m2_decode_layer) F(m2_mixer_params) F(m2_param_sums) \
+    F(m2_rmsnorm_gated_bwd) F(m2_rmsnorm_gated_bwd_partial) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_rows) F(m2_embed_rows) F(m2_decode_layer) F(m2_mixer_params) F(m2_param_sums) \
     F(m2_product_pays) F(m2_product_workspace_bytes) F(m2_product)
 struct Lib {
 #define M2_FIELD(name) decltype(&::name) name = nullptr;
@@ -974,7 +974,8 @@ struct StepArgs {
 // or `x` holds the rows times the next norm's weight and `sq` their sums of squares (chained kernels), or neither.
 struct ResidualStream {
     Tensor rows, delta, x, sq;
-    Tensor first;                  // embedding rows that `rows` is yet to be set to
+    Tensor first;                  // embedding rows that `rows` is yet to be set to, or
+    Tensor table, ids;             // the embedding and the rows of it that will be these
 };
 
 bool starts_at(const Tensor& t, size_t bytes) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % bytes == 0; }
@@ -1008,8 +1009,16 @@ Tensor linear_rows(const Tensor& x, const Tensor& w, const Tensor& bias, void* s
     return out;
 }
 
+// a tensor of the stream's width, on its device; how many rows the stream has
+const Tensor& stream_anchor(const ResidualStream& r) { return r.first.defined() ? r.first : r.ids.defined() ? r.table : r.rows; }
+int64_t stream_count(const ResidualStream& r) { return r.ids.defined() ? r.ids.numel() : stream_anchor(r).size(0); }
+
 // the stream's rows, set from the embedding if they are not yet
 const Tensor& stream_rows(ResidualStream& r) {
+    if (r.ids.defined()) {
+        r.first = at::embedding(r.table, r.ids);
+        r.table = r.ids = Tensor();
+    }
     if (r.first.defined()) {
         r.rows = r.first.to(at::kFloat, /*non_blocking=*/false, /*copy=*/true, at::MemoryFormat::Contiguous);
         r.first = Tensor();
@@ -1034,6 +1043,15 @@ Tensor stream_add_norm(ResidualStream& r, const Tensor& norm_w, double eps, at::
 // x and sq of the stream for a norm weight
 void stream_heads(ResidualStream& r, const Tensor& norm_w, void* stream) {
     if (r.x.defined()) return;
+    if (r.ids.defined()) {
+        r.rows = at::empty({r.ids.numel(), r.table.size(1)}, r.table.options().dtype(at::kFloat));
+        r.x = at::empty(r.rows.sizes(), r.rows.options().dtype(at::kBFloat16));
+        r.sq = at::empty({r.rows.size(0), 1}, r.rows.options());
+        check(lib.m2_embed_rows(ptr(r.table), dtype_code(r.table), r.table.size(0), r.ids.data_ptr<int64_t>(), ptr<float>(r.rows), ptr<float>(norm_w), ptr(r.x),
+                                ptr<float>(r.sq), r.rows.size(0), r.rows.size(1), stream), "m2_embed_rows");
+        r.table = r.ids = Tensor();
+        return;
+    }
     const bool set = r.first.defined();
     const Tensor src = set ? r.first.contiguous() : (r.delta.defined() ? r.delta.contiguous() : Tensor());
     if (set) r.rows = at::empty(src.sizes(), src.options().dtype(at::kFloat));
@@ -1112,9 +1130,9 @@ Tensor mixer_step(const OptTensor& hidden_, ResidualStream* r, const OptTensor& 
                   const OptTensor& in_b, const Tensor& conv_w, const OptTensor& conv_b, const Tensor& A, const Tensor& D, const Tensor& dt_bias, const Tensor& norm_w,
                   double eps, int64_t norm_groups, const Tensor& out_w, const OptTensor& out_b, const Tensor& conv_state, const Tensor& ssm_state, int64_t g) {
     const Tensor &hidden = or_none(hidden_), &block_norm = or_none(block_norm_), &next_norm = or_none(next_norm_);
-    const Tensor& x = r ? (r->first.defined() ? r->first : r->rows) : hidden;
+    const Tensor& x = r ? stream_anchor(*r) : hidden;
     TORCH_CHECK_VALUE(x.defined() && (r ? x.dim() == 2 : x.dim() == 3 && x.size(1) == 1), "hidden_states must be (batch, 1, hidden_size)");
-    const int64_t b = x.size(0), width = x.size(-1);
+    const int64_t b = r ? stream_count(*r) : x.size(0), width = x.size(-1);
     require_gpu({&x, &in_w, &or_none(in_b), &conv_w, &or_none(conv_b), &A, &D, &dt_bias, &norm_w, &block_norm, &next_norm, &out_w, &or_none(out_b),
                  &conv_state, &ssm_state});
     TORCH_CHECK_VALUE(ssm_state.dim() == 4 && ssm_state.size(0) == b && ssm_state.scalar_type() == at::kFloat && ssm_state.is_contiguous(),
@@ -1148,9 +1166,21 @@ ResidualStream residual_stream(const Tensor& embedded) {
     return r;
 }
 
+// A model's stream at its embedding, which the stream's first kernel reads itself where the table lies as it takes it.
+ResidualStream embedded_stream(const Tensor& table, const Tensor& ids) {
+    require_gpu({&table, &ids});
+    const bool reads = (table.scalar_type() == at::kFloat || table.scalar_type() == at::kBFloat16) && table.dim() == 2 && table.is_contiguous() &&
+                       table.size(1) > 0 && ids.scalar_type() == at::kLong && ids.numel() <= 65535;
+    if (!reads) return residual_stream(at::embedding(table, ids));
+    ResidualStream r;
+    r.table = table;
+    r.ids = ids.reshape({-1}).contiguous();
+    return r;
+}
+
 // the stream's rows as they are, everything added
 Tensor stream_sum(ResidualStream& r) {
-    const Tensor& any = r.first.defined() ? r.first : r.rows;
+    const Tensor any = stream_anchor(r);
     Scope scope(any);
     const Tensor& rows = stream_rows(r);
     if (r.delta.defined()) { rows.add_(r.delta); r.delta = Tensor(); }
@@ -1169,11 +1199,11 @@ Tensor stream_norm_linear(ResidualStream& r, const Tensor& norm_w, double eps, c
     const Tensor& bias = or_none(bias_);
     require_gpu({&norm_w, &w, &bias});
     check_fp32({&norm_w}, "the norm weight");
-    const Tensor& any = r.first.defined() ? r.first : r.rows;
+    const Tensor any = stream_anchor(r);
     require_gpu({&any, &w});
     TORCH_CHECK_VALUE(w.dim() == 2 && any.size(1) == w.size(1) && norm_w.numel() == w.size(1), "the norm weight and the product must have the width of the residual stream");
     Scope scope(w);
-    m2_linear_params p = linear_params(w, bias, any.size(0));
+    m2_linear_params p = linear_params(w, bias, stream_count(r));
     if (!linear_takes(w, bias) || !lib.m2_linear_small_fits(p.M, p.N, p.K, 1)) {
         const at::ScalarType normed = w.scalar_type() == at::kBFloat16 ? at::kBFloat16 : at::kFloat;      // the norm's output types
         return linear_rows(stream_add_norm(r, norm_w, eps, normed).to(w.scalar_type()), w, bias, scope.stream).to(at::kFloat);
@@ -1210,6 +1240,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("fused_prefill", &fused_prefill);
     m.def("mixer_step", &mixer_step);
     m.def("residual_stream", &residual_stream);
+    m.def("embedded_stream", &embedded_stream);
     m.def("stream_sum", &stream_sum);
     m.def("stream_norm", &stream_norm);
     m.def("linear", &linear);

@@ -112,6 +112,7 @@ SYMBOLS = {
     "m2_linear_small_fits": (C.c_int, [_i64, _i64, _i64, _i32]),
     "m2_linear_small": (C.c_int, [C.POINTER(LinearParams), _vp]),
     "m2_decode_rows": (C.c_int, [_vp, _vp, _i32, _i32, _vp, _vp, _vp, _i64, _i64, _vp]),
+    "m2_embed_rows": (C.c_int, [_vp, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp]),
     "m2_decode_layer": (C.c_int, [C.POINTER(LinearParams), C.POINTER(DecodeParams), _vp, C.POINTER(LinearParams), _vp]),
     "m2_product_fits": (C.c_int, [_i64, _i64, _i64, _i32, _i32]),
     "m2_product_pays": (C.c_int, [_i64, _i64, _i64, _i32, _i32]),

@@ -198,7 +198,11 @@ class Mamba2Model(Mamba2PreTrainedModel):
         if not (len(self.layers) and _plain(self.norm_f, Mamba2RMSNorm) and all(_own_step(blk, Mamba2Block) and blk._native_step() for blk in self.layers)):
             return None
         norms = [blk.norm for blk in self.layers] + [self.norm_f]
-        stream = _lib.native().residual_stream(self.embeddings(input_ids))
+        emb = self.embeddings
+        if _plain(emb, nn.Embedding) and emb.max_norm is None:
+            stream = _lib.native().embedded_stream(emb.weight, input_ids)
+        else:
+            stream = _lib.native().residual_stream(emb(input_ids))
         for i, mixer_block in enumerate(self.layers):
             mixer_block.mixer._step(cache_params, stream=stream, block_norm=norms[i], next_norm=norms[i + 1])
         return stream

@@ -100,3 +100,24 @@ def test_linear_small_few_rows(M, N, K, groups):
 @pytest.mark.parametrize("W", [5, 8])
 def test_layer_step_conv_widths(W):
     test_layer_step_against_oracle(3, 8, 64, 64, 1, W, True, False)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,channels,offset", [(1, 64, 0), (3, 1030, 0), (8, 1024, 0), (5, 2048, 1), (33, 7, 0)])      # offset: a table on no vector
+def test_embed_rows(rows, channels, offset, dtype):
+    from mamba2 import _lib
+    lib, gen = _lib.load(), torch.Generator().manual_seed(channels)
+    vocab = 11
+    table = torch.randn(vocab * channels + offset, generator=gen).to(DEV, dtype)[offset:].view(vocab, channels)
+    ids = torch.randint(0, vocab, (rows,), generator=gen)
+    ids[0] = vocab                                  # outside the table
+    ids, w = ids.to(DEV), torch.rand(channels, generator=gen).to(DEV) + 0.5
+    res, x, sq = torch.empty(rows, channels, device=DEV), torch.empty(rows, channels, device=DEV, dtype=torch.bfloat16), torch.empty(rows, 1, device=DEV)
+    rc = lib.m2_embed_rows(table.data_ptr(), _lib.M2_F32 if dtype == torch.float32 else _lib.M2_BF16, vocab, ids.data_ptr(), res.data_ptr(), w.data_ptr(),
+                           x.data_ptr(), sq.data_ptr(), rows, channels, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert res[0].isnan().all() and x[0].isnan().all() and sq[0].isnan().all()
+    want = table[ids[1:]].float()
+    assert torch.equal(res[1:], want) and torch.equal(x[1:], (want * w).bfloat16())
+    # fp32 sums of `channels` squares in another order: at most channels roundings of 2^-24 each
+    assert torch.allclose(sq[1:, 0], want.pow(2).sum(1), rtol=channels * 2.0 ** -24, atol=0.0)
