@@ -302,6 +302,13 @@ int m2_product_pays(int64_t M, int64_t N, int64_t K, int32_t a_k, int32_t b_k);
 size_t m2_product_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int m2_product(const m2_product_params* p, void* stream);
 
+/* Both products of a linear layer's backward in one launch: x: dy W (a_k 1, b_k 0), w: dy^T x (a_k 0, b_k 0), as m2_product takes
+ * them, without a bias; x's workspace as m2_product_pair_workspace_bytes says (0: none).  m2_product_pair_pays: the faster choice
+ * over one after the other. */
+int m2_product_pair_pays(const m2_product_params* x, const m2_product_params* w);
+size_t m2_product_pair_workspace_bytes(const m2_product_params* x, const m2_product_params* w);
+int m2_product_pair(const m2_product_params* x, const m2_product_params* w, void* stream);
+
 /* The small parameters of a mixer layer as the kernels take them, and their gradients back, in one launch each
  * (mamba2/mamba2_mixer.py:225-236: A = -exp(A_log.float()) and the casts around it).
  * m2_mixer_params:       out (3 * nheads + channels) fp32 = [ -exp(A_log) | D | dt_bias | norm_weight ].

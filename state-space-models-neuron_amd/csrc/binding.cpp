@@ -32,7 +32,8 @@ using torch::autograd::variable_list;
     F(m2_ssd_fwd_workspace_bytes) F(m2_ssd_fwd_check) F(m2_ssd_fwd) F(m2_ssd_bwd_workspace_bytes) F(m2_ssd_bwd) F(m2_decode_workspace_bytes) \
     F(m2_decode_step) F(m2_decode_step_static) F(m2_rmsnorm_gated_fwd_check) F(m2_rmsnorm_gated_fwd) F(m2_rmsnorm_gated_bwd_workspace_bytes) \
     F(m2_rmsnorm_gated_bwd) F(m2_rmsnorm_gated_bwd_partial) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_rows) F(m2_embed_rows) F(m2_decode_layer) F(m2_mixer_params) F(m2_param_sums) \
-    F(m2_product_pays) F(m2_product_workspace_bytes) F(m2_product)
+    F(m2_product_pays) F(m2_product_workspace_bytes) F(m2_product) \
+    F(m2_product_pair_pays) F(m2_product_pair_workspace_bytes) F(m2_product_pair)
 struct Lib {
 #define M2_FIELD(name) decltype(&::name) name = nullptr;
     M2_BOUND(M2_FIELD)
@@ -762,26 +763,48 @@ Tensor fused_core(const Tensor& zx, const Tensor& A, const OptTensor& D, const T
 // two, by what the tuner's own timing preferred; 11.8 with the default ones).  Asking costs 2 ns.
 bool library_is_tuned() { return at::cuda::tunable::getTuningContext()->IsTunableOpEnabled(); }
 
-// out (M, N) = A B (+ bias): `a` is A or, if !a_k, A^T (K, M); `b` is B^T (N, K) or, if !b_k, B
-Tensor product(const Tensor& a, bool a_k, const Tensor& b, bool b_k, const Tensor& bias, void* stream) {
+m2_product_params product_params(const Tensor& a, bool a_k, const Tensor& b, bool b_k) {
     m2_product_params p{};
     p.M = a.size(a_k ? 0 : 1); p.K = a.size(a_k ? 1 : 0); p.N = b.size(b_k ? 0 : 1);
-    p.lda = a.stride(0); p.ldb = b.stride(0); p.ldo = p.N; p.a_k = a_k; p.b_k = b_k;
-    auto rows = [](const Tensor& t) {
-        return t.scalar_type() == at::kBFloat16 && t.stride(1) == 1 && t.stride(0) % 8 == 0 && t.stride(0) >= t.size(1) &&
-               t.size(0) * t.stride(0) < (int64_t{1} << 31) && reinterpret_cast<uintptr_t>(ptr(t)) % 16 == 0;
-    };
+    p.a = ptr(a); p.b = ptr(b); p.lda = a.stride(0); p.ldb = b.stride(0); p.ldo = p.N; p.a_k = a_k; p.b_k = b_k;
+    return p;
+}
+// an operand as the kernels read it
+bool product_rows(const Tensor& t) {
+    return t.scalar_type() == at::kBFloat16 && t.stride(1) == 1 && t.stride(0) % 8 == 0 && t.stride(0) >= t.size(1) &&
+           t.size(0) * t.stride(0) < (int64_t{1} << 31) && reinterpret_cast<uintptr_t>(ptr(t)) % 16 == 0;
+}
+
+// out (M, N) = A B (+ bias): `a` is A or, if !a_k, A^T (K, M); `b` is B^T (N, K) or, if !b_k, B
+Tensor product(const Tensor& a, bool a_k, const Tensor& b, bool b_k, const Tensor& bias, void* stream) {
+    m2_product_params p = product_params(a, a_k, b, b_k);
     const bool plain_bias = !bias.defined() || (bias.scalar_type() == at::kBFloat16 && bias.is_contiguous() && bias.dim() == 1 && bias.size(0) == p.N);
-    if (!plain_bias || !rows(a) || !rows(b) || b.size(b_k ? 1 : 0) != p.K || !lib.m2_product_pays(p.M, p.N, p.K, a_k, b_k) || library_is_tuned()) {
+    if (!plain_bias || !product_rows(a) || !product_rows(b) || b.size(b_k ? 1 : 0) != p.K || !lib.m2_product_pays(p.M, p.N, p.K, a_k, b_k) || library_is_tuned()) {
         const Tensor at_ = a_k ? a : a.t(), bt = b_k ? b.t() : b;
         return bias.defined() ? at::addmm(bias, at_, bt) : at::mm(at_, bt);
     }
     const Tensor out = at::empty({p.M, p.N}, a.options());
     p.workspace_bytes = lib.m2_product_workspace_bytes(p.M, p.N, p.K);
     const Tensor ws = p.workspace_bytes ? at::empty({static_cast<int64_t>(p.workspace_bytes)}, a.options().dtype(at::kByte)) : Tensor();
-    p.a = ptr(a); p.b = ptr(b); p.bias = ptr(bias); p.out = ptr(out); p.workspace = ptr(ws);
+    p.bias = ptr(bias); p.out = ptr(out); p.workspace = ptr(ws);
     check(lib.m2_product(&p, stream), "m2_product");
     return out;
+}
+
+// What a linear layer's backward needs of its products, (dy W, dy^T x) or only one of them: in one launch where that pays.
+std::pair<Tensor, Tensor> linear_grads(const Tensor& dy, const Tensor& w, const Tensor& x, bool want_x, bool want_w, void* stream) {
+    if (want_x && want_w && product_rows(dy) && product_rows(w) && product_rows(x) && !library_is_tuned()) {
+        m2_product_params px = product_params(dy, true, w, false), pw = product_params(dy, false, x, false);
+        if (w.size(0) == px.K && x.size(0) == pw.K && lib.m2_product_pair_pays(&px, &pw)) {
+            const Tensor dx = at::empty({px.M, px.N}, dy.options()), dw = at::empty({pw.M, pw.N}, dy.options());
+            px.workspace_bytes = lib.m2_product_pair_workspace_bytes(&px, &pw);
+            const Tensor ws = px.workspace_bytes ? at::empty({static_cast<int64_t>(px.workspace_bytes)}, dy.options().dtype(at::kByte)) : Tensor();
+            px.out = ptr(dx); pw.out = ptr(dw); px.workspace = ptr(ws);
+            check(lib.m2_product_pair(&px, &pw, stream), "m2_product_pair");
+            return {dx, dw};
+        }
+    }
+    return {want_x ? product(dy, true, w, false, Tensor(), stream) : Tensor(), want_w ? product(dy, false, x, false, Tensor(), stream) : Tensor()};
 }
 Tensor project(const Tensor& x, const Tensor& w, const Tensor& bias, void* stream) { return product(x, true, w, true, bias, stream); }
 
@@ -839,9 +862,10 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
         const CoreParams params = params_in(small, k.h);
         variable_list out(17);
         const Tensor dy = grads[0].reshape({rows, s[kOutW].size(0)});
-        if (ctx->needs_input_grad(kOutW)) out[kOutW] = product(dy, false, s[kNormOut], false, Tensor(), scope.stream);
+        Tensor d_core;
+        std::tie(d_core, out[kOutW]) = linear_grads(dy, s[kOutW], s[kNormOut], true, ctx->needs_input_grad(kOutW), scope.stream);
+        d_core = d_core.view({k.b, k.l, k.d});
         if (s[kOutB].defined()) out[kOutB] = dy.sum(0);
-        const Tensor d_core = product(dy, true, s[kOutW], false, Tensor(), scope.stream).view({k.b, k.l, k.d});
         CoreOut f;
         if (s.size() > kConvOut) { f.conv_out = s[kConvOut]; f.scan_out = s[kScanOut]; f.states = s[kStates]; }
         else f = core_forward(k, params, s[kConvW], s[kConvB], true, false, scope.stream);
@@ -853,8 +877,9 @@ struct MixerFn : torch::autograd::Function<MixerFn> {
             if (!casts(s[i])) out[i] = out[i].to(s[i].scalar_type());
         out[kConvW] = r.conv_w; out[kConvB] = r.conv_b;
         const Tensor d_zx = r.zx.view({rows, zx.size(2)});
-        if (ctx->needs_input_grad(kHidden)) out[kHidden] = product(d_zx, true, s[kInW], false, Tensor(), scope.stream).view(s[kHidden].sizes());
-        if (ctx->needs_input_grad(kInW)) out[kInW] = product(d_zx, false, s[kHidden].reshape({rows, s[kHidden].size(2)}), false, Tensor(), scope.stream);
+        std::tie(out[kHidden], out[kInW]) = linear_grads(d_zx, s[kInW], s[kHidden].reshape({rows, s[kHidden].size(2)}), ctx->needs_input_grad(kHidden),
+                                                         ctx->needs_input_grad(kInW), scope.stream);
+        if (out[kHidden].defined()) out[kHidden] = out[kHidden].view(s[kHidden].sizes());
         if (s[kInB].defined()) out[kInB] = d_zx.sum(0);
         return out;
     }

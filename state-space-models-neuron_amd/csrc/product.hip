@@ -64,9 +64,9 @@ __device__ __forceinline__ Frag<bf16_t> tile_frag(const bf16_t* t, int r0, int k
     return f;
 }
 
+// Workgroup `block` of `blocks` (a multiple of 8, and block 0 on the first XCD) of a product.
 template <bool AK, bool BK, int R>
-__global__ void __launch_bounds__(256, R == 64 ? 2 : 1)
-product_kernel(const ProductArgs p) {
+__device__ __forceinline__ void product_body(const ProductArgs& p, unsigned block, unsigned blocks) {
     static_assert(R == 64 || R == 128, "tiles of 64 x 64 or 128 x 128");
     constexpr bool KSPLIT = R == 64;                               // the waves split k, else the tile
     constexpr int kElems = R * kK, NP = R / 32, PER = 2 * NP;      // an operand tile; copies per wave of one operand, of both
@@ -78,7 +78,7 @@ product_kernel(const ProductArgs p) {
     // another on it, and its L2 hands them the same rows of B.  Whole columns dealt round the XCDs instead left some with half as much
     // again as others, and two rounds where one would do (20 columns of 3 tiles, four splits: 36 workgroups on the 32 CUs of half of
     // them): 257 x 2560 x 10576 63 -> 39 us, 737 x 1792 x 7480 65 -> 40, 1326 x 2560 x 10576 216 -> 120.
-    const int tiles = p.tiles_m * p.tiles_n, at = (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3));
+    const int tiles = p.tiles_m * p.tiles_n, at = (int)((block & 7) * (blocks >> 3) + (block >> 3));
     if (at >= tiles * p.splits) return;
     const int split = at / tiles, tn = (at - split * tiles) / p.tiles_m, tm = (at - split * tiles) % p.tiles_m;
     const int m0 = tm * R, n0 = tn * R;
@@ -191,6 +191,23 @@ product_kernel(const ProductArgs p) {
     }
 }
 
+template <bool AK, bool BK, int R>
+__global__ void __launch_bounds__(256, R == 64 ? 2 : 1)
+product_kernel(const ProductArgs p) { product_body<AK, BK, R>(p, blockIdx.x, gridDim.x); }
+
+// Both products of a linear layer's backward in one launch: dx = dy W (x) and dW = dy^T x (w), in tiles of 64.  On a few hundred tokens
+// either alone leaves half of the chip to wait through its prologue and its last tile (4.6 us of the 7 to 15 that it takes).  The
+// workgroups with the longer sums go first.  500 tokens,
+// 768 channels: out_proj's 13.8 -> 8.4 us, in_proj's (dx split in two) 24.8 -> 18.6.
+__global__ void __launch_bounds__(256, 2)
+product_pair_kernel(const ProductArgs x, const ProductArgs w, unsigned x_blocks, unsigned w_blocks, int x_first) {
+    const unsigned first = x_first ? x_blocks : w_blocks;
+    const bool is_x = (blockIdx.x < first) == (x_first != 0);
+    const unsigned block = blockIdx.x < first ? blockIdx.x : blockIdx.x - first;
+    if (is_x) product_body<true, false, 64>(x, block, x_blocks);
+    else product_body<false, false, 64>(w, block, w_blocks);
+}
+
 __global__ void __launch_bounds__(256)
 product_sum_kernel(const float* __restrict__ part, const bf16_t* __restrict__ bias, bf16_t* __restrict__ out, int64_t ldo, int M, int N, int splits) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x, n8 = N / 8;
@@ -216,11 +233,10 @@ product_sum_kernel(const float* __restrict__ part, const bf16_t* __restrict__ bi
 // fitted to 144 products of layers of 256 to 3072 channels over 33 to 2048 tokens, in all forms (the choice is within 1 % of the best of
 // tiles and one to six splits there on average, within 20 % for all).  Two workgroups of the small tile share a CU and hide each
 // other's waits; a split costs its second launch and the partials' way out and back.
-struct ProductPlan { int r, splits, ksteps; };
+struct ProductPlan { int r, splits, ksteps; float us; };
 ProductPlan product_plan(int64_t M, int64_t N, int64_t K) {
     const int64_t cus = device_cus() / 8, ktiles = ceil_div(K, (int64_t)kK);
-    ProductPlan best{64, 1, (int)ktiles};
-    float best_us = 1e30f;
+    ProductPlan best{64, 1, (int)ktiles, 1e30f};
     for (const int r : {64, 128}) {
         const int64_t tiles = ceil_div(M, (int64_t)r) * ceil_div(N, (int64_t)r);
         for (int64_t want = 1; want <= 6 && (want == 1 || ktiles / want >= 4); ++want) {
@@ -228,8 +244,25 @@ ProductPlan product_plan(int64_t M, int64_t N, int64_t K) {
             float us = r == 64 ? (float)ks * 0.3f * (1.6f * (busiest / 2) + busiest % 2) + 1.2f * ceil_div(busiest, (int64_t)2)
                                : (float)busiest * (ks * 0.54f + 1.8f);
             if (s > 1) us += 1.6f + 3e-6f * s * M * N;
-            if (us < best_us) { best_us = us; best = {r, (int)s, (int)ks}; }
+            if (us < best.us) best = {r, (int)s, (int)ks, us};
         }
+    }
+    return best;
+}
+
+// Both products of a linear layer's backward in one launch, in the same count: the longer chain of k steps, or all of them at the rate
+// of CUs with two workgroups each.  Only dx's sum, over the layer's outputs, gets long enough to be split.
+struct PairPlan { int splits, ksteps; float us, work; };      // work: k steps per CU
+PairPlan pair_plan(const m2_product_params& x, const m2_product_params& w) {
+    const int64_t kx = ceil_div(x.K, (int64_t)kK), kw = ceil_div(w.K, (int64_t)kK);
+    const int64_t tx = ceil_div(x.M, (int64_t)64) * ceil_div(x.N, (int64_t)64), tw = ceil_div(w.M, (int64_t)64) * ceil_div(w.N, (int64_t)64);
+    const float work = (float)(tx * kx + tw * kw) / (float)device_cus();
+    PairPlan best{1, (int)kx, 1e30f, work};
+    for (int64_t want = 1; want <= 6 && (want == 1 || kx / want >= 4); ++want) {
+        const int64_t ks = ceil_div(kx, want), n = ceil_div(kx, ks);
+        const float chain = 0.3f * (float)(ks > kw ? ks : kw);
+        const float us = (chain > 0.24f * work ? chain : 0.24f * work) + 1.2f + (n > 1 ? 1.6f + 3e-6f * (float)(n * x.M * x.N) : 0.f);
+        if (us < best.us) best = {(int)n, (int)ks, us, work};
     }
     return best;
 }
@@ -264,8 +297,10 @@ extern "C" size_t m2_product_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
 }
 
-extern "C" int m2_product(const m2_product_params* p, void* stream) {
-    using namespace m2;
+namespace m2 {
+namespace {
+
+int check_product(const m2_product_params* p) {
     M2_REQUIRE(p && p->a && p->b && p->out, M2_ERR_NULL, "product: a, b and out are required");
     M2_REQUIRE(m2_product_fits(p->M, p->N, p->K, p->a_k, p->b_k), M2_ERR_SHAPE, "product: shape %lld x %lld x %lld is not taken",
                (long long)p->M, (long long)p->N, (long long)p->K);
@@ -274,20 +309,39 @@ extern "C" int m2_product(const m2_product_params* p, void* stream) {
     M2_REQUIRE(p->lda >= (p->a_k ? p->K : p->M) && p->ldb >= (p->b_k ? p->K : p->N) && p->ldo >= p->N, M2_ERR_SHAPE, "product: row strides too short");
     M2_REQUIRE((p->a_k ? p->M : 64) * p->lda < ((int64_t)1 << 31) && (p->b_k ? p->N : 64) * p->ldb < ((int64_t)1 << 31), M2_ERR_SHAPE,
                "product: operand too large for 32-bit offsets");
-    hipStream_t st = static_cast<hipStream_t>(stream);
+    return M2_OK;
+}
+
+ProductArgs product_args(const m2_product_params* p, int r, int splits, int ksteps) {
     ProductArgs a{};
     a.A = static_cast<const bf16_t*>(p->a); a.B = static_cast<const bf16_t*>(p->b); a.bias = static_cast<const bf16_t*>(p->bias);
     a.out = static_cast<bf16_t*>(p->out); a.lda = p->lda; a.ldb = p->ldb; a.ldo = p->ldo;
     a.M = (int)p->M; a.N = (int)p->N; a.K = (int)p->K;
+    a.tiles_m = (int)ceil_div(p->M, (int64_t)r); a.tiles_n = (int)ceil_div(p->N, (int64_t)r);
+    a.splits = splits; a.ksteps = ksteps;
+    return a;
+}
+int launch_sum(const ProductArgs& a, hipStream_t st) {
+    product_sum_kernel<<<(unsigned)ceil_div((int64_t)a.M * (a.N / 8), (int64_t)256), 256, 0, st>>>(a.part, a.bias, a.out, a.ldo, a.M, a.N, a.splits);
+    return check_launch("product_sum_kernel");
+}
+unsigned product_blocks(const ProductArgs& a) { return (unsigned)(ceil_div((int64_t)a.tiles_m * a.tiles_n * a.splits, (int64_t)8) * 8); }
+
+}  // namespace
+}  // namespace m2
+
+extern "C" int m2_product(const m2_product_params* p, void* stream) {
+    using namespace m2;
+    if (const int bad = check_product(p)) return bad;
+    hipStream_t st = static_cast<hipStream_t>(stream);
     const ProductPlan plan = product_plan(p->M, p->N, p->K);
     const int splits = plan.splits;
-    a.tiles_m = (int)ceil_div(p->M, (int64_t)plan.r); a.tiles_n = (int)ceil_div(p->N, (int64_t)plan.r); a.ksteps = plan.ksteps;
+    ProductArgs a = product_args(p, plan.r, splits, plan.ksteps);
     if (splits > 1) {
         M2_REQUIRE(p->workspace && p->workspace_bytes >= (size_t)splits * p->M * p->N * 4, M2_ERR_WORKSPACE, "product: workspace too small");
         a.part = static_cast<float*>(p->workspace);
     }
-    a.splits = splits;
-    const unsigned grid = (unsigned)(ceil_div((int64_t)a.tiles_m * a.tiles_n * splits, (int64_t)8) * 8);
+    const unsigned grid = product_blocks(a);
     const size_t sm = (size_t)kRing * 2 * plan.r * kK * 2;
     auto launch = [&](auto k) -> int {
         if (const int rc = allow_smem(k, sm)) return rc;
@@ -301,6 +355,47 @@ extern "C" int m2_product(const m2_product_params* p, void* stream) {
     };
     const int rc = plan.r == 64 ? form(std::integral_constant<int, 64>{}) : form(std::integral_constant<int, 128>{});
     if (rc || splits == 1) return rc;
-    product_sum_kernel<<<(unsigned)ceil_div(p->M * (p->N / 8), (int64_t)256), 256, 0, st>>>(a.part, a.bias, a.out, a.ldo, a.M, a.N, splits);
-    return check_launch("product_sum_kernel");
+    return launch_sum(a, st);
+}
+
+// Against two products of this file their own count decides (1.5 us for the launch more): 1.1 to 1.8 times as fast over the 40 such pairs
+// of layers of 256 to 1024 channels on 40 to 2000 tokens, and the one that it turns away is 3 % slower.  Where either would go to the
+// general library: up to 150 k steps per CU.  Below it 40 tokens, 1024 channels 24.5 -> 14.1 us, 1000 tokens 54 -> 40, 500 tokens, 1536
+// channels, out_proj 30 -> 23.6, in_proj 48.5 -> 46.9; above it 1000 tokens, 1280 channels, in_proj 59 -> 67, 2048 channels, out_proj 54 -> 65.
+extern "C" int m2_product_pair_pays(const m2_product_params* x, const m2_product_params* w) {
+    using namespace m2;
+    if (!x || !w || !x->a_k || x->b_k || w->a_k || w->b_k || x->bias || w->bias) return 0;
+    if (!m2_product_fits(x->M, x->N, x->K, 1, 0) || !m2_product_fits(w->M, w->N, w->K, 0, 0)) return 0;
+    const PairPlan plan = pair_plan(*x, *w);
+    if (!m2_product_pays(x->M, x->N, x->K, 1, 0) || !m2_product_pays(w->M, w->N, w->K, 0, 0)) return plan.work <= 150.f;
+    return plan.us < product_plan(x->M, x->N, x->K).us + product_plan(w->M, w->N, w->K).us + 1.5f;
+}
+
+extern "C" size_t m2_product_pair_workspace_bytes(const m2_product_params* x, const m2_product_params* w) {
+    const int n = x && w ? m2::pair_plan(*x, *w).splits : 1;
+    return n > 1 ? (size_t)n * x->M * x->N * sizeof(float) : 0;
+}
+
+extern "C" int m2_product_pair(const m2_product_params* x, const m2_product_params* w, void* stream) {
+    using namespace m2;
+    int rc = check_product(x);
+    if (!rc) rc = check_product(w);
+    if (rc) return rc;
+    M2_REQUIRE(x->a_k && !x->b_k && !w->a_k && !w->b_k && !x->bias && !w->bias, M2_ERR_SHAPE, "product_pair: dy W and dy^T x, without a bias");
+    M2_REQUIRE(ceil_div(x->M, (int64_t)64) * ceil_div(x->N, (int64_t)64) + ceil_div(w->M, (int64_t)64) * ceil_div(w->N, (int64_t)64) < (1 << 30), M2_ERR_SHAPE,
+               "product_pair: too many tiles");
+    const PairPlan plan = pair_plan(*x, *w);
+    ProductArgs ax = product_args(x, 64, plan.splits, plan.ksteps);
+    const ProductArgs aw = product_args(w, 64, 1, (int)ceil_div(w->K, (int64_t)kK));
+    if (plan.splits > 1) {
+        M2_REQUIRE(x->workspace && x->workspace_bytes >= m2_product_pair_workspace_bytes(x, w), M2_ERR_WORKSPACE, "product_pair: workspace too small");
+        ax.part = static_cast<float*>(x->workspace);
+    }
+    const unsigned bx = product_blocks(ax), bw = product_blocks(aw);
+    const size_t sm = (size_t)kRing * 2 * 64 * kK * 2;
+    if ((rc = allow_smem(product_pair_kernel, sm))) return rc;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    product_pair_kernel<<<bx + bw, 256, sm, st>>>(ax, aw, bx, bw, ax.ksteps >= aw.ksteps);
+    if ((rc = check_launch("product_pair_kernel")) || plan.splits == 1) return rc;
+    return launch_sum(ax, st);
 }

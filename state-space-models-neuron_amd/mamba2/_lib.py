@@ -118,6 +118,9 @@ SYMBOLS = {
     "m2_product_pays": (C.c_int, [_i64, _i64, _i64, _i32, _i32]),
     "m2_product_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "m2_product": (C.c_int, [C.POINTER(ProductParams), _vp]),
+    "m2_product_pair_pays": (C.c_int, [C.POINTER(ProductParams), C.POINTER(ProductParams)]),
+    "m2_product_pair_workspace_bytes": (_sz, [C.POINTER(ProductParams), C.POINTER(ProductParams)]),
+    "m2_product_pair": (C.c_int, [C.POINTER(ProductParams), C.POINTER(ProductParams), _vp]),
     "m2_mixer_params": (C.c_int, [_vp, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _vp, _i64, _i64, _vp]),
     "m2_mixer_params_grads": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _i64, _i64, _vp]),
     "m2_param_sums": (C.c_int, [_vp, _i64, _i64, _vp, _i32, _vp, _i64, _i64, _vp, _vp, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _i32,

@@ -62,3 +62,35 @@ def test_product_refuses_other_storage(M, N, K, a_k, b_k):
     p = _lib.ProductParams(a=_lib.ptr(t), b=_lib.ptr(t), out=_lib.ptr(t), M=M, N=N, K=K, lda=8, ldb=8, ldo=8, a_k=a_k, b_k=b_k)
     with pytest.raises(ValueError, match="is not taken"):
         _lib.check(lib.m2_product(p, _lib.stream_ptr()), "m2_product")
+
+
+# both products of a linear layer's backward in one launch: single and ragged tiles, either chain the longer one, dx split over k
+@pytest.mark.parametrize("tokens,outs,ins", [(1, 8, 8), (64, 64, 64), (65, 72, 200), (1000, 72, 136), (500, 3352, 264), (40, 4104, 64)])
+@pytest.mark.parametrize("pad", [0, 8])
+def test_product_pair(tokens, outs, ins, pad):
+    from mamba2 import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(tokens + outs)
+    dy, w, x = (torch.randn(r, c, generator=gen).bfloat16() for r, c in ((tokens, outs), (outs, ins), (tokens, ins)))
+
+    def stored(t):      # NaN behind the rows' ends
+        buf = torch.full((t.shape[0], t.shape[1] + pad), float("nan"), dtype=t.dtype)
+        buf[:, :t.shape[1]] = t
+        return buf.to(DEV)
+
+    dyd, wd, xd = stored(dy), stored(w), stored(x)
+    dx, dw = (torch.full((r, ins + pad), 7.0, dtype=torch.bfloat16, device=DEV) for r in (tokens, outs))
+    px = _lib.ProductParams(a=_lib.ptr(dyd), b=_lib.ptr(wd), out=_lib.ptr(dx), M=tokens, N=ins, K=outs, lda=outs + pad, ldb=ins + pad, ldo=ins + pad, a_k=1, b_k=0)
+    pw = _lib.ProductParams(a=_lib.ptr(dyd), b=_lib.ptr(xd), out=_lib.ptr(dw), M=outs, N=ins, K=tokens, lda=outs + pad, ldb=ins + pad, ldo=ins + pad, a_k=0, b_k=0)
+    n = lib.m2_product_pair_workspace_bytes(px, pw)
+    ws = torch.empty(max(n, 1), dtype=torch.uint8, device=DEV)
+    px.workspace, px.workspace_bytes = _lib.ptr(ws), n
+    _lib.check(lib.m2_product_pair(px, pw, _lib.stream_ptr()), "m2_product_pair")
+    for out, ref in ((dx, dy.double() @ w.double()), (dw, dy.double().T @ x.double())):
+        got = out.double().cpu()
+        assert ((got[:, :ins] - ref).norm() / ref.norm()).item() < 4e-3      # one rounding to bf16: 2^-9 at most per value
+        assert (got[:, ins:] == 7.0).all()
+    if n:
+        px.workspace_bytes = n - 1
+        with pytest.raises(RuntimeError, match="workspace too small"):
+            _lib.check(lib.m2_product_pair(px, pw, _lib.stream_ptr()), "m2_product_pair")
