@@ -437,15 +437,57 @@ conv_reduce_partials_kernel(const float* __restrict__ part, int64_t nslots, int6
 // ------------------------------------------------------------------------------------------
 // Channel-major path, k == 4: tokens contiguous in x, y (and dx).
 //
-// N tokens [t, t + N) of a row of l as fp32: one vector access where they all exist, zeros outside the row.
+// N tokens of a row: one vector access.  Where the row's last vector is cut by its end, the lanes that hold it read the row's last N
+// tokens instead and move the ones that are theirs down: no lane's branch stands in front of a load.  (With one, a row's first and last
+// lanes made their whole wave wait for one load after the other.)
+template <typename T, int N> using Tokens = T __attribute__((ext_vector_type(N)));
 template <typename T, int N>
-__device__ __forceinline__ void ld_tokens(const T* __restrict__ row, int64_t t, int64_t l, float (&out)[N]) {
-    if (t >= 0 && t + N <= l) {
-        ld_elems<T, N>(row + t, out);
+__device__ __forceinline__ Tokens<T, N> ld_whole(const T* __restrict__ p) {
+    using S = typename StreamVec<N * (int)sizeof(T)>::type;
+    return __builtin_bit_cast(Tokens<T, N>, *reinterpret_cast<const S*>(p));
+}
+// `v` without its first `gone` tokens (the same number for the whole launch), zeros behind the others, in the lanes that `cut` says.
+// By words and then by half of one: a 64-bit shift by a lane's amount gave wrong high words here where the compiler had put the amount
+// into a wave's last register.
+template <typename T, int N>
+__device__ __forceinline__ Tokens<T, N> move_down(const Tokens<T, N>& v, int gone, bool cut) {
+    if (gone <= 0) return v;
+    constexpr int W = N * (int)sizeof(T) / 4;
+    uint32_t old[W], w[W + 1];
+    __builtin_memcpy(old, &v, sizeof(v));
+    if (gone >= N) {
+#pragma unroll
+        for (int i = 0; i < W; ++i) w[i] = 0;
     } else {
 #pragma unroll
-        for (int i = 0; i < N; ++i) out[i] = (t + i >= 0 && t + i < l) ? to_f32(row[t + i]) : 0.f;
+        for (int i = 0; i < W; ++i) w[i] = old[i];
+        w[W] = 0;
+        const int words = gone * (int)sizeof(T) / 4;
+#pragma unroll
+        for (int by = W / 2; by > 0; by /= 2)
+            if (words & by) {
+#pragma unroll
+                for (int i = 0; i < W; ++i) w[i] = i + by < W ? w[i + by] : 0u;
+            }
+        if (sizeof(T) == 2 && (gone & 1)) {
+#pragma unroll
+            for (int i = 0; i < W; ++i) w[i] = (w[i] >> 16) | (w[i + 1] << 16);
+        }
     }
+    uint32_t o[W];
+#pragma unroll
+    for (int i = 0; i < W; ++i) o[i] = cut ? w[i] : old[i];
+    Tokens<T, N> r;
+    __builtin_memcpy(&r, o, sizeof(r));
+    return r;
+}
+// the same N tokens one by one, for rows shorter than a vector
+template <typename T, int N>
+__device__ __forceinline__ Tokens<T, N> ld_short(const T* __restrict__ row, int64_t t, int64_t l) {
+    Tokens<T, N> r;
+#pragma unroll
+    for (int i = 0; i < N; ++i) r[i] = (t + i >= 0 && t + i < l) ? row[t + i] : from_f32<T>(0.f);
+    return r;
 }
 template <typename T, int N>
 __device__ __forceinline__ void st_tokens(T* __restrict__ row, int64_t t, int64_t l, const float (&in)[N]) {
@@ -464,7 +506,8 @@ __device__ __forceinline__ void ld_row_taps(const void* __restrict__ w, const vo
 }
 
 // One thread per 16-byte piece of a row: its own tokens and the 4 before them (an L1 hit: the neighbour's own), eight
-// waves' worth of pieces per SIMD in flight.  HBM bound.
+// waves' worth of pieces per SIMD in flight.  HBM bound: b4 C5376 l2048 bf16 37.5 -> 30.5 us with both loads of a wave behind one another
+// (176 MB, 5.8 TB/s).
 template <typename T, typename WT, int ACT>
 __global__ void __launch_bounds__(256)
 conv_fwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias, T* __restrict__ y,
@@ -476,9 +519,23 @@ conv_fwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     const int64_t t0 = (int64_t)(idx - row * pieces) * V;
     const T* xr = x + b * xsb + c * xsc;
     float h[4], cur[V], wv[4], bv, o[V];
-    ld_tokens<T, V>(xr, t0, l, cur);
-    ld_tokens<T, 4>(xr, t0 - 4, l, h);
+    Tokens<T, 4> rh;
+    Tokens<T, V> rc;
     ld_row_taps<WT>(w, bias, c, wv, bv);
+    if (l >= V) {
+        const int gone = (int)((int64_t)pieces * V - l);      // what the row's last piece lacks
+        const bool cut = idx - row * pieces == pieces - 1;
+        rc = ld_whole<T, V>(xr + t0 - (cut ? gone : 0));
+        rh = ld_whole<T, 4>(xr + (t0 > 0 ? t0 - 4 : 0));
+        if (gone > 0 && __any(cut)) rc = move_down<T, V>(rc, gone, cut);
+    } else {
+        rc = ld_short<T, V>(xr, t0, l);
+        for (int i = 0; i < 4; ++i) rh[i] = (T)0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) h[i] = t0 > 0 ? to_f32(rh[i]) : 0.f;
+#pragma unroll
+    for (int i = 0; i < V; ++i) cur[i] = to_f32(rc[i]);
 #pragma unroll
     for (int i = 0; i < V; ++i) {
         float z = bv;
@@ -490,21 +547,26 @@ conv_fwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
 }
 
 // One wave per (channel, split): its lanes walk the channel's pieces of two vectors of tokens over all rows of the batch,
-// so the sums of dw and db stay in registers until the end.  The 1, 2 or 4 (`inner`) splits of a channel inside a workgroup meet in
-// LDS and finish it there; only with more of them (few channels) do fp32 partials go to conv_reduce_partials_kernel, whose launch
-// took 4.3 us beside the 70 of this kernel at b4 l2048 C5376 (two splits; forward and backward 125.0-126.1 -> 122.9-124.1 us in a stream of
-// them over eight sessions; with one split the chip is short of waves, 131 -> 141 in an eager loop).
+// so the sums of dw and db stay in registers until the end, and the next piece is on its way while this one is computed.  The 1, 2 or
+// 4 (`inner`) splits of a channel inside a workgroup meet in LDS and finish it there; only with more of them (a few channels) do fp32
+// partials go to conv_reduce_partials_kernel, whose launch is 4 us.  Where a channel has no more than 32 pieces, `lanes` of the wave (a
+// power of two) take it and the others the channels behind it.
 // A lane recomputes the three tokens behind its own for the dx lag: 3 in 16
 // (bf16) more activations, against a cross-lane exchange that would break at every row end.
+// What bounds it: the vector units (some 40 us of activations recomputed, at b4 C5376 l2048 bf16) beside 264 MB of traffic (44 us), in
+// waves of their own each waiting for its loads: 95 -> 69 us there without a lane's branch in front of the loads and with the next piece
+// under way (four waves a SIMD: 69, five, with spills: 77); 3 x 4097 rows of 1001 38 -> 27, 10240 rows of 77 19.7 -> 6.0.
 template <typename T, typename WT, int ACT>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 4)
 conv_bwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias, const T* __restrict__ dy,
                    T* __restrict__ dx, float* __restrict__ part, void* __restrict__ dw, void* __restrict__ db,
-                   int64_t l, uint32_t C, uint32_t inner, uint32_t outer, uint32_t pieces, uint32_t per_split, uint32_t total,
+                   int64_t l, uint32_t C, uint32_t lanes, uint32_t inner, uint32_t outer, uint32_t pieces, uint32_t per_split, uint32_t total,
                    int64_t xsb, int64_t xsc, int64_t gsb, int64_t gsc, int64_t dsb, int64_t dsc) {
     constexpr int V = VecTraits<T>::kVec, N = 2 * V;
+    constexpr int pd = std::is_same<WT, float>::value ? M2_F32 : M2_BF16;
     __shared__ float red[4][5];
-    const uint32_t wave = threadIdx.x >> 6, unit = (blockIdx.x * 4u + wave) / inner, sub = wave & (inner - 1);
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & (lanes - 1), sub = wave & (inner - 1);
+    const uint32_t unit = lanes < 64 ? (blockIdx.x * 256u + threadIdx.x) / lanes : (blockIdx.x * 4u + wave) / inner;
     const bool live = unit < C * outer;            // the last workgroup may have fewer channels
     const uint32_t part_row = live ? unit / C : 0, c = live ? unit - part_row * C : 0, split = part_row * inner + sub;
     const uint32_t end = !live ? 0 : (split + 1) * per_split < total ? (split + 1) * per_split : total;
@@ -512,25 +574,55 @@ conv_bwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     ld_row_taps<WT>(w, bias, c, wv, bv);
 #pragma unroll
     for (int k = 0; k < 5; ++k) acc[k] = 0.f;
-    for (uint32_t p = split * per_split + (threadIdx.x & 63); p < end; p += 64) {
+    struct Piece { Tokens<T, 4> xa, xd, gc; Tokens<T, V> xb, xc, ga, gb; };
+    auto load = [&](uint32_t p) {
         const uint32_t b = p / pieces;
         const int64_t t0 = (int64_t)(p - b * pieces) * N;
         const T* xr = x + b * xsb + c * xsc;
         const T* gr = dy + b * gsb + c * gsc;
+        Piece q;
+        if (l >= V) {
+            // what the row's last piece lacks of its two vectors, and the piece before it of the four tokens behind it
+            const int lacks = (int)((int64_t)pieces * N - l);
+            const bool last = t0 + N >= l, near = t0 + N + 4 > l;
+            const int64_t tb = t0 + V > l ? l - V : t0, tc = t0 + N > l ? l - V : t0 + V, td = near ? l - 4 : t0 + N;
+            q.xb = ld_whole<T, V>(xr + tb); q.ga = ld_whole<T, V>(gr + tb); q.xc = ld_whole<T, V>(xr + tc); q.gb = ld_whole<T, V>(gr + tc);
+            q.xa = ld_whole<T, 4>(xr + (t0 > 0 ? t0 - 4 : 0)); q.xd = ld_whole<T, 4>(xr + td); q.gc = ld_whole<T, 4>(gr + td);
+            if (lacks > 0 && __any(near)) {
+                q.xb = move_down<T, V>(q.xb, lacks - V, last); q.ga = move_down<T, V>(q.ga, lacks - V, last);
+                q.xc = move_down<T, V>(q.xc, lacks, last); q.gb = move_down<T, V>(q.gb, lacks, last);
+                q.xd = move_down<T, 4>(q.xd, lacks - (N - 4), near); q.gc = move_down<T, 4>(q.gc, lacks - (N - 4), near);
+            }
+        } else {
+            q.xb = ld_short<T, V>(xr, t0, l); q.ga = ld_short<T, V>(gr, t0, l);
+            q.xc = q.gb = (T)0.f;
+            q.xa = q.xd = q.gc = (T)0.f;
+        }
+        return q;
+    };
+    Piece next{};
+    uint32_t p = split * per_split + lane;
+    if (p < end) next = load(p);
+    for (; p < end; p += lanes) {
+        const Piece q = next;
+        if (p + lanes < end) next = load(p + lanes);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t b = p / pieces;
+        const int64_t t0 = (int64_t)(p - b * pieces) * N;
+        const bool more = t0 + N < l;
         T* dr = dx + b * dsb + c * dsc;
-        float xa[4], xb[V], xc[V], xd[4], ga[V], gb[V], gc[4];
-        ld_tokens<T, V>(xr, t0, l, xb);
-        ld_tokens<T, V>(gr, t0, l, ga);
-        ld_tokens<T, V>(xr, t0 + V, l, xc);
-        ld_tokens<T, V>(gr, t0 + V, l, gb);
-        ld_tokens<T, 4>(xr, t0 - 4, l, xa);
-        ld_tokens<T, 4>(xr, t0 + N, l, xd);
-        ld_tokens<T, 4>(gr, t0 + N, l, gc);
         float xw[N + 8], g[N + 4];                 // x[t0 - 4 ...], dy -> g = dy * act'(z) from t0 on
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { xw[i] = xa[i]; xw[4 + N + i] = xd[i]; g[N + i] = gc[i]; }
+        for (int i = 0; i < 4; ++i) {
+            xw[i] = t0 > 0 ? to_f32(q.xa[i]) : 0.f;
+            xw[4 + N + i] = more ? to_f32(q.xd[i]) : 0.f;
+            g[N + i] = more ? to_f32(q.gc[i]) : 0.f;
+        }
 #pragma unroll
-        for (int i = 0; i < V; ++i) { xw[4 + i] = xb[i]; xw[4 + V + i] = xc[i]; g[i] = ga[i]; g[V + i] = gb[i]; }
+        for (int i = 0; i < V; ++i) {
+            xw[4 + i] = to_f32(q.xb[i]); xw[4 + V + i] = to_f32(q.xc[i]);
+            g[i] = to_f32(q.ga[i]); g[V + i] = to_f32(q.gb[i]);
+        }
 #pragma unroll
         for (int i = 0; i < N + 3; ++i) {
             const float z = bv + wv[0] * xw[i + 1] + wv[1] * xw[i + 2] + wv[2] * xw[i + 3] + wv[3] * xw[i + 4];
@@ -551,14 +643,30 @@ conv_bwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
         if (t0 + V < l) st_tokens<T, V>(dr, t0 + V, l, ob);
     }
 #pragma unroll
-    for (int k = 0; k < 5; ++k) acc[k] = warp_sum(acc[k]);
+    for (int k = 0; k < 5; ++k) {
+        float v = acc[k];
+        if (lanes > 1) v = lane_xor_add<1>(v);
+        if (lanes > 2) v = lane_xor_add<2>(v);
+        if (lanes > 4) v = lane_xor_add<4>(v);
+        if (lanes > 8) v = lane_xor_add<8>(v);
+        if (lanes > 16) v = lane_xor_add<16>(v);
+        if (lanes > 32) v = lane_xor_add<32>(v);
+        acc[k] = v;
+    }
+    if (lanes < 64) {                              // a channel's only lanes
+        if (live && lane == 0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) st_param(dw, pd, (int64_t)c * 4 + k, acc[k]);
+            if (db) st_param(db, pd, c, acc[4]);
+        }
+        return;
+    }
     if ((threadIdx.x & 63) == 0) {
 #pragma unroll
         for (int k = 0; k < 5; ++k) red[wave][k] = acc[k];
     }
     __syncthreads();
     if (const uint32_t k = threadIdx.x & 63; live && sub == 0 && k < 5) {
-        constexpr int pd = std::is_same<WT, float>::value ? M2_F32 : M2_BF16;
         float v = 0.f;
         for (uint32_t q = 0; q < inner; ++q) v += red[wave + q][k];
         if (outer > 1) part[((int64_t)part_row * C + c) * 5 + k] = v;
@@ -791,18 +899,21 @@ int launch_bwd(const m2_conv1d_params* p, int64_t* slots, hipStream_t st) {
     }
     if (channel_major_ok(p, true)) {
         const int64_t pieces = ceil_div(l, (int64_t)(2 * VecTraits<T>::kVec)), total = nb * pieces;
-        // enough waves to fill the chip (about 24 per CU), each with at least one whole round of its lanes; never more
-        // partial rows than m2_conv1d_bwd_workspace_bytes sizes
-        int64_t splits = ceil_div((int64_t)24 * device_cus(), C);
-        if (splits > total / 64) splits = total / 64;
-        if (splits < 1) splits = 1;
-        const int64_t inner = splits > 2 ? 4 : splits, outer = ceil_div(splits, inner), per_split = ceil_div(total, inner * outer);
+        int64_t lanes = 64;
+        while (lanes > 1 && lanes / 2 >= total) lanes /= 2;
+        const int64_t rounds = ceil_div(total, lanes);
+        // four splits of a channel where its workgroup's four waves have a round each; more, through partials, while the chip has not
+        // eight waves a CU and the splits that come of it have two rounds at least (one, two, four, eight of them: b4 l2048 C5376
+        // 83 / 77 / 69 / 72 us, C256 12.1 / 7.8 / 6.0 / 8.1; b16 l8192 C128 four, eight, sixteen: 53 / 47 / 35)
+        int64_t splits = rounds >= 4 ? 4 : rounds >= 2 ? 2 : 1;
+        while (C * splits < 8 * device_cus() && rounds >= 4 * splits) splits *= 2;
+        const int64_t inner = splits > 4 ? 4 : splits, outer = splits / inner, per_split = ceil_div(rounds, inner * outer) * lanes;
         float* part = static_cast<float*>(p->workspace);
         M2_REQUIRE(outer == 1 || (part && p->workspace_bytes >= (size_t)(outer * C * 5) * sizeof(float)), M2_ERR_WORKSPACE,
                    "conv1d_bwd: workspace %zu bytes < %zu needed", p->workspace_bytes, (size_t)(outer * C * 5) * sizeof(float));
         conv_dispatch(p, [&](auto wt, auto act) {
-            conv_bwd_cm_kernel<T, decltype(wt), decltype(act)::value><<<(unsigned)ceil_div(C * outer * inner, (int64_t)4), 256, 0, st>>>(
-                x, p->w, p->bias, dy, dx, part, p->dw, p->db, l, (uint32_t)C, (uint32_t)inner, (uint32_t)outer, (uint32_t)pieces, (uint32_t)per_split,
+            conv_bwd_cm_kernel<T, decltype(wt), decltype(act)::value><<<(unsigned)(lanes < 64 ? ceil_div(C * lanes, (int64_t)256) : ceil_div(C * outer * inner, (int64_t)4)), 256, 0, st>>>(
+                x, p->w, p->bias, dy, dx, part, p->dw, p->db, l, (uint32_t)C, (uint32_t)lanes, (uint32_t)inner, (uint32_t)outer, (uint32_t)pieces, (uint32_t)per_split,
                 (uint32_t)total, p->x_stride_b, p->x_stride_c, p->y_stride_b, p->y_stride_c, p->dx_stride_b, p->dx_stride_c);
         });
         int rc = check_launch("conv1d_bwd");

@@ -110,3 +110,11 @@ def test_conv_segment_lengths(b, l, C):
 @pytest.mark.parametrize("b,l,C,act", [(1, 2048, 3075, "silu"), (2, 2050, 2049, None), (2, 4100, 1023, "silu")])
 def test_conv_channel_major_splits(dtype, b, l, C, act):
     test_conv_layout_edges(dtype, False, b, l, C, act)
+
+
+# channel-major: every way a row can end inside its last pieces, several channels to a wave and (few channels, long rows) partial rows of sums
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,l,C", [(2, l, 37) for l in (2, 4, 7, 8, 9, 10, 11, 12, 13, 15, 18, 19, 20, 22, 24, 27, 29, 31, 34)] +
+                         [(3, 160, 70), (9, 115, 65), (2, 5001, 9), (9, 8190, 3)])
+def test_conv_channel_major_row_ends(dtype, b, l, C):
+    test_conv_layout_edges(dtype, False, b, l, C, "silu")
