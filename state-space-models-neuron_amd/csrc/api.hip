@@ -28,7 +28,7 @@ int check_launch(const char* what) {
 
 namespace {
 
-// C[M][N] = A[M][K] * Bt[N][K]^T through stage_rows + wave_mma; block = one 128x128 tile, 256 threads.
+// C[M][N] = A[M][K] * Bt[N][K]^T through StagedRows + wave_mma; block = one 128x128 tile, 256 threads.
 template <typename T>
 __global__ void __launch_bounds__(256)
 mfma_selftest_kernel(const T* __restrict__ A, const T* __restrict__ Bt, float* __restrict__ C, int64_t N, int64_t K) {
@@ -42,8 +42,11 @@ mfma_selftest_kernel(const T* __restrict__ A, const T* __restrict__ Bt, float* _
     floatx16 acc[2][2];
     acc_zero(acc);
     for (int64_t k0 = 0; k0 < K; k0 += KB) {
-        stage_rows<T, 128, KB, 256, false>(sA, LD, A + m0 * K + k0, K, 128, nullptr, tid);
-        stage_rows<T, 128, KB, 256, false>(sB, LD, Bt + n0 * K + k0, K, 128, nullptr, tid);
+        StagedRows<T, 128, KB, 256> ra, rb;
+        ra.load(A + m0 * K + k0, K, 128, tid);
+        rb.load(Bt + n0 * K + k0, K, 128, tid);
+        ra.put(sA, LD, 128, tid);
+        rb.put(sB, LD, 128, tid);
         __syncthreads();
         wave_mma<2, 2>(acc, sA + wm * 64 * LD, LD, sB + wn * 64 * LD, LD, 0, KB);
         __syncthreads();

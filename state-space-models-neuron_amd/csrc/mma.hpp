@@ -150,43 +150,30 @@ __device__ __forceinline__ void wave_mma(floatx16 (&acc)[BM][BN], const T* __res
 // ------------------------------------------------------------------------------------------
 // Cooperative staging, global -> LDS.  NT threads; `tid` in [0, NT).
 //
-// stage_rows: global tile [ROWS][COLS] (COLS contiguous, row stride gstride) -> LDS [ROWS][ld].
-// Rows >= valid are zero-filled.  If SCALE, row r is multiplied by rowscale[r] (fp32) first.
-template <typename T, int ROWS, int COLS, int NT, bool SCALE>
-__device__ __forceinline__ void stage_rows(T* __restrict__ s, int ld, const T* __restrict__ g, int64_t gstride,
-                                           int valid, const float* __restrict__ rowscale, int tid) {
-    constexpr int V = VecTraits<T>::kVec;
-    constexpr int VPR = COLS / V;
-    constexpr int TOTAL = ROWS * VPR;
-    static_assert(COLS % V == 0, "tile width must be a multiple of the vector width");
-    if (!SCALE) {
-        // plain copy: 16 bytes stay 16 bytes, no conversion
-#pragma unroll 4
-        for (int e = tid; e < TOTAL; e += NT) {
-            const int r = e / VPR, cv = e % VPR;
-            uint4 raw = uint4{0u, 0u, 0u, 0u};
-            if (r < valid) raw = *reinterpret_cast<const uint4*>(g + (int64_t)r * gstride + cv * V);
-            *reinterpret_cast<uint4*>(s + r * ld + cv * V) = raw;
-        }
-        return;
-    }
-#pragma unroll 4
-    for (int e = tid; e < TOTAL; e += NT) {
-        const int r = e / VPR, cv = e % VPR;
-        float v[V];
-        if (r < valid) load16(g + (int64_t)r * gstride + cv * V, v);
-        else {
+// StagedRows: global tile [ROWS][COLS] (COLS contiguous, row stride gstride) -> LDS [ROWS][ld], rows >= valid zero-filled: load() and
+// put(), so that the loads of several tiles are under way together.  Rows past the end read the last one there is (valid may be
+// negative: that row then lies in front of the tile), so that no branch stands in front of a load: with one, each of a thread's eight
+// loads of two tiles waited for the one before it.
+template <typename T, int ROWS, int COLS, int NT>
+struct StagedRows {
+    static constexpr int V = VecTraits<T>::kVec, VPR = COLS / V, PER = ROWS * VPR / NT;
+    static_assert(COLS % V == 0 && ROWS * VPR % NT == 0, "whole vectors, the same many per thread");
+    uint4 raw[PER];
+    __device__ __forceinline__ void load(const T* __restrict__ g, int64_t gstride, int valid, int tid) {
 #pragma unroll
-            for (int i = 0; i < V; ++i) v[i] = 0.f;
+        for (int i = 0; i < PER; ++i) {
+            const int e = i * NT + tid, r = e / VPR, cv = e % VPR;
+            raw[i] = *reinterpret_cast<const uint4*>(g + (int64_t)(r < valid ? r : valid - 1) * gstride + cv * V);
         }
-        if (SCALE) {
-            const float sc = rowscale[r];
-#pragma unroll
-            for (int i = 0; i < V; ++i) v[i] *= sc;
-        }
-        store16(s + r * ld + cv * V, v);
     }
-}
+    __device__ __forceinline__ void put(T* __restrict__ s, int ld, int valid, int tid) const {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int e = i * NT + tid, r = e / VPR, cv = e % VPR;
+            *reinterpret_cast<uint4*>(s + r * ld + cv * V) = r < valid ? raw[i] : uint4{0u, 0u, 0u, 0u};
+        }
+    }
+};
 
 // Sum of v over the 32 lanes that share (lane >> 5), for 16 values at once (the 16 accumulator rows of a lane),
 // by a butterfly reduce-scatter: 16 cross-lane moves instead of 80 (the widest step selects and adds with one row swap, the

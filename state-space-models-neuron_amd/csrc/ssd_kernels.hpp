@@ -96,8 +96,11 @@ cb_body(const T* __restrict__ Bm, const T* __restrict__ Cm, float* __restrict__ 
         T* sBt = sC + 32 * LDT;
         T* Btp = Bt + grp * (int64_t)(N * kQ);
         T* Ctp = Ct ? Ct + grp * (int64_t)(N * kQ) : nullptr;
-        if (Ct) stage_rows<T, 32, N, 256, false>(sC, LDT, Cp + (int64_t)tk0 * Csl, Csl, valid - tk0, nullptr, tid);
-        stage_rows<T, 32, N, 256, false>(sBt, LDT, Bp + (int64_t)tk0 * Bsl, Bsl, valid - tk0, nullptr, tid);
+        StagedRows<T, 32, N, 256> rc, rb;
+        rb.load(Bp + (int64_t)tk0 * Bsl, Bsl, valid - tk0, tid);
+        if (Ct) rc.load(Cp + (int64_t)tk0 * Csl, Csl, valid - tk0, tid);
+        rb.put(sBt, LDT, valid - tk0, tid);
+        if (Ct) rc.put(sC, LDT, valid - tk0, tid);
         __syncthreads();
         for (int e = tid; e < N * (32 / V); e += 256) {
             const int n = e % N, s0 = (e / N) * V;
@@ -122,8 +125,11 @@ cb_body(const T* __restrict__ Bm, const T* __restrict__ Cm, float* __restrict__ 
 #pragma unroll
     for (int n0 = 0; n0 < N; n0 += KH) {
         if (n0) __syncthreads();
-        stage_rows<T, 64, KH, 256, false>(sC, LD, Cp + (int64_t)(wm * 64) * Csl + n0, Csl, valid - wm * 64, nullptr, tid);
-        stage_rows<T, 64, KH, 256, false>(sB, LD, Bp + (int64_t)(wn * 64) * Bsl + n0, Bsl, valid - wn * 64, nullptr, tid);
+        StagedRows<T, 64, KH, 256> rc, rb;
+        rc.load(Cp + (int64_t)(wm * 64) * Csl + n0, Csl, valid - wm * 64, tid);
+        rb.load(Bp + (int64_t)(wn * 64) * Bsl + n0, Bsl, valid - wn * 64, tid);
+        rc.put(sC, LD, valid - wm * 64, tid);
+        rb.put(sB, LD, valid - wn * 64, tid);
         __syncthreads();
         if (live) wave_mma<1, 1>(acc, sC + wi * 32 * LD, LD, sB + wj * 32 * LD, LD, 0, KH);
     }
@@ -151,7 +157,9 @@ cb_body(const T* __restrict__ Bm, const T* __restrict__ Cm, float* __restrict__ 
             if (Gmt) {
                 floatx4 v;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = i0 + k + e >= j0 + r ? blk[(k + e) * LDG + r] : 0.f;
+                for (int e = 0; e < 4; ++e) v[e] = blk[(k + e) * LDG + r];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = i0 + k + e >= j0 + r ? v[e] : 0.f;
                 *reinterpret_cast<floatx4*>(Gmt + grp * (int64_t)(kQ * kQ) + op32_offset<16>(J, 4 * I + it, lane)) = v;
             }
         }
@@ -169,9 +177,12 @@ cb_body(const T* __restrict__ Bm, const T* __restrict__ Cm, float* __restrict__ 
             *reinterpret_cast<RawVec<T, 4>*>(Gm + grp * (int64_t)(kQ * kQ) + (i0 + a) * kQ + j0 + k0) = *reinterpret_cast<const RawVec<T, 4>*>(o);
         }
         if (Gmt) {
+            float t[4];
             T o[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = from_f32<T>(i0 + k0 + e >= j0 + a ? blk[(k0 + e) * LDG + a] : 0.f);
+            for (int e = 0; e < 4; ++e) t[e] = blk[(k0 + e) * LDG + a];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = from_f32<T>(i0 + k0 + e >= j0 + a ? t[e] : 0.f);
             *reinterpret_cast<RawVec<T, 4>*>(Gmt + grp * (int64_t)(kQ * kQ) + (j0 + a) * kQ + i0 + k0) = *reinterpret_cast<const RawVec<T, 4>*>(o);
         }
     }
