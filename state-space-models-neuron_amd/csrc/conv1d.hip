@@ -126,6 +126,14 @@ __device__ __forceinline__ void ld_elems(const T* __restrict__ p, float (&out)[V
     for (int i = 0; i < V; ++i) out[i] = to_f32(e[i]);
 }
 
+// N neighbouring elements, as they lie
+template <typename T, int N> using Tokens = T __attribute__((ext_vector_type(N)));
+template <typename T, int N>
+__device__ __forceinline__ Tokens<T, N> ld_whole(const T* __restrict__ p) {
+    using S = typename StreamVec<N * (int)sizeof(T)>::type;
+    return __builtin_bit_cast(Tokens<T, N>, *reinterpret_cast<const S*>(p));
+}
+
 __device__ __forceinline__ float ld_param(const void* p, int pd, int64_t i) {
     return pd == M2_F32 ? reinterpret_cast<const float*>(p)[i] : to_f32(reinterpret_cast<const bf16_t*>(p)[i]);
 }
@@ -183,10 +191,24 @@ conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     if (cv * V >= C || t0 >= l) return;
     const int64_t c0 = cv * V < C - V ? cv * V : C - V;     // the last vector ends with the row (it may repeat channels: same values)
 
-    float wv[4][V], bv[V];
-    load_taps<WT, V>(w, bias, c0, wv, bv);
     const T* xp = x + b * xsb + c0;
     T* yp = y + b * ysb + c0;
+    // A cache of four columns (the usual one): a channel's are one vector, the first segment's thread asks for its channels' and for the
+    // sequence's last four inputs ahead of everything, and the columns leave in one store each (read, sorted and stored one by one
+    // behind the segment they kept its workgroups 2 to 3 us longer than the others)
+    const bool quick = PREFILL && (flags & kTail) && W == 4 && l >= 4 && t0 == 0;
+    RawVec<T, V> last[4];
+    Tokens<T, 4> was[V];
+    if (quick) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) last[q] = ld_stream<T, V>(xp + (l - 4 + q) * xsl);
+        if (flags & kContinuing) {
+#pragma unroll
+            for (int j = 0; j < V; ++j) was[j] = ld_whole<T, 4>(state + (b * C + c0 + j) * 4);
+        }
+    }
+    float wv[4][V], bv[V];
+    load_taps<WT, V>(w, bias, c0, wv, bv);
     float h0[V], h1[V], h2[V];   // x[t-3], x[t-2], x[t-1]
 #pragma unroll
     for (int j = 0; j < V; ++j) h0[j] = h1[j] = h2[j] = 0.f;
@@ -196,15 +218,30 @@ conv_fwd_cl_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     if (PREFILL && (flags & kContinuing) && t0 == 0) {
         // the inputs in front of the sequence come out of the decode cache (three short reads per channel in the first
         // segment only; putting cache and sequence behind one another in memory first took 35 us of 145 at b8 l333 C5376)
+        if (quick) {
+#pragma unroll
+            for (int j = 0; j < V; ++j) { h0[j] = to_f32(was[j][1]); h1[j] = to_f32(was[j][2]); h2[j] = to_f32(was[j][3]); }
+        } else {
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                const T* hp = state + (b * C + c0 + j) * W + (W - 3);
+                h0[j] = to_f32(hp[0]); h1[j] = to_f32(hp[1]); h2[j] = to_f32(hp[2]);
+            }
+        }
+    }
+    if (quick) {      // (what was there has been read above)
+        T* sp = state + (b * C + c0) * 4;
 #pragma unroll
         for (int j = 0; j < V; ++j) {
-            const T* hp = state + (b * C + c0 + j) * W + (W - 3);
-            h0[j] = to_f32(hp[0]); h1[j] = to_f32(hp[1]); h2[j] = to_f32(hp[2]);
+            Tokens<T, 4> v;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = reinterpret_cast<const T*>(&last[q])[j];
+            *reinterpret_cast<typename StreamVec<4 * (int)sizeof(T)>::type*>(sp + j * 4) = __builtin_bit_cast(typename StreamVec<4 * (int)sizeof(T)>::type, v);
         }
     }
     // the last W inputs, four columns at a time; where the sequence is shorter, what is left of the cache (or zeros) moves up
     auto leave_tail = [&] {
-        if (!PREFILL || !(flags & kTail) || t0 != 0) return;
+        if (!PREFILL || !(flags & kTail) || t0 != 0 || quick) return;
         T* sp = state + (b * C + c0) * W;
         for (int w0 = 0; w0 < W; w0 += 4) {
             T v[4][V];
@@ -440,12 +477,6 @@ conv_reduce_partials_kernel(const float* __restrict__ part, int64_t nslots, int6
 // N tokens of a row: one vector access.  Where the row's last vector is cut by its end, the lanes that hold it read the row's last N
 // tokens instead and move the ones that are theirs down: no lane's branch stands in front of a load.  (With one, a row's first and last
 // lanes made their whole wave wait for one load after the other.)
-template <typename T, int N> using Tokens = T __attribute__((ext_vector_type(N)));
-template <typename T, int N>
-__device__ __forceinline__ Tokens<T, N> ld_whole(const T* __restrict__ p) {
-    using S = typename StreamVec<N * (int)sizeof(T)>::type;
-    return __builtin_bit_cast(Tokens<T, N>, *reinterpret_cast<const S*>(p));
-}
 // `v` without its first `gone` tokens (the same number for the whole launch), zeros behind the others, in the lanes that `cut` says.
 // By words and then by half of one: a 64-bit shift by a lane's amount gave wrong high words here where the compiler had put the amount
 // into a wave's last register.
