@@ -304,29 +304,6 @@ rmsnorm_gated_kernel(const NormArgs a) {
     }
 }
 
-// rows per workgroup: about 512 workgroups in all for the backward (each leaves a partial row of dw), about 2048 for
-// the forward, at least 4 rows each
-int64_t norm_rows_per_block(int64_t rows, int64_t groups, bool bwd) {
-    int64_t rb = rows * groups / (bwd ? 512 : 1024);
-    if (rb < 4) rb = 4;
-    return (rb + 3) / 4 * 4;
-}
-// The backward with a whole workgroup per (row, group): one workgroup per compute unit as well (it is alone there by its
-// register count anyway; 256 workgroups 77 us, 512 -> 80, 768 -> 95 at 8192 rows of 5120 channels).
-int64_t norm_rows_per_block_bwd(int64_t rows, int64_t groups, int64_t nvec) {
-    if (nvec > 256 && rows * groups >= 4096) return ceil_div(rows * groups, device_cus());
-    return norm_rows_per_block(rows, groups, true);
-}
-// The forward with a whole workgroup per (row, group): few rows (a decode step) are spread one per workgroup; many rows go
-// to exactly ONE workgroup per compute unit (measured at 8192 rows of 5120 channels, rows dealt round-robin: 256 workgroups
-// 46 us, 192 -> 55, 320 -> 57, 512 -> 52, 1024 -> 54: more resident waves only disturb the three streams).
-int64_t norm_rows_per_block_fwd(int64_t rows, int64_t groups, int64_t nvec) {
-    if (nvec > 256) {
-        if (rows * groups < 4096) return 1;
-        return ceil_div(rows * groups, device_cus());
-    }
-    return norm_rows_per_block(rows, groups, false);
-}
 // waves per (row, group) and vectors per lane for a group of `nvec` 16-byte vectors; false if it does not fit
 bool norm_shape(int64_t nvec, int vec_elems, int* wpg, int* nv) {
     if (nvec <= 0) return false;
@@ -336,6 +313,45 @@ bool norm_shape(int64_t nvec, int vec_elems, int* wpg, int* nv) {
     // up to 8192 channels per group in either type: 4 vectors of 8 per lane (16-bit), 8 vectors of 4 (fp32)
     if (nvec * vec_elems <= 8192) { *wpg = 4; *nv = (int)((nvec + 255) / 256); return true; }
     return false;
+}
+
+// What a workspace has room for: a backward of about 512 workgroups of at least 4 rows each.
+int64_t norm_rows_per_block(int64_t rows, int64_t groups) {
+    int64_t rb = rows * groups / 512;
+    if (rb < 4) rb = 4;
+    return (rb + 3) / 4 * 4;
+}
+// Rows per workgroup.  A workgroup (or, with a wave per row, each of its four waves) is a chain of rows, dealt round-robin, and the chip
+// likes one or two of them per CU: with a few more (834 of four rows for 3333) a second round is nearly empty, and in the backward every
+// one leaves a partial row of dw.  Workgroups per CU, from 180 sizes (300 to 26000 rows, groups of 512 to 7168 channels, both types;
+// time with one | two | three | four per CU, us, forward and backward):
+//   a wave per row, more than two vectors a lane: one.  3333 x 2048 8.8 | 8.7 | 8.7 | 9.8 and 19.5 | 20.9 | 21.0 | 26.0, 8192 x 2048
+//     18.4 | 19.1 | 20.6 | 20.5 and 34.4 | 37.1 | 39.5 | 41.3
+//   two vectors: two forward, one backward, two for many rows of one group.  8192 x 8 x 1024 79.6 | 80.3 | 82.5 | 83.6 and 128 | 140 |
+//     144 | 143; 16384 x 1024 20.5 | 18.2 | 19.0 | 19.3 and 33.5 | 33.2 | 36.1 | 36.4
+//   one vector: four forward, two backward, one for few rows.  8192 x 8 x 512 52.3 | 35.0 | 32.7 | 33.4 and 82 | 67 | 70 | 69
+//   a workgroup per row: one, but forward, of 16-bit rows of two vectors a lane, two up to 9000 rows, and a row each up to 1100.
+//     2664 x 5120 17.8 | 16.5 | 17.0 | 18.3 and 32.0 | 36.4 | 38.1 | 38.9, 16384 x 5120 90 | 96 | 100 | 101 and 162 | 173 | 174 | 178,
+//     2664 x 7168 24.1 | 25.5 | 28.3 | 30.8; rows that leave lanes idle (2560, 3072) want two for longer: 8192 x 3072 36.8 | 29.8 | 30.1
+//     | 29.5, backward 51.7 | 48.0 | 58.5 | 52.9
+int64_t norm_rows_per_workgroup(int64_t rows, int64_t groups, int64_t nvec, int vec_elems, bool bwd) {
+    int wpg = 1, nv = 1;
+    if (!norm_shape(nvec, vec_elems, &wpg, &nv)) return norm_rows_per_block(rows, groups);
+    const int64_t all = rows * groups;
+    const bool exact = (int64_t)wpg * 64 * nv == nvec;
+    int64_t per_cu = 1;
+    if (wpg == 1) {
+        if (nv == 2) per_cu = bwd ? (groups == 1 && rows > 7000 ? 2 : 1) : 2;
+        if (nv == 1) per_cu = bwd ? (all > 5000 ? 2 : 1) : 4;
+        const int64_t rb = ceil_div(all, per_cu * device_cus());
+        return rb < 4 ? 4 : (rb + 3) / 4 * 4;
+    }
+    if (nv == 2 && bwd && !exact && all >= 3000 && all <= 12000) per_cu = 2;
+    if (nv == 2 && !bwd) {
+        if (all <= 1100 && exact) return 1;
+        if (all > 1100 && (!exact || (vec_elems == 8 && all <= 9000))) per_cu = 2;
+    }
+    return ceil_div(all, per_cu * device_cus());
 }
 
 template <typename T, bool BWD>
@@ -539,7 +555,7 @@ extern "C" int m2_rmsnorm_gated_fwd(const m2_rmsnorm_params* p, void* stream) {
     a.x = p->x; a.x_sr = p->x_stride_row; a.z = p->z; a.z_sr = p->z_stride_row; a.w = p->weight;
     a.out = p->out; a.out_sr = p->out_stride_row; a.out_f32 = p->out_f32 || p->dtype == M2_F32;
     a.rows = p->rows; a.d = p->channels; a.gw = p->channels / p->n_groups; a.eps = p->eps;
-    a.rows_per_block = norm_rows_per_block_fwd(p->rows, p->n_groups, a.gw / V);
+    a.rows_per_block = norm_rows_per_workgroup(p->rows, p->n_groups, a.gw / V, V, false);
     hipStream_t st = static_cast<hipStream_t>(stream);
     M2_DISPATCH_DTYPE(p->dtype, T, return (launch_norm<T, false>(a, p->n_groups, st)));
     return M2_OK;
@@ -550,9 +566,9 @@ extern "C" size_t m2_rmsnorm_gated_bwd_workspace_bytes(int64_t rows, int64_t cha
     // A partial row per workgroup.  Where one workgroup per compute unit runs, room for the general rule's count (about 512) is
     // asked for all the same: a size that followed the units would depend on the device that is current when it is asked for, and
     // a caller may size its scratch without one.
-    const int64_t nvec = channels / n_groups / (dtype == M2_F32 ? 4 : 8);
-    const int64_t used = m2::ceil_div(rows, m2::norm_rows_per_block_bwd(rows, n_groups, nvec));
-    const int64_t most = m2::ceil_div(rows, m2::norm_rows_per_block(rows, n_groups, true));
+    const int V = dtype == M2_F32 ? 4 : 8;
+    const int64_t used = m2::ceil_div(rows, m2::norm_rows_per_workgroup(rows, n_groups, channels / n_groups / V, V, true));
+    const int64_t most = m2::ceil_div(rows, m2::norm_rows_per_block(rows, n_groups));
     return m2::align_up((size_t)(used > most ? used : most) * (size_t)channels * sizeof(float), 256);
 }
 
@@ -580,7 +596,7 @@ extern "C" int m2_rmsnorm_gated_bwd_partial(const m2_rmsnorm_params* p, int64_t*
         a.g = p->d_out; a.g_sr = p->d_out_stride_row; a.dx = p->dx; a.dx_sr = p->dx_stride_row; a.dz = p->dz; a.dz_sr = p->dz_stride_row;
         a.partial = static_cast<float*>(p->workspace);
         a.rows = p->rows; a.d = p->channels; a.gw = p->channels / p->n_groups; a.eps = p->eps;
-        a.rows_per_block = norm_rows_per_block_bwd(p->rows, p->n_groups, a.gw / V);
+        a.rows_per_block = norm_rows_per_workgroup(p->rows, p->n_groups, a.gw / V, V, true);
         int wpg = 0, nv = 0;
         if (!norm_shape(a.gw / V, V, &wpg, &nv))
             return fail(M2_ERR_SHAPE, "rmsnorm_gated_bwd: %lld channels per group exceed the supported 8192", (long long)a.gw);

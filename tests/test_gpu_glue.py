@@ -220,3 +220,11 @@ def test_mixer_params_and_their_gradients(heads, channels, with_D, types):
                                          code(types[1]), ptr(got[2]), code(types[2]), ptr(got[3]), code(types[3]), heads, channels, _lib.stream_ptr()), "mixer_params_grads")
     for name, a, want in zip(("A_log", "D", "dt_bias", "norm"), got, (A * dA, dD, db, dn)):
         assert torch.equal(a, want.to(a.dtype)) if name != "D" or with_D else (a == 7).all(), name
+
+
+# rows per workgroup: one, two and four workgroups per CU, one row each, a last workgroup (or its last waves) with fewer rows or none
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,d,g", [(1029, 2048, 1), (7003, 1024, 1), (301, 8192, 8), (5001, 512, 1), (641, 4096, 8), (1100, 4096, 1), (1101, 5120, 1), (3001, 2560, 1),
+                                      (515, 7168, 1)])
+def test_rmsnorm_gated_rows_per_workgroup(dtype, rows, d, g):
+    test_rmsnorm_gated_fwd_bwd(dtype, (1, rows), d, g, True)
