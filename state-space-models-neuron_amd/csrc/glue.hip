@@ -8,8 +8,8 @@
 //              backward (fused_kernel.py:159-171):  var = mean(h^2) + eps, r = rsqrt(var), gw = g w,
 //              cf = mean(h gw) / var,  d_h = r (gw - cf h),  dx = d_h silu(z),  dz = d_h x silu'(z),  dw = sum_rows g h r
 //
-// A (row, group) is handled by one wave (groups of up to 2048 channels) or by the four or five waves of a workgroup (up
-// to 8192), its channels in registers as 16-byte vectors; a workgroup takes many rows, so the per-channel weight
+// A (row, group) is handled by a part of a wave (several groups of up to 32 vectors), by one wave (groups of up to 2048
+// channels) or by the four or five waves of a workgroup (up to 8192), its channels in registers as 16-byte vectors; a workgroup takes many rows, so the per-channel weight
 // and -- in the backward -- the dw accumulators stay in registers across rows.  dw and d_bias leave as per-block
 // partials in a caller-owned workspace and are summed in a fixed order by a second small kernel (no atomics).
 #include <initializer_list>
@@ -119,9 +119,17 @@ __device__ __forceinline__ void store_vec(T* p, const float (&v)[GlueVec<T>::V])
 
 // sum over the WPG waves that share a (row, group); `slot` alternates between two LDS rows so that one barrier per
 // reduction is enough
-template <int WPG>
+template <int LPG>
+__device__ __forceinline__ float lanes_sum(float v) {      // over runs of LPG lanes
+    if constexpr (LPG == 64) return warp_sum(v);
+    if constexpr (LPG >= 32) v = lane_xor_add<16>(v);
+    if constexpr (LPG >= 16) v = lane_xor_add<8>(v);
+    v = lane_xor_add<4>(v); v = lane_xor_add<2>(v); v = lane_xor_add<1>(v);
+    return v;
+}
+template <int WPG, int LPG>
 __device__ __forceinline__ void group_sum2(float& a, float& b, float (*red)[2][16], int slot) {
-    a = warp_sum(a); b = warp_sum(b);
+    a = lanes_sum<LPG>(a); b = lanes_sum<LPG>(b);
     if constexpr (WPG > 1) {
         const int wave = threadIdx.x >> 6;
         if ((threadIdx.x & 63) == 0) { red[slot][0][wave] = a; red[slot][1][wave] = b; }
@@ -133,19 +141,23 @@ __device__ __forceinline__ void group_sum2(float& a, float& b, float (*red)[2][1
 }
 
 // grid (row blocks, groups).  WPG = waves per (row, group): 1 (256 threads, each wave its own rows) or 4 or 5 (the whole
-// workgroup of WPG waves shares a row).  NV = vectors per lane.  GATED: z given.  EXACT: the group is exactly WPG x 64 x NV
+// workgroup of WPG waves shares a row).  LPG < 64: a wave takes 64 / LPG neighbouring groups of its row, LPG lanes each, and the
+// grid has as many fewer columns.  NV = vectors per lane.  GATED: z given.  EXACT: the group is exactly WPG x 64 x NV
 // vectors wide, so no lane is idle and nothing is masked (5120 channels of a 16-bit type = 5 waves x 2 vectors).
-template <typename T, int WPG, int NV, bool BWD, bool GATED, bool EXACT>
+template <typename T, int WPG, int NV, bool BWD, bool GATED, bool EXACT, int LPG = 64>
 __global__ void __launch_bounds__(WPG == 1 ? 256 : WPG * 64)
 rmsnorm_gated_kernel(const NormArgs a) {
     constexpr int V = GlueVec<T>::V;
     constexpr int TPG = WPG * 64;                 // threads per (row, group)
     __shared__ float red[2][2][16];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int tl = WPG > 1 ? tid : lane;          // index inside the (row, group)
-    const int64_t grp = blockIdx.y;
-    const int64_t c0 = grp * a.gw;                // first channel of the group
-    const int nvec = (int)(a.gw / V);
+    static_assert(LPG == 64 || (WPG == 1 && NV == 1 && !EXACT), "several groups per wave: one vector a lane, idle lanes masked");
+    constexpr int SUB = 64 / LPG;                 // groups per wave
+    const int tl = WPG > 1 ? tid : lane % LPG;    // index inside the (row, group)
+    const int64_t grp = (int64_t)blockIdx.y * SUB + (SUB > 1 ? lane / LPG : 0), groups = SUB > 1 ? a.d / a.gw : 0;
+    const bool spare = SUB > 1 && grp >= groups;  // lanes behind the last group
+    const int64_t c0 = (spare ? groups - 1 : grp) * a.gw;      // first channel of the group
+    const int nvec = spare ? 0 : (int)(a.gw / V);
     const float inv_n = 1.f / (float)a.gw;
 
     float w[NV][V], dw[BWD ? NV : 1][V];
@@ -218,7 +230,7 @@ rmsnorm_gated_kernel(const NormArgs a) {
             }
         }
         if (!TWO) load_row(r + RSTEP, q);
-        group_sum2<WPG>(ss, dot, red, slot);
+        group_sum2<WPG, LPG>(ss, dot, red, slot);
         slot ^= 1;
         const float var = ss * inv_n + a.eps;
         const float rinv = __builtin_amdgcn_rsqf(var);
@@ -288,6 +300,15 @@ rmsnorm_gated_kernel(const NormArgs a) {
                 for (int q = 0; q < V / 4; ++q)
                     *reinterpret_cast<floatx4*>(&sums[wave][(it * 64 + lane) * V + 4 * q]) = floatx4{dw[it][4 * q], dw[it][4 * q + 1], dw[it][4 * q + 2], dw[it][4 * q + 3]};
             __syncthreads();
+            if constexpr (SUB > 1) {
+                const int e = tid * 4, v = e / V % LPG;
+                const int64_t g = (int64_t)blockIdx.y * SUB + e / V / LPG;
+                if (e < 64 * V && g < groups && (int64_t)v * V < a.gw)
+                    *reinterpret_cast<floatx4*>(a.partial + (int64_t)blockIdx.x * a.d + g * a.gw + v * V + e % V) =
+                        (*reinterpret_cast<const floatx4*>(&sums[0][e]) + *reinterpret_cast<const floatx4*>(&sums[1][e])) +
+                        (*reinterpret_cast<const floatx4*>(&sums[2][e]) + *reinterpret_cast<const floatx4*>(&sums[3][e]));
+                return;
+            }
             for (int e = tid * 4; e < nvec * V; e += 256 * 4)
                 *reinterpret_cast<floatx4*>(pp + e) = (*reinterpret_cast<const floatx4*>(&sums[0][e]) + *reinterpret_cast<const floatx4*>(&sums[1][e])) +
                                                       (*reinterpret_cast<const floatx4*>(&sums[2][e]) + *reinterpret_cast<const floatx4*>(&sums[3][e]));
@@ -315,6 +336,19 @@ bool norm_shape(int64_t nvec, int vec_elems, int* wpg, int* nv) {
     return false;
 }
 
+// Lanes per group: a wave, or a half, a quarter or an eighth of one for several groups of so few vectors.  With a wave per group of 64
+// channels 56 of 64 lanes idle and every access is a piece of 128 bytes.  Time of 53445 rows of 8 x 64 channels
+// 115 -> 29 us and, backward, 223 -> 52; 16384 x 8 x 128 38 -> 19 and 69 -> 31; 16384 x 8 x 192 38 -> 26 and 70 -> 43; 16384 x 2 x
+// 256 13.1 -> 11.9 and 23 -> 19; up to about 1000 rows the same.
+int norm_lanes(int64_t nvec, int64_t groups) {
+    if (nvec > 32) return 64;
+    int lanes = 8;
+    while (lanes < nvec || (lanes < 64 && 64 / lanes > groups)) lanes *= 2;
+    return lanes;
+}
+// columns of a launch's grid
+int64_t norm_columns(int64_t nvec, int64_t groups) { return ceil_div(groups, (int64_t)(64 / norm_lanes(nvec, groups))); }
+
 // What a workspace has room for: a backward of about 512 workgroups of at least 4 rows each.
 int64_t norm_rows_per_block(int64_t rows, int64_t groups) {
     int64_t rb = rows * groups / 512;
@@ -337,7 +371,7 @@ int64_t norm_rows_per_block(int64_t rows, int64_t groups) {
 int64_t norm_rows_per_workgroup(int64_t rows, int64_t groups, int64_t nvec, int vec_elems, bool bwd) {
     int wpg = 1, nv = 1;
     if (!norm_shape(nvec, vec_elems, &wpg, &nv)) return norm_rows_per_block(rows, groups);
-    const int64_t all = rows * groups;
+    const int64_t all = rows * norm_columns(nvec, groups);
     const bool exact = (int64_t)wpg * 64 * nv == nvec;
     int64_t per_cu = 1;
     if (wpg == 1) {
@@ -360,8 +394,15 @@ int launch_norm(const NormArgs& a, int64_t groups, hipStream_t st) {
     int wpg = 0, nv = 0;
     if (!norm_shape(a.gw / V, V, &wpg, &nv))
         return fail(M2_ERR_SHAPE, "rmsnorm_gated: %lld channels per group exceed the supported 8192", (long long)a.gw);
-    const dim3 grid((unsigned)ceil_div(a.rows, a.rows_per_block), (unsigned)groups);
+    const dim3 grid((unsigned)ceil_div(a.rows, a.rows_per_block), (unsigned)norm_columns(a.gw / V, groups));
     const bool exact = (int64_t)wpg * 64 * nv == a.gw / V, gated = a.z != nullptr;
+    const int lanes = norm_lanes(a.gw / V, groups);
+#define M2_NORM_PART(L) if (lanes == L) { \
+        if (gated) rmsnorm_gated_kernel<T, 1, 1, BWD, true, false, L><<<grid, 256, 0, st>>>(a); \
+        else rmsnorm_gated_kernel<T, 1, 1, BWD, false, false, L><<<grid, 256, 0, st>>>(a); \
+        return check_launch("rmsnorm_gated_kernel"); }
+    M2_NORM_PART(8) M2_NORM_PART(16) M2_NORM_PART(32)
+#undef M2_NORM_PART
 #define M2_NORM_LAUNCH(W, N, G, E) { rmsnorm_gated_kernel<T, W, N, BWD, G, E><<<grid, (W == 1 ? 256 : W * 64), 0, st>>>(a); return check_launch("rmsnorm_gated_kernel"); }
 #define M2_NORM_CASE(W, N) if (wpg == W && nv == N) { \
         if (gated) { if (exact) M2_NORM_LAUNCH(W, N, true, true) else M2_NORM_LAUNCH(W, N, true, false) } \

@@ -228,3 +228,12 @@ def test_mixer_params_and_their_gradients(heads, channels, with_D, types):
                                       (515, 7168, 1)])
 def test_rmsnorm_gated_rows_per_workgroup(dtype, rows, d, g):
     test_rmsnorm_gated_fwd_bwd(dtype, (1, rows), d, g, True)
+
+
+# groups that share a wave: eight, four and two of them, with idle lanes in each, spare lanes behind the last group, fewer groups than a wave
+# could take, and 32 vectors against 33
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,d,g", [(2003, 512, 8), (5, 2048, 32), (77, 576, 3), (130, 384, 2), (33, 40, 5), (1, 128, 2), (9, 1024, 4), (9, 1056, 4), (9, 544, 4)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_rmsnorm_gated_groups_that_share_a_wave(dtype, rows, d, g, gated):
+    test_rmsnorm_gated_fwd_bwd(dtype, (1, rows), d, g, gated)
