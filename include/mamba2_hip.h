@@ -241,6 +241,11 @@ size_t m2_rmsnorm_gated_bwd_workspace_bytes(int64_t rows, int64_t channels, int3
 int m2_rmsnorm_gated_bwd(const m2_rmsnorm_params* p, void* stream);
 /* The same without the sum of d_weight: *rows partial rows of `channels` floats are left at the start of the workspace. */
 int m2_rmsnorm_gated_bwd_partial(const m2_rmsnorm_params* p, int64_t* rows, void* stream);
+/* m2_rmsnorm_gated_fwd, _fwd_check and _bwd_partial for a gate in rows of any width (the mixer core's packed projection): z and its stride
+ * may be any number of elements, everything else as above. */
+int m2_core_norm_fwd(const m2_rmsnorm_params* p, void* stream);
+int m2_core_norm_fwd_check(const m2_rmsnorm_params* p);
+int m2_core_norm_bwd_partial(const m2_rmsnorm_params* p, int64_t* rows, void* stream);
 
 /* Block boundary of the token-by-token loop (mamba2/modeling_mamba2.py:133-140 Mamba2Block.step's residual add,
  * followed by the next block's -- or the final -- Mamba2RMSNorm, :94-103), in one pass over the rows:

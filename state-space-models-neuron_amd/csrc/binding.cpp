@@ -30,8 +30,8 @@ using torch::autograd::variable_list;
 #define M2_BOUND(F) \
     F(m2_last_error) F(m2_conv1d_fwd) F(m2_conv1d_prefill) F(m2_conv1d_bwd_workspace_bytes) F(m2_conv1d_bwd) F(m2_conv1d_bwd_partial) F(m2_ssd_chunk_states_bytes) \
     F(m2_ssd_fwd_workspace_bytes) F(m2_ssd_fwd_check) F(m2_ssd_fwd) F(m2_ssd_bwd_workspace_bytes) F(m2_ssd_bwd) F(m2_decode_workspace_bytes) \
-    F(m2_decode_step) F(m2_decode_step_static) F(m2_rmsnorm_gated_fwd_check) F(m2_rmsnorm_gated_fwd) F(m2_rmsnorm_gated_bwd_workspace_bytes) \
-    F(m2_rmsnorm_gated_bwd) F(m2_rmsnorm_gated_bwd_partial) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_rows) F(m2_embed_rows) F(m2_decode_layer) F(m2_mixer_params) F(m2_param_sums) \
+    F(m2_decode_step) F(m2_decode_step_static) F(m2_core_norm_fwd_check) F(m2_rmsnorm_gated_fwd) F(m2_rmsnorm_gated_bwd_workspace_bytes) \
+    F(m2_rmsnorm_gated_bwd) F(m2_core_norm_fwd) F(m2_core_norm_bwd_partial) F(m2_add_rmsnorm) F(m2_linear_small_fits) F(m2_linear_small) F(m2_decode_rows) F(m2_embed_rows) F(m2_decode_layer) F(m2_mixer_params) F(m2_param_sums) \
     F(m2_product_pays) F(m2_product_workspace_bytes) F(m2_product) \
     F(m2_product_pair_pays) F(m2_product_pair_workspace_bytes) F(m2_product_pair)
 struct Lib {
@@ -418,28 +418,17 @@ void check_norm(const Tensor& x, const Tensor& z) {
     TORCH_CHECK_VALUE(!z.defined() || (z.sizes() == x.sizes() && z.scalar_type() == x.scalar_type()), "rmsnorm_gated: z must have the shape and dtype of x");
 }
 
-// A norm that is ready to run: its operands (rows that the kernel does not read where they lie copied) and its output.
-struct NormCall {
-    Tensor x, z, w32, out;
-    m2_rmsnorm_params p;
-    NormCall(const Tensor& x_, const OptTensor& z_, const Tensor& weight, int64_t n_groups, double eps, at::ScalarType out_dtype) {
-        require_gpu({&x_, &or_none(z_), &weight});
-        check_norm(x_, or_none(z_));
-        TORCH_CHECK_VALUE(out_dtype == at::kFloat || out_dtype == x_.scalar_type(), "rmsnorm_gated: out_dtype must be float32 or the dtype of x");
-        x = aligned(x_); z = z_ ? aligned(*z_) : Tensor(); w32 = f32(weight);
-        p = norm_params(x, z, w32, n_groups, eps);
-        out = at::empty(x.sizes(), x.options().dtype(out_dtype));
-        p.out = ptr(out); p.out_stride_row = x.size(-1); p.out_f32 = out_dtype == at::kFloat;
-    }
-    void run(void* stream) { check(lib.m2_rmsnorm_gated_fwd(&p, stream), "m2_rmsnorm_gated_fwd"); }
-};
-
-Tensor rmsnorm_forward(const Tensor& x, const OptTensor& z, const Tensor& weight, int64_t n_groups, double eps, at::ScalarType out_dtype) {
-    require_gpu({&x});
-    Scope scope(x);
-    NormCall norm(x, z, weight, n_groups, eps, out_dtype);
-    norm.run(scope.stream);
-    return norm.out;
+Tensor rmsnorm_forward(const Tensor& x_, const OptTensor& z_, const Tensor& weight, int64_t n_groups, double eps, at::ScalarType out_dtype) {
+    require_gpu({&x_, &or_none(z_), &weight});
+    Scope scope(x_);
+    check_norm(x_, or_none(z_));
+    TORCH_CHECK_VALUE(out_dtype == at::kFloat || out_dtype == x_.scalar_type(), "rmsnorm_gated: out_dtype must be float32 or the dtype of x");
+    const Tensor x = aligned(x_), z = z_ ? aligned(*z_) : Tensor(), w32 = f32(weight);      // rows that the kernel does not read where they lie: copied
+    m2_rmsnorm_params p = norm_params(x, z, w32, n_groups, eps);
+    const Tensor out = at::empty(x.sizes(), x.options().dtype(out_dtype));
+    p.out = ptr(out); p.out_stride_row = x.size(-1); p.out_f32 = out_dtype == at::kFloat;
+    check(lib.m2_rmsnorm_gated_fwd(&p, scope.stream), "m2_rmsnorm_gated_fwd");
+    return out;
 }
 
 // the gradient of a norm's output as its kernel reads it
@@ -539,13 +528,6 @@ struct Packed {
         if (!even && t.size(1) == 1) zx = zx.as_strided(zx.sizes(), {zx.size(2), zx.size(2), 1});
         b = zx.size(0); l = zx.size(1); sb = zx.stride(0); sl = zx.stride(1);
     }
-    Tensor z() const { return zx.narrow(2, 0, d); }
-    // z where the norm reads it: in zx if its rows lie on 16 bytes there, else a copy that `held` keeps
-    std::pair<const void*, int64_t> z_rows(Tensor& held) const {
-        if (reinterpret_cast<uintptr_t>(zx.data_ptr()) % 16 == 0 && (sl * zx.element_size()) % 16 == 0) return {zx.data_ptr(), sl};
-        held = z().clone(at::MemoryFormat::Contiguous);
-        return {ptr(held), d};
-    }
     Strided xBC() const { return {at_column(zx, d), sb, sl, 1}; }
 };
 
@@ -556,10 +538,12 @@ CoreParams core_params(const Tensor& A, const Tensor& D, const Tensor& dt_bias, 
     return {ptr<float>(A), ptr<float>(D), ptr<float>(dt_bias), ptr<float>(norm_w)};
 }
 
-// the norm's parameters: the scan's output, gated by z, per group
-m2_rmsnorm_params core_norm_params(const Packed& k, const CoreParams& w, const void* scan_out, const std::pair<const void*, int64_t>& z) {
+// the norm's parameters: the scan's output, gated by z, per group.  z is read where it lies, on whatever element a row of the packed
+// projection starts (a copy into aligned rows in front of the forward and of the backward was a tenth of a core with an odd number of
+// heads: 22 of 222 us for a prompt of 13115 tokens with 13 heads of 128).
+m2_rmsnorm_params core_norm_params(const Packed& k, const CoreParams& w, const void* scan_out) {
     m2_rmsnorm_params p{};
-    p.x = scan_out; p.x_stride_row = k.d; p.z = z.first; p.z_stride_row = z.second;
+    p.x = scan_out; p.x_stride_row = k.d; p.z = ptr(k.zx); p.z_stride_row = k.sl;
     p.rows = k.b * k.l; p.channels = k.d; p.n_groups = static_cast<int32_t>(k.g);
     p.dtype = dtype_code(k.zx); p.eps = static_cast<float>(kNormEps); p.weight = w.norm_w;
     return p;
@@ -608,11 +592,10 @@ CoreOut core_forward(const Packed& k, const CoreParams& params, const Tensor& co
     p.y = ptr(r.scan_out); p.y_stride_b = k.l * k.d; p.y_stride_l = k.d; p.y_stride_h = k.p;
     launch_ssd_fwd(p, k.zx, stream);
     if (want_norm) {
-        Tensor held;
-        m2_rmsnorm_params q = core_norm_params(k, params, ptr(r.scan_out), k.z_rows(held));
+        m2_rmsnorm_params q = core_norm_params(k, params, ptr(r.scan_out));
         r.norm_out = at::empty({k.b, k.l, k.d}, k.zx.options());
         q.out = ptr(r.norm_out); q.out_stride_row = k.d;
-        check(lib.m2_rmsnorm_gated_fwd(&q, stream), "m2_rmsnorm_gated_fwd");
+        check(lib.m2_core_norm_fwd(&q, stream), "m2_core_norm_fwd");
     }
     return r;
 }
@@ -639,13 +622,11 @@ CoreGrads core_backward(const Packed& k, const Tensor& d_out_, const CoreParams&
     char* const d_zx = static_cast<char*>(r.zx.data_ptr());
     const Tensor d_out = norm_rows(d_out_, k.zx.scalar_type());
     const bool to_heads = !head_grads.empty();
-    // everything that does not leave this function, in one allocation
-    Tensor held;
     require_gpu({&d_out, &scan_out, &conv_out});
     TORCH_CHECK_VALUE(scan_out.dim() == 3 && scan_out.size(0) == k.b && scan_out.size(1) == k.l && scan_out.size(2) == k.d &&
                           scan_out.scalar_type() == k.zx.scalar_type(), "scan_out must be (b, l, d_inner) in the dtype of zxBCdt");
     const Tensor scanned = aligned(scan_out);
-    m2_rmsnorm_params q = core_norm_params(k, w, ptr(scanned), k.z_rows(held));
+    m2_rmsnorm_params q = core_norm_params(k, w, ptr(scanned));
     q.x_stride_row = rows2d(scanned, "scan_out").stride;
     m2_ssd_params p = core_ssd_params(k, conv_out, w);
     p.chunk_states = chunk_states_ptr(p, states);
@@ -658,7 +639,7 @@ CoreGrads core_backward(const Packed& k, const Tensor& d_out_, const CoreParams&
                  heads_bytes = to_heads ? static_cast<size_t>(3 * k.h) * 4 : 0, conv_bytes = lib.m2_conv1d_bwd_workspace_bytes(k.b, k.l, k.conv, conv_w.size(2));
     q.workspace_bytes = lib.m2_rmsnorm_gated_bwd_workspace_bytes(q.rows, q.channels, q.n_groups, q.dtype);
     p.workspace_bytes = lib.m2_ssd_bwd_workspace_bytes(&p);
-    Pieces pieces;
+    Pieces pieces;      // everything that does not leave this function, in one allocation
     for (const size_t bytes : {d_scan_bytes, d_conv_bytes, heads_bytes, conv_bytes, q.workspace_bytes, p.workspace_bytes}) pieces.want(bytes);
     pieces.allocate(k.zx);
     void* const d_scan = pieces.take(d_scan_bytes);
@@ -670,7 +651,7 @@ CoreGrads core_backward(const Packed& k, const Tensor& d_out_, const CoreParams&
     q.d_out = ptr(d_out); q.d_out_stride_row = rows2d(d_out, "d_out").stride;
     q.dx = d_scan; q.dx_stride_row = k.d; q.dz = d_zx; q.dz_stride_row = pitch;
     q.workspace = pieces.take(q.workspace_bytes);
-    check(lib.m2_rmsnorm_gated_bwd_partial(&q, &norm_sums.count, stream), "m2_rmsnorm_gated_bwd");
+    check(lib.m2_core_norm_bwd_partial(&q, &norm_sums.count, stream), "m2_core_norm_bwd");
     norm_sums.rows = static_cast<const float*>(q.workspace);
     // the scan's gradients leave as one packed [dx | dB | dC] buffer, that of the raw dt in its columns of r.zx
     p.dy = d_scan; p.dx = d_conv; p.dB = d_conv + k.d * es; p.dC = d_conv + (k.d + k.g * k.n) * es; p.ddt = d_zx + (k.d + k.conv) * es;
@@ -921,8 +902,9 @@ Tensor fused_prefill(const Tensor& zx, const Tensor& A, const OptTensor& D, cons
     c.y = ptr(conv_out);
     // The conv moves the cache on, so everything behind it is allocated and checked first: a call that is refused leaves the cache
     // as it was.
-    const Tensor A32 = f32(A), D32 = f32(or_none(D)), bias = f32(dt_bias);
-    m2_ssd_params p = core_ssd_params(k, conv_out, core_params(A32, D32, bias, Tensor()));
+    const Tensor A32 = f32(A), D32 = f32(or_none(D)), bias = f32(dt_bias), norm32 = f32(norm_w);
+    const CoreParams params = core_params(A32, D32, bias, norm32);
+    m2_ssd_params p = core_ssd_params(k, conv_out, params);
     const Tensor y = at::empty({k.b, k.l, d}, zx.options());
     p.initial_state = continuing ? ptr<float>(S) : nullptr; p.final_state = ptr<float>(S);
     p.y = ptr(y); p.y_stride_b = k.l * d; p.y_stride_l = d; p.y_stride_h = hd;
@@ -930,14 +912,16 @@ Tensor fused_prefill(const Tensor& zx, const Tensor& A, const OptTensor& D, cons
     const Tensor ws = scratch(p.workspace_bytes, zx);
     p.workspace = ptr(ws);
     check(lib.m2_ssd_fwd_check(&p), "m2_ssd_fwd");
-    NormCall norm(y, k.z(), norm_w, g, kNormEps, zx.scalar_type());
-    check(lib.m2_rmsnorm_gated_fwd_check(&norm.p), "m2_rmsnorm_gated_fwd");
+    const Tensor out = at::empty({k.b, k.l, d}, zx.options());
+    m2_rmsnorm_params q = core_norm_params(k, params, ptr(y));
+    q.out = ptr(out); q.out_stride_row = d;
+    check(lib.m2_core_norm_fwd_check(&q), "m2_core_norm_fwd");
     check(lib.m2_conv1d_prefill(&c, ptr(cs), static_cast<int32_t>(cs.size(2)), continuing, scope.stream), "m2_conv1d_prefill");
     check(lib.m2_ssd_fwd(&p, scope.stream), "m2_ssd_fwd");
     if (!own_conv) conv_state.copy_(cs);
     if (!own_ssm) ssm_state.copy_(S);
-    norm.run(scope.stream);
-    return norm.out;
+    check(lib.m2_core_norm_fwd(&q, scope.stream), "m2_core_norm_fwd");
+    return out;
 }
 
 // ----------------------------------------------------------------------------------------------- decode step

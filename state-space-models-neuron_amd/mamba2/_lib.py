@@ -108,6 +108,9 @@ SYMBOLS = {
     "m2_rmsnorm_gated_bwd_workspace_bytes": (_sz, [_i64, _i64, _i32, _i32]),
     "m2_rmsnorm_gated_bwd": (C.c_int, [C.POINTER(RmsnormParams), _vp]),
     "m2_rmsnorm_gated_bwd_partial": (C.c_int, [C.POINTER(RmsnormParams), C.POINTER(_i64), _vp]),
+    "m2_core_norm_fwd": (C.c_int, [C.POINTER(RmsnormParams), _vp]),
+    "m2_core_norm_fwd_check": (C.c_int, [C.POINTER(RmsnormParams)]),
+    "m2_core_norm_bwd_partial": (C.c_int, [C.POINTER(RmsnormParams), C.POINTER(_i64), _vp]),
     "m2_add_rmsnorm": (C.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, C.c_float, _i32, _vp]),
     "m2_linear_small_fits": (C.c_int, [_i64, _i64, _i64, _i32]),
     "m2_linear_small": (C.c_int, [C.POINTER(LinearParams), _vp]),

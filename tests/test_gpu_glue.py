@@ -237,3 +237,32 @@ def test_rmsnorm_gated_rows_per_workgroup(dtype, rows, d, g):
 @pytest.mark.parametrize("gated", [True, False])
 def test_rmsnorm_gated_groups_that_share_a_wave(dtype, rows, d, g, gated):
     test_rmsnorm_gated_fwd_bwd(dtype, (1, rows), d, g, gated)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,d,g,extra,first", [(131, 512, 8, 13, 0), (70, 2048, 1, 1, 3), (33, 5120, 1, 7, 1), (1, 896, 1, 271, 0), (40, 4096, 1, 2, 5)])
+def test_core_norm_reads_the_gate_on_any_element(dtype, rows, d, g, extra, first):
+    """z in rows of a width that is no multiple of a vector, from any element on: the values of an aligned copy, forward and backward."""
+    import ctypes
+    from mamba2 import _lib
+    lib, ptr = _lib.load(), _lib.ptr
+    packed = _rand((rows * (d + extra) + first,), dtype, 41).to(DEV)
+    z = packed[first:].view(rows, d + extra)[:, :d]
+    x, dout, w = _rand((rows, d), dtype, 42).to(DEV), _rand((rows, d), dtype, 43).to(DEV), (1 + 0.1 * _rand((d,), torch.float32, 44)).to(DEV)
+    need = lib.m2_rmsnorm_gated_bwd_workspace_bytes(rows, d, g, _lib.dtype_code(dtype))
+
+    def call(gate):
+        out, dx, dz, ws = torch.zeros_like(x), torch.zeros_like(x), torch.zeros_like(x), torch.zeros(need // 4, device=DEV)
+        p = _lib.RmsnormParams(x=ptr(x), z=ptr(gate), weight=ptr(w), out=ptr(out), d_out=ptr(dout), dx=ptr(dx), dz=ptr(dz), workspace=ptr(ws), workspace_bytes=need, rows=rows,
+                               channels=d, x_stride_row=d, z_stride_row=gate.stride(0), out_stride_row=d, d_out_stride_row=d, dx_stride_row=d, dz_stride_row=d, n_groups=g,
+                               dtype=_lib.dtype_code(dtype), eps=1e-5)
+        n = ctypes.c_int64(-1)
+        _lib.check(lib.m2_core_norm_fwd(ctypes.byref(p), _lib.stream_ptr()), "core_norm_fwd")
+        _lib.check(lib.m2_core_norm_bwd_partial(ctypes.byref(p), ctypes.byref(n), _lib.stream_ptr()), "core_norm_bwd_partial")
+        refused = lib.m2_rmsnorm_gated_fwd(ctypes.byref(p), _lib.stream_ptr()) != 0
+        return (out, dx, dz, ws[:n.value * d]), refused
+
+    whole = z.clone(memory_format=torch.contiguous_format)
+    for a, b in zip(call(z)[0], call(whole)[0]):
+        assert torch.equal(a, b)
+    assert call(z)[1] and not call(whole)[1]      # the plain entry asks for whole vectors, as before
