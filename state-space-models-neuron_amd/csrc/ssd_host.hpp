@@ -32,6 +32,7 @@ struct SsdWorkspace {
     float* dGs = nullptr; float* dBs = nullptr; float* dCs = nullptr;   // partials summed over the head slices, where there are several
     float* dirp = nullptr; float* rbp = nullptr; float* dDp8 = nullptr; // per token, per wave: what the main kernel leaves for ddt and dD
     int64_t ns_g = 1, hps_g = 1, ns_b = 1, hps_b = 1;   // head slicing of dg16 and of the main backward kernel
+    void* seg = nullptr; float* seg_lam = nullptr;      // the state pass in segments
     bool finished = false;              // the main kernel's workgroups have whole groups and leave dB and dC: no partials of those
     size_t bytes = 0;
     size_t kept_bytes = 0;              // size of the forward -> backward carry-over (chunk_states buffer)
@@ -112,6 +113,12 @@ inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_
         if (p->dtype != M2_F32) w.Ct = keep(grp * p->dstate * kQ * esz);
         w.kept_bytes = koff;
     }
+    if (p->dtype != M2_F32)
+        if (const int64_t m = state_pass_seg_chunks(p->batch * p->nheads, nc)) {
+            const size_t sums = (size_t)((ceil_div(nc, m) - 1) * p->batch * p->nheads);
+            w.seg = take(sums * p->headdim * p->dstate * 4);
+            w.seg_lam = reinterpret_cast<float*>(take(sums * 4));
+        }
     if (bwd) {
         ssd_slicing(p, kWgsDg, true, &w.ns_g, &w.hps_g);
         ssd_slicing(p, kWgsDx, true, &w.ns_b, &w.hps_b);
@@ -179,16 +186,23 @@ inline size_t cb_smem(int n) {      // operand rows; 32 tokens of both to transp
 }
 
 template <typename T, int P, int N, bool REVERSE, int HS, bool HILO>
-inline int launch_state_pass16(const StatePassArgs& a, int64_t batch, hipStream_t st) {
-    auto launch = [&](auto k, size_t sm, int split) -> int {
+inline int launch_state_pass16(StatePassArgs a, const SsdWorkspace& w, int64_t batch, hipStream_t st) {
+    auto launch = [&](auto k, size_t sm, int split, int64_t segs = 1) -> int {
         if (const int rc = allow_smem(k, sm)) return rc;
-        k<<<dim3((unsigned)(a.nheads * split), (unsigned)batch), state_pass_threads<N>(), sm, st>>>(a);
+        k<<<dim3((unsigned)(a.nheads * split), (unsigned)batch, (unsigned)segs), state_pass_threads<N>(), sm, st>>>(a);
         return M2_OK;
     };
     if constexpr (N == 128 && !HILO)
         if (state_pass_split(batch * a.nheads, N) == 1)
             return launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, 1>, state_pass_smem<P, N, HILO, 1>(), 1);
     constexpr int SPLIT = kStatePassSplit;
+    if (const int64_t m = state_pass_seg_chunks(batch * a.nheads, a.nchunks)) {
+        a.seg = static_cast<floatx4*>(w.seg); a.seg_lam = w.seg_lam; a.seg_chunks = m;
+        const int64_t sums = ceil_div(a.nchunks, m) - 1;
+        int rc = launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, SPLIT, 1>, state_pass_smem<P, N, HILO, SPLIT>(), SPLIT, sums);
+        if (!rc) rc = check_launch("ssd state_pass16_kernel, sums of segments");
+        return rc ? rc : launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, SPLIT, 2>, state_pass_smem<P, N, HILO, SPLIT>(), SPLIT, sums);
+    }
     return launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, SPLIT>, state_pass_smem<P, N, HILO, SPLIT>(), SPLIT);
 }
 
@@ -246,11 +260,11 @@ inline int ssd_launch_states(const SsdCall* p, const SsdWorkspace& w, float* fin
         // (3.7 us more per pass at b4 l2048 h80; the states entering the chunks come out of the same accumulators, so y
         // differs from the one-tile form in the last bit here and there)
         const bool hilo = final_out != nullptr;
-        StatePassArgs sa;
+        StatePassArgs sa{};
         sa.X = x; sa.X_sb = p->x_stride_b; sa.X_sl = p->x_stride_l; sa.X_sh = p->x_stride_h;
         sa.ldtab = w.ldtab; sa.Mt = w.Bt; sa.init = p->initial_state; sa.prev = w.prev; sa.final_out = final_out;
         sa.seqlen = p->seqlen; sa.nheads = p->nheads; sa.ngroups = p->ngroups; sa.nchunks = nc;
-        if ((rc = hilo ? launch_state_pass16<T, P, N, false, HS, true>(sa, p->batch, st) : launch_state_pass16<T, P, N, false, HS, false>(sa, p->batch, st))) return rc;
+        if ((rc = hilo ? launch_state_pass16<T, P, N, false, HS, true>(sa, w, p->batch, st) : launch_state_pass16<T, P, N, false, HS, false>(sa, w, p->batch, st))) return rc;
         return check_launch("ssd state_pass16_kernel");
     } else {
         // fp32 operands: per-chunk contributions (workspace), then the recurrence over the chunks

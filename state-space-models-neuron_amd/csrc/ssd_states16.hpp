@@ -17,6 +17,8 @@
 // The state leaves through an LDS tile of the workgroup's whole slab (one per chunk parity), written before the chunk's barrier
 // and read behind it, so that a wave stores whole state rows: its share of the slab is one contiguous piece of memory.
 #pragma once
+#include <type_traits>
+
 #include "ssd_y.hpp"
 
 namespace m2 {
@@ -29,6 +31,8 @@ struct StatePassArgs {
     void* prev;                                    // out [b][c][h][P][N], operand type
     float* final_out;                              // out fp32 [b][h][P][N]: final state / gradient of the initial state, or null
     int64_t seqlen, nheads, ngroups, nchunks;
+    floatx4* seg; float* seg_lam;                  // in segments: a segment's state [segment][b][h] in accumulator order, and the sum of its Lam
+    int64_t seg_chunks;                            // chunks per segment
 };
 
 // What bounds the pass: a CU's vector-memory path.  Its loads retire in order, so the operand fragments (which come from L2)
@@ -47,6 +51,23 @@ inline int state_pass_split(int64_t heads, int n) {
     const int64_t cus = device_cus(), rounds = ceil_div(heads, cus);
     return n == 128 && heads * 5 >= rounds * cus * 4 ? 1 : kStatePassSplit;
 }
+// Chunks per segment, or 0: one pass over the whole sequence.  Half heads that leave half the CUs idle walk a long sequence as a chain
+// of steps of about 1.05 us each; in segments the chain is as long as two of them: the first launch walks the first segment and forms
+// the sums of the others but the last from zero, all side by side, and the second starts each of the others from the sums in front of
+// it, decayed (the decay is one number per head, so this costs a product per element and segment).
+// A launch more and the filling of two chains cost about 3 us; below the line they are not earned.  Whole forward scan, us, whole pass ->
+// segments, for 16, 48, 64, 84 and 128 half heads (16, 5, 4, 3 and 2 sets), 128 state columns:
+//   8 chunks    22.9 -> 23.8   24.3 -> 25.5   24.9 -> 26.0   28.1 -> 30.8   30.2 -> 33.0
+//   12 chunks   25.7 -> 24.7   29.8 -> 29.2   30.8 -> 30.7   31.4 -> 33.2   35.6 -> 37.8
+//   16 chunks   28.4 -> 25.5   33.6 -> 31.9   34.6 -> 35.4   36.5 -> 37.6   39.3 -> 41.4
+//   24 chunks   34.0 -> 27.4   41.8 -> 37.5   43.1 -> 38.9   43.0 -> 42.3   51.1 -> 51.1
+//   64 chunks   65.8 -> 38.2   74.9 -> 53.5   80.3 -> 60.9   81.6 -> 74.5   96.8 -> 88.5
+inline int64_t state_pass_seg_chunks(int64_t heads, int64_t nchunks) {
+    const int64_t sets = heads > 0 ? device_cus() / (heads * kStatePassSplit) : 0;      // of workgroups that the CUs hold, one each
+    if (sets < 2 || nchunks < 12 || nchunks * sets < 72) return 0;
+    const int64_t chunks = ceil_div(nchunks, sets + 1);
+    return chunks < 2 ? 2 : chunks;
+}
 // one wave per 32 state columns
 template <int N> constexpr int state_pass_threads() { return (N / 32) * 64; }
 template <int P, int N, bool HILO = false, int SPLIT = kStatePassSplit>
@@ -57,7 +78,10 @@ constexpr size_t state_pass_smem() {
 // HILO: the scaled rows are staged as TWO 16-bit tiles, the rounded value and the rounded remainder, and each k step takes
 // two products, so that the fp32 scale dt e^{Lam - l} reaches the accumulators with 16 significand bits instead of 8 (the
 // final state is an fp32 output; with one tile its error is that of the operand rounding, 2^-9 of every term).
-template <typename T, int P, int N, bool REVERSE, int HS, bool HILO = false, int SPLIT = kStatePassSplit>
+// PHASE 0: the whole sequence.  1: segment z, up to the last but one, from the initial state (the first, whose states are stored) or from
+// zero, to `seg` and `seg_lam`.  2: segment z + 1 from what `seg` holds for those in front of it.  Segments count in the order of the walk.
+// The initial state is read in the first launch only and the final one written in the second: they may be the same tensor.
+template <typename T, int P, int N, bool REVERSE, int HS, bool HILO = false, int SPLIT = kStatePassSplit, int PHASE = 0>
 __global__ void __launch_bounds__(state_pass_threads<N>(), SPLIT == 1 ? 2 : 3)
 state_pass16_kernel(const StatePassArgs a) {
     static_assert(sizeof(T) == 2, "16-bit operands only");
@@ -98,6 +122,10 @@ state_pass16_kernel(const StatePassArgs a) {
     // The MFMAs are issued with swapped operands: acc[i][j][v] is the state at row pw P/2 + 32 i + r, column
     // n0 + 32 j + acc_row(lane, v), i.e. a lane holds groups of 4 consecutive columns of ONE row (8-byte staging writes).
     floatx16 acc[PBW][NBW];
+    const int64_t seg = PHASE == 0 ? 0 : (int64_t)blockIdx.z + (PHASE == 2 ? 1 : 0);
+    const int64_t seg_pitch = (int64_t)gridDim.y * a.nheads * (P * N / 4);
+    floatx4* const seg_q = PHASE == 0 ? nullptr : a.seg + ((bh * SPLIT + pw) * NWAVES + wave_u) * (PBW * NBW * 4 * 64) + lane;
+    const float* init = PHASE == 0 || (PHASE == 1 && seg == 0) ? a.init : nullptr;
 #pragma unroll
     for (int i = 0; i < PBW; ++i)
 #pragma unroll
@@ -105,8 +133,22 @@ state_pass16_kernel(const StatePassArgs a) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int row = pw * PH + i * 32 + r, col = n0 + j * 32 + acc_row(lane, v);
-                acc[i][j][v] = a.init ? a.init[bh * (P * N) + row * N + col] : 0.f;
+                acc[i][j][v] = init ? init[bh * (P * N) + row * N + col] : 0.f;
             }
+    if constexpr (PHASE == 2)
+        for (int64_t t = 0; t < seg; ++t) {
+            const float dec = t ? __expf(a.seg_lam[t * (int64_t)gridDim.y * a.nheads + bh]) : 0.f;      // nothing in front of the first
+#pragma unroll
+            for (int i = 0; i < PBW; ++i)
+#pragma unroll
+                for (int j = 0; j < NBW; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const floatx4 v = seg_q[t * seg_pitch + ((i * NBW + j) * 4 + q) * 64];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[i][j][4 * q + e] = acc[i][j][4 * q + e] * dec + v[e];
+                    }
+        }
 
     // two chunks ahead in registers, in two sets used alternately: the x / dy pieces with their token's l and dt, and
     // the chunk's Lam.  The values of chunk cc are consumed before the barrier of its iteration; behind it the same set
@@ -121,11 +163,15 @@ state_pass16_kernel(const StatePassArgs a) {
     // The bases walk from chunk to chunk by constant steps: formed anew for each chunk out of 64-bit products (and the issue
     // priority below out of a 64-bit quotient) they were 150 of the 200 scalar instructions of an iteration, which on a chip
     // holding few workgroups stand between one chunk's products and the next: 181 -> 169 us at b1 l16384 h80.
-    const int nci = (int)nc, cfirst = REVERSE ? nci - 1 : 0;
+    const int nci = (int)nc, c0 = PHASE == 0 ? 0 : (int)(seg * a.seg_chunks);      // c0: chunks in front of the segment
+    const bool last_seg = PHASE == 0 || (PHASE == 2 && blockIdx.z + 1 == gridDim.z);
+    const int cfirst = REVERSE ? nci - 1 - c0 : c0, tail_at = (REVERSE ? 0 : nci - 1) - c0;
+    const int count = last_seg ? nci - c0 : (int)a.seg_chunks;
     // Steps of the recurrence: what the last chunk adds reaches only the state behind it, so without a reader of that the last
     // chunk's state is stored and nothing of it is loaded or multiplied (forward and backward at b4 l2048 h80 335.5 -> 332.5 us; fp32
     // operands, whose chunks are workgroups of part-filled rounds, gained nothing by the same).
-    const int nsteps = HILO || a.final_out ? nci : nci - 1;      // (two-tile operands are for a final state)
+    const bool ends = PHASE == 1 || (last_seg && (HILO || a.final_out));      // (two-tile operands are for a final state)
+    const int nsteps = ends ? count : count - 1;
     const int tail_rows = (int)(a.seqlen - (nc - 1) * kQ);      // valid rows of the last chunk
     constexpr int DIR = REVERSE ? -1 : 1;
     const char* xq = reinterpret_cast<const char*>(static_cast<const T*>(a.X) + b * a.X_sb + (int64_t)cfirst * kQ * a.X_sl + head_off<HS>(h, a.X_sh) + pw * PH);
@@ -135,7 +181,7 @@ state_pass16_kernel(const StatePassArgs a) {
     const int64_t x_step = DIR * (int64_t)kQ * a.X_sl * 2, m_step = DIR * a.ngroups * (int64_t)(N * kQ * 2), o_step = DIR * a.nheads * (int64_t)(P * N * 2);
     int kload = 0;                                      // processing index of the chunk xq and tq stand at
     auto load_ahead = [&](Ahead& s) {
-        const uint32_t last = (uint32_t)((kload == (REVERSE ? 0 : nci - 1) ? tail_rows : kQ) - 1);      // last valid row
+        const uint32_t last = (uint32_t)((kload == tail_at ? tail_rows : kQ) - 1);      // last valid row
         const uint32_t last_off = last * x_row_bytes;
         const char* xp = xq;
         const float* tab = tq;
@@ -193,7 +239,10 @@ state_pass16_kernel(const StatePassArgs a) {
         op += o_step;
     };
     int next_drop = q1;
+    float lam_sum = 0.f;
     __builtin_amdgcn_s_setprio(3);
+    auto walk = [&](auto keeps) {      // keeps: the states leave
+    constexpr bool KEEPS = decltype(keeps)::value;
     auto step = [&](int cc, Ahead& s) {
         const int buf = cc & 1;
         // Issue priority falls as the workgroup advances, so that of the workgroups sharing a CU the one furthest behind
@@ -237,14 +286,15 @@ state_pass16_kernel(const StatePassArgs a) {
             *reinterpret_cast<u32x4*>(cX + (row * SPR_X + (slot ^ tile_swz<SPR_X>(row))) * 8) = o;
         }
         const float dec = __expf(s.lam);
+        if (PHASE == 1) lam_sum += s.lam;
         // the state as it enters this chunk goes into the slab tile of this parity (the other one may still be read by a
         // wave that is behind: it was filled one barrier ago)
-        put_state(sO + buf * (PH * LDO));
+        if (KEEPS) put_state(sO + buf * (PH * LDO));
         __syncthreads();          // both tiles are complete; every wave is done with the other buffers
         load_ahead(s);            // the rows two chunks on
 
         // ---- the state entering (forward) / the gradient leaving (reverse) this chunk
-        store_rows(sO + buf * (PH * LDO));
+        if (KEEPS) store_rows(sO + buf * (PH * LDO));
 
         // ---- S = e^{Lam} S + X_scaled^T M  (accumulated as its transpose M^T X_scaled)
 #pragma unroll
@@ -297,7 +347,20 @@ state_pass16_kernel(const StatePassArgs a) {
         step(cc, s0);
         step(cc + 1, s1);
     }
-    if (HILO || a.final_out) {
+    };
+    if (PHASE == 1 && seg > 0) walk(std::false_type{});
+    else walk(std::true_type{});
+    if (PHASE == 1) {
+#pragma unroll
+        for (int i = 0; i < PBW; ++i)
+#pragma unroll
+            for (int j = 0; j < NBW; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    seg_q[seg * seg_pitch + ((i * NBW + j) * 4 + q) * 64] =
+                        floatx4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        if (tid == 0 && pw == 0) a.seg_lam[seg * (int64_t)gridDim.y * a.nheads + bh] = lam_sum;
+    } else if (ends) {
 #pragma unroll
         for (int i = 0; i < PBW; ++i)
 #pragma unroll

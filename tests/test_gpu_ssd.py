@@ -360,3 +360,36 @@ def test_ssd_gradients_without_the_initial_states_own(l, b, h, p, n, dtype):
     g1 = torch.autograd.grad(y1, leaves, d["dy"])
     g2 = torch.autograd.grad(y2, leaves + [zero], d["dy"])
     assert torch.equal(y1, y2) and all(torch.equal(a, c) for a, c in zip(g1, g2))
+
+
+# the state pass in segments: two chunks each and a last one with one; a whole last chunk and one with a single token; two columns of waves; 
+# three sets of workgroups in four segments of six chunks; wide heads; several sequences and groups
+@pytest.mark.parametrize("b,l,h,p,n,g", [(1, 1536, 2, 64, 128, 1), (1, 1665, 3, 128, 64, 1), (1, 3050, 42, 64, 64, 1), (2, 2944, 16, 64, 128, 2), (3, 2049, 4, 128, 128, 4)])
+def test_ssd_states_in_segments(b, l, h, p, n, g):
+    """Few heads and many chunks: both recurrences, with and without the states at their ends."""
+    test_ssd_packed_views_with_pad_columns_fwd_bwd(torch.bfloat16, b, l, h, p, n, g)
+    test_ssd_gradients_without_the_initial_states_own(l, b, h, p, n, torch.bfloat16)
+
+
+@pytest.mark.parametrize("l,cut,h,n", [(1921, 900, 8, 128), (2560, 1280, 12, 64)])
+def test_prefill_states_in_segments_in_place(l, cut, h, n):
+    """A long prompt behind a cached prefix, whose state is read and written in place, against the same prompt in two shorter pieces."""
+    from mamba2.fused_kernel import mamba2_fused_prefill
+    torch.manual_seed(l)
+    p, d = 64, 64 * h
+    conv = d + 2 * n
+    zx = torch.randn(2, l, 2 * d + 2 * n + h, device=DEV).bfloat16() * 0.5
+    params = (-torch.rand(h, device=DEV) - 0.2, torch.ones(h, device=DEV), (torch.rand(conv, 1, 4, device=DEV) - 0.5).bfloat16(), torch.zeros(conv, device=DEV).bfloat16(),
+              -4 + torch.rand(h, device=DEV), torch.ones(d, device=DEV))
+    conv0, S0 = torch.randn(2, conv, 4, device=DEV).bfloat16(), 0.1 * torch.randn(2, h, p, n, device=DEV)
+
+    def run(cuts):
+        c, S = conv0.clone(), S0.clone()
+        return torch.cat([mamba2_fused_prefill(zx[:, a:e], *params, 1, n, d, p, c, S, continuing=True) for a, e in cuts], 1), c, S
+
+    (y1, c1, S1), (y2, c2, S2) = run([(0, l)]), run([(0, cut), (cut, l)])
+    # each result is rounded to bf16 (2^-9 at most, uniform: an L2 of 2^-9 / sqrt(3)) behind operands that are, in chunks that lie elsewhere: a few
+    # such roundings on either side; the final state's operands keep 16 bits, behind a conv output that has 8 on both sides alike
+    def l2(a, b):
+        return float((a.double() - b.double()).norm() / b.double().norm())
+    assert torch.equal(c1, c2) and l2(y1, y2) < 2.0 ** -7 and l2(S1, S2) < 2.0 ** -12, (l2(y1, y2), l2(S1, S2))
