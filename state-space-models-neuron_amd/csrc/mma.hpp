@@ -24,6 +24,12 @@ constexpr int kP = 64;         // channels of a head as the SSD kernels see it
 template <int HS>
 __device__ __forceinline__ int64_t head_off(int64_t h, int64_t sh) { return HS ? (h >> 1) * sh + (h & 1) * kP : h * sh; }
 
+// Heads of a slice of a group's: `most`, and in the last slice what is left of them.
+__device__ __forceinline__ int64_t slice_heads(int64_t hpg, int64_t slice, int64_t most) {
+    const int64_t left = hpg - slice * most;
+    return left < most ? left : most;
+}
+
 template <typename T> struct MmaTraits;
 template <> struct MmaTraits<bf16_t> { static constexpr int kPad = 8; };
 template <> struct MmaTraits<float> { static constexpr int kPad = 4; };

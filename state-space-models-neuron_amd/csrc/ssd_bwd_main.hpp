@@ -89,7 +89,7 @@ ssd_bwd16_kernel(const Bwd16Args a) {
     const int64_t t0 = c * kQ;
     const int valid = (int)((a.seqlen - t0) < kQ ? (a.seqlen - t0) : kQ);
     const int row0 = rbk * 32;
-    const int64_t h_first = g * hpg + slice * a.hps;
+    const int64_t h_first = g * hpg + slice * a.hps, hps = slice_heads(hpg, slice, a.hps);
     // transpose-read lane roles: the 16 lanes of a group fetch a [4 rows][16 columns] block; lane (i0 = bits 3:2, i1 = bits 1:0)
     // supplies the address of row i0, columns 4 i1 .. 4 i1 + 3 and receives column (lane & 15) of rows 0..3
     const int tr_row = (lane >> 2) & 3;
@@ -154,7 +154,7 @@ ssd_bwd16_kernel(const Bwd16Args a) {
         wait_vmem_all();              // this wave's blocks of dG have landed
         __syncthreads();
         const int64_t grp = ((b * a.nchunks + c) * a.ngroups + g) * (int64_t)(N * kQ);
-        const uint32_t dst = lds_T + (uint32_t)(((a.hps - 1) & 1) * TILES * 2);
+        const uint32_t dst = lds_T + (uint32_t)(((hps - 1) & 1) * TILES * 2);
         constexpr int PIECES = N * kQ * 2 / 1024 / 8;                                   // per wave and tile
 #pragma unroll
         for (int it = 0; it < PIECES; ++it) {
@@ -208,7 +208,7 @@ ssd_bwd16_kernel(const Bwd16Args a) {
                 }
             }
         }
-        for (int64_t hh = 0; hh < a.hps; ++hh) {
+        for (int64_t hh = 0; hh < hps; ++hh) {
             const int64_t h = h_first + hh;
             const int buf = (int)(hh & 1);
             const int64_t bhc = (b * a.nheads + h) * a.nchunks + c;
@@ -224,7 +224,7 @@ ssd_bwd16_kernel(const Bwd16Args a) {
             wv[lane + 64] = lane + 64 >= row0 ? __expf(sl[lane + 64] - lref) : 0.f;
             if (lane < 32) wu[lane] = __expf(fminf(lref - sl[row0 + lane], 0.f));
             __syncthreads();
-            if (hh + 1 < a.hps) issue_tiles(h + 1, buf ^ 1);
+            if (hh + 1 < hps) issue_tiles(h + 1, buf ^ 1);
             else if constexpr (FINISH) issue_dg(buf ^ 1);
             tiles_dot(buf, bhc, Lam);
             const T* cS = tiles + buf * TILES;
@@ -375,14 +375,14 @@ ssd_bwd16_kernel(const Bwd16Args a) {
                     else sCw[((jn - JCR) * 4 + q) * 64 + lane] = v;
                 }
         }
-        for (int64_t hh = 0; hh < a.hps; ++hh) {
+        for (int64_t hh = 0; hh < hps; ++hh) {
             const int64_t h = h_first + hh;
             const int buf = (int)(hh & 1);
             wait_vmem_all();
             const float* sl = sLD + buf * 2 * kQ;
             const float* sd = sl + kQ;
             __syncthreads();
-            if (hh + 1 < a.hps) issue_tiles(h + 1, buf ^ 1);
+            if (hh + 1 < hps) issue_tiles(h + 1, buf ^ 1);
             else if constexpr (FINISH) issue_dg(buf ^ 1);
             // lane-dependent LDS offsets are rebuilt from the lane number for every head (a few integer instructions):
             // carried across the head loop they are spilled, and every reload waits for the tile copies in flight
@@ -461,8 +461,8 @@ ssd_bwd16_kernel(const Bwd16Args a) {
         }
         if constexpr (FINISH) {
             fetch_operands();
-            const char* dg = reinterpret_cast<const char*>(tiles + (a.hps & 1) * TILES);
-            const char* ops = reinterpret_cast<const char*>(tiles + ((a.hps - 1) & 1) * TILES);
+            const char* dg = reinterpret_cast<const char*>(tiles + (hps & 1) * TILES);
+            const char* ops = reinterpret_cast<const char*>(tiles + ((hps - 1) & 1) * TILES);
             // acc[tok][n] += sum_k dG[tok][k] B[k][n], or dG[k][tok] C[k][n]
             auto finish = [&](floatx16 (&acc)[1][NBN], auto side, const char* tile, T* out) {
                 constexpr bool SIDE_B = decltype(side)::value;

@@ -28,7 +28,7 @@ template <typename T, int P, int HS>
 __global__ void __launch_bounds__(kDgWaves * 64)
 dg16_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
             const T* __restrict__ dY, const float* __restrict__ Gf, float* __restrict__ dGp, float* __restrict__ dl_diag,
-            int64_t seqlen, int64_t nheads, int64_t ngroups, int64_t nchunks, int64_t nslices, int64_t hps,
+            int64_t seqlen, int64_t nheads, int64_t ngroups, int64_t nchunks, int64_t nslices, int64_t most_heads,
             int64_t Xsb, int64_t Xsl, int64_t Xsh, int64_t dYsb, int64_t dYsl, int64_t dYsh) {
     static_assert(sizeof(T) == 2, "16-bit operands only");
     constexpr int SPR = P / 8;                    // 16-byte slots per tile row
@@ -81,7 +81,7 @@ dg16_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
         }
         if (wave_u == 8) async_copy_ldtab(ldtab, (b * nheads + h) * nchunks + c, lds_LD + (uint32_t)(buf * 2 * kQ * 4));
     };
-    const int64_t h_first = g * hpg + slice * hps;
+    const int64_t h_first = g * hpg + slice * most_heads, hps = slice_heads(hpg, slice, most_heads);
 #pragma unroll
     for (int j = 0; j < RING - 1; ++j)
         if (j < hps) issue_tiles(h_first + j, j);

@@ -145,7 +145,7 @@ chunk_state32_kernel(const ChunkState32Args a) {
     const int lane = threadIdx.x & 63, r = lane & 31, half = lane >> 5;
     const int wave = (int)uniform(threadIdx.x >> 6), pb = wave & 1, nb = wave >> 1;
     const int64_t c = blockIdx.x, b = blockIdx.z, g = blockIdx.y / a.nslices, slice = blockIdx.y % a.nslices;
-    const int64_t t0 = c * kQ, h0 = g * (a.nheads / a.ngroups) + slice * a.hps;
+    const int64_t t0 = c * kQ, hpg = a.nheads / a.ngroups, h0 = g * hpg + slice * a.hps, hps = slice_heads(hpg, slice, a.hps);
     const int valid = (int)(a.seqlen - t0 < kQ ? a.seqlen - t0 : kQ);
     TileCopy32<kQ, P, WAVES> cp;
     cp.set(wave, a.X_sl, valid);
@@ -166,7 +166,7 @@ chunk_state32_kernel(const ChunkState32Args a) {
             }
     }
     issue(h0, 0);
-    for (int64_t hh = 0; hh < a.hps; ++hh) {
+    for (int64_t hh = 0; hh < hps; ++hh) {
         const int buf = (int)(hh & 1);
         wait_vmem_all();
         {
@@ -176,7 +176,7 @@ chunk_state32_kernel(const ChunkState32Args a) {
             wsc[lane + 64] = DSTATE ? (lane + 64 < valid ? __expf(lb) : 0.f) : sl[kQ + lane + 64] * __expf(Lam - lb);
         }
         __syncthreads();      // the tile is whole, and everyone is done with the other buffer
-        if (hh + 1 < a.hps) issue(h0 + hh + 1, buf ^ 1);
+        if (hh + 1 < hps) issue(h0 + hh + 1, buf ^ 1);
         const float* tx = sX + buf * kQ * P;
         const int lane = lane_here(), r = lane & 31, half = lane >> 5;
         floatx16 acc[1][1];
@@ -208,7 +208,7 @@ ssd_y32_kernel(const YArgs a) {
     const int wave = (int)uniform(threadIdx.x >> 6), rb = wave < 4 ? wave : 7 - wave, pb = wave >> 2, row0 = rb * 32, tok = row0 + r;
     float* wv = sLD + 2 * 2 * kQ + wave * kQ;            // this wave's v
     const int64_t c = blockIdx.x, b = blockIdx.z, g = blockIdx.y / a.nslices, slice = blockIdx.y % a.nslices;
-    const int64_t t0 = c * kQ, h0 = g * (a.nheads / a.ngroups) + slice * a.hps;
+    const int64_t t0 = c * kQ, hpg = a.nheads / a.ngroups, h0 = g * hpg + slice * a.hps, hps = slice_heads(hpg, slice, a.hps);
     const int valid = (int)(a.seqlen - t0 < kQ ? a.seqlen - t0 : kQ);
     TileCopy32<P, N, 8> cs;
     TileCopy32<kQ, P, 8> cx;
@@ -231,7 +231,7 @@ ssd_y32_kernel(const YArgs a) {
             if (u < 4 * rb + 4) fd[u] = *reinterpret_cast<const floatx4*>(Gp + op32_offset<16>(rb, u, lane));
     }
     issue(h0, 0);
-    for (int64_t hh = 0; hh < a.hps; ++hh) {
+    for (int64_t hh = 0; hh < hps; ++hh) {
         const int64_t h = h0 + hh;
         const int buf = (int)(hh & 1);
         const float Dh = a.D ? load_uniform_f32(a.D + (h >> HS)) : 0.f;
@@ -243,7 +243,7 @@ ssd_y32_kernel(const YArgs a) {
         wv[lane] = lane < row0 + 32 ? __expf(lref - sl[lane]) * sd[lane] : 0.f;
         wv[lane + 64] = lane + 64 < row0 + 32 ? __expf(lref - sl[lane + 64]) * sd[lane + 64] : 0.f;
         __syncthreads();      // the tiles are whole, and everyone is done with the other buffers
-        if (hh + 1 < a.hps) issue(h + 1, buf ^ 1);
+        if (hh + 1 < hps) issue(h + 1, buf ^ 1);
         const float* tS = sS + buf * P * N;
         const float* tX = sX + buf * kQ * P;
         const int lane = lane_here(), r = lane & 31, half = lane >> 5, tok = row0 + r;
@@ -380,7 +380,7 @@ ssd_bwd32_kernel(const Bwd32Args a) {
     float* wv = tabs + wave * (kQ + 64);
     float* wg = wv + kQ;
     const int64_t c = blockIdx.x, b = blockIdx.z, g = blockIdx.y / a.nslices, slice = blockIdx.y % a.nslices;
-    const int64_t t0 = c * kQ, h0 = g * (a.nheads / a.ngroups) + slice * a.hps, grp = (b * a.nchunks + c) * a.ngroups + g;
+    const int64_t t0 = c * kQ, hpg = a.nheads / a.ngroups, h0 = g * hpg + slice * a.hps, hps = slice_heads(hpg, slice, a.hps), grp = (b * a.nchunks + c) * a.ngroups + g;
     const int valid = (int)(a.seqlen - t0 < kQ ? a.seqlen - t0 : kQ);
 
     TileCopy32<P, N, 8> cs;
@@ -425,9 +425,9 @@ ssd_bwd32_kernel(const Bwd32Args a) {
 
     wait_vmem_all();
     __syncthreads();
-    for (int64_t hh = 0; hh < a.hps; ++hh) {
+    for (int64_t hh = 0; hh < hps; ++hh) {
         const int64_t h = h0 + hh, bhc = (b * a.nheads + h) * a.nchunks + c;
-        const bool more = hh + 1 < a.hps;
+        const bool more = hh + 1 < hps;
         const float Dh = a.D ? load_uniform_f32(a.D + (h >> HS)) : 0.f;
         const float* sl = sLD + (hh & 1) * 2 * kQ;
         const float* sd = sl + kQ;

@@ -39,8 +39,10 @@ struct SsdWorkspace {
 };
 
 // A workgroup owns one chunk of one group and loops over a slice of that group's heads (operands shared by the
-// group stay on chip, group-level reductions happen in registers).  The slice count is the divisor of heads-per-group with the
-// least of: workgroups on the busiest CU times heads per slice -- a CU that could hold two (`wgs_per_cu`) and has one takes three
+// group stay on chip, group-level reductions happen in registers).  The slices have equal numbers of heads but the last, which has
+// what is left (with divisors of the heads per group only, a prime count had one head a slice or all of them: forward and backward at
+// b3 l1111 h31 166 -> 102 us, b1 l2130 h106 406 -> 266, fp32 b4 l416 h83 346 -> 258).  Their count is the one with the least of:
+// workgroups on the busiest CU times heads per slice -- a CU that could hold two (`wgs_per_cu`) and has one takes three
 // quarters of two's time --, 1.5 heads' worth for filling and draining each of them, and, `partials`, what the slices' partial
 // sums cost on their way out and back (128 KiB each: a head's worth per 110 workgroups).  Taking whatever first filled the chip
 // instead left a nearly empty last round and twice the partials at b3 l1111 h32: main backward kernel 41 -> 31 us, dG 17.7 ->
@@ -53,13 +55,14 @@ inline void ssd_slicing(const SsdCall* p, int wgs_per_cu, bool partials, int64_t
     int64_t best = 1;
     float least = 1e30f;
     for (int64_t s = 1; s <= hpg; ++s) {
-        if (hpg % s) continue;
+        const int64_t heads = ceil_div(hpg, s);
+        if (ceil_div(hpg, heads) != s) continue;      // fewer slices hold them
         const float n = (float)ceil_div(base * s, cus), busy = n < (float)wgs_per_cu ? 0.75f * (float)wgs_per_cu : n;
-        const float cost = busy * (float)(hpg / s) + 1.5f * n + (partials ? 0.009f * (float)(base * s) : 0.f);
+        const float cost = busy * (float)heads + 1.5f * n + (partials ? 0.009f * (float)(base * s) : 0.f);
         if (cost < least) { least = cost; best = s; }
     }
     *nslices = best;
-    *hps = hpg / best;
+    *hps = ceil_div(hpg, best);
 }
 constexpr int kWgsChunkState32 = 2, kWgsY = 2, kWgsY32 = 1, kWgsDx = 1, kWgsDg = 1;
 
@@ -71,12 +74,13 @@ inline void ssd_slicing32(const SsdCall* p, int64_t* nslices, int64_t* hps) {
     int64_t best = 1;
     float least = 1e30f;
     for (int64_t s = 1; s <= hpg; ++s) {
-        if (hpg % s) continue;
-        const float cost = (float)ceil_div(base * s, device_cus()) * ((float)(hpg / s) + 1.f) + (s > 1 ? 1.f + 0.007f * (float)(base * s) : 0.f);
+        const int64_t heads = ceil_div(hpg, s);
+        if (ceil_div(hpg, heads) != s) continue;
+        const float cost = (float)ceil_div(base * s, device_cus()) * ((float)heads + 1.f) + (s > 1 ? 1.f + 0.007f * (float)(base * s) : 0.f);
         if (cost < least) { least = cost; best = s; }
     }
     *nslices = best;
-    *hps = hpg / best;
+    *hps = ceil_div(hpg, best);
 }
 
 inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_only = false) {

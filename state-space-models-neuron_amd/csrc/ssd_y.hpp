@@ -193,7 +193,7 @@ ssd_y16_kernel(const YArgs a) {
         async_copy_ldtab(a.ldtab, (b * a.nheads + h) * a.nchunks + c, lds_LD + (uint32_t)(buf * 2 * kQ * 4));
     };
 
-    const int64_t h_first = g * hpg + slice * a.hps;
+    const int64_t h_first = g * hpg + slice * a.hps, hps = slice_heads(hpg, slice, a.hps);
     issue_tiles(h_first, 0);
 
     // ---- head-independent operands, resident in registers
@@ -215,7 +215,7 @@ ssd_y16_kernel(const YArgs a) {
         }
     }
 
-    for (int64_t hh = 0; hh < a.hps; ++hh) {
+    for (int64_t hh = 0; hh < hps; ++hh) {
         const int64_t h = h_first + hh;
         const int buf = (int)(hh & 1);
         const float Dh = a.D ? load_uniform_f32(a.D + (h >> HS)) : 0.f;
@@ -234,7 +234,7 @@ ssd_y16_kernel(const YArgs a) {
         wv[lane + 64] = lane + 64 < row0 + 32 ? __expf(lref - sl[lane + 64]) * sd[lane + 64] : 0.f;
         if (lane < 32) wu[lane] = __expf(fminf(sl[row0 + lane] - lref, 0.f));
         __syncthreads();          // everyone's share has landed; every wave is also done with head hh-1 (the other buffer)
-        if (hh + 1 < a.hps) issue_tiles(h + 1, buf ^ 1);
+        if (hh + 1 < hps) issue_tiles(h + 1, buf ^ 1);
         const T* cS = sS + buf * (P * N);
         const T* cX = sX + buf * (kQ * P);
 

@@ -393,3 +393,11 @@ def test_prefill_states_in_segments_in_place(l, cut, h, n):
     def l2(a, b):
         return float((a.double() - b.double()).norm() / b.double().norm())
     assert torch.equal(c1, c2) and l2(y1, y2) < 2.0 ** -7 and l2(S1, S2) < 2.0 ** -12, (l2(y1, y2), l2(S1, S2))
+
+
+# head counts that no useful number of slices divides: the last slice has one head of two, four of five, one of three; wide heads as pairs
+@pytest.mark.parametrize("b,l,h,p,n,g", [(16, 129, 11, 64, 128, 1), (40, 130, 14, 64, 64, 1), (20, 129, 14, 64, 128, 2), (40, 129, 7, 128, 64, 1)])
+def test_ssd_last_slice_of_fewer_heads(b, l, h, p, n, g):
+    test_ssd_forward(torch.bfloat16, b, l, h, p, n, g)
+    test_ssd_bf16_whole_groups(b, l, h, p, n, g)
+    test_ssd_fp32_heads_in_sequence(b, l, h, p, n, g, "usual")
