@@ -34,7 +34,7 @@
 //                                                                partial state parts of dB / dC
 //   [ssd_bwd32_kernel         what those two do in one pass; dB and dC too where a workgroup has all heads of its group]
 //   tail1_kernel              da_body: ddt, dA partials per (b, head, chunk);  slice_sum_body: partials over the head slices
-//   tail2_kernel              group_finish16_body per (b, chunk, group, token block) [bc_final32_body per (b, chunk, group)], unless done
+//   tail2_kernel              group_finish16_body per (b, chunk, group, token block) [bc_final32_body per (b, chunk, group, side)], unless done
 //                             already: dC = dG B + dCoff, dB = dG^T C + dBoff;  ad_reduce_body per head: dA, dD (fixed order, no atomics)
 #include "ssd_host.hpp"
 
@@ -207,10 +207,14 @@ __global__ void __launch_bounds__(512)
 tail2_32_kernel(const Tail2Args32 a) {
     const int64_t blk = blockIdx.x;
     if (blk < a.n_bc) {
-        const int64_t c = blk % a.nchunks, g = (blk / a.nchunks) % a.ngroups, b = blk / (a.nchunks * a.ngroups);
-        bc_final32_body<N>(a.dGp, a.dCp, a.dBp, static_cast<const float*>(a.B), a.Bsb, a.Bsl, a.Bsg, static_cast<const float*>(a.C), a.Csb, a.Csl, a.Csg,
-                           static_cast<float*>(a.dB), a.dBsb, a.dBsl, a.dBsg, static_cast<float*>(a.dC), a.dCsb, a.dCsl, a.dCsg, a.seqlen, a.ngroups,
-                           a.nchunks, c, g, b);
+        const int64_t grp = blk >> 1, c = grp % a.nchunks, g = (grp / a.nchunks) % a.ngroups, b = grp / (a.nchunks * a.ngroups);
+        auto finish = [&](auto side) {
+            bc_final32_body<N, decltype(side)::value>(a.dGp, a.dCp, a.dBp, static_cast<const float*>(a.B), a.Bsb, a.Bsl, a.Bsg, static_cast<const float*>(a.C), a.Csb,
+                                                      a.Csl, a.Csg, static_cast<float*>(a.dB), a.dBsb, a.dBsl, a.dBsg, static_cast<float*>(a.dC), a.dCsb, a.dCsl, a.dCsg,
+                                                      a.seqlen, a.ngroups, a.nchunks, c, g, b);
+        };
+        if (blk & 1) finish(std::integral_constant<int, 2>{});
+        else finish(std::integral_constant<int, 1>{});
     } else {
         ad_reduce_body(a.dAp, a.dDp, a.dbp, a.dA, a.dD, a.dbias, a.batch, a.nheads, a.nchunks, blk - a.n_bc);
     }
@@ -347,10 +351,10 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
             ta.Bsb = p->B_stride_b; ta.Bsl = p->B_stride_l; ta.Bsg = p->B_stride_g; ta.Csb = p->C_stride_b; ta.Csl = p->C_stride_l; ta.Csg = p->C_stride_g;
             ta.dBsb = p->dB_stride_b; ta.dBsl = p->dB_stride_l; ta.dBsg = p->dB_stride_g;
             ta.dCsb = p->dC_stride_b; ta.dCsl = p->dC_stride_l; ta.dCsg = p->dC_stride_g;
-            ta.n_bc = n_bc;
+            ta.n_bc = 2 * n_bc;
             auto k = tail2_32_kernel<N>;
             if ((rc = allow_smem(k, finish32_smem<N>()))) return rc;
-            k<<<(unsigned)(n_bc + p->true_heads), 512, n_bc ? finish32_smem<N>() : 0, st>>>(ta);
+            k<<<(unsigned)(2 * n_bc + p->true_heads), 512, n_bc ? finish32_smem<N>() : 0, st>>>(ta);
         }
         if ((rc = check_launch("ssd tail2_kernel"))) return rc;
     }

@@ -317,25 +317,29 @@ template <int N> constexpr size_t bwd32_smem() { return (size_t)(2 * kQ * kP + 2
 
 // The group-level finish of one (batch, chunk, group):  dC[i] += sum_{j<=i} dG[i][j] B[j],  dB[j] += sum_{i>=j} dG[i][j] C[i].
 // dG lies in sG ([kQ][kQ], swizzled; blocks above the diagonal are not read), sM takes B and then C.  Wave: row block rb, column
-// blocks nb0 .. nb0 + NBW - 1 of both sides, a token per lane.
-template <int N, int NBW>
+// blocks nb0 .. nb0 + NBW - 1, a token per lane.  SIDES: 1 dC, 2 dB, 3 both, one behind the other.
+template <int N, int NBW, int SIDES = 3>
 __device__ __forceinline__ void finish32(const float* sG, float* sM, floatx16 (&accB)[NBW], floatx16 (&accC)[NBW], const float* Bp, int64_t B_sl, const float* Cp,
                                          int64_t C_sl, float* dB, int64_t dB_sl, float* dC, int64_t dC_sl, int valid, int wave, int rb, int nb0) {
     const int lane = threadIdx.x & 63, r = lane & 31, half = lane >> 5, tok = rb * 32 + r;
     const uint32_t lds_M = uniform(lds_addr_of(sM));
     TileCopy32<kQ, N, 8> cp;
-    cp.set(wave, B_sl, valid);
-    cp.issue(Bp, wave, lds_M);
-    wait_vmem_all();
-    __syncthreads();      // dG and B are there
     auto m = [&](int u, int q) { return col_step32<N>(sM, (nb0 + q) * 32 + r, half, u); };
-    by_row_block(rb, [&](auto k) {
-        products32<NBW, false, 1>(accC, 0, 4 * decltype(k)::value + 4, [&](int u) { return row_step32<kQ>(sG, tok, half, u); }, NoScale32{}, m, NoLast32{});
-    });
-    __syncthreads();      // everyone is done with B
-    cp.set(wave, C_sl, valid);
-    cp.issue(Cp, wave, lds_M);
-    if (tok < valid) {
+    if constexpr (SIDES & 1) {
+        cp.set(wave, B_sl, valid);
+        cp.issue(Bp, wave, lds_M);
+        wait_vmem_all();
+        __syncthreads();      // dG and B are there
+        by_row_block(rb, [&](auto k) {
+            products32<NBW, false, 1>(accC, 0, 4 * decltype(k)::value + 4, [&](int u) { return row_step32<kQ>(sG, tok, half, u); }, NoScale32{}, m, NoLast32{});
+        });
+        if (SIDES & 2) __syncthreads();      // everyone is done with B
+    }
+    if constexpr (SIDES & 2) {
+        cp.set(wave, C_sl, valid);
+        cp.issue(Cp, wave, lds_M);
+    }
+    if ((SIDES & 1) && tok < valid) {
         float* o = dC + tok * dC_sl + nb0 * 32 + 4 * half;
 #pragma unroll
         for (int q = 0; q < NBW; ++q)
@@ -343,6 +347,7 @@ __device__ __forceinline__ void finish32(const float* sG, float* sM, floatx16 (&
             for (int v = 0; v < 4; ++v)
                 *reinterpret_cast<floatx4*>(o + q * 32 + 8 * v) = floatx4{accC[q][4 * v], accC[q][4 * v + 1], accC[q][4 * v + 2], accC[q][4 * v + 3]};
     }
+    if constexpr (!(SIDES & 2)) return;
     wait_vmem_all();
     __syncthreads();
     by_row_block(rb, [&](auto k) {
@@ -688,9 +693,11 @@ ssd_bwd32_kernel(const Bwd32Args a) {
         }
 }
 
-// The finish from partials that are already summed over the head slices: one workgroup of 512 threads per (batch, chunk, group).
+// The finish from partials that are already summed over the head slices: a workgroup of 512 threads per (batch, chunk, group) and side.
+// It is one chain of memory latencies, a CU to itself (128 KiB of LDS): both sides in one workgroup took 22.5 us at b1 l785 g2 and
+// at b1 l347 g1, 12.5 a side (and 12.5 for both, side by side).
 template <int N> constexpr size_t finish32_smem() { return (size_t)(kQ * kQ + kQ * N) * sizeof(float); }
-template <int N>
+template <int N, int SIDE>
 __device__ __forceinline__ void bc_final32_body(const float* dGs, const float* dCs, const float* dBs, const float* Bm, int64_t B_sb, int64_t B_sl, int64_t B_sg,
                                                 const float* Cm, int64_t C_sb, int64_t C_sl, int64_t C_sg, float* dB, int64_t dB_sb, int64_t dB_sl, int64_t dB_sg,
                                                 float* dC, int64_t dC_sb, int64_t dC_sl, int64_t dC_sg, int64_t seqlen, int64_t ngroups, int64_t nchunks,
@@ -704,22 +711,31 @@ __device__ __forceinline__ void bc_final32_body(const float* dGs, const float* d
     const int64_t t0 = c * kQ, grp = (b * nchunks + c) * ngroups + g;
     const int valid = (int)(seqlen - t0 < kQ ? seqlen - t0 : kQ);
     const float* gp = dGs + grp * (int64_t)(kQ * kQ);
+    // every load out before the first is waited for; pieces above the diagonal: the row's first in their place
+    constexpr int PIECES = kQ * kQ / 4 / 512;
+    floatx4 gv[PIECES];
 #pragma unroll
-    for (int it = 0; it < kQ * kQ / 4 / 512; ++it) {
+    for (int it = 0; it < PIECES; ++it) {
         const int e = it * 512 + tid, i = e / (kQ / 4), s = e % (kQ / 4);
-        if ((s >> 3) <= (i >> 5)) *reinterpret_cast<floatx4*>(sG + i * kQ + ((s ^ (i & 15)) * 4)) = *reinterpret_cast<const floatx4*>(gp + i * kQ + s * 4);
+        gv[it] = *reinterpret_cast<const floatx4*>(gp + i * kQ + ((s >> 3) <= (i >> 5) ? s : 0) * 4);
     }
-    floatx16 accB[NBW], accC[NBW];
+    floatx16 acc[NBW];
     const int64_t o = grp * (int64_t)(kQ * N) + tok * N + nb0 * 32 + 4 * half;
+    const float* part = (SIDE == 1 ? dCs : dBs) + o;
 #pragma unroll
     for (int q = 0; q < NBW; ++q)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const floatx4 cb = *reinterpret_cast<const floatx4*>(dBs + o + q * 32 + 8 * v), cc = *reinterpret_cast<const floatx4*>(dCs + o + q * 32 + 8 * v);
+            const floatx4 p = *reinterpret_cast<const floatx4*>(part + q * 32 + 8 * v);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { accB[q][4 * v + e] = cb[e]; accC[q][4 * v + e] = cc[e]; }
+            for (int e = 0; e < 4; ++e) acc[q][4 * v + e] = p[e];
         }
-    finish32<N, NBW>(sG, sM, accB, accC, Bm + b * B_sb + t0 * B_sl + g * B_sg, B_sl, Cm + b * C_sb + t0 * C_sl + g * C_sg, C_sl,
+#pragma unroll
+    for (int it = 0; it < PIECES; ++it) {
+        const int e = it * 512 + tid, i = e / (kQ / 4), s = e % (kQ / 4);
+        if ((s >> 3) <= (i >> 5)) *reinterpret_cast<floatx4*>(sG + i * kQ + ((s ^ (i & 15)) * 4)) = gv[it];
+    }
+    finish32<N, NBW, SIDE>(sG, sM, acc, acc, Bm + b * B_sb + t0 * B_sl + g * B_sg, B_sl, Cm + b * C_sb + t0 * C_sl + g * C_sg, C_sl,
                      dB + b * dB_sb + t0 * dB_sl + g * dB_sg, dB_sl, dC + b * dC_sb + t0 * dC_sl + g * dC_sg, dC_sl, valid, wave, rb, nb0);
 }
 
