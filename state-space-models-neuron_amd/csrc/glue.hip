@@ -358,12 +358,6 @@ int norm_lanes(int64_t nvec, int64_t groups) {
 // columns of a launch's grid
 int64_t norm_columns(int64_t nvec, int64_t groups) { return ceil_div(groups, (int64_t)(64 / norm_lanes(nvec, groups))); }
 
-// What a workspace has room for: a backward of about 512 workgroups of at least 4 rows each.
-int64_t norm_rows_per_block(int64_t rows, int64_t groups) {
-    int64_t rb = rows * groups / 512;
-    if (rb < 4) rb = 4;
-    return (rb + 3) / 4 * 4;
-}
 // Rows per workgroup.  A workgroup (or, with a wave per row, each of its four waves) is a chain of rows, dealt round-robin, and the chip
 // likes one or two of them per CU: with a few more (834 of four rows for 3333) a second round is nearly empty, and in the backward every
 // one leaves a partial row of dw.  Workgroups per CU, from 180 sizes (300 to 26000 rows, groups of 512 to 7168 channels, both types;
@@ -379,7 +373,7 @@ int64_t norm_rows_per_block(int64_t rows, int64_t groups) {
 //     | 29.5, backward 51.7 | 48.0 | 58.5 | 52.9
 int64_t norm_rows_per_workgroup(int64_t rows, int64_t groups, int64_t nvec, int vec_elems, bool bwd) {
     int wpg = 1, nv = 1;
-    if (!norm_shape(nvec, vec_elems, &wpg, &nv)) return norm_rows_per_block(rows, groups);
+    if (!norm_shape(nvec, vec_elems, &wpg, &nv)) return ceil_div(rows, (int64_t)512);      // refused before any launch
     const int64_t all = rows * norm_columns(nvec, groups);
     const bool exact = (int64_t)wpg * 64 * nv == nvec;
     int64_t per_cu = 1;
@@ -650,12 +644,13 @@ extern "C" int m2_core_norm_fwd(const m2_rmsnorm_params* p, void* stream) { retu
 
 extern "C" size_t m2_rmsnorm_gated_bwd_workspace_bytes(int64_t rows, int64_t channels, int32_t n_groups, int32_t dtype) {
     if (rows <= 0 || channels <= 0 || n_groups <= 0) return 256;
-    // A partial row per workgroup.  Where one workgroup per compute unit runs, room for the general rule's count (about 512) is
-    // asked for all the same: a size that followed the units would depend on the device that is current when it is asked for, and
-    // a caller may size its scratch without one.
+    // A partial row per workgroup.  The rule gives a column of the grid at most 512 of them on 256 compute units, and room for as many is
+    // asked for whatever it gives here: a size that followed the units would depend on the device that is current when it is asked
+    // for, and a caller may size its scratch without one.
     const int V = dtype == M2_F32 ? 4 : 8;
-    const int64_t used = m2::ceil_div(rows, m2::norm_rows_per_workgroup(rows, n_groups, channels / n_groups / V, V, true));
-    const int64_t most = m2::ceil_div(rows, m2::norm_rows_per_block(rows, n_groups));
+    const int64_t nvec = channels / n_groups / V, per_column = m2::ceil_div((int64_t)512, m2::norm_columns(nvec, n_groups));
+    const int64_t used = m2::ceil_div(rows, m2::norm_rows_per_workgroup(rows, n_groups, nvec, V, true));
+    const int64_t most = rows < per_column ? rows : per_column;
     return m2::align_up((size_t)(used > most ? used : most) * (size_t)channels * sizeof(float), 256);
 }
 
