@@ -7,7 +7,8 @@
 //
 //   1. prep_kernel         l = cumsum(A dt) per (b, head, chunk);  G = C B^T (+ operand tiles) per (b, chunk, group)
 //   2. states entering the chunks, final state
-//        16-bit: state_pass16_kernel   contributions B^T (decay o dt o X) and recurrence fused, per (b, head)
+//        16-bit: state_pass16_kernel   contributions B^T (decay o dt o X) and recurrence fused, per (b, head);
+//                two launches over segments of the sequence where the heads are few
 //        fp32  : chunk_state32_kernel + state_scan_kernel
 //   3. ssd_y16_kernel / ssd_y32_kernel      Y = (L o G)(dt o X) + e^l C S_prev + D X   MFMA
 //
