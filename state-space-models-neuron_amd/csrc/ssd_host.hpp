@@ -196,9 +196,11 @@ inline int launch_state_pass16(StatePassArgs a, const SsdWorkspace& w, int64_t b
         k<<<dim3((unsigned)(a.nheads * split), (unsigned)batch, (unsigned)segs), state_pass_threads<N>(), sm, st>>>(a);
         return M2_OK;
     };
+    const bool staged = state_pass_staged(a.init != nullptr, a.nchunks);
     if constexpr (N == 128 && !HILO)
         if (state_pass_split(batch * a.nheads, N) == 1)
-            return launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, 1>, state_pass_smem<P, N, HILO, 1>(), 1);
+            return staged ? launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, 1, 0, true>, state_pass_smem<P, N, HILO, 1>(), 1) :
+                            launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, 1>, state_pass_smem<P, N, HILO, 1>(), 1);
     constexpr int SPLIT = kStatePassSplit;
     if (const int64_t m = state_pass_seg_chunks(batch * a.nheads, a.nchunks)) {
         a.seg = static_cast<floatx4*>(w.seg); a.seg_lam = w.seg_lam; a.seg_chunks = m;
@@ -207,7 +209,8 @@ inline int launch_state_pass16(StatePassArgs a, const SsdWorkspace& w, int64_t b
         if (!rc) rc = check_launch("ssd state_pass16_kernel, sums of segments");
         return rc ? rc : launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, SPLIT, 2>, state_pass_smem<P, N, HILO, SPLIT>(), SPLIT, sums);
     }
-    return launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, SPLIT>, state_pass_smem<P, N, HILO, SPLIT>(), SPLIT);
+    return staged ? launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, SPLIT, 0, true>, state_pass_smem<P, N, HILO, SPLIT>(), SPLIT) :
+                    launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, SPLIT>, state_pass_smem<P, N, HILO, SPLIT>(), SPLIT);
 }
 
 // Local chunk states of fp32 operands: X = x, M = B, or (DSTATE) dy and C.

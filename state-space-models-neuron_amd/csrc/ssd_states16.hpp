@@ -68,6 +68,11 @@ inline int64_t state_pass_seg_chunks(int64_t heads, int64_t nchunks) {
     const int64_t chunks = ceil_div(nchunks, sets + 1);
     return chunks < 2 ? 2 : chunks;
 }
+// Lane by lane, an instruction that reads the initial state touches 32 rows for 32 bytes each.  STAGED takes whole rows through LDS, but its
+// loop comes out of the compiler about 20 ns a chunk slower.  Whole prefill core with 80 heads of 64 x 128 states behind a cached prefix, us, as
+// lanes -> staged: 8 x 1 chunk 57.4 -> 50.1, 8 x 3 91.1 -> 83.5, 1 x 8 48.3 -> 47.6, 1 x 32 115.2 -> 115.0, 4 x 32 380.0 -> 377.1, 1 x 64 221.9 ->
+// 222.9, 1 x 128 424.8 -> 426.8.
+inline bool state_pass_staged(bool init, int64_t nchunks) { return init && nchunks <= 32; }
 // one wave per 32 state columns
 template <int N> constexpr int state_pass_threads() { return (N / 32) * 64; }
 template <int P, int N, bool HILO = false, int SPLIT = kStatePassSplit>
@@ -78,10 +83,11 @@ constexpr size_t state_pass_smem() {
 // HILO: the scaled rows are staged as TWO 16-bit tiles, the rounded value and the rounded remainder, and each k step takes
 // two products, so that the fp32 scale dt e^{Lam - l} reaches the accumulators with 16 significand bits instead of 8 (the
 // final state is an fp32 output; with one tile its error is that of the operand rounding, 2^-9 of every term).
+// STAGED: the initial state comes as whole rows through the slab tiles (see state_pass_staged).
 // PHASE 0: the whole sequence.  1: segment z, up to the last but one, from the initial state (the first, whose states are stored) or from
 // zero, to `seg` and `seg_lam`.  2: segment z + 1 from what `seg` holds for those in front of it.  Segments count in the order of the walk.
 // The initial state is read in the first launch only and the final one written in the second: they may be the same tensor.
-template <typename T, int P, int N, bool REVERSE, int HS, bool HILO = false, int SPLIT = kStatePassSplit, int PHASE = 0>
+template <typename T, int P, int N, bool REVERSE, int HS, bool HILO = false, int SPLIT = kStatePassSplit, int PHASE = 0, bool STAGED = false>
 __global__ void __launch_bounds__(state_pass_threads<N>(), SPLIT == 1 ? 2 : 3)
 state_pass16_kernel(const StatePassArgs a) {
     static_assert(sizeof(T) == 2, "16-bit operands only");
@@ -126,15 +132,44 @@ state_pass16_kernel(const StatePassArgs a) {
     const int64_t seg_pitch = (int64_t)gridDim.y * a.nheads * (P * N / 4);
     floatx4* const seg_q = PHASE == 0 ? nullptr : a.seg + ((bh * SPLIT + pw) * NWAVES + wave_u) * (PBW * NBW * 4 * 64) + lane;
     const float* init = PHASE == 0 || (PHASE == 1 && seg == 0) ? a.init : nullptr;
+    static_assert(!STAGED || PHASE == 0, "a whole walk");
+    constexpr int NI = PH * N / 4 / THREADS, CV = N / 4;
+    typedef float AnyFloat4 __attribute__((ext_vector_type(4), aligned(4)));      // a caller's tensor: any element
+    [[maybe_unused]] floatx4 first[NI];
+    if constexpr (STAGED) {
 #pragma unroll
-    for (int i = 0; i < PBW; ++i)
+        for (int it = 0; it < NI; ++it) first[it] = *reinterpret_cast<const AnyFloat4*>(init + bh * (P * N) + pw * (PH * N) + (it * THREADS + tid) * 4);
+    } else {
 #pragma unroll
-        for (int j = 0; j < NBW; ++j)
+        for (int i = 0; i < PBW; ++i)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int row = pw * PH + i * 32 + r, col = n0 + j * 32 + acc_row(lane, v);
-                acc[i][j][v] = init ? init[bh * (P * N) + row * N + col] : 0.f;
-            }
+            for (int j = 0; j < NBW; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int row = pw * PH + i * 32 + r, col = n0 + j * 32 + acc_row(lane, v);
+                    acc[i][j][v] = init ? init[bh * (P * N) + row * N + col] : 0.f;
+                }
+    }
+    auto take_init = [&] {      // behind the first rows' loads
+        float* const sI = reinterpret_cast<float*>(sO);      // [PH][LDO]: the slab tiles are as large as the workgroup's rows in fp32
+#pragma unroll
+        for (int it = 0; it < NI; ++it) {
+            const int e = it * THREADS + tid;
+            *reinterpret_cast<floatx4*>(sI + e / CV * LDO + e % CV * 4) = first[it];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < PBW; ++i)
+#pragma unroll
+            for (int j = 0; j < NBW; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const floatx4 v = *reinterpret_cast<const floatx4*>(sI + (i * 32 + r) * LDO + n0 + j * 32 + 8 * q + 4 * half);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][j][4 * q + e] = v[e];
+                }
+        __syncthreads();      // the first state's tile is written over it
+    };
     if constexpr (PHASE == 2)
         for (int64_t t = 0; t < seg; ++t) {
             const float dec = t ? __expf(a.seg_lam[t * (int64_t)gridDim.y * a.nheads + bh]) : 0.f;      // nothing in front of the first
@@ -336,11 +371,15 @@ state_pass16_kernel(const StatePassArgs a) {
     if (nsteps & 1) {
         load_ahead(s1);
         load_ahead(s0);
+        if constexpr (STAGED) take_init();
         step(0, s1);
         cc = 1;
-    } else if (nsteps > 0) {
-        load_ahead(s0);
-        load_ahead(s1);
+    } else {
+        if (nsteps > 0) {
+            load_ahead(s0);
+            load_ahead(s1);
+        }
+        if constexpr (STAGED) take_init();
     }
 #pragma unroll 1
     for (; cc < nsteps; cc += 2) {

@@ -401,3 +401,24 @@ def test_ssd_last_slice_of_fewer_heads(b, l, h, p, n, g):
     test_ssd_forward(torch.bfloat16, b, l, h, p, n, g)
     test_ssd_bf16_whole_groups(b, l, h, p, n, g)
     test_ssd_fp32_heads_in_sequence(b, l, h, p, n, g, "usual")
+
+
+@pytest.mark.parametrize("b,l,h,p,n", [(2, 1, 3, 64, 128), (8, 129, 32, 64, 128), (2, 300, 3, 128, 64)])      # the second: whole heads per workgroup
+def test_ssd_initial_state_on_any_element(b, l, h, p, n):
+    """The state's rows come in 16-byte pieces: from a tensor that starts on any element the same bits, forward and backward."""
+    from mamba2.mamba2_kernel import mamba2_kernel
+    d = _dev(make_ssd_inputs(b, l, h, p, n, 1, seed=l, dtype=torch.bfloat16))
+    S0 = 0.1 * torch.randn(b, h, p, n, device=DEV)
+    odd = torch.empty(S0.numel() + 1, device=DEV)[1:].view_as(S0).copy_(S0)
+    got = []
+    for S in (S0, odd):
+        S = S.detach().requires_grad_(True)
+        X = d["X"].detach().requires_grad_(True)
+        y = mamba2_kernel(d["dt"], d["A"], X, d["B"], d["C"], d["D"], initial_state=S)
+        got.append((y, *torch.autograd.grad(y, [X, S], d["dy"])))
+    assert all(torch.equal(a, c) for a, c in zip(*got))
+
+
+def test_prefill_initial_state_of_a_long_walk():
+    """34 chunks behind a prefix, the state read lane by lane, against two pieces whose states come as rows."""
+    test_prefill_states_in_segments_in_place(4300, 2100, 40, 64)
