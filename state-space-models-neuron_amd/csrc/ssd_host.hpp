@@ -118,7 +118,7 @@ inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_
         w.kept_bytes = koff;
     }
     if (p->dtype != M2_F32)
-        if (const int64_t m = state_pass_seg_chunks(p->batch * p->nheads, nc)) {
+        if (const int64_t m = state_pass_seg_chunks(p->batch * p->nheads, nc, true)) {
             const size_t sums = (size_t)((ceil_div(nc, m) - 1) * p->batch * p->nheads);
             w.seg = take(sums * p->headdim * p->dstate * 4);
             w.seg_lam = reinterpret_cast<float*>(take(sums * 4));
@@ -202,7 +202,7 @@ inline int launch_state_pass16(StatePassArgs a, const SsdWorkspace& w, int64_t b
             return staged ? launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, 1, 0, true>, state_pass_smem<P, N, HILO, 1>(), 1) :
                             launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, 1>, state_pass_smem<P, N, HILO, 1>(), 1);
     constexpr int SPLIT = kStatePassSplit;
-    if (const int64_t m = state_pass_seg_chunks(batch * a.nheads, a.nchunks)) {
+    if (const int64_t m = state_pass_seg_chunks(batch * a.nheads, a.nchunks, HILO)) {
         a.seg = static_cast<floatx4*>(w.seg); a.seg_lam = w.seg_lam; a.seg_chunks = m;
         const int64_t sums = ceil_div(a.nchunks, m) - 1;
         int rc = launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, SPLIT, 1>, state_pass_smem<P, N, HILO, SPLIT>(), SPLIT, sums);

@@ -362,16 +362,16 @@ def test_ssd_gradients_without_the_initial_states_own(l, b, h, p, n, dtype):
     assert torch.equal(y1, y2) and all(torch.equal(a, c) for a, c in zip(g1, g2))
 
 
-# the state pass in segments: two chunks each and a last one with one; a whole last chunk and one with a single token; two columns of waves; 
-# three sets of workgroups in four segments of six chunks; wide heads; several sequences and groups
-@pytest.mark.parametrize("b,l,h,p,n,g", [(1, 1536, 2, 64, 128, 1), (1, 1665, 3, 128, 64, 1), (1, 3050, 42, 64, 64, 1), (2, 2944, 16, 64, 128, 2), (3, 2049, 4, 128, 128, 4)])
+# the state pass in segments: two chunks each; a whole last chunk and one with a single token; two columns of waves; 
+# three and four sets of workgroups, the forward with a final state alone in segments; wide heads; several sequences and groups
+@pytest.mark.parametrize("b,l,h,p,n,g", [(1, 6144, 2, 64, 128, 1), (1, 6017, 3, 128, 64, 1), (1, 4100, 42, 64, 64, 1), (2, 3000, 16, 64, 128, 2), (2, 6017, 4, 128, 128, 4)])
 def test_ssd_states_in_segments(b, l, h, p, n, g):
     """Few heads and many chunks: both recurrences, with and without the states at their ends."""
     test_ssd_packed_views_with_pad_columns_fwd_bwd(torch.bfloat16, b, l, h, p, n, g)
     test_ssd_gradients_without_the_initial_states_own(l, b, h, p, n, torch.bfloat16)
 
 
-@pytest.mark.parametrize("l,cut,h,n", [(1921, 900, 8, 128), (2560, 1280, 12, 64)])
+@pytest.mark.parametrize("l,cut,h,n", [(2561, 1200, 8, 128), (2560, 1280, 12, 64)])
 def test_prefill_states_in_segments_in_place(l, cut, h, n):
     """A long prompt behind a cached prefix, whose state is read and written in place, against the same prompt in two shorter pieces."""
     from mamba2.fused_kernel import mamba2_fused_prefill
