@@ -474,9 +474,12 @@ conv_reduce_partials_kernel(const float* __restrict__ part, int64_t nslots, int6
 // ------------------------------------------------------------------------------------------
 // Channel-major path, k == 4: tokens contiguous in x, y (and dx).
 //
-// N tokens of a row: one vector access.  Where the row's last vector is cut by its end, the lanes that hold it read the row's last N
-// tokens instead and move the ones that are theirs down: no lane's branch stands in front of a load.  (With one, a row's first and last
-// lanes made their whole wave wait for one load after the other.)
+// The kernels take N tokens of a row with one vector access.  Where the row's last vector is cut by its end, the lanes that hold it read the
+// row's last N tokens instead (ld_whole) and move the ones that are theirs down (move_down): no lane's branch stands in front of a load.
+// (With one, a row's first and last lanes made their whole wave wait for one load after the other.)  Rows shorter than a vector
+// (ld_short) have kernels of their own, WHOLE false: as a branch of the same kernel they made the others wait for the taps before they asked
+// for x (fp32 forward, b4 C256 l2048 5.0 us, 4.3 without).
+
 // `v` without its first `gone` tokens (the same number for the whole launch), zeros behind the others, in the lanes that `cut` says.
 // By words and then by half of one: a 64-bit shift by a lane's amount gave wrong high words here where the compiler had put the amount
 // into a wave's last register.
@@ -520,6 +523,19 @@ __device__ __forceinline__ Tokens<T, N> ld_short(const T* __restrict__ row, int6
     for (int i = 0; i < N; ++i) r[i] = (t + i >= 0 && t + i < l) ? row[t + i] : from_f32<T>(0.f);
     return r;
 }
+// The last four tokens of the lane below's V, which stand in front of this lane's own; lane 0 keeps `own`.
+template <typename T, int V>
+__device__ __forceinline__ Tokens<T, 4> tokens_below(const Tokens<T, 4>& own, const Tokens<T, V>& v) {
+    constexpr int W = (int)sizeof(T), F = (V - 4) * W / 4;      // words of four tokens; the first of them in v
+    uint32_t o[W], all[V * W / 4];
+    __builtin_memcpy(o, &own, sizeof(own));
+    __builtin_memcpy(all, &v, sizeof(v));
+#pragma unroll
+    for (int i = 0; i < W; ++i) o[i] = __builtin_amdgcn_update_dpp(o[i], all[F + i], 0x138, 0xF, 0xF, false);      // wave_shr:1
+    Tokens<T, 4> r;
+    __builtin_memcpy(&r, o, sizeof(r));
+    return r;
+}
 template <typename T, int N>
 __device__ __forceinline__ void st_tokens(T* __restrict__ row, int64_t t, int64_t l, const float (&in)[N]) {
     if (t + N <= l) {
@@ -536,10 +552,10 @@ __device__ __forceinline__ void ld_row_taps(const void* __restrict__ w, const vo
     bv = bias ? to_f32(static_cast<const WT*>(bias)[c]) : 0.f;
 }
 
-// One thread per 16-byte piece of a row: its own tokens and the 4 before them (an L1 hit: the neighbour's own), eight
-// waves' worth of pieces per SIMD in flight.  HBM bound: b4 C5376 l2048 bf16 37.5 -> 30.5 us with both loads of a wave behind one another
-// (176 MB, 5.8 TB/s).
-template <typename T, typename WT, int ACT>
+// One thread per 16-byte piece of a row: its own tokens, and the 4 before them from the lane below, eight
+// waves' worth of pieces per SIMD in flight.  HBM bound, kernel alone in a stream of them with its inputs cold: b4 C5376 l2048 bf16 30 us (176 MB,
+// 5.9 TB/s; 37 with a branch in front of the row ends' loads), fp32 58.3 (62 with the four tokens loaded and behind the taps).
+template <typename T, typename WT, int ACT, bool WHOLE>
 __global__ void __launch_bounds__(256)
 conv_fwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias, T* __restrict__ y,
                    int64_t l, uint32_t C, uint32_t pieces, uint32_t total, int64_t xsb, int64_t xsc, int64_t ysb, int64_t ysc) {
@@ -550,18 +566,20 @@ conv_fwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     const int64_t t0 = (int64_t)(idx - row * pieces) * V;
     const T* xr = x + b * xsb + c * xsc;
     float h[4], cur[V], wv[4], bv, o[V];
-    Tokens<T, 4> rh;
+    Tokens<T, 4> rh{};
     Tokens<T, V> rc;
-    ld_row_taps<WT>(w, bias, c, wv, bv);
-    if (l >= V) {
-        const int gone = (int)((int64_t)pieces * V - l);      // what the row's last piece lacks
-        const bool cut = idx - row * pieces == pieces - 1;
+    const int gone = WHOLE ? (int)((int64_t)pieces * V - l) : 0;      // what the row's last piece lacks
+    const bool cut = WHOLE && idx - row * pieces == pieces - 1;
+    if constexpr (WHOLE) {
         rc = ld_whole<T, V>(xr + t0 - (cut ? gone : 0));
-        rh = ld_whole<T, 4>(xr + (t0 > 0 ? t0 - 4 : 0));
-        if (gone > 0 && __any(cut)) rc = move_down<T, V>(rc, gone, cut);
+        if ((threadIdx.x & 63) == 0 && t0 > 0) rh = ld_whole<T, 4>(xr + t0 - 4);
     } else {
         rc = ld_short<T, V>(xr, t0, l);
-        for (int i = 0; i < 4; ++i) rh[i] = (T)0.f;
+    }
+    ld_row_taps<WT>(w, bias, c, wv, bv);
+    if constexpr (WHOLE) {
+        rh = tokens_below<T, V>(rh, rc);
+        if (gone > 0 && __any(cut)) rc = move_down<T, V>(rc, gone, cut);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) h[i] = t0 > 0 ? to_f32(rh[i]) : 0.f;
@@ -883,8 +901,12 @@ int launch_fwd(const m2_conv1d_params* p, void* state_, int W, bool continuing, 
     } else if (!hist && channel_major_ok(p, false)) {
         const int64_t pieces = ceil_div(l, (int64_t)VecTraits<T>::kVec), total = nb * C * pieces;
         conv_dispatch(p, [&](auto wt, auto act) {
-            conv_fwd_cm_kernel<T, decltype(wt), decltype(act)::value><<<(unsigned)ceil_div(total, (int64_t)256), 256, 0, st>>>(
-                x, p->w, p->bias, y, l, (uint32_t)C, (uint32_t)pieces, (uint32_t)total, p->x_stride_b, p->x_stride_c, p->y_stride_b, p->y_stride_c);
+            auto go = [&](auto k) {
+                k<<<(unsigned)ceil_div(total, (int64_t)256), 256, 0, st>>>(x, p->w, p->bias, y, l, (uint32_t)C, (uint32_t)pieces, (uint32_t)total, p->x_stride_b, p->x_stride_c,
+                                                                          p->y_stride_b, p->y_stride_c);
+            };
+            if (l >= VecTraits<T>::kVec) go(conv_fwd_cm_kernel<T, decltype(wt), decltype(act)::value, true>);
+            else go(conv_fwd_cm_kernel<T, decltype(wt), decltype(act)::value, false>);
         });
     } else {
         const int64_t total = nb * l * C;
