@@ -19,6 +19,8 @@
 // of one row, so the taps of an output come from the lane's own window and nothing is loaded per tap.
 //
 // A generic path (any strides, k <= 8) covers the rest with one thread per output element.
+#include <algorithm>
+
 #include "sums.hpp"
 
 namespace m2 {
@@ -597,15 +599,16 @@ conv_fwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
 
 // One wave per (channel, split): its lanes walk the channel's pieces of two vectors of tokens over all rows of the batch,
 // so the sums of dw and db stay in registers until the end, and the next piece is on its way while this one is computed.  The 1, 2 or
-// 4 (`inner`) splits of a channel inside a workgroup meet in LDS and finish it there; only with more of them (a few channels) do fp32
-// partials go to conv_reduce_partials_kernel, whose launch is 4 us.  Where a channel has no more than 32 pieces, `lanes` of the wave (a
+// 4 (`inner`) splits of a channel inside a workgroup meet in LDS and finish it there; only with more of them (long channels) do fp32
+// partials go to conv_reduce_partials_kernel, whose launch is 2 to 4 us.  Where a channel has no more than 32 pieces, `lanes` of the wave (a
 // power of two) take it and the others the channels behind it.
 // A lane recomputes the three tokens behind its own for the dx lag: 3 in 16
 // (bf16) more activations, against a cross-lane exchange that would break at every row end.
 // What bounds it: the vector units (some 40 us of activations recomputed, at b4 C5376 l2048 bf16) beside 264 MB of traffic (44 us), in
-// waves of their own each waiting for its loads: 95 -> 69 us there without a lane's branch in front of the loads and with the next piece
-// under way (four waves a SIMD: 69, five, with spills: 77); 3 x 4097 rows of 1001 38 -> 27, 10240 rows of 77 19.7 -> 6.0.
-template <typename T, typename WT, int ACT>
+// waves of their own each waiting for its loads: 94 -> 67 us there, cold and in a stream of them, without a lane's branch in front of the loads and
+// with the next piece under way (in a row of forward and backward passes of autograd, which find some of their inputs cached, 71 -> 61; five waves a
+// SIMD spill: 77); 3 x 4097 rows of 1001 38 -> 27, 10240 rows of 77 19.7 -> 5.9.
+template <typename T, typename WT, int ACT, bool WHOLE>
 __global__ void __launch_bounds__(256, 4)
 conv_bwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const void* __restrict__ bias, const T* __restrict__ dy,
                    T* __restrict__ dx, float* __restrict__ part, void* __restrict__ dw, void* __restrict__ db,
@@ -615,9 +618,9 @@ conv_bwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
     constexpr int pd = std::is_same<WT, float>::value ? M2_F32 : M2_BF16;
     __shared__ float red[4][5];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & (lanes - 1), sub = wave & (inner - 1);
-    const uint32_t unit = lanes < 64 ? (blockIdx.x * 256u + threadIdx.x) / lanes : (blockIdx.x * 4u + wave) / inner;
+    const uint32_t unit = lanes < 64 ? (blockIdx.x * 256u + threadIdx.x) >> __builtin_ctz(lanes) : (blockIdx.x * 4u + wave) >> __builtin_ctz(inner);      // powers of two
     const bool live = unit < C * outer;            // the last workgroup may have fewer channels
-    const uint32_t part_row = live ? unit / C : 0, c = live ? unit - part_row * C : 0, split = part_row * inner + sub;
+    const uint32_t part_row = live && outer > 1 ? unit / C : 0, c = live ? unit - part_row * C : 0, split = part_row * inner + sub;
     const uint32_t end = !live ? 0 : (split + 1) * per_split < total ? (split + 1) * per_split : total;
     float wv[4], bv, acc[5];
     ld_row_taps<WT>(w, bias, c, wv, bv);
@@ -630,7 +633,7 @@ conv_bwd_cm_kernel(const T* __restrict__ x, const void* __restrict__ w, const vo
         const T* xr = x + b * xsb + c * xsc;
         const T* gr = dy + b * gsb + c * gsc;
         Piece q;
-        if (l >= V) {
+        if constexpr (WHOLE) {
             // what the row's last piece lacks of its two vectors, and the piece before it of the four tokens behind it
             const int lacks = (int)((int64_t)pieces * N - l);
             const bool last = t0 + N >= l, near = t0 + N + 4 > l;
@@ -955,19 +958,38 @@ int launch_bwd(const m2_conv1d_params* p, int64_t* slots, hipStream_t st) {
         int64_t lanes = 64;
         while (lanes > 1 && lanes / 2 >= total) lanes /= 2;
         const int64_t rounds = ceil_div(total, lanes);
-        // four splits of a channel where its workgroup's four waves have a round each; more, through partials, while the chip has not
-        // eight waves a CU and the splits that come of it have two rounds at least (one, two, four, eight of them: b4 l2048 C5376
-        // 83 / 77 / 69 / 72 us, C256 12.1 / 7.8 / 6.0 / 8.1; b16 l8192 C128 four, eight, sixteen: 53 / 47 / 35)
-        int64_t splits = rounds >= 4 ? 4 : rounds >= 2 ? 2 : 1;
-        while (C * splits < 8 * device_cus() && rounds >= 4 * splits) splits *= 2;
-        const int64_t inner = splits > 4 ? 4 : splits, outer = splits / inner, per_split = ceil_div(rounds, inner * outer) * lanes;
+        // A channel's rounds over the four waves of one workgroup; where they are many, over several workgroups, whose partials cost a launch
+        // more, in as many rounds a wave as take the least time: a chain of rounds (1.6 us each) or, beyond one workgroup per CU, what a
+        // CU's workgroups do at 1.2 us a round; chains of more than three lose an eighth to that.  Four waves | one | two | four rounds, us: 17 x 20
+        // channels x 795 bf16 10.9 | 7.8 | 9.5, fp32 11.5 | 7.3 | 8.2 | 10.0; 35 x 3 x 2818 bf16 38.9 | 8.7 | 10.0 | 12.2; 31 x 188 x 9665 bf16 141 |
+        // 115 | 108 | 114, fp32 209 | 169 | 174 | 196; 25 x 118 x 1798 bf16 23 | 16.0 | 15.5 | 17.4; 4 x 5376 x 2048 fp32 139 | 122 | 127; 1 x 5646 x 4789
+        // fp32 82 | 93 | 101; 7 x 412 x 1279 fp32 13.8 | 16.7 | 17.5 | 15.4.  Up to eight rounds the launch is not earned: 4 x 5376 x 2048
+        // bf16 68 | 72, 1 x 16 x 8192 6.2 | 6.8.
+        int64_t inner = rounds >= 3 ? 4 : rounds, outer = 1, r = ceil_div(rounds, inner);
+        if (rounds > 8) {
+            auto cost = [&](int64_t k, int64_t n) {
+                const float us = (float)k * std::max(1.6f, 1.2f * (float)(C * n) / (float)device_cus());
+                return (k > 3 ? 1.13f * us : us) + (n > 1 ? 3.f + 0.04f * (float)n : 0.f);
+            };
+            float least = cost(r, 1);
+            for (int64_t k = 1; ceil_div(rounds, k) > 4; k *= 2) {
+                const int64_t n = ceil_div(rounds, 4 * k);
+                const float us = cost(k, n);
+                if (us < least) { least = us; outer = n; r = k; }
+            }
+        }
+        const int64_t per_split = r * lanes;
         float* part = static_cast<float*>(p->workspace);
         M2_REQUIRE(outer == 1 || (part && p->workspace_bytes >= (size_t)(outer * C * 5) * sizeof(float)), M2_ERR_WORKSPACE,
                    "conv1d_bwd: workspace %zu bytes < %zu needed", p->workspace_bytes, (size_t)(outer * C * 5) * sizeof(float));
         conv_dispatch(p, [&](auto wt, auto act) {
-            conv_bwd_cm_kernel<T, decltype(wt), decltype(act)::value><<<(unsigned)(lanes < 64 ? ceil_div(C * lanes, (int64_t)256) : ceil_div(C * outer * inner, (int64_t)4)), 256, 0, st>>>(
-                x, p->w, p->bias, dy, dx, part, p->dw, p->db, l, (uint32_t)C, (uint32_t)lanes, (uint32_t)inner, (uint32_t)outer, (uint32_t)pieces, (uint32_t)per_split,
-                (uint32_t)total, p->x_stride_b, p->x_stride_c, p->y_stride_b, p->y_stride_c, p->dx_stride_b, p->dx_stride_c);
+            auto go = [&](auto k) {
+                k<<<(unsigned)(lanes < 64 ? ceil_div(C * lanes, (int64_t)256) : ceil_div(C * outer * inner, (int64_t)4)), 256, 0, st>>>(
+                    x, p->w, p->bias, dy, dx, part, p->dw, p->db, l, (uint32_t)C, (uint32_t)lanes, (uint32_t)inner, (uint32_t)outer, (uint32_t)pieces, (uint32_t)per_split,
+                    (uint32_t)total, p->x_stride_b, p->x_stride_c, p->y_stride_b, p->y_stride_c, p->dx_stride_b, p->dx_stride_c);
+            };
+            if (l >= VecTraits<T>::kVec) go(conv_bwd_cm_kernel<T, decltype(wt), decltype(act)::value, true>);
+            else go(conv_bwd_cm_kernel<T, decltype(wt), decltype(act)::value, false>);
         });
         int rc = check_launch("conv1d_bwd");
         if (rc || outer == 1) return rc;

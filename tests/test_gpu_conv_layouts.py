@@ -118,3 +118,11 @@ def test_conv_channel_major_splits(dtype, b, l, C, act):
                          [(3, 160, 70), (9, 115, 65), (2, 5001, 9), (9, 8190, 3)])
 def test_conv_channel_major_row_ends(dtype, b, l, C):
     test_conv_layout_edges(dtype, False, b, l, C, "silu")
+
+
+# channel-major: a channel's rounds over three of a workgroup's four waves, over several workgroups with one round a wave and with more, and the last of
+# them without work
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,l,C", [(3, 1000, 5), (17, 795, 20), (2, 70001, 2), (5, 2600, 300)])
+def test_conv_channel_major_rounds(dtype, b, l, C):
+    test_conv_layout_edges(dtype, False, b, l, C, "silu")
