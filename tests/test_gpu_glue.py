@@ -266,3 +266,16 @@ def test_core_norm_reads_the_gate_on_any_element(dtype, rows, d, g, extra, first
     for a, b in zip(call(z)[0], call(whole)[0]):
         assert torch.equal(a, b)
     assert call(z)[1] and not call(whole)[1]      # the plain entry asks for whole vectors, as before
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,d,g", [(5, 512, 8), (3, 512, 1), (4, 2560, 1), (2, 1088, 1)])
+def test_rmsnorm_gated_weight_on_any_element(dtype, rows, d, g):
+    """The weights come in 16-byte pieces: from a tensor that starts on any element the same bits, forward and backward."""
+    from mamba2 import glue
+    x, z, dout = (_rand((rows, d), dtype, s).to(DEV) for s in (51, 52, 53))
+    w = (1 + 0.2 * _rand((d,), torch.float32, 54)).to(DEV)
+    odd = torch.empty(d + 1, device=DEV)[1:].copy_(w)
+    assert odd.data_ptr() % 16 == 4
+    got = [(glue.rmsnorm_gated_hip(x, z, v, g, 1e-5), *glue.rmsnorm_gated_bwd_hip(x, z, v, dout, g, 1e-5)) for v in (w, odd)]
+    assert all(torch.equal(a, b) for a, b in zip(*got))
