@@ -367,36 +367,41 @@ int norm_lanes(int64_t nvec, int64_t groups) {
 int64_t norm_columns(int64_t nvec, int64_t groups) { return ceil_div(groups, (int64_t)(64 / norm_lanes(nvec, groups))); }
 
 // Rows per workgroup.  A workgroup (or, with a wave per row, each of its four waves) is a chain of rows, dealt round-robin, and the chip
-// likes one or two of them per CU: with a few more (834 of four rows for 3333) a second round is nearly empty, and in the backward every
-// one leaves a partial row of dw.  Workgroups per CU, from 180 sizes (300 to 26000 rows, groups of 512 to 7168 channels, both types;
-// time with one | two | three | four per CU, us, forward and backward):
-//   a wave per row, more than two vectors a lane: one.  3333 x 2048 8.8 | 8.7 | 8.7 | 9.8 and 19.5 | 20.9 | 21.0 | 26.0, 8192 x 2048
-//     18.4 | 19.1 | 20.6 | 20.5 and 34.4 | 37.1 | 39.5 | 41.3
-//   two vectors: two forward, one backward, two for many rows of one group.  8192 x 8 x 1024 79.6 | 80.3 | 82.5 | 83.6 and 128 | 140 |
-//     144 | 143; 16384 x 1024 20.5 | 18.2 | 19.0 | 19.3 and 33.5 | 33.2 | 36.1 | 36.4
-//   one vector: four forward, two backward, one for few rows.  8192 x 8 x 512 52.3 | 35.0 | 32.7 | 33.4 and 82 | 67 | 70 | 69
-//   a workgroup per row: one, but forward, of 16-bit rows of two vectors a lane, two up to 9000 rows, and a row each up to 1100.
-//     2664 x 5120 17.8 | 16.5 | 17.0 | 18.3 and 32.0 | 36.4 | 38.1 | 38.9, 16384 x 5120 90 | 96 | 100 | 101 and 162 | 173 | 174 | 178,
-//     2664 x 7168 24.1 | 25.5 | 28.3 | 30.8; rows that leave lanes idle (2560, 3072) want two for longer: 8192 x 3072 36.8 | 29.8 | 30.1
-//     | 29.5, backward 51.7 | 48.0 | 58.5 | 52.9
+// likes a few of them per CU: one more than fit run alone at the end, and in the backward every one leaves a partial row of dw.
+// Workgroups per CU by the form of a row, from 990 sizes (64 to 16000 rows, groups of 64 to 8192 channels, both types; one | two | three | four
+// per CU, us; `all`: rows times columns of the grid):
+//   forward, a wave per row, one vector a lane: four (8192 x 8 x 512 52.3 | 35.0 | 32.7 | 33.4, 6500 x 512 6.9 | 6.1 | 6.2 | 5.7); two vectors: two
+//     (16384 x 1024 20.5 | 18.2 | 19.0 | 19.3); more: one (8192 x 2048 18.4 | 19.1 | 20.6 | 20.5).  16-bit rows that are few enough for chains of up
+//     to three go one to a wave instead where the busiest CU then has fewer: 2100 x 1024 5.1 | 5.2, a row each 4.9; 513 x 8 x 1024 7.0, 6.4; not
+//     3700 x 1024 6.3 | 5.9, 6.1.  fp32 does not gain by it (600 x 8 x 512 6.2, a row each 6.8).
+//   backward, a wave per row, up to one and a half vectors a lane: two for many rows or where a partial row is short, else one (9001 x 2 x 320 fp32
+//     28.8 | 24.2 | 24.9 | 27.1, 1500 x 512 bf16 6.9 | 7.2, 3001 x 512 8.4 | 8.9 | 9.1, 6500 x 512 11.6 | 11.7; 400 x 8 x 512 8.65 | 8.3); more vectors:
+//     one (3333 x 2048 19.5 | 20.9 | 21.0 | 26.0, 9001 x 512 fp32 19.8 | 21.1 | 22.2).
+//   a workgroup per row, two vectors a lane, idle lanes: two (6500 x 2560 27.8 | 22.6 | 21.4 | 21.6, backward 9001 x 2560 52.8 | 47.0 | 54.5 | 49.9),
+//     the backward of few rows one (1500 x 2560 14.2 | 14.3, 1800 16.3 | 15.6).
+//   ... no idle lane: forward a row each up to five per CU (1101 x 5120 9.3 | 9.2, each 8.6; 1300: 10.3 | 9.6, 9.5; 1500: 10.5 | 10.05, 10.5), then
+//     two of 16-bit rows up to 35 rows per CU (6500 x 5120 36.4 | 33.3 | 34.6 | 37.2, 12001 67.2 | 70.6), else one, and the backward one
+//     (2664 x 5120 32.0 | 36.4 | 38.1 | 38.9).
+//   ... more vectors a lane: one (2664 x 7168 24.1 | 25.5 | 28.3 | 30.8).
 int64_t norm_rows_per_workgroup(int64_t rows, int64_t groups, int64_t nvec, int vec_elems, bool bwd) {
     int wpg = 1, nv = 1;
     if (!norm_shape(nvec, vec_elems, &wpg, &nv)) return ceil_div(rows, (int64_t)512);      // refused before any launch
-    const int64_t all = rows * norm_columns(nvec, groups);
+    const int64_t columns = norm_columns(nvec, groups), all = rows * columns, cus = device_cus();
+    if (wpg == 1) {
+        const int64_t per_cu = bwd ? (nvec <= 96 && (all > 20 * cus || columns >= 4) ? 2 : 1) : (nv == 1 ? 4 : nv == 2 ? 2 : 1);
+        const int64_t chain = ceil_div(all, 4 * per_cu * cus);      // rows per wave
+        auto busiest = [&](int64_t c) { return ceil_div(ceil_div(rows, 4 * c) * columns, cus) * c; };
+        if (!bwd && nv <= 2 && vec_elems == 8 && chain <= 3 && busiest(1) < busiest(chain)) return 4;
+        return 4 * chain;
+    }
     const bool exact = (int64_t)wpg * 64 * nv == nvec;
     int64_t per_cu = 1;
-    if (wpg == 1) {
-        if (nv == 2) per_cu = bwd ? (groups == 1 && rows > 7000 ? 2 : 1) : 2;
-        if (nv == 1) per_cu = bwd ? (all > 5000 ? 2 : 1) : 4;
-        const int64_t rb = ceil_div(all, per_cu * device_cus());
-        return rb < 4 ? 4 : (rb + 3) / 4 * 4;
+    if (nv == 2 && !exact) per_cu = !bwd || all > 6 * cus ? 2 : 1;
+    if (nv == 2 && exact && !bwd) {
+        if (all <= 5 * cus) return 1;
+        if (vec_elems == 8 && all <= 35 * cus) per_cu = 2;
     }
-    if (nv == 2 && bwd && !exact && all >= 3000 && all <= 12000) per_cu = 2;
-    if (nv == 2 && !bwd) {
-        if (all <= 1100 && exact) return 1;
-        if (all > 1100 && (!exact || (vec_elems == 8 && all <= 9000))) per_cu = 2;
-    }
-    return ceil_div(all, per_cu * device_cus());
+    return ceil_div(all, per_cu * cus);
 }
 
 template <typename T, bool BWD>

@@ -279,3 +279,11 @@ def test_rmsnorm_gated_weight_on_any_element(dtype, rows, d, g):
     assert odd.data_ptr() % 16 == 4
     got = [(glue.rmsnorm_gated_hip(x, z, v, g, 1e-5), *glue.rmsnorm_gated_bwd_hip(x, z, v, dout, g, 1e-5)) for v in (w, odd)]
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+# rows per workgroup: a row each and chains of two in one launch shape's range, five rows per CU and one more, idle lanes with few and many rows, a vector
+# and a quarter a lane
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,d,g", [(513, 8192, 8), (3700, 1024, 1), (4500, 512, 1), (1280, 4096, 1), (1281, 4096, 1), (257, 2560, 1), (1537, 2560, 1), (2600, 640, 2), (400, 1536, 8)])
+def test_rmsnorm_gated_workgroups_per_cu(dtype, rows, d, g):
+    test_rmsnorm_gated_fwd_bwd(dtype, (1, rows), d, g, True)
