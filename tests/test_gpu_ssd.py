@@ -422,3 +422,27 @@ def test_ssd_initial_state_on_any_element(b, l, h, p, n):
 def test_prefill_initial_state_of_a_long_walk():
     """34 chunks behind a prefix, the state read lane by lane, against two pieces whose states come as rows."""
     test_prefill_states_in_segments_in_place(4300, 2100, 40, 64)
+
+
+@pytest.mark.parametrize("h,growth", [(2, 60.0), (42, 12.0)])      # two and twelve chunks a segment
+def test_ssd_segments_of_nothing(h, growth):
+    """A state of zeros stays zero however its segments grow (e^120 and e^144, past fp32; a chunk's own factor is not): a sequence with inputs in its
+    last chunk only is that chunk, and its gradients from the first chunk only are that chunk's."""
+    from mamba2.mamba2_kernel import mamba2_kernel
+    l = 48 * 128
+    d = _dev(make_ssd_inputs(1, l, h, 64, 128, 1, seed=h, dtype=torch.bfloat16))
+    dt, A = torch.full_like(d["dt"], 0.5), torch.full_like(d["A"], growth / 64)
+
+    def run(x, B, C, dt):
+        leaves = [v.detach().requires_grad_(True) for v in (x, B, C)]
+        return mamba2_kernel(dt, A, *leaves, d["D"]), leaves
+
+    first, last = slice(0, 128), slice(l - 128, l)
+    x, dy = torch.zeros_like(d["X"]), torch.zeros_like(d["dy"])
+    x[:, last], dy[:, first] = d["X"][:, last], d["dy"][:, first]
+    y, leaves = run(x, d["B"], d["C"], dt)
+    grads = torch.autograd.grad(y, leaves, dy)
+    assert torch.equal(y[:, last], run(*(v[:, last].contiguous() for v in (x, d["B"], d["C"], dt)))[0]) and (y[:, :l - 128] == 0).all()
+    y1, leaves = run(*(v[:, first].contiguous() for v in (x, d["B"], d["C"], dt)))
+    for name, a, b in zip(("dX", "dB", "dC"), grads, torch.autograd.grad(y1, leaves, dy[:, first].contiguous())):
+        assert torch.equal(a[:, first], b) and (a[:, 128:] == 0).all(), name
