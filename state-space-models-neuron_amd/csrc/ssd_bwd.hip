@@ -248,7 +248,7 @@ int ssd_bwd_impl(const SsdCall* p, hipStream_t st) {
         sa.X = dy; sa.X_sb = p->dy_stride_b; sa.X_sl = p->dy_stride_l; sa.X_sh = p->dy_stride_h;
         sa.ldtab = w.ldtab; sa.Mt = w.Ct; sa.init = p->d_final_state; sa.prev = w.dprev; sa.final_out = p->d_initial_state;
         sa.seqlen = p->seqlen; sa.nheads = p->nheads; sa.ngroups = p->ngroups; sa.nchunks = nc;
-        if ((rc = launch_state_pass16<T, P, N, true, HS, false>(sa, w, p->batch, st))) return rc;
+        if ((rc = launch_state_pass16<T, P, N, true, HS, false>(sa, w, p->batch, kSegOneTile, st))) return rc;
         if ((rc = check_launch("ssd state_pass16_kernel<reverse>"))) return rc;
     } else
     {   // fp32: local dS contributions (reuses the `local` region), then the reverse recurrence

@@ -117,8 +117,9 @@ inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_
         if (p->dtype != M2_F32) w.Ct = keep(grp * p->dstate * kQ * esz);
         w.kept_bytes = koff;
     }
+    // (a forward's size does not look at final_state: a caller may ask for it before there is one)
     if (p->dtype != M2_F32)
-        if (const int64_t m = state_pass_seg_chunks(p->batch * p->nheads, nc, true)) {
+        if (const int64_t m = state_pass_seg_chunks(p->batch * p->nheads, nc, p->chunk_states ? kSegKept : kSegPrompt)) {
             const size_t sums = (size_t)((ceil_div(nc, m) - 1) * p->batch * p->nheads);
             w.seg = take(sums * p->headdim * p->dstate * 4);
             w.seg_lam = reinterpret_cast<float*>(take(sums * 4));
@@ -190,7 +191,7 @@ inline size_t cb_smem(int n) {      // operand rows; 32 tokens of both to transp
 }
 
 template <typename T, int P, int N, bool REVERSE, int HS, bool HILO>
-inline int launch_state_pass16(StatePassArgs a, const SsdWorkspace& w, int64_t batch, hipStream_t st) {
+inline int launch_state_pass16(StatePassArgs a, const SsdWorkspace& w, int64_t batch, int64_t seg_least, hipStream_t st) {
     auto launch = [&](auto k, size_t sm, int split, int64_t segs = 1) -> int {
         if (const int rc = allow_smem(k, sm)) return rc;
         k<<<dim3((unsigned)(a.nheads * split), (unsigned)batch, (unsigned)segs), state_pass_threads<N>(), sm, st>>>(a);
@@ -202,7 +203,7 @@ inline int launch_state_pass16(StatePassArgs a, const SsdWorkspace& w, int64_t b
             return staged ? launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, 1, 0, true>, state_pass_smem<P, N, HILO, 1>(), 1) :
                             launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, 1>, state_pass_smem<P, N, HILO, 1>(), 1);
     constexpr int SPLIT = kStatePassSplit;
-    if (const int64_t m = state_pass_seg_chunks(batch * a.nheads, a.nchunks, HILO)) {
+    if (const int64_t m = state_pass_seg_chunks(batch * a.nheads, a.nchunks, seg_least)) {
         a.seg = static_cast<floatx4*>(w.seg); a.seg_lam = w.seg_lam; a.seg_chunks = m;
         const int64_t sums = ceil_div(a.nchunks, m) - 1;
         int rc = launch(state_pass16_kernel<T, P, N, REVERSE, HS, HILO, SPLIT, 1>, state_pass_smem<P, N, HILO, SPLIT>(), SPLIT, sums);
@@ -271,7 +272,9 @@ inline int ssd_launch_states(const SsdCall* p, const SsdWorkspace& w, float* fin
         sa.X = x; sa.X_sb = p->x_stride_b; sa.X_sl = p->x_stride_l; sa.X_sh = p->x_stride_h;
         sa.ldtab = w.ldtab; sa.Mt = w.Bt; sa.init = p->initial_state; sa.prev = w.prev; sa.final_out = final_out;
         sa.seqlen = p->seqlen; sa.nheads = p->nheads; sa.ngroups = p->ngroups; sa.nchunks = nc;
-        if ((rc = hilo ? launch_state_pass16<T, P, N, false, HS, true>(sa, w, p->batch, st) : launch_state_pass16<T, P, N, false, HS, false>(sa, w, p->batch, st))) return rc;
+        rc = hilo ? launch_state_pass16<T, P, N, false, HS, true>(sa, w, p->batch, p->chunk_states ? kSegKept : kSegPrompt, st) :
+                    launch_state_pass16<T, P, N, false, HS, false>(sa, w, p->batch, kSegOneTile, st);
+        if (rc) return rc;
         return check_launch("ssd state_pass16_kernel");
     } else {
         // fp32 operands: per-chunk contributions (workspace), then the recurrence over the chunks

@@ -55,19 +55,21 @@ inline int state_pass_split(int64_t heads, int n) {
 // of steps of about 1.05 us each; in segments the chain is as long as two of them: the first launch walks the first segment and forms
 // the sums of the others but the last from zero, all side by side, and the second starts each of the others from the sums in front of
 // it, decayed (the decay is one number per head, so this costs a product per element and segment).
-// A launch more and the filling of two chains cost about 3 us on the device: below the line they are not earned.  The launch also costs 2.5 us
-// of the host, which a prompt's forward (the one that wants the final state) does not wait for, and training few heads does up to some 32
-// chunks (forward and backward at b1 l4000 h8 g8 98 -> 104 us, l7519 h16 g8 243 -> 170): a line of its own.  Whole forward scan alone, us,
-// whole pass ->
+// A launch more and the filling of two chains cost about 3 us on the device: below a line they are not earned.  The launch also costs 2.5 us
+// of the host, which a prompt's forward does not wait for and training few heads does: lines of their own for a forward that keeps its states
+// for the backward (with the final state, forward and backward: b1 l2600 h8 g8 112.9 -> 115.5 us, l3000 h4 111 -> 114.5, l4000 h8 g8 120 -> 114, l4000
+// h16 126 -> 114) and for the passes that leave no final state, where the operands of one tile walk faster (l4000 h8 g8 98 -> 104, l7519 h16 g8
+// 243 -> 170).  Whole forward scan alone, us, whole pass ->
 // segments, for 16, 48, 64, 84 and 128 half heads (16, 5, 4, 3 and 2 sets), 128 state columns:
 //   8 chunks    22.9 -> 23.8   24.3 -> 25.5   24.9 -> 26.0   28.1 -> 30.8   30.2 -> 33.0
 //   12 chunks   25.7 -> 24.7   29.8 -> 29.2   30.8 -> 30.7   31.4 -> 33.2   35.6 -> 37.8
 //   16 chunks   28.4 -> 25.5   33.6 -> 31.9   34.6 -> 35.4   36.5 -> 37.6   39.3 -> 41.4
 //   24 chunks   34.0 -> 27.4   41.8 -> 37.5   43.1 -> 38.9   43.0 -> 42.3   51.1 -> 51.1
 //   64 chunks   65.8 -> 38.2   74.9 -> 53.5   80.3 -> 60.9   81.6 -> 74.5   96.8 -> 88.5
-inline int64_t state_pass_seg_chunks(int64_t heads, int64_t nchunks, bool prompt) {
+constexpr int64_t kSegPrompt = 20, kSegKept = 28, kSegOneTile = 48;      // chunks from which a walk goes in segments
+inline int64_t state_pass_seg_chunks(int64_t heads, int64_t nchunks, int64_t least) {
     const int64_t sets = heads > 0 ? device_cus() / (heads * kStatePassSplit) : 0;      // of workgroups that the CUs hold, one each
-    if (sets < 2 || nchunks < (prompt ? 20 : 48) || nchunks * sets < 96) return 0;
+    if (sets < 2 || nchunks < least || nchunks * sets < 96) return 0;
     const int64_t chunks = ceil_div(nchunks, sets + 1);
     return chunks < 2 ? 2 : chunks;
 }

@@ -86,3 +86,17 @@ def test_scan_backward_asks_for_what_its_kernels_write(lib, dtype, b, l, h, p, n
     want += groups * q * q * 4 * ((0 if done and not dtype else s_g) + (s_g > 1)) + 2 * groups * q * n * 4 * ((0 if done else s_b) + (s_b > 1))
     got = lib.m2_ssd_bwd_workspace_bytes(ctypes.byref(params))
     assert want <= got <= want + 20 * 256, (got, want)
+
+
+@pytest.mark.parametrize("chunks", [19, 20, 27, 28, 47, 48])
+def test_scan_asks_for_segments_where_a_walk_goes_in_them(lib, chunks):
+    """Few heads, many chunks: room for the segments' states from 20 chunks (a forward) or 28 (one that keeps its states for the backward)."""
+    from mamba2 import _lib
+    h, n, q = 8, 128, 128
+    m = max(2, -(-chunks // 17))                       # 16 half heads: 16 sets of them on 256 CUs
+    seg = (-(-chunks // m) - 1) * h * (64 * n + 1) * 4
+    p = _lib.SsdParams(batch=1, seqlen=chunks * q, nheads=h, headdim=64, dstate=n, ngroups=h, dtype=1, dt_dtype=1)
+    kept = lib.m2_ssd_chunk_states_bytes(ctypes.byref(p))
+    assert 0 <= lib.m2_ssd_fwd_workspace_bytes(ctypes.byref(p)) - kept - (seg if chunks >= 20 else 0) <= 4 * 256
+    p.chunk_states = 256
+    assert 0 <= lib.m2_ssd_fwd_workspace_bytes(ctypes.byref(p)) - (seg if chunks >= 28 else 0) <= 4 * 256
