@@ -119,7 +119,7 @@ inline SsdWorkspace ssd_carve(const SsdCall* p, void* base, bool bwd, bool kept_
     }
     // (a forward's size does not look at final_state: a caller may ask for it before there is one)
     if (p->dtype != M2_F32)
-        if (const int64_t m = state_pass_seg_chunks(p->batch * p->nheads, nc, p->chunk_states ? kSegKept : kSegPrompt)) {
+        if (const int64_t m = state_pass_seg_chunks(p->batch * p->nheads, nc, bwd ? kSegOneTile : p->chunk_states ? kSegKept : kSegPrompt)) {
             const size_t sums = (size_t)((ceil_div(nc, m) - 1) * p->batch * p->nheads);
             w.seg = take(sums * p->headdim * p->dstate * 4);
             w.seg_lam = reinterpret_cast<float*>(take(sums * 4));

@@ -90,7 +90,7 @@ def test_scan_backward_asks_for_what_its_kernels_write(lib, dtype, b, l, h, p, n
 
 @pytest.mark.parametrize("chunks", [19, 20, 27, 28, 47, 48])
 def test_scan_asks_for_segments_where_a_walk_goes_in_them(lib, chunks):
-    """Few heads, many chunks: room for the segments' states from 20 chunks (a forward) or 28 (one that keeps its states for the backward)."""
+    """Few heads, many chunks: room for the segments' states from 20 chunks (a forward), 28 (one that keeps its states for the backward) and 48 (a backward)."""
     from mamba2 import _lib
     h, n, q = 8, 128, 128
     m = max(2, -(-chunks // 17))                       # 16 half heads: 16 sets of them on 256 CUs
@@ -100,3 +100,6 @@ def test_scan_asks_for_segments_where_a_walk_goes_in_them(lib, chunks):
     assert 0 <= lib.m2_ssd_fwd_workspace_bytes(ctypes.byref(p)) - kept - (seg if chunks >= 20 else 0) <= 4 * 256
     p.chunk_states = 256
     assert 0 <= lib.m2_ssd_fwd_workspace_bytes(ctypes.byref(p)) - (seg if chunks >= 28 else 0) <= 4 * 256
+    bhc = h * chunks
+    want = bhc * 64 * n * 2 + bhc * 4 * (8 + 3 + 4 * q + 8) + bhc * q * q * 4 + (seg if chunks >= 48 else 0)      # a head a group: whole groups, one slice
+    assert 0 <= lib.m2_ssd_bwd_workspace_bytes(ctypes.byref(p)) - want <= 20 * 256
