@@ -176,17 +176,17 @@ state_pass16_kernel(const StatePassArgs a) {
         __syncthreads();      // the first state's tile is written over it
     };
     if constexpr (PHASE == 2) {
-        // A segment's e^Lam can leave fp32 where no chunk's does.  Then it is taken in factors that do not, so that a state of zeros stays zero (not
-        // 0 inf) and a tiny one grows as it did chunk by chunk; three of them take any other to 0 or inf.  (Found out behind the loop: a branch in
-        // it stands in front of the next segment's loads, 1.5 us at 24 segments.)
+        // A segment's e^Lam can overflow where no chunk's does (dt A > 0).  Then it is taken in factors that fp32 holds, so that a state of zeros stays
+        // zero (not 0 inf) and a tiny one grows as it did chunk by chunk; three of them take any other to inf.  (Found out behind the loop: a branch
+        // in it stands in front of the next segment's loads, 1.5 us at 24 segments.)
         float most = 0.f;
         auto in_front = [&](auto safe) {
             for (int64_t t = 0; t < seg; ++t) {
                 float lam = t ? a.seg_lam[t * (int64_t)gridDim.y * a.nheads + bh] : 0.f;      // nothing in front of the first
                 if constexpr (decltype(safe)::value) {
-                    for (int k = 0; k < 3 && fabsf(lam) > 80.f; ++k) {
-                        const float part = lam > 0.f ? 80.f : -80.f, f = __expf(part);
-                        lam -= part;
+                    for (int k = 0; k < 3 && lam > 80.f; ++k) {
+                        const float f = __expf(80.f);
+                        lam -= 80.f;
 #pragma unroll
                         for (int i = 0; i < PBW; ++i)
 #pragma unroll
@@ -194,9 +194,9 @@ state_pass16_kernel(const StatePassArgs a) {
 #pragma unroll
                                 for (int v = 0; v < 16; ++v) acc[i][j][v] *= f;
                     }
-                    lam = lam > 80.f ? 80.f : lam < -80.f ? -80.f : lam;      // (NaN stays)
+                    lam = lam > 80.f ? 80.f : lam;      // (NaN stays)
                 } else {
-                    most = fmaxf(most, fabsf(lam));
+                    most = fmaxf(most, lam);
                 }
                 const float dec = t ? __expf(lam) : 0.f;
 #pragma unroll
@@ -212,7 +212,7 @@ state_pass16_kernel(const StatePassArgs a) {
             }
         };
         in_front(std::false_type{});
-        if (most > 80.f) {
+        if (__builtin_expect(most > 80.f, false)) {
             acc_zero(acc);
             in_front(std::true_type{});
         }
