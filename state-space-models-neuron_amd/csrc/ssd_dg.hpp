@@ -49,12 +49,14 @@ dg16_kernel(const T* __restrict__ X, const float* __restrict__ ldtab,
     const int64_t hpg = nheads / ngroups;
     const int64_t t0 = c * kQ;
     const int valid = (int)((seqlen - t0) < kQ ? (seqlen - t0) : kQ);
-    // block (rb, cb) of this wave (one nibble per wave): the four diagonal blocks sit on waves 2, 3, 6, 7, i.e. on the two
+    // block (rb, cb) of this wave (two bits per wave): the four diagonal blocks sit on waves 2, 3, 6, 7, i.e. on the two
     // SIMDs that carry two waves; the six blocks below the diagonal on the two SIMDs that carry three
     //   wave   0     1     2     3     4     5     6     7     8     9
     //   block (1,0) (2,0) (0,0) (1,1) (2,1) (3,0) (2,2) (3,3) (3,1) (3,2)
-    const int rb = (int)((0x3332321021ull >> (4 * wave)) & 15);
-    const int cb = (int)((0x2132011000ull >> (4 * wave)) & 15);
+    // In 32 bits: a 64-bit shift by a lane's amount has given wrong high words where the compiler put the amount into a wave's last register.  (Per
+    // lane: out of scalar registers the kernel took 2 us of 42 more at b4 l2048 h80.)
+    const int rb = (int)((0xfee49u >> (2 * wave)) & 3u);
+    const int cb = (int)((0x9e140u >> (2 * wave)) & 3u);
     const bool masked = (rb == cb) || valid < kQ;      // wave-uniform
     const bool copier = wave < 8;
 
