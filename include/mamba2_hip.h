@@ -269,7 +269,7 @@ int m2_add_rmsnorm(float* residual, int64_t residual_stride_row, const void* del
  * m2_decode_rows: the head of such a chain: residual (rows, channels) fp32 += delta (set != 0: = delta; delta may be NULL
  * otherwise), x = bf16(residual * weight), sq (rows, 1).
  * m2_embed_rows: the same with residual = table[ids], the embedding of a model's step: table (vocab, channels) fp32 or bf16, ids
- * (rows) on the device; an id outside the table gives a row of NaN.
+ * (rows) on the device; an id outside the table gives a row of NaN.  weight, x and sq NULL: the residual alone.
  * m2_decode_layer: one decode step of a whole mixer layer in three launches (mamba2/mamba2_mixer.py:243-282): `in` writes
  * zxBCdt (bf16 rows, in->out), the scan reads it and the states of `dec` (updated in place; dec's xBC, dt, y and workspace
  * are not used) and writes the gated rows times norm_weight to out->x (batch, nheads * headdim) bf16 and their sums to

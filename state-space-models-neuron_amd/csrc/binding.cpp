@@ -1022,12 +1022,22 @@ Tensor linear_rows(const Tensor& x, const Tensor& w, const Tensor& bias, void* s
 const Tensor& stream_anchor(const ResidualStream& r) { return r.first.defined() ? r.first : r.ids.defined() ? r.table : r.rows; }
 int64_t stream_count(const ResidualStream& r) { return r.ids.defined() ? r.ids.numel() : stream_anchor(r).size(0); }
 
+// the stream's rows out of the embedding; norm_w: that norm's x and sq of them too
+void embed_rows(ResidualStream& r, const Tensor& norm_w) {
+    Scope scope(r.table);
+    r.rows = at::empty({r.ids.numel(), r.table.size(1)}, r.table.options().dtype(at::kFloat));
+    if (norm_w.defined()) {
+        r.x = at::empty(r.rows.sizes(), r.rows.options().dtype(at::kBFloat16));
+        r.sq = at::empty({r.rows.size(0), 1}, r.rows.options());
+    }
+    check(lib.m2_embed_rows(ptr(r.table), dtype_code(r.table), r.table.size(0), r.ids.data_ptr<int64_t>(), ptr<float>(r.rows), ptr<float>(norm_w), ptr(r.x),
+                            ptr<float>(r.sq), r.rows.size(0), r.rows.size(1), scope.stream), "m2_embed_rows");
+    r.table = r.ids = Tensor();
+}
+
 // the stream's rows, set from the embedding if they are not yet
 const Tensor& stream_rows(ResidualStream& r) {
-    if (r.ids.defined()) {
-        r.first = at::embedding(r.table, r.ids);
-        r.table = r.ids = Tensor();
-    }
+    if (r.ids.defined()) embed_rows(r, Tensor());
     if (r.first.defined()) {
         r.rows = r.first.to(at::kFloat, /*non_blocking=*/false, /*copy=*/true, at::MemoryFormat::Contiguous);
         r.first = Tensor();
@@ -1052,15 +1062,7 @@ Tensor stream_add_norm(ResidualStream& r, const Tensor& norm_w, double eps, at::
 // x and sq of the stream for a norm weight
 void stream_heads(ResidualStream& r, const Tensor& norm_w, void* stream) {
     if (r.x.defined()) return;
-    if (r.ids.defined()) {
-        r.rows = at::empty({r.ids.numel(), r.table.size(1)}, r.table.options().dtype(at::kFloat));
-        r.x = at::empty(r.rows.sizes(), r.rows.options().dtype(at::kBFloat16));
-        r.sq = at::empty({r.rows.size(0), 1}, r.rows.options());
-        check(lib.m2_embed_rows(ptr(r.table), dtype_code(r.table), r.table.size(0), r.ids.data_ptr<int64_t>(), ptr<float>(r.rows), ptr<float>(norm_w), ptr(r.x),
-                                ptr<float>(r.sq), r.rows.size(0), r.rows.size(1), stream), "m2_embed_rows");
-        r.table = r.ids = Tensor();
-        return;
-    }
+    if (r.ids.defined()) return embed_rows(r, norm_w);
     const bool set = r.first.defined();
     const Tensor src = set ? r.first.contiguous() : (r.delta.defined() ? r.delta.contiguous() : Tensor());
     if (set) r.rows = at::empty(src.sizes(), src.options().dtype(at::kFloat));
@@ -1179,7 +1181,7 @@ ResidualStream residual_stream(const Tensor& embedded) {
 ResidualStream embedded_stream(const Tensor& table, const Tensor& ids) {
     require_gpu({&table, &ids});
     const bool reads = (table.scalar_type() == at::kFloat || table.scalar_type() == at::kBFloat16) && table.dim() == 2 && table.is_contiguous() &&
-                       table.size(1) > 0 && ids.scalar_type() == at::kLong && ids.numel() <= 65535;
+                       table.size(1) > 0 && ids.scalar_type() == at::kLong && ids.numel() <= INT32_MAX;
     if (!reads) return residual_stream(at::embedding(table, ids));
     ResidualStream r;
     r.table = table;

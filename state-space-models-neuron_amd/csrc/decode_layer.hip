@@ -324,8 +324,8 @@ decode_rows_kernel(float* __restrict__ res, const T* __restrict__ add, const int
     const bool known = !ids || (id >= 0 && id < vocab);
     float s = 0.f;
     for (int64_t k = threadIdx.x * V; k < K; k += 256 * V) {
-        const fvec wv = *reinterpret_cast<const fvec*>(w + k);
-        fvec v = 0.f;
+        fvec wv = 0.f, v = 0.f;
+        if (w) wv = *reinterpret_cast<const fvec*>(w + k);
         if (!set) v = *reinterpret_cast<const fvec*>(res + row + k);
         if (!known) v = __builtin_nanf("");
         else if (add) {
@@ -334,6 +334,7 @@ decode_rows_kernel(float* __restrict__ res, const T* __restrict__ add, const int
             for (int e = 0; e < V; ++e) v[e] += to_f32(av[e]);
         }
         *reinterpret_cast<fvec*>(res + row + k) = v;
+        if (!w) continue;
         xvec xv;
 #pragma unroll
         for (int e = 0; e < V; ++e) {
@@ -342,6 +343,7 @@ decode_rows_kernel(float* __restrict__ res, const T* __restrict__ add, const int
         }
         *reinterpret_cast<xvec*>(x + row + k) = xv;
     }
+    if (!w) return;
     s = warp_sum(s);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
@@ -537,10 +539,10 @@ extern "C" int m2_decode_rows(float* residual, const void* delta, int32_t delta_
 extern "C" int m2_embed_rows(const void* table, int32_t table_dtype, int64_t vocab, const int64_t* ids, float* residual, const float* weight, void* x, float* sq,
                              int64_t rows, int64_t channels, void* stream) {
     using namespace m2;
-    M2_REQUIRE(rows >= 0 && rows <= 65535 && channels > 0 && vocab >= 0, M2_ERR_SHAPE, "embed_rows: rows %lld, channels %lld, vocab %lld", (long long)rows,
+    M2_REQUIRE(rows >= 0 && rows <= INT32_MAX && channels > 0 && vocab >= 0, M2_ERR_SHAPE, "embed_rows: rows %lld, channels %lld, vocab %lld", (long long)rows,
                (long long)channels, (long long)vocab);
     if (rows == 0) return M2_OK;
-    M2_REQUIRE(table && ids && residual && weight && x && sq, M2_ERR_NULL, "embed_rows: table, ids, residual, weight, x and sq are required");
+    M2_REQUIRE(table && ids && residual && !weight == !x && !weight == !sq, M2_ERR_NULL, "embed_rows: table, ids and residual are required, and weight, x and sq together or not at all");
     M2_DISPATCH_DTYPE(table_dtype, T, return launch_decode_rows<T>(residual, static_cast<const T*>(table), ids, vocab, 1, weight, static_cast<bf16_t*>(x), sq, rows,
                                                                    channels, static_cast<hipStream_t>(stream)));
     return M2_OK;

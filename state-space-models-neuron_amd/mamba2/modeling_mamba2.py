@@ -180,7 +180,8 @@ class Mamba2Model(Mamba2PreTrainedModel):
 
     def step(self, input_ids, cache_params: Optional[Mamba2Cache] = None):
         """input_ids: int64 (batch, 1), one token per sequence -> hidden states (batch, 1, hidden) after the final norm.
-        The caller advances ``cache_params.seqlen_offset`` (a host integer, so that a captured step stays replayable)."""
+        Where the model steps in its native residual stream, an id outside the embedding's table raises nothing: its sequence's results are NaN
+        and its states in the cache, which take them in, are lost; the other sequences are not touched.  The caller advances ``cache_params.seqlen_offset`` (a host integer, so that a captured step stays replayable)."""
         stream = self._step_stream(input_ids, cache_params)
         if stream is not None:
             act = self.layers[0].mixer.in_proj.weight.dtype
@@ -254,7 +255,8 @@ class Mamba2ForCausalLM(Mamba2PreTrainedModel):
         return Mamba2CausalLMOutput(loss=loss, logits=logits, cache_params=out.cache_params, hidden_states=out.hidden_states)
 
     def step(self, idx, cache_params: Optional[Mamba2Cache] = None):
-        """idx: int64 (batch, 1) -> logits (batch, 1, vocab) fp32; the layers' states in ``cache_params`` advance by one token."""
+        """idx: int64 (batch, 1) -> logits (batch, 1, vocab) fp32; the layers' states in ``cache_params`` advance by one token
+        (an id outside the table: see ``Mamba2Model.step``)."""
         native = _own_step(self.backbone, Mamba2Model) and _plain_linear(self.lm_head) and not torch.is_grad_enabled()
         stream = self.backbone._step_stream(idx, cache_params) if native else None
         if stream is not None:
@@ -316,7 +318,7 @@ class GraphedStep:
 
     The graph reads the token ids from ``self.input_ids`` and the states from ``cache_params`` (updated in place by the
     decode kernel, so each replay continues from the last) and leaves the logits in ``self.logits``; ``__call__`` copies
-    the ids in, replays and returns ``self.logits`` (overwritten by the next call).  The model's parameters and the cache
+    the ids in, replays and returns ``self.logits`` (overwritten by the next call; an id outside the table: see ``Mamba2Model.step``).  The model's parameters and the cache
     tensors must stay where they are, and the parameters unchanged, while the object lives (the graph holds their
     addresses, and for a model kept in bfloat16 the fp32 copies of the small per-head and norm parameters made before the
     capture): build a new object after loading other weights.  ``cache_params`` may be reset or refilled by a prefill

@@ -121,3 +121,15 @@ def test_embed_rows(rows, channels, offset, dtype):
     assert torch.equal(res[1:], want) and torch.equal(x[1:], (want * w).bfloat16())
     # fp32 sums of `channels` squares in another order: at most channels roundings of 2^-24 each
     assert torch.allclose(sq[1:, 0], want.pow(2).sum(1), rtol=channels * 2.0 ** -24, atol=0.0)
+
+
+def test_embed_rows_the_residual_alone():
+    from mamba2 import _lib
+    lib = _lib.load()
+    table = torch.randn(7, 130, device=DEV)
+    ids = torch.tensor([3, 7, 0], device=DEV)
+    res = torch.empty(3, 130, device=DEV)
+    args = (table.data_ptr(), _lib.M2_F32, 7, ids.data_ptr(), res.data_ptr())
+    assert lib.m2_embed_rows(*args, None, None, None, 3, 130, torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(res[[0, 2]], table[[3, 0]]) and res[1].isnan().all()
+    assert lib.m2_embed_rows(*args, table.data_ptr(), None, None, 3, 130, None) == -6      # weight, x and sq together

@@ -302,3 +302,26 @@ def test_greedy_generate_matches_recomputing_the_prefix(use_graph):
             assert ((top2[:, 0] - top2[:, 1]) > 1e-3).all(), "near tie: the comparison of token ids would not be meaningful"
             seq = torch.cat([seq, logits.argmax(-1, keepdim=True)], dim=1)
     assert got.shape == (3, 49) and torch.equal(got, seq)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("batch", [3, 33])      # the layers' own launches, and kernels behind one another
+@pytest.mark.parametrize("outside", [97, -1, 1 << 40])
+def test_step_with_an_id_outside_the_table(batch, dtype, outside):
+    """Its sequence is NaN, on whichever path; the others have the results and states that they have without it."""
+    from mamba2.mamba2_mixer import Mamba2Cache
+    cfg, m = _model(dtype)
+    ids = torch.randint(0, 97, (2, batch, 1), generator=torch.Generator().manual_seed(batch)).to(DEV)
+    wrong = ids[1].clone()
+    wrong[1] = outside
+    got = []
+    with torch.no_grad():
+        for second in (ids[1], wrong):
+            cache = Mamba2Cache(cfg, batch, dtype=dtype, device=DEV)
+            m.step(ids[0], cache)
+            logits = m.step(second, cache)
+            got.append([logits] + [t.clone() for t in cache.conv_states + cache.ssm_states])
+    others = [i for i in range(batch) if i != 1]
+    for a, b in zip(*got):
+        assert torch.equal(a[others], b[others])
+    assert got[1][0][1].isnan().all() and not got[0][0].isnan().any()
