@@ -54,7 +54,9 @@ template <typename F> void each_slicing(int64_t hpg, F&& f) {
 // what is left (with divisors of the heads per group only, a prime count had one head a slice or all of them: forward and backward at
 // b3 l1111 h31 166 -> 102 us, b1 l2130 h106 406 -> 266, fp32 b4 l416 h83 346 -> 258).  Their count is the one with the least of:
 // workgroups on the busiest CU times heads per slice -- a CU that could hold two (`wgs_per_cu`) and has one takes three
-// quarters of two's time --, 1.5 heads' worth for filling and draining each of them, and, `partials`, what the slices' partial
+// quarters of two's time, and with few tokens, where a head is latency, all of it (y at b9 l1 h58 p128 13.1 -> 9.9 us, b11 l9 h96 whole forward
+// 34.5 -> 32.2) --, 1.5 heads' worth for filling and draining each of them (of the longer fp32 heads half of that with few tokens: forward at b33 l6
+// h31 102 -> 98, b38 l4 h13 62 -> 58; with whole chunks b9 l903 h15 102 | 106), and, `partials`, what the slices' partial
 // sums cost on their way out and back (128 KiB each: a head's worth per 110 workgroups).  Taking whatever first filled the chip
 // instead left a nearly empty last round and twice the partials at b3 l1111 h32: main backward kernel 41 -> 31 us, dG 17.7 ->
 // 14.2, slice sums 17.9 -> 10.1, y 17.4 -> 15.4; y at b8 l333 h80 25.9 -> 22.1.
@@ -63,11 +65,13 @@ inline void ssd_slicing(const SsdCall* p, int wgs_per_cu, bool partials, int64_t
     const int64_t hpg = p->nheads / p->ngroups;
     const int64_t base = p->batch * nc * p->ngroups;
     const int64_t cus = device_cus();
+    const float whole = (float)(p->seqlen < kQ ? p->seqlen : kQ) / (float)kQ;      // how much of a chunk there is
+    const float alone = 1.f - 0.25f * whole, fill = p->dtype == M2_F32 ? 0.75f + 0.75f * whole : 1.5f;
     int64_t best = 1;
     float least = 1e30f;
     each_slicing(hpg, [&](int64_t s, int64_t heads) {
-        const float n = (float)ceil_div(base * s, cus), busy = n < (float)wgs_per_cu ? 0.75f * (float)wgs_per_cu : n;
-        const float cost = busy * (float)heads + 1.5f * n + (partials ? 0.009f * (float)(base * s) : 0.f);
+        const float n = (float)ceil_div(base * s, cus), busy = n < (float)wgs_per_cu ? alone * (float)wgs_per_cu : n;
+        const float cost = busy * (float)heads + fill * n + (partials ? 0.009f * (float)(base * s) : 0.f);
         if (cost < least) { least = cost; best = s; }
     });
     *nslices = best;
