@@ -250,19 +250,20 @@ ProductPlan product_plan(int64_t M, int64_t N, int64_t K) {
     return best;
 }
 
-// Both products of a linear layer's backward in one launch, in the same count: the longer chain of k steps, or all of them at the rate
-// of CUs with two workgroups each.  Only dx's sum, over the layer's outputs, gets long enough to be split.
-struct PairPlan { int splits, ksteps; float us, work; };      // work: k steps per CU
+// Both products of a linear layer's backward in one launch, in the same count: the longer chain of k steps (0.36 us each beside the other
+// product's), or all of them at the rate of CUs with two workgroups each.  Only dx's sum, over the layer's outputs, is split.
+struct PairPlan { int splits, ksteps; float us, work, dw_chain; };      // work: k steps per CU; dw_chain: us of dW's sum over the tokens
 PairPlan pair_plan(const m2_product_params& x, const m2_product_params& w) {
     const int64_t kx = ceil_div(x.K, (int64_t)kK), kw = ceil_div(w.K, (int64_t)kK);
     const int64_t tx = ceil_div(x.M, (int64_t)64) * ceil_div(x.N, (int64_t)64), tw = ceil_div(w.M, (int64_t)64) * ceil_div(w.N, (int64_t)64);
     const float work = (float)(tx * kx + tw * kw) / (float)device_cus();
-    PairPlan best{1, (int)kx, 1e30f, work};
+    const float dw_chain = 0.36f * (float)kw;
+    PairPlan best{1, (int)kx, 1e30f, work, dw_chain};
     for (int64_t want = 1; want <= 6 && (want == 1 || kx / want >= 4); ++want) {
         const int64_t ks = ceil_div(kx, want), n = ceil_div(kx, ks);
-        const float chain = 0.3f * (float)(ks > kw ? ks : kw);
+        const float dx_chain = 0.36f * (float)ks, chain = dx_chain > dw_chain ? dx_chain : dw_chain;
         const float us = (chain > 0.24f * work ? chain : 0.24f * work) + 1.2f + (n > 1 ? 1.6f + 3e-6f * (float)(n * x.M * x.N) : 0.f);
-        if (us < best.us) best = {(int)n, (int)ks, us, work};
+        if (us < best.us) best = {(int)n, (int)ks, us, work, dw_chain};
     }
     return best;
 }
@@ -358,17 +359,18 @@ extern "C" int m2_product(const m2_product_params* p, void* stream) {
     return launch_sum(a, st);
 }
 
-// Against two products of this file their own count decides (1.5 us for the launch more): 1.1 to 1.8 times as fast over the 40 such pairs
-// of layers of 256 to 1024 channels on 40 to 2000 tokens, and the one that it turns away is 3 % slower.  Where either would go to the
+// Against two products of this file their own count decides (3 us for the launch more): 1.1 to 1.8 times as fast over 40 such pairs
+// of layers of 256 to 1024 channels on 40 to 2000 tokens and 230 of 32 to 3000 channels on 8 to 60000.  Where either would go to the
 // general library: up to 150 k steps per CU.  Below it 40 tokens, 1024 channels 24.5 -> 14.1 us, 1000 tokens 54 -> 40, 500 tokens, 1536
 // channels, out_proj 30 -> 23.6, in_proj 48.5 -> 46.9; above it 1000 tokens, 1280 channels, in_proj 59 -> 67, 2048 channels, out_proj 54 -> 65.
+// And not where dW's sum over many tokens, which nothing splits here, outlasts the rest: 15785 tokens, 736 x 368 63 -> 87 us.
 extern "C" int m2_product_pair_pays(const m2_product_params* x, const m2_product_params* w) {
     using namespace m2;
     if (!x || !w || !x->a_k || x->b_k || w->a_k || w->b_k || x->bias || w->bias) return 0;
     if (!m2_product_fits(x->M, x->N, x->K, 1, 0) || !m2_product_fits(w->M, w->N, w->K, 0, 0)) return 0;
     const PairPlan plan = pair_plan(*x, *w);
-    if (!m2_product_pays(x->M, x->N, x->K, 1, 0) || !m2_product_pays(w->M, w->N, w->K, 0, 0)) return plan.work <= 150.f;
-    return plan.us < product_plan(x->M, x->N, x->K).us + product_plan(w->M, w->N, w->K).us + 1.5f;
+    if (!m2_product_pays(x->M, x->N, x->K, 1, 0) || !m2_product_pays(w->M, w->N, w->K, 0, 0)) return plan.work <= 150.f && (plan.dw_chain <= 12.f || plan.dw_chain <= 0.24f * plan.work);
+    return plan.us < product_plan(x->M, x->N, x->K).us + product_plan(w->M, w->N, w->K).us + 3.f;
 }
 
 extern "C" size_t m2_product_pair_workspace_bytes(const m2_product_params* x, const m2_product_params* w) {

@@ -103,3 +103,11 @@ def test_scan_asks_for_segments_where_a_walk_goes_in_them(lib, chunks):
     bhc = h * chunks
     want = bhc * 64 * n * 2 + bhc * 4 * (8 + 3 + 4 * q + 8) + bhc * q * q * 4 + (seg if chunks >= 48 else 0)      # a head a group: whole groups, one slice
     assert 0 <= lib.m2_ssd_bwd_workspace_bytes(ctypes.byref(p)) - want <= 20 * 256
+
+
+@pytest.mark.parametrize("tokens,ins,outs,pays", [(500, 768, 3352, 1), (40, 2048, 1024, 1), (23291, 592, 296, 0), (15785, 736, 368, 0), (4395, 896, 448, 0)])
+def test_product_pairs_leave_long_sums_to_products_that_split_them(lib, tokens, ins, outs, pays):
+    from mamba2 import _lib
+    x = _lib.ProductParams(M=tokens, N=ins, K=outs, a_k=1, b_k=0)
+    w = _lib.ProductParams(M=outs, N=ins, K=tokens, a_k=0, b_k=0)
+    assert lib.m2_product_pair_pays(x, w) == pays
