@@ -446,3 +446,20 @@ def test_ssd_segments_of_nothing(h, growth):
     y1, leaves = run(*(v[:, first].contiguous() for v in (x, d["B"], d["C"], dt)))
     for name, a, b in zip(("dX", "dB", "dC"), grads, torch.autograd.grad(y1, leaves, dy[:, first].contiguous())):
         assert torch.equal(a[:, first], b) and (a[:, 128:] == 0).all(), name
+
+
+@pytest.mark.parametrize("b,l,h,p,n,g", [(1, 6144, 2, 64, 128, 1), (1, 6017, 3, 128, 64, 1), (2, 6200, 12, 64, 64, 2)])
+def test_ssd_training_in_segments_against_the_oracle(b, l, h, p, n, g):
+    """Without a final state: the one-tile form of both recurrences, forward (from kept states and recomputed) and backward, against 64 bits."""
+    from mamba2.mamba2_kernel import alloc_chunk_states, ssd_backward, ssd_forward
+    d = make_ssd_inputs(b, l, h, p, n, g, seed=l + h, dtype=torch.bfloat16)
+    r, dv = _f64(d), _dev(d)
+    ref = ssd_grads_ref(r["dt"], r["A"], r["X"], r["B"], r["C"], r["D"], r["dy"], chunk=64)
+    five = [dv[k] for k in ("dt", "A", "X", "B", "C")]
+    states = alloc_chunk_states(*five)
+    y, _ = ssd_forward(*five, dv["D"], want_final_state=False, chunk_states=states)
+    tol, metric = _tol(torch.bfloat16)
+    assert metric(y, ref["y"]) < tol, "y"
+    for st in (states, None):
+        for name, v in zip(("ddt", "dA", "dX", "dB", "dC", "dD"), ssd_backward(*five, dv["D"], dv["dy"], chunk_states=st)):
+            assert metric(v, ref[name]) < tol, name

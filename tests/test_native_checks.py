@@ -111,3 +111,18 @@ def test_product_pairs_leave_long_sums_to_products_that_split_them(lib, tokens, 
     x = _lib.ProductParams(M=tokens, N=ins, K=outs, a_k=1, b_k=0)
     w = _lib.ProductParams(M=outs, N=ins, K=tokens, a_k=0, b_k=0)
     assert lib.m2_product_pair_pays(x, w) == pays
+
+
+def test_norm_checks_say_what_the_norms_refuse(lib):
+    """Both checks, on the host alone: a group of over 8192 channels, an output off its vectors, and a gate off its vectors, which the core's takes."""
+    from mamba2 import _lib
+    plain, core = lib.m2_rmsnorm_gated_fwd_check, lib.m2_core_norm_fwd_check
+
+    def params(channels=512, z=32, z_stride=512, out=48, out_stride=512, groups=1):
+        return _lib.RmsnormParams(x=16, z=z, weight=4, out=out, rows=3, channels=channels, x_stride_row=channels, z_stride_row=z_stride, out_stride_row=out_stride,
+                                  n_groups=groups, dtype=1, eps=1e-5)
+
+    for p, wanted in ((params(), (0, 0)), (params(z=34), (-3, 0)), (params(z_stride=515), (-3, 0)), (params(out=50), (-3, -3)), (params(out_stride=516), (-3, -3)),
+                      (params(channels=8256, z_stride=8256, out_stride=8256), (-1, -1)), (params(channels=8256, z_stride=8257, out_stride=8256, groups=3), (-3, 0)),
+                      (params(z=0, out=0), (-6, -6))):
+        assert (plain(ctypes.byref(p)), core(ctypes.byref(p))) == wanted
