@@ -126,16 +126,17 @@ __device__ __forceinline__ void store_vec(T* p, const float (&v)[GlueVec<T>::V])
     }
 }
 
-// sum over the WPG waves that share a (row, group); `slot` alternates between two LDS rows so that one barrier per
-// reduction is enough
+// sum over runs of LPG lanes
 template <int LPG>
-__device__ __forceinline__ float lanes_sum(float v) {      // over runs of LPG lanes
+__device__ __forceinline__ float lanes_sum(float v) {
     if constexpr (LPG == 64) return warp_sum(v);
     if constexpr (LPG >= 32) v = lane_xor_add<16>(v);
     if constexpr (LPG >= 16) v = lane_xor_add<8>(v);
     v = lane_xor_add<4>(v); v = lane_xor_add<2>(v); v = lane_xor_add<1>(v);
     return v;
 }
+// two sums over the lanes or, where WPG waves share a (row, group), over those; `slot` alternates between two LDS rows so that one barrier
+// per reduction is enough
 template <int WPG, int LPG>
 __device__ __forceinline__ void group_sum2(float& a, float& b, float (*red)[2][16], int slot) {
     a = lanes_sum<LPG>(a); b = lanes_sum<LPG>(b);

@@ -4,8 +4,10 @@
 //   forward:  S = init;   for c = 0 .. nc-1:   prev[c] = T(S);   S = e^{Lam_c} S + sum_j (dt_j e^{Lam_c - l_j}) x_j (x) B_j;   final = S
 //   reverse:  R = dfinal; for c = nc-1 .. 0:   prev[c] = T(R);   R = e^{Lam_c} R + sum_i e^{l_i} dy_i (x) C_i;   dinit = R
 //
-// grid (nheads * SPLIT, batch), N / 32 waves; a workgroup owns 1 / SPLIT of the ROWS of the [P][N] state (head channels; all N
-// columns), wave w the columns [32 w, +32) of them, as 32x32 MFMA accumulator blocks: only that part of the x / dy columns
+// grid (nheads * SPLIT, batch, segments), N / 32 waves.  Segments: one, the walk over all chunks (PHASE 0); or, of few heads' long walks, two
+// launches over all segments but one (PHASE 1 walks the first, storing the states, and forms the sums of the middle ones from zero, storing nothing
+// else; PHASE 2 walks the second to the last from the sums in front of each).  A workgroup owns 1 / SPLIT of the ROWS of the [P][N] state (head
+// channels; all N columns), wave w the columns [32 w, +32) of them, as 32x32 MFMA accumulator blocks: only that part of the x / dy columns
 // is loaded, scaled and staged, so the workgroups of a head share no work.  Per chunk the MFMA computes
 // X_scaled^T [P/2 x kQ] * M [kQ x N]:
 //   * M (B or C of the group) comes from the transposed tiles that prep_kernel wrote in MFMA operand order: a wave's
